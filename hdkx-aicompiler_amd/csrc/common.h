@@ -153,11 +153,14 @@ int32_t LaunchPreparedWinograd(const PreparedWinograd* p, const float* x, const 
 void FreePreparedWinograd(PreparedWinograd* p);
 
 // The filter transforms of several Winograd layers in one launch (conv2d_wino_f32.hip).
+constexpr uint32_t kWinoFormF32 = 1, kWinoFormThreePart = 2;
 struct WinoWeightJob {
     const kxc_hip_conv2d_desc* desc;
     const float* w;      // OIHW weights
     float* u;            // kxc_hip_conv2d_winograd_weight_bytes(desc) bytes
+    uint32_t forms;      // kWinoForm*: the forms of the filter to write (PreparedWinogradForms: what a launch reads)
 };
+uint32_t PreparedWinogradForms(const PreparedWinograd* p);
 int32_t LaunchWinogradWeightTransforms(const WinoWeightJob* jobs, int32_t count, hipStream_t stream);
 
 // The int8 weight tensors of several convolutions packed by one launch (qconv_c16_i8.hip); kind = KXC_HIP_QPACK_*.

@@ -109,6 +109,12 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* p, uint3
 
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
+}  // namespace
+
+#include "conv_bf16x3.h"
+
+namespace {
+
 // KS: split of the reduction inside the workgroup.  The waves form KS groups; group g owns its own pair of
 // LDS tiles and works on chunks g, g+KS, ...; the partial accumulators are added through LDS in group
 // order at the end (deterministic).  It multiplies the waves per output block for launches that have too
@@ -1127,14 +1133,114 @@ bool PairTap(const kxc_hip_conv2d_desc* d, int* rh, int* rw) {
     return oh == (d->h - 1) / d->stride_h + 1 && ow == (d->w - 1) / d->stride_w + 1;
 }
 
+// ------------------------------------------------------------------------------------------
+// Launches on the bf16 matrix cores with three-part operands (conv_bf16x3.h).
+// ------------------------------------------------------------------------------------------
+struct BxVariant {
+    const char* tile;           // name = mfma_k<kh>x<kw>_bf16x3_<tile>
+    int to, tp, threads, ks, ix, iw, c4;
+    void (*kernel)(const conv_bx::Args);
+    void (*ds_kernel)(const conv_bx::Args);
+};
+#define KXC_BX(TILE, RO, RP, WO, WP, KS, IX, IW)                                                                          \
+    {TILE, 32 * RO * WO, 32 * RP * WP, 64 * WO * WP * KS, KS, IX, IW, 0, conv_bx::conv_bf16x3_kernel<RO, RP, WO, WP, KS, IX, IW, false, false>, \
+     conv_bx::conv_bf16x3_kernel<RO, RP, WO, WP, KS, IX, IW, false, true>}
+#define KXC_BX_C4(TILE, RO, RP, WO, WP, KS, IX, IW)                                                                       \
+    {TILE, 32 * RO * WO, 32 * RP * WP, 64 * WO * WP * KS, KS, IX, IW, 1, conv_bx::conv_bf16x3_kernel<RO, RP, WO, WP, KS, IX, IW, true, false>, nullptr}
+const BxVariant kBx[] = {
+    KXC_BX("o64_p256", 2, 2, 1, 4, 1, 4, 3),
+    KXC_BX("o64_p128", 2, 1, 1, 4, 1, 4, 3),
+    KXC_BX("o64_p64", 1, 1, 2, 2, 1, 4, 3),
+    KXC_BX("o32_p32_ks4", 1, 1, 1, 1, 4, 5, 5),
+    KXC_BX_C4("c4_o64_p256", 2, 2, 1, 4, 1, 13, 4),
+    KXC_BX_C4("c4_o64_p64", 1, 1, 2, 2, 1, 8, 4),
+};
+constexpr int kNumBx = sizeof(kBx) / sizeof(kBx[0]);
+
+struct BxChoice {
+    const BxVariant* v = nullptr;
+    int32_t cb = 1, nq = 0, nq_main = 0, group_steps = 0, ngroups = 0, chs = 0;
+    size_t lds_bytes = 0;
+};
+
+bool BxFits(const BxVariant& v, const ConvArgs& a, int kh, int kw, bool ds, BxChoice* out) {
+    if (ds && !v.ds_kernel) return false;
+    if (v.c4 && (a.C > 4 || a.dw != 1)) return false;
+    const int64_t positions = static_cast<int64_t>(MaxTileRows(a, kh, v.tp)) * a.Wp;
+    const int32_t chs = static_cast<int32_t>((positions + 3) / 4 * 4);
+    const int cbs = (a.C + 7) / 8, wrow = (v.to + 1) * 16;
+    const int max_cb = v.c4 ? 1 : kh * kw == 1 || v.ks > 1 ? 16 : 1;
+    for (int cb = max_cb < cbs ? max_cb : cbs; cb >= 1; --cb) {
+        if (positions > (1 << 20) || static_cast<int64_t>(cb) * chs > static_cast<int64_t>(v.ix) * v.threads) continue;
+        const int nq_main = v.c4 ? (kh * ((kw + 1) / 2) + 1) / 2 * 2 : (kh * kw * cb + 1) / 2 * 2;
+        const int nq = nq_main + (ds ? (cb + 1) / 2 * 2 : 0);
+        if (nq > conv_bx::kMaxQ) continue;
+        const int max_steps = v.iw * v.threads / (2 * v.to);
+        const int groups = (nq / 2 + max_steps - 1) / max_steps, gs = (nq / 2 + groups - 1) / groups;
+        if (v.ks > 1 && groups > 1) continue;
+        size_t lds = conv_bx::kMaxQ * 4 + 3 * static_cast<size_t>(cb) * chs * (v.c4 ? 8 : 16) + 3 * 2 * static_cast<size_t>(gs) * wrow;
+        const size_t red = static_cast<size_t>(v.ks - 1) * v.to * v.tp * sizeof(float);
+        if (red > lds) lds = red;
+        if (lds > kMaxLdsBytes) continue;
+        out->v = &v; out->cb = cb; out->nq = nq; out->nq_main = nq_main; out->group_steps = gs;
+        out->ngroups = (nq / 2 + gs - 1) / gs; out->chs = chs; out->lds_bytes = lds;
+        return true;
+    }
+    return false;
+}
+
+const char* BxName(const BxVariant& v, int kh, int kw) {
+    static std::mutex mu;
+    static std::vector<std::unique_ptr<std::string>> names;      // a handful: one per filter size and tile in use
+    const std::string name = "mfma_k" + std::to_string(kh) + "x" + std::to_string(kw) + "_bf16x3_" + v.tile;
+    std::lock_guard<std::mutex> lock(mu);
+    for (const auto& n : names)
+        if (*n == name) return n->c_str();
+    names.emplace_back(new std::string(name));
+    return names.back()->c_str();
+}
+
+// The three-part launch of a shape (after FillArgs and ApplyRowView), or v == nullptr for the fp32-instruction kernels.
+void BxSelect(const ConvArgs& a, const kxc_hip_conv2d_desc* d, bool ds, BxChoice* choice) {
+    choice->v = nullptr;
+    if ((d->flags & (KXC_HIP_CONV_FORCE_DIRECT | KXC_HIP_CONV_HPOOL)) || a.M <= 0) return;
+    const int64_t x_bytes = static_cast<int64_t>(a.N) * a.C * a.H * a.W * 4, y_elems = static_cast<int64_t>(a.N) * a.O * a.OHW;
+    const int64_t w_bytes = static_cast<int64_t>(a.O) * a.C * d->kh * d->kw * 4, q_rows = static_cast<int64_t>(a.N + 1) * a.Hp + static_cast<int64_t>(d->kh) * a.dh;
+    if (x_bytes >= (1LL << 31) || y_elems * 4 >= (1LL << 31) || w_bytes >= (1LL << 31) || q_rows * a.Wp >= (1LL << 31)) return;
+    const char* forced = std::getenv("KXC_HIP_CONV_VARIANT");
+    const char* bx = std::getenv("KXC_HIP_CONV_BF16X3");
+    if (bx && bx[0] == '0') return;
+    for (const BxVariant& v : kBx) {
+        if (forced && *forced) {
+            if (std::strcmp(forced, BxName(v, d->kh, d->kw)) != 0) continue;
+        } else {
+            return;
+        }
+        if (BxFits(v, a, d->kh, d->kw, ds, choice)) return;
+        choice->v = nullptr;
+    }
+}
+
+// Parts of a split reduction of a three-part launch.
+int BxSplit(const BxChoice& c, int32_t nchunks, int64_t tiles, int64_t total) {
+    int split = 1;
+    if (const char* e = std::getenv("KXC_HIP_CONV_GSPLIT")) {
+        const int f = std::atoi(e);
+        if (f >= 1 && f <= nchunks && total * static_cast<int64_t>(sizeof(float)) * f <= (256LL << 20)) split = f;
+    }
+    return split;
+}
+
 // Everything about a launch that the descriptor alone decides (kernel, tile shape, grid, the split of the reduction,
 // the switches read from the environment): resolved once per call by the entry points, once per node by a launch
 // plan (kxc_hip::PreparedConv), and combined with the operand pointers and the stream at launch time.
 struct ConvLaunch {
-    enum Path { kEmpty, kSmall1x1, kMfma, kDirect };
+    enum Path { kEmpty, kSmall1x1, kMfma, kDirect, kBf16x3 };
     Path path = kEmpty;
     ConvArgs a;                     // without operand pointers and partial-sum buffer
     ConvArgs direct_args;
+    conv_bx::Args bx;               // kBf16x3: instead of `a` (which keeps the flags and the split)
+    void (*bx_kernel)(const conv_bx::Args) = nullptr;
     void (*kernel)(const ConvArgs) = nullptr;
     const char* name = "";
     dim3 grid, block;
@@ -1144,6 +1250,48 @@ struct ConvLaunch {
     int64_t total = 0;
     bool second = false;
 };
+
+int32_t BxResolve(const kxc_hip_conv2d_desc* desc, bool second, const char* who, const BxChoice& c, ConvLaunch* L) {
+    ConvArgs& a = L->a;
+    conv_bx::Args& b = L->bx;
+    std::memset(&b, 0, sizeof(b));
+    b.N = a.N; b.C = a.C; b.H = a.H; b.W = a.W; b.O = a.O; b.OH = a.OH; b.OW = a.OW; b.KH = desc->kh; b.KW = desc->kw;
+    b.sh = a.sh; b.sw = a.sw; b.ph = a.ph; b.pw = a.pw; b.dh = a.dh; b.dw = a.dw;
+    b.Hp = a.Hp; b.Wp = a.Wp; b.Hv = a.Hv; b.row_step = a.row_step; b.M = a.M; b.OHW = a.OHW;
+    b.chs = c.chs; b.cb = c.cb; b.nq = c.nq; b.nq_main = c.nq_main; b.group_steps = c.group_steps; b.ngroups = c.ngroups;
+    b.nchunks = c.v->c4 ? 1 : (a.C + 8 * c.cb - 1) / (8 * c.cb);
+    if (second) {
+        int rh = 0, rw = 0;
+        KXC_HIP_REQUIRE(PairTap(desc, &rh, &rw), "%s: no kernel with a second output covers this shape", who);
+        b.ds_off = rh * a.dh * a.Wp + rw * a.dw;
+        b.w2_bytes = static_cast<uint32_t>(static_cast<int64_t>(a.O) * a.C * 4);
+    }
+    b.p_tiles = static_cast<int32_t>(CeilDiv(a.M, c.v->tp));
+    b.o_tiles = static_cast<int32_t>(CeilDiv(a.O, c.v->to));
+    const int64_t tiles = static_cast<int64_t>(b.p_tiles) * b.o_tiles;
+    KXC_HIP_REQUIRE(tiles < (1LL << 30), "%s: too many tiles", who);
+    b.num_tiles = static_cast<int32_t>(tiles);
+    b.out_elems = L->total;
+    const int split = BxSplit(c, b.nchunks, tiles, L->total * (second ? 2 : 1));
+    b.cps = static_cast<int32_t>(CeilDiv(b.nchunks, split));
+    b.gsplit = static_cast<int32_t>(CeilDiv(b.nchunks, b.cps));      // no empty part
+    a.gsplit = b.gsplit;
+    if (b.gsplit > 1) L->scratch_bytes = static_cast<size_t>(b.gsplit) * L->total * sizeof(float) * (second ? 2 : 1);
+    b.tiles_per_xcd = static_cast<int32_t>(CeilDiv(tiles * b.gsplit, 8));
+    b.x_bytes = a.x_bytes; b.w_bytes = a.w_bytes; b.flags = a.flags;
+    b.div_wp = MakeFastDiv(a.Wp); b.div_hp = MakeFastDiv(a.Hp); b.div_ohw = MakeFastDiv(a.OHW); b.div_ow = MakeFastDiv(a.OW);
+    a.div_ohw = b.div_ohw;
+    b.div_otiles = MakeFastDiv(b.o_tiles); b.div_ptiles = MakeFastDiv(b.p_tiles); b.div_gsplit = MakeFastDiv(b.gsplit);
+    b.div_chs = MakeFastDiv(b.chs); b.div_gq = MakeFastDiv(2 * b.group_steps); b.div_cb = MakeFastDiv(b.cb); b.div_kw = MakeFastDiv(b.KW);
+    b.o_fastest = static_cast<int64_t>(a.w_bytes) <= (2 << 20) ? 1 : 0;
+    L->path = ConvLaunch::kBf16x3;
+    L->bx_kernel = second ? c.v->ds_kernel : c.v->kernel;
+    L->name = BxName(*c.v, desc->kh, desc->kw);
+    L->grid = dim3(static_cast<unsigned>(b.tiles_per_xcd * 8));
+    L->block = dim3(static_cast<unsigned>(c.v->threads));
+    L->lds_bytes = c.lds_bytes;
+    return KXC_HIP_OK;
+}
 
 int32_t Conv2dResolve(const kxc_hip_conv2d_desc* desc, bool second, const char* who, ConvLaunch* L) {
     ConvArgs& a = L->a;
@@ -1178,6 +1326,9 @@ int32_t Conv2dResolve(const kxc_hip_conv2d_desc* desc, bool second, const char* 
     }
     L->direct_args = a;
     ApplyRowView(&a, desc->kh);
+    BxChoice bc;
+    BxSelect(a, desc, second, &bc);
+    if (bc.v) return BxResolve(desc, second, who, bc, L);
     Choice c;
     if (hpool) {
         KXC_HIP_REQUIRE(!second && HpoolChoice(desc, a, &c), "%s: no kernel with the pooling epilogue covers this shape", who);
@@ -1245,12 +1396,11 @@ int32_t Conv2dResolve(const kxc_hip_conv2d_desc* desc, bool second, const char* 
 }
 
 // Above the default 64 KiB the dynamic LDS size has to be granted per kernel and device (once).
-int32_t GrantLds(void (*kernel)(const ConvArgs), size_t lds_bytes) {
+int32_t GrantLds(const void* fn) {
     static std::mutex mu;
     static std::vector<std::pair<int, const void*>> granted;
     int dev = 0;
     KXC_HIP_CALL(hipGetDevice(&dev), "hipGetDevice");
-    const void* fn = reinterpret_cast<const void*>(kernel);
     std::lock_guard<std::mutex> lock(mu);
     for (const auto& g : granted)
         if (g.first == dev && g.second == fn) return KXC_HIP_OK;
@@ -1307,8 +1457,15 @@ int32_t Conv2dLaunch(const ConvLaunch& L, const char* who, const float* x, const
         }
     }
     if (L.lds_bytes > 64 * 1024)
-        if (int32_t rc = GrantLds(L.kernel, L.lds_bytes)) return rc;
-    hipLaunchKernelGGL(L.kernel, NoteGrid(L.grid), NoteBlock(L.block), NoteLds(L.lds_bytes), s, a);
+        if (int32_t rc = GrantLds(L.path == ConvLaunch::kBf16x3 ? reinterpret_cast<const void*>(L.bx_kernel) : reinterpret_cast<const void*>(L.kernel))) return rc;
+    if (L.path == ConvLaunch::kBf16x3) {
+        conv_bx::Args b = L.bx;
+        b.x = x; b.w = w; b.bias = bias; b.res = residual; b.y = y; b.partial = a.partial;
+        b.w2 = a.w2; b.bias2 = a.bias2; b.y2 = a.y2;
+        hipLaunchKernelGGL(L.bx_kernel, NoteGrid(L.grid), NoteBlock(L.block), NoteLds(L.lds_bytes), s, b);
+    } else {
+        hipLaunchKernelGGL(L.kernel, NoteGrid(L.grid), NoteBlock(L.block), NoteLds(L.lds_bytes), s, a);
+    }
     if (int32_t rc = CheckLaunch(L.name)) return rc;
     if (a.gsplit > 1) {
         SplitReduceArgs r;
@@ -1373,6 +1530,9 @@ const char* kxc_hip_conv2d_variant(const kxc_hip_conv2d_desc* desc) {
     if (desc->flags & KXC_HIP_CONV_FORCE_DIRECT) return "direct";
     if (UseSmall1x1(desc, a)) return "mfma_k1x1_small";
     ApplyRowView(&a, desc->kh);
+    BxChoice bc;
+    BxSelect(a, desc, false, &bc);
+    if (bc.v) return BxName(*bc.v, desc->kh, desc->kw);
     Choice c;
     Select(a, desc->kh, desc->kw, &c);
     return c.v ? c.v->name : "direct";
@@ -1459,6 +1619,14 @@ int32_t kxc_hip_conv2d_scratch_needed(const kxc_hip_conv2d_desc* desc, size_t* o
     const int64_t total = static_cast<int64_t>(a.N) * a.O * a.OHW;
     if (total == 0 || (desc->flags & (KXC_HIP_CONV_FORCE_DIRECT | KXC_HIP_CONV_HPOOL)) || UseSmall1x1(desc, a) || a.M <= 0) return KXC_HIP_OK;
     ApplyRowView(&a, desc->kh);
+    BxChoice bc;
+    BxSelect(a, desc, false, &bc);
+    if (bc.v) {
+        ConvLaunch L;
+        if (int32_t rc = Conv2dResolve(desc, false, "kxc_hip_conv2d_scratch_needed", &L)) return rc;
+        *out_bytes = L.scratch_bytes;
+        return KXC_HIP_OK;
+    }
     Choice c;
     Select(a, desc->kh, desc->kw, &c);
     if (!c.v) return KXC_HIP_OK;

@@ -86,6 +86,12 @@ __device__ __forceinline__ float load_f32(__amdgpu_buffer_rsrc_t rsrc, uint32_t 
 // max(v, 0) with NaN -> 0, as (v > 0 ? v : 0) gives; one instruction instead of a compare and a select
 __device__ __forceinline__ float relu_sel(float v) { return __builtin_fmaxf(v, 0.0f); }
 
+}  // namespace
+
+#include "wino_bf16x3.h"
+
+namespace {
+
 // ------------------------------------------------------------------------------------------
 // Filter transform, for o < 32*ceil(O/32) (absent output channels give zero blocks).
 // packed index: ((o/32 * csteps + c/4) * 2048) + (((c%4)*2 + (o%32)/16)*4 + i)*64 + (o%16)*4 + j  for U[i][j]
@@ -140,26 +146,24 @@ __device__ __forceinline__ void wino_weight_tile(const float* __restrict__ w, fl
 }
 inline int64_t WeightTiles(int64_t o_padded, int64_t C) { return (o_padded / 32) * ((C + kWeightTileC - 1) / kWeightTileC); }
 
-__global__ void __launch_bounds__(256) wino_weight_kernel(const float* __restrict__ w, float* __restrict__ u, int32_t O,
-                                                          int32_t C) {
-    __shared__ float raw[32 * (kWeightTileC * 9 + 1)];
-    wino_weight_tile(w, u, O, C, blockIdx.x, raw);
-}
-
 // The filter transforms of several layers in one launch (a launch plan transforms all its Winograd layers' weights
 // at the start of a run): block b belongs to the job whose [first_block, next first_block) range holds it.
+// A job is one form of one tensor: fp32 (wino_kernel) or three-part bf16 (wino_bf16x3_kernel).
 constexpr int kMaxWeightJobs = 32;
 struct WinoWeightBatch {
     const float* w[kMaxWeightJobs];
-    float* u[kMaxWeightJobs];
+    char* u[kMaxWeightJobs];
     int32_t O[kMaxWeightJobs], C[kMaxWeightJobs], first_block[kMaxWeightJobs + 1];
+    uint32_t three_part;       // bit j: job j writes the three-part form
     int32_t count;
 };
 __global__ void __launch_bounds__(256) wino_weight_batch_kernel(const WinoWeightBatch b) {
-    __shared__ float raw[32 * (kWeightTileC * 9 + 1)];
+    __shared__ float raw[32 * (wino_bx::kStep * 9 + 1)];
     int j = 0;
     while (j + 1 < b.count && static_cast<int32_t>(blockIdx.x) >= b.first_block[j + 1]) ++j;
-    wino_weight_tile(b.w[j], b.u[j], b.O[j], b.C[j], static_cast<int>(blockIdx.x) - b.first_block[j], raw);
+    const int tile = static_cast<int>(blockIdx.x) - b.first_block[j];
+    if ((b.three_part >> j) & 1u) wino_bx::weight_tile(b.w[j], b.u[j], b.O[j], b.C[j], tile, raw);
+    else wino_weight_tile(b.w[j], reinterpret_cast<float*>(b.u[j]), b.O[j], b.C[j], tile, raw);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -575,6 +579,7 @@ wino_kernel(const WinoArgs a) {
     store_all(make_rsrc(a.y, y_bytes), yv, Cached{});
 }
 
+constexpr const char* kThreePart = "winograd_f2k3_bf16x3";
 struct WinoVariant {
     const char* name;
     int wk, wt, ks;
@@ -592,6 +597,7 @@ const WinoVariant kWino[] = {
     KXC_WINO(1, 2),   // 32 x 32, 2 waves
     KXC_WINO_KS2(2, 2),  // 64 x 32, input channels split over two groups of 4 waves (96 KiB of LDS)
     KXC_WINO_KS2(2, 1),  // 64 x 16, two groups of 2 waves
+    {kThreePart, 2, 4, 1, nullptr, nullptr},      // 64 x 64 on the bf16 matrix cores, 8 waves (wino_bf16x3.h)
 };
 constexpr int kNumWino = sizeof(kWino) / sizeof(kWino[0]);
 
@@ -608,6 +614,17 @@ bool Supported(const kxc_hip_conv2d_desc* d) {
     const int64_t u_bytes = CeilDiv(d->o, 32) * 32 * static_cast<int64_t>(d->c) * 64;
     const int64_t tiles = static_cast<int64_t>(d->n) * CeilDiv(oh, 2) * CeilDiv(ow, 2);
     return x_bytes < (1LL << 31) && y_elems * 4 < (1LL << 31) && u_bytes < (1LL << 31) && tiles < (1LL << 30);
+}
+
+// A filter buffer holds both forms, the fp32 one first: which of them a launch reads depends on the batch it runs on.
+size_t F32FilterBytes(const kxc_hip_conv2d_desc* d) { return static_cast<size_t>(CeilDiv(d->o, 32)) * 32 * static_cast<size_t>(d->c) * 64; }
+
+// Whether the patch of every workgroup of the three-part kernel fits its LDS planes.
+bool ThreePartFits(const kxc_hip_conv2d_desc* d) {
+    const int64_t oh = static_cast<int64_t>(d->h) + 2 * d->pad_h - 2, ow = static_cast<int64_t>(d->w) + 2 * d->pad_w - 2;
+    const int64_t TW = CeilDiv(ow, 2), TH = CeilDiv(oh, 2), Hq = 2 * TH + 2, Wq = 2 * TW + 2;
+    if (wino_bx::WeightBytes(d->o, d->c) >= (1ull << 31) || (static_cast<int64_t>(d->n) + 1) * Hq * Wq >= (1LL << 30)) return false;
+    return wino_bx::MaxPatchRows(static_cast<int64_t>(d->n) * TH * TW, TH * TW, TW, Hq) * Wq <= wino_bx::kPlanes[1];
 }
 
 int64_t Tiles(const kxc_hip_conv2d_desc* d) {
@@ -641,19 +658,40 @@ int GroupSplit(int64_t units, int csteps, int64_t out_elems) {
     return split;
 }
 
+// Parts of a split reduction of the three-part kernel, one workgroup of which fills a compute unit: as many as there are
+// compute units for, of at least two steps each, with partial outputs below 16 MiB.
+int ThreePartSplit(int64_t units, int ksteps, int64_t out_elems) {
+    int split = 1;
+    while (split < 8 && units * split * 2 <= 256 && ksteps / (split * 2) >= 2 &&
+           out_elems * static_cast<int64_t>(sizeof(float)) * split * 2 <= (16LL << 20))
+        split *= 2;
+    return split;
+}
+
 // Measured on MI355X: 64 x 32 workgroups (four waves) are the fastest shape once there is one per compute unit;
 // smaller launches run faster as twice as many 64 x 16 workgroups of two waves.
 const WinoVariant* SelectWino(const kxc_hip_conv2d_desc* d) {
     if (const char* e = std::getenv("KXC_HIP_WINOGRAD_VARIANT")) {
         for (int i = 0; i < kNumWino; ++i)
-            if (std::strcmp(e, kWino[i].name) == 0 && (kWino[i].ks == 1 || (d->c / 4) % kWino[i].ks == 0)) return &kWino[i];
+            if (std::strcmp(e, kWino[i].name) == 0 && (kWino[i].ks == 1 || (d->c / 4) % kWino[i].ks == 0) &&
+                (kWino[i].kernel || ThreePartFits(d)))
+                return &kWino[i];
     }
     const int csteps = d->c / 4;
     const int64_t oh = static_cast<int64_t>(d->h) + 2 * d->pad_h - 2, ow = static_cast<int64_t>(d->w) + 2 * d->pad_w - 2;
+    const int64_t lanes = SelectLanes();
+    // From about 28 million (tile, output channel, input channel) triples on the bf16 matrix cores win: 12 images of the
+    // 56 x 56 / 28 x 28 / 14 x 14 / 7 x 7 layers (38 million each) 21.5 / 27.3 / 27.0 / 27.3 us against 27.4 / 30.8 / 30.5 /
+    // 29.7, 8 images (26 million) 22.7 / 21.9 / 23.8 / 25.5 against 21.7 / 20.4 / 26.1 / 26.5, 4 images 20.0 / 19.5 / 19.3 /
+    // 23.8 against 14.0 / 16.8 / 17.2 / 17.7.  KXC_HIP_WINOGRAD_BF16X3=0 keeps the fp32 instructions.
+    const char* bx = std::getenv("KXC_HIP_WINOGRAD_BF16X3");
+    if (!(bx && bx[0] == '0') && Tiles(d) * lanes * d->o * d->c >= 28000000LL && ThreePartFits(d)) {
+        for (int i = 0; i < kNumWino; ++i)
+            if (!kWino[i].kernel) return &kWino[i];
+    }
     // Small launches (batch 1-8 of ResNet-18): 64 x 16 groups with the channels split over workgroups beat both
     // the split inside the workgroup and the implicit-GEMM kernel (batch 1, 512 channels: 14.7 against 62.9 and
     // 20.0 us).
-    const int64_t lanes = SelectLanes();
     const int64_t units_t1 = CeilDiv(Tiles(d), 16) * CeilDiv(d->o, 64) * lanes;
     if (GroupSplit(units_t1, csteps, static_cast<int64_t>(d->n) * d->o * oh * ow) > 1) {
         for (int i = 0; i < kNumWino; ++i)
@@ -679,7 +717,47 @@ struct WinoLaunch {
     size_t scratch_bytes = 0;   // partial outputs of a split over workgroups (0: none)
     size_t lds_bytes = 0;
     bool fuse = false;          // the part that arrives last adds the parts: no adding kernel
+    bool three_part = false;    // wino_bf16x3_kernel with `bx` instead of v->kernel with `a`
+    wino_bx::Args bx;
+    int bx_plane = 0;
+    size_t u_offset = 0;        // of the three-part form in the filter buffer
 };
+
+// Shape, grid and split of a three-part launch.
+void ThreePartResolve(const kxc_hip_conv2d_desc* d, WinoLaunch* L) {
+    wino_bx::Args& b = L->bx;
+    std::memset(&b, 0, sizeof(b));
+    const WinoArgs& a = L->a;
+    b.N = a.N; b.C = a.C; b.H = a.H; b.W = a.W; b.O = a.O; b.OH = a.OH; b.OW = a.OW; b.ph = a.ph; b.pw = a.pw;
+    b.TW = a.TW; b.TI = a.TI; b.NT = a.NT; b.HW = a.HW; b.OHW = a.OHW;
+    b.Hq = 2 * (a.TI / a.TW) + 2; 
+    const int64_t rows = wino_bx::MaxPatchRows(b.NT, b.TI, b.TW, b.Hq);
+    b.pitch = wino_bx::RowPitch(b.TW, rows, wino_bx::kPlanes[1]);
+    L->bx_plane = rows * 2 * b.pitch <= wino_bx::kPlanes[0] ? 0 : 1;
+    b.ksteps = static_cast<int32_t>(CeilDiv(a.C, wino_bx::kStep));
+    b.t_groups = static_cast<int32_t>(CeilDiv(a.NT, wino_bx::kTiles));
+    b.k_groups = static_cast<int32_t>(CeilDiv(a.O, wino_bx::kOut));
+    b.num_units = b.t_groups * b.k_groups;
+    b.x_bytes = a.x_bytes; b.flags = a.flags;
+    b.u_bytes = static_cast<uint32_t>(wino_bx::WeightBytes(a.O, a.C));
+    L->u_offset = F32FilterBytes(d);
+    int split = ThreePartSplit(b.num_units * static_cast<int64_t>(SelectLanes()), b.ksteps, L->out_elems);
+    if (const char* e = std::getenv("KXC_HIP_WINOGRAD_GSPLIT")) {
+        const int f = std::atoi(e);
+        if (f >= 1 && f <= b.ksteps && L->out_elems * static_cast<int64_t>(sizeof(float)) * f <= (256LL << 20)) split = f;
+    }
+    b.steps_per_split = static_cast<int32_t>(CeilDiv(b.ksteps, split));
+    b.gsplit = static_cast<int32_t>(CeilDiv(b.ksteps, b.steps_per_split));      // no empty part
+    if (b.gsplit > 1) L->scratch_bytes = static_cast<size_t>(b.gsplit) * L->out_elems * sizeof(float);
+    b.units_per_xcd = static_cast<int32_t>(CeilDiv(static_cast<int64_t>(b.num_units) * b.gsplit, 8));
+    b.k_fastest = b.u_bytes <= (2u << 20) ? 1 : 0;
+    if (const char* e = std::getenv("KXC_HIP_WINOGRAD_KFAST")) b.k_fastest = std::atoi(e);
+    b.div_ti = MakeFastDiv(b.TI); b.div_tw = MakeFastDiv(b.TW);
+    b.div_kgroups = MakeFastDiv(b.k_groups); b.div_tgroups = MakeFastDiv(b.t_groups); b.div_gsplit = MakeFastDiv(b.gsplit);
+    b.div_pitch = MakeFastDiv(b.pitch); b.div_hq = MakeFastDiv(b.Hq);
+    L->three_part = true;
+    L->lds_bytes = wino_bx::kLdsBytes;
+}
 
 int32_t WinoResolve(const kxc_hip_conv2d_desc* desc, WinoLaunch* L) {
     KXC_HIP_REQUIRE(desc && Supported(desc), "kxc_hip_conv2d_winograd_nchw_f32: unsupported shape");
@@ -709,6 +787,7 @@ int32_t WinoResolve(const kxc_hip_conv2d_desc* desc, WinoLaunch* L) {
     a.steps_per_split = a.csteps;
     const int64_t out_elems = static_cast<int64_t>(a.N) * a.O * a.OHW;
     L->out_elems = out_elems;
+    if (!v->kernel) { ThreePartResolve(desc, L); return KXC_HIP_OK; }
     if (v->ks == 1) {
         int split = GroupSplit(static_cast<int64_t>(a.num_units) * SelectLanes(), a.csteps, out_elems);
         if (const char* e = std::getenv("KXC_HIP_WINOGRAD_GSPLIT")) {
@@ -738,6 +817,21 @@ int32_t WinoResolve(const kxc_hip_conv2d_desc* desc, WinoLaunch* L) {
     return KXC_HIP_OK;
 }
 
+// Above the default 64 KiB the dynamic LDS size has to be granted per kernel and device (once).
+int32_t GrantLds(const void* fn, size_t bytes) {
+    static std::mutex mu;
+    static std::vector<std::pair<int, const void*>> granted;
+    int dev = 0;
+    KXC_HIP_CALL(hipGetDevice(&dev), "hipGetDevice");
+    std::lock_guard<std::mutex> lock(mu);
+    for (const auto& g : granted)
+        if (g.first == dev && g.second == fn) return KXC_HIP_OK;
+    KXC_HIP_CALL(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes)),
+                 "hipFuncSetAttribute(MaxDynamicSharedMemorySize)");
+    granted.emplace_back(dev, fn);
+    return KXC_HIP_OK;
+}
+
 int32_t WinoRun(const WinoLaunch& L, const float* x, const float* u, const float* bias, const float* residual, float* y,
                 hipStream_t s) {
     const WinoVariant* v = L.v;
@@ -753,23 +847,24 @@ int32_t WinoRun(const WinoLaunch& L, const float* x, const float* u, const float
         a.partial = lease.ptr;
         a.counters = lease.counters;
     }
-    void (*const kernel)(const WinoArgs) = L.fuse ? v->fuse_kernel : v->kernel;
-    if (L.lds_bytes > 64 * 1024) {
-        // above the default 64 KiB the dynamic LDS size has to be granted per kernel and device (once)
-        static std::mutex mu;
-        static std::vector<std::pair<int, const void*>> granted;
-        int dev = 0;
-        KXC_HIP_CALL(hipGetDevice(&dev), "hipGetDevice");
-        const void* fn = reinterpret_cast<const void*>(kernel);
-        std::lock_guard<std::mutex> lock(mu);
-        bool have = false;
-        for (const auto& g : granted) have = have || (g.first == dev && g.second == fn);
-        if (!have) {
-            KXC_HIP_CALL(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(L.lds_bytes)),
-                         "hipFuncSetAttribute(MaxDynamicSharedMemorySize)");
-            granted.emplace_back(dev, fn);
-        }
+    if (L.three_part) {
+        wino_bx::Args b = L.bx;
+        b.x = x; b.u = reinterpret_cast<const char*>(u) + L.u_offset; b.bias = bias; b.res = residual; b.y = y; b.partial = a.partial;
+        void (*const bx)(const wino_bx::Args) = L.bx_plane == 0 ? wino_bx::wino_bf16x3_kernel<512> : wino_bx::wino_bf16x3_kernel<768>;
+        if (int32_t rc = GrantLds(reinterpret_cast<const void*>(bx), L.lds_bytes)) return rc;
+        hipLaunchKernelGGL(bx, NoteGrid(dim3(static_cast<unsigned>(b.units_per_xcd * 8))), NoteBlock(dim3(wino_bx::kThreads)),
+                           NoteLds(L.lds_bytes), s, b);
+        if (int32_t rc = CheckLaunch(v->name)) return rc;
+        if (b.gsplit == 1) return KXC_HIP_OK;
+        SplitReduceArgs r;
+        r.partial = b.partial; r.bias = bias; r.res = residual; r.y = y;
+        r.gsplit = b.gsplit; r.total = static_cast<int32_t>(L.out_elems); r.O = b.O; r.flags = b.flags;
+        r.div_ohw = MakeFastDiv(b.OHW);
+        return LaunchSplitReduce(s, r);
     }
+    void (*const kernel)(const WinoArgs) = L.fuse ? v->fuse_kernel : v->kernel;
+    if (L.lds_bytes > 64 * 1024)
+        if (int32_t rc = GrantLds(reinterpret_cast<const void*>(kernel), L.lds_bytes)) return rc;
     hipLaunchKernelGGL(kernel, NoteGrid(dim3(static_cast<unsigned>(a.units_per_xcd * 8))),
                        NoteBlock(dim3(64 * v->wk * v->wt * v->ks)), NoteLds(L.lds_bytes), s, a);
     if (int32_t rc = CheckLaunch(v->name)) return rc;
@@ -805,26 +900,41 @@ int32_t LaunchPreparedWinograd(const PreparedWinograd* p, const float* x, const 
 
 void FreePreparedWinograd(PreparedWinograd* p) { delete p; }
 
+uint32_t PreparedWinogradForms(const PreparedWinograd* p) { return p->launch.three_part ? kWinoFormThreePart : kWinoFormF32; }
+
 int32_t LaunchWinogradWeightTransforms(const WinoWeightJob* jobs, int32_t count, hipStream_t stream) {
-    for (int32_t base = 0; base < count; base += kMaxWeightJobs) {
-        WinoWeightBatch b;
-        std::memset(&b, 0, sizeof(b));
-        b.count = std::min<int32_t>(kMaxWeightJobs, count - base);
-        int64_t blocks = 0;
-        for (int32_t j = 0; j < b.count; ++j) {
-            const WinoWeightJob& job = jobs[base + j];
-            KXC_HIP_REQUIRE(job.desc && Supported(job.desc) && job.w && job.u, "winograd weight transform: bad job %d", base + j);
-            b.w[j] = job.w; b.u[j] = job.u;
-            b.O[j] = job.desc->o; b.C[j] = job.desc->c;
-            b.first_block[j] = static_cast<int32_t>(blocks);
-            blocks += WeightTiles(CeilDiv(job.desc->o, 32) * 32, job.desc->c);
-            KXC_HIP_REQUIRE(blocks < kMaxGridX, "winograd weight transform: too many blocks");
-        }
+    WinoWeightBatch b;
+    std::memset(&b, 0, sizeof(b));
+    int64_t blocks = 0;
+    auto flush = [&]() -> int32_t {
+        if (b.count == 0) return KXC_HIP_OK;
         b.first_block[b.count] = static_cast<int32_t>(blocks);
         wino_weight_batch_kernel<<<NoteGrid(static_cast<int>(blocks)), NoteBlock(256), NoteLds(0), stream>>>(b);
-        if (int32_t rc = CheckLaunch("wino_weight_batch_kernel")) return rc;
+        const int32_t rc = CheckLaunch("wino_weight_batch_kernel");
+        std::memset(&b, 0, sizeof(b));
+        blocks = 0;
+        return rc;
+    };
+    for (int32_t j = 0; j < count; ++j) {
+        const WinoWeightJob& job = jobs[j];
+        KXC_HIP_REQUIRE(job.desc && Supported(job.desc) && job.w && job.u, "winograd weight transform: bad job %d", j);
+        for (uint32_t form : {kWinoFormF32, kWinoFormThreePart}) {
+            if (!(job.forms & form)) continue;
+            if (b.count == kMaxWeightJobs)
+                if (int32_t rc = flush()) return rc;
+            const bool three = form == kWinoFormThreePart;
+            const int64_t O = job.desc->o, C = job.desc->c;
+            b.w[b.count] = job.w;
+            b.u[b.count] = reinterpret_cast<char*>(job.u) + (three ? F32FilterBytes(job.desc) : 0);
+            b.O[b.count] = static_cast<int32_t>(O); b.C[b.count] = static_cast<int32_t>(C);
+            b.first_block[b.count] = static_cast<int32_t>(blocks);
+            if (three) b.three_part |= 1u << b.count;
+            ++b.count;
+            blocks += three ? wino_bx::WeightTiles(O, C) : WeightTiles(CeilDiv(O, 32) * 32, C);
+            KXC_HIP_REQUIRE(blocks < kMaxGridX, "winograd weight transform: too many blocks");
+        }
     }
-    return KXC_HIP_OK;
+    return flush();
 }
 
 }  // namespace kxc_hip
@@ -850,18 +960,15 @@ const char* kxc_hip_conv2d_winograd_variant(const kxc_hip_conv2d_desc* desc) {
 int32_t kxc_hip_conv2d_winograd_weight_bytes(const kxc_hip_conv2d_desc* desc, size_t* out_bytes) {
     KXC_HIP_REQUIRE(desc && out_bytes, "kxc_hip_conv2d_winograd_weight_bytes: NULL argument");
     KXC_HIP_REQUIRE(Supported(desc), "kxc_hip_conv2d_winograd_weight_bytes: shape is not a 3x3 stride-1 convolution with C %% 4 == 0");
-    *out_bytes = static_cast<size_t>(CeilDiv(desc->o, 32)) * 32 * static_cast<size_t>(desc->c) * 16 * sizeof(float);
+    *out_bytes = F32FilterBytes(desc) + wino_bx::WeightBytes(desc->o, desc->c);
     return KXC_HIP_OK;
 }
 
 int32_t kxc_hip_conv2d_winograd_transform_weights(const kxc_hip_conv2d_desc* desc, const float* w, float* u, void* stream) {
     KXC_HIP_REQUIRE(desc && Supported(desc), "kxc_hip_conv2d_winograd_transform_weights: unsupported shape");
     KXC_HIP_REQUIRE(w && u, "kxc_hip_conv2d_winograd_transform_weights: NULL pointer");
-    const int64_t tiles = WeightTiles(CeilDiv(desc->o, 32) * 32, desc->c);
-    KXC_HIP_REQUIRE(tiles < kMaxGridX, "kxc_hip_conv2d_winograd_transform_weights: too many blocks");
-    wino_weight_kernel<<<NoteGrid(static_cast<int>(tiles)), NoteBlock(256), NoteLds(0), ResolveStream(stream)>>>(
-        w, u, static_cast<int32_t>(desc->o), static_cast<int32_t>(desc->c));
-    return CheckLaunch("wino_weight_kernel");
+    const WinoWeightJob job{desc, w, u, kWinoFormF32 | kWinoFormThreePart};
+    return LaunchWinogradWeightTransforms(&job, 1, ResolveStream(stream));
 }
 
 int32_t kxc_hip_conv2d_winograd_nchw_f32(const kxc_hip_conv2d_desc* desc, const float* x, const float* u, const float* bias,

@@ -866,8 +866,10 @@ int32_t TransformConstants(kxc_hip_plan* plan, void** args, hipStream_t stream, 
         // (nodes of different chains that share a transformed-weight buffer: one transform)
         float* const u = static_cast<float*>(Resolve(plan, n.bufs[5], args));
         bool have = false;
-        for (const WinoWeightJob& j : jobs) have = have || (j.u == u && j.w == w);
-        if (!have) jobs.push_back({&n.conv, static_cast<const float*>(w), u});
+        const uint32_t forms = kxc_hip::PreparedWinogradForms(n.prepared_wino.get());
+        for (WinoWeightJob& j : jobs)
+            if (j.u == u && j.w == w) { have = true; j.forms |= forms; }
+        if (!have) jobs.push_back({&n.conv, static_cast<const float*>(w), u, forms});
     }
     std::vector<QPackJob> packs;
     std::vector<std::pair<PackJob*, const void*>> packed;
