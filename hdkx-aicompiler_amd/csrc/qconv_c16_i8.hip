@@ -1247,6 +1247,171 @@ __global__ void __launch_bounds__(kBlock) gap_c16_kernel(const int8_t* __restric
     reinterpret_cast<uint32_t*>(y)[t] = o;
 }
 
+// ------------------------------------------------------------------------------------------------
+// The same convolution without LDS staging, the reduction split over the waves of a workgroup.
+// A workgroup owns ONE tile of 32*RO output channels x 32*RP pixels; wave w of KS takes the chunks w, w + KS, ... and
+// reads both operands straight into registers: a weight fragment is one contiguous KiB, a pixel fragment is the 16-byte
+// c16 word of each lane's own pixel and tap (one buffer offset per tap and lane, computed once; out of range at the
+// zero padding).  All loads of a chunk are in flight together, so a wave pays about one memory round trip per chunk and
+// no barrier; the KS partial tiles meet in LDS at the end (integers: the order of the sum does not matter).
+// Every wave loads its own operands, so the vector cache bounds it once there are many tiles; with few, its chain is the
+// shortest: 512 -> 512 channels at 7 x 7, batch 5: 23.1 -> 4.8 us.  SelectDirect has the line between the two.
+template <int KH, int RO, int RP, int KS, bool DS = false>
+__global__ void __launch_bounds__(64 * KS) __attribute__((amdgpu_waves_per_eu(KS >= 16 ? 4 : 2))) qconv_direct_kernel(const QArgs a) {
+    constexpr int KHW = KH * KH, CBC = KH == 1 ? 4 : 2, NS = KHW * CBC / 2;
+    constexpr int G = KH == 1 ? 3 : 1;               // chunks per loop trip
+    constexpr int NB = RO * RP, NBA = DS ? 2 * NB : NB;
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    const int lane = threadIdx.x & 63, half = lane >> 5, r = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+    const int tile = (blockIdx.x & 7) * a.tiles_per_xcd + (blockIdx.x >> 3);
+    if (tile >= a.num_tiles || static_cast<int>(blockIdx.x >> 3) >= a.tiles_per_xcd) return;
+    const int o_tile = fast_div(tile, a.div_otiles), p_tile = tile - o_tile * a.p_tiles;
+    const int m0 = p_tile * 32 * RP, ob0 = o_tile * RO;
+
+    const __amdgpu_buffer_rsrc_t xr = make_rsrc(a.x, a.x_bytes);
+    const __amdgpu_buffer_rsrc_t wr = make_rsrc(a.wp, a.w_bytes);
+    const __amdgpu_buffer_rsrc_t wr2 = make_rsrc(DS ? a.wp2 : a.wp, DS ? a.w2_bytes : 0u);
+    const uint32_t plane = static_cast<uint32_t>(a.H * a.W) * 16u;
+    uint32_t xoff[RP][KHW];
+    int ypix[RP];
+#pragma unroll
+    for (int j = 0; j < RP; ++j) {
+        const int m = m0 + j * 32 + r;
+        const int n = fast_div(m, a.div_ohw), rem = m - n * a.OHW;
+        const int oh = fast_div(rem, a.div_ow), ow = rem - oh * a.OW;
+        const bool in = m < a.M;
+        ypix[j] = in ? n * (a.O >> 4) * a.OHW + rem : -1;
+        const int ih = oh * a.sh - a.ph, iw = ow * a.sw - a.pw;
+        const uint32_t base = static_cast<uint32_t>(n) * a.CB * plane + static_cast<uint32_t>(half) * plane;
+#pragma unroll
+        for (int t = 0; t < KHW; ++t) {
+            const int y = ih + t / KH, x = iw + t % KH;
+            const bool ok = in && static_cast<uint32_t>(y) < static_cast<uint32_t>(a.H) && static_cast<uint32_t>(x) < static_cast<uint32_t>(a.W);
+            xoff[j][t] = ok ? base + static_cast<uint32_t>(y * a.W + x) * 16u : kOob;
+        }
+    }
+    uint32_t woff[RO], woff2[RO];
+#pragma unroll
+    for (int i = 0; i < RO; ++i) {
+        woff[i] = static_cast<uint32_t>((ob0 + i) * a.nchunks) * (NS * 1024u) + static_cast<uint32_t>(lane) * 16u;
+        woff2[i] = static_cast<uint32_t>((ob0 + i) * a.nchunks) * 1024u + static_cast<uint32_t>(lane) * 16u;
+    }
+    intx16 acc[RP][RO], acc2[DS ? RP : 1][DS ? RO : 1];
+#pragma unroll
+    for (int j = 0; j < RP; ++j)
+#pragma unroll
+        for (int i = 0; i < RO; ++i)
+#pragma unroll
+            for (int g = 0; g < 16; ++g) {
+                acc[j][i][g] = 0;
+                if constexpr (DS) acc2[j][i][g] = 0;
+            }
+
+    intx4 wf[G * NS][RO], xf[G * NS][RP], wf2[DS ? RO : 1];
+    // step s of a trip: the lane half's channel block is masked where the last chunk is not whole (its weights are zero,
+    // but the word may lie behind the tensor)
+    auto load = [&](int chunk0, int s) __attribute__((always_inline)) {
+        const int chunk = chunk0 + (s / NS) * KS;
+        const int cb = chunk * CBC + (KH == 1 ? 2 * (s % NS) : 0);
+        const uint32_t mask = cb + half < a.CB ? 0u : kOob;
+        const uint32_t wmask = G > 1 && chunk >= a.nchunks ? kOob : 0u;
+        const uint32_t wt = static_cast<uint32_t>(chunk * NS + s % NS) * 1024u;
+#pragma unroll
+        for (int i = 0; i < RO; ++i) wf[s][i] = __builtin_amdgcn_raw_buffer_load_b128(wr, woff[i] | wmask, wt, 0);
+#pragma unroll
+        for (int j = 0; j < RP; ++j)
+            xf[s][j] = __builtin_amdgcn_raw_buffer_load_b128(xr, xoff[j][KH == 1 ? 0 : s] | mask, static_cast<uint32_t>(cb) * plane, 0);
+        if constexpr (DS) {
+            if (s == 0) {
+#pragma unroll
+                for (int i = 0; i < RO; ++i) wf2[i] = __builtin_amdgcn_raw_buffer_load_b128(wr2, woff2[i], static_cast<uint32_t>(chunk) * 1024u, 0);
+            }
+        }
+    };
+    auto trip = [&](auto more_c, int chunk) __attribute__((always_inline)) {
+        constexpr bool kMore = decltype(more_c)::value;
+        intx4 w2[DS ? RO : 1];
+        if constexpr (DS) {
+#pragma unroll
+            for (int i = 0; i < RO; ++i) w2[i] = wf2[i];
+        }
+#pragma unroll
+        for (int s = 0; s < G * NS; ++s) {
+#pragma unroll
+            for (int j = 0; j < RP; ++j)
+#pragma unroll
+                for (int i = 0; i < RO; ++i) {
+                    acc[j][i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wf[s][i], xf[s][j], acc[j][i], 0, 0, 0);
+                    if constexpr (DS) {
+                        if (s == KHW / 2) acc2[j][i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w2[i], xf[s][j], acc2[j][i], 0, 0, 0);
+                    }
+                }
+            if constexpr (kMore) load(chunk + G * KS, s);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    int chunk = wave;
+    if (chunk < a.nchunks) {
+#pragma unroll
+        for (int s = 0; s < G * NS; ++s) load(chunk, s);
+        __builtin_amdgcn_sched_barrier(0);
+        for (; chunk + G * KS < a.nchunks; chunk += G * KS) trip(std::true_type{}, chunk);
+        trip(std::false_type{}, chunk);
+    }
+
+    // block b's partial sums of wave w: [w][b][register quad][lane][16 bytes]
+    auto at = [&](int w, int b, int g) { return reinterpret_cast<intx4*>(lds + (((w * NBA + b) * 4 + g) * 64 + lane) * 16); };
+    auto quad = [](const intx16& v, int g) { return intx4{v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]}; };
+#pragma unroll
+    for (int b = 0; b < NBA; ++b) {
+        if (b % KS == wave) continue;                // (its own block stays in registers)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            if constexpr (DS) *at(wave, b, g) = quad(b < NB ? acc[b / RO][b % RO] : acc2[(b % NB) / RO][b % RO], g);
+            else *at(wave, b, g) = quad(acc[b / RO][b % RO], g);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < NBA; ++b) {
+        if (b % KS != wave) continue;
+        const int i = b % RO, j = (b % NB) / RO;
+        const bool second = b >= NB;
+        intx16 sum[1][1];
+        if constexpr (DS) {
+            if (second) init_acc_with_bias<1>(sum[0], a.bias2, a.bias2 != nullptr, a.O, ob0 + i, half);
+            else init_acc_with_bias<1>(sum[0], a.bias, (a.flags & KXC_HIP_CONV_BIAS) != 0, a.O, ob0 + i, half);
+        } else {
+            init_acc_with_bias<1>(sum[0], a.bias, (a.flags & KXC_HIP_CONV_BIAS) != 0, a.O, ob0 + i, half);
+        }
+        const intx16 own = [&] {
+            if constexpr (DS) return second ? acc2[j][i] : acc[j][i];
+            else return acc[j][i];
+        }();
+#pragma unroll
+        for (int g = 0; g < 16; ++g) sum[0][0][g] += own[g];
+#pragma unroll 2
+        for (int w = 0; w < KS; ++w) {
+            if (w == wave) continue;
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const intx4 q = *at(w, b, g);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sum[0][0][4 * g + e] += q[e];
+            }
+        }
+        const int yp[1] = {ypix[j]};
+        if (DS && second) {
+            QArgs other = a;
+            other.mult = a.mult2; other.res = nullptr; other.y = a.y2; other.flags = 0u;
+            epilogue_c16<1, 1>(sum, other, yp, ob0 + i, half);
+        } else {
+            epilogue_c16<1, 1>(sum, a, yp, ob0 + i, half);
+        }
+    }
+}
+
 // ------------------------------------------------------------------ host side
 struct QVariant {
     const char* name;
@@ -1315,6 +1480,19 @@ const QRowVariant kQRowVariants[] = {
     KXC_QR(3, 3, 2, 4, 2, 4, 4, 64),
 };
 
+// qconv_direct_kernel by (window, tile, waves per workgroup)
+struct QDirectVariant {
+    const char* name;
+    int k, ro, rp, ks;
+    void (*kernel)(const QArgs);
+    void (*ds_kernel)(const QArgs);
+};
+#define KXC_QD(K, RO, RP, KS) {"qmfma_k" #K "x" #K "_direct_o" #RO "_p" #RP "_ks" #KS, K, RO, RP, KS, qconv_direct_kernel<K, RO, RP, KS>, nullptr}
+#define KXC_QD_DS(K, RO, RP, KS) {"qmfma_k" #K "x" #K "_direct_o" #RO "_p" #RP "_ks" #KS, K, RO, RP, KS, qconv_direct_kernel<K, RO, RP, KS>, qconv_direct_kernel<K, RO, RP, KS, true>}
+const QDirectVariant kQDirect[] = {
+    KXC_QD_DS(3, 1, 1, 2), KXC_QD_DS(3, 2, 1, 2), KXC_QD(3, 2, 2, 4), KXC_QD(1, 1, 1, 2), KXC_QD(1, 2, 1, 4),
+};
+
 // Channel blocks (of 16 channels) per LDS chunk.  Larger chunks (64 or 128 channels) were measured on the ResNet-18
 // layers at batch 64 and were slower everywhere (512 -> 512 channels at 7 x 7: 14.3 -> 15-20 us; 256 -> 512 with
 // stride 2: 11 -> 23 us): with few chunks the first, large patch load is exposed and nothing overlaps it.
@@ -1326,10 +1504,10 @@ int CbcFor(int c, int kh, int kw) {
 }
 
 struct QLaunch {
-    const QVariant* v = nullptr;
+    int cbc = 0;                        // channel blocks per chunk of the chosen kernel; 0: nothing to launch
     QArgs args;
     int grid = 0;
-    size_t lds_bytes = 0;
+    size_t lds_bytes = 0, ds_lds_extra = 0;      // (the second: what the second output's kernel takes on top)
     // what is launched: the variant's kernels, or those of the row-pitch variant that replaced it
     const char* name = "";
     void (*kernel)(const QArgs) = nullptr;
@@ -1351,29 +1529,72 @@ int MaxRows(const QArgs& a, int KH, int TP) {
     return best;
 }
 
-int32_t PrepareUncached(const kxc_hip_qconv2d_desc* d, QLaunch* L, const char* who);
+int32_t PrepareUncached(const kxc_hip_qconv2d_desc* d, QLaunch* L, const char* who, bool pair);
+
+// The kernel without staging wins while the launch has few 32 x 32 blocks: the staged kernels then leave compute units
+// idle and pay a chain of (chunks) x (memory round trip + barrier).  Measured over the ResNet-18 layers at batches 1 to 64,
+// operands rotating through memory:
+//   up to 512 blocks, one block per workgroup: 512 -> 512 channels at 7 x 7, batch 5: 23.1 -> 4.8 us; 256 at 14 x 14,
+//     batch 1: 8.8 -> 3.8; 128 -> 256 with stride 2 and the second output, batch 5: 8.3 -> 4.1;
+//   up to 1600, two output-channel blocks (a pixel operand then feeds two matrix instructions): 256 at 14 x 14, batch 16:
+//     13.3 -> 6.9; 256 -> 512 with stride 2, batch 64: 17.5 -> 14.1.  Beyond, every wave's own loads bound it (256 at
+//     14 x 14, batch 64: 14.6 against 12.7);
+//   with 16 chunks and more (512 channels), 64 x 64 tiles over four waves: 7 x 7, batch 32: 22.7 -> 9.5; batch 64: 16.7 -> 14.7.
+// 1x1 filters: up to 1600 blocks (batch 16, 512 -> 128 at 14 x 14: 7.3 -> 4.3), with fewer than 256 channels up to 1024
+// (128 -> 512 at 28 x 28, 800 blocks: 4.6 -> 3.5; 2000 blocks: 4.6 -> 5.2).
+// Rows that fit the 64-position pitch stay with qconv_rows_kernel: at 64 channels the reduction is too short to split.
+// Eight and sixteen waves per tile were slower everywhere (512 at 7 x 7, batch 5: 5.4 and 6.2 us).
+const QDirectVariant* SelectDirect(const QArgs& a, const kxc_hip_qconv2d_desc* d, int cbc, bool pair) {
+    const int k = d->kh;
+    // (the second output reads the middle tap: padding 1; more than 16 channels, so that a chunk is whole words)
+    if (k != d->kw || (k != 1 && k != 3) || cbc != (k == 1 ? 4 : 2) || (k == 3 && (d->pad_h != 1 || d->pad_w != 1))) return nullptr;
+    const int ob = a.O / 32;
+    const int64_t blocks = CeilDiv(a.M, 32) * ob;
+    int ro = 1, rp = 1, ks = 2;
+    const char* forced = std::getenv("KXC_HIP_QCONV_VARIANT");
+    if (!(forced && *forced)) {
+        const bool pair_ok = ob % 2 == 0;
+        if (k == 3) {
+            if (blocks > 1600 || (d->stride_h == 1 && d->stride_w == 1 && a.Wp > 32 && a.Wp <= 64)) return nullptr;
+            if (blocks > 512 && pair_ok) {
+                ro = 2;
+                if (a.nchunks >= 16 && !pair) { rp = 2; ks = 4; }
+            }
+        } else {
+            if (blocks > (a.nchunks >= 4 ? 1600 : 1024)) return nullptr;
+            if (blocks > 512 && a.nchunks >= 4 && pair_ok) { ro = 2; ks = 4; }
+        }
+    }
+    for (const QDirectVariant& v : kQDirect) {
+        if (v.k != k || ob % v.ro != 0) continue;
+        if (forced && *forced ? std::strcmp(forced, v.name) == 0 : v.ro == ro && v.rp == rp && v.ks == ks) return &v;
+    }
+    return nullptr;
+}
 
 // The selection walks every pixel tile once; a forward pass repeats the same few descriptors, so the last
 // results are kept per thread (pointers are filled in by the caller afterwards).
-int32_t Prepare(const kxc_hip_qconv2d_desc* d, QLaunch* L, const char* who) {
+// pair: for a launch with the second output.
+int32_t Prepare(const kxc_hip_qconv2d_desc* d, QLaunch* L, const char* who, bool pair = false) {
     KXC_HIP_REQUIRE(d != nullptr, "%s: desc is NULL", who);
-    struct Entry { kxc_hip_qconv2d_desc desc; QLaunch launch; };
+    struct Entry { kxc_hip_qconv2d_desc desc; bool pair; QLaunch launch; };
     thread_local std::vector<Entry> cache;
     if (const char* f = std::getenv("KXC_HIP_QCONV_VARIANT"))
-        if (*f) return PrepareUncached(d, L, who);          // forced variants are not cached
-    if (std::getenv("KXC_HIP_QCONV_ROWS") || std::getenv("KXC_HIP_QCONV_BIG_TILE")) return PrepareUncached(d, L, who);
+        if (*f) return PrepareUncached(d, L, who, pair);          // forced variants are not cached
+    if (std::getenv("KXC_HIP_QCONV_ROWS") || std::getenv("KXC_HIP_QCONV_BIG_TILE")) return PrepareUncached(d, L, who, pair);
     for (const Entry& e : cache)
-        if (std::memcmp(&e.desc, d, sizeof(*d)) == 0) { *L = e.launch; return KXC_HIP_OK; }
-    if (int32_t rc = PrepareUncached(d, L, who)) return rc;
+        if (e.pair == pair && std::memcmp(&e.desc, d, sizeof(*d)) == 0) { *L = e.launch; return KXC_HIP_OK; }
+    if (int32_t rc = PrepareUncached(d, L, who, pair)) return rc;
     if (cache.size() >= 128) cache.clear();
     Entry e;
     std::memcpy(&e.desc, d, sizeof(*d));
+    e.pair = pair;
     e.launch = *L;
     cache.push_back(e);
     return KXC_HIP_OK;
 }
 
-int32_t PrepareUncached(const kxc_hip_qconv2d_desc* d, QLaunch* L, const char* who) {
+int32_t PrepareUncached(const kxc_hip_qconv2d_desc* d, QLaunch* L, const char* who, bool pair) {
     KXC_HIP_REQUIRE(d->n >= 0 && d->c > 0 && d->h > 0 && d->w > 0 && d->o > 0 && d->kh > 0 && d->kw > 0,
                     "%s: bad shape", who);
     KXC_HIP_REQUIRE(d->stride_h > 0 && d->stride_w > 0 && d->pad_h >= 0 && d->pad_w >= 0, "%s: bad stride or padding", who);
@@ -1403,6 +1624,20 @@ int32_t PrepareUncached(const kxc_hip_qconv2d_desc* d, QLaunch* L, const char* w
     const int cbc = CbcFor(d->c, d->kh, d->kw);
     a.nchunks = (a.CB + cbc - 1) / cbc;
     if (M == 0) return KXC_HIP_OK;
+    if (const QDirectVariant* dv = SelectDirect(a, d, cbc, pair)) {
+        a.p_tiles = static_cast<int32_t>(CeilDiv(M, 32 * dv->rp));
+        a.o_tiles = a.O / 32 / dv->ro;
+        a.num_tiles = a.p_tiles * a.o_tiles;
+        a.tiles_per_xcd = (a.num_tiles + 7) / 8;
+        a.div_ohw = MakeFastDiv(a.OHW); a.div_ow = MakeFastDiv(a.OW);
+        a.div_otiles = MakeFastDiv(a.p_tiles);
+        a.w_bytes = static_cast<uint32_t>(static_cast<int64_t>(a.O / 32) * a.nchunks * (d->kh * d->kw * cbc / 2) * 1024);
+        L->grid = a.tiles_per_xcd * 8;
+        L->cbc = cbc;
+        L->name = dv->name; L->kernel = dv->kernel; L->ds_kernel = dv->ds_kernel; L->threads = 64 * dv->ks;
+        L->lds_bytes = L->ds_lds_extra = static_cast<size_t>(dv->ks) * dv->ro * dv->rp * 4096;
+        return KXC_HIP_OK;
+    }
     // pick the first variant that fits, preferring enough workgroups to fill 256 CUs a few times over
     const QVariant* best = nullptr;
     int best_chs = 0;
@@ -1463,7 +1698,7 @@ int32_t PrepareUncached(const kxc_hip_qconv2d_desc* d, QLaunch* L, const char* w
     a.div_wp = MakeFastDiv(a.Wp); a.div_hp = MakeFastDiv(a.Hp); a.div_ohw = MakeFastDiv(a.OHW);
     a.div_ow = MakeFastDiv(a.OW); a.div_otiles = MakeFastDiv(a.o_tiles);
     L->grid = a.tiles_per_xcd * 8;
-    L->v = best;
+    L->cbc = cbc;
     L->name = best->name; L->kernel = best->kernel; L->ds_kernel = best->ds_kernel; L->threads = 64 * best->wp;
     const int NS = (best->kh * best->kw * cbc + 1) / 2;
     a.w_bytes = static_cast<uint32_t>(static_cast<int64_t>(a.O / 32) * a.nchunks * NS * 1024);
@@ -1526,7 +1761,7 @@ int32_t kxc_hip_qconv2d_c16_pack_weights(const kxc_hip_qconv2d_desc* d, const in
 const char* kxc_hip_qconv2d_c16_variant(const kxc_hip_qconv2d_desc* d) {
     QLaunch L;
     if (Prepare(d, &L, "kxc_hip_qconv2d_c16_variant") != KXC_HIP_OK) return "none";
-    return L.v ? L.name : "empty";
+    return L.cbc ? L.name : "empty";
 }
 
 int32_t kxc_hip_qconv2d_c16_i8(const kxc_hip_qconv2d_desc* d, const int8_t* x, const int8_t* w_packed,
@@ -1562,8 +1797,8 @@ static bool PairGeometry(const kxc_hip_qconv2d_desc* d) {
 int32_t kxc_hip_qconv2d_c16_pair_supported(const kxc_hip_qconv2d_desc* d) {
     QLaunch L;
     if (!PairGeometry(d)) return 0;
-    if (Prepare(d, &L, "kxc_hip_qconv2d_c16_pair_supported") != KXC_HIP_OK) { LastError().clear(); return 0; }
-    return (L.v && L.ds_kernel) ? 1 : 0;
+    if (Prepare(d, &L, "kxc_hip_qconv2d_c16_pair_supported", true) != KXC_HIP_OK) { LastError().clear(); return 0; }
+    return L.cbc && L.ds_kernel ? 1 : 0;
 }
 
 int32_t kxc_hip_qconv2d_c16_pair_packed_bytes(const kxc_hip_qconv2d_desc* d, size_t* out_bytes) {
@@ -1597,8 +1832,8 @@ int32_t kxc_hip_qconv2d_c16_pair_i8(const kxc_hip_qconv2d_desc* d, const int8_t*
                                     const int32_t* bias2, const float* mult2, int8_t* y2, void* stream) {
     const char* who = "kxc_hip_qconv2d_c16_pair_i8";
     QLaunch L;
-    if (int32_t rc = Prepare(d, &L, who)) return rc;
-    KXC_HIP_REQUIRE(L.v && L.ds_kernel && PairGeometry(d), "%s: no kernel with a second output covers this shape", who);
+    if (int32_t rc = Prepare(d, &L, who, true)) return rc;
+    KXC_HIP_REQUIRE(L.cbc && L.ds_kernel && PairGeometry(d), "%s: no kernel with a second output covers this shape", who);
     if (L.args.M == 0) return KXC_HIP_OK;
     KXC_HIP_REQUIRE(x && w_packed && mult && y && w2_packed && mult2 && y2, "%s: NULL pointer", who);
     KXC_HIP_REQUIRE(!(d->flags & KXC_HIP_CONV_BIAS) || bias, "%s: bias flag without bias", who);
@@ -1606,11 +1841,12 @@ int32_t kxc_hip_qconv2d_c16_pair_i8(const kxc_hip_qconv2d_desc* d, const int8_t*
     QArgs& a = L.args;
     a.x = x; a.wp = w_packed; a.bias = bias; a.mult = mult; a.res = residual; a.y = y;
     a.wp2 = w2_packed; a.bias2 = bias2; a.mult2 = mult2; a.y2 = y2;
-    a.w2_bytes = static_cast<uint32_t>(static_cast<int64_t>(a.O / 32) * a.nchunks * ((L.v->cbc + 1) / 2) * 1024);
+    a.w2_bytes = static_cast<uint32_t>(static_cast<int64_t>(a.O / 32) * a.nchunks * ((L.cbc + 1) / 2) * 1024);
     // the second output's tap in the staged patch: rows are Wp positions apart, or the row pitch of a qrows variant
     int row_positions = a.Wp;
     if (std::strncmp(L.name, "qrows", 5) == 0) row_positions = 64;
     a.ds_off = (d->pad_h * row_positions + d->pad_w) * 16;
+    L.lds_bytes += L.ds_lds_extra;
     if (L.lds_bytes > 64 * 1024) {
         KXC_HIP_CALL(hipFuncSetAttribute(reinterpret_cast<const void*>(L.ds_kernel),
                                          hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(L.lds_bytes)),

@@ -165,6 +165,36 @@ def test_qconv_c16_largest_wave_tile_against_cpu(pkg, orc, monkeypatch):
     assert "p4x2_o1" in variant(32) and "p4x2_o1" in variant(96) and "p2x2_o1" in variant(31)
 
 
+@pytest.mark.parametrize("shape", [
+    # n, c, h, w, o, k, stride, tile: one pixel; partial channel blocks and an odd block count; tiles across images; more
+    # chunks than waves and fewer; the line between one and two output-channel blocks; the last tile of one pixel
+    (1, 17, 1, 1, 32, 3, 1, "o1_p1_ks2"), (3, 80, 13, 9, 96, 3, 2, "o1_p1_ks2"), (5, 512, 7, 7, 512, 3, 1, "o1_p1_ks2"),
+    (1, 32, 32, 512, 32, 3, 1, "o1_p1_ks2"), (1, 48, 27, 19, 1088, 3, 1, "o2_p1_ks2"), (21, 512, 7, 7, 512, 3, 1, "o2_p2_ks4"),
+    (1, 65, 1, 1, 32, 1, 1, "o1_p1_ks2"), (3, 250, 11, 13, 64, 1, 2, "o1_p1_ks2"), (2, 496, 31, 34, 256, 1, 1, "o2_p1_ks4"),
+], ids=lambda s: "x".join(map(str, s)))
+def test_qconv_c16_direct_kernel(pkg, orc, monkeypatch, shape):
+    """The kernel of small launches, at the edges of its tiles and of the rule that chooses its tile: the same bytes as the
+    CPU operator, or where that would take long as the staged kernel."""
+    n, c, h, w, o, k, s, tile = shape
+    rng = np.random.default_rng(hash(shape) % (2 ** 31))
+    x = rng.integers(-128, 128, (n, c, h, w), dtype=np.int8)
+    wq = rng.integers(-127, 128, (o, c, k, k), dtype=np.int8)
+    bias = rng.integers(-20000, 20000, (o,), dtype=np.int32)
+    mult = rng.uniform(0.5, 2.0, (o,)).astype(np.float32) * np.float32(1.0 / (8.0 * np.sqrt(c * k * k) * 64))
+    oh, ow = (h + 2 * (k // 2) - k) // s + 1, (w + 2 * (k // 2) - k) // s + 1
+    res = rng.integers(-128, 128, (n, o, oh, ow), dtype=np.int8)
+    d = pkg.qconv_desc(n, c, h, w, o, k, k, s, k // 2)
+    assert pkg.qconv2d_c16_variant(d) == "qmfma_k%dx%d_direct_%s" % (k, k, tile)
+    args = (to_c16(pkg, x), c, pkg.qconv2d_c16_pack_weights(dev(wq)), wq.shape, dev(bias), dev(mult), to_c16(pkg, res), 0.37, s, k // 2, True)
+    got = pkg.qconv2d_c16(*args)
+    if 2 * n * o * oh * ow * c * k * k < 10 ** 9:
+        assert_bit_exact(from_c16(pkg, got, o), orc.qconv(x, wq, bias, mult, s, k // 2, res, 0.37, True), "direct %s" % (shape,))
+    else:
+        monkeypatch.setenv("KXC_HIP_QCONV_VARIANT", "qmfma_k%dx%d_cb%d_p4_o2" % (k, k, 2 if k == 3 else 4))
+        assert "direct" not in pkg.qconv2d_c16_variant(d)
+        assert torch.equal(got, pkg.qconv2d_c16(*args))
+
+
 QPAIR_SHAPES = [
     # n, c, h, w, o, stride: the three ResNet-18 blocks, a ragged shape with a partial channel block and an odd block count
     (2, 64, 56, 56, 128, 2), (64, 64, 56, 56, 128, 2), (3, 128, 28, 28, 256, 2), (5, 256, 14, 14, 512, 2),
