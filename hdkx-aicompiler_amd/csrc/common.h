@@ -101,6 +101,10 @@ struct SplitScratchLease {
 int32_t AcquireSplitScratch(hipStream_t stream, size_t bytes, SplitScratchLease* lease);
 int32_t LaunchSplitReduce(hipStream_t stream, const SplitReduceArgs& a);
 
+constexpr size_t kMaxLdsBytes = 160 * 1024;  // LDS of one gfx950 compute unit
+// Above the default 64 KiB the dynamic LDS size has to be granted per kernel and device (once; device_api.hip).
+int32_t GrantLds(const void* kernel);
+
 // A split reduction without the adding kernel: every part stores its raw partial outputs as before, then counts
 // itself in at its tile's arrival counter; the part that arrives last adds all parts in split order (the same
 // order, hence the same bits, as the adding kernel) and applies the epilogue.  The counters sit in front of the

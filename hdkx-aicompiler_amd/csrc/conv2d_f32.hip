@@ -874,7 +874,6 @@ int32_t MaxTileRows(const ConvArgs& a, int kh, int tp) {
     return best;
 }
 
-constexpr size_t kMaxLdsBytes = 160 * 1024;  // LDS of one gfx950 compute unit
 constexpr int kNumCUs = 256;
 
 bool Fits(const Variant& v, const ConvArgs& a, Choice* out, bool ds = false) {
@@ -1392,21 +1391,6 @@ int32_t Conv2dResolve(const kxc_hip_conv2d_desc* desc, bool second, const char* 
     L->grid = dim3(static_cast<unsigned>(a.tiles_per_xcd * 8));
     L->block = dim3(64 * c.v->nw * c.v->ks);
     L->lds_bytes = c.lds_bytes;
-    return KXC_HIP_OK;
-}
-
-// Above the default 64 KiB the dynamic LDS size has to be granted per kernel and device (once).
-int32_t GrantLds(const void* fn) {
-    static std::mutex mu;
-    static std::vector<std::pair<int, const void*>> granted;
-    int dev = 0;
-    KXC_HIP_CALL(hipGetDevice(&dev), "hipGetDevice");
-    std::lock_guard<std::mutex> lock(mu);
-    for (const auto& g : granted)
-        if (g.first == dev && g.second == fn) return KXC_HIP_OK;
-    KXC_HIP_CALL(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kMaxLdsBytes)),
-                 "hipFuncSetAttribute(MaxDynamicSharedMemorySize)");
-    granted.emplace_back(dev, fn);
     return KXC_HIP_OK;
 }
 

@@ -817,21 +817,6 @@ int32_t WinoResolve(const kxc_hip_conv2d_desc* desc, WinoLaunch* L) {
     return KXC_HIP_OK;
 }
 
-// Above the default 64 KiB the dynamic LDS size has to be granted per kernel and device (once).
-int32_t GrantLds(const void* fn, size_t bytes) {
-    static std::mutex mu;
-    static std::vector<std::pair<int, const void*>> granted;
-    int dev = 0;
-    KXC_HIP_CALL(hipGetDevice(&dev), "hipGetDevice");
-    std::lock_guard<std::mutex> lock(mu);
-    for (const auto& g : granted)
-        if (g.first == dev && g.second == fn) return KXC_HIP_OK;
-    KXC_HIP_CALL(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes)),
-                 "hipFuncSetAttribute(MaxDynamicSharedMemorySize)");
-    granted.emplace_back(dev, fn);
-    return KXC_HIP_OK;
-}
-
 int32_t WinoRun(const WinoLaunch& L, const float* x, const float* u, const float* bias, const float* residual, float* y,
                 hipStream_t s) {
     const WinoVariant* v = L.v;
@@ -851,7 +836,7 @@ int32_t WinoRun(const WinoLaunch& L, const float* x, const float* u, const float
         wino_bx::Args b = L.bx;
         b.x = x; b.u = reinterpret_cast<const char*>(u) + L.u_offset; b.bias = bias; b.res = residual; b.y = y; b.partial = a.partial;
         void (*const bx)(const wino_bx::Args) = L.bx_plane == 0 ? wino_bx::wino_bf16x3_kernel<512> : wino_bx::wino_bf16x3_kernel<768>;
-        if (int32_t rc = GrantLds(reinterpret_cast<const void*>(bx), L.lds_bytes)) return rc;
+        if (int32_t rc = GrantLds(reinterpret_cast<const void*>(bx))) return rc;
         hipLaunchKernelGGL(bx, NoteGrid(dim3(static_cast<unsigned>(b.units_per_xcd * 8))), NoteBlock(dim3(wino_bx::kThreads)),
                            NoteLds(L.lds_bytes), s, b);
         if (int32_t rc = CheckLaunch(v->name)) return rc;
@@ -864,7 +849,7 @@ int32_t WinoRun(const WinoLaunch& L, const float* x, const float* u, const float
     }
     void (*const kernel)(const WinoArgs) = L.fuse ? v->fuse_kernel : v->kernel;
     if (L.lds_bytes > 64 * 1024)
-        if (int32_t rc = GrantLds(reinterpret_cast<const void*>(kernel), L.lds_bytes)) return rc;
+        if (int32_t rc = GrantLds(reinterpret_cast<const void*>(kernel))) return rc;
     hipLaunchKernelGGL(kernel, NoteGrid(dim3(static_cast<unsigned>(a.units_per_xcd * 8))),
                        NoteBlock(dim3(64 * v->wk * v->wt * v->ks)), NoteLds(L.lds_bytes), s, a);
     if (int32_t rc = CheckLaunch(v->name)) return rc;

@@ -5,6 +5,9 @@
 #include <cstring>
 
 #include <atomic>
+#include <mutex>
+#include <utility>
+#include <vector>
 
 #include "common.h"
 
@@ -20,6 +23,19 @@ LaunchNote& LastLaunch() {
 hipStream_t& CurrentStream() {
     static thread_local hipStream_t s = nullptr;
     return s;
+}
+int32_t GrantLds(const void* kernel) {
+    static std::mutex mu;
+    static std::vector<std::pair<int, const void*>> granted;
+    int dev = 0;
+    KXC_HIP_CALL(hipGetDevice(&dev), "hipGetDevice");
+    std::lock_guard<std::mutex> lock(mu);
+    for (const auto& g : granted)
+        if (g.first == dev && g.second == kernel) return KXC_HIP_OK;
+    KXC_HIP_CALL(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kMaxLdsBytes)),
+                 "hipFuncSetAttribute(MaxDynamicSharedMemorySize)");
+    granted.emplace_back(dev, kernel);
+    return KXC_HIP_OK;
 }
 }  // namespace kxc_hip
 

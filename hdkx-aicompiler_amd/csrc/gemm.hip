@@ -1,25 +1,15 @@
-// gemm.hip -- nn_dense / nn_gemm on the fp32 matrix cores.
+// gemm.hip -- nn_dense / nn_gemm on the matrix cores.
 //
-//   y[m,n] = alpha * sum_k a[m,k] * b[n,k]  (+ beta * c[n])          (transB = 1, the ResNet FC layer)
+//   y[m,n] = alpha * sum_k a[m,k] * b[n,k]  (+ beta * c[n])          (transB = 1, the ResNet FC layer; transB = 0: b[k,n])
 //
-// MFMA kernel (v_mfma_f32_32x32x2_f32): one workgroup of four waves owns a 32x32 output tile; the
-// waves split K four ways and, inside a wave, the two half-waves take the lower and upper half of
-// the wave's K range, so every lane walks ONE contiguous run of its own row of `a` and of `b`
-// with 16-byte loads straight into the MFMA operand registers (no LDS staging, no shuffles: the
-// matrix instruction only needs the two half-waves to hold different k, not adjacent k).  The four
-// partial tiles are combined through LDS in a fixed order, so results are deterministic.
-// The FC layer of ResNet-18 (64x512 by 1000x512) is launch-latency/weight-read bound: 64 tiles of
-// four waves each keep 64 CUs busy for a few microseconds.
-//
-// Everything else (transB = 0, K not a multiple of 32, unaligned rows) goes to a one-thread-per-
-// output kernel that adds in the CPU loop's exact order (k ascending, separate multiply and add).
+// Up to four rows go to gemv_nt_kernel, everything else to gemm_bf16x3_kernel (three-part fp32 operands, bf16x3.h); tiny
+// products that no vector load fits keep a one-thread-per-output kernel in the CPU loop's exact order.
+#include "bf16x3.h"
 #include "common.h"
 
 using namespace kxc_hip;
 
 namespace {
-
-typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 __device__ __forceinline__ float epilogue(float acc, float alpha, float beta, const float* c, int64_t j, int64_t c_len,
                                           bool scale_a, bool scale_c) {
@@ -33,50 +23,258 @@ __device__ __forceinline__ float epilogue(float acc, float alpha, float beta, co
     return v;
 }
 
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) gemm_nt_mfma_kernel(const float* __restrict__ a, const float* __restrict__ b,
-                                                           const float* __restrict__ c, float* __restrict__ y,
-                                                           int32_t M, int32_t N, int32_t K, float alpha, float beta,
-                                                           int64_t c_len, int scale_a, int scale_c) {
-    __shared__ float part[4][32 * 33];
-    const int wave = threadIdx.x >> 6;
-    const int lane = threadIdx.x & 63;
-    const int half = lane >> 5;
-    const int r = lane & 31;
-    const int m0 = blockIdx.y * 32, n0 = blockIdx.x * 32;
-    const int arow = min(m0 + r, M - 1);       // clamped rows are computed and never stored
-    const int brow = min(n0 + r, N - 1);
-    const int kw = K / 4;                      // K range of this wave
-    const int kh = kw / 2;                     // K range of this half-wave (multiple of 4)
-    const float* ap = a + static_cast<int64_t>(arow) * K + wave * kw + half * kh;
-    const float* bp = b + static_cast<int64_t>(brow) * K + wave * kw + half * kh;
-    floatx16 acc = {0};
-    for (int k = 0; k < kh; k += 4) {
-        const float4 va = *reinterpret_cast<const float4*>(ap + k);
-        const float4 vb = *reinterpret_cast<const float4*>(bp + k);
-        // D[i][j] += A[i][k] * B[k][j]: operand A from rows of a (i = m), operand B from rows of b (j = n)
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(va.x, vb.x, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(va.y, vb.y, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(va.z, vb.z, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(va.w, vb.w, acc, 0, 0, 0);
-    }
-    // accumulator register g holds D[i][j] with j = lane % 32, i = 8*(g/4) + 4*(lane/32) + g%4
+constexpr uint32_t kOob = 0x80000000u;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* p, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, static_cast<int>(bytes), 0x00020000);
+}
+
+// 16 bytes per lane from a buffer straight into LDS (lane l writes lds + 16*l; see qconv_c16_i8.hip)
+typedef __attribute__((address_space(3))) void* lds_ptr_t;
+__device__ __forceinline__ void load16_to_lds(__amdgpu_buffer_rsrc_t rsrc, char* lds, uint32_t voffset, uint32_t soffset) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)lds, 16, voffset, soffset, 0, 0);
+#endif
+}
+
+// The KS partial tiles of a workgroup meet in LDS: [wave][register quad][lane][16 bytes]; register g of a block is row
+// 8*(g/4) + 4*half + g%4, column r.  Every wave finishes its share of the quads.
+template <int RO, int RP, int KS, bool TB>
+__device__ __forceinline__ void finish_tile(const f32x16 (&acc)[RO][RP], char* lds, int wave, int lane, const float* __restrict__ a, const float* __restrict__ b,
+                                            const float* __restrict__ c, float* __restrict__ y, int32_t M, int32_t N, int32_t K, int m0, int n0,
+                                            float alpha, float beta, int64_t c_len, int scale_a, int scale_c) {
+    constexpr int NB = RO * RP;
+    const int half = lane >> 5, r = lane & 31;
+    auto at = [&](int w, int q) { return reinterpret_cast<f32x4*>(lds + ((w * NB * 4 + q) * 64 + lane) * 16); };
 #pragma unroll
-    for (int g = 0; g < 16; ++g) {
-        const int i = 8 * (g / 4) + 4 * half + (g % 4);
-        part[wave][i * 33 + r] = acc[g];
+    for (int q = 0; q < NB * 4; ++q) {
+        const f32x16& v = acc[q / 4 / RP][q / 4 % RP];
+        *at(wave, q) = f32x4{v[4 * (q % 4)], v[4 * (q % 4) + 1], v[4 * (q % 4) + 2], v[4 * (q % 4) + 3]};
     }
     __syncthreads();
-    // 1024 outputs, 256 threads: 4 each, consecutive threads on consecutive n
-    for (int e = threadIdx.x; e < 1024; e += 256) {
-        const int i = e >> 5, j = e & 31;
-        float s = part[0][i * 33 + j];
-        s = __fadd_rn(s, part[1][i * 33 + j]);
-        s = __fadd_rn(s, part[2][i * 33 + j]);
-        s = __fadd_rn(s, part[3][i * 33 + j]);
-        const int m = m0 + i, n = n0 + j;
-        if (m < M && n < N)
-            y[static_cast<int64_t>(m) * N + n] = epilogue(s, alpha, beta, c, n, c_len, scale_a != 0, scale_c != 0);
+#pragma unroll
+    for (int t = 0; t < (NB * 4 + KS - 1) / KS; ++t) {
+        const int q = t * KS + wave;
+        if (q >= NB * 4) break;
+        f32x4 v = *at(0, q);
+#pragma unroll
+        for (int w = 1; w < KS; ++w) {
+            const f32x4 p = *at(w, q);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = __fadd_rn(v[e], p[e]);
+        }
+        const int n = n0 + (q / 4 % RP) * 32 + r;
+        if (n >= N) continue;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int m = m0 + (q / 4 / RP) * 32 + 8 * (q % 4) + 4 * half + e;
+            if (m >= M) continue;
+            float x = v[e];
+            if (__builtin_expect(x != x, 0)) {                // a non-finite operand: the fp32 loop spreads it
+                x = 0.0f;
+                for (int k = 0; k < K; ++k)
+                    x = fmaf(a[static_cast<int64_t>(m) * K + k], TB ? b[static_cast<int64_t>(n) * K + k] : b[static_cast<int64_t>(k) * N + n], x);
+            }
+            y[static_cast<int64_t>(m) * N + n] = epilogue(x, alpha, beta, c, n, c_len, scale_a != 0, scale_c != 0);
+        }
     }
+}
+
+// A workgroup owns one tile of 32*RO rows of `a` by 32*RP columns of y; its KS waves split the k-steps of 16 (contiguous
+// runs), read both operands straight into registers D steps ahead, split them into their three bf16 parts and multiply;
+// the partial tiles meet in LDS and every wave finishes its share of the rows.  Lane (r, half) of a step holds eight
+// consecutive k of row r: two 16-byte loads, or eight 4-byte loads of neighbouring columns when b is [k][n].
+// What bounds it: the splitting (11 instructions per two values on the vector ALU) beside the matrix instructions of the
+// other waves; before that, with few tiles, the chain launch - first load - last store.  No LDS staging: a tile's operands
+// are read by one workgroup and the vector cache serves the two halves of a line.  Measured (us, one thread per output before):
+// b = [k][n] 300 x 1000 x 2048 474 -> 23.5, 33 x 500 x 900 211 -> 7.5; k not a multiple of four 257 x 333 x 777 202 -> 9.6.
+template <int RO, int RP, int KS, int D, bool TB>
+__global__ void __launch_bounds__(64 * KS) __attribute__((amdgpu_waves_per_eu(2))) gemm_bf16x3_kernel(
+    const float* __restrict__ a, const float* __restrict__ b, const float* __restrict__ c, float* __restrict__ y, int32_t M, int32_t N, int32_t K,
+    int32_t m_tiles, int32_t tiles, int32_t tiles_per_xcd, float alpha, float beta, int64_t c_len, int scale_a, int scale_c) {
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    const int lane = threadIdx.x & 63, half = lane >> 5, r = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+    // an XCD (own L2) takes a contiguous run of tiles: all row tiles of a column tile before the next one
+    const int tile = static_cast<int>(blockIdx.x & 7) * tiles_per_xcd + static_cast<int>(blockIdx.x >> 3);
+    if (tile >= tiles || static_cast<int>(blockIdx.x >> 3) >= tiles_per_xcd) return;
+    const int n_tile = tile / m_tiles, m0 = (tile - n_tile * m_tiles) * 32 * RO, n0 = n_tile * 32 * RP;
+
+    // rows past the last one lie beyond the buffers and read as zero
+    const __amdgpu_buffer_rsrc_t ar = make_rsrc(a + static_cast<int64_t>(m0) * K, static_cast<uint32_t>(min(32 * RO, M - m0)) * static_cast<uint32_t>(K) * 4u);
+    const __amdgpu_buffer_rsrc_t br = TB ? make_rsrc(b + static_cast<int64_t>(n0) * K, static_cast<uint32_t>(min(32 * RP, N - n0)) * static_cast<uint32_t>(K) * 4u)
+                                         : make_rsrc(b, static_cast<uint32_t>(K) * static_cast<uint32_t>(N) * 4u);
+    uint32_t ao[RO], bo[RP];
+#pragma unroll
+    for (int i = 0; i < RO; ++i) ao[i] = m0 + i * 32 + r < M ? static_cast<uint32_t>((i * 32 + r) * K + 8 * half) * 4u : kOob;
+#pragma unroll
+    for (int j = 0; j < RP; ++j) {
+        const int n = n0 + j * 32 + r;
+        bo[j] = n >= N ? kOob : TB ? static_cast<uint32_t>((j * 32 + r) * K + 8 * half) * 4u : static_cast<uint32_t>(8 * half * N + n) * 4u;
+    }
+    const uint32_t row_bytes = static_cast<uint32_t>(N) * 4u;
+
+    f32x16 acc[RO][RP];
+#pragma unroll
+    for (int i = 0; i < RO; ++i)
+#pragma unroll
+        for (int j = 0; j < RP; ++j)
+#pragma unroll
+            for (int g = 0; g < 16; ++g) acc[i][j][g] = 0.0f;
+
+    float av[D][RO][8], bv[D][RP][8];
+    auto load8 = [](float (&v)[8], __amdgpu_buffer_rsrc_t rs, uint32_t vo, uint32_t so) __attribute__((always_inline)) {
+        const f32x4 lo = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, vo, so, 0));
+        const f32x4 hi = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, vo + 16u, so, 0));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { v[e] = lo[e]; v[4 + e] = hi[e]; }
+    };
+    auto ldf = [](__amdgpu_buffer_rsrc_t rs, uint32_t vo, uint32_t so) __attribute__((always_inline)) {
+        return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, vo, so, 0));
+    };
+    auto load = [&](int step, int d) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < RO; ++i) load8(av[d][i], ar, ao[i], static_cast<uint32_t>(step) * 64u);
+#pragma unroll
+        for (int j = 0; j < RP; ++j) {
+            if constexpr (TB) {
+                load8(bv[d][j], br, bo[j], static_cast<uint32_t>(step) * 64u);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) bv[d][j][e] = ldf(br, bo[j], static_cast<uint32_t>(step * 16 + e) * row_bytes);
+            }
+        }
+    };
+    auto multiply = [&](int d) __attribute__((always_inline)) {
+        u32x4 af[RO][3], bf[RP][3];
+#pragma unroll
+        for (int i = 0; i < RO; ++i) { const Split8 p = split8(av[d][i]); af[i][0] = p.h; af[i][1] = p.m; af[i][2] = p.l; }
+#pragma unroll
+        for (int j = 0; j < RP; ++j) { const Split8 p = split8(bv[d][j]); bf[j][0] = p.h; bf[j][1] = p.m; bf[j][2] = p.l; }
+        mfma6<RO, RP>(acc, af, bf);
+    };
+    const int steps = K >> 4;                                 // whole ones
+    const int per = ((steps + KS - 1) / KS + 1) & ~1;         // (two steps share a 128-byte line)
+    const int lo = min(steps, wave * per), hi = min(steps, lo + per);
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+        if (lo + d < hi) load(lo + d, d);
+    int s = lo;
+    for (; s + 2 * D <= hi; s += D) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            multiply(d);
+            load(s + D + d, d);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    for (; s < hi; s += D) {
+#pragma unroll
+        for (int d = 0; d < D; ++d)
+            if (s + d < hi) {
+                multiply(d);
+                if (s + D + d < hi) load(s + D + d, d);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+    }
+    if ((K & 15) != 0 && wave == KS - 1) {                    // what is left of k, element by element
+        const int k0 = steps << 4;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const bool in = k0 + 8 * half + e < K;
+#pragma unroll
+            for (int i = 0; i < RO; ++i) av[0][i][e] = ldf(ar, in ? ao[i] + 4u * e : kOob, static_cast<uint32_t>(k0) * 4u);
+#pragma unroll
+            for (int j = 0; j < RP; ++j)
+                bv[0][j][e] = ldf(br, in ? bo[j] + (TB ? 4u * e : 0u) : kOob, TB ? static_cast<uint32_t>(k0) * 4u : static_cast<uint32_t>(k0 + e) * row_bytes);
+        }
+        multiply(0);
+    }
+
+    finish_tile<RO, RP, KS, TB>(acc, lds, wave, lane, a, b, c, y, M, N, K, m0, n0, alpha, beta, c_len, scale_a, scale_c);
+}
+
+// The same tiles where rows of both operands are whole 16-byte words (b = [n][k], k a multiple of four).  Lane (r, half)
+// reading its own row touches 32 cache lines with every load, and the vector cache takes those one after the other:
+// here a load covers eight rows by 128 bytes (eight lines) and goes straight into LDS, into a chunk of 32 k that belongs to
+// the wave alone: no barrier, the wave waits for its own loads, moves the chunk into registers, requests the next one and
+// multiplies (a ring of two or four chunks was slower or equal: fewer workgroups fit a compute unit).  Within a row the 16-byte words are stored in
+// the order (word ^ row % 8), so the 32 rows that a fragment read takes at once hit all banks.
+// Measured (us; before: fp32 matrix instructions on operands read row by row): 300 x 1000 x 2048 54.6 -> 18.4,
+// 512 x 4096 x 4096 514 -> 113, 8 x 4096 x 4096 47.6 -> 20.0, 64 x 1000 x 512 7.6 -> 5.7; k = 1000 (no multiple of 32 before)
+// 200 x 2000 x 1000 1667 -> 14.4.
+template <int RO, int RP, int KS>
+__global__ void __launch_bounds__(64 * KS) __attribute__((amdgpu_waves_per_eu(2))) gemm_nt_staged_kernel(
+    const float* __restrict__ a, const float* __restrict__ b, const float* __restrict__ c, float* __restrict__ y, int32_t M, int32_t N, int32_t K,
+    int32_t m_tiles, int32_t tiles, int32_t tiles_per_xcd, float alpha, float beta, int64_t c_len, int scale_a, int scale_c) {
+    constexpr int L = 4 * (RO + RP);                          // loads of 1 KiB per chunk
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    const int lane = threadIdx.x & 63, half = lane >> 5, r = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+    const int tile = static_cast<int>(blockIdx.x & 7) * tiles_per_xcd + static_cast<int>(blockIdx.x >> 3);
+    if (tile >= tiles || static_cast<int>(blockIdx.x >> 3) >= tiles_per_xcd) return;
+    const int n_tile = tile / m_tiles, m0 = (tile - n_tile * m_tiles) * 32 * RO, n0 = n_tile * 32 * RP;
+
+    // rows past the last one lie beyond the buffers and read as zero
+    const __amdgpu_buffer_rsrc_t ar = make_rsrc(a + static_cast<int64_t>(m0) * K, static_cast<uint32_t>(min(32 * RO, M - m0)) * static_cast<uint32_t>(K) * 4u);
+    const __amdgpu_buffer_rsrc_t br = make_rsrc(b + static_cast<int64_t>(n0) * K, static_cast<uint32_t>(min(32 * RP, N - n0)) * static_cast<uint32_t>(K) * 4u);
+    char* const ring = lds + wave * (L * 1024);
+    const int kword = (lane & 7) ^ (lane >> 3);               // the word of its row's chunk that a lane loads
+    uint32_t vo[4 * (RO > RP ? RO : RP)];
+#pragma unroll
+    for (int i = 0; i < 4 * (RO > RP ? RO : RP); ++i) vo[i] = static_cast<uint32_t>((i * 8 + (lane >> 3)) * K + kword * 4) * 4u;
+    const int chunks = (K + 31) >> 5, per = (chunks + KS - 1) / KS;
+    const int lo = min(chunks, wave * per), hi = min(chunks, lo + per);
+    auto issue = [&](int chunk) __attribute__((always_inline)) {
+        const uint32_t mask = chunk * 32 + kword * 4 < K ? 0u : kOob;
+#pragma unroll
+        for (int i = 0; i < 4 * RO; ++i) load16_to_lds(ar, ring + i * 1024, vo[i] | mask, static_cast<uint32_t>(chunk) * 128u);
+#pragma unroll
+        for (int i = 0; i < 4 * RP; ++i) load16_to_lds(br, ring + (4 * RO + i) * 1024, vo[i] | mask, static_cast<uint32_t>(chunk) * 128u);
+    };
+    f32x16 acc[RO][RP];
+#pragma unroll
+    for (int i = 0; i < RO; ++i)
+#pragma unroll
+        for (int j = 0; j < RP; ++j)
+#pragma unroll
+            for (int g = 0; g < 16; ++g) acc[i][j][g] = 0.0f;
+    if (lo < hi) {
+        issue(lo);
+        for (int chunk = lo; chunk < hi; ++chunk) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            float av[2][RO][8], bv[2][RP][8];
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                auto read8 = [&](float (&v)[8], int row0) __attribute__((always_inline)) {
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) {
+                        const f32x4 w = *reinterpret_cast<const f32x4*>(ring + row0 * 128 + r * 128 + (((4 * s + 2 * half + q) ^ (r & 7)) << 4));
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) v[4 * q + e] = w[e];
+                    }
+                };
+#pragma unroll
+                for (int i = 0; i < RO; ++i) read8(av[s][i], i * 32);
+#pragma unroll
+                for (int j = 0; j < RP; ++j) read8(bv[s][j], (RO + j) * 32);
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // read before it is filled again
+            __builtin_amdgcn_sched_barrier(0);
+            if (chunk + 1 < hi) issue(chunk + 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                u32x4 af[RO][3], bf[RP][3];
+#pragma unroll
+                for (int i = 0; i < RO; ++i) { const Split8 p = split8(av[s][i]); af[i][0] = p.h; af[i][1] = p.m; af[i][2] = p.l; }
+#pragma unroll
+                for (int j = 0; j < RP; ++j) { const Split8 p = split8(bv[s][j]); bf[j][0] = p.h; bf[j][1] = p.m; bf[j][2] = p.l; }
+                mfma6<RO, RP>(acc, af, bf);
+            }
+        }
+    }
+    __syncthreads();                                          // the chunks become the partial tiles
+    finish_tile<RO, RP, KS, true>(acc, lds, wave, lane, a, b, c, y, M, N, K, m0, n0, alpha, beta, c_len, scale_a, scale_c);
 }
 
 // A handful of rows (batch 1-4 of a classifier layer): the matrix-core tile above would be 32 rows of which at
@@ -284,7 +482,7 @@ int32_t kxc_hip_gemm_f32(const float* a, const float* b, const float* c, float* 
     const int scale_a = (static_cast<double>(alpha) != 1.0) ? 1 : 0;   // ScaleTensor, src/relay/op/nn/dense.cc:17-24
     const int scale_c = (static_cast<double>(beta) != 1.0) ? 1 : 0;
     const bool aligned = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15u) == 0;
-    // (the same shapes as the matrix-core kernel below: whatever took the reference-order kernel still does)
+    // (rows of whole 16-byte words)
     if (transB && k > 0 && (k % 32) == 0 && aligned && m <= kGemvRows && n < (1 << 20) && k < (1 << 30)) {
         const unsigned grid = static_cast<unsigned>(CeilDiv(n, 4 * kGemvCols));
         const int32_t n32 = static_cast<int32_t>(n), k32 = static_cast<int32_t>(k);
@@ -298,12 +496,32 @@ int32_t kxc_hip_gemm_f32(const float* a, const float* b, const float* c, float* 
 #undef KXC_GEMV
         return CheckLaunch("gemv_nt");
     }
-    if (transB && k > 0 && (k % 32) == 0 && aligned && m < (1 << 20) && n < (1 << 20) && k < (1 << 30)) {
-        dim3 grid(static_cast<unsigned>(CeilDiv(n, 32)), static_cast<unsigned>(CeilDiv(m, 32)));
-        KXC_HIP_REQUIRE(grid.y <= 65535u, "kxc_hip_gemm_f32: m too large");
-        gemm_nt_mfma_kernel<<<NoteGrid(grid), NoteBlock(256), NoteLds(0), s>>>(a, b, c, y, static_cast<int32_t>(m), static_cast<int32_t>(n),
-                                                  static_cast<int32_t>(k), alpha, beta, c_len, scale_a, scale_c);
-        return CheckLaunch("gemm_nt_mfma");
+    // (row offsets of a tile and, for b = [k][n], all of b are addressed with 31 bits)
+    const bool small = m * n * k < (1 << 15);
+    if (k > 0 && (!small || (transB && k % 32 == 0)) && m < (1 << 20) && n < (1 << 20) && k < (1 << 24) && (transB || n * (k + 16) < (1 << 29))) {
+        struct Tile { int ro, rp, ks; void (*kernel[3])(const float*, const float*, const float*, float*, int32_t, int32_t, int32_t, int32_t, int32_t, int32_t,
+                                                        float, float, int64_t, int, int); };
+#define KXC_GEMM(RO, RP, KS, D) {RO, RP, KS, {gemm_bf16x3_kernel<RO, RP, KS, D, false>, gemm_bf16x3_kernel<RO, RP, KS, D, true>, gemm_nt_staged_kernel<RO, RP, KS>}}
+        static const Tile kTiles[] = {KXC_GEMM(1, 1, 8, 2), KXC_GEMM(2, 1, 8, 2), KXC_GEMM(2, 2, 4, 1)};
+#undef KXC_GEMM
+        // The largest tile (least splitting per product) that still leaves enough workgroups: 64 x 64 from 1024 blocks of
+        // 32 x 32 on (512 x 4096 x 512: 21.5 us, 27.5 with 64 x 32, 28.3 with 32 x 32), 64 x 32 while the compute units do
+        // not get one 32 x 32 tile each (300 x 1000 x 2048, 320 blocks: 18.4 against 19.6; 512 x 512 x 4096, 256: 30.7
+        // against 22.8)
+        const int64_t blocks = CeilDiv(m, 32) * CeilDiv(n, 32);
+        const Tile& t = kTiles[blocks <= 256 || k >= (1 << 22) ? 0 : blocks < 1024 ? 1 : 2];
+        const int64_t m_tiles = CeilDiv(m, 32 * t.ro), tiles = m_tiles * CeilDiv(n, 32 * t.rp);
+        KXC_HIP_REQUIRE(tiles < (1 << 28), "kxc_hip_gemm_f32: too many tiles");
+        const int32_t per_xcd = static_cast<int32_t>(CeilDiv(tiles, 8));
+        const bool staged = transB && k % 4 == 0 && aligned;
+        const size_t lds = static_cast<size_t>(t.ks) * (staged ? t.ro + t.rp : t.ro * t.rp) * 4096;      // (a chunk is never smaller than a partial tile)
+        const auto kernel = t.kernel[staged ? 2 : transB ? 1 : 0];
+        if (lds > 64 * 1024)
+            if (int32_t rc = GrantLds(reinterpret_cast<const void*>(kernel))) return rc;
+        kernel<<<NoteGrid(static_cast<int>(per_xcd * 8)), NoteBlock(64 * t.ks), NoteLds(lds), s>>>(
+            a, b, c, y, static_cast<int32_t>(m), static_cast<int32_t>(n), static_cast<int32_t>(k), static_cast<int32_t>(m_tiles),
+            static_cast<int32_t>(tiles), per_xcd, alpha, beta, c_len, scale_a, scale_c);
+        return CheckLaunch("gemm_bf16x3");
     }
     int64_t g = CeilDiv(m * n, 256);
     if (g > 256 * 32) g = 256 * 32;

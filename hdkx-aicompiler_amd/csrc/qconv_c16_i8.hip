@@ -1775,11 +1775,8 @@ int32_t kxc_hip_qconv2d_c16_i8(const kxc_hip_qconv2d_desc* d, const int8_t* x, c
     KXC_HIP_REQUIRE(!(d->flags & KXC_HIP_CONV_RESIDUAL) || residual, "kxc_hip_qconv2d_c16_i8: residual flag without residual");
     QArgs& a = L.args;
     a.x = x; a.wp = w_packed; a.bias = bias; a.mult = mult; a.res = residual; a.y = y;
-    if (L.lds_bytes > 64 * 1024) {
-        KXC_HIP_CALL(hipFuncSetAttribute(reinterpret_cast<const void*>(L.kernel),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(L.lds_bytes)),
-                     "hipFuncSetAttribute");
-    }
+    if (L.lds_bytes > 64 * 1024)
+        if (int32_t rc = GrantLds(reinterpret_cast<const void*>(L.kernel))) return rc;
     hipLaunchKernelGGL(L.kernel, NoteGrid(dim3(L.grid)), NoteBlock(dim3(L.threads)), NoteLds(L.lds_bytes), ResolveStream(stream), a);
     return CheckLaunch(L.name);
 }
@@ -1847,11 +1844,8 @@ int32_t kxc_hip_qconv2d_c16_pair_i8(const kxc_hip_qconv2d_desc* d, const int8_t*
     if (std::strncmp(L.name, "qrows", 5) == 0) row_positions = 64;
     a.ds_off = (d->pad_h * row_positions + d->pad_w) * 16;
     L.lds_bytes += L.ds_lds_extra;
-    if (L.lds_bytes > 64 * 1024) {
-        KXC_HIP_CALL(hipFuncSetAttribute(reinterpret_cast<const void*>(L.ds_kernel),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(L.lds_bytes)),
-                     "hipFuncSetAttribute");
-    }
+    if (L.lds_bytes > 64 * 1024)
+        if (int32_t rc = GrantLds(reinterpret_cast<const void*>(L.ds_kernel))) return rc;
     hipLaunchKernelGGL(L.ds_kernel, NoteGrid(dim3(L.grid)), NoteBlock(dim3(L.threads)), NoteLds(L.lds_bytes), ResolveStream(stream), a);
     return CheckLaunch(L.name);
 }

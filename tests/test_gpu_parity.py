@@ -962,6 +962,30 @@ def test_gemm_random_shapes(pkg):
         assert_close(got, want.astype(np.float32), what="case %d: m=%d n=%d k=%d transB=%d" % (case, m, n, k, trans_b))
 
 
+@pytest.mark.parametrize("trans_b", [1, 0])
+@pytest.mark.parametrize("m,n,k", [
+    # one element past the few-row kernel and past a tile in each direction; k below one step, one past a step, a chunk or
+    # a wave's share (rows that are whole 16-byte words and rows that are not); the three tiles with ragged edges
+    (5, 1, 6600), (33, 65, 16), (6, 400, 15), (31, 97, 17), (40, 33, 36), (64, 64, 255), (129, 31, 260), (7, 50, 1001),
+    (290, 1030, 50), (65, 4001, 33), (300, 4000, 20), (515, 2111, 37),
+])
+def test_gemm_tile_edges(pkg, m, n, k, trans_b):
+    """The matrix-core products at the edges of their tiles, against float64: an fp32 sum of k products in any order is
+    within k * 2^-24 * sum |a b| of the exact one.  A non-finite operand spreads to its row or column and no further."""
+    rng = np.random.default_rng(m * 7 + n * 3 + k)
+    a = rng.uniform(-1, 1, (m, k)).astype(np.float32)
+    b = rng.uniform(-1, 1, (n, k) if trans_b else (k, n)).astype(np.float32)
+    b64 = (b.T if trans_b else b).astype(np.float64)
+    got = host(pkg.gemm(dev(a), dev(b), None, 1.0, 1.0, trans_b))
+    bound = k * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(b64))
+    assert (np.abs(got - a.astype(np.float64) @ b64) <= bound).all()
+    a[m - 1, k - 1] = np.inf
+    a[0, 0] = np.nan
+    again = host(pkg.gemm(dev(a), dev(b), None, 1.0, 1.0, trans_b))
+    assert np.isnan(again[0]).all() and np.array_equal(again[m - 1], np.inf * np.sign(b64[k - 1]))
+    assert_bit_exact(again[1:m - 1], got[1:m - 1], "other rows")
+
+
 def test_bias_add_and_flatten(pkg, orc, synth):
     x = synth.uniform((3, 6, 5, 7), 2040); b = synth.uniform((6,), 2041)
     assert_bit_exact(host(pkg.bias_add(dev(x), dev(b))), orc.bias_add(x, b), "bias_add")
