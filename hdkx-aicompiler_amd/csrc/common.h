@@ -149,6 +149,7 @@ int32_t PrepareConv2d(const kxc_hip_conv2d_desc* desc, bool second_output, Prepa
 int32_t LaunchPreparedConv2d(const PreparedConv* p, const float* x, const float* w, const float* bias, const float* residual,
                              float* y, const float* w2, const float* bias2, float* y2, hipStream_t stream);
 const char* PreparedConvName(const PreparedConv* p);
+bool SmallConvBeatsWinograd(const kxc_hip_conv2d_desc* desc);      // a plan's Winograd node is better launched as PreparedConv
 void FreePreparedConv(PreparedConv* p);
 struct PreparedWinograd;
 int32_t PrepareWinograd(const kxc_hip_conv2d_desc* desc, PreparedWinograd** out);

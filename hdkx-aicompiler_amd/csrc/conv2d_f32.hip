@@ -28,6 +28,7 @@
 //    (rc, rh, rw ascending from 0.0f, multiply and add rounded separately, padded taps add
 //    0.0f * w).  Bit-identical to the CPU backend; used for shapes the MFMA tiling does not
 //    cover (output channels not a multiple of 32, very wide rows) and on request.
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <memory>
@@ -111,7 +112,7 @@ typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
 }  // namespace
 
-#include "conv_bf16x3.h"
+#include "conv_small.h"
 
 namespace {
 
@@ -1135,114 +1136,83 @@ bool PairTap(const kxc_hip_conv2d_desc* d, int* rh, int* rw) {
     return oh == (d->h - 1) / d->stride_h + 1 && ow == (d->w - 1) / d->stride_w + 1;
 }
 
-// ------------------------------------------------------------------------------------------
-// Launches on the bf16 matrix cores with three-part operands (conv_bf16x3.h).
-// ------------------------------------------------------------------------------------------
-struct BxVariant {
-    const char* tile;           // name = mfma_k<kh>x<kw>_bf16x3_<tile>
-    int to, tp, threads, ks, ix, iw, c4;
-    void (*kernel)(const conv_bx::Args);
-    void (*ds_kernel)(const conv_bx::Args);
+// conv_small_kernel by (filter, tile, waves per workgroup): conv_small.h
+struct SmallVariant {
+    const char* name;
+    int k, chunk, ro, ks;               // filter extent, channels per chunk, blocks of 16 output channels, waves
+    int wi, xi;                         // KiB of weights and of input rows per wave and chunk
+    void (*kernel)(const conv_small::Args);
+    void (*ds_kernel)(const conv_small::Args);
 };
-#define KXC_BX(TILE, RO, RP, WO, WP, KS, IX, IW)                                                                          \
-    {TILE, 32 * RO * WO, 32 * RP * WP, 64 * WO * WP * KS, KS, IX, IW, 0, conv_bx::conv_bf16x3_kernel<RO, RP, WO, WP, KS, IX, IW, false, false>, \
-     conv_bx::conv_bf16x3_kernel<RO, RP, WO, WP, KS, IX, IW, false, true>}
-#define KXC_BX_C4(TILE, RO, RP, WO, WP, KS, IX, IW)                                                                       \
-    {TILE, 32 * RO * WO, 32 * RP * WP, 64 * WO * WP * KS, KS, IX, IW, 1, conv_bx::conv_bf16x3_kernel<RO, RP, WO, WP, KS, IX, IW, true, false>, nullptr}
-const BxVariant kBx[] = {
-    KXC_BX("o64_p256", 2, 2, 1, 4, 1, 4, 3),
-    KXC_BX("o64_p128", 2, 1, 1, 4, 1, 4, 3),
-    KXC_BX("o64_p64", 1, 1, 2, 2, 1, 4, 3),
-    KXC_BX("o32_p32_ks4", 1, 1, 1, 1, 4, 5, 5),
-    KXC_BX_C4("c4_o64_p256", 2, 2, 1, 4, 1, 13, 4),
-    KXC_BX_C4("c4_o64_p64", 1, 1, 2, 2, 1, 8, 4),
-};
-constexpr int kNumBx = sizeof(kBx) / sizeof(kBx[0]);
-
-struct BxChoice {
-    const BxVariant* v = nullptr;
-    int32_t cb = 1, nq = 0, nq_main = 0, group_steps = 0, ngroups = 0, chs = 0;
-    size_t lds_bytes = 0;
+#define KXC_SMALL(NAME, K, CPG, XI, RO, KS) \
+    {NAME, K, 4 * CPG, RO, KS, RO * CPG * K * K / 4, XI, conv_small::conv_small_kernel<K, K, CPG, XI, RO, KS>, nullptr}
+#define KXC_SMALL_DS(NAME, K, CPG, XI, RO, KS) \
+    {NAME, K, 4 * CPG, RO, KS, RO * CPG * K * K / 4, XI, conv_small::conv_small_kernel<K, K, CPG, XI, RO, KS>, conv_small::conv_small_kernel<K, K, CPG, XI, RO, KS, true>}
+const SmallVariant kSmall[] = {
+    KXC_SMALL_DS("mfma_k3x3_small_rows", 3, 4, 8, 1, 8), KXC_SMALL_DS("mfma_k3x3_small_o1", 3, 4, 0, 1, 4), KXC_SMALL_DS("mfma_k3x3_small_o2", 3, 4, 0, 2, 4),
+    KXC_SMALL("mfma_k1x1_small", 1, 4, 0, 2, 4), KXC_SMALL("mfma_k1x1_small", 1, 4, 0, 4, 4),
 };
 
-bool BxFits(const BxVariant& v, const ConvArgs& a, int kh, int kw, bool ds, BxChoice* out) {
-    if (ds && !v.ds_kernel) return false;
-    if (v.c4 && (a.C > 4 || a.dw != 1)) return false;
-    const int64_t positions = static_cast<int64_t>(MaxTileRows(a, kh, v.tp)) * a.Wp;
-    const int32_t chs = static_cast<int32_t>((positions + 3) / 4 * 4);
-    const int cbs = (a.C + 7) / 8, wrow = (v.to + 1) * 16;
-    const int max_cb = v.c4 ? 1 : kh * kw == 1 || v.ks > 1 ? 16 : 1;
-    for (int cb = max_cb < cbs ? max_cb : cbs; cb >= 1; --cb) {
-        if (positions > (1 << 20) || static_cast<int64_t>(cb) * chs > static_cast<int64_t>(v.ix) * v.threads) continue;
-        const int nq_main = v.c4 ? (kh * ((kw + 1) / 2) + 1) / 2 * 2 : (kh * kw * cb + 1) / 2 * 2;
-        const int nq = nq_main + (ds ? (cb + 1) / 2 * 2 : 0);
-        if (nq > conv_bx::kMaxQ) continue;
-        const int max_steps = v.iw * v.threads / (2 * v.to);
-        const int groups = (nq / 2 + max_steps - 1) / max_steps, gs = (nq / 2 + groups - 1) / groups;
-        if (v.ks > 1 && groups > 1) continue;
-        size_t lds = conv_bx::kMaxQ * 4 + 3 * static_cast<size_t>(cb) * chs * (v.c4 ? 8 : 16) + 3 * 2 * static_cast<size_t>(gs) * wrow;
-        const size_t red = static_cast<size_t>(v.ks - 1) * v.to * v.tp * sizeof(float);
-        if (red > lds) lds = red;
-        if (lds > kMaxLdsBytes) continue;
-        out->v = &v; out->cb = cb; out->nq = nq; out->nq_main = nq_main; out->group_steps = gs;
-        out->ngroups = (nq / 2 + gs - 1) / gs; out->chs = chs; out->lds_bytes = lds;
-        return true;
+// 16-byte words of the rows that a tile touches in one channel (a run starts up to three values behind a 16-byte boundary)
+int SmallWords(const SmallVariant& v, const ConvArgs& a) {
+    int rows = 0;
+    for (int q0 = 0; q0 < a.OHW; q0 += 16) {
+        const int q1 = (q0 + 16 < a.OHW ? q0 + 16 : a.OHW) - 1;
+        const int r0 = q0 / a.OW * a.sh - a.ph, r1 = q1 / a.OW * a.sh - a.ph + (v.k - 1) * a.dh;
+        const int lo = std::min(std::max(r0, 0), a.H - 1), hi = std::max(std::min(r1, a.H - 1), lo);
+        rows = std::max(rows, hi - lo + 1);
     }
-    return false;
+    return (rows * a.W + 3 + 3) / 4;
 }
 
-const char* BxName(const BxVariant& v, int kh, int kw) {
-    static std::mutex mu;
-    static std::vector<std::unique_ptr<std::string>> names;      // a handful: one per filter size and tile in use
-    const std::string name = "mfma_k" + std::to_string(kh) + "x" + std::to_string(kw) + "_bf16x3_" + v.tile;
-    std::lock_guard<std::mutex> lock(mu);
-    for (const auto& n : names)
-        if (*n == name) return n->c_str();
-    names.emplace_back(new std::string(name));
-    return names.back()->c_str();
-}
-
-// The three-part launch of a shape (after FillArgs and ApplyRowView), or v == nullptr for the fp32-instruction kernels.
-void BxSelect(const ConvArgs& a, const kxc_hip_conv2d_desc* d, bool ds, BxChoice* choice) {
-    choice->v = nullptr;
-    if ((d->flags & (KXC_HIP_CONV_FORCE_DIRECT | KXC_HIP_CONV_HPOOL)) || a.M <= 0) return;
-    const int64_t x_bytes = static_cast<int64_t>(a.N) * a.C * a.H * a.W * 4, y_elems = static_cast<int64_t>(a.N) * a.O * a.OHW;
-    const int64_t w_bytes = static_cast<int64_t>(a.O) * a.C * d->kh * d->kw * 4, q_rows = static_cast<int64_t>(a.N + 1) * a.Hp + static_cast<int64_t>(d->kh) * a.dh;
-    if (x_bytes >= (1LL << 31) || y_elems * 4 >= (1LL << 31) || w_bytes >= (1LL << 31) || q_rows * a.Wp >= (1LL << 31)) return;
+// Which small-launch kernel takes a shape (after FillArgs, before ApplyRowView), if any.  Channels are a multiple of a chunk (16).
+// 1x1: always, except wide maps of few channels, where the general tiles are as fast or faster: batch 64, 64 channels at 56 x 56:
+//   51 us both; 48 -> 200 at 30 x 30: 44 against 39; ahead from 96 channels on (128 -> 512 at 28 x 28, batch 64: 125 -> 117;
+//   256 -> 512 at 14 x 14, batch 16: 49 -> 15).  Four blocks of output channels per workgroup once there are two such
+//   tiles per compute unit (64 -> 128 with stride 2, batch 16: 10.9 -> 9.2), two before (512 -> 128 at 14 x 14, batch 4: 5.9 against 6.8).
+// 3x3: up to 800 tiles of 16 x 16, 1600 with the second output (a launch plan's two-output node otherwise needs an adding launch
+//   for both): 128 channels at 28 x 28 12.5 -> 7.9 us at batch 1 (392 tiles), 17 -> 12 at batch 2 (784), equal at batch 4;
+//   128 -> 256 with stride 2 and the second output, batch 8 (1568): 28.9 -> 26.1.  At least 64 channels, a chunk per wave.
+//   Staged rows for narrow maps while every tile has a compute unit to itself (256 at 14 x 14, batch 1: 8.5 -> 7.5; 512 at 7 x
+//   7: 13.2 -> 10.9); two blocks of output channels from 257 tiles on (64 at 56 x 56, batch 1: 9.6 -> 8.7).
+//   Outside a plan, only from 400 tiles on: below, kxc_hip_conv2d_scratch_needed promises the callers of the single
+//   operator a reduction split over workgroups.
+const SmallVariant* SelectSmall(const kxc_hip_conv2d_desc* d, const ConvArgs& a, bool second, bool in_plan) {
+    if ((d->flags & (KXC_HIP_CONV_FORCE_DIRECT | KXC_HIP_CONV_HPOOL)) || a.M <= 0 || a.C % 16 != 0 || d->kh != d->kw) return nullptr;
+    const int64_t x_elems = static_cast<int64_t>(a.N) * a.C * a.H * a.W, y_elems = static_cast<int64_t>(a.N) * a.O * a.OHW;
+    const int64_t w_elems = static_cast<int64_t>(a.O) * a.C * d->kh * d->kw;
+    if (x_elems >= (1 << 29) || y_elems >= (1 << 29) || w_elems >= (1 << 29)) return nullptr;       // 31-bit byte offsets
     const char* forced = std::getenv("KXC_HIP_CONV_VARIANT");
-    const char* bx = std::getenv("KXC_HIP_CONV_BF16X3");
-    if (bx && bx[0] == '0') return;
-    for (const BxVariant& v : kBx) {
-        if (forced && *forced) {
-            if (std::strcmp(forced, BxName(v, d->kh, d->kw)) != 0) continue;
-        } else {
-            return;
-        }
-        if (BxFits(v, a, d->kh, d->kw, ds, choice)) return;
-        choice->v = nullptr;
+    const bool by_name = forced && *forced;
+    const int64_t tiles = CeilDiv(a.M, 16) * CeilDiv(a.O, 16) * SelectLanes();
+    const SmallVariant* const v = kSmall;
+    if (d->kh == 1) {
+        if (by_name ? std::strcmp(forced, v[3].name) != 0 : a.C < 96 && static_cast<int64_t>(a.M) * a.O > 6000000) return nullptr;
+        return second ? nullptr : CeilDiv(a.M, 16) * CeilDiv(a.O, 64) * SelectLanes() >= 512 ? v + 4 : v + 3;
     }
-}
-
-// Parts of a split reduction of a three-part launch.
-int BxSplit(const BxChoice& c, int32_t nchunks, int64_t tiles, int64_t total) {
-    int split = 1;
-    if (const char* e = std::getenv("KXC_HIP_CONV_GSPLIT")) {
-        const int f = std::atoi(e);
-        if (f >= 1 && f <= nchunks && total * static_cast<int64_t>(sizeof(float)) * f <= (256LL << 20)) split = f;
+    if (d->kh != 3 || (second && !in_plan)) return nullptr;
+    const bool rows_fit = a.dw == 1 && SmallWords(v[0], a) * v[0].chunk <= v[0].xi * 64;
+    if (by_name) {
+        for (int i = rows_fit ? 0 : 1; i < 3; ++i)
+            if (std::strcmp(forced, v[i].name) == 0) return v + i;
+        return nullptr;
     }
-    return split;
+    if (a.C < 64 || tiles > (second ? 1600 : 800) || (!in_plan && tiles < 400)) return nullptr;
+    if (rows_fit && a.N * CeilDiv(a.OHW, 16) * CeilDiv(a.O, 16) * SelectLanes() <= kNumCUs) return v;
+    return tiles <= kNumCUs ? v + 1 : v + 2;
 }
 
 // Everything about a launch that the descriptor alone decides (kernel, tile shape, grid, the split of the reduction,
 // the switches read from the environment): resolved once per call by the entry points, once per node by a launch
 // plan (kxc_hip::PreparedConv), and combined with the operand pointers and the stream at launch time.
 struct ConvLaunch {
-    enum Path { kEmpty, kSmall1x1, kMfma, kDirect, kBf16x3 };
+    enum Path { kEmpty, kSmall1x1, kSmall, kMfma, kDirect };
     Path path = kEmpty;
+    kxc_hip_conv2d_desc desc;
     ConvArgs a;                     // without operand pointers and partial-sum buffer
     ConvArgs direct_args;
-    conv_bx::Args bx;               // kBf16x3: instead of `a` (which keeps the flags and the split)
-    void (*bx_kernel)(const conv_bx::Args) = nullptr;
+    conv_small::Args sm;            // kSmall
+    void (*small_kernel)(const conv_small::Args) = nullptr;
     void (*kernel)(const ConvArgs) = nullptr;
     const char* name = "";
     dim3 grid, block;
@@ -1253,52 +1223,12 @@ struct ConvLaunch {
     bool second = false;
 };
 
-int32_t BxResolve(const kxc_hip_conv2d_desc* desc, bool second, const char* who, const BxChoice& c, ConvLaunch* L) {
-    ConvArgs& a = L->a;
-    conv_bx::Args& b = L->bx;
-    std::memset(&b, 0, sizeof(b));
-    b.N = a.N; b.C = a.C; b.H = a.H; b.W = a.W; b.O = a.O; b.OH = a.OH; b.OW = a.OW; b.KH = desc->kh; b.KW = desc->kw;
-    b.sh = a.sh; b.sw = a.sw; b.ph = a.ph; b.pw = a.pw; b.dh = a.dh; b.dw = a.dw;
-    b.Hp = a.Hp; b.Wp = a.Wp; b.Hv = a.Hv; b.row_step = a.row_step; b.M = a.M; b.OHW = a.OHW;
-    b.chs = c.chs; b.cb = c.cb; b.nq = c.nq; b.nq_main = c.nq_main; b.group_steps = c.group_steps; b.ngroups = c.ngroups;
-    b.nchunks = c.v->c4 ? 1 : (a.C + 8 * c.cb - 1) / (8 * c.cb);
-    if (second) {
-        int rh = 0, rw = 0;
-        KXC_HIP_REQUIRE(PairTap(desc, &rh, &rw), "%s: no kernel with a second output covers this shape", who);
-        b.ds_off = rh * a.dh * a.Wp + rw * a.dw;
-        b.w2_bytes = static_cast<uint32_t>(static_cast<int64_t>(a.O) * a.C * 4);
-    }
-    b.p_tiles = static_cast<int32_t>(CeilDiv(a.M, c.v->tp));
-    b.o_tiles = static_cast<int32_t>(CeilDiv(a.O, c.v->to));
-    const int64_t tiles = static_cast<int64_t>(b.p_tiles) * b.o_tiles;
-    KXC_HIP_REQUIRE(tiles < (1LL << 30), "%s: too many tiles", who);
-    b.num_tiles = static_cast<int32_t>(tiles);
-    b.out_elems = L->total;
-    const int split = BxSplit(c, b.nchunks, tiles, L->total * (second ? 2 : 1));
-    b.cps = static_cast<int32_t>(CeilDiv(b.nchunks, split));
-    b.gsplit = static_cast<int32_t>(CeilDiv(b.nchunks, b.cps));      // no empty part
-    a.gsplit = b.gsplit;
-    if (b.gsplit > 1) L->scratch_bytes = static_cast<size_t>(b.gsplit) * L->total * sizeof(float) * (second ? 2 : 1);
-    b.tiles_per_xcd = static_cast<int32_t>(CeilDiv(tiles * b.gsplit, 8));
-    b.x_bytes = a.x_bytes; b.w_bytes = a.w_bytes; b.flags = a.flags;
-    b.div_wp = MakeFastDiv(a.Wp); b.div_hp = MakeFastDiv(a.Hp); b.div_ohw = MakeFastDiv(a.OHW); b.div_ow = MakeFastDiv(a.OW);
-    a.div_ohw = b.div_ohw;
-    b.div_otiles = MakeFastDiv(b.o_tiles); b.div_ptiles = MakeFastDiv(b.p_tiles); b.div_gsplit = MakeFastDiv(b.gsplit);
-    b.div_chs = MakeFastDiv(b.chs); b.div_gq = MakeFastDiv(2 * b.group_steps); b.div_cb = MakeFastDiv(b.cb); b.div_kw = MakeFastDiv(b.KW);
-    b.o_fastest = static_cast<int64_t>(a.w_bytes) <= (2 << 20) ? 1 : 0;
-    L->path = ConvLaunch::kBf16x3;
-    L->bx_kernel = second ? c.v->ds_kernel : c.v->kernel;
-    L->name = BxName(*c.v, desc->kh, desc->kw);
-    L->grid = dim3(static_cast<unsigned>(b.tiles_per_xcd * 8));
-    L->block = dim3(static_cast<unsigned>(c.v->threads));
-    L->lds_bytes = c.lds_bytes;
-    return KXC_HIP_OK;
-}
-
-int32_t Conv2dResolve(const kxc_hip_conv2d_desc* desc, bool second, const char* who, ConvLaunch* L) {
+// small = false: without the small-launch kernels (operands that are not aligned for them).
+int32_t Conv2dResolve(const kxc_hip_conv2d_desc* desc, bool second, const char* who, ConvLaunch* L, bool in_plan = false, bool small = true) {
     ConvArgs& a = L->a;
     if (int32_t rc = FillArgs(desc, &a, who)) return rc;
     L->second = second;
+    L->desc = *desc;
     L->kh = desc->kh; L->kw = desc->kw;
     L->total = static_cast<int64_t>(a.N) * a.O * a.OHW;
     if (L->total == 0) { L->path = ConvLaunch::kEmpty; return KXC_HIP_OK; }
@@ -1310,6 +1240,35 @@ int32_t Conv2dResolve(const kxc_hip_conv2d_desc* desc, bool second, const char* 
     // downsample convolutions): the matrix kernel then sees an image of OH rows that are stride rows apart, so
     // the skipped rows are neither loaded nor staged.
     const bool hpool = (desc->flags & KXC_HIP_CONV_HPOOL) != 0;
+    if (const SmallVariant* v = small ? SelectSmall(desc, a, second, in_plan) : nullptr) {
+        conv_small::Args& b = L->sm;
+        std::memset(&b, 0, sizeof(b));
+        b.N = a.N; b.C = a.C; b.H = a.H; b.W = a.W; b.O = a.O; b.OH = a.OH; b.OW = a.OW;
+        b.sh = a.sh; b.sw = a.sw; b.ph = a.ph; b.pw = a.pw; b.dh = a.dh; b.dw = a.dw;
+        b.M = a.M; b.OHW = a.OHW; b.nchunks = a.C / v->chunk;
+        if (v->xi > 0) {
+            b.words = SmallWords(*v, a);
+            b.image_tiles = static_cast<int32_t>(CeilDiv(a.OHW, 16));
+            b.div_image = MakeFastDiv(b.image_tiles); b.div_words = MakeFastDiv(b.words);
+            b.p_tiles = a.N * b.image_tiles;
+        } else {
+            b.p_tiles = static_cast<int32_t>(CeilDiv(a.M, 16));
+        }
+        b.o_tiles = static_cast<int32_t>(CeilDiv(a.O, 16 * v->ro));
+        b.num_tiles = b.p_tiles * b.o_tiles;
+        b.tiles_per_xcd = (b.num_tiles + 7) / 8;
+        b.x_bytes = a.x_bytes; b.w_bytes = a.w_bytes; b.w2_bytes = static_cast<uint32_t>(static_cast<int64_t>(a.O) * a.C * 4); b.flags = a.flags;
+        b.o_fastest = a.x_bytes > a.w_bytes ? 1 : 0;       // an XCD's run of tiles shares the larger operand
+        b.div_ow = MakeFastDiv(a.OW); b.div_tiles = MakeFastDiv(b.o_fastest ? b.o_tiles : b.p_tiles);
+        b.div_ohw = MakeFastDiv(a.OHW);
+        L->path = ConvLaunch::kSmall;
+        L->small_kernel = second ? v->ds_kernel : v->kernel;
+        L->name = v->name;
+        L->grid = dim3(static_cast<unsigned>(b.tiles_per_xcd * 8));
+        L->block = dim3(static_cast<unsigned>(64 * v->ks));
+        L->lds_bytes = static_cast<size_t>(v->ks) * ((v->wi + v->xi) * 1024 + (v->xi > 0 ? 32 : 0));
+        return KXC_HIP_OK;
+    }
     if (!second && !hpool && UseSmall1x1(desc, a)) {
         a.div_ohw = MakeFastDiv(a.OHW); a.div_ow = MakeFastDiv(a.OW);
         L->path = ConvLaunch::kSmall1x1;
@@ -1328,9 +1287,6 @@ int32_t Conv2dResolve(const kxc_hip_conv2d_desc* desc, bool second, const char* 
     }
     L->direct_args = a;
     ApplyRowView(&a, desc->kh);
-    BxChoice bc;
-    BxSelect(a, desc, second, &bc);
-    if (bc.v) return BxResolve(desc, second, who, bc, L);
     Choice c;
     if (hpool) {
         KXC_HIP_REQUIRE(!second && HpoolChoice(desc, a, &c), "%s: no kernel with the pooling epilogue covers this shape", who);
@@ -1430,6 +1386,22 @@ int32_t Conv2dLaunch(const ConvLaunch& L, const char* who, const float* x, const
         KXC_HIP_REQUIRE(second->w2 && second->y2, "%s: NULL pointer", who);
         a.w2 = second->w2; a.bias2 = second->bias2; a.y2 = second->y2;
     }
+    if (L.path == ConvLaunch::kSmall) {
+        if (((reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(second ? second->w2 : w)) & 15u) != 0) {
+            ConvLaunch other;       // weights are read in 16-byte words
+            if (int32_t rc = Conv2dResolve(&L.desc, L.second, who, &other, false, false)) return rc;
+            return Conv2dLaunch(other, who, x, w, bias, residual, y, stream, no_alloc, second);
+        }
+        conv_small::Args b = L.sm;
+        b.x = x; b.w = w; b.bias = bias; b.res = residual; b.y = y;
+        b.w2 = a.w2; b.bias2 = a.bias2; b.y2 = a.y2;
+        b.delta = static_cast<int32_t>(reinterpret_cast<uintptr_t>(x) & 15u) / 4;
+        if (b.words > 0) b.x_bytes = (b.x_bytes + static_cast<uint32_t>(b.delta) * 4u + 15u) & ~15u;      // (whole words: no page ends within one)
+        if (L.lds_bytes > 64 * 1024)
+            if (int32_t rc = GrantLds(reinterpret_cast<const void*>(L.small_kernel))) return rc;
+        hipLaunchKernelGGL(L.small_kernel, NoteGrid(L.grid), NoteBlock(L.block), NoteLds(L.lds_bytes), s, b);
+        return CheckLaunch(L.name);
+    }
     SplitScratchLease lease;      // held until the adding kernel is enqueued
     if (L.scratch_bytes > 0) {
         if (no_alloc) {
@@ -1444,15 +1416,8 @@ int32_t Conv2dLaunch(const ConvLaunch& L, const char* who, const float* x, const
         }
     }
     if (L.lds_bytes > 64 * 1024)
-        if (int32_t rc = GrantLds(L.path == ConvLaunch::kBf16x3 ? reinterpret_cast<const void*>(L.bx_kernel) : reinterpret_cast<const void*>(L.kernel))) return rc;
-    if (L.path == ConvLaunch::kBf16x3) {
-        conv_bx::Args b = L.bx;
-        b.x = x; b.w = w; b.bias = bias; b.res = residual; b.y = y; b.partial = a.partial;
-        b.w2 = a.w2; b.bias2 = a.bias2; b.y2 = a.y2;
-        hipLaunchKernelGGL(L.bx_kernel, NoteGrid(L.grid), NoteBlock(L.block), NoteLds(L.lds_bytes), s, b);
-    } else {
-        hipLaunchKernelGGL(L.kernel, NoteGrid(L.grid), NoteBlock(L.block), NoteLds(L.lds_bytes), s, a);
-    }
+        if (int32_t rc = GrantLds(reinterpret_cast<const void*>(L.kernel))) return rc;
+    hipLaunchKernelGGL(L.kernel, NoteGrid(L.grid), NoteBlock(L.block), NoteLds(L.lds_bytes), s, a);
     if (int32_t rc = CheckLaunch(L.name)) return rc;
     if (a.gsplit > 1) {
         SplitReduceArgs r;
@@ -1487,7 +1452,7 @@ struct PreparedConv {
 int32_t PrepareConv2d(const kxc_hip_conv2d_desc* desc, bool second_output, PreparedConv** out) {
     std::unique_ptr<PreparedConv> p(new PreparedConv);
     p->who = second_output ? "kxc_hip_conv2d_pair_nchw_f32 (plan node)" : "kxc_hip_conv2d_nchw_f32 (plan node)";
-    if (int32_t rc = Conv2dResolve(desc, second_output, p->who.c_str(), &p->launch)) return rc;
+    if (int32_t rc = Conv2dResolve(desc, second_output, p->who.c_str(), &p->launch, true)) return rc;
     *out = p.release();
     return KXC_HIP_OK;
 }
@@ -1500,6 +1465,16 @@ int32_t LaunchPreparedConv2d(const PreparedConv* p, const float* x, const float*
 }
 
 const char* PreparedConvName(const PreparedConv* p) { return p->launch.name; }
+
+// Against the Winograd kernel with its adding launch (us, residual and ReLU): 64 channels at 56 x 56 batch 1 10.2 -> 8.7, batch 2
+// (1568 tiles) 12.9 against 14.6; 128 at 28 x 28 batch 2 13.0 -> 12.0; 256 at 14 x 14 batch 1 10.7 -> 7.5, batch 2 13.0 -> 11.2,
+// batch 4 (tiles * k = 1.8 M) equal; 512 at 7 x 7 batch 2 (1.03 M) 13.9 -> 11.6, batch 4 equal.
+bool SmallConvBeatsWinograd(const kxc_hip_conv2d_desc* d) {
+    const char* variant = std::getenv("KXC_HIP_WINOGRAD_VARIANT");
+    ConvArgs a;
+    if ((variant && *variant) || std::getenv("KXC_HIP_WINOGRAD_GSPLIT") || FillArgs(d, &a, "plan") != KXC_HIP_OK) return false;
+    return SelectSmall(d, a, false, true) && CeilDiv(a.M, 16) * CeilDiv(a.O, 16) * SelectLanes() * a.C * 9 <= 1100000;
+}
 
 void FreePreparedConv(PreparedConv* p) { delete p; }
 
@@ -1515,11 +1490,9 @@ const char* kxc_hip_conv2d_variant(const kxc_hip_conv2d_desc* desc) {
         return HpoolChoice(desc, a, &hp) ? hp.v->name : "unsupported";
     }
     if (desc->flags & KXC_HIP_CONV_FORCE_DIRECT) return "direct";
+    if (const SmallVariant* v = SelectSmall(desc, a, false, false)) return v->name;
     if (UseSmall1x1(desc, a)) return "mfma_k1x1_small";
     ApplyRowView(&a, desc->kh);
-    BxChoice bc;
-    BxSelect(a, desc, false, &bc);
-    if (bc.v) return BxName(*bc.v, desc->kh, desc->kw);
     Choice c;
     Select(a, desc->kh, desc->kw, &c);
     return c.v ? c.v->name : "direct";
@@ -1604,16 +1577,8 @@ int32_t kxc_hip_conv2d_scratch_needed(const kxc_hip_conv2d_desc* desc, size_t* o
     ConvArgs a;
     if (int32_t rc = FillArgs(desc, &a, "kxc_hip_conv2d_scratch_needed")) return rc;
     const int64_t total = static_cast<int64_t>(a.N) * a.O * a.OHW;
-    if (total == 0 || (desc->flags & (KXC_HIP_CONV_FORCE_DIRECT | KXC_HIP_CONV_HPOOL)) || UseSmall1x1(desc, a) || a.M <= 0) return KXC_HIP_OK;
+    if (total == 0 || (desc->flags & (KXC_HIP_CONV_FORCE_DIRECT | KXC_HIP_CONV_HPOOL)) || SelectSmall(desc, a, false, false) || UseSmall1x1(desc, a) || a.M <= 0) return KXC_HIP_OK;
     ApplyRowView(&a, desc->kh);
-    BxChoice bc;
-    BxSelect(a, desc, false, &bc);
-    if (bc.v) {
-        ConvLaunch L;
-        if (int32_t rc = Conv2dResolve(desc, false, "kxc_hip_conv2d_scratch_needed", &L)) return rc;
-        *out_bytes = L.scratch_bytes;
-        return KXC_HIP_OK;
-    }
     Choice c;
     Select(a, desc->kh, desc->kw, &c);
     if (!c.v) return KXC_HIP_OK;

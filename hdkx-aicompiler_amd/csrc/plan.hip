@@ -788,16 +788,11 @@ int32_t kxc_hip_plan_finalize(kxc_hip_plan* plan, size_t workspace_bytes) {
     for (Node& n : plan->nodes) {
         if (n.kind != NodeKind::kConv2D) continue;
         KXC_HIP_CALL(hipSetDevice(plan->device_id), "HIP SetDevice");
-        {
-            const std::string prefix = "kxc_conv2d_nchw_f32.";
-            const char* variant = n.i32[0] == 1   ? kxc_hip_conv2d_winograd_variant(&n.conv)
-                                  : n.i32[0] == 2 ? kxc_hip_conv2d_pair_variant(&n.conv)
-                                                  : kxc_hip_conv2d_variant(&n.conv);
-            const size_t end = n.symbol.find_first_of("+|", prefix.size());
-            if (n.symbol.compare(0, prefix.size(), prefix) == 0)
-                n.symbol = prefix + variant + (end == std::string::npos ? std::string() : n.symbol.substr(end));
-        }
-        if (n.i32[0] == 1) {
+        const char* variant = n.i32[0] == 1   ? kxc_hip_conv2d_winograd_variant(&n.conv)
+                              : n.i32[0] == 2 ? kxc_hip_conv2d_pair_variant(&n.conv)
+                                              : kxc_hip_conv2d_variant(&n.conv);
+        // (a small Winograd node runs on its weights as they are, in one launch)
+        if (n.i32[0] == 1 && !kxc_hip::SmallConvBeatsWinograd(&n.conv)) {
             kxc_hip::PreparedWinograd* p = nullptr;
             if (int32_t rc = kxc_hip::PrepareWinograd(&n.conv, &p)) return rc;
             n.prepared_wino.reset(p, kxc_hip::FreePreparedWinograd);
@@ -805,7 +800,12 @@ int32_t kxc_hip_plan_finalize(kxc_hip_plan* plan, size_t workspace_bytes) {
             kxc_hip::PreparedConv* p = nullptr;
             if (int32_t rc = kxc_hip::PrepareConv2d(&n.conv, n.i32[0] == 2, &p)) return rc;
             n.prepared_conv.reset(p, kxc_hip::FreePreparedConv);
+            if (std::strstr(kxc_hip::PreparedConvName(p), "_small")) variant = kxc_hip::PreparedConvName(p);
         }
+        const std::string prefix = "kxc_conv2d_nchw_f32.";
+        const size_t end = n.symbol.find_first_of("+|", prefix.size());
+        if (n.symbol.compare(0, prefix.size(), prefix) == 0)
+            n.symbol = prefix + variant + (end == std::string::npos ? std::string() : n.symbol.substr(end));
     }
     // Streams, events and the workspace: what a failed call has created so far is kept by the plan and reused by a
     // second call (kxc_hip_plan_destroy releases it either way).
@@ -859,7 +859,7 @@ int32_t TransformConstants(kxc_hip_plan* plan, void** args, hipStream_t stream, 
     std::vector<WinoWeightJob> jobs;
     std::vector<std::pair<Node*, const void*>> touched;
     for (Node& n : plan->nodes) {
-        if (n.kind != NodeKind::kConv2D || n.i32[0] != 1) continue;
+        if (!n.prepared_wino) continue;
         const void* w = Resolve(plan, n.bufs[1], args);
         if (only_changed && n.transformed_from == w) continue;
         touched.emplace_back(&n, w);
@@ -919,7 +919,7 @@ int32_t RunNode(kxc_hip_plan* plan, Node& n, void** args, void* s) {
         switch (n.kind) {
             case NodeKind::kConv2D:
                 // (launches resolved at finalize; s is never NULL here)
-                if (n.i32[0] == 1) {
+                if (n.prepared_wino) {
                     // (the transformed weights in B(5) were written by TransformConstants at the start of the run)
                     rc = kxc_hip::LaunchPreparedWinograd(n.prepared_wino.get(), static_cast<const float*>(B(0)),
                                                          static_cast<const float*>(B(5)), static_cast<const float*>(B(2)),

@@ -693,6 +693,58 @@ def test_conv1x1_small_launch_kernel(pkg, fast_orc, orc, synth, shape):
                      orc.conv_chain(xi, wi, None, stride, 0, None, False), "1x1 small on small integers")
 
 
+@pytest.mark.parametrize("shape", [
+    # n, c, h, w, o, k, stride, pad, dilation, kernel: staged rows (one pixel tile, tiles across rows of 1 to 14 pixels, runs that
+    # start off a 16-byte boundary, windows partly and wholly in the padding), rows that are too wide to stage, more than
+    # 256 tiles; ragged output channels everywhere; 1x1 with two and four blocks of output channels
+    (1, 64, 1, 1, 16, 3, 1, 1, 1, "k3x3_small_rows"), (2, 80, 9, 13, 40, 3, 2, 1, 1, "k3x3_small_rows"), (3, 112, 7, 7, 33, 3, 1, 1, 1, "k3x3_small_rows"),
+    (1, 64, 5, 6, 70, 3, 1, 0, 1, "k3x3_small_rows"), (1, 64, 6, 5, 32, 3, 3, 3, 1, "k3x3_small_rows"), (1, 64, 9, 9, 40, 3, 1, 2, 2, "k3x3_small_o1"),
+    (1, 64, 20, 60, 47, 3, 1, 1, 1, "k3x3_small_o1"), (2, 64, 31, 30, 72, 3, 1, 1, 1, "k3x3_small_o2"), (5, 96, 27, 29, 50, 3, 2, 1, 1, "k3x3_small_o2"),
+    (1, 16, 1, 1, 32, 1, 1, 0, 1, "k1x1_small"), (3, 48, 11, 13, 33, 1, 2, 1, 1, "k1x1_small"), (3, 96, 61, 59, 190, 1, 1, 0, 1, "k1x1_small"),
+], ids=lambda s: "x".join(map(str, s)))
+def test_conv_small_launch_kernels(pkg, orc, fast_orc, synth, shape):
+    """The one-launch kernels of small convolutions as a plan runs them (and, with a stride and padding that allow it, with the
+    second output), on tensors that start off a 16-byte boundary too: against the CPU path, and bit for bit on small
+    integers, whose sums are exact in any order."""
+    n, c, h, w, o, k, s, p, dil, kernel = shape
+    rng = np.random.default_rng(hash(shape[:9]) % (2 ** 31))
+    oh, ow = (h + 2 * p - dil * (k - 1) - 1) // s + 1, (w + 2 * p - dil * (k - 1) - 1) // s + 1
+    d = pkg.ConvDesc(n, c, h, w, o, k, k, s, s, p, p, dil, dil, pkg.CONV_BIAS | pkg.CONV_RESIDUAL | pkg.CONV_RELU)
+    plan = pkg.Plan(5)
+    plan.add_conv2d(d, *[pkg.Buf.arg(i) for i in range(5)])
+    plan.finalize(0)
+    assert plan.node_symbol(0).startswith("kxc_conv2d_nchw_f32.mfma_%s+" % kernel), plan.node_symbol(0)
+    pair = k == 3 and dil == 1 and p == 1
+
+    def shifted(a, by):      # the same values in a tensor that starts `by` floats behind an allocation
+        t = torch.zeros(a.size + 4, device="cuda")
+        t[by:by + a.size] = torch.from_numpy(np.ascontiguousarray(a).reshape(-1)).cuda()
+        return t[by:by + a.size].view(a.shape)
+
+    for exact in (False, True):
+        if exact:
+            x, wt, b, r, w2 = (rng.integers(-3, 4, sh).astype(np.float32) for sh in ((n, c, h, w), (o, c, k, k), (o,), (n, o, oh, ow), (o, c, 1, 1)))
+            check = lambda got, want, what: assert_bit_exact(got, want, what)
+        else:
+            x, r, b = (rng.uniform(-1, 1, sh).astype(np.float32) for sh in ((n, c, h, w), (n, o, oh, ow), (o,)))
+            wt, w2 = ((rng.standard_normal(sh) * np.sqrt(2.0 / (c * sh[2] ** 2))).astype(np.float32) for sh in ((o, c, k, k), (o, c, 1, 1)))
+            check = lambda got, want, what: assert_close(got, want, what=what)
+        conv = orc.conv2d(x, wt, s, p, dil)
+        want = np.maximum(conv + b[None, :, None, None] + r, 0.0).astype(np.float32)
+        for dx, dw in ((0, 0), (1, 0), (3, 0), (0, 1)):
+            y = torch.full((n, o, oh, ow), float("nan"), device="cuda")
+            plan.run([shifted(x, dx), shifted(wt, dw), dev(b), dev(r), y]); torch.cuda.synchronize()
+            check(host(y), want, "%s, x + %d, w + %d" % (shape, dx, dw))
+        if pair and pkg.conv2d_pair_supported(x.shape, wt.shape, s, p):
+            both = pkg.Plan(8)
+            both.add_conv2d_pair(d, *[pkg.Buf.arg(i) for i in range(8)])
+            both.finalize(0)
+            y, y2 = (torch.full((n, o, oh, ow), float("nan"), device="cuda") for _ in range(2))
+            both.run([dev(x), dev(wt), dev(b), dev(r), y, dev(w2), dev(b), y2]); torch.cuda.synchronize()
+            check(host(y), want, "first output %s" % (shape,))
+            check(host(y2), (orc.conv2d(x, w2, s, 0) + b[None, :, None, None]).astype(np.float32), "second output %s" % (shape,))
+
+
 def test_conv_dilation(pkg, orc, synth):
     x = synth.uniform((1, 8, 20, 20), 300); w = synth.uniform((32, 8, 3, 3), 301)
     want = orc.conv2d(x, w, 1, 2, 2)
