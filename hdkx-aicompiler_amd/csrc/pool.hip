@@ -51,16 +51,21 @@ __global__ void __launch_bounds__(kBlock) pool_generic_kernel(const float* __res
 }
 
 // ---------------------------------------------------------------- max 3x3 / stride 2 / pad 1
-// Requirements (checked on the host): W % 8 == 0, OW == W/2, OH == H/2 (H even), 16-byte aligned
-// planes.  One thread produces a 4-wide strip of ROWS consecutive output rows.  Per input row it
-// issues two aligned 16-byte loads (columns 2*ow0 .. 2*ow0+7); the ninth value, column 2*ow0-1,
+// One thread produces a 4-wide strip of ROWS consecutive output rows.  Per input row it
+// issues two 16-byte loads (columns 2*ow0 .. 2*ow0+7); the ninth value, column 2*ow0-1,
 // is the left neighbour lane's last element, taken with a lane shuffle (a scalar reload only for
 // the first lane of a wave).  Consecutive lanes read consecutive 32-byte pieces of a row, every
 // input element is requested once per strip (plus the one shared row between vertical strips).
-template <int ROWS>
+// ALIGNED (checked on the host): W % 8 == 0, OW == W/2, OH == H/2 (H even), 16-byte aligned planes.
+// Otherwise any extent: the same loads on 4-byte boundaries, columns past the row replaced by the padding value, single
+// elements where a load would pass the end of the tensor (64 channels at 97 x 97, batch 6: 9.8 us one thread per output with
+// nine loads, 5.9 here).
+struct __attribute__((packed, aligned(4))) Float4U { float x, y, z, w; };
+template <int ROWS, bool ALIGNED>
 __global__ void __launch_bounds__(kBlock) maxpool3x3s2_kernel(const float* __restrict__ x, float* __restrict__ y,
                                                               int32_t h, int32_t w, int32_t oh_total, int32_t ow_total,
-                                                              int32_t col_groups, int32_t row_groups, int64_t total) {
+                                                              int32_t col_groups, int32_t row_groups, int64_t planes,
+                                                              int64_t total) {
     const int64_t tid = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
     const bool active = tid < total;
     const int64_t t = active ? tid : total - 1;
@@ -69,6 +74,7 @@ __global__ void __launch_bounds__(kBlock) maxpool3x3s2_kernel(const float* __res
     const int32_t rg = static_cast<int32_t>(t2 % row_groups);
     const int64_t plane = t2 / row_groups;
     const float* xp = x + plane * h * w;
+    const int64_t left_in_tensor = (planes - plane) * h * w;
     float* yp = y + plane * oh_total * ow_total;
     const int32_t oh0 = rg * ROWS;
     const int32_t iw0 = cg * 8;
@@ -85,13 +91,26 @@ __global__ void __launch_bounds__(kBlock) maxpool3x3s2_kernel(const float* __res
             for (int j = 0; j < 9; ++j) v[j] = kPadValue;
             return;
         }
-        const float4 a = *reinterpret_cast<const float4*>(xp + static_cast<int64_t>(ih) * w + iw0);
-        const float4 b = *reinterpret_cast<const float4*>(xp + static_cast<int64_t>(ih) * w + iw0 + 4);
-        v[1] = a.x; v[2] = a.y; v[3] = a.z; v[4] = a.w;
-        v[5] = b.x; v[6] = b.y; v[7] = b.z; v[8] = b.w;
-        float left = __shfl_up(b.w, 1, 64);                      // neighbour lane's column iw0-1
+        const float* const row = xp + static_cast<int64_t>(ih) * w;
+        if constexpr (ALIGNED) {
+            const float4 a = *reinterpret_cast<const float4*>(row + iw0);
+            const float4 b = *reinterpret_cast<const float4*>(row + iw0 + 4);
+            v[1] = a.x; v[2] = a.y; v[3] = a.z; v[4] = a.w;
+            v[5] = b.x; v[6] = b.y; v[7] = b.z; v[8] = b.w;
+        } else if (iw0 + 8 <= left_in_tensor - static_cast<int64_t>(ih) * w) {
+            const Float4U a = *reinterpret_cast<const Float4U*>(row + iw0);
+            const Float4U b = *reinterpret_cast<const Float4U*>(row + iw0 + 4);
+            v[1] = a.x; v[2] = a.y; v[3] = a.z; v[4] = a.w;
+            v[5] = b.x; v[6] = b.y; v[7] = b.z; v[8] = b.w;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[1 + j] = iw0 + j < w ? v[1 + j] : kPadValue;
+        } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[1 + j] = iw0 + j < w ? row[iw0 + j] : kPadValue;
+        }
+        float left = __shfl_up(v[8], 1, 64);                     // neighbour lane's column iw0-1
         if (cg == 0) left = kPadValue;                           // column -1 is padding
-        else if (lane == 0) left = xp[static_cast<int64_t>(ih) * w + iw0 - 1];
+        else if (lane == 0) left = ALIGNED || iw0 - 1 < w ? row[iw0 - 1] : kPadValue;
         v[0] = left;
     };
 
@@ -119,8 +138,16 @@ __global__ void __launch_bounds__(kBlock) maxpool3x3s2_kernel(const float* __res
             out[k] = acc;
         }
         if (active && oh < oh_total) {
-            *reinterpret_cast<float4*>(yp + static_cast<int64_t>(oh) * ow_total + cg * 4) =
-                make_float4(out[0], out[1], out[2], out[3]);
+            float* const dst = yp + static_cast<int64_t>(oh) * ow_total + cg * 4;
+            if constexpr (ALIGNED) {
+                *reinterpret_cast<float4*>(dst) = make_float4(out[0], out[1], out[2], out[3]);
+            } else if (cg * 4 + 4 <= ow_total) {
+                *reinterpret_cast<Float4U*>(dst) = Float4U{out[0], out[1], out[2], out[3]};
+            } else {
+#pragma unroll
+                for (int k = 0; k < 3; ++k)
+                    if (cg * 4 + k < ow_total) dst[k] = out[k];
+            }
         }
 #pragma unroll
         for (int j = 0; j < 9; ++j) prev_row_vals[j] = rows[2][j];
@@ -204,18 +231,45 @@ __global__ void __launch_bounds__(kGapThreads) gap_lds_kernel(const float* __res
     }
 }
 
-// Large planes: one thread per plane would serialise; use one wave per plane with a strided
-// partial sum and a wave reduction (order differs from the CPU loop; within fp32 tolerance).
-__global__ void __launch_bounds__(64) gap_wave_kernel(const float* __restrict__ x, float* __restrict__ y,
-                                                      int64_t planes, int64_t hw) {
+// Large planes: WAVES waves per plane, partial sums and a wave reduction (order differs from the CPU loop; within fp32
+// tolerance).  Bound by HBM once enough loads are in flight: a lane issues kGapLoads, 16 bytes each where the planes are
+// whole 16-byte words, before it adds the first (4096 planes of 56 x 56, 51 MB: 17.7 us with one 4-byte load at a time, 8.9 =
+// 5.8 TB/s here).
+constexpr int kGapLoads = 8;
+template <int WAVES, int VEC>
+__global__ void __launch_bounds__(64 * WAVES) gap_wave_kernel(const float* __restrict__ x, float* __restrict__ y, int64_t hw) {
+    typedef float vec_t __attribute__((ext_vector_type(VEC)));
     const int64_t plane = blockIdx.x;
-    if (plane >= planes) return;
-    const float* src = x + plane * hw;
-    float acc = 0.0f;
-    for (int64_t i = threadIdx.x; i < hw; i += 64) acc += src[i];
+    const float* const src = x + plane * hw;
+    const int64_t words = hw / VEC;
+    const int32_t tid = static_cast<int32_t>(threadIdx.x);
+    float acc[VEC] = {};
+    for (int64_t i = tid; i < words; i += 64 * WAVES * kGapLoads) {
+        vec_t v[kGapLoads];
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);
-    if (threadIdx.x == 0) y[plane] = __fdiv_rn(acc, static_cast<float>(hw));
+        for (int k = 0; k < kGapLoads; ++k) {
+            const int64_t at = i + k * 64 * WAVES;
+            v[k] = at < words ? *reinterpret_cast<const vec_t*>(src + at * VEC) : vec_t(0.0f);
+        }
+#pragma unroll
+        for (int k = 0; k < kGapLoads; ++k)
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) acc[e] = __fadd_rn(acc[e], v[k][e]);
+    }
+    float sum = acc[0];
+#pragma unroll
+    for (int e = 1; e < VEC; ++e) sum = __fadd_rn(sum, acc[e]);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) sum += __shfl_down(sum, off, 64);
+    if constexpr (WAVES > 1) {
+        __shared__ float part[WAVES];
+        if ((tid & 63) == 0) part[tid >> 6] = sum;
+        __syncthreads();
+        sum = part[0];
+#pragma unroll
+        for (int k = 1; k < WAVES; ++k) sum = __fadd_rn(sum, part[k]);
+    }
+    if (tid == 0) y[plane] = __fdiv_rn(sum, static_cast<float>(hw));
 }
 
 // ---------------------------------------------------------------- int8
@@ -294,26 +348,23 @@ int32_t kxc_hip_pool2d_f32(const kxc_hip_pool2d_desc* desc, const float* x, floa
     if (total == 0) return KXC_HIP_OK;
     KXC_HIP_REQUIRE(x && y, "kxc_hip_pool2d_f32: NULL pointer");
     hipStream_t s = ResolveStream(stream);
-    const bool fast = !desc->is_avg && d.kh == 3 && d.kw == 3 && d.sh == 2 && d.sw == 2 && d.pt == 1 && d.pl == 1 &&
-                      desc->pad_bottom == 1 && desc->pad_right == 1 && !desc->ceil_mode && (d.w % 8) == 0 &&
-                      (d.h % 2) == 0 && d.ow == d.w / 2 && d.oh == d.h / 2 &&
-                      (reinterpret_cast<uintptr_t>(x) & 15u) == 0 && (reinterpret_cast<uintptr_t>(y) & 15u) == 0;
-    if (fast) {
+    if (!desc->is_avg && d.kh == 3 && d.kw == 3 && d.sh == 2 && d.sw == 2 && d.pt == 1 && d.pl == 1) {
+        const bool aligned = desc->pad_bottom == 1 && desc->pad_right == 1 && !desc->ceil_mode && (d.w % 8) == 0 &&
+                             (d.h % 2) == 0 && d.ow == d.w / 2 && d.oh == d.h / 2 &&
+                             (reinterpret_cast<uintptr_t>(x) & 15u) == 0 && (reinterpret_cast<uintptr_t>(y) & 15u) == 0;
         // four output rows per thread share input rows between them; a launch too small to give every compute
         // unit a workgroup that way (batch 1) takes one row per thread and four times the threads instead
-        const int32_t col_groups = d.ow / 4;
+        const int32_t col_groups = (d.ow + 3) / 4;
         const bool small = planes * ((d.oh + 3) / 4) * col_groups < 256LL * kBlock;   // 256 compute units
         const int32_t rows = small ? 1 : 4;
         const int32_t row_groups = (d.oh + rows - 1) / rows;
         const int64_t threads = planes * row_groups * col_groups;
         const int64_t blocks = CeilDiv(threads, kBlock);
         KXC_HIP_REQUIRE(blocks <= kMaxGridX, "kxc_hip_pool2d_f32: tensor too large");
-        if (small)
-            maxpool3x3s2_kernel<1><<<NoteGrid(static_cast<int>(blocks)), NoteBlock(kBlock), NoteLds(0), s>>>(
-                x, y, d.h, d.w, d.oh, d.ow, col_groups, row_groups, threads);
-        else
-            maxpool3x3s2_kernel<4><<<NoteGrid(static_cast<int>(blocks)), NoteBlock(kBlock), NoteLds(0), s>>>(
-                x, y, d.h, d.w, d.oh, d.ow, col_groups, row_groups, threads);
+        auto* const kernel = small ? (aligned ? maxpool3x3s2_kernel<1, true> : maxpool3x3s2_kernel<1, false>)
+                                   : (aligned ? maxpool3x3s2_kernel<4, true> : maxpool3x3s2_kernel<4, false>);
+        kernel<<<NoteGrid(static_cast<int>(blocks)), NoteBlock(kBlock), NoteLds(0), s>>>(x, y, d.h, d.w, d.oh, d.ow, col_groups, row_groups,
+                                                                                         planes, threads);
         return CheckLaunch("maxpool3x3s2");
     }
     const bool columns = !desc->is_avg && d.kh == 3 && d.kw == 1 && d.sh == 2 && d.sw == 1 && d.pt == 1 && d.pl == 0 &&
@@ -358,7 +409,10 @@ int32_t kxc_hip_global_avg_pool2d_f32(const float* x, float* y, int64_t n, int64
         return CheckLaunch("global_avg_pool2d");
     }
     KXC_HIP_REQUIRE(planes <= kMaxGridX, "kxc_hip_global_avg_pool2d_f32: tensor too large");
-    gap_wave_kernel<<<NoteGrid(static_cast<int>(planes)), NoteBlock(64), NoteLds(0), s>>>(x, y, planes, hw);
+    const bool vec = hw % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
+    const bool few = planes < 2048;       // (fewer than eight waves per compute unit: four waves per plane)
+    auto* const kernel = few ? (vec ? gap_wave_kernel<4, 4> : gap_wave_kernel<4, 1>) : (vec ? gap_wave_kernel<1, 4> : gap_wave_kernel<1, 1>);
+    kernel<<<NoteGrid(static_cast<int>(planes)), NoteBlock(few ? 256 : 64), NoteLds(0), s>>>(x, y, hw);
     return CheckLaunch("global_avg_pool2d");
 }
 

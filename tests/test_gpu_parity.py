@@ -834,6 +834,33 @@ def test_maxpool_edge_semantics(pkg, orc):
         assert_bit_exact(host(pkg.pool2d(dev(x), k, s, p, avg=True)), orc.pool2d(x, k, s, p, avg=True), "avg")
 
 
+@pytest.mark.parametrize("shape", [(1, 1, 1, 1), (1, 2, 1, 9), (3, 2, 2, 3), (2, 3, 7, 7), (1, 2, 9, 15), (5, 7, 13, 17), (2, 64, 97, 97), (64, 33, 31, 40)])
+def test_maxpool_3x3s2_any_extent_bit_exact(pkg, fast_orc, shape):
+    """The row-reusing kernel on maps that are not whole 16-byte words: both row counts per thread (few and many planes),
+    the padding candidate, NaN, the last elements of the tensor, one row and column more by ceil_mode, an input that
+    starts on a 4-byte boundary."""
+    x = np.random.default_rng(sum(shape)).standard_normal(shape).astype(np.float32)
+    x.reshape(-1)[::11] = -3e30; x.reshape(-1)[5::97] = np.nan; x.reshape(-1)[-1] = 7.0
+    room = torch.empty(x.size + 1, device="cuda")
+    shifted = room[1:].view(shape)
+    shifted.copy_(dev(x))
+    for ceil in (False, True):
+        want = fast_orc.pool2d(x, 3, 2, 1, ceil_mode=ceil)
+        assert_bit_exact(host(pkg.pool2d(dev(x), 3, 2, 1, ceil_mode=ceil)), want, "3x3/2 %s ceil %d" % (shape, ceil))
+        assert_bit_exact(host(pkg.pool2d(shifted, 3, 2, 1, ceil_mode=ceil)), want, "3x3/2 %s ceil %d, 4-byte boundary" % (shape, ceil))
+
+
+@pytest.mark.parametrize("planes, h, w", [(3, 3, 43), (2050, 10, 13), (5, 14, 14), (2048, 16, 16), (7, 47, 51), (2100, 28, 28), (2, 128, 130), (1, 1, 4097)])
+def test_global_avg_pool_large_planes(pkg, planes, h, w):
+    """Planes above 128 elements against float64: one and four waves per plane, 4- and 16-byte loads.  A sum of hw terms
+    in chains of at most hw / 64 + 16 additions (and one division) is off by at most that many roundings of sum |x|."""
+    x = np.random.default_rng(planes + h * w).uniform(-1, 1, (1, planes, h, w)).astype(np.float32)
+    got = host(pkg.global_avg_pool2d(dev(x))).reshape(-1).astype(np.float64)
+    x64 = x.astype(np.float64).reshape(planes, -1)
+    bound = (h * w / 64 + 16) * 2.0 ** -24 * np.abs(x64).mean(axis=1)
+    assert (np.abs(got - x64.mean(axis=1)) <= bound).all()
+
+
 def test_column_maxpool_bit_exact(pkg, fast_orc, orc, synth):
     """The 3x1 window with stride (2,1) that finishes a 3x3/2 max pool whose column maxima were taken by the
     convolution before it: bit for bit against the CPU checker, on the first layer's half-width map (four rows per
