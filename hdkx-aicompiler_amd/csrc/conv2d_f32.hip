@@ -917,7 +917,11 @@ bool Fits(const Variant& v, const ConvArgs& a, Choice* out, bool ds = false) {
 // Picks the MFMA variant for a shape, or leaves choice.v == nullptr for the direct kernel.
 void Select(const ConvArgs& real, int kh, int kw, Choice* choice, bool ds = false) {
     choice->v = nullptr;
-    if (real.O < 32 || real.M < 32) return;
+    // Fewer than 32 channels or pixels leave part of a 32 x 32 block empty, and the block still wins against one thread per
+    // output with a serial sum unless that sum is short (us, one thread per output and here; 3x3 unless said): 156 -> 18
+    // channels at 20 x 97, batch 22 713 and 60; 5x5, 200 -> 31 at 33 x 35, batch 3 744 and 24; 7x7, 25 -> 24 at 25 x 20, batch 5
+    // 170 and 14; 73 -> 22 at 21 x 23, batch 2 109 and 15.  1x1, 37 -> 10 at 30 x 30: 13.3 and 15.2.
+    if ((real.O < 32 || real.M < 32) && (ds || static_cast<int64_t>(real.C) * kh * kw < 64)) return;
     // the rules below see the pixels of all launches expected to run side by side
     ConvArgs a = real;
     if (static_cast<int64_t>(a.M) * SelectLanes() < (1LL << 31)) a.M *= SelectLanes();
@@ -1172,7 +1176,8 @@ int SmallWords(const SmallVariant& v, const ConvArgs& a) {
 //   tiles per compute unit (64 -> 128 with stride 2, batch 16: 10.9 -> 9.2), two before (512 -> 128 at 14 x 14, batch 4: 5.9 against 6.8).
 // 3x3: up to 800 tiles of 16 x 16, 1600 with the second output (a launch plan's two-output node otherwise needs an adding launch
 //   for both): 128 channels at 28 x 28 12.5 -> 7.9 us at batch 1 (392 tiles), 17 -> 12 at batch 2 (784), equal at batch 4;
-//   128 -> 256 with stride 2 and the second output, batch 8 (1568): 28.9 -> 26.1.  At least 64 channels, a chunk per wave.
+//   128 -> 256 with stride 2 and the second output, batch 8 (1568): 28.9 -> 26.1.  Up to 1600 also for at most 16 output channels,
+//   half a block of the general tiles: 64 -> 16 at 56 x 56, batch 8 (1568) 25.9 -> 14.8.  At least 64 channels, a chunk per wave.
 //   Staged rows for narrow maps while every tile has a compute unit to itself (256 at 14 x 14, batch 1: 8.5 -> 7.5; 512 at 7 x
 //   7: 13.2 -> 10.9); two blocks of output channels from 257 tiles on (64 at 56 x 56, batch 1: 9.6 -> 8.7).
 //   Outside a plan, only from 400 tiles on: below, kxc_hip_conv2d_scratch_needed promises the callers of the single
@@ -1197,7 +1202,7 @@ const SmallVariant* SelectSmall(const kxc_hip_conv2d_desc* d, const ConvArgs& a,
             if (std::strcmp(forced, v[i].name) == 0) return v + i;
         return nullptr;
     }
-    if (a.C < 64 || tiles > (second ? 1600 : 800) || (!in_plan && tiles < 400)) return nullptr;
+    if (a.C < 64 || tiles > (second || a.O <= 16 ? 1600 : 800) || (!in_plan && tiles < 400)) return nullptr;
     if (rows_fit && a.N * CeilDiv(a.OHW, 16) * CeilDiv(a.O, 16) * SelectLanes() <= kNumCUs) return v;
     return tiles <= kNumCUs ? v + 1 : v + 2;
 }

@@ -784,6 +784,25 @@ def test_conv_full_batch_properties(pkg, synth):
 
 
 # ------------------------------------------------------------------ pooling / elementwise at full sizes
+@pytest.mark.parametrize("n, c, h, w, o, k, s, p", [
+    (1, 64, 9, 9, 1, 3, 1, 1), (2, 65, 8, 7, 17, 3, 1, 1), (1, 64, 13, 11, 31, 1, 1, 0), (3, 30, 12, 17, 5, 5, 1, 2), (2, 16, 19, 23, 16, 7, 2, 3),
+    (1, 7, 5, 5, 31, 3, 2, 1), (1, 96, 3, 3, 48, 3, 1, 1), (1, 72, 1, 1, 40, 3, 1, 1), (1, 50, 7, 4, 33, 5, 2, 2), (1, 63, 5, 6, 70, 1, 1, 0), (9, 64, 56, 50, 16, 3, 1, 1)])
+def test_conv_fewer_channels_or_pixels_than_a_block(pkg, n, c, h, w, o, k, s, p):
+    """Output channels or output pixels below the 32 of a matrix block (their rows and columns are masked; 63 terms and
+    fewer keep the kernel without blocks), residual and ReLU included."""
+    rng = np.random.default_rng(n * c + h * w + o)
+    x, wt = rng.standard_normal((n, c, h, w)).astype(np.float32), (rng.standard_normal((o, c, k, k)) / np.sqrt(c * k * k)).astype(np.float32)
+    b = rng.standard_normal(o).astype(np.float32)
+    res = rng.standard_normal((n, o, (h + 2 * p - k) // s + 1, (w + 2 * p - k) // s + 1)).astype(np.float32)
+    few = o < 32 or res[0, 0].size * n < 32
+    assert (pkg.conv2d_variant(x.shape, wt.shape, s, p) == "direct") == (few and c * k * k < 64 and not (k == 1 and c % 8 == 0))
+    got = host(pkg.conv2d(dev(x), dev(wt), dev(b), dev(res), s, p, 1, True))
+    want = torch.nn.functional.conv2d(*(torch.from_numpy(v).double() for v in (x, wt, b)), s, p).numpy() + res
+    # c k k products and sums of numbers of size 1 / sqrt(c k k), each rounded once, plus bias and residual
+    bound = (c * k * k + 4) * 2.0 ** -24 * (torch.nn.functional.conv2d(torch.from_numpy(np.abs(x)).double(), torch.from_numpy(np.abs(wt)).double(), None, s, p).numpy() + np.abs(res) + np.abs(b)[:, None, None])
+    assert (np.abs(got - np.maximum(want, 0)) <= bound).all()
+
+
 def test_maxpool_full_size_bit_exact(pkg, fast_orc, synth):
     x = synth.uniform((64, 64, 112, 112), 2000)
     xd = dev(x)
