@@ -249,9 +249,15 @@ def main():
     lb = dev(synth.uniform((64,), 4103, -0.1, 0.1))
     ly = torch.empty((batch, 64, 56, 56), device="cuda")
     conv_flop = 2.0 * batch * 64 * 56 * 56 * 64 * 9          # multiply-adds of the direct definition, x2
+    operator_winograd = os.environ.pop("KXC_HIP_CONV_WINOGRAD", None)
+    os.environ["KXC_HIP_CONV_WINOGRAD"] = "0"           # the single operator would take its Winograd kernel here
+    gemm_variant = pkg.conv2d_variant((batch, 64, 56, 56), (64, 64, 3, 3), 1, 1)
     gemm_ms = _event_time_ms(torch, lambda: pkg.conv2d(lx, lw, lb, None, 1, 1, 1, True, out=ly), 30, 5)
+    del os.environ["KXC_HIP_CONV_WINOGRAD"]
+    if operator_winograd is not None:
+        os.environ["KXC_HIP_CONV_WINOGRAD"] = operator_winograd
     gemm_tflops = conv_flop / (gemm_ms * 1e-3) / 1e12
-    gemm_row = {"kernel": "conv_mfma_kernel<3,3> (implicit GEMM)", "variant": pkg.conv2d_variant((batch, 64, 56, 56), (64, 64, 3, 3), 1, 1),
+    gemm_row = {"kernel": "conv_mfma_kernel<3,3> (implicit GEMM)", "variant": gemm_variant,
                 "avg_launch_ms": round(gemm_ms, 4), "achieved": round(gemm_tflops, 3), "frac": round(gemm_tflops / PEAK_FP32_MFMA_TFLOPS, 4),
                 "traffic": _profiled_traffic_bytes("conv3x3_layer1_bs64_counters.md") if batch == 64 else None}
     algorithmic_bytes = 4 * (2 * batch * 64 * 56 * 56 + 64 * 64 * 9 + 64)

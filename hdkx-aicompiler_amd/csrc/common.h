@@ -98,7 +98,9 @@ struct SplitScratchLease {
     uint32_t* counters = nullptr;      // kSplitCounters arrival counters, all zero between launches
     std::unique_lock<std::mutex> lock;
 };
-int32_t AcquireSplitScratch(hipStream_t stream, size_t bytes, SplitScratchLease* lease);
+// With `ready`: a buffer that would have to grow while the stream is being captured (no allocation is allowed there) is
+// not an error; *ready tells, and the caller takes a launch that needs none.
+int32_t AcquireSplitScratch(hipStream_t stream, size_t bytes, SplitScratchLease* lease, bool* ready = nullptr);
 int32_t LaunchSplitReduce(hipStream_t stream, const SplitReduceArgs& a);
 
 constexpr size_t kMaxLdsBytes = 160 * 1024;  // LDS of one gfx950 compute unit
@@ -156,6 +158,13 @@ int32_t PrepareWinograd(const kxc_hip_conv2d_desc* desc, PreparedWinograd** out)
 int32_t LaunchPreparedWinograd(const PreparedWinograd* p, const float* x, const float* u, const float* bias,
                                const float* residual, float* y, hipStream_t stream);
 void FreePreparedWinograd(PreparedWinograd* p);
+
+// A single nn_conv2d by the three-part Winograd kernel, filter transform included (conv2d_wino_f32.hip): which shapes it is
+// for, and the call.  *launched = false: the stream is being captured and the scratch for the filter would have to grow.
+bool WinogradOperatorPreferred(const kxc_hip_conv2d_desc* desc);
+int32_t RunWinogradOperator(const kxc_hip_conv2d_desc* desc, const float* x, const float* w, const float* bias, const float* residual,
+                            float* y, hipStream_t stream, bool* launched);
+extern const char* const kWinogradOperatorName;
 
 // The filter transforms of several Winograd layers in one launch (conv2d_wino_f32.hip).
 constexpr uint32_t kWinoFormF32 = 1, kWinoFormThreePart = 2;

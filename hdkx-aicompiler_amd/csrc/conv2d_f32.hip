@@ -1441,6 +1441,15 @@ int32_t Conv2dRun(const kxc_hip_conv2d_desc* desc, const float* x, const float* 
                   const float* residual, float* y, void* stream, bool no_alloc, const SecondOutput* second = nullptr) {
     const char* const who = second ? "kxc_hip_conv2d_pair_nchw_f32" : no_alloc ? "kxc_hip_conv2d_nchw_f32_noalloc" : "kxc_hip_conv2d_nchw_f32";
     ConvLaunch L;
+    // (the entry point that allocates nothing has no scratch for a transformed filter)
+    if (!second && !no_alloc && desc && WinogradOperatorPreferred(desc)) {
+        KXC_HIP_REQUIRE(x && w && y, "%s: NULL pointer", who);
+        KXC_HIP_REQUIRE(!(desc->flags & KXC_HIP_CONV_BIAS) || bias, "%s: bias flag without bias", who);
+        KXC_HIP_REQUIRE(!(desc->flags & KXC_HIP_CONV_RESIDUAL) || residual, "%s: residual flag without residual", who);
+        bool launched = false;
+        if (int32_t rc = RunWinogradOperator(desc, x, w, bias, residual, y, ResolveStream(stream), &launched)) return rc;
+        if (launched) return KXC_HIP_OK;
+    }
     if (int32_t rc = Conv2dResolve(desc, second != nullptr, who, &L)) return rc;
     return Conv2dLaunch(L, who, x, w, bias, residual, y, stream, no_alloc, second);
 }
@@ -1487,7 +1496,7 @@ void FreePreparedConv(PreparedConv* p) { delete p; }
 
 extern "C" {
 
-const char* kxc_hip_conv2d_variant(const kxc_hip_conv2d_desc* desc) {
+const char* kxc_hip_conv2d_node_variant(const kxc_hip_conv2d_desc* desc) {
     ConvArgs a;
     if (FillArgs(desc, &a, "kxc_hip_conv2d_variant") != KXC_HIP_OK) return "invalid";
     if (desc->flags & KXC_HIP_CONV_HPOOL) {
@@ -1501,6 +1510,10 @@ const char* kxc_hip_conv2d_variant(const kxc_hip_conv2d_desc* desc) {
     Choice c;
     Select(a, desc->kh, desc->kw, &c);
     return c.v ? c.v->name : "direct";
+}
+
+const char* kxc_hip_conv2d_variant(const kxc_hip_conv2d_desc* desc) {
+    return desc && WinogradOperatorPreferred(desc) ? kWinogradOperatorName : kxc_hip_conv2d_node_variant(desc);
 }
 
 int32_t kxc_hip_conv2d_nchw_f32(const kxc_hip_conv2d_desc* desc, const float* x, const float* w, const float* bias,

@@ -601,9 +601,10 @@ const WinoVariant kWino[] = {
 };
 constexpr int kNumWino = sizeof(kWino) / sizeof(kWino[0]);
 
-bool Supported(const kxc_hip_conv2d_desc* d) {
+// Shapes of the three-part kernel; the fp32-instruction kernel, and so every caller that prepares filters, takes C % 4 == 0.
+bool SupportedAnyC(const kxc_hip_conv2d_desc* d) {
     if (!d || d->kh != 3 || d->kw != 3 || d->stride_h != 1 || d->stride_w != 1 || d->dil_h != 1 || d->dil_w != 1) return false;
-    if (d->n <= 0 || d->c <= 0 || d->c % 4 != 0 || d->o <= 0 || d->h <= 0 || d->w <= 0) return false;
+    if (d->n <= 0 || d->c <= 0 || d->o <= 0 || d->h <= 0 || d->w <= 0) return false;
     if (d->flags & KXC_HIP_CONV_HPOOL) return false;      // the pooling epilogue exists in the direct-convolution kernels only
     // padding beyond the filter's reach only adds all-zero border tiles; cap it so the sizes below cannot overflow
     if (d->pad_h < 0 || d->pad_w < 0 || d->pad_h > (1 << 20) || d->pad_w > (1 << 20)) return false;
@@ -615,6 +616,7 @@ bool Supported(const kxc_hip_conv2d_desc* d) {
     const int64_t tiles = static_cast<int64_t>(d->n) * CeilDiv(oh, 2) * CeilDiv(ow, 2);
     return x_bytes < (1LL << 31) && y_elems * 4 < (1LL << 31) && u_bytes < (1LL << 31) && tiles < (1LL << 30);
 }
+bool Supported(const kxc_hip_conv2d_desc* d) { return SupportedAnyC(d) && d->c % 4 == 0; }
 
 // A filter buffer holds both forms, the fp32 one first: which of them a launch reads depends on the batch it runs on.
 size_t F32FilterBytes(const kxc_hip_conv2d_desc* d) { return static_cast<size_t>(CeilDiv(d->o, 32)) * 32 * static_cast<size_t>(d->c) * 64; }
@@ -724,7 +726,7 @@ struct WinoLaunch {
 };
 
 // Shape, grid and split of a three-part launch.
-void ThreePartResolve(const kxc_hip_conv2d_desc* d, WinoLaunch* L) {
+void ThreePartResolve(const kxc_hip_conv2d_desc* d, WinoLaunch* L, bool may_split = true) {
     wino_bx::Args& b = L->bx;
     std::memset(&b, 0, sizeof(b));
     const WinoArgs& a = L->a;
@@ -741,8 +743,8 @@ void ThreePartResolve(const kxc_hip_conv2d_desc* d, WinoLaunch* L) {
     b.x_bytes = a.x_bytes; b.flags = a.flags;
     b.u_bytes = static_cast<uint32_t>(wino_bx::WeightBytes(a.O, a.C));
     L->u_offset = F32FilterBytes(d);
-    int split = ThreePartSplit(b.num_units * static_cast<int64_t>(SelectLanes()), b.ksteps, L->out_elems);
-    if (const char* e = std::getenv("KXC_HIP_WINOGRAD_GSPLIT")) {
+    int split = !may_split ? 1 : ThreePartSplit(b.num_units * static_cast<int64_t>(SelectLanes()), b.ksteps, L->out_elems);
+    if (const char* e = may_split ? std::getenv("KXC_HIP_WINOGRAD_GSPLIT") : nullptr) {
         const int f = std::atoi(e);
         if (f >= 1 && f <= b.ksteps && L->out_elems * static_cast<int64_t>(sizeof(float)) * f <= (256LL << 20)) split = f;
     }
@@ -759,10 +761,7 @@ void ThreePartResolve(const kxc_hip_conv2d_desc* d, WinoLaunch* L) {
     L->lds_bytes = wino_bx::kLdsBytes;
 }
 
-int32_t WinoResolve(const kxc_hip_conv2d_desc* desc, WinoLaunch* L) {
-    KXC_HIP_REQUIRE(desc && Supported(desc), "kxc_hip_conv2d_winograd_nchw_f32: unsupported shape");
-    const WinoVariant* v = SelectWino(desc);
-    L->v = v;
+void FillWinoArgs(const kxc_hip_conv2d_desc* desc, WinoLaunch* L) {
     WinoArgs& a = L->a;
     std::memset(&a, 0, sizeof(a));
     a.N = static_cast<int32_t>(desc->n); a.C = static_cast<int32_t>(desc->c); a.H = static_cast<int32_t>(desc->h);
@@ -777,6 +776,15 @@ int32_t WinoResolve(const kxc_hip_conv2d_desc* desc, WinoLaunch* L) {
     a.x_bytes = static_cast<uint32_t>(static_cast<int64_t>(a.N) * a.C * a.HW * 4);
     a.u_bytes = static_cast<uint32_t>(CeilDiv(a.O, 32) * 32 * static_cast<int64_t>(a.C) * 64);
     a.flags = desc->flags;
+    L->out_elems = static_cast<int64_t>(a.N) * a.O * a.OHW;
+}
+
+int32_t WinoResolve(const kxc_hip_conv2d_desc* desc, WinoLaunch* L) {
+    KXC_HIP_REQUIRE(desc && Supported(desc), "kxc_hip_conv2d_winograd_nchw_f32: unsupported shape");
+    const WinoVariant* v = SelectWino(desc);
+    L->v = v;
+    FillWinoArgs(desc, L);
+    WinoArgs& a = L->a;
     a.t_groups = static_cast<int32_t>(CeilDiv(a.NT, 16 * v->wt));
     a.k_groups = static_cast<int32_t>(CeilDiv(a.O, 32 * v->wk));
     a.num_units = a.t_groups * a.k_groups;
@@ -785,8 +793,7 @@ int32_t WinoResolve(const kxc_hip_conv2d_desc* desc, WinoLaunch* L) {
     // applies the epilogue.
     a.gsplit = 1;
     a.steps_per_split = a.csteps;
-    const int64_t out_elems = static_cast<int64_t>(a.N) * a.O * a.OHW;
-    L->out_elems = out_elems;
+    const int64_t out_elems = L->out_elems;
     if (!v->kernel) { ThreePartResolve(desc, L); return KXC_HIP_OK; }
     if (v->ks == 1) {
         int split = GroupSplit(static_cast<int64_t>(a.num_units) * SelectLanes(), a.csteps, out_elems);
@@ -835,7 +842,7 @@ int32_t WinoRun(const WinoLaunch& L, const float* x, const float* u, const float
     if (L.three_part) {
         wino_bx::Args b = L.bx;
         b.x = x; b.u = reinterpret_cast<const char*>(u) + L.u_offset; b.bias = bias; b.res = residual; b.y = y; b.partial = a.partial;
-        void (*const bx)(const wino_bx::Args) = L.bx_plane == 0 ? wino_bx::wino_bf16x3_kernel<512> : wino_bx::wino_bf16x3_kernel<768>;
+        void (*const bx)(const wino_bx::Args) = L.bx_plane == 0 ? wino_bx::wino_bf16x3_kernel<512, false> : wino_bx::wino_bf16x3_kernel<768, false>;
         if (int32_t rc = GrantLds(reinterpret_cast<const void*>(bx))) return rc;
         hipLaunchKernelGGL(bx, NoteGrid(dim3(static_cast<unsigned>(b.units_per_xcd * 8))), NoteBlock(dim3(wino_bx::kThreads)),
                            NoteLds(L.lds_bytes), s, b);
@@ -886,6 +893,55 @@ int32_t LaunchPreparedWinograd(const PreparedWinograd* p, const float* x, const 
 void FreePreparedWinograd(PreparedWinograd* p) { delete p; }
 
 uint32_t PreparedWinogradForms(const PreparedWinograd* p) { return p->launch.three_part ? kWinoFormThreePart : kWinoFormF32; }
+
+const char* const kWinogradOperatorName = kThreePart;
+
+// A call pays for the filter transform (a launch, about 5 us) and for whole workgroups of 64 channels x 64 tiles, one per
+// compute unit at a time.  Both sides' times follow a line within about 10 % (us): here 12 + rounds * (10 + 2.5 * steps of 16
+// channels), the other kernels 14 + 10.5 per GFLOP.  Measured, other kernels and here: 90 -> 150 channels at 37 x 51, batch 7
+// 54 and 40; 64 -> 64 at 56 x 56, batch 8 29.6 both, 16 52 and 33, 64 148 and 94; 128 -> 128 at 28 x 28, batch 8 34 and 41, 16
+// 50 and 42, 64 153 and 76; 256 -> 256 at 14 x 14, batch 16 52 and 59, 64 161 and 64; 512 -> 512 at 7 x 7, batch 64 169 and
+// 98; 16 -> 64 at 60 x 60, batch 40 41 and 46.  A tenth in hand also keeps out the launches whose reduction the other
+// kernels split, where their error against float64 is the smaller one (256 channels at 14 x 14, batch 16: 2.9e-7, 3.7e-7
+// here); on the shapes taken it is the larger one (2.6e-7 / 2.3e-7, 3.1e-7 / 2.0e-7, 5.9e-7 / 3.7e-7, 5.6e-7 / 5.3e-7).
+bool WinogradOperatorPreferred(const kxc_hip_conv2d_desc* d) {
+    if (!SupportedAnyC(d) || (d->flags & KXC_HIP_CONV_FORCE_DIRECT) || !ThreePartFits(d)) return false;
+    if (const char* forced = std::getenv("KXC_HIP_CONV_VARIANT"); forced && *forced) return std::strcmp(forced, kThreePart) == 0;
+    // (KXC_HIP_CONV_WINOGRAD=0 keeps single operators on the kernels that read their weights as they are)
+    for (const char* name : {"KXC_HIP_WINOGRAD_BF16X3", "KXC_HIP_CONV_WINOGRAD"})
+        if (const char* e = std::getenv(name); e && e[0] == '0') return false;
+    const int64_t units = CeilDiv(Tiles(d), wino_bx::kTiles) * CeilDiv(d->o, wino_bx::kOut);
+    const double rounds = static_cast<double>(CeilDiv(units, 256)), steps = static_cast<double>(CeilDiv(d->c, wino_bx::kStep));
+    const double oh = d->h + 2.0 * d->pad_h - 2, ow = d->w + 2.0 * d->pad_w - 2;
+    const double gflop = 18e-9 * d->n * d->c * d->o * oh * ow;
+    return 1.1 * (12 + rounds * (10 + 2.5 * steps)) < 14 + 10.5 * gflop;
+}
+
+int32_t RunWinogradOperator(const kxc_hip_conv2d_desc* desc, const float* x, const float* w, const float* bias, const float* residual,
+                            float* y, hipStream_t stream, bool* launched) {
+    WinoLaunch L;
+    FillWinoArgs(desc, &L);
+    ThreePartResolve(desc, &L, false);
+    SplitScratchLease lease;      // held until the kernel that reads the filter is enqueued
+    *launched = true;
+    // (the filter is transformed by every call: the caller may have changed it)
+    if (int32_t rc = AcquireSplitScratch(stream, L.bx.u_bytes, &lease, launched)) return rc;
+    if (!*launched) return KXC_HIP_OK;
+    WinoWeightBatch jobs;
+    std::memset(&jobs, 0, sizeof(jobs));
+    const int64_t blocks = wino_bx::WeightTiles(desc->o, desc->c);
+    KXC_HIP_REQUIRE(blocks < kMaxGridX, "kxc_hip_conv2d_nchw_f32: too many filter tiles");
+    jobs.w[0] = w; jobs.u[0] = reinterpret_cast<char*>(lease.ptr); jobs.O[0] = static_cast<int32_t>(desc->o); jobs.C[0] = static_cast<int32_t>(desc->c);
+    jobs.first_block[1] = static_cast<int32_t>(blocks); jobs.three_part = 1; jobs.count = 1;
+    wino_weight_batch_kernel<<<NoteGrid(static_cast<int>(blocks)), NoteBlock(256), NoteLds(0), stream>>>(jobs);
+    if (int32_t rc = CheckLaunch("wino_weight_batch_kernel")) return rc;
+    wino_bx::Args b = L.bx;
+    b.x = x; b.u = reinterpret_cast<const char*>(lease.ptr); b.w = w; b.bias = bias; b.res = residual; b.y = y;
+    void (*const bx)(const wino_bx::Args) = L.bx_plane == 0 ? wino_bx::wino_bf16x3_kernel<512, true> : wino_bx::wino_bf16x3_kernel<768, true>;
+    if (int32_t rc = GrantLds(reinterpret_cast<const void*>(bx))) return rc;
+    hipLaunchKernelGGL(bx, NoteGrid(dim3(static_cast<unsigned>(b.units_per_xcd * 8))), NoteBlock(dim3(wino_bx::kThreads)), NoteLds(L.lds_bytes), stream, b);
+    return CheckLaunch(kThreePart);
+}
 
 int32_t LaunchWinogradWeightTransforms(const WinoWeightJob* jobs, int32_t count, hipStream_t stream) {
     WinoWeightBatch b;

@@ -339,7 +339,7 @@ int32_t kxc_hip_plan_add_conv2d(kxc_hip_plan* plan, const kxc_hip_conv2d_desc* d
     n.kind = NodeKind::kConv2D;
     n.conv = *desc;
     n.bufs[0] = x; n.bufs[1] = w; n.bufs[2] = bias; n.bufs[3] = residual; n.bufs[4] = y;
-    n.symbol = std::string("kxc_conv2d_nchw_f32.") + kxc_hip_conv2d_variant(desc);
+    n.symbol = std::string("kxc_conv2d_nchw_f32.") + kxc_hip_conv2d_node_variant(desc);
     if (desc->flags & KXC_HIP_CONV_BIAS) n.symbol += "+bias";
     if (desc->flags & KXC_HIP_CONV_RESIDUAL) n.symbol += "+add";
     if (desc->flags & KXC_HIP_CONV_RELU) n.symbol += "+relu";
@@ -790,7 +790,7 @@ int32_t kxc_hip_plan_finalize(kxc_hip_plan* plan, size_t workspace_bytes) {
         KXC_HIP_CALL(hipSetDevice(plan->device_id), "HIP SetDevice");
         const char* variant = n.i32[0] == 1   ? kxc_hip_conv2d_winograd_variant(&n.conv)
                               : n.i32[0] == 2 ? kxc_hip_conv2d_pair_variant(&n.conv)
-                                              : kxc_hip_conv2d_variant(&n.conv);
+                                              : kxc_hip_conv2d_node_variant(&n.conv);
         // (a small Winograd node runs on its weights as they are, in one launch)
         if (n.i32[0] == 1 && !kxc_hip::SmallConvBeatsWinograd(&n.conv)) {
             kxc_hip::PreparedWinograd* p = nullptr;

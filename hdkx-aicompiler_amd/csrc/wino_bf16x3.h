@@ -76,6 +76,7 @@ struct Args {
     const float* res;
     float* y;
     float* partial;
+    const float* w;                    // RECHECK: OIHW weights
     int32_t N, C, H, W, O, OH, OW, ph, pw;
     int32_t TW, TI, NT, Hq, pitch;      // tiles per row, per image, in total; rows per image of the patch, row pitch of a half plane
     int32_t HW, OHW, ksteps;
@@ -135,7 +136,9 @@ __device__ __forceinline__ void weight_tile(const float* __restrict__ w, char* _
 }
 inline int64_t WeightTiles(int64_t O, int64_t C) { return CeilDiv(O, 32) * CeilDiv(C, kStep); }
 
-template <int kPlane>
+// RECHECK (the single operator): the transforms spread an Inf or NaN over the whole 2x2 tile, and so do sums beyond the
+// largest float; a thread that finds such a tile evaluates its outputs by the loop of the operator's definition.
+template <int kPlane, bool RECHECK>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) wino_bf16x3_kernel(const Args a) {
     constexpr int kHalf = kPlane / 2, kSegs = kPlane / 64;
     constexpr int NP = kSegs * kStep / 8;                 // patch loads of a wave per step
@@ -368,6 +371,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
     const uint32_t rowb_bytes = static_cast<uint32_t>(a.OW) * 4u, o_bytes = static_cast<uint32_t>(a.OHW) * 4u;
     constexpr int kArea = 8 * 2 * 1024;
     auto bits = [](float v) { return __builtin_bit_cast(uint32_t, v); };
+    uint32_t again = 0;               // RECHECK: bit 2 j + i = this thread's outputs of the block
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         uint32_t off[2][2], cm[2];      // [tile][row] byte offset within channel 0 of a block; mask of the second column
@@ -400,7 +404,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
                 }
             }
             const int ob = kg * kOut + i * 32;                                   // uniform: the block's first channel
-            const uint32_t om = ob + ol < a.O ? 0u : kOob;
+            uint32_t om = ob + ol < a.O ? 0u : kOob;
             const uint32_t so = ob < a.O ? static_cast<uint32_t>(ob) * o_bytes : 0u;      // (the mask decides about absent channels)
             const float bv = load_f32(br, (static_cast<uint32_t>(ob + ol) * 4u) | om, 0);
             auto ld = [&](uint32_t o) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rr, o, so, 0)); };
@@ -439,6 +443,17 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
                     out[e][1][p] = __fsub_rn(__fsub_rn(row[1][e], row[2][e]), row[3][e]);
                 }
             }
+            if constexpr (RECHECK) {
+                float odd = 0.0f;
+#pragma unroll
+                for (int e = 0; e < 2; ++e)
+#pragma unroll
+                    for (int row = 0; row < 2; ++row) odd = __builtin_fmaf(out[e][row][0], 0.0f, __builtin_fmaf(out[e][row][1], 0.0f, odd));
+                if (!(odd == 0.0f) && om == 0) {
+                    again |= 1u << (2 * j + i);
+                    om = kOob;                  // (nothing is stored now: the residual may be the output's own buffer)
+                }
+            }
 #pragma unroll
             for (int e = 0; e < 2; ++e)
 #pragma unroll
@@ -473,6 +488,34 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
                         __builtin_amdgcn_raw_buffer_store_b32(bits(out[e][row][1]), yr, (off[e][row] + 4u) | cm[e] | om, so, 0);
                     }
             }
+        }
+    }
+    if constexpr (RECHECK) {
+        if (again == 0) return;
+#pragma unroll 1
+        for (int k = 0; k < 32; ++k) {
+            const int block = k >> 3, e = (k >> 2) & 1, row = (k >> 1) & 1, p = k & 1;
+            const int tile = t0 + (block >> 1) * 32 + 2 * tp + e, o = kg * kOut + (block & 1) * 32 + ol;
+            if (!((again >> block) & 1u) || tile >= a.NT) continue;
+            const int n = fast_div(tile, a.div_ti), rem = tile - n * a.TI;
+            const int ty = fast_div(rem, a.div_tw), oh = 2 * ty + row, ow = 2 * (rem - ty * a.TW) + p;
+            if (oh >= a.OH || ow >= a.OW) continue;
+            float s = 0.0f;
+#pragma unroll 1
+            for (int c = 0; c < a.C; ++c) {
+                const float* const xc = a.x + static_cast<int64_t>(n * a.C + c) * a.HW;
+                const float* const wc = a.w + (static_cast<int64_t>(o) * a.C + c) * 9;
+#pragma unroll 1
+                for (int q = 0; q < 9; ++q) {
+                    const int ih = oh + q / 3 - a.ph, iw = ow + q % 3 - a.pw;
+                    const bool in = ih >= 0 && ih < a.H && iw >= 0 && iw < a.W;
+                    s = __fadd_rn(s, __fmul_rn(in ? xc[ih * a.W + iw] : 0.0f, wc[q]));
+                }
+            }
+            const int64_t at = (static_cast<int64_t>(n * a.O + o) * a.OH + oh) * a.OW + ow;
+            if (has_bias) s = __fadd_rn(s, a.bias[o]);
+            if (has_res) s = __fadd_rn(s, a.res[at]);
+            a.y[at] = do_relu ? relu_sel(s) : s;
         }
     }
 }

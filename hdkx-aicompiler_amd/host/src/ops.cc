@@ -118,7 +118,7 @@ std::string Conv2DDispatch(const HIPDispatchContext& c, kxc_hip_plan* plan) {
         q.kh = 3; q.kw = 1; q.stride_h = 2; q.stride_w = 1;
         q.pad_top = 1; q.pad_bottom = 1;
         Check(kxc_hip_plan_add_pool2d(plan, &q, B(half), B(c.output)), "nn_conv2d dispatch (column pool)");
-        return std::string("kxc_conv2d_nchw_f32.") + kxc_hip_conv2d_variant(&d) + (has_bias ? "+bias" : "") + "+relu+maxpool3w";
+        return std::string("kxc_conv2d_nchw_f32.") + kxc_hip_conv2d_node_variant(&d) + (has_bias ? "+bias" : "") + "+relu+maxpool3w";
     }
     if (c.has_pair) {
         const bool bias2 = c.pair_inputs.size() == 3;
@@ -145,7 +145,7 @@ std::string Conv2DDispatch(const HIPDispatchContext& c, kxc_hip_plan* plan) {
     Check(kxc_hip_plan_add_conv2d(plan, &d, B(c.inputs[0]), B(c.inputs[1]), has_bias ? B(c.inputs[2]) : none,
                                   c.has_residual ? B(c.residual) : none, B(c.output)),
           "nn_conv2d dispatch");
-    return std::string("kxc_conv2d_nchw_f32.") + kxc_hip_conv2d_variant(&d) + (has_bias ? "+bias" : "") +
+    return std::string("kxc_conv2d_nchw_f32.") + kxc_hip_conv2d_node_variant(&d) + (has_bias ? "+bias" : "") +
            (c.has_residual ? "+add" : "") + (c.fused_relu ? "+relu" : "");
 }
 

@@ -167,11 +167,14 @@ typedef struct kxc_hip_conv2d_desc {
 } kxc_hip_conv2d_desc;
 int32_t kxc_hip_conv2d_nchw_f32(const kxc_hip_conv2d_desc* desc, const float* x, const float* w,
                                 const float* bias, const float* residual, float* y, void* stream);
-/* Name of the kernel variant the library would launch for this shape ("mfma_..." or "direct"). */
+/* Name of the kernel variant the library would launch for this shape ("mfma_...", "winograd_..." or "direct"). */
 const char* kxc_hip_conv2d_variant(const kxc_hip_conv2d_desc* desc);
+/* The same for a launch plan's kxc_hip_plan_add_conv2d node, which reads its weights as they are ("mfma_..." or "direct"). */
+const char* kxc_hip_conv2d_node_variant(const kxc_hip_conv2d_desc* desc);
 /* The same operator for callers that cannot allocate device memory (code under HIP graph capture, tight serving
- * loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  Same arguments, kernels and results
- * as kxc_hip_conv2d_nchw_f32, but it calls no hipMalloc / hipFree or allocating library routine: the partial sums
+ * loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  Same arguments and
+ * results (up to fp32 rounding where kxc_hip_conv2d_variant says "winograd_...", whose filter takes scratch this entry
+ * point does not have) as kxc_hip_conv2d_nchw_f32, but it calls no hipMalloc / hipFree or allocating library routine: the partial sums
  * of a reduction split over workgroups (small launches with long reductions, e.g. batch-1 512-channel layers) go
  * to a device array built into the library, kxc_hip_conv2d_noalloc_scratch_bytes() = 8 MiB per GPU, held until the
  * process ends.  A launch whose partial sums would not fit fails with KXC_HIP_ERR_INVALID and launches nothing

@@ -784,6 +784,44 @@ def test_conv_full_batch_properties(pkg, synth):
 
 
 # ------------------------------------------------------------------ pooling / elementwise at full sizes
+@pytest.mark.parametrize("n, c, h, w, o, p, forced", [
+    (1, 1, 3, 3, 1, 1, True), (2, 17, 9, 12, 65, 1, True), (3, 90, 13, 15, 64, 0, True), (1, 33, 31, 64, 33, 2, True), (5, 16, 7, 7, 130, 1, True),
+    (7, 90, 37, 51, 150, 1, False), (16, 64, 56, 56, 64, 1, False)])
+def test_conv_operator_by_winograd(pkg, monkeypatch, n, c, h, w, o, p, forced):
+    """nn_conv2d on the three-part Winograd kernel with the filter transformed in the call: partial groups of tiles,
+    output and input channels (any count), odd extents, a residual that is the output's own buffer, new weights in the same
+    buffer; Inf, NaN and sums past the largest float come out where the operator's definition puts them."""
+    name = "winograd_f2k3_bf16x3"
+    if forced:
+        monkeypatch.setenv("KXC_HIP_CONV_VARIANT", name)
+    rng = np.random.default_rng(n * c + h * w + o)
+    x = rng.standard_normal((n, c, h, w)).astype(np.float32)
+    assert pkg.conv2d_variant(x.shape, (o, c, 3, 3), 1, p) == name
+    wd = torch.empty((o, c, 3, 3), device="cuda")
+    b = rng.standard_normal(o).astype(np.float32)
+    res = rng.standard_normal((n, o, h + 2 * p - 2, w + 2 * p - 2)).astype(np.float32)
+    conv = lambda a, f: torch.nn.functional.conv2d(torch.from_numpy(a).double(), torch.from_numpy(f).double(), None, 1, p).numpy()
+    for turn in range(2):
+        wt = (rng.standard_normal((o, c, 3, 3)) / np.sqrt(9 * c)).astype(np.float32)
+        wd.copy_(dev(wt))
+        y = dev(res)
+        got = pkg.conv2d(dev(x), wd, dev(b), y, 1, p, 1, turn == 1, out=y)
+        want = conv(x, wt) + b[:, None, None] + res
+        want = np.maximum(want, 0) if turn == 1 else want
+        # 9 c + 16 roundings (terms, and the transforms' additions) of at most 2^-23 of a sum, of independent signs
+        assert np.linalg.norm(host(got) - want) <= (9 * c + 16) ** 0.5 * 2.0 ** -23 * np.linalg.norm(want)
+    x[0, 0, h // 2, w // 2] = np.inf; x[-1, -1, 0, 0] = np.nan; x[0, 0, h - 1, w - 1] = -3e38
+    wt[0] = np.abs(wt[0]) + 2
+    wd.copy_(dev(wt))
+    got, want = host(pkg.conv2d(dev(x), wd, dev(b), None, 1, p, 1, False)), host(pkg.conv2d(dev(x), wd, dev(b), None, 1, p, 1, False, force_direct=True))
+    for f in (np.isnan, np.isposinf, np.isneginf):
+        assert np.array_equal(f(got), f(want)), f.__name__
+    # (tiles of four outputs next to -3e38 lose their small ones to its rounding, as sums that hold it do)
+    near = np.isfinite(want)
+    near[0, :, max(0, h - 6 + p):, max(0, w - 6 + p):] = False
+    assert np.linalg.norm(got[near] - want[near]) <= 2 * (9 * c + 16) ** 0.5 * 2.0 ** -23 * np.linalg.norm(want[near].astype(np.float64)) + 1e-30
+
+
 @pytest.mark.parametrize("n, c, h, w, o, k, s, p", [
     (1, 64, 9, 9, 1, 3, 1, 1), (2, 65, 8, 7, 17, 3, 1, 1), (1, 64, 13, 11, 31, 1, 1, 0), (3, 30, 12, 17, 5, 5, 1, 2), (2, 16, 19, 23, 16, 7, 2, 3),
     (1, 7, 5, 5, 31, 3, 2, 1), (1, 96, 3, 3, 48, 3, 1, 1), (1, 72, 1, 1, 40, 3, 1, 1), (1, 50, 7, 4, 33, 5, 2, 2), (1, 63, 5, 6, 70, 1, 1, 0), (9, 64, 56, 50, 16, 3, 1, 1)])
