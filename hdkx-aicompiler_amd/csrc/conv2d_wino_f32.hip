@@ -670,7 +670,7 @@ int ThreePartSplit(int64_t units, int ksteps, int64_t out_elems) {
     return split;
 }
 
-// Measured on MI355X: 64 x 32 workgroups (four waves) are the fastest shape once there is one per compute unit;
+// Measured on MI355X: 64 x 32 workgroups (four waves) are the fastest shape once there is one per two compute units;
 // smaller launches run faster as twice as many 64 x 16 workgroups of two waves.
 const WinoVariant* SelectWino(const kxc_hip_conv2d_desc* d) {
     if (const char* e = std::getenv("KXC_HIP_WINOGRAD_VARIANT")) {
@@ -682,28 +682,32 @@ const WinoVariant* SelectWino(const kxc_hip_conv2d_desc* d) {
     const int csteps = d->c / 4;
     const int64_t oh = static_cast<int64_t>(d->h) + 2 * d->pad_h - 2, ow = static_cast<int64_t>(d->w) + 2 * d->pad_w - 2;
     const int64_t lanes = SelectLanes();
-    // From about 28 million (tile, output channel, input channel) triples on the bf16 matrix cores win: 12 images of the
-    // 56 x 56 / 28 x 28 / 14 x 14 / 7 x 7 layers (38 million each) 21.5 / 27.3 / 27.0 / 27.3 us against 27.4 / 30.8 / 30.5 /
-    // 29.7, 8 images (26 million) 22.7 / 21.9 / 23.8 / 25.5 against 21.7 / 20.4 / 26.1 / 26.5, 4 images 20.0 / 19.5 / 19.3 /
-    // 23.8 against 14.0 / 16.8 / 17.2 / 17.7.  KXC_HIP_WINOGRAD_BF16X3=0 keeps the fp32 instructions.
+    // From about 36 million (tile, output channel, input channel) triples on the bf16 matrix cores win: 12 images of the
+    // 56 x 56 / 28 x 28 / 14 x 14 / 7 x 7 layers (38 million each) 23.5 / 27.5 / 27.7 / 28.9 us against 30.6 / 29.6 / 31.3 /
+    // 30.0, 10 images (32 million; 7 x 7: 42) 27.1 / - / 26.1 / 28.0 against 20.7 / - / 25.6 / 30.6, 8 images (26 million; 7 x 7: 34)
+    // 23.7 / 22.4 / 24.3 / 26.6 against 19.9 / 22.4 / 24.0 / 24.6.  KXC_HIP_WINOGRAD_BF16X3=0 keeps the fp32 instructions.
     const char* bx = std::getenv("KXC_HIP_WINOGRAD_BF16X3");
-    if (!(bx && bx[0] == '0') && Tiles(d) * lanes * d->o * d->c >= 28000000LL && ThreePartFits(d)) {
+    if (!(bx && bx[0] == '0') && Tiles(d) * lanes * d->o * d->c >= 36000000LL && ThreePartFits(d)) {
         for (int i = 0; i < kNumWino; ++i)
             if (!kWino[i].kernel) return &kWino[i];
     }
     // Small launches (batch 1-8 of ResNet-18): 64 x 16 groups with the channels split over workgroups beat both
     // the split inside the workgroup and the implicit-GEMM kernel (batch 1, 512 channels: 14.7 against 62.9 and
-    // 20.0 us).
+    // 20.0 us).  From 12 million triples on 64 x 32 groups in twice as many parts, which read each filter half as often:
+    // 256 channels at 13 x 13, batch 6 26.0 -> 22.9 us, 512 at 7 x 7 26.4 -> 22.8, 128 at 28 x 28, batch 4 18.2 -> 16.3;
+    // below it 13.0 against 13.5 (128 at 28 x 28, batch 2), 14.2 against 16.3 (512 at 7 x 7).
     const int64_t units_t1 = CeilDiv(Tiles(d), 16) * CeilDiv(d->o, 64) * lanes;
     if (GroupSplit(units_t1, csteps, static_cast<int64_t>(d->n) * d->o * oh * ow) > 1) {
+        const int wt = Tiles(d) * lanes * d->o * d->c >= 12000000LL ? 2 : 1;
         for (int i = 0; i < kNumWino; ++i)
-            if (kWino[i].wk == 2 && kWino[i].wt == 1 && kWino[i].ks == 1) return &kWino[i];
+            if (kWino[i].wk == 2 && kWino[i].wt == wt && kWino[i].ks == 1) return &kWino[i];
     }
-    // 64 x 32 groups from one per compute unit on; below that twice as many 64 x 16 groups.  A launch that cannot
+    // 64 x 32 groups once the 64 x 16 ones are more than one per compute unit (64 channels at 56 x 56, batch 8: 196 against
+    // 392, 19.9 against 24.7 us; at 49 x 49, batch 6: 118 against 235, 19.0 against 17.3).  A launch that cannot
     // give every SIMD two waves (at most one 64 x 32 group per compute unit) and has a long reduction splits the
     // input channels over two groups of waves inside the workgroup instead.
     const int64_t units = CeilDiv(Tiles(d), 32) * CeilDiv(d->o, 64) * lanes;
-    const int wt = units < 256 ? 1 : 2;
+    const int wt = units <= 128 ? 1 : 2;
     const int ks = (units <= 256 && csteps % 2 == 0 && csteps >= 32) ? 2 : 1;
     for (int i = 0; i < kNumWino; ++i)
         if (kWino[i].wk == 2 && kWino[i].wt == wt && kWino[i].ks == ks) return &kWino[i];
