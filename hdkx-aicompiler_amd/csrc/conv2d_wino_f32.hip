@@ -909,16 +909,17 @@ const char* const kWinogradOperatorName = kThreePart;
 // kernels split, where their error against float64 is the smaller one (256 channels at 14 x 14, batch 16: 2.9e-7, 3.7e-7
 // here); on the shapes taken it is the larger one (2.6e-7 / 2.3e-7, 3.1e-7 / 2.0e-7, 5.9e-7 / 3.7e-7, 5.6e-7 / 5.3e-7).
 bool WinogradOperatorPreferred(const kxc_hip_conv2d_desc* d) {
-    if (!SupportedAnyC(d) || (d->flags & KXC_HIP_CONV_FORCE_DIRECT) || !ThreePartFits(d)) return false;
-    if (const char* forced = std::getenv("KXC_HIP_CONV_VARIANT"); forced && *forced) return std::strcmp(forced, kThreePart) == 0;
-    // (KXC_HIP_CONV_WINOGRAD=0 keeps single operators on the kernels that read their weights as they are)
-    for (const char* name : {"KXC_HIP_WINOGRAD_BF16X3", "KXC_HIP_CONV_WINOGRAD"})
-        if (const char* e = std::getenv(name); e && e[0] == '0') return false;
+    if (!SupportedAnyC(d) || (d->flags & KXC_HIP_CONV_FORCE_DIRECT)) return false;
+    if (const char* forced = std::getenv("KXC_HIP_CONV_VARIANT"); forced && *forced) return std::strcmp(forced, kThreePart) == 0 && ThreePartFits(d);
     const int64_t units = CeilDiv(Tiles(d), wino_bx::kTiles) * CeilDiv(d->o, wino_bx::kOut);
     const double rounds = static_cast<double>(CeilDiv(units, 256)), steps = static_cast<double>(CeilDiv(d->c, wino_bx::kStep));
     const double oh = d->h + 2.0 * d->pad_h - 2, ow = d->w + 2.0 * d->pad_w - 2;
     const double gflop = 18e-9 * d->n * d->c * d->o * oh * ow;
-    return 1.1 * (12 + rounds * (10 + 2.5 * steps)) < 14 + 10.5 * gflop;
+    if (1.1 * (12 + rounds * (10 + 2.5 * steps)) >= 14 + 10.5 * gflop) return false;
+    // (KXC_HIP_CONV_WINOGRAD=0 keeps single operators on the kernels that read their weights as they are)
+    for (const char* name : {"KXC_HIP_WINOGRAD_BF16X3", "KXC_HIP_CONV_WINOGRAD"})
+        if (const char* e = std::getenv(name); e && e[0] == '0') return false;
+    return ThreePartFits(d);
 }
 
 int32_t RunWinogradOperator(const kxc_hip_conv2d_desc* desc, const float* x, const float* w, const float* bias, const float* residual,
