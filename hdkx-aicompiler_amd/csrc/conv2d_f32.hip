@@ -976,13 +976,17 @@ void Select(const ConvArgs& real, int kh, int kw, Choice* choice, bool ds = fals
         }
         if (pass == 1) {
             *choice = first_fit;
-            // (a 1x1 filter's reduction is only as long as its input channels: splitting 64 or 128 of them costs more
-            // than the idle SIMDs -- batch 32, 64 -> 128 channels at 56 x 56, stride 2: 26.6 us split two ways, 21.4 whole)
-            if (first_fit.v && first_waves < kEnoughWaves && !(kh == 1 && a.C < 256)) {
+            // (a 1x1 filter's reduction is only as long as its input channels: splitting 64 of them costs more than the idle
+            // SIMDs -- batch 32, 64 -> 128 channels at 56 x 56, stride 2: 26.6 us split two ways, 21.4 whole; from 80 on it
+            // pays: 90 -> 32 at 28 x 28, batch 16 15.1 -> 11.9, 100 -> 200 at 40 x 40, batch 8 27.3 -> 23.7, 169 -> 141 at 104 x 15,
+            // stride 2, batch 45 44.3 -> 33.5, 250 -> 300 at 14 x 14, batch 20 49.9 -> 33.9)
+            if (first_fit.v && first_waves < kEnoughWaves && !(kh == 1 && a.C < 80)) {
                 for (int k = 0; k < 3; ++k) {
                     if (!split[k].v) continue;
                     *choice = split[k];
-                    if (split_waves[k] >= 2560) break;      // enough waves: stop splitting further
+                    // enough waves: stop splitting further (1x1: 500 -> 400 at 20 x 20, batch 2 23.7 us four ways, 27.7 eight;
+                    // 333 -> 100 at 33 x 33, batch 5, 1376 waves two ways 29.2, four 25.4)
+                    if (split_waves[k] >= (kh == 1 ? 1400 : 2560)) break;
                     // 3x3: two wave groups on the 32 x 128 tile plus the split over workgroups beat the deeper
                     // splits on 32 x 64 tiles from batch 1 to 16, at stride 2 (batch 8, 128 -> 256 channels at
                     // 28 x 28: 20.5 against 31.5 us) and at stride 1 (batch 1, 256 channels at 14 x 14: 12.6
