@@ -22,6 +22,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 PEAK_FP32_MFMA_TFLOPS = 157.3
+PEAK_BF16_MFMA_TFLOPS = 2500.0
 PEAK_HBM_GBS = 8000.0
 
 
@@ -268,21 +269,25 @@ def main():
         lu = pkg.conv2d_winograd_transform_weights(lx.shape, lw, 1)
         conv_ms = _event_time_ms(torch, lambda: pkg.conv2d_winograd(lx, lu, lw.shape, lb, None, 1, True, out=ly), 30, 5)
         conv_tflops = conv_flop / (conv_ms * 1e-3) / 1e12
-        executed = conv_flop * 16.0 / 36.0
-        roofline = {"bound": "mfma", "kernel": "wino_kernel (layer1: [%d,64,56,56]x[64,64,3,3] s1 p1 +bias+relu, Winograd F(2x2,3x3))" % batch,
+        # (the three-part kernel multiplies every pair of operands as six bf16 products, on the bf16 matrix cores)
+        three_part = pkg.conv2d_winograd_variant(lx.shape, lw.shape).endswith("bf16x3")
+        executed = conv_flop * 16.0 / 36.0 * (6 if three_part else 1)
+        matrix_peak = PEAK_BF16_MFMA_TFLOPS if three_part else PEAK_FP32_MFMA_TFLOPS
+        roofline = {"bound": "mfma", "kernel": ("wino_bf16x3_kernel" if three_part else "wino_kernel") + " (layer1: [%d,64,56,56]x[64,64,3,3] s1 p1 +bias+relu, Winograd F(2x2,3x3))" % batch,
                     "variant": pkg.conv2d_winograd_variant(lx.shape, lw.shape),
                     "achieved": round(conv_tflops, 3), "peak": PEAK_FP32_MFMA_TFLOPS, "unit": "TFLOP/s",
                     "frac": round(conv_tflops / PEAK_FP32_MFMA_TFLOPS, 4), "avg_launch_ms": round(conv_ms, 4),
                     "flop_per_launch": conv_flop,
                     "matrix_core_flop_per_launch": executed,
                     "matrix_core_tflops": round(executed / (conv_ms * 1e-3) / 1e12, 3),
-                    "matrix_core_frac": round(executed / (conv_ms * 1e-3) / 1e12 / PEAK_FP32_MFMA_TFLOPS, 4),
-                    "traffic": _profiled_traffic_bytes("winograd_layer1_bs64_counters.md") if batch == 64 else None,
+                    "matrix_core_frac": round(executed / (conv_ms * 1e-3) / 1e12 / matrix_peak, 4), "matrix_core_peak": matrix_peak,
+                    "traffic": _profiled_traffic_bytes("winograd_%slayer1_bs64_counters.md" % ("bf16x3_" if three_part else "")) if batch == 64 else None,
                     "traffic_unit": "bytes per launch (FETCH_SIZE + WRITE_SIZE, calibrated on a copy; from profiles/)",
                     "algorithmic_bytes_per_launch": algorithmic_bytes, "same_layer_implicit_gemm": gemm_row,
                     "accounting": "achieved and frac divide the OPERATOR's FLOP (2*N*O*OH*OW*C*9, every output computed) by the measured "
-                                  "time; Winograd F(2x2,3x3) executes 16/36 of those multiplies, so frac can reach or pass 1 while the "
-                                  "matrix cores run at matrix_core_frac of their peak"}
+                                  "time, against the fp32 matrix peak; Winograd F(2x2,3x3) executes 16/36 of those multiplies, the three-part "
+                                  "kernel each as six bf16 products, so frac can reach or pass 1 while the matrix cores run at "
+                                  "matrix_core_frac of matrix_core_peak (the bf16 peak for the three-part kernel)"}
         if shares > 1 and batch % shares == 0:
             # what the plan does with this layer: one launch per share of the batch, side by side on streams of
             # their own between a fork and a join on the timed stream (variants chosen for `shares` equal launches)
@@ -311,7 +316,7 @@ def main():
                 "what": "%d launches of [%d,64,56,56] on %d streams, fork to join: the layer as the timed plan runs it" % (shares, part, shares),
                 "variant": part_variant, "ms": round(pair_ms, 4), "achieved": round(conv_flop / (pair_ms * 1e-3) / 1e12, 3),
                 "frac": round(conv_flop / (pair_ms * 1e-3) / 1e12 / PEAK_FP32_MFMA_TFLOPS, 4),
-                "matrix_core_frac": round(executed / (pair_ms * 1e-3) / 1e12 / PEAK_FP32_MFMA_TFLOPS, 4)}
+                "matrix_core_frac": round(executed / (pair_ms * 1e-3) / 1e12 / matrix_peak, 4)}
     else:
         roofline = {"bound": "mfma", "kernel": "conv_mfma_kernel<3,3> (layer1: [%d,64,56,56]x[64,64,3,3] s1 p1 +bias+relu)" % batch,
                     "variant": gemm_row["variant"], "achieved": gemm_row["achieved"], "peak": PEAK_FP32_MFMA_TFLOPS,

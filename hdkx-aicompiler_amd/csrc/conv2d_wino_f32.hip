@@ -916,6 +916,7 @@ bool WinogradOperatorPreferred(const kxc_hip_conv2d_desc* d) {
     const double oh = d->h + 2.0 * d->pad_h - 2, ow = d->w + 2.0 * d->pad_w - 2;
     const double gflop = 18e-9 * d->n * d->c * d->o * oh * ow;
     if (1.1 * (12 + rounds * (10 + 2.5 * steps)) >= 14 + 10.5 * gflop) return false;
+    if (wino_bx::WeightBytes(d->o, d->c) > (32u << 20)) return false;      // (bounds the scratch kept per stream; 512 x 512 channels: 25 MB)
     // (KXC_HIP_CONV_WINOGRAD=0 keeps single operators on the kernels that read their weights as they are)
     for (const char* name : {"KXC_HIP_WINOGRAD_BF16X3", "KXC_HIP_CONV_WINOGRAD"})
         if (const char* e = std::getenv(name); e && e[0] == '0') return false;
