@@ -110,11 +110,7 @@ __device__ __forceinline__ void wino_weight_tile(const float* __restrict__ w, fl
     const int o0 = ob * 32, c0 = cb * kWeightTileC;
     const int cn = min(kWeightTileC, C - c0);     // 4 or 8 (C is a multiple of 4)
     const int tid = threadIdx.x;
-    for (int idx = tid; idx < 32 * kWeightTileC * 9; idx += 256) {
-        const int ol = idx / (kWeightTileC * 9), r = idx - ol * (kWeightTileC * 9);
-        const bool ok = o0 + ol < O && r < cn * 9;
-        raw[ol * RS + r] = ok ? w[(static_cast<int64_t>(o0 + ol) * C + c0) * 9 + r] : 0.0f;
-    }
+    wino_bx::stage_filters<kWeightTileC>(w, O, C, o0, c0, cn, raw);
     __syncthreads();
     const int cl = tid >> 5, ol = tid & 31;
     if (cl >= cn) return;
