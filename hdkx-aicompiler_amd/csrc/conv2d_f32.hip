@@ -1200,13 +1200,13 @@ const SmallVariant* SelectSmall(const kxc_hip_conv2d_desc* d, const ConvArgs& a,
         return second ? nullptr : CeilDiv(a.M, 16) * CeilDiv(a.O, 64) * SelectLanes() >= 512 ? v + 4 : v + 3;
     }
     if (d->kh != 3 || (second && !in_plan)) return nullptr;
-    const bool rows_fit = a.dw == 1 && SmallWords(v[0], a) * v[0].chunk <= v[0].xi * 64;
+    if (!by_name && (a.C < 64 || tiles > (second || a.O <= 16 ? 1600 : 800) || (!in_plan && tiles < 400))) return nullptr;
+    const bool rows_fit = a.dw == 1 && SmallWords(v[0], a) * v[0].chunk <= v[0].xi * 64;      // (walks the map: behind the cheap tests)
     if (by_name) {
         for (int i = rows_fit ? 0 : 1; i < 3; ++i)
             if (std::strcmp(forced, v[i].name) == 0) return v + i;
         return nullptr;
     }
-    if (a.C < 64 || tiles > (second || a.O <= 16 ? 1600 : 800) || (!in_plan && tiles < 400)) return nullptr;
     if (rows_fit && a.N * CeilDiv(a.OHW, 16) * CeilDiv(a.O, 16) * SelectLanes() <= kNumCUs) return v;
     return tiles <= kNumCUs ? v + 1 : v + 2;
 }
