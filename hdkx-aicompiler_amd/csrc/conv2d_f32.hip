@@ -1200,6 +1200,9 @@ const SmallVariant* SelectSmall(const kxc_hip_conv2d_desc* d, const ConvArgs& a,
         return second ? nullptr : CeilDiv(a.M, 16) * CeilDiv(a.O, 64) * SelectLanes() >= 512 ? v + 4 : v + 3;
     }
     if (d->kh != 3 || (second && !in_plan)) return nullptr;
+    // the second output reads the middle tap (padding 0 at stride 3, say, wants tap 0: the general kernel's ds_off)
+    int rh = 0, rw = 0;
+    if (second && (!PairTap(d, &rh, &rw) || rh != 1 || rw != 1)) return nullptr;
     if (!by_name && (a.C < 64 || tiles > (second || a.O <= 16 ? 1600 : 800) || (!in_plan && tiles < 400))) return nullptr;
     const bool rows_fit = a.dw == 1 && SmallWords(v[0], a) * v[0].chunk <= v[0].xi * 64;      // (walks the map: behind the cheap tests)
     if (by_name) {

@@ -5,6 +5,7 @@ convolution / gemm kernels, all int8), within 1e-3 for the matrix-core kernels w
 differs.  Large (full-size) cases use properties that need no CPU run: agreement between the
 matrix-core kernel and the bit-exact direct kernel, linearity, batch independence.
 """
+import ctypes
 import os
 
 import numpy as np
@@ -743,6 +744,35 @@ def test_conv_small_launch_kernels(pkg, orc, fast_orc, synth, shape):
             both.run([dev(x), dev(wt), dev(b), dev(r), y, dev(w2), dev(b), y2]); torch.cuda.synchronize()
             check(host(y), want, "first output %s" % (shape,))
             check(host(y2), (orc.conv2d(x, w2, s, 0) + b[None, :, None, None]).astype(np.float32), "second output %s" % (shape,))
+
+
+@pytest.mark.parametrize("h, w, stride, pad_h, pad_w, dil", [
+    (48, 48, 3, 0, 0, 1), (48, 48, 3, 1, 0, 1), (48, 48, 3, 0, 1, 1), (46, 48, 3, 2, 1, 1), (24, 24, 2, 1, 1, 1), (20, 20, 1, 2, 2, 2)])
+def test_plan_pair_second_output_reads_its_tap(pkg, h, w, stride, pad_h, pad_w, dil):
+    """A plan's two-output node: the 1x1 convolution's operand x[oh*s, ow*s] is tap (pad / dil) of the 3x3 window, which at
+    stride 3 need not be the middle one.  Both outputs against float64; a sum of k rounded products in any order is within
+    k * 2^-24 * sum |a b| of the exact one (4 more for bias, residual and the rounding of the output)."""
+    n, c, o = 1, 64, 64
+    d = pkg.ConvDesc(n, c, h, w, o, 3, 3, stride, stride, pad_h, pad_w, dil, dil, pkg.CONV_BIAS | pkg.CONV_RELU)
+    assert pkg.lib().kxc_hip_conv2d_pair_supported(ctypes.byref(d))
+    rng = np.random.default_rng(1000 * pad_h + 100 * pad_w + 10 * stride + dil)
+    x = rng.standard_normal((n, c, h, w)).astype(np.float32)
+    wt, w2 = (rng.standard_normal((o, c, k, k)).astype(np.float32) / np.float32(k * c ** 0.5) for k in (3, 1))
+    b, b2 = (rng.standard_normal(o).astype(np.float32) for _ in range(2))
+    t = lambda a: torch.from_numpy(a).double()
+    conv = lambda f, x, wt, b: f(torch.nn.functional.conv2d(t(f(x)), t(f(wt)), t(f(b)), stride, (pad_h, pad_w), dil).numpy())
+    one = lambda f, x, w2, b: f(torch.nn.functional.conv2d(t(f(x)), t(f(w2)), t(f(b)), stride).numpy())
+    same = lambda a: a
+    want, bound = conv(same, x, wt, b), (9 * c + 4) * 2.0 ** -24 * conv(np.abs, x, wt, b)
+    want2, bound2 = one(same, x, w2, b2), (c + 4) * 2.0 ** -24 * one(np.abs, x, w2, b2)
+    assert want.shape == want2.shape
+    plan = pkg.Plan(7)
+    plan.add_conv2d_pair(d, *([pkg.Buf.arg(i) for i in range(3)] + [pkg.Buf.none()] + [pkg.Buf.arg(i) for i in range(3, 7)]))
+    plan.finalize(0)
+    y, y2 = (torch.full(want.shape, float("nan"), device="cuda") for _ in range(2))
+    plan.run([dev(x), dev(wt), dev(b), y, dev(w2), dev(b2), y2]); torch.cuda.synchronize()
+    assert (np.abs(host(y) - np.maximum(want, 0)) <= bound).all()
+    assert (np.abs(host(y2) - want2) <= bound2).all()
 
 
 def test_conv_dilation(pkg, orc, synth):
