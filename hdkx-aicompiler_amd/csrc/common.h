@@ -98,9 +98,11 @@ struct SplitScratchLease {
     uint32_t* counters = nullptr;      // kSplitCounters arrival counters, all zero between launches
     std::unique_lock<std::mutex> lock;
 };
-// With `ready`: a buffer that would have to grow while the stream is being captured (no allocation is allowed there) is
-// not an error; *ready tells, and the caller takes a launch that needs none.
-int32_t AcquireSplitScratch(hipStream_t stream, size_t bytes, SplitScratchLease* lease, bool* ready = nullptr);
+int32_t AcquireSplitScratch(hipStream_t stream, size_t bytes, SplitScratchLease* lease);
+// Whether launches enqueued on a stream run one behind the other for as long as they live, so that they can share the
+// buffer of its handle: not while it is being captured (the graph may be replayed on another stream, beside calls on this
+// one or beside a second graph captured on it), and not hipStreamPerThread (one handle, a stream for every thread).
+bool StreamOrdersScratch(hipStream_t stream);
 int32_t LaunchSplitReduce(hipStream_t stream, const SplitReduceArgs& a);
 
 constexpr size_t kMaxLdsBytes = 160 * 1024;  // LDS of one gfx950 compute unit
@@ -160,7 +162,7 @@ int32_t LaunchPreparedWinograd(const PreparedWinograd* p, const float* x, const 
 void FreePreparedWinograd(PreparedWinograd* p);
 
 // A single nn_conv2d by the three-part Winograd kernel, filter transform included (conv2d_wino_f32.hip): which shapes it is
-// for, and the call.  *launched = false: the stream is being captured and the scratch for the filter would have to grow.
+// for, and the call.  *launched = false, nothing enqueued: the stream does not order the scratch that the filter takes.
 bool WinogradOperatorPreferred(const kxc_hip_conv2d_desc* desc);
 int32_t RunWinogradOperator(const kxc_hip_conv2d_desc* desc, const float* x, const float* w, const float* bias, const float* residual,
                             float* y, hipStream_t stream, bool* launched);

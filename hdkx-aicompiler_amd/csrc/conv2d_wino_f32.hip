@@ -921,14 +921,15 @@ bool WinogradOperatorPreferred(const kxc_hip_conv2d_desc* d) {
 
 int32_t RunWinogradOperator(const kxc_hip_conv2d_desc* desc, const float* x, const float* w, const float* bias, const float* residual,
                             float* y, hipStream_t stream, bool* launched) {
+    // (two kernels meet in the scratch: the filter's transform writes it, the convolution reads it)
+    *launched = StreamOrdersScratch(stream);
+    if (!*launched) return KXC_HIP_OK;
     WinoLaunch L;
     FillWinoArgs(desc, &L);
     ThreePartResolve(desc, &L, false);
     SplitScratchLease lease;      // held until the kernel that reads the filter is enqueued
-    *launched = true;
     // (the filter is transformed by every call: the caller may have changed it)
-    if (int32_t rc = AcquireSplitScratch(stream, L.bx.u_bytes, &lease, launched)) return rc;
-    if (!*launched) return KXC_HIP_OK;
+    if (int32_t rc = AcquireSplitScratch(stream, L.bx.u_bytes, &lease)) return rc;
     WinoWeightBatch jobs;
     std::memset(&jobs, 0, sizeof(jobs));
     const int64_t blocks = wino_bx::WeightTiles(desc->o, desc->c);

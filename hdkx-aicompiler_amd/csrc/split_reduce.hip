@@ -74,7 +74,7 @@ int32_t SelectLanes() {
 // A buffer that has been handed out stays allocated until the process ends, also after a larger one replaced it:
 // a captured graph may still hold its address.  Buffers double, so the retired ones add up to less than the
 // current one.
-int32_t AcquireSplitScratch(hipStream_t stream, size_t bytes, SplitScratchLease* lease, bool* ready) {
+int32_t AcquireSplitScratch(hipStream_t stream, size_t bytes, SplitScratchLease* lease) {
     struct Entry { int device; hipStream_t stream; float* ptr; uint32_t* counters; size_t bytes; std::mutex in_use; };
     static std::mutex mu;
     static std::vector<std::unique_ptr<Entry>> entries;      // entries are never removed: their addresses are stable
@@ -91,12 +91,6 @@ int32_t AcquireSplitScratch(hipStream_t stream, size_t bytes, SplitScratchLease*
         }
     }
     std::unique_lock<std::mutex> in_use(e->in_use);
-    if (e->bytes < bytes && ready) {
-        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-        KXC_HIP_CALL(hipStreamIsCapturing(stream, &status), "hipStreamIsCapturing");
-        *ready = status == hipStreamCaptureStatusNone;
-        if (!*ready) return KXC_HIP_OK;
-    }
     if (e->bytes < bytes) {
         size_t want = e->bytes ? 2 * e->bytes : (static_cast<size_t>(1) << 20);
         while (want < bytes) want *= 2;
@@ -115,6 +109,16 @@ int32_t AcquireSplitScratch(hipStream_t stream, size_t bytes, SplitScratchLease*
     lease->counters = e->counters;
     lease->lock = std::move(in_use);
     return KXC_HIP_OK;
+}
+
+bool StreamOrdersScratch(hipStream_t stream) {
+    if (stream == hipStreamPerThread) return false;
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &status) != hipSuccess) {
+        (void)hipGetLastError();      // (the null stream beside a global capture)
+        return false;
+    }
+    return status == hipStreamCaptureStatusNone;
 }
 
 int32_t LaunchSplitReduce(hipStream_t stream, const SplitReduceArgs& a) {

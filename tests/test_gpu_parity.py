@@ -852,6 +852,50 @@ def test_conv_operator_by_winograd(pkg, monkeypatch, n, c, h, w, o, p, forced):
     assert np.linalg.norm(got[near] - want[near]) <= 2 * (9 * c + 16) ** 0.5 * 2.0 ** -23 * np.linalg.norm(want[near].astype(np.float64)) + 1e-30
 
 
+def test_conv_operator_by_winograd_under_capture(pkg, monkeypatch):
+    """A large 3x3 call transforms its filter into the buffer of its stream handle, so a graph of it must not hold that buffer:
+    captured after an eager call has grown it, on hipStreamPerThread and in the entry point that allocates nothing the call runs
+    on the kernel without scratch, bit for bit the same.  Replays on another stream beside eager calls with other weights on
+    the capture stream, and of two graphs of one capture stream side by side, give what each gives alone."""
+    n, c, h, o = 16, 64, 56, 64
+    rng = np.random.default_rng(77)
+    x = dev(rng.standard_normal((n, c, h, h)).astype(np.float32))
+    w = [dev((rng.standard_normal((o, c, 3, 3)) / 24).astype(np.float32)) for _ in range(3)]
+    b = dev(rng.standard_normal(o).astype(np.float32))
+    assert pkg.conv2d_variant(x.shape, w[0].shape, 1, 1) == "winograd_f2k3_bf16x3"
+    plain = [pkg.conv2d(x, v, b, None, 1, 1, 1, True, out=torch.empty((n, o, h, h), device="cuda"), no_alloc=True) for v in w]
+    fast = pkg.conv2d(x, w[2], b, None, 1, 1, 1, True)
+    torch.cuda.synchronize()
+    assert not torch.equal(fast, plain[2])                   # (the other kernel: other roundings)
+    capture, other, third = (torch.cuda.Stream() for _ in range(3))
+    with torch.cuda.stream(capture):
+        assert torch.equal(pkg.conv2d(x, w[2], b, None, 1, 1, 1, True), fast)
+    torch.cuda.synchronize()
+    y = [torch.empty((n, o, h, h), device="cuda") for _ in range(2)]
+    graphs = [torch.cuda.CUDAGraph() for _ in range(2)]
+    for k in range(2):
+        with torch.cuda.graph(graphs[k], stream=capture):
+            pkg.conv2d(x, w[k], b, None, 1, 1, 1, True, out=y[k])
+    eager = torch.empty((n, o, h, h), device="cuda")
+    for replay in range(6):
+        for t in y + [eager]:
+            t.zero_()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(other):
+            graphs[0].replay()
+        with torch.cuda.stream(third):
+            graphs[1].replay()
+        with torch.cuda.stream(capture):
+            pkg.conv2d(x, w[2], b, None, 1, 1, 1, True, out=eager)
+        torch.cuda.synchronize()
+        assert torch.equal(y[0], plain[0]) and torch.equal(y[1], plain[1]) and torch.equal(eager, fast), "replay %d" % replay
+        assert torch.isfinite(pkg.relu(x)).all()             # eager work between the replays
+    monkeypatch.setattr(pkg.hipabi, "_stream", lambda: ctypes.c_void_p(2))        # hipStreamPerThread
+    got = pkg.conv2d(x, w[0], b, None, 1, 1, 1, True, out=y[0].zero_())
+    torch.cuda.synchronize()
+    assert torch.equal(got, plain[0])
+
+
 @pytest.mark.parametrize("n, c, h, w, o, k, s, p", [
     (1, 64, 9, 9, 1, 3, 1, 1), (2, 65, 8, 7, 17, 3, 1, 1), (1, 64, 13, 11, 31, 1, 1, 0), (3, 30, 12, 17, 5, 5, 1, 2), (2, 16, 19, 23, 16, 7, 2, 3),
     (1, 7, 5, 5, 31, 3, 2, 1), (1, 96, 3, 3, 48, 3, 1, 1), (1, 72, 1, 1, 40, 3, 1, 1), (1, 50, 7, 4, 33, 5, 2, 2), (1, 63, 5, 6, 70, 1, 1, 0), (9, 64, 56, 50, 16, 3, 1, 1)])
