@@ -1233,6 +1233,7 @@ struct ConvLaunch {
     int32_t kh = 0, kw = 0;
     int64_t total = 0;
     bool second = false;
+    bool in_plan = false;
 };
 
 // small = false: without the small-launch kernels (operands that are not aligned for them).
@@ -1240,6 +1241,7 @@ int32_t Conv2dResolve(const kxc_hip_conv2d_desc* desc, bool second, const char* 
     ConvArgs& a = L->a;
     if (int32_t rc = FillArgs(desc, &a, who)) return rc;
     L->second = second;
+    L->in_plan = in_plan;
     L->desc = *desc;
     L->kh = desc->kh; L->kw = desc->kw;
     L->total = static_cast<int64_t>(a.N) * a.O * a.OHW;
@@ -1401,7 +1403,7 @@ int32_t Conv2dLaunch(const ConvLaunch& L, const char* who, const float* x, const
     if (L.path == ConvLaunch::kSmall) {
         if (((reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(second ? second->w2 : w)) & 15u) != 0) {
             ConvLaunch other;       // weights are read in 16-byte words
-            if (int32_t rc = Conv2dResolve(&L.desc, L.second, who, &other, false, false)) return rc;
+            if (int32_t rc = Conv2dResolve(&L.desc, L.second, who, &other, L.in_plan, false)) return rc;
             return Conv2dLaunch(other, who, x, w, bias, residual, y, stream, no_alloc, second);
         }
         conv_small::Args b = L.sm;
@@ -1415,6 +1417,7 @@ int32_t Conv2dLaunch(const ConvLaunch& L, const char* who, const float* x, const
         return CheckLaunch(L.name);
     }
     SplitScratchLease lease;      // held until the adding kernel is enqueued
+    dim3 grid = L.grid;
     if (L.scratch_bytes > 0) {
         if (no_alloc) {
             // every kernel of the pair overwrites what it reads later, nothing has to start at zero
@@ -1423,13 +1426,26 @@ int32_t Conv2dLaunch(const ConvLaunch& L, const char* who, const float* x, const
                             who, L.scratch_bytes, kNoAllocScratchBytes);
             if (int32_t rc = NoAllocScratch(&a.partial)) return rc;
         } else {
-            if (int32_t rc = AcquireSplitScratch(s, L.scratch_bytes, &lease)) return rc;
+            // Launches that can do without the buffer of the stream's handle do so where the stream does not order its users:
+            // one thread per output, without scratch, is what these filters and shapes are compared with.  For the others
+            // a reduction in one piece would take up to five times as long (kxc_hip.h says what their graphs need); a
+            // plan's own graph is replayed on its capture stream.
+            bool split = L.in_plan || !(a.O < 32 || a.M < 32 || L.kh == 5) || StreamOrdersScratch(s);
+            if (split)
+                if (int32_t rc = AcquireSplitScratch(s, L.scratch_bytes, &lease)) return rc;
             a.partial = lease.ptr;
+            if (!split) {
+                a.gsplit = 1;
+                a.cps = a.nchunks;
+                a.div_gsplit = MakeFastDiv(1);
+                a.tiles_per_xcd = static_cast<int32_t>(CeilDiv(a.num_tiles, 8));
+                grid = dim3(static_cast<unsigned>(a.tiles_per_xcd * 8));
+            }
         }
     }
     if (L.lds_bytes > 64 * 1024)
         if (int32_t rc = GrantLds(reinterpret_cast<const void*>(L.kernel))) return rc;
-    hipLaunchKernelGGL(L.kernel, NoteGrid(L.grid), NoteBlock(L.block), NoteLds(L.lds_bytes), s, a);
+    hipLaunchKernelGGL(L.kernel, NoteGrid(grid), NoteBlock(L.block), NoteLds(L.lds_bytes), s, a);
     if (int32_t rc = CheckLaunch(L.name)) return rc;
     if (a.gsplit > 1) {
         SplitReduceArgs r;

@@ -668,11 +668,12 @@ int ThreePartSplit(int64_t units, int ksteps, int64_t out_elems) {
 
 // Measured on MI355X: 64 x 32 workgroups (four waves) are the fastest shape once there is one per two compute units;
 // smaller launches run faster as twice as many 64 x 16 workgroups of two waves.
-const WinoVariant* SelectWino(const kxc_hip_conv2d_desc* d) {
+// (three_part = false: the fp32 instructions)
+const WinoVariant* SelectWino(const kxc_hip_conv2d_desc* d, bool three_part = true) {
     if (const char* e = std::getenv("KXC_HIP_WINOGRAD_VARIANT")) {
         for (int i = 0; i < kNumWino; ++i)
             if (std::strcmp(e, kWino[i].name) == 0 && (kWino[i].ks == 1 || (d->c / 4) % kWino[i].ks == 0) &&
-                (kWino[i].kernel || ThreePartFits(d)))
+                (kWino[i].kernel || (three_part && ThreePartFits(d))))
                 return &kWino[i];
     }
     const int csteps = d->c / 4;
@@ -683,7 +684,7 @@ const WinoVariant* SelectWino(const kxc_hip_conv2d_desc* d) {
     // 30.0, 10 images (32 million; 7 x 7: 42) 27.1 / - / 26.1 / 28.0 against 20.7 / - / 25.6 / 30.6, 8 images (26 million; 7 x 7: 34)
     // 23.7 / 22.4 / 24.3 / 26.6 against 19.9 / 22.4 / 24.0 / 24.6.  KXC_HIP_WINOGRAD_BF16X3=0 keeps the fp32 instructions.
     const char* bx = std::getenv("KXC_HIP_WINOGRAD_BF16X3");
-    if (!(bx && bx[0] == '0') && Tiles(d) * lanes * d->o * d->c >= 36000000LL && ThreePartFits(d)) {
+    if (three_part && !(bx && bx[0] == '0') && Tiles(d) * lanes * d->o * d->c >= 36000000LL && ThreePartFits(d)) {
         for (int i = 0; i < kNumWino; ++i)
             if (!kWino[i].kernel) return &kWino[i];
     }
@@ -779,9 +780,9 @@ void FillWinoArgs(const kxc_hip_conv2d_desc* desc, WinoLaunch* L) {
     L->out_elems = static_cast<int64_t>(a.N) * a.O * a.OHW;
 }
 
-int32_t WinoResolve(const kxc_hip_conv2d_desc* desc, WinoLaunch* L) {
+int32_t WinoResolve(const kxc_hip_conv2d_desc* desc, WinoLaunch* L, bool three_part = true) {
     KXC_HIP_REQUIRE(desc && Supported(desc), "kxc_hip_conv2d_winograd_nchw_f32: unsupported shape");
-    const WinoVariant* v = SelectWino(desc);
+    const WinoVariant* v = SelectWino(desc, three_part);
     L->v = v;
     FillWinoArgs(desc, L);
     WinoArgs& a = L->a;
@@ -1017,9 +1018,15 @@ int32_t kxc_hip_conv2d_winograd_transform_weights(const kxc_hip_conv2d_desc* des
 
 int32_t kxc_hip_conv2d_winograd_nchw_f32(const kxc_hip_conv2d_desc* desc, const float* x, const float* u, const float* bias,
                                          const float* residual, float* y, void* stream) {
+    hipStream_t s = ResolveStream(stream);
     WinoLaunch L;
     if (int32_t rc = WinoResolve(desc, &L)) return rc;
-    return WinoRun(L, x, u, bias, residual, y, ResolveStream(stream));
+    // (launches that the fp32 instructions run in one piece stay without the shared buffer; `u` holds both forms)
+    if (L.three_part && L.scratch_bytes > 0 && !StreamOrdersScratch(s)) {
+        L = WinoLaunch();
+        if (int32_t rc = WinoResolve(desc, &L, false)) return rc;
+    }
+    return WinoRun(L, x, u, bias, residual, y, s);
 }
 
 }  // extern "C"

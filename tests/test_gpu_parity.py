@@ -896,6 +896,49 @@ def test_conv_operator_by_winograd_under_capture(pkg, monkeypatch):
     assert torch.equal(got, plain[0])
 
 
+@pytest.mark.parametrize("n, c, h, w, o, k, s, p, winograd", [
+    (2, 65, 8, 7, 17, 3, 1, 1, False), (1, 96, 3, 3, 48, 3, 1, 1, False), (8, 64, 27, 27, 96, 5, 1, 2, False), (12, 128, 28, 28, 128, 3, 1, 1, True)])
+def test_conv_split_launches_keep_shared_scratch_out_of_graphs(pkg, n, c, h, w, o, k, s, p, winograd):
+    """Launches whose eager form splits its reduction into the buffer of the stream's handle and that can do without: a graph of
+    one is captured without a first call, replays on another stream beside eager calls on the capture stream, and gives the
+    same bits when it is captured again after those calls.  9 c + 16 roundings of at most 2^-23 of a sum, of independent signs."""
+    rng = np.random.default_rng(n * c + o)
+    x, wt = rng.standard_normal((n, c, h, w)).astype(np.float32), [(rng.standard_normal((o, c, k, k)) / np.sqrt(c * k * k)).astype(np.float32) for _ in range(2)]
+    xd, wd = dev(x), [dev(v) for v in wt]
+    need = ctypes.c_size_t(0)
+    assert pkg.lib().kxc_hip_conv2d_scratch_needed(ctypes.byref(pkg.conv_desc(x.shape, wt[0].shape, s, p)), ctypes.byref(need)) == 0
+    assert winograd or need.value > 0
+    if winograd:
+        assert pkg.conv2d_winograd_variant(x.shape, wt[0].shape) == "winograd_f2k3_bf16x3"
+        wd = [pkg.conv2d_winograd_transform_weights(x.shape, v, p) for v in wd]
+    call = lambda i, y: pkg.conv2d_winograd(xd, wd[i], wt[i].shape, None, None, p, False, out=y) if winograd else pkg.conv2d(xd, wd[i], None, None, s, p, out=y)
+    want = [torch.nn.functional.conv2d(torch.from_numpy(x).double(), torch.from_numpy(v).double(), None, s, p).numpy() for v in wt]
+    y = [torch.empty(want[0].shape, device="cuda") for _ in range(3)]
+    close = lambda got, i: np.linalg.norm(host(got) - want[i]) <= (k * k * c + 16) ** 0.5 * 2.0 ** -23 * np.linalg.norm(want[i])
+    capture, other = torch.cuda.Stream(), torch.cuda.Stream()
+    graphs = [torch.cuda.CUDAGraph() for _ in range(2)]
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graphs[0], stream=capture):
+        call(0, y[0])
+    for replay in range(5):
+        y[0].zero_(); y[1].zero_()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(other):
+            graphs[0].replay()
+        with torch.cuda.stream(capture):
+            call(1, y[1])
+        torch.cuda.synchronize()
+        assert close(y[0], 0) and close(y[1], 1), "replay %d" % replay
+        if replay == 0:
+            first, eager = y[0].clone(), y[1].clone()
+        assert torch.equal(y[0], first) and torch.equal(y[1], eager), "replay %d" % replay
+    with torch.cuda.graph(graphs[1], stream=capture):
+        call(0, y[2])
+    graphs[1].replay()
+    torch.cuda.synchronize()
+    assert torch.equal(y[2], first)
+
+
 @pytest.mark.parametrize("n, c, h, w, o, k, s, p", [
     (1, 64, 9, 9, 1, 3, 1, 1), (2, 65, 8, 7, 17, 3, 1, 1), (1, 64, 13, 11, 31, 1, 1, 0), (3, 30, 12, 17, 5, 5, 1, 2), (2, 16, 19, 23, 16, 7, 2, 3),
     (1, 7, 5, 5, 31, 3, 2, 1), (1, 96, 3, 3, 48, 3, 1, 1), (1, 72, 1, 1, 40, 3, 1, 1), (1, 50, 7, 4, 33, 5, 2, 2), (1, 63, 5, 6, 70, 1, 1, 0), (9, 64, 56, 50, 16, 3, 1, 1)])
