@@ -98,7 +98,10 @@ struct SplitScratchLease {
     uint32_t* counters = nullptr;      // kSplitCounters arrival counters, all zero between launches
     std::unique_lock<std::mutex> lock;
 };
-int32_t AcquireSplitScratch(hipStream_t stream, size_t bytes, SplitScratchLease* lease);
+// A buffer that would have to grow while the stream is being captured (no allocation is allowed there), or that cannot be
+// allocated (KXC_HIP_SCRATCH_MAX bytes per buffer at most, where set), is not an error: *available tells, and the caller
+// takes a launch that needs none.
+int32_t AcquireSplitScratch(hipStream_t stream, size_t bytes, SplitScratchLease* lease, bool* available);
 // Whether launches enqueued on a stream run one behind the other for as long as they live, so that they can share the
 // buffer of its handle: not while it is being captured (the graph may be replayed on another stream, beside calls on this
 // one or beside a second graph captured on it), and not hipStreamPerThread (one handle, a stream for every thread).
@@ -162,7 +165,7 @@ int32_t LaunchPreparedWinograd(const PreparedWinograd* p, const float* x, const 
 void FreePreparedWinograd(PreparedWinograd* p);
 
 // A single nn_conv2d by the three-part Winograd kernel, filter transform included (conv2d_wino_f32.hip): which shapes it is
-// for, and the call.  *launched = false, nothing enqueued: the stream does not order the scratch that the filter takes.
+// for, and the call.  *launched = false, nothing enqueued: there is no scratch for the filter, or the stream does not order it.
 bool WinogradOperatorPreferred(const kxc_hip_conv2d_desc* desc);
 int32_t RunWinogradOperator(const kxc_hip_conv2d_desc* desc, const float* x, const float* w, const float* bias, const float* residual,
                             float* y, hipStream_t stream, bool* launched);

@@ -1432,7 +1432,7 @@ int32_t Conv2dLaunch(const ConvLaunch& L, const char* who, const float* x, const
             // plan's own graph is replayed on its capture stream.
             bool split = L.in_plan || !(a.O < 32 || a.M < 32 || L.kh == 5) || StreamOrdersScratch(s);
             if (split)
-                if (int32_t rc = AcquireSplitScratch(s, L.scratch_bytes, &lease)) return rc;
+                if (int32_t rc = AcquireSplitScratch(s, L.scratch_bytes, &lease, &split)) return rc;
             a.partial = lease.ptr;
             if (!split) {
                 a.gsplit = 1;

@@ -835,13 +835,22 @@ int32_t WinoRun(const WinoLaunch& L, const float* x, const float* u, const float
     WinoArgs a = L.a;
     a.x = x; a.u = u; a.bias = bias; a.res = residual; a.y = y;
     SplitScratchLease lease;      // held until the adding kernel is enqueued
-    if (L.scratch_bytes > 0) {
-        if (int32_t rc = AcquireSplitScratch(s, L.scratch_bytes, &lease)) return rc;
+    bool split = L.scratch_bytes > 0;
+    if (split) {
+        if (int32_t rc = AcquireSplitScratch(s, L.scratch_bytes, &lease, &split)) return rc;
         a.partial = lease.ptr;
         a.counters = lease.counters;
     }
+    // (no buffer to be had: the reduction in one piece)
+    auto whole = [](auto& args, int32_t steps) {
+        args.gsplit = 1;
+        args.steps_per_split = steps;
+        args.div_gsplit = MakeFastDiv(1);
+        args.units_per_xcd = static_cast<int32_t>(CeilDiv(args.num_units, 8));
+    };
     if (L.three_part) {
         wino_bx::Args b = L.bx;
+        if (!split) whole(b, b.ksteps);
         b.x = x; b.u = reinterpret_cast<const char*>(u) + L.u_offset; b.bias = bias; b.res = residual; b.y = y; b.partial = a.partial;
         void (*const bx)(const wino_bx::Args) = L.bx_plane == 0 ? wino_bx::wino_bf16x3_kernel<512, false> : wino_bx::wino_bf16x3_kernel<768, false>;
         if (int32_t rc = GrantLds(reinterpret_cast<const void*>(bx))) return rc;
@@ -855,13 +864,15 @@ int32_t WinoRun(const WinoLaunch& L, const float* x, const float* u, const float
         r.div_ohw = MakeFastDiv(b.OHW);
         return LaunchSplitReduce(s, r);
     }
-    void (*const kernel)(const WinoArgs) = L.fuse ? v->fuse_kernel : v->kernel;
+    if (L.scratch_bytes > 0 && !split) whole(a, a.csteps);
+    const bool fuse = L.fuse && split;
+    void (*const kernel)(const WinoArgs) = fuse ? v->fuse_kernel : v->kernel;
     if (L.lds_bytes > 64 * 1024)
         if (int32_t rc = GrantLds(reinterpret_cast<const void*>(kernel))) return rc;
     hipLaunchKernelGGL(kernel, NoteGrid(dim3(static_cast<unsigned>(a.units_per_xcd * 8))),
                        NoteBlock(dim3(64 * v->wk * v->wt * v->ks)), NoteLds(L.lds_bytes), s, a);
     if (int32_t rc = CheckLaunch(v->name)) return rc;
-    if (a.gsplit > 1 && !L.fuse) {
+    if (a.gsplit > 1 && !fuse) {
         SplitReduceArgs r;
         r.partial = a.partial; r.bias = bias; r.res = residual; r.y = y;
         r.gsplit = a.gsplit; r.total = static_cast<int32_t>(L.out_elems); r.O = a.O; r.flags = a.flags;
@@ -930,7 +941,8 @@ int32_t RunWinogradOperator(const kxc_hip_conv2d_desc* desc, const float* x, con
     ThreePartResolve(desc, &L, false);
     SplitScratchLease lease;      // held until the kernel that reads the filter is enqueued
     // (the filter is transformed by every call: the caller may have changed it)
-    if (int32_t rc = AcquireSplitScratch(stream, L.bx.u_bytes, &lease)) return rc;
+    if (int32_t rc = AcquireSplitScratch(stream, L.bx.u_bytes, &lease, launched)) return rc;
+    if (!*launched) return KXC_HIP_OK;
     WinoWeightBatch jobs;
     std::memset(&jobs, 0, sizeof(jobs));
     const int64_t blocks = wino_bx::WeightTiles(desc->o, desc->c);

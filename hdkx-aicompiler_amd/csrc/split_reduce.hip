@@ -74,7 +74,7 @@ int32_t SelectLanes() {
 // A buffer that has been handed out stays allocated until the process ends, also after a larger one replaced it:
 // a captured graph may still hold its address.  Buffers double, so the retired ones add up to less than the
 // current one.
-int32_t AcquireSplitScratch(hipStream_t stream, size_t bytes, SplitScratchLease* lease) {
+int32_t AcquireSplitScratch(hipStream_t stream, size_t bytes, SplitScratchLease* lease, bool* available) {
     struct Entry { int device; hipStream_t stream; float* ptr; uint32_t* counters; size_t bytes; std::mutex in_use; };
     static std::mutex mu;
     static std::vector<std::unique_ptr<Entry>> entries;      // entries are never removed: their addresses are stable
@@ -91,11 +91,21 @@ int32_t AcquireSplitScratch(hipStream_t stream, size_t bytes, SplitScratchLease*
         }
     }
     std::unique_lock<std::mutex> in_use(e->in_use);
+    *available = true;
     if (e->bytes < bytes) {
         size_t want = e->bytes ? 2 * e->bytes : (static_cast<size_t>(1) << 20);
         while (want < bytes) want *= 2;
         char* fresh = nullptr;
-        KXC_HIP_CALL(hipMalloc(reinterpret_cast<void**>(&fresh), kSplitCounterBytes + want), "hipMalloc(split scratch)");
+        const char* limit = std::getenv("KXC_HIP_SCRATCH_MAX");
+        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+        *available = !(limit && bytes > static_cast<size_t>(std::strtoull(limit, nullptr, 10))) &&
+                     hipStreamIsCapturing(stream, &status) == hipSuccess && status == hipStreamCaptureStatusNone &&
+                     (hipMalloc(reinterpret_cast<void**>(&fresh), kSplitCounterBytes + want) == hipSuccess ||
+                      hipMalloc(reinterpret_cast<void**>(&fresh), kSplitCounterBytes + (want = bytes)) == hipSuccess);
+        if (!*available) {
+            (void)hipGetLastError();      // (the refused call's: the next launch check must not find it)
+            return KXC_HIP_OK;
+        }
         NoteDeviceAllocation();
         // the arrival counters in front start at zero: a fill kernel on the caller's stream, ahead of the first
         // launch that counts (under stream capture it becomes a node of the graph, which is harmless)

@@ -171,7 +171,8 @@ typedef struct kxc_hip_conv2d_desc {
  * stride-1 calls, 5x5 filters and calls of fewer than 32 output channels or pixels take a kernel that needs no buffer (the
  * same bits whether or not an earlier call grew one).  Other launches with a split reduction use the buffer there too:
  * their graph must be replayed on the stream it was captured on (or with nothing else running on that stream's buffer),
- * after one eager call of the shape, and threads must not run them on hipStreamPerThread at the same time. */
+ * and threads must not run them on hipStreamPerThread at the same time.  A buffer that cannot be had (a first call under
+ * capture, no memory, more than KXC_HIP_SCRATCH_MAX bytes where the environment sets it) is done without, never an error. */
 int32_t kxc_hip_conv2d_nchw_f32(const kxc_hip_conv2d_desc* desc, const float* x, const float* w,
                                 const float* bias, const float* residual, float* y, void* stream);
 /* Name of the kernel variant the library would launch for this shape ("mfma_...", "winograd_..." or "direct") on a stream

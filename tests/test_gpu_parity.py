@@ -1473,6 +1473,89 @@ def test_plan_text_versions_1_and_2_still_load(pkg, synth):
     plan.close(); old.close()
 
 
+@pytest.mark.parametrize("n, c, h, o, stride, kind", [
+    (16, 64, 56, 64, 1, "winograd operator"), (1, 512, 7, 512, 1, "implicit GEMM"), (1, 256, 14, 256, 2, "implicit GEMM"),
+    (1, 256, 14, 512, 2, "pair"), (2, 128, 28, 128, 1, "fp32 filters"), (12, 128, 28, 128, 1, "three-part filters")])
+def test_conv_without_scratch(pkg, monkeypatch, n, c, h, o, stride, kind):
+    """Launches that keep intermediate values in the library's buffer run without it where it cannot be had: bounded to nothing
+    by KXC_HIP_SCRATCH_MAX, as when the device is out of memory, and in a first call under capture.  Nothing is allocated,
+    and results are within (9 c + 16)^1/2 roundings of 2^-23 of float64."""
+    rng = np.random.default_rng(n + c + h)
+    x, wt = rng.standard_normal((n, c, h, h)).astype(np.float32), (rng.standard_normal((o, c, 3, 3)) / np.sqrt(9 * c)).astype(np.float32)
+    w2 = (rng.standard_normal((o, c, 1, 1)) / np.sqrt(c)).astype(np.float32)
+    xd, wd, w2d = dev(x), dev(wt), dev(w2)
+    t = lambda a: torch.from_numpy(a).double()
+    want = [torch.nn.functional.conv2d(t(x), t(wt), None, stride, 1).numpy()]
+    if "filters" in kind:
+        assert pkg.conv2d_winograd_variant(x.shape, wt.shape).endswith("bf16x3") == ("three" in kind)
+        u = pkg.conv2d_winograd_transform_weights(x.shape, wd)
+    if kind == "pair":
+        want.append(torch.nn.functional.conv2d(t(x), t(w2), None, stride).numpy())
+    if kind == "winograd operator":
+        assert pkg.conv2d_variant(x.shape, wt.shape, 1, 1).startswith("winograd")
+    call = {"pair": lambda: pkg.conv2d_pair(xd, wd, None, None, w2d, None, stride, 1),
+            "winograd operator": lambda: [pkg.conv2d(xd, wd, None, None, stride, 1)], "implicit GEMM": lambda: [pkg.conv2d(xd, wd, None, None, stride, 1)],
+            "fp32 filters": lambda: [pkg.conv2d_winograd(xd, u, wt.shape)], "three-part filters": lambda: [pkg.conv2d_winograd(xd, u, wt.shape)]}[kind]
+    check = lambda got: all(np.linalg.norm(host(g) - v) <= (9 * c + 16) ** 0.5 * 2.0 ** -23 * np.linalg.norm(v) for g, v in zip(got, want))
+    allocations = pkg.lib().kxc_hip_debug_device_allocations
+    allocations.restype = ctypes.c_int64
+    for attempt in range(64):
+        handle = ctypes.c_void_p()                           # (kept: a destroyed stream's handle, and its buffer, may come again)
+        assert pkg.lib().kxc_hip_stream_create(0, ctypes.byref(handle)) == 0
+        stream = torch.cuda.ExternalStream(handle.value)
+        torch.cuda.synchronize()
+        before = allocations()
+        monkeypatch.setenv("KXC_HIP_SCRATCH_MAX", "0")
+        with torch.cuda.stream(stream):
+            limited = call()
+        torch.cuda.synchronize()
+        assert check(limited) and allocations() == before
+        monkeypatch.delenv("KXC_HIP_SCRATCH_MAX")
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            captured = call()
+        for _ in range(3):
+            for g in captured:
+                g.zero_()
+            graph.replay()
+            assert check(captured) and torch.isfinite(pkg.relu(xd)).all()
+        assert allocations() == before
+        with torch.cuda.stream(stream):
+            eager = call()
+        torch.cuda.synchronize()
+        assert check(eager)
+        if allocations() > before:                           # the stream's handle had no buffer all along
+            return
+    raise AssertionError("every stream handle had a buffer")
+
+
+def test_plan_graph_captured_on_weights_off_a_16_byte_boundary(pkg):
+    """A small-launch node reads its weights in 16-byte words; weights that are not aligned take the general kernel, whose
+    split reduction needs a buffer that the plan's eager first run, on aligned weights, did not ask for.  The run that
+    captures must do without it."""
+    n, c, h, o = 1, 64, 28, 64
+    rng = np.random.default_rng(31)
+    x, wt = rng.standard_normal((n, c, h, h)).astype(np.float32), (rng.standard_normal((o, c, 3, 3)) / 24).astype(np.float32)
+    want = torch.nn.functional.conv2d(torch.from_numpy(x).double(), torch.from_numpy(wt).double(), None, 1, 1).numpy()
+    plan = pkg.Plan(3)
+    plan.add_conv2d(pkg.ConvDesc(n, c, h, h, o, 3, 3, 1, 1, 1, 1, 1, 1, 0), pkg.Buf.arg(0), pkg.Buf.arg(1), pkg.Buf.none(), pkg.Buf.none(), pkg.Buf.arg(2))
+    plan.finalize(0)
+    assert "_small" in plan.node_symbol(0)
+    room = torch.zeros(wt.size + 4, device="cuda")
+    room[1:1 + wt.size] = dev(wt).reshape(-1)
+    shifted = room[1:1 + wt.size].view(wt.shape)
+    xd, wd, y = dev(x), dev(wt), torch.empty(want.shape, device="cuda")
+    stream = torch.cuda.Stream()
+    plan.enable_graph(True)
+    torch.cuda.synchronize()
+    for w in (wd, shifted, shifted, shifted, wd, wd):
+        y.zero_(); torch.cuda.synchronize()
+        plan.run([xd, w, y], stream.cuda_stream)
+        stream.synchronize()
+        assert np.linalg.norm(host(y) - want) <= (9 * c + 16) ** 0.5 * 2.0 ** -23 * np.linalg.norm(want)
+    plan.close()
+
+
 def test_plan_hip_graph_replay(pkg):
     """A launch plan replayed as a captured HIP graph gives the eager result on every replay, with eager work and
     synchronisations in between, and re-captures when an argument pointer changes.  Batch 1 exercises the
