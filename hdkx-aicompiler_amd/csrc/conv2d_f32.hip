@@ -1501,7 +1501,10 @@ int32_t LaunchPreparedConv2d(const PreparedConv* p, const float* x, const float*
     return Conv2dLaunch(p->launch, p->who.c_str(), x, w, bias, residual, y, stream, false, p->launch.second ? &second : nullptr);
 }
 
-const char* PreparedConvName(const PreparedConv* p) { return p->launch.name; }
+const char* PreparedConvName(const PreparedConv* p) {
+    if (p->launch.path == ConvLaunch::kSmall) return p->launch.name;
+    return p->launch.second ? kxc_hip_conv2d_pair_variant(&p->launch.desc) : kxc_hip_conv2d_node_variant(&p->launch.desc);
+}
 
 // Against the Winograd kernel with its adding launch (us, residual and ReLU): 64 channels at 56 x 56 batch 1 10.2 -> 8.7, batch 2
 // (1568 tiles) 12.9 against 14.6; 128 at 28 x 28 batch 2 13.0 -> 12.0; 256 at 14 x 14 batch 1 10.7 -> 7.5, batch 2 13.0 -> 11.2,
@@ -1519,7 +1522,7 @@ void FreePreparedConv(PreparedConv* p) { delete p; }
 
 extern "C" {
 
-const char* kxc_hip_conv2d_node_variant(const kxc_hip_conv2d_desc* desc) {
+static const char* ConvVariantName(const kxc_hip_conv2d_desc* desc, bool in_plan) {
     ConvArgs a;
     if (FillArgs(desc, &a, "kxc_hip_conv2d_variant") != KXC_HIP_OK) return "invalid";
     if (desc->flags & KXC_HIP_CONV_HPOOL) {
@@ -1527,7 +1530,7 @@ const char* kxc_hip_conv2d_node_variant(const kxc_hip_conv2d_desc* desc) {
         return HpoolChoice(desc, a, &hp) ? hp.v->name : "unsupported";
     }
     if (desc->flags & KXC_HIP_CONV_FORCE_DIRECT) return "direct";
-    if (const SmallVariant* v = SelectSmall(desc, a, false, false)) return v->name;
+    if (const SmallVariant* v = SelectSmall(desc, a, false, in_plan)) return v->name;
     if (UseSmall1x1(desc, a)) return "mfma_k1x1_small";
     ApplyRowView(&a, desc->kh);
     Choice c;
@@ -1535,8 +1538,10 @@ const char* kxc_hip_conv2d_node_variant(const kxc_hip_conv2d_desc* desc) {
     return c.v ? c.v->name : "direct";
 }
 
+const char* kxc_hip_conv2d_node_variant(const kxc_hip_conv2d_desc* desc) { return ConvVariantName(desc, true); }
+
 const char* kxc_hip_conv2d_variant(const kxc_hip_conv2d_desc* desc) {
-    return desc && WinogradOperatorPreferred(desc) ? kWinogradOperatorName : kxc_hip_conv2d_node_variant(desc);
+    return desc && WinogradOperatorPreferred(desc) ? kWinogradOperatorName : ConvVariantName(desc, false);
 }
 
 int32_t kxc_hip_conv2d_nchw_f32(const kxc_hip_conv2d_desc* desc, const float* x, const float* w, const float* bias,

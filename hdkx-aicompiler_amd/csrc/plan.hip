@@ -788,19 +788,18 @@ int32_t kxc_hip_plan_finalize(kxc_hip_plan* plan, size_t workspace_bytes) {
     for (Node& n : plan->nodes) {
         if (n.kind != NodeKind::kConv2D) continue;
         KXC_HIP_CALL(hipSetDevice(plan->device_id), "HIP SetDevice");
-        const char* variant = n.i32[0] == 1   ? kxc_hip_conv2d_winograd_variant(&n.conv)
-                              : n.i32[0] == 2 ? kxc_hip_conv2d_pair_variant(&n.conv)
-                                              : kxc_hip_conv2d_node_variant(&n.conv);
+        const char* variant = nullptr;
         // (a small Winograd node runs on its weights as they are, in one launch)
         if (n.i32[0] == 1 && !kxc_hip::SmallConvBeatsWinograd(&n.conv)) {
             kxc_hip::PreparedWinograd* p = nullptr;
             if (int32_t rc = kxc_hip::PrepareWinograd(&n.conv, &p)) return rc;
             n.prepared_wino.reset(p, kxc_hip::FreePreparedWinograd);
+            variant = kxc_hip_conv2d_winograd_variant(&n.conv);
         } else {
             kxc_hip::PreparedConv* p = nullptr;
             if (int32_t rc = kxc_hip::PrepareConv2d(&n.conv, n.i32[0] == 2, &p)) return rc;
             n.prepared_conv.reset(p, kxc_hip::FreePreparedConv);
-            if (std::strstr(kxc_hip::PreparedConvName(p), "_small")) variant = kxc_hip::PreparedConvName(p);
+            variant = kxc_hip::PreparedConvName(p);
         }
         const std::string prefix = "kxc_conv2d_nchw_f32.";
         const size_t end = n.symbol.find_first_of("+|", prefix.size());

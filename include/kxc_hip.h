@@ -178,7 +178,8 @@ int32_t kxc_hip_conv2d_nchw_f32(const kxc_hip_conv2d_desc* desc, const float* x,
 /* Name of the kernel variant the library would launch for this shape ("mfma_...", "winograd_..." or "direct") on a stream
  * that is not being captured. */
 const char* kxc_hip_conv2d_variant(const kxc_hip_conv2d_desc* desc);
-/* The same for a launch plan's kxc_hip_plan_add_conv2d node, which reads its weights as they are ("mfma_..." or "direct"). */
+/* The same for a launch plan's kxc_hip_plan_add_conv2d node, which reads its weights as they are ("mfma_..." or "direct"):
+ * the name in the node's symbol. */
 const char* kxc_hip_conv2d_node_variant(const kxc_hip_conv2d_desc* desc);
 /* The same operator for callers that cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  Same arguments and

@@ -1556,6 +1556,24 @@ def test_plan_graph_captured_on_weights_off_a_16_byte_boundary(pkg):
     plan.close()
 
 
+@pytest.mark.parametrize("desc", [
+    (1, 256, 14, 14, 256, 3, 1, 1), (1, 512, 7, 7, 512, 3, 1, 1), (1, 128, 28, 28, 128, 3, 1, 1), (2, 128, 28, 28, 128, 3, 1, 1), (8, 64, 56, 56, 64, 3, 1, 1),
+    (1, 64, 56, 56, 128, 1, 2, 0), (1, 3, 224, 224, 64, 7, 2, 3), (1, 5, 4, 4, 3, 3, 1, 1)], ids=lambda d: "x".join(map(str, d)))
+def test_plan_node_variant_names_the_launched_kernel(pkg, desc):
+    """kxc_hip_conv2d_node_variant says beforehand what a plan's node launches (the single operator may take another kernel)."""
+    n, c, h, w, o, k, s, p = desc
+    d = pkg.ConvDesc(n, c, h, w, o, k, k, s, s, p, p, 1, 1, 0)
+    name = pkg.lib().kxc_hip_conv2d_node_variant
+    name.restype = ctypes.c_char_p
+    expected = name(ctypes.byref(d)).decode()
+    plan = pkg.Plan(3)
+    plan.add_conv2d(d, pkg.Buf.arg(0), pkg.Buf.arg(1), pkg.Buf.none(), pkg.Buf.none(), pkg.Buf.arg(2))
+    added = plan.node_symbol(0)
+    plan.finalize(0)
+    assert plan.node_symbol(0) == added == "kxc_conv2d_nchw_f32." + expected
+    plan.close()
+
+
 def test_plan_hip_graph_replay(pkg):
     """A launch plan replayed as a captured HIP graph gives the eager result on every replay, with eager work and
     synchronisations in between, and re-captures when an argument pointer changes.  Batch 1 exercises the
