@@ -159,7 +159,10 @@ const char* PreparedConvName(const PreparedConv* p);
 bool SmallConvBeatsWinograd(const kxc_hip_conv2d_desc* desc);      // a plan's Winograd node is better launched as PreparedConv
 void FreePreparedConv(PreparedConv* p);
 struct PreparedWinograd;
-int32_t PrepareWinograd(const kxc_hip_conv2d_desc* desc, PreparedWinograd** out);
+// A node whose filter buffer has u_bytes, holding the one form that the launch reads.  *out = nullptr: no form fits.
+int32_t PrepareWinograd(const kxc_hip_conv2d_desc* desc, size_t u_bytes, PreparedWinograd** out);
+const char* PreparedWinogradName(const PreparedWinograd* p);
+size_t WinogradF32FilterBytes(const kxc_hip_conv2d_desc* desc);
 int32_t LaunchPreparedWinograd(const PreparedWinograd* p, const float* x, const float* u, const float* bias,
                                const float* residual, float* y, hipStream_t stream);
 void FreePreparedWinograd(PreparedWinograd* p);
@@ -176,8 +179,8 @@ constexpr uint32_t kWinoFormF32 = 1, kWinoFormThreePart = 2;
 struct WinoWeightJob {
     const kxc_hip_conv2d_desc* desc;
     const float* w;      // OIHW weights
-    float* u;            // kxc_hip_conv2d_winograd_weight_bytes(desc) bytes
-    uint32_t forms;      // kWinoForm*: the forms of the filter to write (PreparedWinogradForms: what a launch reads)
+    float* u;            // where they go, the fp32 form first
+    uint32_t forms;      // kWinoForm*: the forms of the filter to write (PreparedWinogradForms: what a node's launch reads)
 };
 uint32_t PreparedWinogradForms(const PreparedWinograd* p);
 int32_t LaunchWinogradWeightTransforms(const WinoWeightJob* jobs, int32_t count, hipStream_t stream);

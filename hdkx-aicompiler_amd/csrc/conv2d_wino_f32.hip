@@ -27,6 +27,7 @@
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <type_traits>
 #include <utility>
@@ -614,7 +615,8 @@ bool SupportedAnyC(const kxc_hip_conv2d_desc* d) {
 }
 bool Supported(const kxc_hip_conv2d_desc* d) { return SupportedAnyC(d) && d->c % 4 == 0; }
 
-// A filter buffer holds both forms, the fp32 one first: which of them a launch reads depends on the batch it runs on.
+// The filter buffer of the entry points holds both forms, the fp32 one first: which of them a launch reads depends on the
+// batch it runs on.  A plan's node, whose launch is known, has a buffer for one form (PrepareWinograd).
 size_t F32FilterBytes(const kxc_hip_conv2d_desc* d) { return static_cast<size_t>(CeilDiv(d->o, 32)) * 32 * static_cast<size_t>(d->c) * 64; }
 
 // Whether the patch of every workgroup of the three-part kernel fits its LDS planes.
@@ -890,12 +892,19 @@ struct PreparedWinograd {
     WinoLaunch launch;
 };
 
-int32_t PrepareWinograd(const kxc_hip_conv2d_desc* desc, PreparedWinograd** out) {
-    PreparedWinograd* p = new PreparedWinograd;
-    if (int32_t rc = WinoResolve(desc, &p->launch)) { delete p; return rc; }
-    *out = p;
+int32_t PrepareWinograd(const kxc_hip_conv2d_desc* desc, size_t u_bytes, PreparedWinograd** out) {
+    *out = nullptr;
+    std::unique_ptr<PreparedWinograd> p(new PreparedWinograd);
+    if (int32_t rc = WinoResolve(desc, &p->launch, u_bytes >= wino_bx::WeightBytes(desc->o, desc->c))) return rc;
+    if (!p->launch.three_part && u_bytes < F32FilterBytes(desc)) return KXC_HIP_OK;
+    p->launch.u_offset = 0;
+    *out = p.release();
     return KXC_HIP_OK;
 }
+
+const char* PreparedWinogradName(const PreparedWinograd* p) { return p->launch.v->name; }
+
+size_t WinogradF32FilterBytes(const kxc_hip_conv2d_desc* desc) { return F32FilterBytes(desc); }
 
 int32_t LaunchPreparedWinograd(const PreparedWinograd* p, const float* x, const float* u, const float* bias,
                                const float* residual, float* y, hipStream_t stream) {
@@ -982,7 +991,7 @@ int32_t LaunchWinogradWeightTransforms(const WinoWeightJob* jobs, int32_t count,
             const bool three = form == kWinoFormThreePart;
             const int64_t O = job.desc->o, C = job.desc->c;
             b.w[b.count] = job.w;
-            b.u[b.count] = reinterpret_cast<char*>(job.u) + (three ? F32FilterBytes(job.desc) : 0);
+            b.u[b.count] = reinterpret_cast<char*>(job.u) + (three && (job.forms & kWinoFormF32) ? F32FilterBytes(job.desc) : 0);
             b.O[b.count] = static_cast<int32_t>(O); b.C[b.count] = static_cast<int32_t>(C);
             b.first_block[b.count] = static_cast<int32_t>(blocks);
             if (three) b.three_part |= 1u << b.count;
@@ -1018,6 +1027,13 @@ int32_t kxc_hip_conv2d_winograd_weight_bytes(const kxc_hip_conv2d_desc* desc, si
     KXC_HIP_REQUIRE(desc && out_bytes, "kxc_hip_conv2d_winograd_weight_bytes: NULL argument");
     KXC_HIP_REQUIRE(Supported(desc), "kxc_hip_conv2d_winograd_weight_bytes: shape is not a 3x3 stride-1 convolution with C %% 4 == 0");
     *out_bytes = F32FilterBytes(desc) + wino_bx::WeightBytes(desc->o, desc->c);
+    return KXC_HIP_OK;
+}
+
+int32_t kxc_hip_conv2d_winograd_node_bytes(const kxc_hip_conv2d_desc* desc, size_t* out_bytes) {
+    KXC_HIP_REQUIRE(desc && out_bytes, "kxc_hip_conv2d_winograd_node_bytes: NULL argument");
+    KXC_HIP_REQUIRE(Supported(desc), "kxc_hip_conv2d_winograd_node_bytes: shape is not a 3x3 stride-1 convolution with C %% 4 == 0");
+    *out_bytes = SmallConvBeatsWinograd(desc) ? 0 : SelectWino(desc)->kernel ? F32FilterBytes(desc) : wino_bx::WeightBytes(desc->o, desc->c);
     return KXC_HIP_OK;
 }
 

@@ -69,6 +69,13 @@ int64_t PoolOutDim(const kxc_hip_pool2d_desc& d, int64_t in, int64_t k, int64_t 
     return (d.ceil_mode ? (span + s - 1) / s : span / s) + 1;      // as the pooling entry points size their output
 }
 
+// Bytes of a Winograd node's transformed-filter buffer: dims[0], and kFilterRoomNone for an empty one.  Plans written
+// before the field was used have 0 there and room for the fp32 form.
+constexpr int64_t kFilterRoomNone = -1;
+size_t FilterRoom(const Node& n) {
+    return n.dims[0] > 0 ? static_cast<size_t>(n.dims[0]) : n.dims[0] == 0 ? kxc_hip::WinogradF32FilterBytes(&n.conv) : 0;
+}
+
 // Bytes of every operand whose size follows from the node's geometry (module kernels' parameters are checked by
 // offset only).
 void OperandExtents(const Node& n, std::vector<std::pair<kxc_hip_buf, size_t>>* out) {
@@ -87,10 +94,7 @@ void OperandExtents(const Node& n, std::vector<std::pair<kxc_hip_buf, size_t>>* 
             add(n.bufs[2], d.o);
             add(n.bufs[3], y);
             add(n.bufs[4], y);
-            if (n.i32[0] == 1) {
-                size_t u = 0;
-                if (kxc_hip_conv2d_winograd_weight_bytes(&d, &u) == KXC_HIP_OK) add(n.bufs[5], static_cast<int64_t>(u), 1);
-            }
+            if (n.i32[0] == 1) add(n.bufs[5], static_cast<int64_t>(FilterRoom(n)), 1);
             if (n.i32[0] == 2 && n.params.size() == 3) {
                 add(n.params[0], static_cast<int64_t>(d.o) * d.c);
                 add(n.params[1], d.o);
@@ -350,6 +354,14 @@ int32_t kxc_hip_plan_add_conv2d(kxc_hip_plan* plan, const kxc_hip_conv2d_desc* d
 
 int32_t kxc_hip_plan_add_conv2d_winograd(kxc_hip_plan* plan, const kxc_hip_conv2d_desc* desc, kxc_hip_buf x, kxc_hip_buf w,
                                          kxc_hip_buf bias, kxc_hip_buf residual, kxc_hip_buf y, kxc_hip_buf u) {
+    size_t u_bytes = 0;
+    if (desc && kxc_hip_conv2d_winograd_supported(desc))
+        if (int32_t rc = kxc_hip_conv2d_winograd_weight_bytes(desc, &u_bytes)) return rc;
+    return kxc_hip_plan_add_conv2d_winograd_sized(plan, desc, x, w, bias, residual, y, u, u_bytes);
+}
+
+int32_t kxc_hip_plan_add_conv2d_winograd_sized(kxc_hip_plan* plan, const kxc_hip_conv2d_desc* desc, kxc_hip_buf x, kxc_hip_buf w,
+                                               kxc_hip_buf bias, kxc_hip_buf residual, kxc_hip_buf y, kxc_hip_buf u, size_t u_bytes) {
     const char* who = "kxc_hip_plan_add_conv2d_winograd";
     KXC_PLAN_BEGIN(who);
     KXC_HIP_REQUIRE(desc != nullptr, "%s: desc is NULL", who);
@@ -361,6 +373,7 @@ int32_t kxc_hip_plan_add_conv2d_winograd(kxc_hip_plan* plan, const kxc_hip_conv2
     Node& n = plan->nodes.back();
     n.i32[0] = 1;
     n.bufs[5] = u;
+    n.dims[0] = u_bytes > 0 ? static_cast<int64_t>(u_bytes) : kFilterRoomNone;
     n.symbol = std::string("kxc_conv2d_nchw_f32.") + kxc_hip_conv2d_winograd_variant(desc);
     if (desc->flags & KXC_HIP_CONV_BIAS) n.symbol += "+bias";
     if (desc->flags & KXC_HIP_CONV_RESIDUAL) n.symbol += "+add";
@@ -788,19 +801,40 @@ int32_t kxc_hip_plan_finalize(kxc_hip_plan* plan, size_t workspace_bytes) {
     for (Node& n : plan->nodes) {
         if (n.kind != NodeKind::kConv2D) continue;
         KXC_HIP_CALL(hipSetDevice(plan->device_id), "HIP SetDevice");
-        const char* variant = nullptr;
-        // (a small Winograd node runs on its weights as they are, in one launch)
+        n.prepared_wino.reset();
+        n.prepared_conv.reset();
+        // (a small Winograd node, and one whose filter buffer holds no form, runs on its weights as they are, in one launch)
         if (n.i32[0] == 1 && !kxc_hip::SmallConvBeatsWinograd(&n.conv)) {
             kxc_hip::PreparedWinograd* p = nullptr;
-            if (int32_t rc = kxc_hip::PrepareWinograd(&n.conv, &p)) return rc;
-            n.prepared_wino.reset(p, kxc_hip::FreePreparedWinograd);
-            variant = kxc_hip_conv2d_winograd_variant(&n.conv);
-        } else {
+            if (int32_t rc = kxc_hip::PrepareWinograd(&n.conv, FilterRoom(n), &p)) return rc;
+            if (p) n.prepared_wino.reset(p, kxc_hip::FreePreparedWinograd);
+        }
+        if (!n.prepared_wino) {
             kxc_hip::PreparedConv* p = nullptr;
             if (int32_t rc = kxc_hip::PrepareConv2d(&n.conv, n.i32[0] == 2, &p)) return rc;
             n.prepared_conv.reset(p, kxc_hip::FreePreparedConv);
-            variant = kxc_hip::PreparedConvName(p);
         }
+    }
+    // Nodes that share a filter buffer (the shares of a batch) read one form of it: where their shapes would take different
+    // ones, or one of them has room for the fp32 form only, that one.
+    auto shares_filter = [](const Node& a, const Node& b) {
+        return a.bufs[5].kind == b.bufs[5].kind && a.bufs[5].index_or_offset == b.bufs[5].index_or_offset;
+    };
+    for (Node& n : plan->nodes) {
+        if (!n.prepared_wino || kxc_hip::PreparedWinogradForms(n.prepared_wino.get()) == kxc_hip::kWinoFormF32) continue;
+        for (const Node& other : plan->nodes) {
+            if (!other.prepared_wino || !shares_filter(n, other) || kxc_hip::PreparedWinogradForms(other.prepared_wino.get()) != kxc_hip::kWinoFormF32) continue;
+            KXC_HIP_REQUIRE(FilterRoom(n) >= kxc_hip::WinogradF32FilterBytes(&n.conv),
+                            "kxc_hip_plan_finalize: nodes that share a transformed filter need room for its fp32 form");
+            kxc_hip::PreparedWinograd* p = nullptr;
+            if (int32_t rc = kxc_hip::PrepareWinograd(&n.conv, kxc_hip::WinogradF32FilterBytes(&n.conv), &p)) return rc;
+            n.prepared_wino.reset(p, kxc_hip::FreePreparedWinograd);
+            break;
+        }
+    }
+    for (Node& n : plan->nodes) {
+        if (n.kind != NodeKind::kConv2D) continue;
+        const char* variant = n.prepared_wino ? kxc_hip::PreparedWinogradName(n.prepared_wino.get()) : kxc_hip::PreparedConvName(n.prepared_conv.get());
         const std::string prefix = "kxc_conv2d_nchw_f32.";
         const size_t end = n.symbol.find_first_of("+|", prefix.size());
         if (n.symbol.compare(0, prefix.size(), prefix) == 0)
@@ -1286,8 +1320,15 @@ int32_t kxc_hip_plan_serialize(const kxc_hip_plan* plan, char* buffer, size_t ca
     char tmp[96];
     auto I = [&](long long v) { std::snprintf(tmp, sizeof(tmp), " %lld", v); out += tmp; };
     auto F = [&](float v) { std::snprintf(tmp, sizeof(tmp), " %a", static_cast<double>(v)); out += tmp; };
-    // (version 2 added the plan's select_lanes and every node's chain, version 3 the weight packs)
-    out += "kxc_hip_plan 3";
+    // (version 2 added the plan's select_lanes and every node's chain, version 3 the weight packs; version 4, written only
+    // where a reader of version 3 would assume more, Winograd nodes whose filter buffer has room for one form or none)
+    bool one_form = false;
+    for (const Node& n : plan->nodes) {
+        size_t both = 0;
+        if (n.kind == NodeKind::kConv2D && n.i32[0] == 1 && n.dims[0] != 0 && kxc_hip_conv2d_winograd_weight_bytes(&n.conv, &both) == KXC_HIP_OK)
+            one_form = one_form || FilterRoom(n) < both;
+    }
+    out += one_form ? "kxc_hip_plan 4" : "kxc_hip_plan 3";
     I(plan->num_args); I(static_cast<long long>(plan->workspace_bytes)); I(static_cast<long long>(plan->nodes.size()));
     I(plan->select_lanes);
     I(static_cast<long long>(plan->packs.size()));
@@ -1354,7 +1395,7 @@ int32_t kxc_hip_plan_deserialize(const char* text, int32_t device_id, kxc_hip_mo
     in >> magic >> version >> num_args >> workspace >> count;
     if (in && version >= 2) in >> select_lanes;
     if (in && version >= 3) in >> num_packs;
-    KXC_HIP_REQUIRE(in && magic == "kxc_hip_plan" && version >= 1 && version <= 3, "%s: not a version-1, -2 or -3 plan", who);
+    KXC_HIP_REQUIRE(in && magic == "kxc_hip_plan" && version >= 1 && version <= 4, "%s: not a version-1, -2, -3 or -4 plan", who);
     KXC_HIP_REQUIRE(num_packs >= 0 && num_packs < (1 << 20), "%s: implausible header", who);
     KXC_HIP_REQUIRE(select_lanes >= 1 && select_lanes <= 16, "%s: implausible header", who);
     KXC_HIP_REQUIRE(num_args >= 0 && num_args < (1 << 20) && workspace >= 0 && count >= 0 && count < (1 << 24),
@@ -1420,7 +1461,7 @@ int32_t kxc_hip_plan_deserialize(const char* text, int32_t device_id, kxc_hip_mo
             (n.i32[0] != 0 || !kxc_hip_conv2d_hpool_supported(&n.conv)))
             return fail("bad convolution node with the pooling epilogue");
         if (n.kind == NodeKind::kConv2D && n.i32[0] == 1 &&
-            (!kxc_hip_conv2d_winograd_supported(&n.conv) || n.bufs[5].kind != KXC_HIP_BUF_WORKSPACE))
+            (!kxc_hip_conv2d_winograd_supported(&n.conv) || n.bufs[5].kind != KXC_HIP_BUF_WORKSPACE || n.dims[0] < kFilterRoomNone))
             return fail("bad Winograd convolution node");
         if (n.kind == NodeKind::kConv2D && n.i32[0] == 2 &&
             (!kxc_hip_conv2d_pair_supported(&n.conv) || n.params.size() != 3 || n.params[0].kind == KXC_HIP_BUF_NONE ||

@@ -214,6 +214,13 @@ def conv2d_winograd_weight_bytes(x_shape, w_shape, pad=1):
     return nbytes.value
 
 
+def conv2d_winograd_node_bytes(desc):
+    """Bytes of transformed filter that a plan's Winograd node of this shape reads (0: it reads its weights as they are)."""
+    nbytes = C.c_size_t(0)
+    _check(lib().kxc_hip_conv2d_winograd_node_bytes(C.byref(desc), C.byref(nbytes)))
+    return nbytes.value
+
+
 def set_select_lanes(lanes):
     """Variant selection of this thread's stand-alone launches and queries assumes `lanes` equal launches side by
     side (kxc_hip_set_select_lanes); returns the previous value."""
@@ -625,8 +632,11 @@ class Plan:
     def add_conv2d(self, desc, x, w, bias, residual, y):
         _check(lib().kxc_hip_plan_add_conv2d(self._h, C.byref(desc), x, w, bias, residual, y))
 
-    def add_conv2d_winograd(self, desc, x, w, bias, residual, y, u):
-        _check(lib().kxc_hip_plan_add_conv2d_winograd(self._h, C.byref(desc), x, w, bias, residual, y, u))
+    def add_conv2d_winograd(self, desc, x, w, bias, residual, y, u, u_bytes=None):
+        if u_bytes is None:
+            _check(lib().kxc_hip_plan_add_conv2d_winograd(self._h, C.byref(desc), x, w, bias, residual, y, u))
+        else:
+            _check(lib().kxc_hip_plan_add_conv2d_winograd_sized(self._h, C.byref(desc), x, w, bias, residual, y, u, C.c_size_t(u_bytes)))
 
     def add_conv2d_pair(self, desc, x, w, bias, residual, y, w2, bias2, y2):
         _check(lib().kxc_hip_plan_add_conv2d_pair(self._h, C.byref(desc), x, w, bias, residual, y, w2, bias2, y2))

@@ -134,10 +134,10 @@ std::string Conv2DDispatch(const HIPDispatchContext& c, kxc_hip_plan* plan) {
     if (c.winograd_allowed && c.alloc_persistent && c.input_constant.size() > 1 && c.input_constant[1] &&
         kxc_hip_conv2d_winograd_preferred(&d)) {
         size_t u_bytes = 0;
-        Check(kxc_hip_conv2d_winograd_weight_bytes(&d, &u_bytes), "nn_conv2d dispatch");
+        Check(kxc_hip_conv2d_winograd_node_bytes(&d, &u_bytes), "nn_conv2d dispatch");
         const HIPBuffer u = c.alloc_persistent(static_cast<int64_t>(u_bytes));
-        Check(kxc_hip_plan_add_conv2d_winograd(plan, &d, B(c.inputs[0]), B(c.inputs[1]), has_bias ? B(c.inputs[2]) : none,
-                                               c.has_residual ? B(c.residual) : none, B(c.output), B(u)),
+        Check(kxc_hip_plan_add_conv2d_winograd_sized(plan, &d, B(c.inputs[0]), B(c.inputs[1]), has_bias ? B(c.inputs[2]) : none,
+                                                     c.has_residual ? B(c.residual) : none, B(c.output), B(u), u_bytes),
               "nn_conv2d dispatch");
         return std::string("kxc_conv2d_nchw_f32.") + kxc_hip_conv2d_winograd_variant(&d) + (has_bias ? "+bias" : "") +
                (c.has_residual ? "+add" : "") + (c.fused_relu ? "+relu" : "");

@@ -235,7 +235,8 @@ int32_t kxc_hip_conv2d_hpool_preferred(const kxc_hip_conv2d_desc* desc);
 /* nn_conv2d with a 3x3 filter, stride 1, dilation 1 and c % 4 == 0 as Winograd F(2x2, 3x3) on the matrix cores:
  * same operator and epilogue as kxc_hip_conv2d_nchw_f32 (convolution.cc:38-75, nn.h:107-158) with 2.25x fewer
  * multiplies; the sums are formed in a different order, results agree within the operator's fp32 tolerance.
- * The filter is passed in transformed form: `u` holds weight_bytes bytes written by ..._transform_weights from
+ * The filter is passed in transformed form: `u` holds weight_bytes bytes written by ..._transform_weights (two forms, so
+ * that a filter transformed once serves every batch and extent: 160 bytes per pair of channels) from
  * the OIHW tensor (the reference keeps weights as module constants, CompiledModule::GetConstants,
  * include/compiler.h:83, so a caller transforms them once per module).
  *   ..._supported: 1 when the shape qualifies, else 0 (no error is recorded). */
@@ -435,6 +436,14 @@ int32_t kxc_hip_plan_add_conv2d(kxc_hip_plan* plan, const kxc_hip_conv2d_desc* d
 int32_t kxc_hip_plan_add_conv2d_winograd(kxc_hip_plan* plan, const kxc_hip_conv2d_desc* desc, kxc_hip_buf x,
                                          kxc_hip_buf w, kxc_hip_buf bias, kxc_hip_buf residual, kxc_hip_buf y,
                                          kxc_hip_buf u);
+/* The same with the size of `u` given: a node reads one form of the filter at most, chosen when the plan is finalized
+ * among those that fit u_bytes (none: the node runs on `w` itself).  kxc_hip_conv2d_winograd_node_bytes says what the
+ * form costs that a node of this shape would take under the calling thread's kxc_hip_set_select_lanes; it may be 0
+ * (`u` is then any workspace offset).  Nodes of a plan may share `u` when they share `w` (the shares of a batch). */
+int32_t kxc_hip_plan_add_conv2d_winograd_sized(kxc_hip_plan* plan, const kxc_hip_conv2d_desc* desc, kxc_hip_buf x,
+                                               kxc_hip_buf w, kxc_hip_buf bias, kxc_hip_buf residual, kxc_hip_buf y,
+                                               kxc_hip_buf u, size_t u_bytes);
+int32_t kxc_hip_conv2d_winograd_node_bytes(const kxc_hip_conv2d_desc* desc, size_t* out_bytes);
 /* Both convolutions of kxc_hip_conv2d_pair_nchw_f32 as one node. */
 int32_t kxc_hip_plan_add_conv2d_pair(kxc_hip_plan* plan, const kxc_hip_conv2d_desc* desc, kxc_hip_buf x,
                                      kxc_hip_buf w, kxc_hip_buf bias, kxc_hip_buf residual, kxc_hip_buf y,

@@ -1574,6 +1574,71 @@ def test_plan_node_variant_names_the_launched_kernel(pkg, desc):
     plan.close()
 
 
+def test_plan_winograd_filter_buffers_hold_what_the_node_reads(pkg):
+    """Two large 3x3 layers in a row, their filter buffers side by side with the activations behind: whatever room the buffers
+    have -- both forms, the form that the node takes, the fp32 form, nothing --, and in a plan text written before the
+    buffer's size was part of it (room for the fp32 form), no node writes past its own.  Float64; 9 c + 16 roundings of at
+    most 2^-23 of a sum per layer, of independent signs."""
+    n, c, h = 16, 64, 56
+    rng = np.random.default_rng(91)
+    x, w1, w2 = (rng.standard_normal(s).astype(np.float32) for s in ((n, c, h, h), (c, c, 3, 3), (c, c, 3, 3)))
+    w1 /= np.float32(24); w2 /= np.float32(24)
+    t = lambda a: torch.from_numpy(a).double()
+    want = torch.nn.functional.conv2d(torch.nn.functional.conv2d(t(x), t(w1), None, 1, 1), t(w2), None, 1, 1).numpy()
+    d = pkg.ConvDesc(n, c, h, h, c, 3, 3, 1, 1, 1, 1, 1, 1, 0)
+    both, three, fp32 = pkg.conv2d_winograd_weight_bytes(x.shape, w1.shape), c * c * 96, c * c * 64
+    assert both == three + fp32 and pkg.conv2d_winograd_node_bytes(d) == three
+    args = [dev(x), dev(w1), dev(w2), torch.empty(want.shape, device="cuda")]
+
+    def check(plan, kernel):
+        assert all(kernel in plan.node_symbol(i) for i in range(2)), plan.node_symbol(0)
+        for _ in range(2):
+            args[3].zero_()
+            plan.run(args); torch.cuda.synchronize()
+            assert np.linalg.norm(host(args[3]) - want) <= (2 * (9 * c + 16)) ** 0.5 * 2.0 ** -23 * np.linalg.norm(want)
+
+    for room, kernel, version in ((None, "winograd_f2k3_bf16x3", 3), (both, "winograd_f2k3_bf16x3", 3), (three, "winograd_f2k3_bf16x3", 4),
+                                  (fp32, "winograd_f2k3_o", 4), (0, "mfma_k3x3", 4)):
+        step = both if room is None else room
+        plan = pkg.Plan(4)
+        plan.add_conv2d_winograd(d, pkg.Buf.arg(0), pkg.Buf.arg(1), pkg.Buf.none(), pkg.Buf.none(), pkg.Buf.ws(2 * step), pkg.Buf.ws(0), room)
+        plan.add_conv2d_winograd(d, pkg.Buf.ws(2 * step), pkg.Buf.arg(2), pkg.Buf.none(), pkg.Buf.none(), pkg.Buf.arg(3), pkg.Buf.ws(step), room)
+        plan.finalize(2 * step + x.nbytes)
+        check(plan, kernel)
+        text = plan.serialize()
+        assert text.startswith("kxc_hip_plan %d " % version)
+        again = pkg.Plan.deserialize(text, 0)
+        assert again.serialize() == text
+        check(again, kernel)
+        again.close()
+        if room == fp32:
+            old = []
+            for line in text.splitlines():
+                f = line.split()
+                if f[0] == "node":
+                    assert f[56] == str(fp32)
+                    f[56] = "0"
+                else:
+                    f[1] = "3"
+                old.append(" ".join(f))
+            old = pkg.Plan.deserialize("\n".join(old) + "\n", 0)
+            check(old, kernel)
+            old.close()
+        plan.close()
+    # a node whose share of the batch has the fp32 form only takes it along with the one it shares the buffer with
+    plan = pkg.Plan(4)
+    plan.add_conv2d_winograd(d, pkg.Buf.arg(0), pkg.Buf.arg(1), pkg.Buf.none(), pkg.Buf.none(), pkg.Buf.arg(3), pkg.Buf.ws(0), both)
+    plan.add_conv2d_winograd(pkg.ConvDesc(8, c, h, h, c, 3, 3, 1, 1, 1, 1, 1, 1, 0), pkg.Buf.arg(0), pkg.Buf.arg(1), pkg.Buf.none(), pkg.Buf.none(), pkg.Buf.arg(2), pkg.Buf.ws(0), both)
+    plan.finalize(both)
+    assert all("winograd_f2k3_o" in plan.node_symbol(i) for i in range(2))
+    y2 = torch.empty((8, c, h, h), device="cuda")
+    plan.run([args[0], args[1], y2, args[3]]); torch.cuda.synchronize()
+    one = torch.nn.functional.conv2d(t(x), t(w1), None, 1, 1).numpy()
+    for got, ref in ((args[3], one), (y2, one[:8])):
+        assert np.linalg.norm(host(got) - ref) <= (9 * c + 16) ** 0.5 * 2.0 ** -23 * np.linalg.norm(ref)
+    plan.close()
+
+
 def test_plan_hip_graph_replay(pkg):
     """A launch plan replayed as a captured HIP graph gives the eager result on every replay, with eager work and
     synchronisations in between, and re-captures when an argument pointer changes.  Batch 1 exercises the
