@@ -2,8 +2,9 @@
 //
 //   y[m,n] = alpha * sum_k a[m,k] * b[n,k]  (+ beta * c[n])          (transB = 1, the ResNet FC layer; transB = 0: b[k,n])
 //
-// Up to four rows go to gemv_nt_kernel, everything else to gemm_bf16x3_kernel (three-part fp32 operands, bf16x3.h); tiny
-// products that no vector load fits keep a one-thread-per-output kernel in the CPU loop's exact order.
+// Up to four rows go to gemv_nt_kernel, everything else to gemm_nt_staged_kernel / gemm_bf16x3_kernel (three-part fp32
+// operands, bf16x3.h), k from 2^24 on to gemm_nt_long_kernel; tiny products that no vector load fits keep a
+// one-thread-per-output kernel in the CPU loop's exact order.
 #include "bf16x3.h"
 #include "common.h"
 
@@ -277,6 +278,39 @@ __global__ void __launch_bounds__(64 * KS) __attribute__((amdgpu_waves_per_eu(2)
     finish_tile<RO, RP, KS, true>(acc, lds, wave, lane, a, b, c, y, M, N, K, m0, n0, alpha, beta, c_len, scale_a, scale_c);
 }
 
+// k from 2^24 on: row offsets of a tile no longer fit the 31 bits of a buffer offset, so the lanes walk their rows with 64-bit
+// addresses, on the fp32 instructions: a workgroup of four waves owns 32 x 32 outputs, the waves split k four ways and
+// the two half-waves of a wave two ways.  Bound by the latency of its loads (5 x 2 x 2^25:
+// 235 ms; one thread per output, which this range fell to, 2.5 s and a single running sum).
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) gemm_nt_long_kernel(
+    const float* __restrict__ a, const float* __restrict__ b, const float* __restrict__ c, float* __restrict__ y, int32_t M, int32_t N, int32_t K,
+    float alpha, float beta, int64_t c_len, int scale_a, int scale_c) {
+    __shared__ float part[4][32 * 33];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, half = lane >> 5, r = lane & 31;
+    const int m0 = blockIdx.y * 32, n0 = blockIdx.x * 32;
+    const int run = K / 8;                     // k values of a half-wave (a multiple of 4)
+    // (rows past the last one are computed and never stored)
+    const float* const ap = a + static_cast<int64_t>(min(m0 + r, M - 1)) * K + static_cast<int64_t>(wave * 2 + half) * run;
+    const float* const bp = b + static_cast<int64_t>(min(n0 + r, N - 1)) * K + static_cast<int64_t>(wave * 2 + half) * run;
+    f32x16 acc = {0};
+#pragma unroll 4
+    for (int k = 0; k < run; k += 4) {
+        const f32x4 va = *reinterpret_cast<const f32x4*>(ap + k), vb = *reinterpret_cast<const f32x4*>(bp + k);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(va[e], vb[e], acc, 0, 0, 0);
+    }
+#pragma unroll
+    for (int g = 0; g < 16; ++g) part[wave][(8 * (g / 4) + 4 * half + g % 4) * 33 + r] = acc[g];
+    __syncthreads();
+    for (int e = threadIdx.x; e < 1024; e += 256) {
+        const int i = e >> 5, j = e & 31, m = m0 + i, n = n0 + j;
+        float s = part[0][i * 33 + j];
+#pragma unroll
+        for (int w = 1; w < 4; ++w) s = __fadd_rn(s, part[w][i * 33 + j]);
+        if (m < M && n < N) y[static_cast<int64_t>(m) * N + n] = epilogue(s, alpha, beta, c, n, c_len, scale_a != 0, scale_c != 0);
+    }
+}
+
 // A handful of rows (batch 1-4 of a classifier layer): the matrix-core tile above would be 32 rows of which at
 // most 4 are real, and its k loop is a chain of dependent load latencies.  Here a wave owns four output columns for
 // every row; its lanes split k (a lane takes 4 consecutive floats of every 256), all loads of a 256-chunk are in
@@ -522,6 +556,12 @@ int32_t kxc_hip_gemm_f32(const float* a, const float* b, const float* c, float* 
             a, b, c, y, static_cast<int32_t>(m), static_cast<int32_t>(n), static_cast<int32_t>(k), static_cast<int32_t>(m_tiles),
             static_cast<int32_t>(tiles), per_xcd, alpha, beta, c_len, scale_a, scale_c);
         return CheckLaunch("gemm_bf16x3");
+    }
+    if (transB && k >= (1 << 24) && (k % 32) == 0 && aligned && m < (1 << 20) && n < (1 << 20) && k < (1 << 30)) {
+        const dim3 grid(static_cast<unsigned>(CeilDiv(n, 32)), static_cast<unsigned>(CeilDiv(m, 32)));
+        gemm_nt_long_kernel<<<NoteGrid(grid), NoteBlock(256), NoteLds(0), s>>>(a, b, c, y, static_cast<int32_t>(m), static_cast<int32_t>(n),
+                                                                               static_cast<int32_t>(k), alpha, beta, c_len, scale_a, scale_c);
+        return CheckLaunch("gemm_nt_long");
     }
     int64_t g = CeilDiv(m * n, 256);
     if (g > 256 * 32) g = 256 * 32;

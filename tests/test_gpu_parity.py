@@ -1239,6 +1239,19 @@ def test_gemm_tile_edges(pkg, m, n, k, trans_b):
     assert_bit_exact(again[1:m - 1], got[1:m - 1], "other rows")
 
 
+@pytest.mark.parametrize("m, n, k", [(33, 2, (1 << 24) + 64), (5, 33, (1 << 24) + 32)])
+def test_gemm_long_reductions(pkg, m, n, k):
+    """k from 2^24 on (rows of a tile beyond 31-bit offsets): powers of two, whose sums are exact in eight partial sums and
+    lose their last bits in one running sum.  Two tiles of rows and of columns, both with a partial one."""
+    a, b = torch.ones((m, k), device="cuda"), torch.ones((n, k), device="cuda")
+    fa, fb = 2.0 ** (np.arange(m) % 5), 2.0 ** (np.arange(n) % 3)
+    a *= dev(fa.astype(np.float32))[:, None]; b *= dev(fb.astype(np.float32))[:, None]
+    c = np.arange(n).astype(np.float32) * np.float32(k)
+    want = k * fa[:, None] * fb[None, :]
+    assert np.array_equal(host(pkg.gemm(a, b)).astype(np.float64), want)
+    assert np.array_equal(host(pkg.gemm(a, b, dev(c), 0.5, 2.0)).astype(np.float64), (0.5 * want + 2.0 * c).astype(np.float32))
+
+
 def test_bias_add_and_flatten(pkg, orc, synth):
     x = synth.uniform((3, 6, 5, 7), 2040); b = synth.uniform((6,), 2041)
     assert_bit_exact(host(pkg.bias_add(dev(x), dev(b))), orc.bias_add(x, b), "bias_add")
