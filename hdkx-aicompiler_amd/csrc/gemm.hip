@@ -70,7 +70,8 @@ __device__ __forceinline__ void finish_tile(const f32x16 (&acc)[RO][RP], char* l
             const int m = m0 + (q / 4 / RP) * 32 + 8 * (q % 4) + 4 * half + e;
             if (m >= M) continue;
             float x = v[e];
-            if (__builtin_expect(x != x, 0)) {                // a non-finite operand: the fp32 loop spreads it
+            // a non-finite operand, or a sum next to the largest float (h h' alone may round past it): the fp32 loop decides
+            if (__builtin_expect(!(__builtin_fabsf(x) <= 3.402823466e38f), 0)) {
                 x = 0.0f;
                 for (int k = 0; k < K; ++k)
                     x = fmaf(a[static_cast<int64_t>(m) * K + k], TB ? b[static_cast<int64_t>(n) * K + k] : b[static_cast<int64_t>(k) * N + n], x);
@@ -293,7 +294,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) g
     const float* const ap = a + static_cast<int64_t>(min(m0 + r, M - 1)) * K + static_cast<int64_t>(wave * 2 + half) * run;
     const float* const bp = b + static_cast<int64_t>(min(n0 + r, N - 1)) * K + static_cast<int64_t>(wave * 2 + half) * run;
     f32x16 acc = {0};
-#pragma unroll 4
     for (int k = 0; k < run; k += 4) {
         const f32x4 va = *reinterpret_cast<const f32x4*>(ap + k), vb = *reinterpret_cast<const f32x4*>(bp + k);
 #pragma unroll

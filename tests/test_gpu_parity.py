@@ -1252,6 +1252,23 @@ def test_gemm_long_reductions(pkg, m, n, k):
     assert np.array_equal(host(pkg.gemm(a, b, dev(c), 0.5, 2.0)).astype(np.float64), (0.5 * want + 2.0 * c).astype(np.float32))
 
 
+@pytest.mark.parametrize("trans_b", [1, 0])
+def test_gemm_sums_next_to_the_largest_float(pkg, trans_b):
+    """Products whose leading bf16 parts round up past the largest float although the product does not: finite results stay
+    finite (two roundings of the largest term, two of the sum), true overflows are infinite, opposite ones NaN or finite as
+    in the fp32 loop."""
+    m, n, k = 40, 70, 48
+    a, b = np.zeros((m, k), np.float32), np.zeros((n, k), np.float32)
+    a[:, 3] = 2 - 2.0 ** -10; b[:, 3] = np.float32(2.0 ** 127) * np.float32(1 - 2.0 ** -10)        # 0.9985 of the largest float
+    a[1] = -a[1]
+    a[2, 20], b[:, 20] = 2.0 ** 100, np.float32(2.0 ** 28)      # with the term above, beyond it
+    want = a.astype(np.float64) @ b.T.astype(np.float64)
+    got = host(pkg.gemm(dev(a), dev(b if trans_b else np.ascontiguousarray(b.T)), None, 1.0, 1.0, trans_b))
+    over = np.abs(want) > np.finfo(np.float32).max
+    assert over[2].all() and not over[0].any() and (got[over] == np.sign(want[over]) * np.inf).all()
+    assert (np.abs(got[~over] - want[~over]) <= 4 * 2.0 ** -24 * np.abs(want[~over])).all()
+
+
 def test_bias_add_and_flatten(pkg, orc, synth):
     x = synth.uniform((3, 6, 5, 7), 2040); b = synth.uniform((6,), 2041)
     assert_bit_exact(host(pkg.bias_add(dev(x), dev(b))), orc.bias_add(x, b), "bias_add")
