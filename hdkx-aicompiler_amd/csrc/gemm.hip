@@ -5,6 +5,8 @@
 // Up to four rows go to gemv_nt_kernel, everything else to gemm_nt_staged_kernel / gemm_bf16x3_kernel (three-part fp32
 // operands, bf16x3.h), k from 2^24 on to gemm_nt_long_kernel; tiny products that no vector load fits keep a
 // one-thread-per-output kernel in the CPU loop's exact order.
+#include <cstdlib>
+
 #include "bf16x3.h"
 #include "common.h"
 
@@ -530,9 +532,12 @@ int32_t kxc_hip_gemm_f32(const float* a, const float* b, const float* c, float* 
 #undef KXC_GEMV
         return CheckLaunch("gemv_nt");
     }
-    // (row offsets of a tile and, for b = [k][n], all of b are addressed with 31 bits)
+    // (row offsets of a tile and, for b = [k][n], all of b are addressed with 31 bits; KXC_HIP_GEMM_BF16X3=0 keeps the fp32
+    // instructions and the one-thread-per-output kernel, for operands below 2^-109: bf16x3.h)
     const bool small = m * n * k < (1 << 15);
-    if (k > 0 && (!small || (transB && k % 32 == 0)) && m < (1 << 20) && n < (1 << 20) && k < (1 << 24) && (transB || n * (k + 16) < (1 << 29))) {
+    const char* const bx = std::getenv("KXC_HIP_GEMM_BF16X3");
+    const bool three_part = !(bx && bx[0] == '0');
+    if (three_part && k > 0 && (!small || (transB && k % 32 == 0)) && m < (1 << 20) && n < (1 << 20) && k < (1 << 24) && (transB || n * (k + 16) < (1 << 29))) {
         struct Tile { int ro, rp, ks; void (*kernel[3])(const float*, const float*, const float*, float*, int32_t, int32_t, int32_t, int32_t, int32_t, int32_t,
                                                         float, float, int64_t, int, int); };
 #define KXC_GEMM(RO, RP, KS, D) {RO, RP, KS, {gemm_bf16x3_kernel<RO, RP, KS, D, false>, gemm_bf16x3_kernel<RO, RP, KS, D, true>, gemm_nt_staged_kernel<RO, RP, KS>}}
@@ -557,7 +562,7 @@ int32_t kxc_hip_gemm_f32(const float* a, const float* b, const float* c, float* 
             static_cast<int32_t>(tiles), per_xcd, alpha, beta, c_len, scale_a, scale_c);
         return CheckLaunch("gemm_bf16x3");
     }
-    if (transB && k >= (1 << 24) && (k % 32) == 0 && aligned && m < (1 << 20) && n < (1 << 20) && k < (1 << 30)) {
+    if (transB && k >= (three_part ? 1 << 24 : 1) && (k % 32) == 0 && aligned && m < (1 << 20) && n < (1 << 20) && k < (1 << 30)) {
         const dim3 grid(static_cast<unsigned>(CeilDiv(n, 32)), static_cast<unsigned>(CeilDiv(m, 32)));
         gemm_nt_long_kernel<<<NoteGrid(grid), NoteBlock(256), NoteLds(0), s>>>(a, b, c, y, static_cast<int32_t>(m), static_cast<int32_t>(n),
                                                                                static_cast<int32_t>(k), alpha, beta, c_len, scale_a, scale_c);

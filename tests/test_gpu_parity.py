@@ -1269,6 +1269,55 @@ def test_gemm_sums_next_to_the_largest_float(pkg, trans_b):
     assert (np.abs(got[~over] - want[~over]) <= 4 * 2.0 ** -24 * np.abs(want[~over])).all()
 
 
+@pytest.mark.parametrize("exponent", [-100, -109, -116, -126, -140])
+def test_small_operands_of_the_three_part_kernels(pkg, exponent):
+    """Operands below 2^-109 keep what bf16's smallest step leaves of their low parts: an operand is off by at most 2^-134 (half of
+    2^-133), on top of fp32 rounding.  Products of both layouts, the single convolution (whose transforms add four operands)
+    and a prepared filter; the other operand has ordinary size."""
+    rng = np.random.default_rng(-exponent)
+    scale = 2.0 ** exponent
+    small = lambda *shape: (rng.standard_normal(shape) * scale).astype(np.float32)
+    lost = 2.0 ** -134
+    m, n, k = 64, 96, 260
+    a, b = small(m, k), rng.standard_normal((n, k)).astype(np.float32)
+    want, size = a.astype(np.float64) @ b.T.astype(np.float64), np.abs(a).astype(np.float64) @ np.abs(b.T).astype(np.float64)
+    bound = k * 2.0 ** -24 * size + lost * np.abs(b).astype(np.float64).sum(axis=1) + 2.0 ** -149 * k
+    for trans_b in (1, 0):
+        got = host(pkg.gemm(dev(a), dev(b if trans_b else np.ascontiguousarray(b.T)), None, 1.0, 1.0, trans_b))
+        assert (np.abs(got - want) <= bound).all(), trans_b
+    nb, c, h, o = 16, 64, 56, 64
+    x, w = small(nb, c, h, h), (rng.standard_normal((o, c, 3, 3)) / 24).astype(np.float32)
+    xd, wd = dev(x), dev(w)
+    t = lambda v: torch.from_numpy(v).double()
+    conv = lambda x, w: torch.nn.functional.conv2d(x, w, None, 1, 1).numpy()
+    want = conv(t(x[:1]), t(w))
+    # (an output adds nine of the sixteen products of transformed operands, |U| <= sum |w|, each V off by `lost`; ordinary
+    # rounding of the transforms as in the tests above)
+    off = 16 * lost * np.abs(w).astype(np.float64).sum(axis=(1, 2, 3))[None, :, None, None]
+    for got in (pkg.conv2d(xd, wd, None, None, 1, 1), pkg.conv2d_winograd(xd, pkg.conv2d_winograd_transform_weights(x.shape, wd), w.shape)):
+        err = np.abs(host(got[:1]) - want)
+        assert (err <= 64 * 2.0 ** -23 * scale * np.sqrt(9 * c) + off).all()
+        assert np.linalg.norm(err / scale) <= (9 * c + 16) ** 0.5 * 2.0 ** -23 * np.linalg.norm(want / scale) + np.linalg.norm(np.broadcast_to(off, err.shape) / scale)
+
+
+def test_fp32_instruction_switches_keep_small_operands(pkg, monkeypatch):
+    """KXC_HIP_GEMM_BF16X3=0 and KXC_HIP_WINOGRAD_BF16X3=0: fp32 arithmetic down to the smallest normal number, k rounded products in
+    any order within k * 2^-24 * sum |a b| (and half of 2^-149 for each that comes out subnormal)."""
+    monkeypatch.setenv("KXC_HIP_GEMM_BF16X3", "0"); monkeypatch.setenv("KXC_HIP_WINOGRAD_BF16X3", "0")
+    rng = np.random.default_rng(8)
+    small = lambda *shape: (rng.standard_normal(shape) * 2.0 ** -120).astype(np.float32)
+    for m, n, k, trans_b in ((64, 96, 256, 1), (33, 70, 250, 1), (33, 70, 256, 0)):
+        a, b = small(m, k), rng.standard_normal((n, k)).astype(np.float32)
+        want, size = a.astype(np.float64) @ b.T.astype(np.float64), np.abs(a).astype(np.float64) @ np.abs(b.T).astype(np.float64)
+        got = host(pkg.gemm(dev(a), dev(b if trans_b else np.ascontiguousarray(b.T)), None, 1.0, 1.0, trans_b))
+        assert (np.abs(got - want) <= k * (2.0 ** -24 * size + 2.0 ** -149)).all()
+    x, w = small(16, 64, 56, 56), (rng.standard_normal((64, 64, 3, 3)) / 24).astype(np.float32)
+    assert "bf16x3" not in pkg.conv2d_variant(x.shape, w.shape, 1, 1) + pkg.conv2d_winograd_variant(x.shape, w.shape)
+    want = torch.nn.functional.conv2d(torch.from_numpy(x[:1]).double(), torch.from_numpy(w).double(), None, 1, 1).numpy()
+    for got in (pkg.conv2d(dev(x), dev(w), None, None, 1, 1), pkg.conv2d_winograd(dev(x), pkg.conv2d_winograd_transform_weights(x.shape, dev(w)), w.shape)):
+        assert np.linalg.norm((host(got[:1]) - want) * 2.0 ** 120) <= (9 * 64 + 16) ** 0.5 * 2.0 ** -23 * np.linalg.norm(want * 2.0 ** 120)
+
+
 def test_bias_add_and_flatten(pkg, orc, synth):
     x = synth.uniform((3, 6, 5, 7), 2040); b = synth.uniform((6,), 2041)
     assert_bit_exact(host(pkg.bias_add(dev(x), dev(b))), orc.bias_add(x, b), "bias_add")
