@@ -624,7 +624,7 @@ bool ThreePartFits(const kxc_hip_conv2d_desc* d) {
     const int64_t oh = static_cast<int64_t>(d->h) + 2 * d->pad_h - 2, ow = static_cast<int64_t>(d->w) + 2 * d->pad_w - 2;
     const int64_t TW = CeilDiv(ow, 2), TH = CeilDiv(oh, 2), Hq = 2 * TH + 2, Wq = 2 * TW + 2;
     if (wino_bx::WeightBytes(d->o, d->c) >= (1ull << 31) || (static_cast<int64_t>(d->n) + 1) * Hq * Wq >= (1LL << 30)) return false;
-    return wino_bx::MaxPatchRows(static_cast<int64_t>(d->n) * TH * TW, TH * TW, TW, Hq) * Wq <= wino_bx::kPlanes[1];
+    return wino_bx::MaxPatchRows(static_cast<int64_t>(d->n) * TH * TW, TH * TW, TW) * Wq <= wino_bx::kPlanes[1];
 }
 
 int64_t Tiles(const kxc_hip_conv2d_desc* d) {
@@ -735,8 +735,8 @@ void ThreePartResolve(const kxc_hip_conv2d_desc* d, WinoLaunch* L, bool may_spli
     const WinoArgs& a = L->a;
     b.N = a.N; b.C = a.C; b.H = a.H; b.W = a.W; b.O = a.O; b.OH = a.OH; b.OW = a.OW; b.ph = a.ph; b.pw = a.pw;
     b.TW = a.TW; b.TI = a.TI; b.NT = a.NT; b.HW = a.HW; b.OHW = a.OHW;
-    b.Hq = 2 * (a.TI / a.TW) + 2; 
-    const int64_t rows = wino_bx::MaxPatchRows(b.NT, b.TI, b.TW, b.Hq);
+    b.Hq = 2 * (a.TI / a.TW) + 2;
+    const int64_t rows = wino_bx::MaxPatchRows(b.NT, b.TI, b.TW);
     b.pitch = wino_bx::RowPitch(b.TW, rows, wino_bx::kPlanes[1]);
     L->bx_plane = rows * 2 * b.pitch <= wino_bx::kPlanes[0] ? 0 : 1;
     b.ksteps = static_cast<int32_t>(CeilDiv(a.C, wino_bx::kStep));

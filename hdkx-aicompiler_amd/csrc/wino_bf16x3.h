@@ -23,6 +23,8 @@
 // float64 (2-norm): 1.0e-7 to 1.4e-7, the fp32-instruction kernel 1.3e-7 to 1.7e-7.
 #pragma once
 
+#include <algorithm>
+
 #include "bf16x3.h"
 
 namespace kxc_hip {
@@ -56,17 +58,25 @@ inline int32_t RowPitch(int64_t TW, int64_t rows, int64_t limit) {
     return best;
 }
 
-// Rows of the patch that a workgroup's tiles touch at most, in the row space Q = image * Hq + padded row.
-inline int64_t MaxPatchRows(int64_t NT, int64_t TI, int64_t TW, int64_t Hq) {
-    int64_t best = 0;
-    for (int64_t t0 = 0; t0 < NT; t0 += kTiles) {
-        const int64_t t1 = (t0 + kTiles < NT ? t0 + kTiles : NT) - 1;
-        const int64_t q0 = t0 / TI * Hq + t0 % TI / TW * 2, q1 = t1 / TI * Hq + t1 % TI / TW * 2 + 3;
-        if (q1 - q0 + 1 > best) best = q1 - q0 + 1;
-        // (the pattern repeats with the images: a few groups past the first image's end cover every alignment)
-        if (t0 > 64 * TI + 64 * kTiles) break;
+// Rows of the patch that a workgroup's tiles touch at most, in the row space Q = image * (2 TH + 2) + padded row of TH * TW = TI
+// tiles per image: tiles t0 .. t1 take two rows per tile row and image border between them and four more.  Where a group
+// starts within an image repeats after TI / gcd(TI, 64) groups, and a partial last group takes no more than a full one
+// there (an eager call pays for this walk: 49 groups at 56 x 56 and 112 x 112, any batch).
+inline int64_t MaxPatchRows(int64_t NT, int64_t TI, int64_t TW) {
+    int64_t rem = TI, gcd = kTiles;
+    while (rem != 0) { const int64_t r = gcd % rem; gcd = rem; rem = r; }
+    const int64_t groups = std::min(CeilDiv(NT, kTiles), TI / gcd);
+    const int64_t step_image = kTiles % TI, step_row = kTiles % TW;
+    int64_t best = 0, in_image = 0, in_row = 0;
+    for (int64_t g = 0; g < groups; ++g) {
+        const int64_t last = std::min<int64_t>(kTiles, NT - g * kTiles) - 1;
+        best = std::max(best, (in_row + last) / TW + (in_image + last) / TI);
+        in_image += step_image;
+        if (in_image >= TI) in_image -= TI;
+        in_row += step_row;
+        if (in_row >= TW) in_row -= TW;
     }
-    return best;
+    return 2 * best + 4;
 }
 
 struct Args {

@@ -106,3 +106,22 @@ def test_resnet18_plan_shape(pkg):
     so build it but skip finalize by checking the symbols through a dry builder)."""
     r = __import__("importlib").import_module("hdkx-aicompiler_amd.resnet18")
     assert r.flops_per_image() == 3628146688        # 2 x 1 814 073 344 multiply-accumulates per image (convolutions + FC)
+
+
+def test_large_convolution_rule_costs_the_host_little(pkg):
+    """Whether a large 3x3 call takes the Winograd kernel is decided in every call, and the patch geometry is part of it: it must
+    not grow with the batch (52 us at 112 x 112, batch 64, while it walked every group of tiles)."""
+    import time
+    best = {}
+    for batch in (4, 64):
+        d = pkg.conv_desc((batch, 64, 112, 112), (64, 64, 3, 3), 1, 1)
+        variant, ref = pkg.lib().kxc_hip_conv2d_variant, ctypes.byref(d)
+        assert variant(ref).startswith(b"winograd")
+        times = []
+        for _ in range(20):
+            t = time.perf_counter()
+            for _ in range(50):
+                variant(ref)
+            times.append((time.perf_counter() - t) / 50)
+        best[batch] = min(times)
+    assert best[64] < 10e-6 and best[64] < 3 * best[4], best
