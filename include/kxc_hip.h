@@ -165,7 +165,13 @@ typedef struct kxc_hip_conv2d_desc {
     int32_t dil_h, dil_w;
     uint32_t flags;
 } kxc_hip_conv2d_desc;
-/* Scratch.  A launch that splits its reduction over workgroups, and a large 3x3 stride-1 call that runs as Winograd and
+/* Numerics.  fp32 sums in an order of the kernel's own.  Large 3x3 stride-1 calls run as Winograd F(2x2, 3x3) (..._variant says
+ * "winograd_..."), which adds and subtracts inputs inside 4x4 patches: the four outputs of a patch carry rounding errors of
+ * about 2^-24 times its largest input, also those whose own 3x3 window does not hold it (a finite sentinel like 1e9 among
+ * values of 1 costs its neighbours their digits; Inf and NaN do not: such outputs are evaluated by the definition).
+ * KXC_HIP_CONV_WINOGRAD=0 in the environment keeps the kernels that add only what an output's window holds.
+ *
+ * Scratch.  A launch that splits its reduction over workgroups, and a large 3x3 stride-1 call that runs as Winograd and
  * transforms its filter first, keep intermediate values in a buffer that the library holds per (device, stream handle):
  * calls on one stream are safe from any thread.  While the stream is being captured, and on hipStreamPerThread, large 3x3
  * stride-1 calls, 5x5 filters and calls of fewer than 32 output channels or pixels take a kernel that needs no buffer (the
