@@ -176,7 +176,7 @@ def test_qconv_c16_direct_kernel(pkg, orc, monkeypatch, shape):
     """The kernel of small launches, at the edges of its tiles and of the rule that chooses its tile: the same bytes as the
     CPU operator, or where that would take long as the staged kernel."""
     n, c, h, w, o, k, s, tile = shape
-    rng = np.random.default_rng(hash(shape) % (2 ** 31))
+    rng = np.random.default_rng(hash(shape[:-1]) % (2 ** 31))      # (numbers only: the hash of a text differs from run to run)
     x = rng.integers(-128, 128, (n, c, h, w), dtype=np.int8)
     wq = rng.integers(-127, 128, (o, c, k, k), dtype=np.int8)
     bias = rng.integers(-20000, 20000, (o,), dtype=np.int32)

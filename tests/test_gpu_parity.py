@@ -860,6 +860,31 @@ def test_conv_operator_by_winograd(pkg, monkeypatch, n, c, h, w, o, p, forced):
     assert np.linalg.norm(got[far] - want[far]) <= 2 * (9 * c + 16) ** 0.5 * 2.0 ** -23 * np.linalg.norm(want[far].astype(np.float64)) + 1e-30
 
 
+@pytest.mark.parametrize("n, c, h, w, o, p, split", [
+    (1, 4, 3, 3, 1, 1, 1), (2, 20, 9, 12, 65, 1, 2), (3, 92, 13, 15, 64, 0, 3), (1, 72, 31, 64, 33, 2, 2), (5, 16, 7, 7, 130, 1, 1),
+    (12, 128, 28, 28, 128, 1, 0), (9, 256, 13, 13, 200, 1, 0), (2, 140, 17, 5, 96, 1, 9)])
+def test_conv_winograd_three_part_prepared_filter(pkg, monkeypatch, n, c, h, w, o, p, split):
+    """The three-part kernel on a filter transformed beforehand, as networks run it: partial groups of tiles and of output
+    channels, input channels that leave 4, 8 and 12 of a step of 16, its split over workgroups (forced, by its own rule
+    where 0) with the adding kernel, odd extents.  9 c + 16 roundings of at most 2^-23 of a sum, of independent signs."""
+    monkeypatch.setenv("KXC_HIP_WINOGRAD_VARIANT", "winograd_f2k3_bf16x3")
+    if split:
+        monkeypatch.setenv("KXC_HIP_WINOGRAD_GSPLIT", str(split))
+    rng = np.random.default_rng(n * c + h * w + o)
+    x = rng.standard_normal((n, c, h, w)).astype(np.float32)
+    wt = (rng.standard_normal((o, c, 3, 3)) / np.sqrt(9 * c)).astype(np.float32)
+    b, res = rng.standard_normal(o).astype(np.float32), rng.standard_normal((n, o, h + 2 * p - 2, w + 2 * p - 2)).astype(np.float32)
+    assert pkg.conv2d_winograd_variant(x.shape, wt.shape, 1, p) == "winograd_f2k3_bf16x3"
+    u = pkg.conv2d_winograd_transform_weights(x.shape, dev(wt), p)
+    conv = torch.nn.functional.conv2d(torch.from_numpy(x).double(), torch.from_numpy(wt).double(), None, 1, p).numpy()
+    for bias, residual, relu in ((b, res, True), (None, None, False), (b, None, True)):
+        want = conv + (0 if bias is None else bias[:, None, None]) + (0 if residual is None else residual)
+        want = np.maximum(want, 0) if relu else want
+        out = torch.full(want.shape, float("nan"), device="cuda")
+        got = pkg.conv2d_winograd(dev(x), u, wt.shape, None if bias is None else dev(bias), None if residual is None else dev(residual), p, relu, out=out)
+        assert np.linalg.norm(host(got) - want) <= (9 * c + 16) ** 0.5 * 2.0 ** -23 * np.linalg.norm(want), (bias is None, residual is None)
+
+
 def test_conv_operator_by_winograd_under_capture(pkg, monkeypatch):
     """A large 3x3 call transforms its filter into the buffer of its stream handle, so a graph of it must not hold that buffer:
     captured after an eager call has grown it, on hipStreamPerThread and in the entry point that allocates nothing the call runs
