@@ -269,14 +269,12 @@ def main():
         lu = pkg.conv2d_winograd_transform_weights(lx.shape, lw, 1)
         conv_ms = _event_time_ms(torch, lambda: pkg.conv2d_winograd(lx, lu, lw.shape, lb, None, 1, True, out=ly), 30, 5)
         conv_tflops = conv_flop / (conv_ms * 1e-3) / 1e12
-        # (the three-part kernel multiplies every pair of operands as six bf16 products, on the bf16 matrix cores)
         three_part = pkg.conv2d_winograd_variant(lx.shape, lw.shape).endswith("bf16x3")
-        executed = conv_flop * 16.0 / 36.0 * (6 if three_part else 1)
-        matrix_peak = PEAK_BF16_MFMA_TFLOPS if three_part else PEAK_FP32_MFMA_TFLOPS
+        executed, matrix_peak, product_peak = _winograd_matrix_work(pkg.conv2d_winograd_variant(lx.shape, lw.shape), conv_flop)
         roofline = {"bound": "mfma", "kernel": ("wino_bf16x3_kernel" if three_part else "wino_kernel") + " (layer1: [%d,64,56,56]x[64,64,3,3] s1 p1 +bias+relu, Winograd F(2x2,3x3))" % batch,
                     "variant": pkg.conv2d_winograd_variant(lx.shape, lw.shape),
-                    "achieved": round(conv_tflops, 3), "peak": PEAK_FP32_MFMA_TFLOPS, "unit": "TFLOP/s",
-                    "frac": round(conv_tflops / PEAK_FP32_MFMA_TFLOPS, 4), "avg_launch_ms": round(conv_ms, 4),
+                    "achieved": round(conv_tflops, 3), "peak": round(product_peak, 1), "unit": "TFLOP/s",
+                    "frac": round(conv_tflops / product_peak, 4), "avg_launch_ms": round(conv_ms, 4),
                     "flop_per_launch": conv_flop,
                     "matrix_core_flop_per_launch": executed,
                     "matrix_core_tflops": round(executed / (conv_ms * 1e-3) / 1e12, 3),
@@ -285,9 +283,10 @@ def main():
                     "traffic_unit": "bytes per launch (FETCH_SIZE + WRITE_SIZE, calibrated on a copy; from profiles/)",
                     "algorithmic_bytes_per_launch": algorithmic_bytes, "same_layer_implicit_gemm": gemm_row,
                     "accounting": "achieved and frac divide the OPERATOR's FLOP (2*N*O*OH*OW*C*9, every output computed) by the measured "
-                                  "time, against the fp32 matrix peak; Winograd F(2x2,3x3) executes 16/36 of those multiplies, the three-part "
-                                  "kernel each as six bf16 products, so frac can reach or pass 1 while the matrix cores run at "
-                                  "matrix_core_frac of matrix_core_peak (the bf16 peak for the three-part kernel)"}
+                                  "time, against the rate at which the matrix cores that the kernel uses multiply fp32 operands (the fp32 "
+                                  "peak, or for the three-part kernel a sixth of the bf16 peak: six bf16 products each); Winograd "
+                                  "F(2x2,3x3) executes 16/36 of those multiplies, so the matrix cores run at matrix_core_frac of "
+                                  "matrix_core_peak, 16/36 of frac"}
         if shares > 1 and batch % shares == 0:
             # what the plan does with this layer: one launch per share of the batch, side by side on streams of
             # their own between a fork and a join on the timed stream (variants chosen for `shares` equal launches)
@@ -310,13 +309,14 @@ def main():
                         cur.wait_event(done[k])
                 pair_ms = _event_time_ms(torch, pair, 30, 5)
                 part_variant = pkg.conv2d_winograd_variant(lx[:part].shape, lw.shape)
+                part_work = _winograd_matrix_work(part_variant, conv_flop)
             finally:
                 pkg.set_select_lanes(prev)
             roofline["side_by_side"] = {
                 "what": "%d launches of [%d,64,56,56] on %d streams, fork to join: the layer as the timed plan runs it" % (shares, part, shares),
                 "variant": part_variant, "ms": round(pair_ms, 4), "achieved": round(conv_flop / (pair_ms * 1e-3) / 1e12, 3),
-                "frac": round(conv_flop / (pair_ms * 1e-3) / 1e12 / PEAK_FP32_MFMA_TFLOPS, 4),
-                "matrix_core_frac": round(executed / (pair_ms * 1e-3) / 1e12 / matrix_peak, 4)}
+                "frac": round(conv_flop / (pair_ms * 1e-3) / 1e12 / part_work[2], 4),
+                "matrix_core_frac": round(part_work[0] / (pair_ms * 1e-3) / 1e12 / part_work[1], 4)}
     else:
         roofline = {"bound": "mfma", "kernel": "conv_mfma_kernel<3,3> (layer1: [%d,64,56,56]x[64,64,3,3] s1 p1 +bias+relu)" % batch,
                     "variant": gemm_row["variant"], "achieved": gemm_row["achieved"], "peak": PEAK_FP32_MFMA_TFLOPS,
@@ -411,6 +411,13 @@ CONV_LAYERS = [  # name, C, H, O, k, s, p, count per network, residual
 ]
 
 
+def _winograd_matrix_work(variant, flop):
+    """(FLOP that the matrix cores execute for `flop` of the operator, the peak of the cores that do, the rate at which those
+    multiply fp32 operands): F(2x2, 3x3) does 16 of 36 multiplies, the three-part kernel each as six bf16 products."""
+    products, peak = (6, PEAK_BF16_MFMA_TFLOPS) if variant.endswith("bf16x3") else (1, PEAK_FP32_MFMA_TFLOPS)
+    return flop * 16.0 / 36.0 * products, peak, peak / products
+
+
 def bench_conv_layers(torch, pkg, synth, dev, batch):
     rows = []
     for i, (name, c, h, o, k, s, p, count, res) in enumerate(CONV_LAYERS):
@@ -429,10 +436,12 @@ def bench_conv_layers(torch, pkg, synth, dev, batch):
             # what the launch plan uses for this layer; tflops = direct-definition FLOP / time
             u = pkg.conv2d_winograd_transform_weights(x.shape, w, p)
             wms = _event_time_ms(torch, lambda: pkg.conv2d_winograd(x, u, w.shape, b, skip, p, True, out=y), 20, 3)
-            row["winograd"] = {"variant": pkg.conv2d_winograd_variant(x.shape, w.shape, s, p), "ms": round(wms, 4),
+            variant = pkg.conv2d_winograd_variant(x.shape, w.shape, s, p)
+            executed, matrix_peak, _ = _winograd_matrix_work(variant, flop)
+            row["winograd"] = {"variant": variant, "ms": round(wms, 4),
                                "tflops": round(flop / (wms * 1e-3) / 1e12, 2),
                                "frac_fp32_mfma_peak": round(flop / (wms * 1e-3) / 1e12 / PEAK_FP32_MFMA_TFLOPS, 4),
-                               "matrix_core_frac": round(flop * 16.0 / 36.0 / (wms * 1e-3) / 1e12 / PEAK_FP32_MFMA_TFLOPS, 4)}
+                               "matrix_core_frac": round(executed / (wms * 1e-3) / 1e12 / matrix_peak, 4), "matrix_core_peak": matrix_peak}
         if name == "conv1":
             row["note"] = ("launched back to back: the 205 MB of output of one launch compete with the write-back of the "
                            "launch before; inside the network the same launch takes about 0.18 ms (launches_in_network)")
