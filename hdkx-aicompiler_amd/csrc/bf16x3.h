@@ -1,17 +1,19 @@
 // bf16x3.h -- fp32 contractions on the bf16 matrix cores of gfx950 without giving up fp32's precision.
 //
-// An fp32 number has 24 significant bits, a bf16 number 8 and the same exponent range, so x = h + m + l with
-// h = bf16(x), m = bf16(x - h), l = bf16(x - h - m): both subtractions are exact, |m| <= 2^-8 |x|, |l| <= 2^-17 |x|, and
-// from |x| = 2^-109 on the three parts hold all 24 bits of x.  Below, the last bits lie under bf16's smallest step, 2^-133
-// (the matrix instructions take subnormal parts as they are), and h + m + l is off by at most 2^-134, which is all of an x
-// of that size.  Multiplying operands by 2^16 while they are split, and sums by 2^-32, keeps those bits as well and was not
-// taken: 300 x 1000 x 2048 15.4 -> 16.6 us, 64 x 1000 x 512 4.7 -> 5.0; KXC_HIP_GEMM_BF16X3=0 and KXC_HIP_WINOGRAD_BF16X3=0 keep the
-// fp32 instructions for callers whose operands are that small.
-// A product of two such numbers is nine bf16 products, each exact in fp32; the three that are left out (m*l', l*m', l*l') add
-// up to at most 2^-24 |x x'|, what rounding the product to fp32 may lose as well.  The six others are accumulated in fp32
-// by v_mfma_f32_32x32x16_bf16, smallest first.  Measured on random dot products of 64, 576 and 4608 terms against a float64
-// evaluation (relative error in the 2-norm): 1.1e-7 / 3.6e-7 / 1.1e-6, v_mfma_f32_32x32x2_f32 on the same data 1.4e-7 / 4.3e-7 /
-// 1.2e-6; all nine products change nothing (what is left is the fp32 accumulation).
+// The three-term split of Henry, Tang and Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype For
+// Higher-Precision Computations" (ARITH 2019).  An fp32 number has 24 significant bits, a bf16 number 8 and the same exponent
+// range, so x = h + m + l with h = bf16(x), m = bf16(x - h), l = bf16(x - h - m): both subtractions are exact,
+// |m| <= 2^-8 |x|, |l| <= 2^-17 |x|, and from |x| = 2^-109 on the three parts hold all 24 bits of x.  Below, the last bits lie
+// under bf16's smallest step, 2^-133 (the matrix instructions take subnormal parts as they are), and h + m + l is off by
+// at most 2^-134, which is all of an x of that size.  Multiplying operands by 2^16 while they are split, and sums by 2^-32,
+// keeps those bits as well and was not taken: 300 x 1000 x 2048 15.4 -> 16.6 us, 64 x 1000 x 512 4.7 -> 5.0 (with
+// v_dot2_f32_bf16 in the place of each unpacking and subtraction, which is exact, 16.8 and 4.9); KXC_HIP_GEMM_BF16X3=0 and
+// KXC_HIP_WINOGRAD_BF16X3=0 keep the fp32 instructions for callers whose operands are that small.
+// A product of two such numbers is nine bf16 products, each exact in fp32; the three that are left out (m*l', l*m', l*l')
+// add up to at most 2^-24 |x x'|, what rounding the product to fp32 may lose as well.  The six others are accumulated in
+// fp32 by v_mfma_f32_32x32x16_bf16, smallest first.  Measured on random dot products of 64, 576 and 4608 terms against a
+// float64 evaluation (relative error in the 2-norm): 1.1e-7 / 3.6e-7 / 1.1e-6, v_mfma_f32_32x32x2_f32 on the same data
+// 1.4e-7 / 4.3e-7 / 1.2e-6; all nine products change nothing (what is left is the fp32 accumulation).
 //
 // Why: a bf16 matrix instruction does 16x the work of an fp32 one per cycle and runs beside the vector ALU (the fp32
 // one shares its datapath), so six of them cost 6/16 of the fp32 instruction.  Measured in a loop of independent

@@ -1,6 +1,7 @@
 // conv2d_f32.hip -- nn_conv2d (NCHW data, OIHW weights, fp32) for gfx950.
 //
-// Two kernels behind one entry point:
+// Two kernels here behind one entry point (small launches: conv_small.h; large 3x3 stride-1 calls:
+// conv2d_wino_f32.hip):
 //
 //  * conv_mfma_kernel: implicit GEMM on the fp32 matrix cores (v_mfma_f32_32x32x2_f32),
 //    D[o][pixel] += W[o][k] * X[k][pixel], k = (channel, rh, rw).
@@ -26,8 +27,10 @@
 //
 //  * conv_direct_kernel: one thread per output element, the CPU loop nest's exact order
 //    (rc, rh, rw ascending from 0.0f, multiply and add rounded separately, padded taps add
-//    0.0f * w).  Bit-identical to the CPU backend; used for shapes the MFMA tiling does not
-//    cover (output channels not a multiple of 32, very wide rows) and on request.
+//    0.0f * w).  Bit-identical to the CPU backend; used on request and for what the matrix-core
+//    kernels do not take: filter extents without a tile, tensors beyond 31-bit offsets, very wide
+//    rows, and sums of fewer than 64 terms with fewer than 32 output channels or pixels (Select).
+//    Everything else sums in another order.
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
@@ -833,8 +836,9 @@ const Variant kVariants[] = {
     // each keep 32 channels x 224 pixels (seven blocks) in registers reach 192 us.
     KXC_VARIANT_TP_HP(7, 7, 1, 2, 2, 1, 7, 12),  // 64 x 448, 4 waves of 32 x 224
     KXC_VARIANT_TP_HP(7, 7, 1, 1, 7, 2, 1, 8),   // 64 x 224, 7 waves of 64 x 32
-    // 32 x 256, 2-channel chunks: the fastest or within 3 % of it among eight tiles of 64 to 256 pixels with 2- and 4-channel
-    // chunks (64 -> 96 channels at 27 x 27, batch 8: 530 us one thread per output, 38.9 here, 41 to 62 the others)
+    // The one 5x5 tile, whatever the size: 32 x 256, 2-channel chunks, the fastest or within 3 % of it among eight tiles of 64 to
+    // 256 pixels with 2- and 4-channel chunks on one layer (64 -> 96 channels at 27 x 27, batch 8: 530 us one thread per
+    // output, 38.9 here, 41 to 62 the others); small launches split their reduction over workgroups only
     KXC_VARIANT(5, 5, 2, 1, 8, 1, 1, 4),
     KXC_VARIANT(7, 7, 2, 1, 8, 1, 1, 8),   // 32 x 256; 2-channel chunks: two chunks for RGB, loads overlap compute
     KXC_VARIANT(7, 7, 2, 1, 7, 1, 1, 8),   // 32 x 224: two full output rows of a 112-wide map
@@ -1180,12 +1184,14 @@ int SmallWords(const SmallVariant& v, const ConvArgs& a) {
 //   tiles per compute unit (64 -> 128 with stride 2, batch 16: 10.9 -> 9.2), two before (512 -> 128 at 14 x 14, batch 4: 5.9 against 6.8).
 // 3x3: up to 800 tiles of 16 x 16, 1600 with the second output (a launch plan's two-output node otherwise needs an adding launch
 //   for both): 128 channels at 28 x 28 12.5 -> 7.9 us at batch 1 (392 tiles), 17 -> 12 at batch 2 (784), equal at batch 4;
-//   128 -> 256 with stride 2 and the second output, batch 8 (1568): 28.9 -> 26.1.  Up to 1600 also for at most 16 output channels,
+//   128 -> 256 with stride 2 and the second output, batch 8 (1568): 28.9 -> 26.1.  (Between 784, ahead, and 1568, equal, nothing
+//   was measured: 800 is the near side.)  Up to 1600 also for at most 16 output channels,
 //   half a block of the general tiles: 64 -> 16 at 56 x 56, batch 8 (1568) 25.9 -> 14.8.  At least 64 channels, a chunk per wave.
 //   Staged rows for narrow maps while every tile has a compute unit to itself (256 at 14 x 14, batch 1: 8.5 -> 7.5; 512 at 7 x
 //   7: 13.2 -> 10.9); two blocks of output channels from 257 tiles on (64 at 56 x 56, batch 1: 9.6 -> 8.7).
-//   Outside a plan, only from 400 tiles on: below, kxc_hip_conv2d_scratch_needed promises the callers of the single
-//   operator a reduction split over workgroups.
+//   Outside a plan, only from 400 tiles on.  That is no line of speed (the figures above are from plans and below it, too):
+//   kxc_hip_conv2d_scratch_needed reports a reduction split over workgroups for those calls, and callers of the entry point
+//   that allocates nothing rely on what it reports.
 const SmallVariant* SelectSmall(const kxc_hip_conv2d_desc* d, const ConvArgs& a, bool second, bool in_plan) {
     if ((d->flags & (KXC_HIP_CONV_FORCE_DIRECT | KXC_HIP_CONV_HPOOL)) || a.M <= 0 || a.C % 16 != 0 || d->kh != d->kw) return nullptr;
     const int64_t x_elems = static_cast<int64_t>(a.N) * a.C * a.H * a.W, y_elems = static_cast<int64_t>(a.N) * a.O * a.OHW;

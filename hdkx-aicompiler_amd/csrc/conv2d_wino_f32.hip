@@ -7,7 +7,7 @@
 // sixteen element-wise products are sixteen independent matrix products  M_f[o][tile] = sum_c U_f[o][c] V_f[c][tile]
 // (f = position in the 4x4 transform domain), which is what the matrix cores run.
 //
-//  * The filter transform U = G g G^T is done once per weight tensor by wino_weight_kernel into a packed buffer
+//  * The filter transform U = G g G^T is done once per weight tensor by wino_weight_batch_kernel into a packed buffer
 //    whose blocks are byte-for-byte the LDS image the main kernel wants: [32 output channels][4 input channels]
 //    as [c][o/16][f/4][o%16][f%4], 8 KiB per block, so that a workgroup fills its weight tile with 16-byte
 //    loads that write straight to LDS, and a lane's four f values of one (o, c) are one 16-byte LDS read.

@@ -19,8 +19,7 @@
 // compute unit, behind the chain launch - first loads - last store.  Measured, us, batch 1, residual and ReLU, against the
 // Winograd kernel with its adding launch: 64 channels at 56 x 56 10.2 -> 8.6, 128 at 28 x 28 10.8 -> 7.8, 256 at 14 x 14
 // 10.8 -> 7.6, 512 at 7 x 7 12.3 -> 11.1; against the implicit GEMM with two outputs: 64 -> 128 with stride 2 12.7 -> 8.7,
-// 128 -> 256 13.4 -> 7.2, 256 -> 512 14.0 -> 8.6.  1x1, 256 -> 512 at 14 x 14: 9.3 -> 4.2; 5x5, 64 -> 96 at 27 x 27 (one
-// thread per output before): 235 -> 12.5.
+// 128 -> 256 13.4 -> 7.2, 256 -> 512 14.0 -> 8.6.  1x1, 256 -> 512 at 14 x 14: 9.3 -> 4.2.
 #pragma once
 
 #include "common.h"
@@ -65,8 +64,7 @@ template <int KH, int KW, int CPG, int XI, int RO, int KS, bool DS = false>
 __global__ void __launch_bounds__(64 * KS) __attribute__((amdgpu_waves_per_eu(2))) conv_small_kernel(const Args a) {
     constexpr bool STAGED = XI > 0;
     constexpr int KHW = KH * KW, E = CPG * KHW, WI = RO * E / 4, NB = DS ? 2 * RO : RO;
-    constexpr int D = E <= 36 ? E : E / 5;                    // depth of the ring of X values
-    static_assert(E % 4 == 0 && E % D == 0 && (!DS || CPG == 4), "chunk layout");
+    static_assert(E % 4 == 0 && E <= 36 && (!DS || CPG == 4), "chunk layout");      // (36 loads of X in flight: vmcnt holds 63)
     constexpr int WAVE_LDS = (WI + XI) * 1024 + (STAGED ? 32 : 0);
     extern __shared__ __attribute__((aligned(16))) char lds[];
     const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
@@ -214,19 +212,19 @@ __global__ void __launch_bounds__(64 * KS) __attribute__((amdgpu_waves_per_eu(2)
 #pragma unroll
         for (int t = 0; t < KHW; ++t)
             xo[t] = valid(t) ? static_cast<uint32_t>(n * a.C + g * CPG) * plane + static_cast<uint32_t>((ih + t / KW * a.dh) * a.W + iw + t % KW * a.dw) * 4u : kOutside;
-        float xf[D];
+        float xf[E];
         auto load_x = [&](int chunk, int j) __attribute__((always_inline)) {
-            xf[j % D] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xr, xo[j % KHW], static_cast<uint32_t>(chunk * 4 * CPG + j / KHW) * plane, 0));
+            xf[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xr, xo[j % KHW], static_cast<uint32_t>(chunk * 4 * CPG + j / KHW) * plane, 0));
         };
         if (wave < a.nchunks) {
 #pragma unroll
-            for (int j = 0; j < D; ++j) {
+            for (int j = 0; j < E; ++j) {
                 load_x(wave, j);
                 __builtin_amdgcn_sched_barrier(0);                 // in this order: the waits of the loop count on it
             }
             for (int chunk = wave; chunk < a.nchunks; chunk += KS) {
                 const int next = min(chunk + KS, a.nchunks - 1);   // (the loads past the wave's last chunk are not used)
-                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(D) : "memory");      // all but the D loads of X behind the weights
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(E) : "memory");      // all but the E loads of X behind the weights
                 load_w2(chunk);
                 read_w();
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // read before they are written again
@@ -235,9 +233,8 @@ __global__ void __launch_bounds__(64 * KS) __attribute__((amdgpu_waves_per_eu(2)
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int j = 0; j < E; ++j) {
-                    multiply(j, xf[j % D]);
-                    if (j + D < E) load_x(chunk, j + D);
-                    else load_x(next, j + D - E);
+                    multiply(j, xf[j]);
+                    load_x(next, j);
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }

@@ -544,9 +544,9 @@ int32_t kxc_hip_gemm_f32(const float* a, const float* b, const float* c, float* 
         static const Tile kTiles[] = {KXC_GEMM(1, 1, 8, 2), KXC_GEMM(2, 1, 8, 2), KXC_GEMM(2, 2, 4, 1)};
 #undef KXC_GEMM
         // The largest tile (least splitting per product) that still leaves enough workgroups: 64 x 64 from 1024 blocks of
-        // 32 x 32 on (512 x 4096 x 512: 21.5 us, 27.5 with 64 x 32, 28.3 with 32 x 32), 64 x 32 while the compute units do
-        // not get one 32 x 32 tile each (300 x 1000 x 2048, 320 blocks: 18.4 against 19.6; 512 x 512 x 4096, 256: 30.7
-        // against 22.8)
+        // 32 x 32 on (512 x 4096 x 512: 21.5 us, 27.5 with 64 x 32, 28.3 with 32 x 32); 32 x 32 up to one per compute unit
+        // (512 x 512 x 4096, 256 blocks: 22.8 against 30.7 with 64 x 32), 64 x 32 between (300 x 1000 x 2048, 320: 18.4
+        // against 19.6 with 32 x 32)
         const int64_t blocks = CeilDiv(m, 32) * CeilDiv(n, 32);
         const Tile& t = kTiles[blocks <= 256 || k >= (1 << 22) ? 0 : blocks < 1024 ? 1 : 2];
         const int64_t m_tiles = CeilDiv(m, 32 * t.ro), tiles = m_tiles * CeilDiv(n, 32 * t.rp);

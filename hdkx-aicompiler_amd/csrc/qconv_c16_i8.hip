@@ -1257,7 +1257,7 @@ __global__ void __launch_bounds__(kBlock) gap_c16_kernel(const int8_t* __restric
 // Every wave loads its own operands, so the vector cache bounds it once there are many tiles; with few, its chain is the
 // shortest: 512 -> 512 channels at 7 x 7, batch 5: 23.1 -> 4.8 us.  SelectDirect has the line between the two.
 template <int KH, int RO, int RP, int KS, bool DS = false>
-__global__ void __launch_bounds__(64 * KS) __attribute__((amdgpu_waves_per_eu(KS >= 16 ? 4 : 2))) qconv_direct_kernel(const QArgs a) {
+__global__ void __launch_bounds__(64 * KS) __attribute__((amdgpu_waves_per_eu(2))) qconv_direct_kernel(const QArgs a) {
     constexpr int KHW = KH * KH, CBC = KH == 1 ? 4 : 2, NS = KHW * CBC / 2;
     constexpr int G = KH == 1 ? 3 : 1;               // chunks per loop trip
     constexpr int NB = RO * RP, NBA = DS ? 2 * NB : NB;

@@ -201,7 +201,8 @@ int32_t kxc_hip_conv2d_nchw_f32_noalloc(const kxc_hip_conv2d_desc* desc, const f
                                         const float* bias, const float* residual, float* y, void* stream);
 size_t kxc_hip_conv2d_noalloc_scratch_bytes(void);
 /* Bytes of scratch (partial sums) a launch for this shape uses, 0 when its reduction is not split over workgroups:
- * lets a caller see beforehand whether kxc_hip_conv2d_nchw_f32_noalloc takes the shape. */
+ * lets a caller see beforehand whether kxc_hip_conv2d_nchw_f32_noalloc takes the shape.  (For weights on a 16-byte boundary;
+ * others may take another kernel, which may use the array.) */
 int32_t kxc_hip_conv2d_scratch_needed(const kxc_hip_conv2d_desc* desc, size_t* out_bytes);
 
 /* Two nn_conv2d calls on the same input in one launch: the convolution `desc` describes (convolution.cc:38-75, with

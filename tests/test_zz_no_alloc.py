@@ -1,6 +1,7 @@
 """kxc_hip_conv2d_nchw_f32_noalloc -- the entry point that allocates nothing -- against kxc_hip_conv2d_nchw_f32.
 
-Both run the same kernels, so the outputs must be identical bit for bit; the shapes are ones whose reduction is
+On the shapes here both run the same kernels, so the outputs must be identical bit for bit (a large 3x3 stride-1 call, which
+transforms its filter into scratch, would not); they are ones whose reduction is
 split over workgroups (the launches that use scratch memory: the built-in device array here, a hipMalloc'ed
 buffer there).  Two calls in a row, the second on a smaller input, so stale contents of the shared array from
 the first call would show in the second.
