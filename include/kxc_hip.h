@@ -288,8 +288,8 @@ int32_t kxc_hip_global_avg_pool2d_f32(const float* x, float* y, int64_t n, int64
 
 /* nn_dense (DenseCompute, src/relay/op/nn/dense.cc:27-32) and nn_gemm (GemmCompute :34-61):
  * y[m,n] = alpha * sum_k a[m,k]*b[n,k] (transB=1) or a[m,k]*b[k,n] (transB=0), + beta*c[n].
- * c may be NULL (nn_dense); c_len is n or 1.  fp32 sums in an order of the kernel's own (products of fewer than 2^15
- * multiplies: the CPU loop's).  Products of more than four rows run on the bf16 matrix cores, every operand as three bf16
+ * c may be NULL (nn_dense); c_len is n or 1.  fp32 sums in an order of the kernel's own (the CPU loop's below 2^15
+ * multiplies, unless transB = 1 and k is a multiple of 32).  Products of more than four rows run on the bf16 matrix cores, every operand as three bf16
  * parts: exact from 2^-109 on, below it an operand is off by at most 2^-134; KXC_HIP_GEMM_BF16X3=0 in the environment keeps
  * the fp32 instructions, KXC_HIP_WINOGRAD_BF16X3=0 those of the convolutions (large 3x3 stride-1 ones). */
 int32_t kxc_hip_gemm_f32(const float* a, const float* b, const float* c, float* y,

@@ -929,6 +929,38 @@ def test_conv_operator_by_winograd_under_capture(pkg, monkeypatch):
     assert torch.equal(got, plain[0])
 
 
+def test_conv_operator_by_winograd_from_threads_and_streams(pkg):
+    """Eager calls with filters of their own, four threads on two streams at once: the buffer that a call writes its
+    transformed filter to is kept per stream, whose order keeps the calls of its two threads apart."""
+    import threading
+    n, c, h, o = 16, 64, 56, 64
+    rng = np.random.default_rng(78)
+    x = dev(rng.standard_normal((n, c, h, h)).astype(np.float32))
+    w = [dev((rng.standard_normal((o, c, 3, 3)) / 24).astype(np.float32)) for _ in range(4)]
+    assert pkg.conv2d_variant(x.shape, w[0].shape, 1, 1) == "winograd_f2k3_bf16x3"
+    want = [pkg.conv2d(x, v, None, None, 1, 1) for v in w]
+    out = [[torch.empty((n, o, h, h), device="cuda") for _ in range(8)] for _ in w]
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    errors = []
+
+    def calls(k):
+        try:
+            with torch.cuda.stream(streams[k % 2]):
+                for y in out[k]:
+                    pkg.conv2d(x, w[k], None, None, 1, 1, out=y)
+        except Exception as e:      # (an exception of a thread would pass unseen)
+            errors.append(e)
+    threads = [threading.Thread(target=calls, args=(k,)) for k in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not errors
+    assert all(torch.equal(y, want[k]) for k in range(4) for y in out[k])
+
+
 @pytest.mark.parametrize("n, c, h, w, o, k, s, p, winograd", [
     (2, 65, 8, 7, 17, 3, 1, 1, False), (1, 96, 3, 3, 48, 3, 1, 1, False), (8, 64, 27, 27, 96, 5, 1, 2, False), (12, 128, 28, 28, 128, 3, 1, 1, True)])
 def test_conv_split_launches_keep_shared_scratch_out_of_graphs(pkg, n, c, h, w, o, k, s, p, winograd):
