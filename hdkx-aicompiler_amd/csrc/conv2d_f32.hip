@@ -918,8 +918,9 @@ bool Fits(const Variant& v, const ConvArgs& a, Choice* out, bool ds = false) {
     return true;
 }
 
-// Picks the MFMA variant for a shape, or leaves choice.v == nullptr for the direct kernel.
-void Select(const ConvArgs& real, int kh, int kw, Choice* choice, bool ds = false) {
+// Picks the MFMA variant for a shape, or leaves choice.v == nullptr for the direct kernel.  in_workgroup: 1x1 filters split their
+// reduction as deep over wave groups as 3x3 ones before they split it over workgroups.
+void Select(const ConvArgs& real, int kh, int kw, Choice* choice, bool ds = false, bool in_workgroup = false) {
     choice->v = nullptr;
     // Fewer than 32 channels or pixels leave part of a 32 x 32 block empty, and the block still wins against one thread per
     // output with a serial sum unless that sum is short (us, one thread per output and here; 3x3 unless said): 156 -> 18
@@ -990,7 +991,7 @@ void Select(const ConvArgs& real, int kh, int kw, Choice* choice, bool ds = fals
                     *choice = split[k];
                     // enough waves: stop splitting further (1x1: 500 -> 400 at 20 x 20, batch 2 23.7 us four ways, 27.7 eight;
                     // 333 -> 100 at 33 x 33, batch 5, 1376 waves two ways 29.2, four 25.4)
-                    if (split_waves[k] >= (kh == 1 ? 1400 : 2560)) break;
+                    if (split_waves[k] >= (kh == 1 && !in_workgroup ? 1400 : 2560)) break;
                     // 3x3: two wave groups on the 32 x 128 tile plus the split over workgroups beat the deeper
                     // splits on 32 x 64 tiles from batch 1 to 16, at stride 2 (batch 8, 128 -> 256 channels at
                     // 28 x 28: 20.5 against 31.5 us) and at stride 1 (batch 1, 256 channels at 14 x 14: 12.6
@@ -1242,8 +1243,9 @@ struct ConvLaunch {
     bool in_plan = false;
 };
 
-// small = false: without the small-launch kernels (operands that are not aligned for them).
-int32_t Conv2dResolve(const kxc_hip_conv2d_desc* desc, bool second, const char* who, ConvLaunch* L, bool in_plan = false, bool small = true) {
+// small = false: without the small-launch kernels (operands that are not aligned for them).  in_workgroup: see Select.
+int32_t Conv2dResolve(const kxc_hip_conv2d_desc* desc, bool second, const char* who, ConvLaunch* L, bool in_plan = false, bool small = true,
+                      bool in_workgroup = false) {
     ConvArgs& a = L->a;
     if (int32_t rc = FillArgs(desc, &a, who)) return rc;
     L->second = second;
@@ -1312,7 +1314,7 @@ int32_t Conv2dResolve(const kxc_hip_conv2d_desc* desc, bool second, const char* 
         KXC_HIP_REQUIRE(!second && HpoolChoice(desc, a, &c), "%s: no kernel with the pooling epilogue covers this shape", who);
         a.PW = a.OW / 2;
     } else if (!(desc->flags & KXC_HIP_CONV_FORCE_DIRECT) && a.M > 0) {
-        Select(a, desc->kh, desc->kw, &c, second);
+        Select(a, desc->kh, desc->kw, &c, second, in_workgroup);
     }
     if (second) {
         int rh = 0, rw = 0;
@@ -1435,8 +1437,15 @@ int32_t Conv2dLaunch(const ConvLaunch& L, const char* who, const float* x, const
             // Launches that can do without the buffer of the stream's handle do so where the stream does not order its users:
             // one thread per output, without scratch, is what these filters and shapes are compared with.  For the others
             // a reduction in one piece would take up to five times as long (kxc_hip.h says what their graphs need); a
-            // plan's own graph is replayed on its capture stream.
-            bool split = L.in_plan || !(a.O < 32 || a.M < 32 || L.kh == 5) || StreamOrdersScratch(s);
+            // plan's own graph is replayed on its capture stream.  1x1 launches that take two parts for speed
+            // (697 -> 222 channels at 7 x 188, batch 3) have a kernel that splits over wave groups only.
+            const bool ordered = L.in_plan || StreamOrdersScratch(s);
+            if (!ordered && L.kh == 1) {
+                ConvLaunch other;
+                if (int32_t rc = Conv2dResolve(&L.desc, L.second, who, &other, false, false, true)) return rc;
+                if (other.scratch_bytes == 0) return Conv2dLaunch(other, who, x, w, bias, residual, y, stream, false, second);
+            }
+            bool split = ordered || !(a.O < 32 || a.M < 32 || L.kh == 5);
             if (split)
                 if (int32_t rc = AcquireSplitScratch(s, L.scratch_bytes, &lease, &split)) return rc;
             a.partial = lease.ptr;

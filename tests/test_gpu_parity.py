@@ -962,7 +962,8 @@ def test_conv_operator_by_winograd_from_threads_and_streams(pkg):
 
 
 @pytest.mark.parametrize("n, c, h, w, o, k, s, p, winograd", [
-    (2, 65, 8, 7, 17, 3, 1, 1, False), (1, 96, 3, 3, 48, 3, 1, 1, False), (8, 64, 27, 27, 96, 5, 1, 2, False), (12, 128, 28, 28, 128, 3, 1, 1, True)])
+    (2, 65, 8, 7, 17, 3, 1, 1, False), (1, 96, 3, 3, 48, 3, 1, 1, False), (8, 64, 27, 27, 96, 5, 1, 2, False), (12, 128, 28, 28, 128, 3, 1, 1, True),
+    (4, 385, 27, 25, 99, 1, 1, 0, False), (5, 308, 19, 11, 640, 1, 1, 0, False), (13, 349, 19, 47, 241, 1, 2, 0, False)])
 def test_conv_split_launches_keep_shared_scratch_out_of_graphs(pkg, n, c, h, w, o, k, s, p, winograd):
     """Launches whose eager form splits its reduction into the buffer of the stream's handle and that can do without: a graph of
     one is captured without a first call, replays on another stream beside eager calls on the capture stream, and gives the
