@@ -704,9 +704,11 @@ const WinoVariant* SelectWino(const kxc_hip_conv2d_desc* d, bool three_part = tr
     // 64 x 32 groups once the 64 x 16 ones are more than one per compute unit (64 channels at 56 x 56, batch 8: 196 against
     // 392, 19.9 against 24.7 us; at 49 x 49, batch 6: 118 against 235, 19.0 against 17.3).  A launch that cannot
     // give every SIMD two waves (at most one 64 x 32 group per compute unit) and has a long reduction splits the
-    // input channels over two groups of waves inside the workgroup instead.
+    // input channels over two groups of waves inside the workgroup instead.  With an odd number of steps it cannot, and so few
+    // 64 x 32 groups of a long reduction would be split over workgroups (GroupSplit) into the stream's buffer, which the
+    // 64 x 16 ones do without: those (836 -> 9 channels at 57 x 7, batch 60).
     const int64_t units = CeilDiv(Tiles(d), 32) * CeilDiv(d->o, 64) * lanes;
-    const int wt = units <= 128 ? 1 : 2;
+    const int wt = units <= 128 || (units < 256 && csteps >= 64 && csteps % 2 != 0) ? 1 : 2;
     const int ks = (units <= 256 && csteps % 2 == 0 && csteps >= 32) ? 2 : 1;
     for (int i = 0; i < kNumWino; ++i)
         if (kWino[i].wk == 2 && kWino[i].wt == wt && kWino[i].ks == ks) return &kWino[i];
