@@ -71,7 +71,9 @@ public:
 };
 
 // One launch of a compiled module, as an execution-plan node would describe it
-// (include/base/execution_plan.h:42-50): operator, kernel symbol, value ids.
+// (include/base/execution_plan.h:42-50): operator, kernel symbol, value ids.  kernel_symbol says what the operator asked for
+// while the plan was built; a convolution whose filter was to be transformed, or that has a second output, may launch the kernel
+// for small launches instead, and then the plan node's symbol (kxc_hip_plan_node_symbol) says so.
 struct KernelExecInfo {
     std::string op_name;
     std::string kernel_symbol;

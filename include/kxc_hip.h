@@ -588,7 +588,7 @@ typedef struct kxc_hip_launch_record {
 int32_t kxc_hip_plan_run_profiled(kxc_hip_plan* plan, void** packed_args, void* stream,
                                   kxc_hip_launch_record* records, int32_t capacity, int32_t* count);
 int32_t kxc_hip_plan_num_nodes(const kxc_hip_plan* plan);
-/* kernel_symbol of node i (static storage owned by the plan). */
+/* kernel_symbol of node i (static storage owned by the plan).  After finalize it names the kernel that the node launches. */
 const char* kxc_hip_plan_node_symbol(const kxc_hip_plan* plan, int32_t i);
 /* Device address of the workspace (NULL before finalize): lets tests read intermediates. */
 void* kxc_hip_plan_workspace(const kxc_hip_plan* plan);

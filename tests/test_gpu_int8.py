@@ -171,6 +171,8 @@ def test_qconv_c16_largest_wave_tile_against_cpu(pkg, orc, monkeypatch):
     (1, 17, 1, 1, 32, 3, 1, "o1_p1_ks2"), (3, 80, 13, 9, 96, 3, 2, "o1_p1_ks2"), (5, 512, 7, 7, 512, 3, 1, "o1_p1_ks2"),
     (1, 32, 32, 512, 32, 3, 1, "o1_p1_ks2"), (1, 48, 27, 19, 1088, 3, 1, "o2_p1_ks2"), (21, 512, 7, 7, 512, 3, 1, "o2_p2_ks4"),
     (1, 65, 1, 1, 32, 1, 1, "o1_p1_ks2"), (3, 250, 11, 13, 64, 1, 2, "o1_p1_ks2"), (2, 496, 31, 34, 256, 1, 1, "o2_p1_ks4"),
+    # strides and rows whose patch no staged kernel holds
+    (2, 40, 44, 143, 64, 3, 3, "o1_p1_ks2"), (1, 20, 9, 200, 32, 3, 2, "o1_p1_ks2"), (1, 33, 10, 301, 32, 1, 3, "o1_p1_ks2"),
 ], ids=lambda s: "x".join(map(str, s)))
 def test_qconv_c16_direct_kernel(pkg, orc, monkeypatch, shape):
     """The kernel of small launches, at the edges of its tiles and of the rule that chooses its tile: the same bytes as the

@@ -214,8 +214,8 @@ def test_resnet18_hip_plan_without_gpu():
     with tempfile.TemporaryDirectory() as d:
         run("resnet18", "hip", d, "1", "224")
         one = json.load(open(os.path.join(d, "plan.json")))
-    # batch 1: the same thirteen layers (small launches split their input channels over workgroups); too few tiles
-    # for the first layer's pooling epilogue to pay
+    # batch 1: the same thirteen layers (which of them run without the transform is settled when the plan is finalized); too
+    # few tiles for the first layer's pooling epilogue to pay
     assert sum("winograd" in n["kernel_symbol"] for n in one["nodes"]) == 13
     assert not any("maxpool3w" in n["kernel_symbol"] for n in one["nodes"])
     with tempfile.TemporaryDirectory() as d:
@@ -453,8 +453,8 @@ def test_resnet18_two_shares_replay_from_saved_plan(synth):
 
 @pytest.mark.gpu
 def test_resnet18_benchmarked_plan_batch1_matches_oracle(synth):
-    """Benchmark configuration 3 through the plan the benchmark times at batch 1 (Winograd with the input channels
-    split over workgroups, small-launch 1x1 kernel)."""
+    """Benchmark configuration 3 through the plan the benchmark times at batch 1: thirteen layers that the operators asked
+    Winograd for, which at this size run on the kernel for small launches like the blocks' first convolutions."""
     from gpu_util import assert_close, assert_bit_exact
     x, consts, eager, replay, facts = _compiled_resnet18_logits(synth, 3, 1)
     assert sum(".winograd_f2k3" in s for s in facts["launches"]) == 13, facts["launches"]
