@@ -727,6 +727,7 @@ struct WinoLaunch {
     bool three_part = false;    // wino_bf16x3_kernel with `bx` instead of v->kernel with `a`
     wino_bx::Args bx;
     int bx_plane = 0;
+    int bx_loads = 0;           // wino_bx::PatchLoads
     size_t u_offset = 0;        // of the three-part form in the filter buffer
 };
 
@@ -739,8 +740,16 @@ void ThreePartResolve(const kxc_hip_conv2d_desc* d, WinoLaunch* L, bool may_spli
     b.TW = a.TW; b.TI = a.TI; b.NT = a.NT; b.HW = a.HW; b.OHW = a.OHW;
     b.Hq = 2 * (a.TI / a.TW) + 2;
     const int64_t rows = wino_bx::MaxPatchRows(b.NT, b.TI, b.TW);
-    b.pitch = wino_bx::RowPitch(b.TW, rows, wino_bx::kPlanes[1]);
-    L->bx_plane = rows * 2 * b.pitch <= wino_bx::kPlanes[0] ? 0 : 1;
+    const int64_t wide_pitch = 4 + CeilDiv(b.W, 4) * 4;
+    if (b.pw == 1 && rows * wide_pitch + 4 <= wino_bx::kPlanes[1]) {
+        L->bx_plane = rows * wide_pitch + 4 <= wino_bx::kPlanes[0] ? 0 : 1;
+        L->bx_loads = b.W % 4 == 0 ? wino_bx::kWide : wino_bx::kWideEdge;
+        b.pitch = wino_bx::WideRowPitch(b.W, b.TW, rows, wino_bx::kPlanes[L->bx_plane]);
+    } else {
+        L->bx_loads = wino_bx::kNarrow;
+        b.pitch = wino_bx::RowPitch(b.TW, rows, wino_bx::kPlanes[1]);
+        L->bx_plane = rows * 2 * b.pitch <= wino_bx::kPlanes[0] ? 0 : 1;
+    }
     b.ksteps = static_cast<int32_t>(CeilDiv(a.C, wino_bx::kStep));
     b.t_groups = static_cast<int32_t>(CeilDiv(a.NT, wino_bx::kTiles));
     b.k_groups = static_cast<int32_t>(CeilDiv(a.O, wino_bx::kOut));
@@ -764,6 +773,15 @@ void ThreePartResolve(const kxc_hip_conv2d_desc* d, WinoLaunch* L, bool may_spli
     b.div_pitch = MakeFastDiv(b.pitch); b.div_hq = MakeFastDiv(b.Hq);
     L->three_part = true;
     L->lds_bytes = wino_bx::kLdsBytes;
+}
+
+template <bool RECHECK>
+auto ThreePartKernel(const WinoLaunch& L) -> void (*)(const wino_bx::Args) {
+    using namespace wino_bx;
+    static void (*const kernels[2][3])(const Args) = {
+        {wino_bf16x3_kernel<512, kNarrow, RECHECK>, wino_bf16x3_kernel<512, kWide, RECHECK>, wino_bf16x3_kernel<512, kWideEdge, RECHECK>},
+        {wino_bf16x3_kernel<768, kNarrow, RECHECK>, wino_bf16x3_kernel<768, kWide, RECHECK>, wino_bf16x3_kernel<768, kWideEdge, RECHECK>}};
+    return kernels[L.bx_plane][L.bx_loads];
 }
 
 void FillWinoArgs(const kxc_hip_conv2d_desc* desc, WinoLaunch* L) {
@@ -856,7 +874,7 @@ int32_t WinoRun(const WinoLaunch& L, const float* x, const float* u, const float
         wino_bx::Args b = L.bx;
         if (!split) whole(b, b.ksteps);
         b.x = x; b.u = reinterpret_cast<const char*>(u) + L.u_offset; b.bias = bias; b.res = residual; b.y = y; b.partial = a.partial;
-        void (*const bx)(const wino_bx::Args) = L.bx_plane == 0 ? wino_bx::wino_bf16x3_kernel<512, false> : wino_bx::wino_bf16x3_kernel<768, false>;
+        void (*const bx)(const wino_bx::Args) = ThreePartKernel<false>(L);
         if (int32_t rc = GrantLds(reinterpret_cast<const void*>(bx))) return rc;
         hipLaunchKernelGGL(bx, NoteGrid(dim3(static_cast<unsigned>(b.units_per_xcd * 8))), NoteBlock(dim3(wino_bx::kThreads)),
                            NoteLds(L.lds_bytes), s, b);
@@ -964,7 +982,7 @@ int32_t RunWinogradOperator(const kxc_hip_conv2d_desc* desc, const float* x, con
     if (int32_t rc = CheckLaunch("wino_weight_batch_kernel")) return rc;
     wino_bx::Args b = L.bx;
     b.x = x; b.u = reinterpret_cast<const char*>(lease.ptr); b.w = w; b.bias = bias; b.res = residual; b.y = y;
-    void (*const bx)(const wino_bx::Args) = L.bx_plane == 0 ? wino_bx::wino_bf16x3_kernel<512, true> : wino_bx::wino_bf16x3_kernel<768, true>;
+    void (*const bx)(const wino_bx::Args) = ThreePartKernel<true>(L);
     if (int32_t rc = GrantLds(reinterpret_cast<const void*>(bx))) return rc;
     hipLaunchKernelGGL(bx, NoteGrid(dim3(static_cast<unsigned>(b.units_per_xcd * 8))), NoteBlock(dim3(wino_bx::kThreads)), NoteLds(L.lds_bytes), stream, b);
     return CheckLaunch(kThreePart);

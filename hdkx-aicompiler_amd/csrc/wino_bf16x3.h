@@ -8,18 +8,22 @@
 //    memory in the order the lanes read it (packed once per weight tensor, 96 bytes per (o, c)), and a wave transforms
 //    the input it needs straight into matrix operands.  The L2 traffic of U sets the 64 x 64 block: half as many tiles
 //    would double it to 64 bytes per clock and compute unit, the L2's limit.
-//  * LDS holds only the raw input patches of 16 channels (filled by LDS-direct loads, three in flight).
+//  * LDS holds only the raw input patches of 16 channels (filled by LDS-direct loads, three in flight).  A load occupies the
+//    address unit for 16 cycles however wide it is, and with 4-byte loads the patches took half of every step there (with
+//    three of four left out, timing only, 64 images: 82 -> 65, 63 -> 52, 52 -> 46, 68 -> 53 us for the layers below), so rows
+//    come in pieces of 16 bytes wherever the padding allows it (WIDE).
 //  * A wave's vector instructions do not run beside its own matrix instructions, only beside the other wave's of its
 //    SIMD (measured: four vector instructions between two v_mfma_f32_32x32x16_bf16 of one wave add 15 cycles, issued by
 //    another wave nothing), so the two waves of a SIMD work in opposite phases.  Per step of 16 channels a SIMD has 3072
-//    cycles of matrix instructions; a step takes about 6000 (2.5 us), the serial time of one wave: 48 matrix instructions,
-//    270 vector instructions, 96 LDS reads, 28-36 loads.  Loads issued in a row stall a wave on the address unit (16 cycles
-//    each for all eight waves), so they stand one by one between matrix instructions (2.95 -> 2.5 us per step).
+//    cycles of matrix instructions, 1.8 us at the rate that a loop of nothing else reaches; a step takes about 2.2 us
+//    (2.5-2.7 with 4-byte patch loads).  Loads issued in a row stall a wave on the address unit, so they stand one by one
+//    between matrix instructions.
 // The output transform needs all 16 f of one (o, tile): every wave applies the column half to its own two positions and
 // leaves two values per (o, tile) in LDS, 32 x 32 outputs at a time; the row half sums over the eight waves.
 //
-// Measured (64 images, against the fp32-instruction kernel, us): 64 channels at 56 x 56 84 / 99, 128 at 28 x 28 64 / 90,
-// 256 at 14 x 14 55 / 87, 512 at 7 x 7 68 / 88; 32 images 41 / 51, 34 / 47, 39 / 55, 42 / 55.  Relative error against
+// Measured (64 images, against 4-byte patch loads and the fp32-instruction kernel, us): 64 channels at 56 x 56 71 / 83 / 99,
+// 128 at 28 x 28 54 / 64 / 90, 256 at 14 x 14 48 / 52 / 87, 512 at 7 x 7 62 / 67 / 88; 32 images 35 / 41 / 51, 28 / 33 / 47,
+// 35 / 38 / 55, 39 / 42 / 55.  Relative error against
 // float64 (2-norm): 1.0e-7 to 1.4e-7, the fp32-instruction kernel 1.3e-7 to 1.7e-7.
 #pragma once
 
@@ -40,6 +44,12 @@ constexpr size_t kLdsBytes = 3u * kStep * 768 * sizeof(float);       // 144 KiB:
 // Bytes of the packed three-part filter: [o / 32][c / 16][f][part][lane][16 bytes], lane = o % 32 + 32 * (c / 8 % 2).
 inline size_t WeightBytes(int64_t O, int64_t C) { return static_cast<size_t>(CeilDiv(O, 32) * CeilDiv(C, kStep)) * 16 * 3 * 1024; }
 
+// How the patch gets into LDS (template parameter).  kNarrow: 4-byte loads, even and odd columns in half planes of their own;
+// any padding.  kWide, for a padding of one column: rows as they are in memory in pieces of 16 bytes behind one piece that
+// reads as zero, which is the left border of its row and the right border of the row before.  kWideEdge: the same where the
+// rows are no multiple of four floats; their last piece ends in floats of the next row, which the reader replaces by zeros.
+enum PatchLoads { kNarrow = 0, kWide = 1, kWideEdge = 2 };
+
 // Row pitch of a half plane (at least TW + 1): the smallest that puts 32 neighbouring tiles into different LDS banks, or the
 // best one that fits `limit`.  The rows of a tile row are two pitches apart: at 14 x 14 outputs (7 tiles a row) a pitch of 8
 // puts every second tile row into the same banks (measured: 3072 of 8300 cycles per step lost to conflicts).
@@ -52,6 +62,21 @@ inline int32_t RowPitch(int64_t TW, int64_t rows, int64_t limit) {
             const int c = ++count[(t / TW * 2 * pitch + t % TW) % 32];
             if (c > worst) worst = c;
         }
+        if (worst < best_worst) { best_worst = worst; best = static_cast<int32_t>(pitch); }
+        if (worst == 1) break;
+    }
+    return best;
+}
+
+// Row pitch of a kWide plane: a zero piece and the row, and more zero pieces where that spreads 32 neighbouring tiles better
+// over the banks (a lane reads 8 bytes; the rows of a tile row are two pitches apart).
+inline int32_t WideRowPitch(int64_t W, int64_t TW, int64_t rows, int64_t limit) {
+    const int64_t least = 4 + CeilDiv(W, 4) * 4;
+    int32_t best = static_cast<int32_t>(least);
+    int best_worst = 1 << 30;
+    for (int64_t pitch = least; pitch <= least + 28 && rows * pitch + 4 <= limit; pitch += 4) {
+        int count[32] = {0}, worst = 0;
+        for (int t = 0; t < 32; ++t) worst = std::max(worst, ++count[(t / TW * pitch + t % TW) % 32]);
         if (worst < best_worst) { best_worst = worst; best = static_cast<int32_t>(pitch); }
         if (worst == 1) break;
     }
@@ -88,7 +113,7 @@ struct Args {
     float* partial;
     const float* w;                    // RECHECK: OIHW weights
     int32_t N, C, H, W, O, OH, OW, ph, pw;
-    int32_t TW, TI, NT, Hq, pitch;      // tiles per row, per image, in total; rows per image of the patch, row pitch of a half plane
+    int32_t TW, TI, NT, Hq, pitch;      // tiles per row, per image, in total; rows per image of the patch, row pitch of a (half) plane
     int32_t HW, OHW, ksteps;
     int32_t t_groups, k_groups, num_units, units_per_xcd, k_fastest;
     uint32_t x_bytes, u_bytes, flags;
@@ -165,10 +190,12 @@ inline int64_t WeightTiles(int64_t O, int64_t C) { return CeilDiv(O, 32) * CeilD
 
 // RECHECK (the single operator): the transforms spread an Inf or NaN over the whole 2x2 tile, and so do sums beyond the
 // largest float; a thread that finds such a tile evaluates its outputs by the loop of the operator's definition.
-template <int kPlane, bool RECHECK>
+template <int kPlane, int LOADS, bool RECHECK>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) wino_bf16x3_kernel(const Args a) {
     constexpr int kHalf = kPlane / 2, kSegs = kPlane / 64;
-    constexpr int NP = kSegs * kStep / 8;                 // patch loads of a wave per step
+    constexpr bool kIsWide = LOADS != kNarrow;
+    constexpr int kPieces = kPlane / 256;                 // kWide: loads (64 pieces of 16 bytes) of a channel
+    constexpr int NP = kIsWide ? 2 * kPieces : kSegs * kStep / 8;      // patch loads of a wave per step
     extern __shared__ __attribute__((aligned(16))) float lds[];
     const int tid = static_cast<int>(threadIdx.x), lane = tid & 63, half = lane >> 5, r = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -195,21 +222,40 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
         P = (qlast - qmin + 1) * a.pitch;
     }
     // segments of 64 floats: wave w loads segment w of all 16 channels and, of a plane of 768, segment 8 + w % 4 of eight
-    constexpr int kSecond = NP > kStep ? 1 : 0;
+    // (kWide: wave w loads channels 2 w and 2 w + 1, every lane pieces lane + 64 k)
+    constexpr int kSecond = !kIsWide && NP > kStep ? 1 : 0;
     const int seg2 = 8 + (wave & 3), c2 = (wave >> 2) * 8;
-    uint32_t goff[1 + kSecond];
+    uint32_t goff[kIsWide ? kPieces : 1 + kSecond];
+    if constexpr (kIsWide) {
 #pragma unroll
-    for (int k = 0; k < 1 + kSecond; ++k) {
-        const int at = (k ? seg2 : wave) * 64 + lane, odd = at >= kHalf ? 1 : 0, pos = at - odd * kHalf;
-        const int q = fast_div(pos, a.div_pitch), iw = 2 * (pos - q * a.pitch) + odd - a.pw;
-        const int Q = qmin + q, n = fast_div(Q, a.div_hq), ih = Q - n * a.Hq - a.ph;
-        const bool ok = pos < P && n < a.N && ih >= 0 && ih < a.H && iw >= 0 && iw < a.W;
-        goff[k] = ok ? static_cast<uint32_t>((n * a.C * a.H + ih) * a.W + iw) * 4u : kOob;
+        for (int k = 0; k < kPieces; ++k) {
+            const int pos = (k * 64 + lane) * 4, q = fast_div(pos, a.div_pitch), iw = pos - q * a.pitch - 4;
+            const int Q = qmin + q, n = fast_div(Q, a.div_hq), ih = Q - n * a.Hq - a.ph;
+            const bool ok = pos < P && n < a.N && ih >= 0 && ih < a.H && iw >= 0 && iw < a.W;
+            goff[k] = ok ? static_cast<uint32_t>((n * a.C * a.H + ih) * a.W + iw) * 4u : kOob;
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < 1 + kSecond; ++k) {
+            const int at = (k ? seg2 : wave) * 64 + lane, odd = at >= kHalf ? 1 : 0, pos = at - odd * kHalf;
+            const int q = fast_div(pos, a.div_pitch), iw = 2 * (pos - q * a.pitch) + odd - a.pw;
+            const int Q = qmin + q, n = fast_div(Q, a.div_hq), ih = Q - n * a.Hq - a.ph;
+            const bool ok = pos < P && n < a.N && ih >= 0 && ih < a.H && iw >= 0 && iw < a.W;
+            goff[k] = ok ? static_cast<uint32_t>((n * a.C * a.H + ih) * a.W + iw) * 4u : kOob;
+        }
     }
     const uint32_t plane_bytes = static_cast<uint32_t>(a.HW) * 4u;
     // Always NP loads, so that every wait knows how many are younger: positions past the patch, and channels past the last
     // one or steps past the end (an empty descriptor), read as zero without touching memory.
     auto load_patch_one = [&](int s, float* buf, int e) __attribute__((always_inline)) {
+        if constexpr (kIsWide) {
+            // (the channel is part of the base, so that the range check ends the last piece of a row at the end of the tensor)
+            const int cl = wave * 2 + e / kPieces, c = s * kStep + cl;
+            const uint32_t skip = s < s_hi && c < a.C ? static_cast<uint32_t>(c) * plane_bytes : a.x_bytes;
+            const __amdgpu_buffer_rsrc_t xr = make_rsrc(reinterpret_cast<const char*>(a.x) + skip, a.x_bytes - skip);
+            load16_to_lds(xr, (lds_void_t)(buf + cl * kPlane + (e % kPieces) * 256), goff[e % kPieces], 0);
+            return;
+        }
         const bool second = e >= kStep;
         const int c = second ? c2 + e - kStep : e, seg = second ? seg2 : wave;
         const __amdgpu_buffer_rsrc_t xr = make_rsrc(a.x, s < s_hi && c < a.C - s * kStep ? a.x_bytes : 0u);
@@ -248,6 +294,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
     //   i = 0: d0 - d2, 1: d1 + d2, 2: d2 - d1, 3: d1 - d3,   and columns to t0 - t2, t1 + t2 (jp = 0) or t2 - t1, t1 - t3 (jp = 1)
     const int rowa = wi == 0 ? 0 : wi == 2 ? 2 : 1, rowb = wi == 0 ? 2 : wi == 1 ? 2 : wi == 2 ? 1 : 3;
     const float sr = wi == 1 ? 1.0f : -1.0f;
+    bool in2[2], in3[2];                           // kWideEdge: the patch's third and fourth column lie in the image
     int base[2];                                   // (the second row's base is one addition away: registers are what is short here)
     const int drow = (rowb - rowa) * a.pitch;
 #pragma unroll
@@ -255,7 +302,8 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
         const int tile = min(t0 + j * 32 + r, a.NT - 1);
         const int n = fast_div(tile, a.div_ti), rem = tile - n * a.TI;
         const int ty = fast_div(rem, a.div_tw), tx = rem - ty * a.TW;
-        base[j] = (n * a.Hq + 2 * ty + rowa - qmin) * a.pitch + tx + half * 8 * kPlane;
+        base[j] = (n * a.Hq + 2 * ty + rowa - qmin) * a.pitch + (kIsWide ? 2 * tx + 3 : tx) + half * 8 * kPlane;
+        if constexpr (LOADS == kWideEdge) { in2[j] = 2 * tx + 1 < a.W; in3[j] = 2 * tx + 2 < a.W; }
     }
 
     f32x16 acc[2][2][2];      // [position][o block][tile block]
@@ -284,6 +332,14 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
 #pragma unroll
             for (int c = 0; c < 2; ++c) {
                 const int o = (2 * k + c) * kPlane;
+                if constexpr (kIsWide) {
+                    // columns 1 and 2 of the patch are 8 aligned bytes (the row's columns 2 tx and 2 tx + 1)
+                    const f32x2 ma = *reinterpret_cast<const f32x2*>(pa + o + 1), mb = *reinterpret_cast<const f32x2*>(pb + o + 1);
+                    constexpr int SIDE = JP == 0 ? 0 : 3;
+                    d[k & 1][c][JP == 0 ? 0 : 1] = pa[o + SIDE]; d[k & 1][c][JP == 0 ? 1 : 2] = ma[0]; d[k & 1][c][JP == 0 ? 2 : 0] = ma[1];
+                    d[k & 1][c][JP == 0 ? 3 : 4] = pb[o + SIDE]; d[k & 1][c][JP == 0 ? 4 : 5] = mb[0]; d[k & 1][c][JP == 0 ? 5 : 3] = mb[1];
+                    continue;
+                }
                 d[k & 1][c][0] = pa[o + U]; d[k & 1][c][1] = pa[o + X]; d[k & 1][c][2] = pa[o + W_];
                 d[k & 1][c][3] = pb[o + U]; d[k & 1][c][4] = pb[o + X]; d[k & 1][c][5] = pb[o + W_];
             }
@@ -294,7 +350,15 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
 #pragma unroll
             for (int c = 0; c < 2; ++c) {
                 const float* const e = d[k & 1][c];
-                const float tu = __builtin_fmaf(sr, e[3], e[0]), tx = __builtin_fmaf(sr, e[4], e[1]), tw = __builtin_fmaf(sr, e[5], e[2]);
+                float tu = __builtin_fmaf(sr, e[3], e[0]), tx = __builtin_fmaf(sr, e[4], e[1]), tw = __builtin_fmaf(sr, e[5], e[2]);
+                if constexpr (LOADS == kWideEdge) {
+                    if (JP == 0) {
+                        tw = in2[j] ? tw : 0.0f;
+                    } else {
+                        tu = in2[j] ? tu : 0.0f;
+                        tx = in3[j] ? tx : 0.0f;
+                    }
+                }
                 v0[c] = __fsub_rn(tu, tw);
                 v1[c] = JP == 0 ? __fadd_rn(tx, tw) : __fsub_rn(tw, tx);
             }

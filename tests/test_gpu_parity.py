@@ -885,6 +885,33 @@ def test_conv_winograd_three_part_prepared_filter(pkg, monkeypatch, n, c, h, w, 
         assert np.linalg.norm(host(got) - want) <= (9 * c + 16) ** 0.5 * 2.0 ** -23 * np.linalg.norm(want), (bias is None, residual is None)
 
 
+@pytest.mark.parametrize("n, c, h, w, o", [
+    (2, 16, 56, 56, 64), (5, 20, 14, 14, 33), (9, 16, 7, 7, 64), (3, 18, 13, 25, 64), (2, 32, 37, 51, 65), (2, 16, 30, 30, 64), (1, 16, 31, 63, 32),
+    (40, 16, 1, 1, 8), (1, 16, 1, 70, 8), (30, 16, 2, 4, 8), (1, 4, 5, 3, 1)])
+def test_conv_winograd_three_part_rows_in_pieces_of_16_bytes(pkg, monkeypatch, n, c, h, w, o):
+    """Patches loaded 16 bytes at a time: rows that are and are not a multiple of four floats, planes of 512 and of 768, operands
+    on a 4-byte address.  A row's last piece holds the beginning of the next row, so NaN in every row's first column and behind
+    the tensor must not reach outputs whose windows do not hold it.  9 c + 16 roundings of at most 2^-23, of independent signs."""
+    monkeypatch.setenv("KXC_HIP_WINOGRAD_VARIANT", "winograd_f2k3_bf16x3")
+    rng = np.random.default_rng(n * c + h * w + o)
+    c4 = (c + 3) // 4 * 4
+    x = rng.standard_normal((n, c4, h, w)).astype(np.float32)
+    wt = (rng.standard_normal((o, c4, 3, 3)) / np.sqrt(9 * c4)).astype(np.float32)
+    assert pkg.conv2d_winograd_variant(x.shape, wt.shape, 1, 1) == "winograd_f2k3_bf16x3"
+    u = pkg.conv2d_winograd_transform_weights(x.shape, dev(wt), 1)
+
+    def run(a):
+        room = torch.full((a.size + 9,), float("nan"), device="cuda")
+        xd = room[1:1 + a.size].view(a.shape)
+        xd.copy_(dev(a))
+        return host(pkg.conv2d_winograd(xd, u, wt.shape, None, None, 1, False))
+    want = torch.nn.functional.conv2d(torch.from_numpy(x).double(), torch.from_numpy(wt).double(), None, 1, 1).numpy()
+    got = run(x)
+    assert np.linalg.norm(got - want) <= (9 * c4 + 16) ** 0.5 * 2.0 ** -23 * np.linalg.norm(want)
+    x[:, :, :, 0] = np.nan
+    assert np.array_equal(run(x)[..., 4:], got[..., 4:])      # (the first column is in the patches of outputs 0 to 3 at most)
+
+
 def test_conv_operator_by_winograd_under_capture(pkg, monkeypatch):
     """A large 3x3 call transforms its filter into the buffer of its stream handle, so a graph of it must not hold that buffer:
     captured after an eager call has grown it, on hipStreamPerThread and in the entry point that allocates nothing the call runs
