@@ -7,8 +7,8 @@
 // under bf16's smallest step, 2^-133 (the matrix instructions take subnormal parts as they are), and h + m + l is off by
 // at most 2^-134, which is all of an x of that size.  Multiplying operands by 2^16 while they are split, and sums by 2^-32,
 // keeps those bits as well and was not taken: 300 x 1000 x 2048 15.4 -> 16.6 us, 64 x 1000 x 512 4.7 -> 5.0 (with
-// v_dot2_f32_bf16 in the place of each unpacking and subtraction, which is exact, 16.8 and 4.9); KXC_HIP_GEMM_BF16X3=0 and
-// KXC_HIP_WINOGRAD_BF16X3=0 keep the fp32 instructions for callers whose operands are that small.
+// v_dot2_f32_bf16 in the place of each unpacking and subtraction, which is exact, 16.8 and 4.9); KXC_HIP_GEMM_BF16X3=0,
+// KXC_HIP_WINOGRAD_BF16X3=0 and KXC_HIP_CONV_BF16X3=0 keep the fp32 instructions for callers whose operands are that small.
 // A product of two such numbers is nine bf16 products, each exact in fp32; the three that are left out (m*l', l*m', l*l')
 // add up to at most 2^-24 |x x'|, what rounding the product to fp32 may lose as well.  The six others are accumulated in
 // fp32 by v_mfma_f32_32x32x16_bf16, smallest first.  Measured on random dot products of 64, 576 and 4608 terms against a
@@ -88,6 +88,27 @@ __device__ __forceinline__ void mfma6(f32x16 (&acc)[RO][RP], const u32x4 (&a)[RO
         for (int i = 0; i < RO; ++i)
 #pragma unroll
             for (int j = 0; j < RP; ++j) acc[i][j] = mfma_bf16(a[i][PA[p]], b[j][PB[p]], acc[i][j]);
+}
+
+// The 3x3 filters of 32 output channels x CHANNELS input channels (cn of them present) into LDS, rows of 9 * CHANNELS + 1
+// floats, by 256 threads.  Every thread's loads are in flight together: a launch of few workgroups is one memory round trip
+// (90 -> 150 channels: 11.7 us one load behind the other, 7.4 here; the thirteen layers of ResNet-18, which write 95 MB: 21.2, 20.1).
+template <int CHANNELS>
+__device__ __forceinline__ void stage_filters(const float* __restrict__ w, int32_t O, int32_t C, int o0, int c0, int cn, float* raw) {
+    constexpr int RUN = CHANNELS * 9, N = 32 * RUN / 256;
+    float v[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        const int idx = k * 256 + static_cast<int>(threadIdx.x), ol = idx / RUN, r = idx - ol * RUN;
+        const bool ok = o0 + ol < O && r < cn * 9;
+        const float x = w[ok ? (static_cast<int64_t>(o0 + ol) * C + c0) * 9 + r : 0];
+        v[k] = ok ? x : 0.0f;
+    }
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        const int idx = k * 256 + static_cast<int>(threadIdx.x), ol = idx / RUN;
+        raw[ol * (RUN + 1) + idx - ol * RUN] = v[k];
+    }
 }
 
 #endif  // __HIPCC__

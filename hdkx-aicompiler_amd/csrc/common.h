@@ -167,6 +167,16 @@ int32_t LaunchPreparedWinograd(const PreparedWinograd* p, const float* x, const 
                                const float* residual, float* y, hipStream_t stream);
 void FreePreparedWinograd(PreparedWinograd* p);
 
+// A convolution on a packed filter (conv2d_bf16x3.hip): bytes of the filter that a plan's node of this shape reads (0: it reads
+// its weights as they are), and the launch; *out = nullptr: no such launch, or u_bytes do not hold the filter.
+struct PreparedPacked;
+size_t PackedFilterBytes(const kxc_hip_conv2d_desc* desc, bool second_output);
+void PreparePacked(const kxc_hip_conv2d_desc* desc, bool second_output, size_t u_bytes, PreparedPacked** out);
+const char* PreparedPackedName(const PreparedPacked* p);
+int32_t LaunchPreparedPacked(const PreparedPacked* p, const float* x, const float* w, const void* u, const float* bias, const float* residual,
+                             float* y, const float* w2, const float* bias2, float* y2, hipStream_t stream);
+void FreePreparedPacked(PreparedPacked* p);
+
 // A single nn_conv2d by the three-part Winograd kernel, filter transform included (conv2d_wino_f32.hip): which shapes it is
 // for, and the call.  *launched = false, nothing enqueued: there is no scratch for the filter, or the stream does not order it.
 bool WinogradOperatorPreferred(const kxc_hip_conv2d_desc* desc);
@@ -174,13 +184,15 @@ int32_t RunWinogradOperator(const kxc_hip_conv2d_desc* desc, const float* x, con
                             float* y, hipStream_t stream, bool* launched);
 extern const char* const kWinogradOperatorName;
 
-// The filter transforms of several Winograd layers in one launch (conv2d_wino_f32.hip).
-constexpr uint32_t kWinoFormF32 = 1, kWinoFormThreePart = 2;
+// The filter transforms of several Winograd layers, and the packed filters of other convolutions, in one launch
+// (conv2d_wino_f32.hip).
+constexpr uint32_t kWinoFormF32 = 1, kWinoFormThreePart = 2, kFormPacked = 4;
 struct WinoWeightJob {
     const kxc_hip_conv2d_desc* desc;
     const float* w;      // OIHW weights
     float* u;            // where they go, the fp32 form first
-    uint32_t forms;      // kWinoForm*: the forms of the filter to write (PreparedWinogradForms: what a node's launch reads)
+    uint32_t forms;      // kWinoForm*: the forms of the filter to write (PreparedWinogradForms: what a node's launch reads), or kFormPacked
+    const float* w2;     // kFormPacked: the second output's weights, or nullptr
 };
 uint32_t PreparedWinogradForms(const PreparedWinograd* p);
 int32_t LaunchWinogradWeightTransforms(const WinoWeightJob* jobs, int32_t count, hipStream_t stream);

@@ -1,0 +1,183 @@
+// conv2d_bf16x3.hip -- a launch plan's 3x3 stride-2 convolutions, with or without the second (1x1) output, on the bf16 matrix
+// cores: which launches take the kernel of conv_bf16x3.h, and its launch.  The filter is read in packed form, written
+// by the plan's filter launch (conv2d_wino_f32.hip).
+#include <algorithm>
+#include <cstdlib>
+#include <cstring>
+#include <memory>
+
+#include "conv_bf16x3.h"
+
+using namespace kxc_hip;
+
+namespace {
+
+struct PackedLaunch {
+    conv_bx::Args a;
+    void (*kernel)(const conv_bx::Args) = nullptr;
+    const char* name = "";
+    bool second = false;
+    size_t scratch_bytes = 0;
+};
+
+// Rows of a row phase that a workgroup's pixels touch at most.  Where a tile starts within an image repeats after
+// OHW / gcd(OHW, kPix) tiles.
+int64_t MaxRows(const conv_bx::Args& a, int extra) {
+    int64_t rem = a.OHW, gcd = conv_bx::kPix;
+    while (rem != 0) { const int64_t r = gcd % rem; gcd = rem; rem = r; }
+    const int64_t tiles = std::min<int64_t>(CeilDiv(a.M, conv_bx::kPix), a.OHW / gcd);
+    int64_t best = 0;
+    for (int64_t t = 0; t < tiles; ++t) {
+        const int64_t m0 = t * conv_bx::kPix, ml = std::min<int64_t>(m0 + conv_bx::kPix, a.M) - 1;
+        const int64_t q0 = m0 / a.OHW * a.Hq + m0 % a.OHW / a.OW, q1 = ml / a.OHW * a.Hq + ml % a.OHW / a.OW;
+        best = std::max(best, q1 - q0 + extra + 1);
+    }
+    return best;
+}
+
+// Parts of a reduction, while all of them together are at most one workgroup per compute unit: what gives the shortest of
+// 2.9 us per step of 16 channels + the adding launch (5 us and the parts' way to memory and back at 4.5 TB/s).  us, 1 / 2 / 4 / 8
+// parts without the adding launch: 64 -> 128 channels at 49 x 49, batch 6 (59 workgroups) 19.9 / 14.8 / 12.9; 128 -> 256 at 25 x
+// 25, batch 5 (28) 24.7 / 17.0 / 13.4 / 12.2; 256 -> 512 at 14 x 14, batch 32 (100) 47.5 / 30.8 / 34.2 / 41.9, batch 64 (196)
+// 54.1 / 57.3 / 66.3; with it 64 -> 128 at 56 x 56, batch 8 (98) 22 and 28.
+int Split(int64_t units, int csteps, int64_t out_bytes) {
+    int best = 1;
+    double best_us = 2.9 * csteps;
+    for (int s = 2; s <= 8 && units * s <= 256 && s <= csteps && out_bytes * s <= (16LL << 20); s *= 2) {
+        const double us = 2.9 * static_cast<double>(CeilDiv(csteps, s)) + 5 + 2.0 * s * static_cast<double>(out_bytes) / 4.5e6;
+        if (us < best_us) { best_us = us; best = s; }
+    }
+    return best;
+}
+
+// Whether the kernel covers a launch (`L` is filled if so).
+bool Resolve(const kxc_hip_conv2d_desc* d, bool second, PackedLaunch* L) {
+    using namespace conv_bx;
+    if (!d || d->n <= 0 || d->c <= 0 || d->h <= 0 || d->w <= 0 || d->o <= 0) return false;
+    if (d->kh != 3 || d->kw != 3 || d->stride_h != 2 || d->stride_w != 2 || d->dil_h != 1 || d->dil_w != 1 || d->pad_h != 1 || d->pad_w != 1) return false;
+    if ((d->flags & (KXC_HIP_CONV_FORCE_DIRECT | KXC_HIP_CONV_HPOOL)) || d->c % kStep != 0) return false;
+    const int64_t OH = (static_cast<int64_t>(d->h) - 1) / 2 + 1, OW = (static_cast<int64_t>(d->w) - 1) / 2 + 1;
+    const int64_t x_bytes = 4LL * d->n * d->c * d->h * d->w, y_elems = static_cast<int64_t>(d->n) * d->o * OH * OW;
+    const int64_t u_bytes = static_cast<int64_t>(FilterBytes(d->o, d->c, 3, second));
+    if (d->w > 4 * kPlane || x_bytes >= (1LL << 31) || y_elems >= (1LL << 29) || u_bytes >= (1LL << 31) || (d->n + 1LL) * (OH + 1) >= (1LL << 30)) return false;
+    Args& a = L->a;
+    std::memset(&a, 0, sizeof(a));
+    a.N = d->n; a.C = d->c; a.H = d->h; a.W = d->w; a.O = d->o;
+    a.OH = static_cast<int32_t>(OH); a.OW = static_cast<int32_t>(OW); a.OHW = a.OH * a.OW; a.HW = a.H * a.W;
+    a.M = a.N * a.OHW;
+    a.ph = a.pw = 1;
+    a.Hq = a.OH + 1;
+    const int64_t rows = MaxRows(a, 1);
+    a.w4 = (a.W + 3) / 4;
+    if (2 * rows * a.w4 > 64 * kProducers * kUnits) return false;
+    // even columns 0 .. OW, odd ones behind them.  Where it fits, a row pitch that continues the banks of a row's last pixel with
+    // the next row's first one (a lane reads 16 bytes: 16 positions go through all banks).
+    a.hp = std::max(a.OW + 1, a.W / 2 + 1);
+    a.pitch = 2 * a.hp;
+    if (rows * a.pitch > kPlane) return false;
+    for (int32_t pitch = a.pitch; pitch < a.pitch + 16 && rows * pitch <= kPlane; ++pitch)
+        if ((pitch - a.OW) % 16 == 0) { a.pitch = pitch; break; }
+    a.csteps = a.C / kStep;
+    a.p_tiles = static_cast<int32_t>(CeilDiv(a.M, kPix));
+    a.o_tiles = static_cast<int32_t>(CeilDiv(a.O, kOut));
+    const int64_t units = static_cast<int64_t>(a.p_tiles) * a.o_tiles;
+    if (units >= (1LL << 27)) return false;
+    a.num_units = static_cast<int32_t>(units);
+    a.x_bytes = static_cast<uint32_t>(x_bytes);
+    a.u_bytes = static_cast<uint32_t>(u_bytes);
+    a.flags = d->flags;
+    const int64_t out_bytes = y_elems * 4 * (second ? 2 : 1);
+    const int split = Split(units * SelectLanes(), a.csteps, out_bytes);
+    a.cps = static_cast<int32_t>(CeilDiv(a.csteps, split));
+    a.gsplit = static_cast<int32_t>(CeilDiv(a.csteps, a.cps));      // no empty part
+    if (a.gsplit > 1) L->scratch_bytes = static_cast<size_t>(a.gsplit) * out_bytes;
+    a.units_per_xcd = static_cast<int32_t>(CeilDiv(units * a.gsplit, 8));
+    a.o_fastest = u_bytes <= (2 << 20) ? 1 : 0;      // an XCD's run of workgroups shares its input while the filters stay in the L2
+    a.div_ohw = MakeFastDiv(a.OHW); a.div_ow = MakeFastDiv(a.OW); a.div_hq = MakeFastDiv(a.Hq); a.div_w4 = MakeFastDiv(a.w4);
+    a.div_tiles = MakeFastDiv(a.o_fastest ? a.o_tiles : a.p_tiles); a.div_gsplit = MakeFastDiv(a.gsplit);
+    L->second = second;
+    L->kernel = second ? conv_bf16x3_kernel<3, 2, true> : conv_bf16x3_kernel<3, 2, false>;
+    L->name = second ? "mfma_k3x3s2_bf16x3_ds" : "mfma_k3x3s2_bf16x3";
+    return true;
+}
+
+// Whether a plan's node should take it: from 0.12 GFLOP per step of 16 channels on, 1.4 at most, counting the launches expected
+// side by side.  A workgroup takes 9 us and 2.9 per step however few there are, and the other kernels start with 16 x 16 tiles and
+// split reductions inside a workgroup (us, theirs and here, both outputs): 64 -> 128 channels at 56 x 56, batch 2 (0.26 GFLOP)
+// 12.3 and 16.4, batch 4 (0.51) 23.1 and 20.2, batch 8 32.4 and 20.9, batch 32 59 and 36, batch 64 97 and 60; 128 -> 256 at 28 x 28, batch 6
+// (0.77) 20.5 and 22.1, batch 8 (1.03) 25.5 and 23.7, batch 16 39 and 31, batch 64 94 and 54; 256 -> 512 at 14 x 14, batch 8 (1.03)
+// 21.8 and 22.8, batch 12 (1.54) 31 and 25, batch 32 71 and 37, batch 64 104 and 52; 512 -> 512 at 14 x 14, batch 5 (1.28) 21.5 and 22.6; 512 ->
+// 1024 at 28 x 28, batch 2 68 and 36; 16 -> 32 at 56 x 56, batch 20 (0.16) 15.0 and 11.5.  KXC_HIP_CONV_BF16X3=0 keeps the kernels on the fp32 instructions (=1 takes this one
+// wherever it covers the launch), and so does KXC_HIP_CONV_VARIANT, which names one of theirs.
+bool Preferred(const kxc_hip_conv2d_desc* d, bool second, PackedLaunch* L) {
+    const char* e = std::getenv("KXC_HIP_CONV_BF16X3");
+    const char* variant = std::getenv("KXC_HIP_CONV_VARIANT");
+    if ((e && e[0] == '0') || (variant && *variant) || !Resolve(d, second, L)) return false;
+    const double gflop = 2e-9 * L->a.M * L->a.O * L->a.C * conv_bx::Steps(3, second) * SelectLanes();
+    return (e && e[0] == '1') || gflop >= std::min(0.12 * L->a.csteps, 1.4);
+}
+
+}  // namespace
+
+namespace kxc_hip {
+
+struct PreparedPacked {
+    PackedLaunch launch;
+};
+
+size_t PackedFilterBytes(const kxc_hip_conv2d_desc* desc, bool second) {
+    PackedLaunch L;
+    return Preferred(desc, second, &L) ? L.a.u_bytes : 0;
+}
+
+void PreparePacked(const kxc_hip_conv2d_desc* desc, bool second, size_t u_bytes, PreparedPacked** out) {
+    std::unique_ptr<PreparedPacked> p(new PreparedPacked);
+    *out = Preferred(desc, second, &p->launch) && u_bytes >= p->launch.a.u_bytes ? p.release() : nullptr;
+}
+
+const char* PreparedPackedName(const PreparedPacked* p) { return p->launch.name; }
+void FreePreparedPacked(PreparedPacked* p) { delete p; }
+
+int32_t LaunchPreparedPacked(const PreparedPacked* p, const float* x, const float* w, const void* u, const float* bias, const float* residual,
+                             float* y, const float* w2, const float* bias2, float* y2, hipStream_t s) {
+    const PackedLaunch& L = p->launch;
+    conv_bx::Args a = L.a;
+    KXC_HIP_REQUIRE(x && w && u && y && (!L.second || (w2 && y2)), "%s: NULL pointer", L.name);
+    KXC_HIP_REQUIRE(!(a.flags & KXC_HIP_CONV_BIAS) || bias, "%s: bias flag without bias", L.name);
+    KXC_HIP_REQUIRE(!(a.flags & KXC_HIP_CONV_RESIDUAL) || residual, "%s: residual flag without residual", L.name);
+    a.x = x; a.w = w; a.u = static_cast<const char*>(u); a.bias = bias; a.res = residual; a.y = y;
+    a.w2 = w2; a.bias2 = bias2; a.y2 = y2;
+    SplitScratchLease lease;      // held until the adding kernel is enqueued
+    if (a.gsplit > 1) {
+        bool split = false;
+        if (int32_t rc = AcquireSplitScratch(s, L.scratch_bytes, &lease, &split)) return rc;
+        a.partial = lease.ptr;
+        if (!split) {             // no buffer to be had: the reduction in one piece
+            a.gsplit = 1;
+            a.cps = a.csteps;
+            a.div_gsplit = MakeFastDiv(1);
+            a.units_per_xcd = static_cast<int32_t>(CeilDiv(a.num_units, 8));
+        }
+    }
+    if (int32_t rc = GrantLds(reinterpret_cast<const void*>(L.kernel))) return rc;
+    hipLaunchKernelGGL(L.kernel, NoteGrid(dim3(static_cast<unsigned>(a.units_per_xcd * 8))), NoteBlock(dim3(conv_bx::kThreads)),
+                       NoteLds(conv_bx::kLdsBytes), s, a);
+    if (int32_t rc = CheckLaunch(L.name)) return rc;
+    if (a.gsplit == 1) return KXC_HIP_OK;
+    SplitReduceArgs r;
+    r.partial = a.partial; r.bias = bias; r.res = residual; r.y = y;
+    r.total = a.M * a.O; r.gsplit = a.gsplit; r.O = a.O; r.flags = a.flags; r.div_ohw = a.div_ohw;
+    if (L.second) {
+        r.partial2 = a.partial + static_cast<int64_t>(a.gsplit) * r.total;
+        r.bias2 = bias2; r.y2 = y2; r.flags2 = bias2 ? KXC_HIP_CONV_BIAS : 0u;
+    }
+    return LaunchSplitReduce(s, r);
+}
+
+}  // namespace kxc_hip
+
+extern "C" int32_t kxc_hip_conv2d_node_filter_bytes(const kxc_hip_conv2d_desc* desc, int32_t second_output, size_t* out_bytes) {
+    KXC_HIP_REQUIRE(desc && out_bytes, "kxc_hip_conv2d_node_filter_bytes: NULL argument");
+    *out_bytes = PackedFilterBytes(desc, second_output != 0);
+    return KXC_HIP_OK;
+}

@@ -90,6 +90,7 @@ __device__ __forceinline__ float relu_sel(float v) { return __builtin_fmaxf(v, 0
 }  // namespace
 
 #include "wino_bf16x3.h"
+#include "conv_bf16x3.h"
 
 namespace {
 
@@ -111,7 +112,7 @@ __device__ __forceinline__ void wino_weight_tile(const float* __restrict__ w, fl
     const int o0 = ob * 32, c0 = cb * kWeightTileC;
     const int cn = min(kWeightTileC, C - c0);     // 4 or 8 (C is a multiple of 4)
     const int tid = threadIdx.x;
-    wino_bx::stage_filters<kWeightTileC>(w, O, C, o0, c0, cn, raw);
+    stage_filters<kWeightTileC>(w, O, C, o0, c0, cn, raw);
     __syncthreads();
     const int cl = tid >> 5, ol = tid & 31;
     if (cl >= cn) return;
@@ -145,13 +146,16 @@ inline int64_t WeightTiles(int64_t o_padded, int64_t C) { return (o_padded / 32)
 
 // The filter transforms of several layers in one launch (a launch plan transforms all its Winograd layers' weights
 // at the start of a run): block b belongs to the job whose [first_block, next first_block) range holds it.
-// A job is one form of one tensor: fp32 (wino_kernel) or three-part bf16 (wino_bf16x3_kernel).
+// A job is one form of one tensor: fp32 (wino_kernel) or three-part bf16 (wino_bf16x3_kernel), or a filter that is not
+// transformed, with the second output's (conv_bf16x3_kernel).
 constexpr int kMaxWeightJobs = 32;
 struct WinoWeightBatch {
     const float* w[kMaxWeightJobs];
     char* u[kMaxWeightJobs];
     int32_t O[kMaxWeightJobs], C[kMaxWeightJobs], first_block[kMaxWeightJobs + 1];
+    const float* w2[kMaxWeightJobs];
     uint32_t three_part;       // bit j: job j writes the three-part form
+    uint32_t packed;           // bit j: job j writes the filter of conv_bf16x3.h
     int32_t count;
 };
 __global__ void __launch_bounds__(256) wino_weight_batch_kernel(const WinoWeightBatch b) {
@@ -159,7 +163,8 @@ __global__ void __launch_bounds__(256) wino_weight_batch_kernel(const WinoWeight
     int j = 0;
     while (j + 1 < b.count && static_cast<int32_t>(blockIdx.x) >= b.first_block[j + 1]) ++j;
     const int tile = static_cast<int>(blockIdx.x) - b.first_block[j];
-    if ((b.three_part >> j) & 1u) wino_bx::weight_tile(b.w[j], b.u[j], b.O[j], b.C[j], tile, raw);
+    if ((b.packed >> j) & 1u) conv_bx::pack_tile(b.w[j], b.w2[j], b.u[j], b.O[j], b.C[j], tile, raw);
+    else if ((b.three_part >> j) & 1u) wino_bx::weight_tile(b.w[j], b.u[j], b.O[j], b.C[j], tile, raw);
     else wino_weight_tile(b.w[j], reinterpret_cast<float*>(b.u[j]), b.O[j], b.C[j], tile, raw);
 }
 
@@ -1003,8 +1008,8 @@ int32_t LaunchWinogradWeightTransforms(const WinoWeightJob* jobs, int32_t count,
     };
     for (int32_t j = 0; j < count; ++j) {
         const WinoWeightJob& job = jobs[j];
-        KXC_HIP_REQUIRE(job.desc && Supported(job.desc) && job.w && job.u, "winograd weight transform: bad job %d", j);
-        for (uint32_t form : {kWinoFormF32, kWinoFormThreePart}) {
+        KXC_HIP_REQUIRE(job.desc && (job.forms == kFormPacked || Supported(job.desc)) && job.w && job.u, "winograd weight transform: bad job %d", j);
+        for (uint32_t form : {kWinoFormF32, kWinoFormThreePart, kFormPacked}) {
             if (!(job.forms & form)) continue;
             if (b.count == kMaxWeightJobs)
                 if (int32_t rc = flush()) return rc;
@@ -1015,8 +1020,10 @@ int32_t LaunchWinogradWeightTransforms(const WinoWeightJob* jobs, int32_t count,
             b.O[b.count] = static_cast<int32_t>(O); b.C[b.count] = static_cast<int32_t>(C);
             b.first_block[b.count] = static_cast<int32_t>(blocks);
             if (three) b.three_part |= 1u << b.count;
+            if (form == kFormPacked) b.packed |= 1u << b.count;
+            b.w2[b.count] = job.w2;
             ++b.count;
-            blocks += three ? wino_bx::WeightTiles(O, C) : WeightTiles(CeilDiv(O, 32) * 32, C);
+            blocks += form != kWinoFormF32 ? wino_bx::WeightTiles(O, C) : WeightTiles(CeilDiv(O, 32) * 32, C);
             KXC_HIP_REQUIRE(blocks < kMaxGridX, "winograd weight transform: too many blocks");
         }
     }

@@ -45,9 +45,11 @@ struct Node {
     int32_t chain = 0;
     // Winograd convolution (i32[0] == 1 on a kConv2D node): the weight pointer whose transform bufs[5] holds
     const void* transformed_from = nullptr;
+    const void* transformed_from2 = nullptr;      // (the second output's, kConv2D with i32[0] == 2 and a packed filter)
     // convolution launches resolved at finalize (kernel, tile shape, grid, split, environment switches)
     std::shared_ptr<kxc_hip::PreparedConv> prepared_conv;
     std::shared_ptr<kxc_hip::PreparedWinograd> prepared_wino;
+    std::shared_ptr<kxc_hip::PreparedPacked> prepared_packed;
     // module kernel
     void* function = nullptr;
     uint32_t grid[3], block[3], shared_bytes = 0;
@@ -76,6 +78,9 @@ size_t FilterRoom(const Node& n) {
     return n.dims[0] > 0 ? static_cast<size_t>(n.dims[0]) : n.dims[0] == 0 ? kxc_hip::WinogradF32FilterBytes(&n.conv) : 0;
 }
 
+// A convolution that is not a Winograd node with a buffer for its packed filter: bufs[5], dims[0] bytes.
+bool HasPackedRoom(const Node& n) { return n.kind == NodeKind::kConv2D && n.i32[0] != 1 && n.bufs[5].kind == KXC_HIP_BUF_WORKSPACE && n.dims[0] > 0; }
+
 // Bytes of every operand whose size follows from the node's geometry (module kernels' parameters are checked by
 // offset only).
 void OperandExtents(const Node& n, std::vector<std::pair<kxc_hip_buf, size_t>>* out) {
@@ -95,6 +100,7 @@ void OperandExtents(const Node& n, std::vector<std::pair<kxc_hip_buf, size_t>>* 
             add(n.bufs[3], y);
             add(n.bufs[4], y);
             if (n.i32[0] == 1) add(n.bufs[5], static_cast<int64_t>(FilterRoom(n)), 1);
+            if (HasPackedRoom(n)) add(n.bufs[5], n.dims[0], 1);
             if (n.i32[0] == 2 && n.params.size() == 3) {
                 add(n.params[0], static_cast<int64_t>(d.o) * d.c);
                 add(n.params[1], d.o);
@@ -400,6 +406,33 @@ int32_t kxc_hip_plan_add_conv2d_pair(kxc_hip_plan* plan, const kxc_hip_conv2d_de
     if (desc->flags & KXC_HIP_CONV_RELU) n.symbol += "+relu";
     n.symbol += "|conv1x1";
     if (bias2.kind != KXC_HIP_BUF_NONE) n.symbol += "+bias";
+    return KXC_HIP_OK;
+}
+
+int32_t kxc_hip_plan_add_conv2d_packed(kxc_hip_plan* plan, const kxc_hip_conv2d_desc* desc, kxc_hip_buf x, kxc_hip_buf w,
+                                       kxc_hip_buf bias, kxc_hip_buf residual, kxc_hip_buf y, kxc_hip_buf w2, kxc_hip_buf bias2,
+                                       kxc_hip_buf y2, kxc_hip_buf u, size_t u_bytes) {
+    const char* who = "kxc_hip_plan_add_conv2d_packed";
+    KXC_PLAN_BEGIN(who);
+    KXC_HIP_REQUIRE(u.kind == KXC_HIP_BUF_WORKSPACE && u_bytes > 0, "%s: the packed filter lives in the plan workspace", who);
+    KXC_PLAN_BUF(u, false, who);
+    const bool second = w2.kind != KXC_HIP_BUF_NONE;
+    KXC_HIP_REQUIRE(second || (bias2.kind == KXC_HIP_BUF_NONE && y2.kind == KXC_HIP_BUF_NONE), "%s: a second output without weights", who);
+    // (the filter is packed at the start of a run, in front of every node)
+    for (const kxc_hip_buf& b : {w, w2})
+        KXC_HIP_REQUIRE(b.kind == KXC_HIP_BUF_NONE || b.kind == KXC_HIP_BUF_ARG || b.kind == KXC_HIP_BUF_ARG_OFFSET, "%s: weights must be packed arguments", who);
+    if (int32_t rc = second ? kxc_hip_plan_add_conv2d_pair(plan, desc, x, w, bias, residual, y, w2, bias2, y2)
+                            : kxc_hip_plan_add_conv2d(plan, desc, x, w, bias, residual, y)) return rc;
+    Node& n = plan->nodes.back();
+    n.bufs[5] = u;
+    n.dims[0] = static_cast<int64_t>(u_bytes);
+    kxc_hip::PreparedPacked* p = nullptr;
+    kxc_hip::PreparePacked(desc, second, u_bytes, &p);
+    if (p) {
+        const size_t prefix = std::strlen("kxc_conv2d_nchw_f32."), end = n.symbol.find_first_of("+|", prefix);
+        n.symbol = n.symbol.substr(0, prefix) + kxc_hip::PreparedPackedName(p) + (end == std::string::npos ? std::string() : n.symbol.substr(end));
+        kxc_hip::FreePreparedPacked(p);
+    }
     return KXC_HIP_OK;
 }
 
@@ -803,6 +836,12 @@ int32_t kxc_hip_plan_finalize(kxc_hip_plan* plan, size_t workspace_bytes) {
         KXC_HIP_CALL(hipSetDevice(plan->device_id), "HIP SetDevice");
         n.prepared_wino.reset();
         n.prepared_conv.reset();
+        n.prepared_packed.reset();
+        if (HasPackedRoom(n)) {
+            kxc_hip::PreparedPacked* p = nullptr;
+            kxc_hip::PreparePacked(&n.conv, n.i32[0] == 2, static_cast<size_t>(n.dims[0]), &p);
+            if (p) { n.prepared_packed.reset(p, kxc_hip::FreePreparedPacked); continue; }
+        }
         // (a small Winograd node, and one whose filter buffer holds no form, runs on its weights as they are, in one launch)
         if (n.i32[0] == 1 && !kxc_hip::SmallConvBeatsWinograd(&n.conv)) {
             kxc_hip::PreparedWinograd* p = nullptr;
@@ -834,7 +873,8 @@ int32_t kxc_hip_plan_finalize(kxc_hip_plan* plan, size_t workspace_bytes) {
     }
     for (Node& n : plan->nodes) {
         if (n.kind != NodeKind::kConv2D) continue;
-        const char* variant = n.prepared_wino ? kxc_hip::PreparedWinogradName(n.prepared_wino.get()) : kxc_hip::PreparedConvName(n.prepared_conv.get());
+        const char* variant = n.prepared_packed ? kxc_hip::PreparedPackedName(n.prepared_packed.get())
+                              : n.prepared_wino ? kxc_hip::PreparedWinogradName(n.prepared_wino.get()) : kxc_hip::PreparedConvName(n.prepared_conv.get());
         const std::string prefix = "kxc_conv2d_nchw_f32.";
         const size_t end = n.symbol.find_first_of("+|", prefix.size());
         if (n.symbol.compare(0, prefix.size(), prefix) == 0)
@@ -884,13 +924,25 @@ int32_t CheckRunArgs(kxc_hip_plan* plan, void** args, const char* who) {
     return KXC_HIP_OK;
 }
 
-// The filter transforms of the plan's Winograd nodes and the weight packs of its int8 convolutions, each kind in one
-// launch on `stream`: every one (only_changed: those whose weight pointer differs from the one last prepared, and the
+// The filter transforms of the plan's Winograd nodes with the packed filters of its other convolutions, and the weight packs
+// of its int8 convolutions, each kind in one launch on `stream`: every one (only_changed: those whose weight pointer differs from the one last prepared, and the
 // packs marked every_run).  *launched tells whether anything ran.  What was prepared is recorded only after its
 // launch has been enqueued without error, so a failed run is repeated by the next one.
 int32_t TransformConstants(kxc_hip_plan* plan, void** args, hipStream_t stream, bool only_changed, bool* launched) {
     std::vector<WinoWeightJob> jobs;
     std::vector<std::pair<Node*, const void*>> touched;
+    std::vector<std::pair<Node*, std::pair<const void*, const void*>>> touched_packed;
+    for (Node& n : plan->nodes) {
+        if (!n.prepared_packed) continue;
+        const void* w = Resolve(plan, n.bufs[1], args);
+        const void* w2 = n.i32[0] == 2 ? Resolve(plan, n.params[0], args) : nullptr;
+        if (only_changed && n.transformed_from == w && n.transformed_from2 == w2) continue;
+        touched_packed.emplace_back(&n, std::make_pair(w, w2));
+        float* const u = static_cast<float*>(Resolve(plan, n.bufs[5], args));
+        bool have = false;
+        for (const WinoWeightJob& j : jobs) have = have || (j.u == u && j.w == w && j.w2 == w2);
+        if (!have) jobs.push_back({&n.conv, static_cast<const float*>(w), u, kxc_hip::kFormPacked, static_cast<const float*>(w2)});
+    }
     for (Node& n : plan->nodes) {
         if (!n.prepared_wino) continue;
         const void* w = Resolve(plan, n.bufs[1], args);
@@ -902,7 +954,7 @@ int32_t TransformConstants(kxc_hip_plan* plan, void** args, hipStream_t stream, 
         const uint32_t forms = kxc_hip::PreparedWinogradForms(n.prepared_wino.get());
         for (WinoWeightJob& j : jobs)
             if (j.u == u && j.w == w) { have = true; j.forms |= forms; }
-        if (!have) jobs.push_back({&n.conv, static_cast<const float*>(w), u, forms});
+        if (!have) jobs.push_back({&n.conv, static_cast<const float*>(w), u, forms, nullptr});
     }
     std::vector<QPackJob> packs;
     std::vector<std::pair<PackJob*, const void*>> packed;
@@ -919,6 +971,7 @@ int32_t TransformConstants(kxc_hip_plan* plan, void** args, hipStream_t stream, 
     if (!jobs.empty()) {
         if (int32_t rc = LaunchWinogradWeightTransforms(jobs.data(), static_cast<int32_t>(jobs.size()), stream)) return rc;
         for (auto& t : touched) t.first->transformed_from = t.second;
+        for (auto& t : touched_packed) { t.first->transformed_from = t.second.first; t.first->transformed_from2 = t.second.second; }
     }
     if (!packs.empty()) {
         if (int32_t rc = LaunchQWeightPacks(packs.data(), static_cast<int32_t>(packs.size()), stream)) return rc;
@@ -958,6 +1011,16 @@ int32_t RunNode(kxc_hip_plan* plan, Node& n, void** args, void* s) {
                                                          static_cast<const float*>(B(5)), static_cast<const float*>(B(2)),
                                                          static_cast<const float*>(B(3)), static_cast<float*>(B(4)),
                                                          kxc_hip::ResolveStream(s));
+                    break;
+                }
+                if (n.prepared_packed) {
+                    const bool pair = n.i32[0] == 2;
+                    rc = kxc_hip::LaunchPreparedPacked(
+                        n.prepared_packed.get(), static_cast<const float*>(B(0)), static_cast<const float*>(B(1)), B(5),
+                        static_cast<const float*>(B(2)), static_cast<const float*>(B(3)), static_cast<float*>(B(4)),
+                        pair ? static_cast<const float*>(Resolve(plan, n.params[0], args)) : nullptr,
+                        pair ? static_cast<const float*>(Resolve(plan, n.params[1], args)) : nullptr,
+                        pair ? static_cast<float*>(Resolve(plan, n.params[2], args)) : nullptr, kxc_hip::ResolveStream(s));
                     break;
                 }
                 {
@@ -1321,14 +1384,16 @@ int32_t kxc_hip_plan_serialize(const kxc_hip_plan* plan, char* buffer, size_t ca
     auto I = [&](long long v) { std::snprintf(tmp, sizeof(tmp), " %lld", v); out += tmp; };
     auto F = [&](float v) { std::snprintf(tmp, sizeof(tmp), " %a", static_cast<double>(v)); out += tmp; };
     // (version 2 added the plan's select_lanes and every node's chain, version 3 the weight packs; version 4, written only
-    // where a reader of version 3 would assume more, Winograd nodes whose filter buffer has room for one form or none)
-    bool one_form = false;
+    // where a reader of version 3 would assume more, Winograd nodes whose filter buffer has room for one form or none;
+    // version 5, written only where there are some, convolutions with a packed filter)
+    bool one_form = false, packed = false;
     for (const Node& n : plan->nodes) {
+        packed = packed || HasPackedRoom(n);
         size_t both = 0;
         if (n.kind == NodeKind::kConv2D && n.i32[0] == 1 && n.dims[0] != 0 && kxc_hip_conv2d_winograd_weight_bytes(&n.conv, &both) == KXC_HIP_OK)
             one_form = one_form || FilterRoom(n) < both;
     }
-    out += one_form ? "kxc_hip_plan 4" : "kxc_hip_plan 3";
+    out += packed ? "kxc_hip_plan 5" : one_form ? "kxc_hip_plan 4" : "kxc_hip_plan 3";
     I(plan->num_args); I(static_cast<long long>(plan->workspace_bytes)); I(static_cast<long long>(plan->nodes.size()));
     I(plan->select_lanes);
     I(static_cast<long long>(plan->packs.size()));
@@ -1395,7 +1460,7 @@ int32_t kxc_hip_plan_deserialize(const char* text, int32_t device_id, kxc_hip_mo
     in >> magic >> version >> num_args >> workspace >> count;
     if (in && version >= 2) in >> select_lanes;
     if (in && version >= 3) in >> num_packs;
-    KXC_HIP_REQUIRE(in && magic == "kxc_hip_plan" && version >= 1 && version <= 4, "%s: not a version-1, -2, -3 or -4 plan", who);
+    KXC_HIP_REQUIRE(in && magic == "kxc_hip_plan" && version >= 1 && version <= 5, "%s: not a version-1, -2, -3, -4 or -5 plan", who);
     KXC_HIP_REQUIRE(num_packs >= 0 && num_packs < (1 << 20), "%s: implausible header", who);
     KXC_HIP_REQUIRE(select_lanes >= 1 && select_lanes <= 16, "%s: implausible header", who);
     KXC_HIP_REQUIRE(num_args >= 0 && num_args < (1 << 20) && workspace >= 0 && count >= 0 && count < (1 << 24),
@@ -1467,6 +1532,12 @@ int32_t kxc_hip_plan_deserialize(const char* text, int32_t device_id, kxc_hip_mo
             (!kxc_hip_conv2d_pair_supported(&n.conv) || n.params.size() != 3 || n.params[0].kind == KXC_HIP_BUF_NONE ||
              n.params[2].kind == KXC_HIP_BUF_NONE))
             return fail("bad convolution-pair node");
+        if (n.kind == NodeKind::kConv2D && n.i32[0] != 1 && version < 5) n.dims[0] = 0;      // (nothing read it before)
+        if (n.kind == NodeKind::kConv2D && n.i32[0] != 1 && n.dims[0] != 0) {
+            auto argument = [](const kxc_hip_buf& b) { return b.kind == KXC_HIP_BUF_ARG || b.kind == KXC_HIP_BUF_ARG_OFFSET; };
+            if (n.bufs[5].kind != KXC_HIP_BUF_WORKSPACE || n.dims[0] <= 0 || !argument(n.bufs[1]) || (n.i32[0] == 2 && !argument(n.params[0])))
+                return fail("bad convolution node with a packed filter");
+        }
         if (n.kind == NodeKind::kQConv2D && (n.i32[0] < 0 || n.i32[0] > 4 || (n.i32[0] == 4 && !kxc_hip_qconv2d_c4_maxpool_supported(&n.qconv))))
             return fail("bad int8 convolution node");
         if (n.kind == NodeKind::kQConv2D && n.i32[0] == 3 &&

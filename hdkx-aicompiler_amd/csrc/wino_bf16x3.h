@@ -125,27 +125,6 @@ struct Args {
 
 typedef __attribute__((address_space(3))) void* lds_void_t;
 
-// The 3x3 filters of 32 output channels x CHANNELS input channels (cn of them present) into LDS, rows of 9 * CHANNELS + 1
-// floats, by 256 threads.  Every thread's loads are in flight together: a launch of few workgroups is one memory round trip
-// (90 -> 150 channels: 11.7 us one load behind the other, 7.4 here; the thirteen layers of ResNet-18, which write 95 MB: 21.2, 20.1).
-template <int CHANNELS>
-__device__ __forceinline__ void stage_filters(const float* __restrict__ w, int32_t O, int32_t C, int o0, int c0, int cn, float* raw) {
-    constexpr int RUN = CHANNELS * 9, N = 32 * RUN / 256;
-    float v[N];
-#pragma unroll
-    for (int k = 0; k < N; ++k) {
-        const int idx = k * 256 + static_cast<int>(threadIdx.x), ol = idx / RUN, r = idx - ol * RUN;
-        const bool ok = o0 + ol < O && r < cn * 9;
-        const float x = w[ok ? (static_cast<int64_t>(o0 + ol) * C + c0) * 9 + r : 0];
-        v[k] = ok ? x : 0.0f;
-    }
-#pragma unroll
-    for (int k = 0; k < N; ++k) {
-        const int idx = k * 256 + static_cast<int>(threadIdx.x), ol = idx / RUN;
-        raw[ol * (RUN + 1) + idx - ol * RUN] = v[k];
-    }
-}
-
 // ------------------------------------------------------------------------------------------
 // Filter transform into the packed three-part form.  A workgroup takes 32 output channels x 16 input channels; thread
 // (i, half, o) makes row i of U = G g G^T for eight channels and stores its four positions' fragments: the 32 lanes of a

@@ -221,6 +221,13 @@ def conv2d_winograd_node_bytes(desc):
     return nbytes.value
 
 
+def conv2d_node_filter_bytes(desc, second_output=False):
+    """Bytes of packed filter that a plan's convolution node of this shape reads (0: it reads its weights as they are)."""
+    nbytes = C.c_size_t(0)
+    _check(lib().kxc_hip_conv2d_node_filter_bytes(C.byref(desc), C.c_int32(1 if second_output else 0), C.byref(nbytes)))
+    return nbytes.value
+
+
 def set_select_lanes(lanes):
     """Variant selection of this thread's stand-alone launches and queries assumes `lanes` equal launches side by
     side (kxc_hip_set_select_lanes); returns the previous value."""
@@ -640,6 +647,9 @@ class Plan:
 
     def add_conv2d_pair(self, desc, x, w, bias, residual, y, w2, bias2, y2):
         _check(lib().kxc_hip_plan_add_conv2d_pair(self._h, C.byref(desc), x, w, bias, residual, y, w2, bias2, y2))
+
+    def add_conv2d_packed(self, desc, x, w, bias, residual, y, w2, bias2, y2, u, u_bytes):
+        _check(lib().kxc_hip_plan_add_conv2d_packed(self._h, C.byref(desc), x, w, bias, residual, y, w2, bias2, y2, u, C.c_size_t(u_bytes)))
 
     def invalidate_constants(self):
         _check(lib().kxc_hip_plan_invalidate_constants(self._h))

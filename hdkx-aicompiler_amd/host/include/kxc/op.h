@@ -99,6 +99,7 @@ struct HIPDispatchContext {
     Attrs pair_attrs;
     Array<Type> pair_input_types;
     Array<HIPBuffer> pair_inputs;
+    std::vector<bool> pair_input_constant;
     HIPBuffer pair_output;
     // A pooling call that is the sole reader of this launch's value and that the operator's "FHIPPoolQuery" agreed
     // to produce as well: `output` and `out_type` are then the pooling call's, and alloc_temp(bytes) hands out

@@ -694,6 +694,7 @@ private:
                     ctx.pair_input_types.push_back(a.checked_type());
                     // (input 0 is the first call's; the others are packed arguments, which are always plain)
                     ctx.pair_inputs.push_back(i == 0 ? ctx.inputs[0] : BufferOf(a.get()));
+                    ctx.pair_input_constant.push_back(dynamic_cast<const ConstantNode*>(Resolve(a.get())) != nullptr);
                 }
                 ctx.pair_output = {KXC_HIP_BUF_WORKSPACE, slot_[carried->tail].first};
                 ctx.pair_output_layout = LayoutOf(carried->tail);

@@ -122,6 +122,18 @@ std::string Conv2DDispatch(const HIPDispatchContext& c, kxc_hip_plan* plan) {
     }
     if (c.has_pair) {
         const bool bias2 = c.pair_inputs.size() == 3;
+        // constant weights: the packed copy that the library's kernel for the shape reads, if it has one, gets a workspace region
+        size_t u_bytes = 0;
+        if (c.alloc_persistent && c.input_constant.size() > 1 && c.input_constant[1] && c.pair_input_constant.size() > 1 && c.pair_input_constant[1])
+            Check(kxc_hip_conv2d_node_filter_bytes(&d, 1, &u_bytes), "nn_conv2d pair dispatch");
+        if (u_bytes > 0) {
+            const HIPBuffer u = c.alloc_persistent(static_cast<int64_t>(u_bytes));
+            Check(kxc_hip_plan_add_conv2d_packed(plan, &d, B(c.inputs[0]), B(c.inputs[1]), has_bias ? B(c.inputs[2]) : none,
+                                                 c.has_residual ? B(c.residual) : none, B(c.output), B(c.pair_inputs[1]),
+                                                 bias2 ? B(c.pair_inputs[2]) : none, B(c.pair_output), B(u), u_bytes),
+                  "nn_conv2d pair dispatch");
+            return kxc_hip_plan_node_symbol(plan, kxc_hip_plan_num_nodes(plan) - 1);
+        }
         Check(kxc_hip_plan_add_conv2d_pair(plan, &d, B(c.inputs[0]), B(c.inputs[1]), has_bias ? B(c.inputs[2]) : none,
                                            c.has_residual ? B(c.residual) : none, B(c.output), B(c.pair_inputs[1]),
                                            bias2 ? B(c.pair_inputs[2]) : none, B(c.pair_output)),
@@ -141,6 +153,17 @@ std::string Conv2DDispatch(const HIPDispatchContext& c, kxc_hip_plan* plan) {
               "nn_conv2d dispatch");
         return std::string("kxc_conv2d_nchw_f32.") + kxc_hip_conv2d_winograd_variant(&d) + (has_bias ? "+bias" : "") +
                (c.has_residual ? "+add" : "") + (c.fused_relu ? "+relu" : "");
+    }
+    if (c.alloc_persistent && c.input_constant.size() > 1 && c.input_constant[1]) {
+        size_t u_bytes = 0;
+        Check(kxc_hip_conv2d_node_filter_bytes(&d, 0, &u_bytes), "nn_conv2d dispatch");
+        if (u_bytes > 0) {
+            const HIPBuffer u = c.alloc_persistent(static_cast<int64_t>(u_bytes));
+            Check(kxc_hip_plan_add_conv2d_packed(plan, &d, B(c.inputs[0]), B(c.inputs[1]), has_bias ? B(c.inputs[2]) : none,
+                                                 c.has_residual ? B(c.residual) : none, B(c.output), none, none, none, B(u), u_bytes),
+                  "nn_conv2d dispatch");
+            return kxc_hip_plan_node_symbol(plan, kxc_hip_plan_num_nodes(plan) - 1);
+        }
     }
     Check(kxc_hip_plan_add_conv2d(plan, &d, B(c.inputs[0]), B(c.inputs[1]), has_bias ? B(c.inputs[2]) : none,
                                   c.has_residual ? B(c.residual) : none, B(c.output)),

@@ -292,7 +292,8 @@ int32_t kxc_hip_global_avg_pool2d_f32(const float* x, float* y, int64_t n, int64
  * c may be NULL (nn_dense); c_len is n or 1.  fp32 sums in an order of the kernel's own (the CPU loop's below 2^15
  * multiplies, unless transB = 1 and k is a multiple of 32).  Products of more than four rows run on the bf16 matrix cores, every operand as three bf16
  * parts: exact from 2^-109 on, below it an operand is off by at most 2^-134; KXC_HIP_GEMM_BF16X3=0 in the environment keeps
- * the fp32 instructions, KXC_HIP_WINOGRAD_BF16X3=0 those of the convolutions (large 3x3 stride-1 ones). */
+ * the fp32 instructions, KXC_HIP_WINOGRAD_BF16X3=0 those of the convolutions (large 3x3 stride-1 ones),
+ * KXC_HIP_CONV_BF16X3=0 those of a plan's large 3x3 stride-2 ones. */
 int32_t kxc_hip_gemm_f32(const float* a, const float* b, const float* c, float* y,
                          int64_t m, int64_t n, int64_t k, float alpha, float beta,
                          int32_t transB, int64_t c_len, void* stream);
@@ -459,6 +460,17 @@ int32_t kxc_hip_conv2d_winograd_node_bytes(const kxc_hip_conv2d_desc* desc, size
 int32_t kxc_hip_plan_add_conv2d_pair(kxc_hip_plan* plan, const kxc_hip_conv2d_desc* desc, kxc_hip_buf x,
                                      kxc_hip_buf w, kxc_hip_buf bias, kxc_hip_buf residual, kxc_hip_buf y,
                                      kxc_hip_buf w2, kxc_hip_buf bias2, kxc_hip_buf y2);
+/* nn_conv2d, or both convolutions of kxc_hip_conv2d_pair_nchw_f32 (w2 / bias2 / y2; all absent for one output), with a
+ * workspace region `u` of u_bytes for a packed copy of the filters, which the launch that prepares the Winograd nodes'
+ * filters writes as well, under the same rules (kxc_hip_plan_freeze_constants).  w and w2 are packed arguments.
+ * kxc_hip_conv2d_node_filter_bytes says what a node of this shape reads under the calling thread's
+ * kxc_hip_set_select_lanes (0: its weights as they are; such a node belongs to the calls above).  A node that finds too
+ * little room when the plan is finalized, or whose shape no longer asks for it (KXC_HIP_CONV_BF16X3=0), reads its
+ * weights as they are.  Nodes of a plan may share `u` when they share w and w2 (the shares of a batch). */
+int32_t kxc_hip_plan_add_conv2d_packed(kxc_hip_plan* plan, const kxc_hip_conv2d_desc* desc, kxc_hip_buf x, kxc_hip_buf w,
+                                       kxc_hip_buf bias, kxc_hip_buf residual, kxc_hip_buf y, kxc_hip_buf w2,
+                                       kxc_hip_buf bias2, kxc_hip_buf y2, kxc_hip_buf u, size_t u_bytes);
+int32_t kxc_hip_conv2d_node_filter_bytes(const kxc_hip_conv2d_desc* desc, int32_t second_output, size_t* out_bytes);
 int32_t kxc_hip_plan_invalidate_constants(kxc_hip_plan* plan);
 int32_t kxc_hip_plan_freeze_constants(kxc_hip_plan* plan, int32_t frozen);
 int32_t kxc_hip_plan_add_pool2d(kxc_hip_plan* plan, const kxc_hip_pool2d_desc* desc, kxc_hip_buf x,

@@ -1,0 +1,160 @@
+"""Plan nodes on a packed filter (kxc_hip_plan_add_conv2d_packed): the three-part kernel for 3x3 stride-2 convolutions, with
+and without the second output, at the edges of its tiles, against float64; its values that are not finite; its filters."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import assert_bit_exact, dev, host
+
+pytestmark = pytest.mark.gpu
+
+
+def _want(x, w, bias, residual, relu, stride, pad):
+    t = lambda a: torch.from_numpy(a).double()
+    y = torch.nn.functional.conv2d(t(x), t(w), t(bias) if bias is not None else None, stride, pad).numpy()
+    if residual is not None:
+        y = y + residual
+    return np.maximum(y, 0.0) if relu else y
+
+
+class _Node:
+    """One packed convolution with its operands on the GPU; `run` returns its outputs."""
+
+    def __init__(self, pkg, xs, o, second, residual=False, bias=True, relu=True, seed=0):
+        rng = np.random.default_rng(seed)
+        n, c, h, w = xs
+        f32 = lambda s, k=1.0: (rng.standard_normal(s) * k).astype(np.float32)
+        self.pkg, self.second, self.relu = pkg, second, relu
+        ys = (n, o, (h + 1) // 2, (w + 1) // 2)
+        self.x, self.w, self.w2 = f32(xs), f32((o, c, 3, 3), (2 / (9 * c)) ** 0.5), f32((o, c, 1, 1), (2 / c) ** 0.5)
+        self.b, self.b2 = (f32((o,)), f32((o,))) if bias else (None, None)
+        self.res = f32(ys) if residual else None
+        flags = (pkg.CONV_BIAS if bias else 0) | (pkg.CONV_RESIDUAL if residual else 0) | (pkg.CONV_RELU if relu else 0)
+        self.desc = pkg.ConvDesc(n, c, h, w, o, 3, 3, 2, 2, 1, 1, 1, 1, flags)
+        self.bytes = pkg.conv2d_node_filter_bytes(self.desc, second)
+        z = lambda a, s: dev(a) if a is not None else torch.empty(s, device="cuda")
+        self.args = [dev(self.x), dev(self.w), z(self.b, (o,)), z(self.res, ys), torch.empty(ys, device="cuda"), dev(self.w2), z(self.b2, (o,)),
+                     torch.empty(ys, device="cuda")]
+        A, none = pkg.Buf.arg, pkg.Buf.none()
+        self.plan = pkg.Plan(8)
+        self.plan.add_conv2d_packed(self.desc, A(0), A(1), A(2) if bias else none, A(3) if residual else none, A(4), A(5) if second else none,
+                                    A(6) if second and bias else none, A(7) if second else none, pkg.Buf.ws(0), self.bytes or 256)
+        self.plan.finalize(self.bytes or 256)
+
+    def outputs(self, run):
+        for k in (4, 7):
+            self.args[k].fill_(float("nan"))
+        run()
+        torch.cuda.synchronize()
+        return [host(self.args[4])] + ([host(self.args[7])] if self.second else [])
+
+    def run(self, plan=None, stream=None):
+        return self.outputs(lambda: (plan or self.plan).run(self.args, stream))
+
+    def want(self):
+        y = [_want(self.x, self.w, self.b, self.res, self.relu, 2, 1)]
+        return y + ([_want(self.x, self.w2, self.b2, None, False, 2, 0)] if self.second else [])
+
+    def check(self, got):
+        # sums of 9 c (c) products and a few more terms in float32, against float64
+        c = self.x.shape[1]
+        for y, want, terms in zip(got, self.want(), (9 * c + 16, c + 16)):
+            assert np.isfinite(y).all()
+            assert np.linalg.norm(y - want) <= terms ** 0.5 * 2.0 ** -23 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("xs, o, second, residual, bias, relu", [
+    ((1, 16, 13, 13), 32, True, False, True, True),         # one step of channels, one tile of 49 pixels
+    ((3, 80, 13, 13), 300, True, True, True, True),         # rows of 13, images meet inside a tile, the last block 12 channels
+    ((3, 80, 13, 13), 300, False, True, False, False),
+    ((1, 32, 100, 90), 64, True, False, False, True),       # the widest rows; half of the workgroup's channels absent
+    ((7, 32, 6, 6), 128, True, False, True, False),         # eight images in a tile
+    ((2, 48, 30, 37), 160, False, False, True, True),       # 37 = 9 pieces of four columns and one more
+    ((8, 64, 1, 9), 128, True, False, True, True),          # one row: the rows above and below are padding
+    ((2, 512, 8, 8), 128, True, True, True, True),          # the reduction in eight parts
+    ((16, 64, 56, 56), 128, True, False, True, True),       # a launch that fills the GPU, whole reductions
+])
+def test_conv_on_a_packed_filter(pkg, monkeypatch, xs, o, second, residual, bias, relu):
+    monkeypatch.setenv("KXC_HIP_CONV_BF16X3", "1")
+    node = _Node(pkg, xs, o, second, residual, bias, relu, seed=sum(xs) + o)
+    assert node.bytes > 0 and "bf16x3" in node.plan.node_symbol(0)
+    first = node.run()
+    node.check(first)
+    for a, b in zip(first, node.run()):
+        assert_bit_exact(b, a, "second run")
+    # without scratch the reduction stays in one piece
+    monkeypatch.setenv("KXC_HIP_SCRATCH_MAX", "0")
+    fresh = torch.cuda.Stream()
+    node.check(node.run(stream=fresh.cuda_stream))
+    node.plan.close()
+
+
+def test_conv_on_a_packed_filter_keeps_values_that_are_not_finite(pkg, monkeypatch):
+    """Infinities, NaN and operands next to the largest float reach the outputs that the operator's definition says."""
+    monkeypatch.setenv("KXC_HIP_CONV_BF16X3", "1")
+    node = _Node(pkg, (2, 128, 13, 18), 96, True, relu=False, seed=5)
+    x = node.x
+    x[0, 3, 4, 5] = np.inf
+    x[0, 70, 9, 0] = -np.inf
+    x[1, 127, 12, 17] = np.nan
+    x[1, 0, 0, 0] = 3.4e38
+    node.w[40, 0, 1, 1] = 2.0 ** -20
+    node.w[7, 9, 0, 2] = np.inf
+    node.w2[8, 9, 0, 0] = -np.inf
+    for k, a in ((0, x), (1, node.w), (5, node.w2)):
+        node.args[k].copy_(torch.from_numpy(a))
+    largest = float(np.finfo(np.float32).max)
+    for got, want in zip(node.run(), node.want()):
+        want = np.where(np.abs(want) > largest, np.sign(want) * np.inf, want)
+        assert (np.isnan(got) == np.isnan(want)).all()
+        inf = np.isinf(want)
+        assert (np.isinf(got) == inf).all() and (got[inf] == want[inf]).all()
+        m = np.isfinite(want)
+        assert (np.abs(got[m] - want[m]) <= 1e-5 * np.maximum(np.abs(want[m]), 1.0)).all()
+    node.plan.close()
+
+
+def test_packed_filters_follow_their_weights(pkg, monkeypatch):
+    """Rewritten in place they are read in the next run; frozen, only another pointer or an invalidation counts, for either
+    of the two filters; the plan's text keeps the node; a graph replays it."""
+    monkeypatch.setenv("KXC_HIP_CONV_BF16X3", "1")
+    node = _Node(pkg, (2, 64, 14, 14), 128, True, seed=11)
+    node.check(node.run())
+    scale = lambda k, f: (node.args[k].mul_(f), None)[1]
+    scale(1, 2.0); node.w *= 2
+    scale(5, 0.5); node.w2 *= np.float32(0.5)
+    node.check(node.run())
+    node.plan.freeze_constants(True)
+    frozen = node.run()
+    node.check(frozen)
+    scale(5, 4.0)
+    for a, b in zip(frozen, node.run()):
+        assert_bit_exact(b, a, "frozen")
+    node.w2 *= 4
+    node.plan.invalidate_constants()
+    node.check(node.run())
+    node.w2 = node.w2[::-1].copy()
+    node.args[5] = dev(node.w2)
+    now = node.run()
+    node.check(now)
+    text = node.plan.serialize()
+    assert text.startswith("kxc_hip_plan 5 ")
+    again = pkg.Plan.deserialize(text, 0)
+    assert again.serialize() == text and "bf16x3" in again.node_symbol(0)
+    for a, b in zip(now, node.run(again)):
+        assert_bit_exact(b, a, "from its text")
+    again.close()
+    node.plan.enable_graph(True)
+    stream = torch.cuda.Stream()
+    for replay in range(5):
+        for a, b in zip(now, node.run(stream=stream.cuda_stream)):
+            assert_bit_exact(b, a, "replay %d" % replay)
+        assert torch.isfinite(pkg.conv2d(node.args[0], node.args[1], None, None, 2, 1)).all()
+    node.plan.close()
+    # switched off when the plan is finalized: the node reads its weights as they are
+    monkeypatch.setenv("KXC_HIP_CONV_BF16X3", "0")
+    again = pkg.Plan.deserialize(text, 0)
+    assert "bf16x3" not in again.node_symbol(0)
+    node.check(node.run(again))
+    again.close()
+    assert pkg.conv2d_node_filter_bytes(node.desc, True) == 0
