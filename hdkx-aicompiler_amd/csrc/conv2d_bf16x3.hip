@@ -1,11 +1,13 @@
-// conv2d_bf16x3.hip -- a launch plan's 3x3 stride-2 convolutions, with or without the second (1x1) output, on the bf16 matrix
-// cores: which launches take the kernel of conv_bf16x3.h, and its launch.  The filter is read in packed form, written
-// by the plan's filter launch (conv2d_wino_f32.hip).
+// conv2d_bf16x3.hip -- a launch plan's 3x3 stride-2 convolutions, with or without the second (1x1) output, and its 7x7 stride-2
+// convolution of three-channel images on the bf16 matrix cores: which launches take the kernels of conv_bf16x3.h and
+// conv7_bf16x3.h, and their launch.  The filter is read in packed form, written by the plan's filter launch
+// (conv2d_wino_f32.hip).
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <memory>
 
+#include "conv7_bf16x3.h"
 #include "conv_bf16x3.h"
 
 using namespace kxc_hip;
@@ -15,6 +17,10 @@ namespace {
 struct PackedLaunch {
     conv_bx::Args a;
     void (*kernel)(const conv_bx::Args) = nullptr;
+    conv7_bx::Args a7;                                    // kernel7
+    void (*kernel7)(const conv7_bx::Args) = nullptr;
+    size_t lds_bytes = 0, filter_bytes = 0;
+    double gflop = 0;
     const char* name = "";
     bool second = false;
     size_t scratch_bytes = 0;
@@ -96,8 +102,58 @@ bool Resolve(const kxc_hip_conv2d_desc* d, bool second, PackedLaunch* L) {
     a.div_ohw = MakeFastDiv(a.OHW); a.div_ow = MakeFastDiv(a.OW); a.div_hq = MakeFastDiv(a.Hq); a.div_w4 = MakeFastDiv(a.w4);
     a.div_tiles = MakeFastDiv(a.o_fastest ? a.o_tiles : a.p_tiles); a.div_gsplit = MakeFastDiv(a.gsplit);
     L->second = second;
+    L->filter_bytes = a.u_bytes;
+    L->lds_bytes = kLdsBytes;
+    L->gflop = 2e-9 * a.M * a.O * a.C * Steps(3, second);
     L->kernel = second ? conv_bf16x3_kernel<3, 2, true> : conv_bf16x3_kernel<3, 2, false>;
     L->name = second ? "mfma_k3x3s2_bf16x3_ds" : "mfma_k3x3s2_bf16x3";
+    return true;
+}
+
+// The same for the 7x7 kernel.  LDS for two workgroups (four waves) per compute unit at least.
+bool Resolve7(const kxc_hip_conv2d_desc* d, PackedLaunch* L) {
+    using namespace conv7_bx;
+    if (!d || d->n <= 0 || d->c != kC || d->h <= 0 || d->w <= 0 || d->o <= 0) return false;
+    if (d->kh != kK || d->kw != kK || d->stride_h != 2 || d->stride_w != 2 || d->dil_h != 1 || d->dil_w != 1) return false;
+    if (d->pad_h < 0 || d->pad_w < 0 || d->pad_h >= kK || d->pad_w >= kK || (d->flags & KXC_HIP_CONV_FORCE_DIRECT)) return false;
+    const int64_t Hp = static_cast<int64_t>(d->h) + 2 * d->pad_h, Wp = static_cast<int64_t>(d->w) + 2 * d->pad_w;
+    if (Hp < kK || Wp < kK) return false;
+    const int64_t OH = (Hp - kK) / 2 + 1, OW = (Wp - kK) / 2 + 1;
+    const bool hpool = (d->flags & KXC_HIP_CONV_HPOOL) != 0;
+    const int64_t M = d->n * OH * OW, y_elems = static_cast<int64_t>(d->n) * d->o * OH * (hpool ? OW / 2 : OW);
+    if (4LL * d->n * kC * d->h * d->w >= (1LL << 31) || static_cast<int64_t>(d->n) * d->o * OH * OW >= (1LL << 29) || d->o > (1 << 16)) return false;
+    if ((d->n + 1) * Hp >= (1LL << 30)) return false;
+    if (hpool && (!(d->flags & KXC_HIP_CONV_RELU) || (d->flags & KXC_HIP_CONV_RESIDUAL) || d->o % 8 != 0 || (OW & 1) || kPix % OW != 0 || M % kPix != 0)) return false;
+    Args& a = L->a7;
+    std::memset(&a, 0, sizeof(a));
+    a.N = d->n; a.H = d->h; a.W = d->w; a.O = d->o; a.OH = static_cast<int32_t>(OH); a.OW = static_cast<int32_t>(OW);
+    a.OHW = a.OH * a.OW; a.HW = a.H * a.W; a.M = static_cast<int32_t>(M); a.ph = d->pad_h; a.pw = d->pad_w;
+    a.Hp = static_cast<int32_t>(Hp); a.PW = a.OW / 2;
+    int64_t rows = 0, rem = a.OHW, gcd = kPix;        // (where a tile starts within an image repeats after OHW / gcd(OHW, kPix) tiles)
+    while (rem != 0) { const int64_t r = gcd % rem; gcd = rem; rem = r; }
+    for (int64_t t = 0; t < std::min<int64_t>(CeilDiv(M, kPix), a.OHW / gcd); ++t) {
+        const int64_t m0 = t * kPix, ml = std::min<int64_t>(m0 + kPix, M) - 1;
+        rows = std::max(rows, (ml / a.OHW - m0 / a.OHW) * Hp + 2 * (ml % a.OHW / OW - m0 % a.OHW / OW) + kK);
+    }
+    a.row_max = static_cast<int32_t>(rows);
+    const int pitch = OW + 3 <= 64 ? 64 : 120;      // (the last pixel's window takes four words; three parts within the reach of a ds_read2)
+    if (OW + 3 > pitch || LdsBytes(rows, pitch) > kMaxLdsBytes / 2) return false;
+    a.o_tiles = static_cast<int32_t>(CeilDiv(a.O, kOut));
+    const int64_t units = CeilDiv(M, kPix) * a.o_tiles;
+    if (units >= (1LL << 30)) return false;
+    a.num_units = static_cast<int32_t>(units);
+    a.units_per_xcd = static_cast<int32_t>(CeilDiv(units, 8));
+    a.x_bytes = static_cast<uint32_t>(4LL * d->n * kC * d->h * d->w);
+    a.y_bytes = static_cast<uint32_t>(y_elems * 4);
+    a.u_bytes = static_cast<uint32_t>(FilterBytes(a.O));
+    a.flags = d->flags;
+    a.div_ohw = MakeFastDiv(a.OHW); a.div_ow = MakeFastDiv(a.OW); a.div_hp = MakeFastDiv(a.Hp); a.div_otiles = MakeFastDiv(a.o_tiles);
+    L->filter_bytes = a.u_bytes;
+    L->lds_bytes = std::max(LdsBytes(rows, pitch), kMinLdsBytes);
+    L->gflop = 2e-9 * static_cast<double>(M) * a.O * kC * kK * kK;
+    L->kernel7 = hpool ? (pitch == 64 ? conv7_bf16x3_kernel<64, true> : conv7_bf16x3_kernel<120, true>)
+                       : (pitch == 64 ? conv7_bf16x3_kernel<64, false> : conv7_bf16x3_kernel<120, false>);
+    L->name = "mfma_k7x7s2_bf16x3";
     return true;
 }
 
@@ -107,14 +163,22 @@ bool Resolve(const kxc_hip_conv2d_desc* d, bool second, PackedLaunch* L) {
 // 12.3 and 16.4, batch 4 (0.51) 23.1 and 20.2, batch 8 32.4 and 20.9, batch 32 59 and 36, batch 64 97 and 60; 128 -> 256 at 28 x 28, batch 6
 // (0.77) 20.5 and 22.1, batch 8 (1.03) 25.5 and 23.7, batch 16 39 and 31, batch 64 94 and 54; 256 -> 512 at 14 x 14, batch 8 (1.03)
 // 21.8 and 22.8, batch 12 (1.54) 31 and 25, batch 32 71 and 37, batch 64 104 and 52; 512 -> 512 at 14 x 14, batch 5 (1.28) 21.5 and 22.6; 512 ->
-// 1024 at 28 x 28, batch 2 68 and 36; 16 -> 32 at 56 x 56, batch 20 (0.16) 15.0 and 11.5.  KXC_HIP_CONV_BF16X3=0 keeps the kernels on the fp32 instructions (=1 takes this one
-// wherever it covers the launch), and so does KXC_HIP_CONV_VARIANT, which names one of theirs.
+// 1024 at 28 x 28, batch 2 68 and 36; 16 -> 32 at 56 x 56, batch 20 (0.16) 15.0 and 11.5.  
+// The 7x7 kernel, 3 -> 64 channels: pooled at 224 x 224, batch 16 / 32 / 64 51 / 100 / 169 and 32 / 59 / 108, at 64 x 64, batch 56 (1.1 GFLOP) 33 and
+// 22; not pooled at 224 x 224, batch 4 (0.94) 20.6 and 21.8, batch 8 (1.9) 33 and 30, batch 64 182 and 116; tiles 13 rows high, of which a compute unit holds
+// two, at 193 x 193, batch 16 (2.8) 49 and 54.
+// KXC_HIP_CONV_BF16X3=0 keeps the kernels on the fp32 instructions (=1 takes these wherever they cover the launch), and so
+// does KXC_HIP_CONV_VARIANT, which names one of theirs.
 bool Preferred(const kxc_hip_conv2d_desc* d, bool second, PackedLaunch* L) {
     const char* e = std::getenv("KXC_HIP_CONV_BF16X3");
     const char* variant = std::getenv("KXC_HIP_CONV_VARIANT");
-    if ((e && e[0] == '0') || (variant && *variant) || !Resolve(d, second, L)) return false;
-    const double gflop = 2e-9 * L->a.M * L->a.O * L->a.C * conv_bx::Steps(3, second) * SelectLanes();
-    return (e && e[0] == '1') || gflop >= std::min(0.12 * L->a.csteps, 1.4);
+    if ((e && e[0] == '0') || (variant && *variant)) return false;
+    if (!second && Resolve7(d, L)) {
+        // Pooled rows: always.  Others: four workgroups to a compute unit (tiles that are few rows high) and work for them.
+        const bool pooled = (d->flags & KXC_HIP_CONV_HPOOL) != 0;
+        return (e && e[0] == '1') || pooled || (L->lds_bytes <= kMaxLdsBytes / 4 && L->gflop * SelectLanes() >= 1.8);
+    }
+    return Resolve(d, second, L) && ((e && e[0] == '1') || L->gflop * SelectLanes() >= std::min(0.12 * L->a.csteps, 1.4));
 }
 
 }  // namespace
@@ -127,12 +191,12 @@ struct PreparedPacked {
 
 size_t PackedFilterBytes(const kxc_hip_conv2d_desc* desc, bool second) {
     PackedLaunch L;
-    return Preferred(desc, second, &L) ? L.a.u_bytes : 0;
+    return Preferred(desc, second, &L) ? L.filter_bytes : 0;
 }
 
 void PreparePacked(const kxc_hip_conv2d_desc* desc, bool second, size_t u_bytes, PreparedPacked** out) {
     std::unique_ptr<PreparedPacked> p(new PreparedPacked);
-    *out = Preferred(desc, second, &p->launch) && u_bytes >= p->launch.a.u_bytes ? p.release() : nullptr;
+    *out = Preferred(desc, second, &p->launch) && u_bytes >= p->launch.filter_bytes ? p.release() : nullptr;
 }
 
 const char* PreparedPackedName(const PreparedPacked* p) { return p->launch.name; }
@@ -141,10 +205,20 @@ void FreePreparedPacked(PreparedPacked* p) { delete p; }
 int32_t LaunchPreparedPacked(const PreparedPacked* p, const float* x, const float* w, const void* u, const float* bias, const float* residual,
                              float* y, const float* w2, const float* bias2, float* y2, hipStream_t s) {
     const PackedLaunch& L = p->launch;
-    conv_bx::Args a = L.a;
+    const uint32_t flags = L.kernel7 ? L.a7.flags : L.a.flags;
     KXC_HIP_REQUIRE(x && w && u && y && (!L.second || (w2 && y2)), "%s: NULL pointer", L.name);
-    KXC_HIP_REQUIRE(!(a.flags & KXC_HIP_CONV_BIAS) || bias, "%s: bias flag without bias", L.name);
-    KXC_HIP_REQUIRE(!(a.flags & KXC_HIP_CONV_RESIDUAL) || residual, "%s: residual flag without residual", L.name);
+    KXC_HIP_REQUIRE(!(flags & KXC_HIP_CONV_BIAS) || bias, "%s: bias flag without bias", L.name);
+    KXC_HIP_REQUIRE(!(flags & KXC_HIP_CONV_RESIDUAL) || residual, "%s: residual flag without residual", L.name);
+    if (L.kernel7) {
+        conv7_bx::Args b = L.a7;
+        b.x = x; b.w = w; b.u = static_cast<const char*>(u); b.bias = bias; b.res = residual; b.y = y;
+        if (L.lds_bytes > 64 * 1024)
+            if (int32_t rc = GrantLds(reinterpret_cast<const void*>(L.kernel7))) return rc;
+        hipLaunchKernelGGL(L.kernel7, NoteGrid(dim3(static_cast<unsigned>(b.units_per_xcd * 8))), NoteBlock(dim3(conv7_bx::kThreads)),
+                           NoteLds(L.lds_bytes), s, b);
+        return CheckLaunch(L.name);
+    }
+    conv_bx::Args a = L.a;
     a.x = x; a.w = w; a.u = static_cast<const char*>(u); a.bias = bias; a.res = residual; a.y = y;
     a.w2 = w2; a.bias2 = bias2; a.y2 = y2;
     SplitScratchLease lease;      // held until the adding kernel is enqueued
@@ -161,7 +235,7 @@ int32_t LaunchPreparedPacked(const PreparedPacked* p, const float* x, const floa
     }
     if (int32_t rc = GrantLds(reinterpret_cast<const void*>(L.kernel))) return rc;
     hipLaunchKernelGGL(L.kernel, NoteGrid(dim3(static_cast<unsigned>(a.units_per_xcd * 8))), NoteBlock(dim3(conv_bx::kThreads)),
-                       NoteLds(conv_bx::kLdsBytes), s, a);
+                       NoteLds(L.lds_bytes), s, a);
     if (int32_t rc = CheckLaunch(L.name)) return rc;
     if (a.gsplit == 1) return KXC_HIP_OK;
     SplitReduceArgs r;

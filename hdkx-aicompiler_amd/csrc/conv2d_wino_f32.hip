@@ -90,6 +90,7 @@ __device__ __forceinline__ float relu_sel(float v) { return __builtin_fmaxf(v, 0
 }  // namespace
 
 #include "wino_bf16x3.h"
+#include "conv7_bf16x3.h"
 #include "conv_bf16x3.h"
 
 namespace {
@@ -147,7 +148,7 @@ inline int64_t WeightTiles(int64_t o_padded, int64_t C) { return (o_padded / 32)
 // The filter transforms of several layers in one launch (a launch plan transforms all its Winograd layers' weights
 // at the start of a run): block b belongs to the job whose [first_block, next first_block) range holds it.
 // A job is one form of one tensor: fp32 (wino_kernel) or three-part bf16 (wino_bf16x3_kernel), or a filter that is not
-// transformed, with the second output's (conv_bf16x3_kernel).
+// transformed (conv_bf16x3_kernel, with the second output's; conv7_bf16x3_kernel).
 constexpr int kMaxWeightJobs = 32;
 struct WinoWeightBatch {
     const float* w[kMaxWeightJobs];
@@ -155,7 +156,7 @@ struct WinoWeightBatch {
     int32_t O[kMaxWeightJobs], C[kMaxWeightJobs], first_block[kMaxWeightJobs + 1];
     const float* w2[kMaxWeightJobs];
     uint32_t three_part;       // bit j: job j writes the three-part form
-    uint32_t packed;           // bit j: job j writes the filter of conv_bf16x3.h
+    uint32_t packed, packed7;  // ... the filter of conv_bf16x3.h, of conv7_bf16x3.h
     int32_t count;
 };
 __global__ void __launch_bounds__(256) wino_weight_batch_kernel(const WinoWeightBatch b) {
@@ -163,7 +164,8 @@ __global__ void __launch_bounds__(256) wino_weight_batch_kernel(const WinoWeight
     int j = 0;
     while (j + 1 < b.count && static_cast<int32_t>(blockIdx.x) >= b.first_block[j + 1]) ++j;
     const int tile = static_cast<int>(blockIdx.x) - b.first_block[j];
-    if ((b.packed >> j) & 1u) conv_bx::pack_tile(b.w[j], b.w2[j], b.u[j], b.O[j], b.C[j], tile, raw);
+    if ((b.packed7 >> j) & 1u) conv7_bx::pack_tile(b.w[j], b.u[j], b.O[j], tile);
+    else if ((b.packed >> j) & 1u) conv_bx::pack_tile(b.w[j], b.w2[j], b.u[j], b.O[j], b.C[j], tile, raw);
     else if ((b.three_part >> j) & 1u) wino_bx::weight_tile(b.w[j], b.u[j], b.O[j], b.C[j], tile, raw);
     else wino_weight_tile(b.w[j], reinterpret_cast<float*>(b.u[j]), b.O[j], b.C[j], tile, raw);
 }
@@ -1020,10 +1022,11 @@ int32_t LaunchWinogradWeightTransforms(const WinoWeightJob* jobs, int32_t count,
             b.O[b.count] = static_cast<int32_t>(O); b.C[b.count] = static_cast<int32_t>(C);
             b.first_block[b.count] = static_cast<int32_t>(blocks);
             if (three) b.three_part |= 1u << b.count;
-            if (form == kFormPacked) b.packed |= 1u << b.count;
+            const bool seven = form == kFormPacked && job.desc->kh == conv7_bx::kK;
+            if (form == kFormPacked) (seven ? b.packed7 : b.packed) |= 1u << b.count;
             b.w2[b.count] = job.w2;
             ++b.count;
-            blocks += form != kWinoFormF32 ? wino_bx::WeightTiles(O, C) : WeightTiles(CeilDiv(O, 32) * 32, C);
+            blocks += seven ? CeilDiv(O, 32) : form != kWinoFormF32 ? wino_bx::WeightTiles(O, C) : WeightTiles(CeilDiv(O, 32) * 32, C);
             KXC_HIP_REQUIRE(blocks < kMaxGridX, "winograd weight transform: too many blocks");
         }
     }

@@ -97,6 +97,23 @@ bool Conv2DPoolQuery(const Attrs& attrs, const Array<Type>& inputs, bool fused_r
     return kxc_hip_conv2d_hpool_preferred(&d) != 0;
 }
 
+// Constant weights: the packed copy that the library's kernel for the shape reads, if it has one, gets a workspace region of
+// its own.  "" otherwise: nothing was added.
+std::string AddPackedConv2D(const HIPDispatchContext& c, kxc_hip_plan* plan, const kxc_hip_conv2d_desc& d, const HIPBuffer& output, const kxc_hip_buf& residual) {
+    auto constant = [](const std::vector<bool>& v) { return v.size() > 1 && v[1]; };
+    if (!c.alloc_persistent || !constant(c.input_constant) || (c.has_pair && !constant(c.pair_input_constant))) return "";
+    size_t u_bytes = 0;
+    Check(kxc_hip_conv2d_node_filter_bytes(&d, c.has_pair ? 1 : 0, &u_bytes), "nn_conv2d dispatch");
+    if (u_bytes == 0) return "";
+    const kxc_hip_buf none{KXC_HIP_BUF_NONE, 0};
+    const HIPBuffer u = c.alloc_persistent(static_cast<int64_t>(u_bytes));
+    Check(kxc_hip_plan_add_conv2d_packed(plan, &d, B(c.inputs[0]), B(c.inputs[1]), c.inputs.size() == 3 ? B(c.inputs[2]) : none, residual, B(output),
+                                         c.has_pair ? B(c.pair_inputs[1]) : none, c.has_pair && c.pair_inputs.size() == 3 ? B(c.pair_inputs[2]) : none,
+                                         c.has_pair ? B(c.pair_output) : none, B(u), u_bytes),
+          "nn_conv2d dispatch");
+    return kxc_hip_plan_node_symbol(plan, kxc_hip_plan_num_nodes(plan) - 1);
+}
+
 std::string Conv2DDispatch(const HIPDispatchContext& c, kxc_hip_plan* plan) {
     kxc_hip_conv2d_desc d{};
     if (!ConvDesc(c.attrs, c.input_types, &d) || !IsF32(c.out_type)) return "";
@@ -111,29 +128,22 @@ std::string Conv2DDispatch(const HIPDispatchContext& c, kxc_hip_plan* plan) {
         const int64_t oh = (d.h + 2 * d.pad_h - (d.dil_h * (d.kh - 1) + 1)) / d.stride_h + 1;
         const int64_t ow = (d.w + 2 * d.pad_w - (d.dil_w * (d.kw - 1) + 1)) / d.stride_w + 1;
         const HIPBuffer half = c.alloc_temp(static_cast<int64_t>(d.n) * d.o * oh * (ow / 2) * 4);
-        Check(kxc_hip_plan_add_conv2d(plan, &d, B(c.inputs[0]), B(c.inputs[1]), has_bias ? B(c.inputs[2]) : none, none, B(half)),
-              "nn_conv2d dispatch");
+        const std::string packed = AddPackedConv2D(c, plan, d, half, none);
+        if (packed.empty())
+            Check(kxc_hip_plan_add_conv2d(plan, &d, B(c.inputs[0]), B(c.inputs[1]), has_bias ? B(c.inputs[2]) : none, none, B(half)),
+                  "nn_conv2d dispatch");
         kxc_hip_pool2d_desc q{};
         q.n = d.n; q.c = d.o; q.h = static_cast<int32_t>(oh); q.w = static_cast<int32_t>(ow / 2);
         q.kh = 3; q.kw = 1; q.stride_h = 2; q.stride_w = 1;
         q.pad_top = 1; q.pad_bottom = 1;
         Check(kxc_hip_plan_add_pool2d(plan, &q, B(half), B(c.output)), "nn_conv2d dispatch (column pool)");
+        if (!packed.empty()) return packed;
         return std::string("kxc_conv2d_nchw_f32.") + kxc_hip_conv2d_node_variant(&d) + (has_bias ? "+bias" : "") + "+relu+maxpool3w";
     }
     if (c.has_pair) {
         const bool bias2 = c.pair_inputs.size() == 3;
-        // constant weights: the packed copy that the library's kernel for the shape reads, if it has one, gets a workspace region
-        size_t u_bytes = 0;
-        if (c.alloc_persistent && c.input_constant.size() > 1 && c.input_constant[1] && c.pair_input_constant.size() > 1 && c.pair_input_constant[1])
-            Check(kxc_hip_conv2d_node_filter_bytes(&d, 1, &u_bytes), "nn_conv2d pair dispatch");
-        if (u_bytes > 0) {
-            const HIPBuffer u = c.alloc_persistent(static_cast<int64_t>(u_bytes));
-            Check(kxc_hip_plan_add_conv2d_packed(plan, &d, B(c.inputs[0]), B(c.inputs[1]), has_bias ? B(c.inputs[2]) : none,
-                                                 c.has_residual ? B(c.residual) : none, B(c.output), B(c.pair_inputs[1]),
-                                                 bias2 ? B(c.pair_inputs[2]) : none, B(c.pair_output), B(u), u_bytes),
-                  "nn_conv2d pair dispatch");
-            return kxc_hip_plan_node_symbol(plan, kxc_hip_plan_num_nodes(plan) - 1);
-        }
+        const std::string packed = AddPackedConv2D(c, plan, d, c.output, c.has_residual ? B(c.residual) : none);
+        if (!packed.empty()) return packed;
         Check(kxc_hip_plan_add_conv2d_pair(plan, &d, B(c.inputs[0]), B(c.inputs[1]), has_bias ? B(c.inputs[2]) : none,
                                            c.has_residual ? B(c.residual) : none, B(c.output), B(c.pair_inputs[1]),
                                            bias2 ? B(c.pair_inputs[2]) : none, B(c.pair_output)),
@@ -154,17 +164,8 @@ std::string Conv2DDispatch(const HIPDispatchContext& c, kxc_hip_plan* plan) {
         return std::string("kxc_conv2d_nchw_f32.") + kxc_hip_conv2d_winograd_variant(&d) + (has_bias ? "+bias" : "") +
                (c.has_residual ? "+add" : "") + (c.fused_relu ? "+relu" : "");
     }
-    if (c.alloc_persistent && c.input_constant.size() > 1 && c.input_constant[1]) {
-        size_t u_bytes = 0;
-        Check(kxc_hip_conv2d_node_filter_bytes(&d, 0, &u_bytes), "nn_conv2d dispatch");
-        if (u_bytes > 0) {
-            const HIPBuffer u = c.alloc_persistent(static_cast<int64_t>(u_bytes));
-            Check(kxc_hip_plan_add_conv2d_packed(plan, &d, B(c.inputs[0]), B(c.inputs[1]), has_bias ? B(c.inputs[2]) : none,
-                                                 c.has_residual ? B(c.residual) : none, B(c.output), none, none, none, B(u), u_bytes),
-                  "nn_conv2d dispatch");
-            return kxc_hip_plan_node_symbol(plan, kxc_hip_plan_num_nodes(plan) - 1);
-        }
-    }
+    const std::string packed = AddPackedConv2D(c, plan, d, c.output, c.has_residual ? B(c.residual) : none);
+    if (!packed.empty()) return packed;
     Check(kxc_hip_plan_add_conv2d(plan, &d, B(c.inputs[0]), B(c.inputs[1]), has_bias ? B(c.inputs[2]) : none,
                                   c.has_residual ? B(c.residual) : none, B(c.output)),
           "nn_conv2d dispatch");

@@ -1,5 +1,6 @@
-"""Plan nodes on a packed filter (kxc_hip_plan_add_conv2d_packed): the three-part kernel for 3x3 stride-2 convolutions, with
-and without the second output, at the edges of its tiles, against float64; its values that are not finite; its filters."""
+"""Plan nodes on a packed filter (kxc_hip_plan_add_conv2d_packed): the three-part kernels for 3x3 stride-2 convolutions, with
+and without the second output, and for 7x7 stride-2 convolutions of three channels, with and without the column maxima, at the
+edges of their tiles, against float64; their values that are not finite; their filters."""
 import numpy as np
 import pytest
 import torch
@@ -20,17 +21,19 @@ def _want(x, w, bias, residual, relu, stride, pad):
 class _Node:
     """One packed convolution with its operands on the GPU; `run` returns its outputs."""
 
-    def __init__(self, pkg, xs, o, second, residual=False, bias=True, relu=True, seed=0):
+    def __init__(self, pkg, xs, o, second, residual=False, bias=True, relu=True, seed=0, k=3, pad=1, hpool=False):
         rng = np.random.default_rng(seed)
         n, c, h, w = xs
         f32 = lambda s, k=1.0: (rng.standard_normal(s) * k).astype(np.float32)
-        self.pkg, self.second, self.relu = pkg, second, relu
-        ys = (n, o, (h + 1) // 2, (w + 1) // 2)
-        self.x, self.w, self.w2 = f32(xs), f32((o, c, 3, 3), (2 / (9 * c)) ** 0.5), f32((o, c, 1, 1), (2 / c) ** 0.5)
+        self.pkg, self.second, self.relu, self.k, self.pad, self.hpool = pkg, second, relu, k, pad, hpool
+        ys = (n, o, (h + 2 * pad - k) // 2 + 1, (w + 2 * pad - k) // 2 + 1)
+        if hpool:
+            ys = ys[:3] + (ys[3] // 2,)
+        self.x, self.w, self.w2 = f32(xs), f32((o, c, k, k), (2 / (k * k * c)) ** 0.5), f32((o, c, 1, 1), (2 / c) ** 0.5)
         self.b, self.b2 = (f32((o,)), f32((o,))) if bias else (None, None)
         self.res = f32(ys) if residual else None
-        flags = (pkg.CONV_BIAS if bias else 0) | (pkg.CONV_RESIDUAL if residual else 0) | (pkg.CONV_RELU if relu else 0)
-        self.desc = pkg.ConvDesc(n, c, h, w, o, 3, 3, 2, 2, 1, 1, 1, 1, flags)
+        flags = (pkg.CONV_BIAS if bias else 0) | (pkg.CONV_RESIDUAL if residual else 0) | (pkg.CONV_RELU if relu else 0) | (pkg.CONV_HPOOL if hpool else 0)
+        self.desc = pkg.ConvDesc(n, c, h, w, o, k, k, 2, 2, pad, pad, 1, 1, flags)
         self.bytes = pkg.conv2d_node_filter_bytes(self.desc, second)
         z = lambda a, s: dev(a) if a is not None else torch.empty(s, device="cuda")
         self.args = [dev(self.x), dev(self.w), z(self.b, (o,)), z(self.res, ys), torch.empty(ys, device="cuda"), dev(self.w2), z(self.b2, (o,)),
@@ -52,13 +55,16 @@ class _Node:
         return self.outputs(lambda: (plan or self.plan).run(self.args, stream))
 
     def want(self):
-        y = [_want(self.x, self.w, self.b, self.res, self.relu, 2, 1)]
+        y = [_want(self.x, self.w, self.b, self.res, self.relu, 2, self.pad)]
+        if self.hpool:
+            left = np.concatenate([y[0][..., :1], y[0][..., 1:-1:2]], axis=-1)
+            y = [np.maximum(np.maximum(left, y[0][..., ::2]), y[0][..., 1::2])]
         return y + ([_want(self.x, self.w2, self.b2, None, False, 2, 0)] if self.second else [])
 
     def check(self, got):
-        # sums of 9 c (c) products and a few more terms in float32, against float64
+        # sums of k k c (c) products and a few more terms in float32, against float64
         c = self.x.shape[1]
-        for y, want, terms in zip(got, self.want(), (9 * c + 16, c + 16)):
+        for y, want, terms in zip(got, self.want(), (self.k * self.k * c + 16, c + 16)):
             assert np.isfinite(y).all()
             assert np.linalg.norm(y - want) <= terms ** 0.5 * 2.0 ** -23 * np.linalg.norm(want)
 
@@ -89,23 +95,54 @@ def test_conv_on_a_packed_filter(pkg, monkeypatch, xs, o, second, residual, bias
     node.plan.close()
 
 
-def test_conv_on_a_packed_filter_keeps_values_that_are_not_finite(pkg, monkeypatch):
+@pytest.mark.parametrize("xs, o, pad, residual, bias, relu, hpool", [
+    ((1, 3, 224, 224), 64, 3, False, True, True, True),     # two rows of 112 columns a tile
+    ((7, 3, 64, 64), 40, 3, False, True, True, True),       # seven rows of 32; the second block of channels ends after 8
+    ((7, 3, 32, 56), 8, 3, False, False, True, True),       # eight rows of 28, one block of channels
+    ((3, 3, 224, 224), 96, 3, False, True, True, False),
+    ((2, 3, 33, 61), 20, 3, True, True, False, False),      # odd maps, channels and pixels short of a block
+    ((1, 3, 7, 9), 64, 0, False, False, True, False),       # two outputs a channel
+    ((5, 3, 40, 231), 33, 1, True, True, True, False),      # 114 columns: the last word of the widest rows
+    ((9, 3, 16, 123), 64, 2, False, True, True, False),     # 61: the widest of the narrow rows
+])
+def test_first_layer_on_a_packed_filter(pkg, monkeypatch, xs, o, pad, residual, bias, relu, hpool):
+    monkeypatch.setenv("KXC_HIP_CONV_BF16X3", "1")
+    node = _Node(pkg, xs, o, False, residual, bias, relu, seed=sum(xs) + o, k=7, pad=pad, hpool=hpool)
+    assert node.bytes > 0 and "k7x7s2_bf16x3" in node.plan.node_symbol(0)
+    first = node.run()
+    node.check(first)
+    assert_bit_exact(node.run()[0], first[0], "second run")
+    again = pkg.Plan.deserialize(node.plan.serialize(), 0)
+    assert_bit_exact(node.run(again)[0], first[0], "from its text")
+    again.close()
+    node.plan.close()
+
+
+@pytest.mark.parametrize("xs, o, second, k, hpool", [((2, 128, 13, 18), 96, True, 3, False), ((2, 3, 45, 50), 96, False, 7, False),
+                                                     ((7, 3, 64, 64), 96, False, 7, True)])
+def test_conv_on_a_packed_filter_keeps_values_that_are_not_finite(pkg, monkeypatch, xs, o, second, k, hpool):
     """Infinities, NaN and operands next to the largest float reach the outputs that the operator's definition says."""
     monkeypatch.setenv("KXC_HIP_CONV_BF16X3", "1")
-    node = _Node(pkg, (2, 128, 13, 18), 96, True, relu=False, seed=5)
-    x = node.x
-    x[0, 3, 4, 5] = np.inf
-    x[0, 70, 9, 0] = -np.inf
-    x[1, 127, 12, 17] = np.nan
+    node = _Node(pkg, xs, o, second, relu=hpool, seed=5, k=k, pad=k // 2, hpool=hpool)
+    x, (n, c, h, w) = node.x, xs
+    x[0, c // 2, 4, 5] = np.inf
+    x[0, c // 3, 9, 0] = -np.inf
+    x[1, c - 1, h - 1, w - 1] = np.nan
     x[1, 0, 0, 0] = 3.4e38
-    node.w[40, 0, 1, 1] = 2.0 ** -20
-    node.w[7, 9, 0, 2] = np.inf
-    node.w2[8, 9, 0, 0] = -np.inf
-    for k, a in ((0, x), (1, node.w), (5, node.w2)):
-        node.args[k].copy_(torch.from_numpy(a))
+    node.w[40, 0, k // 2, k // 2] = 2.0 ** -20
+    node.w[7, c // 2, 0, 2] = np.inf
+    node.w2[8, c // 2, 0, 0] = -np.inf
+    for i, a in ((0, x), (1, node.w), (5, node.w2)):
+        node.args[i].copy_(torch.from_numpy(a))
     largest = float(np.finfo(np.float32).max)
-    for got, want in zip(node.run(), node.want()):
-        want = np.where(np.abs(want) > largest, np.sign(want) * np.inf, want)
+    finite = lambda a: np.where(np.abs(a) > largest, np.sign(a) * np.inf, a)
+    if hpool:      # relu(NaN) is 0 in the operator's definition; numpy's maximum would keep it
+        y = finite(_want(node.x, node.w, node.b, None, False, 2, k // 2))
+        y = np.where(y > 0, y, 0.0)
+        wants = [np.maximum(np.maximum(np.concatenate([y[..., :1], y[..., 1:-1:2]], axis=-1), y[..., ::2]), y[..., 1::2])]
+    else:
+        wants = [finite(y) for y in node.want()]
+    for got, want in zip(node.run(), wants):
         assert (np.isnan(got) == np.isnan(want)).all()
         inf = np.isinf(want)
         assert (np.isinf(got) == inf).all() and (got[inf] == want[inf]).all()
