@@ -12,6 +12,9 @@
 //   X  XI = 0: straight from memory, one 4-byte load per matrix instruction (16 neighbouring pixels of four channels), E ahead; a
 //      buffer offset per filter tap, out of range at the zero padding, the channel in the scalar offset.  The address unit
 //      takes 16 cycles an instruction for a whole compute unit, which bounds this form once four waves are at it.
+//      ROWS: one 12-byte load for the three values of a filter row, 12 loads a chunk instead of 36 (us, with a wave's last chunk
+//      requesting nothing behind it: 64 channels at 56 x 56 7.9 -> 7.1, 64 -> 128 with stride 2 and the second output 8.8 -> 6.1, 128 ->
+//      256 7.2 -> 5.4, at batch 3 11.1 -> 8.2).
 //      XI > 0: the whole input rows that a tile touches, one contiguous run per channel, in XI loads of 1 KiB staged like W
 //      (tiles then never cross images); a chunk's operands move into registers at its start.  Fewer loads but more
 //      instructions: better for narrow maps, where few rows hold a tile and few tiles hide nothing.
@@ -48,6 +51,7 @@ struct Args {
 #if defined(__HIPCC__)
 
 typedef float f4 __attribute__((ext_vector_type(4)));
+typedef float f3 __attribute__((ext_vector_type(3)));
 typedef __attribute__((address_space(3))) void* lds_p;
 constexpr uint32_t kOutside = 0x80000000u;
 
@@ -60,7 +64,9 @@ __device__ __forceinline__ void to_lds16(__amdgpu_buffer_rsrc_t rs, char* lds, u
 #endif
 }
 
-template <int KH, int KW, int CPG, int XI, int RO, int KS, bool DS = false>
+// ROWS (XI = 0, 3x3 filters without dilation along a row, one column of padding at most, rows of three values at least): the three
+// values that a filter row touches by one 12-byte load, moved to the row's end where it would reach across it.
+template <int KH, int KW, int CPG, int XI, int RO, int KS, bool DS = false, bool ROWS = false>
 __global__ void __launch_bounds__(64 * KS) __attribute__((amdgpu_waves_per_eu(2))) conv_small_kernel(const Args a) {
     constexpr bool STAGED = XI > 0;
     constexpr int KHW = KH * KW, E = CPG * KHW, WI = RO * E / 4, NB = DS ? 2 * RO : RO;
@@ -208,37 +214,60 @@ __global__ void __launch_bounds__(64 * KS) __attribute__((amdgpu_waves_per_eu(2)
         }
     } else {
         const __amdgpu_buffer_rsrc_t xr = rsrc(a.x, a.x_bytes);
-        uint32_t xo[KHW];
+        static_assert(!ROWS || KW == 3, "rows of three");
+        constexpr int PER = ROWS ? 3 : 1, XL = E / PER;            // values per load; loads of a chunk
+        uint32_t xo[KHW / PER];
+        const int xs = ROWS ? min(max(iw, 0), a.W - 3) : iw, shift = iw - xs;       // (-1, 0, 1)
+        const bool first = iw >= 0, last = iw + 2 < a.W;
 #pragma unroll
-        for (int t = 0; t < KHW; ++t)
-            xo[t] = valid(t) ? static_cast<uint32_t>(n * a.C + g * CPG) * plane + static_cast<uint32_t>((ih + t / KW * a.dh) * a.W + iw + t % KW * a.dw) * 4u : kOutside;
+        for (int t = 0; t < KHW / PER; ++t) {
+            const int y = ih + t * PER / KW * a.dh;
+            const bool there = ROWS ? in && static_cast<uint32_t>(y) < static_cast<uint32_t>(a.H) : valid(t);
+            xo[t] = there ? static_cast<uint32_t>(n * a.C + g * CPG) * plane + static_cast<uint32_t>(y * a.W + (ROWS ? xs : iw + t % KW * a.dw)) * 4u : kOutside;
+        }
         float xf[E];
         auto load_x = [&](int chunk, int j) __attribute__((always_inline)) {
-            xf[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xr, xo[j % KHW], static_cast<uint32_t>(chunk * 4 * CPG + j / KHW) * plane, 0));
+            const uint32_t so = static_cast<uint32_t>(chunk * 4 * CPG + j * PER / KHW) * plane;
+            if constexpr (ROWS) {
+                const f3 v = __builtin_bit_cast(f3, __builtin_amdgcn_raw_buffer_load_b96(xr, xo[j % (KHW / PER)], so, 0));
+#pragma unroll
+                for (int e = 0; e < 3; ++e) xf[3 * j + e] = v[e];
+            } else {
+                xf[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xr, xo[j % KHW], so, 0));
+            }
         };
         if (wave < a.nchunks) {
 #pragma unroll
-            for (int j = 0; j < E; ++j) {
+            for (int j = 0; j < XL; ++j) {
                 load_x(wave, j);
                 __builtin_amdgcn_sched_barrier(0);                 // in this order: the waits of the loop count on it
             }
-            for (int chunk = wave; chunk < a.nchunks; chunk += KS) {
-                const int next = min(chunk + KS, a.nchunks - 1);   // (the loads past the wave's last chunk are not used)
-                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(E) : "memory");      // all but the E loads of X behind the weights
+            // (a wave's last chunk requests nothing: with one or two chunks per wave a chunk more would be a third to half of all loads)
+            auto step = [&](int chunk, auto more) __attribute__((always_inline)) {
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(XL) : "memory");     // all but the loads of X behind the weights
                 load_w2(chunk);
                 read_w();
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // read before they are written again
                 __builtin_amdgcn_sched_barrier(0);
-                load_w(next);
+                if constexpr (decltype(more)::value) load_w(chunk + KS);
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int j = 0; j < E; ++j) {
-                    multiply(j, xf[j]);
-                    load_x(next, j);
+                for (int j = 0; j < XL; ++j) {
+                    if constexpr (ROWS) {
+                        const float v0 = xf[3 * j], v1 = xf[3 * j + 1], v2 = xf[3 * j + 2];
+                        multiply(3 * j, first ? (shift > 0 ? v1 : v0) : 0.0f);
+                        multiply(3 * j + 1, shift == 0 ? v1 : shift > 0 ? v2 : v0);
+                        multiply(3 * j + 2, last ? (shift < 0 ? v1 : v2) : 0.0f);
+                    } else {
+                        multiply(j, xf[j]);
+                    }
+                    if constexpr (decltype(more)::value) load_x(chunk + KS, j);
                     __builtin_amdgcn_sched_barrier(0);
                 }
-            }
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // (nothing may still be on its way into LDS)
+            };
+            int chunk = wave;
+            for (; chunk + KS < a.nchunks; chunk += KS) step(chunk, std::true_type{});
+            step(chunk, std::false_type{});
         }
     }
     __syncthreads();
