@@ -1,7 +1,7 @@
-// conv2d_bf16x3.hip -- a launch plan's 3x3 stride-2 convolutions, with or without the second (1x1) output, and its 7x7 stride-2
-// convolution of three-channel images on the bf16 matrix cores: which launches take the kernels of conv_bf16x3.h and
-// conv7_bf16x3.h, and their launch.  The filter is read in packed form, written by the plan's filter launch
-// (conv2d_wino_f32.hip).
+// conv2d_bf16x3.hip -- a launch plan's 3x3 stride-2 convolutions, with or without the second (1x1) output, its 7x7 stride-2
+// convolution of three-channel images, and large single calls of 1x1 to 7x7 filters on the bf16 matrix cores: which launches take
+// the kernels of conv_bf16x3.h and conv7_bf16x3.h, and their launch.  The filter is read in packed form, written by the
+// plan's filter launch (conv2d_wino_f32.hip) or by the call.
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
@@ -17,6 +17,7 @@ namespace {
 struct PackedLaunch {
     conv_bx::Args a;
     void (*kernel)(const conv_bx::Args) = nullptr;
+    void (*pack)(const float*, char*, int32_t, int32_t) = nullptr;
     conv7_bx::Args a7;                                    // kernel7
     void (*kernel7)(const conv7_bx::Args) = nullptr;
     size_t lds_bytes = 0, filter_bytes = 0;
@@ -42,48 +43,76 @@ int64_t MaxRows(const conv_bx::Args& a, int extra) {
 }
 
 // Parts of a reduction, while all of them together are at most one workgroup per compute unit: what gives the shortest of
-// 2.9 us per step of 16 channels + the adding launch (5 us and the parts' way to memory and back at 4.5 TB/s).  us, 1 / 2 / 4 / 8
+// 0.29 us per tap and 16 channels + the adding launch (5 us and the parts' way to memory and back at 4.5 TB/s).  us, 1 / 2 / 4 / 8
 // parts without the adding launch: 64 -> 128 channels at 49 x 49, batch 6 (59 workgroups) 19.9 / 14.8 / 12.9; 128 -> 256 at 25 x
 // 25, batch 5 (28) 24.7 / 17.0 / 13.4 / 12.2; 256 -> 512 at 14 x 14, batch 32 (100) 47.5 / 30.8 / 34.2 / 41.9, batch 64 (196)
 // 54.1 / 57.3 / 66.3; with it 64 -> 128 at 56 x 56, batch 8 (98) 22 and 28.
-int Split(int64_t units, int csteps, int64_t out_bytes) {
+int Split(int64_t units, int csteps, int steps, int64_t out_bytes) {
     int best = 1;
-    double best_us = 2.9 * csteps;
+    const double step_us = 0.29 * steps;
+    double best_us = step_us * csteps;
     for (int s = 2; s <= 8 && units * s <= 256 && s <= csteps && out_bytes * s <= (16LL << 20); s *= 2) {
-        const double us = 2.9 * static_cast<double>(CeilDiv(csteps, s)) + 5 + 2.0 * s * static_cast<double>(out_bytes) / 4.5e6;
+        const double us = step_us * static_cast<double>(CeilDiv(csteps, s)) + 5 + 2.0 * s * static_cast<double>(out_bytes) / 4.5e6;
         if (us < best_us) { best_us = us; best = s; }
     }
     return best;
 }
 
+struct FilterKernels {
+    int k, s;
+    void (*conv)(const conv_bx::Args);
+    void (*pack)(const float*, char*, int32_t, int32_t);
+    const char* name;
+};
+template <int K, int S>
+__global__ void __launch_bounds__(256) pack_filter_kernel(const float* w, char* u, int32_t O, int32_t C) {
+    __shared__ float raw[conv_bx::PackFloats(K)];
+    conv_bx::pack_block<K, S>(w, nullptr, u, O, C, static_cast<int>(blockIdx.x), raw);
+}
+#define KXC_PACKED(K, S) {K, S, conv_bx::conv_bf16x3_kernel<K, S, false>, pack_filter_kernel<K, S>, "mfma_k" #K "x" #K "s" #S "_bf16x3"}
+const FilterKernels kFilters[] = {KXC_PACKED(1, 1), KXC_PACKED(1, 2), KXC_PACKED(3, 1), KXC_PACKED(3, 2), KXC_PACKED(5, 1), KXC_PACKED(5, 2), KXC_PACKED(7, 1), KXC_PACKED(7, 2)};
+
 // Whether the kernel covers a launch (`L` is filled if so).
 bool Resolve(const kxc_hip_conv2d_desc* d, bool second, PackedLaunch* L) {
     using namespace conv_bx;
-    if (!d || d->n <= 0 || d->c <= 0 || d->h <= 0 || d->w <= 0 || d->o <= 0) return false;
-    if (d->kh != 3 || d->kw != 3 || d->stride_h != 2 || d->stride_w != 2 || d->dil_h != 1 || d->dil_w != 1 || d->pad_h != 1 || d->pad_w != 1) return false;
-    if ((d->flags & (KXC_HIP_CONV_FORCE_DIRECT | KXC_HIP_CONV_HPOOL)) || d->c % kStep != 0) return false;
-    const int64_t OH = (static_cast<int64_t>(d->h) - 1) / 2 + 1, OW = (static_cast<int64_t>(d->w) - 1) / 2 + 1;
+    if (!d || d->n <= 0 || d->c <= 0 || d->h <= 0 || d->w <= 0 || d->o <= 0 || d->kh != d->kw || d->stride_h != d->stride_w) return false;
+    const int K = d->kh, S = d->stride_h;
+    const FilterKernels* kernels = nullptr;
+    for (const FilterKernels& k : kFilters)
+        if (k.k == K && k.s == S) kernels = &k;
+    if (!kernels || d->dil_h != 1 || d->dil_w != 1 || d->pad_h < 0 || d->pad_w < 0 || d->pad_h > 64 || d->pad_w > 64) return false;
+    if (second && (K != 3 || S != 2 || d->pad_h != 1 || d->pad_w != 1)) return false;
+    if (d->flags & (KXC_HIP_CONV_FORCE_DIRECT | KXC_HIP_CONV_HPOOL)) return false;
+    const int64_t Hp = static_cast<int64_t>(d->h) + 2 * d->pad_h, Wp = static_cast<int64_t>(d->w) + 2 * d->pad_w;
+    if (Hp < K || Wp < K) return false;
+    const int64_t OH = (Hp - K) / S + 1, OW = (Wp - K) / S + 1;
     const int64_t x_bytes = 4LL * d->n * d->c * d->h * d->w, y_elems = static_cast<int64_t>(d->n) * d->o * OH * OW;
-    const int64_t u_bytes = static_cast<int64_t>(FilterBytes(d->o, d->c, 3, second));
-    if (d->w > 4 * kPlane || x_bytes >= (1LL << 31) || y_elems >= (1LL << 29) || u_bytes >= (1LL << 31) || (d->n + 1LL) * (OH + 1) >= (1LL << 30)) return false;
+    const int64_t u_bytes = static_cast<int64_t>(FilterBytes(d->o, d->c, K, second));
+    if (x_bytes >= (1LL << 31) || y_elems >= (1LL << 29) || u_bytes >= (1LL << 31) || (d->n + 1LL) * (OH + K) >= (1LL << 30)) return false;
     Args& a = L->a;
     std::memset(&a, 0, sizeof(a));
     a.N = d->n; a.C = d->c; a.H = d->h; a.W = d->w; a.O = d->o;
     a.OH = static_cast<int32_t>(OH); a.OW = static_cast<int32_t>(OW); a.OHW = a.OH * a.OW; a.HW = a.H * a.W;
     a.M = a.N * a.OHW;
-    a.ph = a.pw = 1;
-    a.Hq = a.OH + 1;
-    const int64_t rows = MaxRows(a, 1);
+    a.ph = d->pad_h; a.pw = d->pad_w;
+    a.Hq = a.OH + (K - 1) / S;
     a.w4 = (a.W + 3) / 4;
-    if (2 * rows * a.w4 > 64 * kProducers * kUnits) return false;
-    // even columns 0 .. OW, odd ones behind them.  Where it fits, a row pitch that continues the banks of a row's last pixel with
-    // the next row's first one (a lane reads 16 bytes: 16 positions go through all banks).
-    a.hp = std::max(a.OW + 1, a.W / 2 + 1);
-    a.pitch = 2 * a.hp;
-    if (rows * a.pitch > kPlane) return false;
-    for (int32_t pitch = a.pitch; pitch < a.pitch + 16 && rows * pitch <= kPlane; ++pitch)
-        if ((pitch - a.OW) % 16 == 0) { a.pitch = pitch; break; }
-    a.csteps = a.C / kStep;
+    if (K > 1) {
+        const int64_t rows = MaxRows(a, (K - 1) / S);
+        if (a.W > 4 * kPlane || 2 * rows * a.w4 > 64 * kProducers * kUnits) return false;
+        // Stride 2: even columns, odd ones behind them.  Where it fits, a row pitch that continues the banks of a row's last pixel
+        // with the next row's first one (a lane reads 16 bytes: 16 positions go through all banks).
+        a.hp = std::max(a.OW + (K - 1) / 2, (a.W - 1 + a.pw) / 2 + 1);
+        a.pitch = S == 2 ? 2 * a.hp : std::max(a.OW + K - 1, a.W + a.pw);
+        if (rows * a.pitch > kPlane) return false;
+        const int32_t least = a.pitch;
+        for (int32_t pitch = least; pitch < least + 16 && rows * pitch <= kPlane; ++pitch)
+            if ((pitch - a.OW) % 16 == 0) { a.pitch = pitch; break; }
+    }
+    const int channels = kStep * ChannelSteps(K);
+    a.csteps = static_cast<int32_t>(CeilDiv(a.C, channels));
+    a.tail = a.C % channels != 0 ? 1 : 0;
+    a.quads = S == 1 && a.ph == 0 && a.pw == 0 && a.HW % 4 == 0 ? 1 : 0;
     a.p_tiles = static_cast<int32_t>(CeilDiv(a.M, kPix));
     a.o_tiles = static_cast<int32_t>(CeilDiv(a.O, kOut));
     const int64_t units = static_cast<int64_t>(a.p_tiles) * a.o_tiles;
@@ -93,7 +122,7 @@ bool Resolve(const kxc_hip_conv2d_desc* d, bool second, PackedLaunch* L) {
     a.u_bytes = static_cast<uint32_t>(u_bytes);
     a.flags = d->flags;
     const int64_t out_bytes = y_elems * 4 * (second ? 2 : 1);
-    const int split = Split(units * SelectLanes(), a.csteps, out_bytes);
+    const int split = Split(units * SelectLanes(), a.csteps, Steps(K, second), out_bytes);
     a.cps = static_cast<int32_t>(CeilDiv(a.csteps, split));
     a.gsplit = static_cast<int32_t>(CeilDiv(a.csteps, a.cps));      // no empty part
     if (a.gsplit > 1) L->scratch_bytes = static_cast<size_t>(a.gsplit) * out_bytes;
@@ -103,10 +132,11 @@ bool Resolve(const kxc_hip_conv2d_desc* d, bool second, PackedLaunch* L) {
     a.div_tiles = MakeFastDiv(a.o_fastest ? a.o_tiles : a.p_tiles); a.div_gsplit = MakeFastDiv(a.gsplit);
     L->second = second;
     L->filter_bytes = a.u_bytes;
-    L->lds_bytes = kLdsBytes;
-    L->gflop = 2e-9 * a.M * a.O * a.C * Steps(3, second);
-    L->kernel = second ? conv_bf16x3_kernel<3, 2, true> : conv_bf16x3_kernel<3, 2, false>;
-    L->name = second ? "mfma_k3x3s2_bf16x3_ds" : "mfma_k3x3s2_bf16x3";
+    L->lds_bytes = LdsBytes(K);
+    L->gflop = 2e-9 * a.M * a.O * a.C * (K * K + (second ? 1 : 0));
+    L->kernel = second ? conv_bf16x3_kernel<3, 2, true> : kernels->conv;
+    L->pack = kernels->pack;
+    L->name = second ? "mfma_k3x3s2_bf16x3_ds" : kernels->name;
     return true;
 }
 
@@ -178,12 +208,120 @@ bool Preferred(const kxc_hip_conv2d_desc* d, bool second, PackedLaunch* L) {
         const bool pooled = (d->flags & KXC_HIP_CONV_HPOOL) != 0;
         return (e && e[0] == '1') || pooled || (L->lds_bytes <= kMaxLdsBytes / 4 && L->gflop * SelectLanes() >= 1.8);
     }
-    return Resolve(d, second, L) && ((e && e[0] == '1') || L->gflop * SelectLanes() >= std::min(0.12 * L->a.csteps, 1.4));
+    // (a plan's filter launch packs 3x3 stride-2 filters only)
+    return d && d->kh == 3 && d->stride_h == 2 && d->pad_h == 1 && d->pad_w == 1 && d->c % conv_bx::kStep == 0 && Resolve(d, second, L) &&
+           ((e && e[0] == '1') || L->gflop * SelectLanes() >= std::min(0.12 * L->a.csteps, 1.4));
+}
+
+// `partials`: room for the partial outputs of a split reduction; nullptr: it is acquired here.
+int32_t LaunchConv(const PackedLaunch& L, const float* x, const float* w, const void* u, const float* bias, const float* residual, float* y,
+                   const float* w2, const float* bias2, float* y2, hipStream_t s, float* partials) {
+    conv_bx::Args a = L.a;
+    a.x = x; a.w = w; a.u = static_cast<const char*>(u); a.bias = bias; a.res = residual; a.y = y;
+    a.w2 = w2; a.bias2 = bias2; a.y2 = y2;
+    SplitScratchLease lease;      // held until the adding kernel is enqueued
+    if (a.gsplit > 1) {
+        bool split = partials != nullptr;
+        a.partial = partials;
+        if (!partials) {
+            if (int32_t rc = AcquireSplitScratch(s, L.scratch_bytes, &lease, &split)) return rc;
+            a.partial = lease.ptr;
+        }
+        if (!split) {             // no buffer to be had: the reduction in one piece
+            a.gsplit = 1;
+            a.cps = a.csteps;
+            a.div_gsplit = MakeFastDiv(1);
+            a.units_per_xcd = static_cast<int32_t>(CeilDiv(a.num_units, 8));
+        }
+    }
+    if (L.lds_bytes > 64 * 1024)
+        if (int32_t rc = GrantLds(reinterpret_cast<const void*>(L.kernel))) return rc;
+    hipLaunchKernelGGL(L.kernel, NoteGrid(dim3(static_cast<unsigned>(a.units_per_xcd * 8))), NoteBlock(dim3(conv_bx::kThreads)),
+                       NoteLds(L.lds_bytes), s, a);
+    if (int32_t rc = CheckLaunch(L.name)) return rc;
+    if (a.gsplit == 1) return KXC_HIP_OK;
+    SplitReduceArgs r;
+    r.partial = a.partial; r.bias = bias; r.res = residual; r.y = y;
+    r.total = a.M * a.O; r.gsplit = a.gsplit; r.O = a.O; r.flags = a.flags; r.div_ohw = a.div_ohw;
+    if (L.second) {
+        r.partial2 = a.partial + static_cast<int64_t>(a.gsplit) * r.total;
+        r.bias2 = bias2; r.y2 = y2; r.flags2 = bias2 ? KXC_HIP_CONV_BIAS : 0u;
+    }
+    return LaunchSplitReduce(s, r);
+}
+
+// Whether a single call, which packs its filter first, should take the kernel.  Its time: 10 us for two launches and what surrounds the
+// steps, the longer of the bytes at 4.5 TB/s and 0.29 us per tap and 16 channels (two workgroups on a compute unit take
+// 1.65 times as long as one; a 1x1 filter's few steps do not hide the bytes: the sum), and the adding launch.  The other kernels
+// take 9 us and 12 per GFLOP (13 for 1x1, 16 for 5x5 and 7x7; 14 us where a 1x1 filter's channels are no multiple of 16); at 3x3 a seventh of
+// that in hand (20 -> 439 at 7 x 29, batch 33 21.1 and 23.9).  us, with the
+// residual, theirs and here: 5x5, 64 -> 96 channels at 27 x 27, batch 8 40.0 and 27.3; 16 -> 192 at 76 x 35, stride 2, batch 6 19.5 and 17.4; 7x7,
+// 226 -> 161 at 26 x 33 72 and 44; 13 -> 356 at 64 x 12, batch 4 31.9 and 24.7; 3x3, 220 -> 260 at 9 x 10, batch 27 47.9 and 35.1; 16 -> 221 at 53 x 11,
+// batch 11 13.8 and 12.6; 1x1, 128 -> 512 at 28 x 28, batch 32 57.9 and 44.2; 63 -> 376 at 18 x 32, batch 13 20.1 and 14.4.  Not taken: 5x5,
+// 32 -> 32 at 19 x 12, batch 37 16.0 and 21.2; 7x7, 64 -> 96 at 15 x 16 17.9 and 25.2; 3x3, 16 -> 144 at 90 x 9, batch 11 12.0 and 16.5; 1x1, 224 -> 160 at 30 x 34,
+// batch 21 28.5 and 31.3; images of no whole 16 bytes, whose pixels come one by one, 160 -> 400 at 37 x 23, batch 7 17.5 and 29.6.
+// (Every single call asks: from the shape alone first, then whether the kernel covers it.)
+bool OperatorPreferred(const kxc_hip_conv2d_desc* d, PackedLaunch* L) {
+    using namespace conv_bx;
+    const int K = d->kh, S = d->stride_h;
+    if (K != d->kw || S != d->stride_w || d->n <= 0 || d->c <= 0 || d->o <= 0 || (S != 1 && S != 2) || K > 7) return false;
+    const char* e = std::getenv("KXC_HIP_CONV_BF16X3");
+    if (!(e && e[0] == '1')) {
+        // (3x3, stride 2: single calls agree with the outputs of kxc_hip_conv2d_pair_nchw_f32, which packs nothing.  Stride 1: Winograd
+        // takes large ones; half of a block of 128 output channels empty is no gain)
+        if (K == 3 && (S == 2 || d->o < 96)) return false;
+        const int64_t oh = (static_cast<int64_t>(d->h) + 2 * d->pad_h - K) / S + 1, ow = (static_cast<int64_t>(d->w) + 2 * d->pad_w - K) / S + 1;
+        if (oh <= 0 || ow <= 0) return false;
+        if (K == 1 && (S != 1 || d->pad_h != 0 || d->pad_w != 0 || static_cast<int64_t>(d->h) * d->w % 4 != 0)) return false;
+        const double pixels = static_cast<double>(d->n) * oh * ow, out_bytes = 4.0 * pixels * d->o, gflop = 2e-9 * pixels * d->o * d->c * K * K;
+        const double memory = (4.0 * d->n * d->c * d->h * d->w + out_bytes * ((d->flags & KXC_HIP_CONV_RESIDUAL) ? 2 : 1)) / 4.5e6;
+        const double others = (K == 1 && d->c % 16 != 0 ? 14 : 9) + (K >= 5 ? 16 : K == 1 ? 13 : 12) * gflop - (K == 3 ? 0.15 * (9 + 12 * gflop) : 0);
+        if (10 + memory >= others || pixels >= 1e9) return false;
+        const int64_t units = CeilDiv(static_cast<int64_t>(pixels), kPix) * CeilDiv(d->o, kOut);
+        const int csteps = static_cast<int>(CeilDiv(d->c, kStep * ChannelSteps(K))), steps = Steps(K, false);
+        const int split = Split(units * SelectLanes(), csteps, steps, static_cast<int64_t>(out_bytes));
+        const double groups = static_cast<double>(units) * split * SelectLanes();
+        const double load = groups <= 256 ? 1.0 : groups <= 512 ? 1.65 : 1.65 * groups / 512;
+        const double adding = split > 1 ? 5 + 2.0 * split * out_bytes / 4.5e6 : 0;
+        const double compute = 0.29 * steps * static_cast<double>(CeilDiv(csteps, split)) * load;
+        if (10 + (K == 1 ? compute + memory : std::max(compute, memory)) + adding >= others) return false;
+        const char* w = K == 3 ? std::getenv("KXC_HIP_WINOGRAD_BF16X3") : nullptr;      // (it says so for all large 3x3 stride-1 convolutions)
+        if ((e && e[0] == '0') || (w && w[0] == '0')) return false;
+    }
+    const char* variant = std::getenv("KXC_HIP_CONV_VARIANT");
+    return !(variant && *variant) && Resolve(d, false, L) && L->filter_bytes <= (32u << 20);      // (bounds the scratch kept per stream)
 }
 
 }  // namespace
 
 namespace kxc_hip {
+
+const char* PackedOperatorName(const kxc_hip_conv2d_desc* desc) {
+    PackedLaunch L;
+    return desc && OperatorPreferred(desc, &L) ? L.name : nullptr;
+}
+
+int32_t RunPackedOperator(const kxc_hip_conv2d_desc* desc, const float* x, const float* w, const float* bias, const float* residual, float* y,
+                          hipStream_t stream, bool* launched) {
+    const char* const who = "kxc_hip_conv2d_nchw_f32";
+    *launched = false;
+    PackedLaunch L;
+    // (kernels meet in the scratch: one packs the filter, the convolution reads it, and its parts are added)
+    if (!OperatorPreferred(desc, &L) || !StreamOrdersScratch(stream)) return KXC_HIP_OK;
+    KXC_HIP_REQUIRE(x && w && y, "%s: NULL pointer", who);
+    KXC_HIP_REQUIRE(!(desc->flags & KXC_HIP_CONV_BIAS) || bias, "%s: bias flag without bias", who);
+    KXC_HIP_REQUIRE(!(desc->flags & KXC_HIP_CONV_RESIDUAL) || residual, "%s: residual flag without residual", who);
+    SplitScratchLease lease;      // held until the last kernel that reads the scratch is enqueued
+    const size_t filter = (L.filter_bytes + 255) / 256 * 256;
+    if (int32_t rc = AcquireSplitScratch(stream, filter + L.scratch_bytes, &lease, launched)) return rc;
+    if (!*launched) return KXC_HIP_OK;
+    // (the filter is packed by every call: the caller may have changed it)
+    char* const u = reinterpret_cast<char*>(lease.ptr);
+    hipLaunchKernelGGL(L.pack, NoteGrid(dim3(static_cast<unsigned>(conv_bx::PackBlocks(desc->o, desc->c, desc->kh)))), NoteBlock(dim3(256)), NoteLds(0), stream,
+                       w, u, static_cast<int32_t>(desc->o), static_cast<int32_t>(desc->c));
+    if (int32_t rc = CheckLaunch("pack_filter_kernel")) return rc;
+    return LaunchConv(L, x, w, u, bias, residual, y, nullptr, nullptr, nullptr, stream, reinterpret_cast<float*>(u + filter));
+}
 
 struct PreparedPacked {
     PackedLaunch launch;
@@ -218,34 +356,7 @@ int32_t LaunchPreparedPacked(const PreparedPacked* p, const float* x, const floa
                            NoteLds(L.lds_bytes), s, b);
         return CheckLaunch(L.name);
     }
-    conv_bx::Args a = L.a;
-    a.x = x; a.w = w; a.u = static_cast<const char*>(u); a.bias = bias; a.res = residual; a.y = y;
-    a.w2 = w2; a.bias2 = bias2; a.y2 = y2;
-    SplitScratchLease lease;      // held until the adding kernel is enqueued
-    if (a.gsplit > 1) {
-        bool split = false;
-        if (int32_t rc = AcquireSplitScratch(s, L.scratch_bytes, &lease, &split)) return rc;
-        a.partial = lease.ptr;
-        if (!split) {             // no buffer to be had: the reduction in one piece
-            a.gsplit = 1;
-            a.cps = a.csteps;
-            a.div_gsplit = MakeFastDiv(1);
-            a.units_per_xcd = static_cast<int32_t>(CeilDiv(a.num_units, 8));
-        }
-    }
-    if (int32_t rc = GrantLds(reinterpret_cast<const void*>(L.kernel))) return rc;
-    hipLaunchKernelGGL(L.kernel, NoteGrid(dim3(static_cast<unsigned>(a.units_per_xcd * 8))), NoteBlock(dim3(conv_bx::kThreads)),
-                       NoteLds(L.lds_bytes), s, a);
-    if (int32_t rc = CheckLaunch(L.name)) return rc;
-    if (a.gsplit == 1) return KXC_HIP_OK;
-    SplitReduceArgs r;
-    r.partial = a.partial; r.bias = bias; r.res = residual; r.y = y;
-    r.total = a.M * a.O; r.gsplit = a.gsplit; r.O = a.O; r.flags = a.flags; r.div_ohw = a.div_ohw;
-    if (L.second) {
-        r.partial2 = a.partial + static_cast<int64_t>(a.gsplit) * r.total;
-        r.bias2 = bias2; r.y2 = y2; r.flags2 = bias2 ? KXC_HIP_CONV_BIAS : 0u;
-    }
-    return LaunchSplitReduce(s, r);
+    return LaunchConv(L, x, w, u, bias, residual, y, w2, bias2, y2, s, nullptr);
 }
 
 }  // namespace kxc_hip

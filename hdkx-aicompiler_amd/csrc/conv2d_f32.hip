@@ -1502,6 +1502,11 @@ int32_t Conv2dRun(const kxc_hip_conv2d_desc* desc, const float* x, const float* 
         if (int32_t rc = RunWinogradOperator(desc, x, w, bias, residual, y, ResolveStream(stream), &launched)) return rc;
         if (launched) return KXC_HIP_OK;
     }
+    if (!second && !no_alloc && desc) {
+        bool launched = false;
+        if (int32_t rc = RunPackedOperator(desc, x, w, bias, residual, y, ResolveStream(stream), &launched)) return rc;
+        if (launched) return KXC_HIP_OK;
+    }
     if (int32_t rc = Conv2dResolve(desc, second != nullptr, who, &L)) return rc;
     return Conv2dLaunch(L, who, x, w, bias, residual, y, stream, no_alloc, second);
 }
@@ -1570,7 +1575,10 @@ static const char* ConvVariantName(const kxc_hip_conv2d_desc* desc, bool in_plan
 const char* kxc_hip_conv2d_node_variant(const kxc_hip_conv2d_desc* desc) { return ConvVariantName(desc, true); }
 
 const char* kxc_hip_conv2d_variant(const kxc_hip_conv2d_desc* desc) {
-    return desc && WinogradOperatorPreferred(desc) ? kWinogradOperatorName : ConvVariantName(desc, false);
+    if (!desc) return ConvVariantName(desc, false);
+    if (WinogradOperatorPreferred(desc)) return kWinogradOperatorName;
+    const char* packed = PackedOperatorName(desc);
+    return packed ? packed : ConvVariantName(desc, false);
 }
 
 int32_t kxc_hip_conv2d_nchw_f32(const kxc_hip_conv2d_desc* desc, const float* x, const float* w, const float* bias,

@@ -164,8 +164,9 @@ __global__ void __launch_bounds__(256) wino_weight_batch_kernel(const WinoWeight
     int j = 0;
     while (j + 1 < b.count && static_cast<int32_t>(blockIdx.x) >= b.first_block[j + 1]) ++j;
     const int tile = static_cast<int>(blockIdx.x) - b.first_block[j];
+    static_assert(conv_bx::PackFloats(3) <= sizeof(raw) / sizeof(float), "one block of LDS for all forms");
     if ((b.packed7 >> j) & 1u) conv7_bx::pack_tile(b.w[j], b.u[j], b.O[j], tile);
-    else if ((b.packed >> j) & 1u) conv_bx::pack_tile(b.w[j], b.w2[j], b.u[j], b.O[j], b.C[j], tile, raw);
+    else if ((b.packed >> j) & 1u) conv_bx::pack_block<3, 2>(b.w[j], b.w2[j], b.u[j], b.O[j], b.C[j], tile, raw);
     else if ((b.three_part >> j) & 1u) wino_bx::weight_tile(b.w[j], b.u[j], b.O[j], b.C[j], tile, raw);
     else wino_weight_tile(b.w[j], reinterpret_cast<float*>(b.u[j]), b.O[j], b.C[j], tile, raw);
 }
@@ -1026,7 +1027,7 @@ int32_t LaunchWinogradWeightTransforms(const WinoWeightJob* jobs, int32_t count,
             if (form == kFormPacked) (seven ? b.packed7 : b.packed) |= 1u << b.count;
             b.w2[b.count] = job.w2;
             ++b.count;
-            blocks += seven ? CeilDiv(O, 32) : form != kWinoFormF32 ? wino_bx::WeightTiles(O, C) : WeightTiles(CeilDiv(O, 32) * 32, C);
+            blocks += seven ? CeilDiv(O, 32) : form == kFormPacked ? conv_bx::PackBlocks(O, C, 3) : form != kWinoFormF32 ? wino_bx::WeightTiles(O, C) : WeightTiles(CeilDiv(O, 32) * 32, C);
             KXC_HIP_REQUIRE(blocks < kMaxGridX, "winograd weight transform: too many blocks");
         }
     }

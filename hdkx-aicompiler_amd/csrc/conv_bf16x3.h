@@ -1,10 +1,10 @@
-// conv_bf16x3.h -- strided convolutions as an implicit GEMM on the bf16 matrix cores with three-part operands
-// (bf16x3.h); included by conv2d_bf16x3.hip (selection, launch) and conv2d_wino_f32.hip (the filters of a plan are packed
-// by one launch).
+// conv_bf16x3.h -- convolutions of 1x1 to 7x7 filters with stride 1 and 2 as an implicit GEMM on the bf16 matrix cores with
+// three-part operands (bf16x3.h); included by conv2d_bf16x3.hip (selection, launch) and conv2d_wino_f32.hip (the filters of a
+// plan are packed by one launch).
 //
 // D[o][pixel] += W[o][tap, c] X[tap, c][pixel], pixels flattened over (n, oh, ow).  A workgroup owns 128 output channels x 64 pixels and
-// walks the input channels 16 at a time, in two halves: the input rows of even, then of odd padded position (a 3x3
-// filter's rows 0 and 2, then 1), each with an LDS buffer of its own.
+// walks the input channels 16 at a time, with stride 2 in two halves: the input rows of even, then of odd padded position (a
+// 3x3 filter's rows 0 and 2, then 1).  Two LDS buffers; a 1x1 filter takes 64 channels at a time and no rows, only the tile's pixels.
 //  * Two producer waves load the rows in pieces of four columns x eight channels, split every value into its three parts once,
 //    and leave them in LDS as the 16-byte fragments that the matrix instructions take: [part][channels c .. c + 7][row][column
 //    parity][column], so that neighbouring pixels of a tap are neighbouring fragments.  They load one half ahead of the one that
@@ -35,14 +35,19 @@ namespace conv_bx {
 constexpr int kOut = 128, kPix = 64, kStep = 16;      // output channels and pixels of a workgroup; channels per step
 constexpr int kConsumers = 4, kProducers = 2;         // waves
 constexpr int kThreads = 64 * (kConsumers + kProducers);
-constexpr int kPlane = 384;                           // 16-byte units (one position, eight channels, one part) of an LDS plane
-constexpr int kBufBytes = 6 * kPlane * 16;            // [part][channel half] planes
-constexpr size_t kLdsBytes = 2 * kBufBytes;
+constexpr int kPlane = 384;                           // positions of an LDS plane (16 bytes: eight channels of one part)
 constexpr int kUnits = 2;                             // (channel half, row, four columns) pieces per producer lane
+// Row phases of a filter (two halves of a step as described above, or the step as a whole), steps of 16 channels between two
+// barriers (a 1x1 filter has one tap for each: four of them), bytes of an LDS buffer.
+constexpr int Phases(int K, int S) { return S == 2 && K > 1 ? 2 : 1; }
+constexpr int ChannelSteps(int K) { return K == 1 ? 4 : 1; }
+constexpr int Plane(int K) { return K == 1 ? kPix : kPlane; }
+constexpr int BufBytes(int K) { return 3 * 2 * ChannelSteps(K) * Plane(K) * 16; }
+inline size_t LdsBytes(int K) { return 2 * static_cast<size_t>(BufBytes(K)); }
 
-// Steps of the packed filter per 16 channels: the taps in the order the kernel takes them, the second output's filter
+// Steps of the packed filter between two barriers (per row phase pair): the taps in the order the kernel takes them, the second output's filter
 // behind the tap that it shares its operand with.
-constexpr int Steps(int K, bool second) { return K * K + (second ? 1 : 0); }
+constexpr int Steps(int K, bool second) { return K == 1 ? ChannelSteps(K) : K * K + (second ? 1 : 0); }
 // Taps of row phase rho: rows rh = rho, rho + S, ...
 constexpr int PhaseTaps(int K, int S, int rho) { return (K - rho + S - 1) / S * K; }
 constexpr int PhaseFirst(int K, int S, int rho) { return rho == 0 ? 0 : PhaseTaps(K, S, 0); }
@@ -50,8 +55,10 @@ constexpr int PhaseFirst(int K, int S, int rho) { return rho == 0 ? 0 : PhaseTap
 constexpr int TapOf(int K, int S, int rho, int t) { return (rho + t / K * S) * K + t % K; }
 
 inline size_t FilterBytes(int64_t O, int64_t C, int K, bool second) {
-    return static_cast<size_t>(CeilDiv(O, 32) * CeilDiv(C, kStep)) * Steps(K, second) * 3 * 1024;
+    return static_cast<size_t>(CeilDiv(O, 32) * CeilDiv(C, kStep * ChannelSteps(K))) * Steps(K, second) * 3 * 1024;
 }
+inline int64_t PackBlocks(int64_t O, int64_t C, int K) { return CeilDiv(O, 32) * 4 * CeilDiv(C, kStep * ChannelSteps(K)); }
+constexpr int PackFloats(int K) { return 8 * (kStep * ChannelSteps(K) * K * K + 1); }
 
 struct Args {
     const float* x;
@@ -67,7 +74,8 @@ struct Args {
     int32_t N, C, H, W, O, OH, OW, M, OHW, HW, ph, pw;
     int32_t Hq, pitch, hp;              // rows per image in a row phase; LDS row pitch; positions of the even columns
     int32_t w4;                         // pieces of four columns per row
-    int32_t csteps, cps, gsplit;        // channel steps, per part, parts
+    int32_t csteps, cps, gsplit;        // channel steps (of 16 * ChannelSteps), per part, parts
+    int32_t tail, quads;                // the last step is short of channels; K = 1: four pixels are 16 bytes of one channel
     int32_t p_tiles, o_tiles, num_units, units_per_xcd, o_fastest;
     uint32_t x_bytes, u_bytes, flags;
     FastDiv div_ohw, div_ow, div_hq, div_w4, div_tiles, div_gsplit;
@@ -84,8 +92,8 @@ __device__ __forceinline__ float relu_sel(float v) { return (v > 0.0f) ? v : 0.0
 
 template <int K, int S, bool SECOND>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3, 3))) conv_bf16x3_kernel(const Args a) {
-    static_assert(S == 2 && K == 3, "two row phases, one LDS buffer each");
-    constexpr int NS = Steps(K, SECOND);
+    static_assert(!SECOND || (S == 2 && K == 3), "the second output reads the middle tap of the second phase");
+    constexpr int NS = Steps(K, SECOND), PH = Phases(K, S), CS = ChannelSteps(K), PLANE = Plane(K), PART = 2 * CS * PLANE * 16, BUF = BufBytes(K);
     extern __shared__ __attribute__((aligned(16))) char lds[];
     const int tid = static_cast<int>(threadIdx.x), lane = tid & 63, half = lane >> 5, r = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -108,79 +116,108 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3
     }
     // borders, and rows and columns outside the image, stay zero
     auto clear = [&]() __attribute__((always_inline)) {
-        for (int i = tid; i < static_cast<int>(kLdsBytes / 16); i += kThreads) *reinterpret_cast<u32x4*>(lds + i * 16) = u32x4{0, 0, 0, 0};
+        if (K > 1)
+            for (int i = tid; i < 2 * BUF / 16; i += kThreads) *reinterpret_cast<u32x4*>(lds + i * 16) = u32x4{0, 0, 0, 0};
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     };
 
     if (wave >= kConsumers) {
         // ---- producers: pieces of four columns x eight channels, split into their three parts once per workgroup
         const int ptid = tid - 64 * kConsumers, per_half = rows * a.w4;
-        uint32_t goff[S][kUnits];
-        int lpos[kUnits], left[kUnits];              // position of the first column's unit; columns that exist
+        constexpr int U = K == 1 ? 1 : kUnits;
+        uint32_t goff[K == 1 ? 4 : PH][U];           // K = 1: of the four pixels
+        int lpos[U], left[U], ch[U];                 // position of the first column's unit; columns that exist; first channel
+        if constexpr (K == 1) {
+            // (the positions are the tile's pixels)
+            const int oct = ptid >> 4, q = ptid & 15;
 #pragma unroll
-        for (int k = 0; k < kUnits; ++k) {
-            const int u = ptid + 64 * kProducers * k;
-            const int h = u >= per_half ? 1 : 0, e = u - h * per_half;
-            const int row = fast_div(e, a.div_w4), p4 = e - row * a.w4;
-            const int Q = qmin + row, n = fast_div(Q, a.div_hq), idx = Q - n * a.Hq;
-            const bool ok = u < 2 * per_half && n < a.N;
-#pragma unroll
-            for (int rho = 0; rho < S; ++rho) {
-                const int ih = idx * S + rho - a.ph;
-                goff[rho][k] = ok && ih >= 0 && ih < a.H ? static_cast<uint32_t>(((n * a.C + h * 8) * a.H + ih) * a.W + p4 * 4) * 4u : kOob;
+            for (int i = 0; i < 4; ++i) {
+                const int m = m0 + q * 4 + i, n = fast_div(m, a.div_ohw), rem = m - n * a.OHW, oh = fast_div(rem, a.div_ow);
+                const int ih = oh * S - a.ph, iw = (rem - oh * a.OW) * S - a.pw;
+                const bool ok = m < a.M && ih >= 0 && ih < a.H && iw >= 0 && iw < a.W;
+                goff[i][0] = ok ? static_cast<uint32_t>(((n * a.C + oct * 8) * a.H + ih) * a.W + iw) * 4u : kOob;
             }
-            lpos[k] = h * kPlane + row * a.pitch + p4 * (4 / S);
-            left[k] = ok ? a.W - p4 * 4 : 0;
-        }
-        f32x4 v[S][kUnits][8];          // a phase's next pieces are on their way while the other phase's are split
-        auto load = [&](int c, auto rho_c) __attribute__((always_inline)) {
-            constexpr int RHO = decltype(rho_c)::value;
+            ch[0] = oct * 8;
+            lpos[0] = oct * PLANE + q * 4;
+            left[0] = 4;
+        } else {
 #pragma unroll
-            for (int k = 0; k < kUnits; ++k) {
+            for (int k = 0; k < U; ++k) {
+                const int u = ptid + 64 * kProducers * k;
+                const int h = u >= per_half ? 1 : 0, e = u - h * per_half;
+                const int row = fast_div(e, a.div_w4), p4 = e - row * a.w4;
+                const int Q = qmin + row, n = fast_div(Q, a.div_hq), idx = Q - n * a.Hq;
+                const bool ok = u < 2 * per_half && n < a.N;
+#pragma unroll
+                for (int rho = 0; rho < PH; ++rho) {
+                    const int ih = idx * S + rho - a.ph;
+                    goff[rho][k] = ok && ih >= 0 && ih < a.H ? static_cast<uint32_t>(((n * a.C + h * 8) * a.H + ih) * a.W + p4 * 4) * 4u : kOob;
+                }
+                ch[k] = h * 8;
+                lpos[k] = h * PLANE + row * a.pitch + p4 * (4 / S);
+                left[k] = ok ? a.W - p4 * 4 : 0;
+            }
+        }
+        f32x4 v[2][U][8];          // the next pieces are on their way while the ones before them are split
+        auto load = [&](int q, auto set_c) __attribute__((always_inline)) {
+            constexpr int SET = decltype(set_c)::value, RHO = PH == 2 ? SET : 0;
+            const int c = (c_lo + q / PH) * kStep * CS;
+#pragma unroll
+            for (int k = 0; k < U; ++k) {
                 if (k > 0 && 2 * per_half <= 64 * kProducers * k) break;
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
-                    const uint32_t skip = static_cast<uint32_t>(c * kStep + j) * static_cast<uint32_t>(a.HW) * 4u;
+                    const uint32_t skip = min(static_cast<uint32_t>(c + j) * static_cast<uint32_t>(a.HW) * 4u, a.x_bytes);
                     const __amdgpu_buffer_rsrc_t xr = rsrc(reinterpret_cast<const char*>(a.x) + skip, a.x_bytes - skip);
-                    v[RHO][k][j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, goff[RHO][k], 0, 0));
-                }
-            }
-        };
-        auto store = [&](auto rho_c) __attribute__((always_inline)) {
-            constexpr int RHO = decltype(rho_c)::value;
+                    const bool absent = a.tail && c + ch[k] + j >= a.C;
+                    if (K > 1 || a.quads) {
+                        v[SET][k][j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, absent ? kOob : goff[RHO][k], 0, 0));
+                    } else {
 #pragma unroll
-            for (int k = 0; k < kUnits; ++k) {
-                if (k > 0 && 2 * per_half <= 64 * kProducers * k) break;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const float t[8] = {v[RHO][k][0][j], v[RHO][k][1][j], v[RHO][k][2][j], v[RHO][k][3][j],
-                                        v[RHO][k][4][j], v[RHO][k][5][j], v[RHO][k][6][j], v[RHO][k][7][j]};
-                    const Split8 s = split8(t);
-                    if (j < left[k]) {
-                        char* const dst = lds + RHO * kBufBytes + (lpos[k] + ((j + a.pw) % S) * a.hp + (j + a.pw) / S) * 16;
-                        *reinterpret_cast<u32x4*>(dst) = s.h;
-                        *reinterpret_cast<u32x4*>(dst + 2 * kPlane * 16) = s.m;
-                        *reinterpret_cast<u32x4*>(dst + 4 * kPlane * 16) = s.l;
+                        for (int i = 0; i < 4; ++i)
+                            v[SET][k][j][i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xr, absent ? kOob : goff[K == 1 ? i : 0][k], 0, 0));
                     }
                 }
             }
         };
-        using P0 = std::integral_constant<int, 0>;
-        using P1 = std::integral_constant<int, 1>;
-        load(c_lo, P0{});
-        load(c_lo, P1{});
+        auto store = [&](auto set_c) __attribute__((always_inline)) {
+            constexpr int SET = decltype(set_c)::value;
+#pragma unroll
+            for (int k = 0; k < U; ++k) {
+                if (k > 0 && 2 * per_half <= 64 * kProducers * k) break;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float t[8] = {v[SET][k][0][j], v[SET][k][1][j], v[SET][k][2][j], v[SET][k][3][j],
+                                        v[SET][k][4][j], v[SET][k][5][j], v[SET][k][6][j], v[SET][k][7][j]};
+                    const Split8 s = split8(t);
+                    if (j < left[k]) {
+                        const int at = K == 1 ? j : ((j + a.pw) % S) * a.hp + (j + a.pw) / S;
+                        char* const dst = lds + SET * BUF + (lpos[k] + at) * 16;
+                        *reinterpret_cast<u32x4*>(dst) = s.h;
+                        *reinterpret_cast<u32x4*>(dst + PART) = s.m;
+                        *reinterpret_cast<u32x4*>(dst + 2 * PART) = s.l;
+                    }
+                }
+            }
+        };
+        using S0 = std::integral_constant<int, 0>;
+        using S1 = std::integral_constant<int, 1>;
+        const int count = (c_hi - c_lo) * PH;        // buffers full
+        load(0, S0{});
+        if (count > 1) load(1, S1{});
         clear();
-        store(P0{});
-        if (c_lo + 1 < c_hi) load(c_lo + 1, P0{});
+        store(S0{});
+        if (count > 2) load(2, S0{});
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        for (int c = c_lo; c < c_hi; ++c) {
-            // consumers read phase 0 of step c
-            store(P1{});
-            if (c + 1 < c_hi) load(c + 1, P1{});
+        for (int q = 0; q < count; q += 2) {
+            // consumers read buffer 0
+            if (q + 1 < count) store(S1{});
+            if (q + 3 < count) load(q + 3, S1{});
             asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            // ... phase 1
-            if (c + 1 < c_hi) store(P0{});
-            if (c + 2 < c_hi) load(c + 2, P0{});
+            if (q + 1 == count) break;
+            // ... buffer 1
+            if (q + 2 < count) store(S0{});
+            if (q + 4 < count) load(q + 4, S0{});
             asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         }
         return;
@@ -199,7 +236,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3
         const int m = m0 + j * 32 + r, mc = min(m, a.M - 1);
         const int n = fast_div(mc, a.div_ohw), rem = mc - n * a.OHW;
         const int oh = fast_div(rem, a.div_ow), ow = rem - oh * a.OW;
-        lbase[j] = (half * kPlane + (n * a.Hq + oh - qmin) * a.pitch + ow) * 16;
+        lbase[j] = (half * PLANE + (K == 1 ? j * 32 + r : (n * a.Hq + oh - qmin) * a.pitch + ow)) * 16;
         ybase[j] = m < a.M ? n * a.O * a.OHW + rem : -1;
     }
     f32x16 big[2], small[2], acc2[2];
@@ -216,10 +253,10 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3
         a_so = min(a_so + 3072u, a_last);
     };
     // parts: 0 = h, 1 = m, 2 = l
-    auto read_b = [&](int rho, int toff, int p) __attribute__((always_inline)) {
+    auto read_b = [&](int toff, int p) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < 2; ++j)
-            vb[j][p] = *reinterpret_cast<const u32x4*>(lds + rho * kBufBytes + p * 2 * kPlane * 16 + lbase[j] + toff);
+            vb[j][p] = *reinterpret_cast<const u32x4*>(lds + p * PART + lbase[j] + toff);
         __builtin_amdgcn_sched_barrier(0);
     };
     auto mul = [&](f32x16 (&acc)[2], int b, int pa, int pb) __attribute__((always_inline)) {
@@ -242,22 +279,27 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3
             for (int g = 0; g < 16; ++g) acc[j][g] = __fadd_rn(acc[j][g], small[j][g]);
         __builtin_amdgcn_sched_barrier(0);
     };
-    auto tap_off = [&](int tap) { return ((tap / K / S) * a.pitch + ((tap % K) % S) * a.hp + (tap % K) / S) * 16; };
-    auto phase = [&](auto rho_c) __attribute__((always_inline)) {
+    // offset of the t-th operand of a row phase in its buffer
+    auto operand = [&](int rho, int t) {
+        if (K == 1) return t * 2 * PLANE * 16;
+        const int tap = TapOf(K, PH, rho, t);
+        return ((tap / K / S) * a.pitch + ((tap % K) % S) * a.hp + (tap % K) / S) * 16;
+    };
+    auto phase = [&](auto rho_c, int buf) __attribute__((always_inline)) {
         constexpr int RHO = decltype(rho_c)::value;
-        constexpr int T = PhaseTaps(K, S, RHO);
+        constexpr int T = K == 1 ? CS : PhaseTaps(K, PH, RHO);
         constexpr int CENTRE = SECOND && RHO == 1 ? 1 : -1;
-        constexpr int FIRST = PhaseFirst(K, S, RHO);
+        constexpr int FIRST = K == 1 ? 0 : PhaseFirst(K, PH, RHO);
         {
-            const int t0 = tap_off(TapOf(K, S, RHO, 0));
-            read_b(RHO, t0, 2);
-            read_b(RHO, t0, 1);
-            read_b(RHO, t0, 0);
+            const int t0 = buf + operand(RHO, 0);
+            read_b(t0, 2);
+            read_b(t0, 1);
+            read_b(t0, 0);
         }
 #pragma unroll
         for (int t = 0; t < T; ++t) {
             const int step = FIRST + t + (CENTRE >= 0 && t > CENTRE ? 1 : 0), b = step & 1;
-            const int next = tap_off(TapOf(K, S, RHO, t + 1 < T ? t + 1 : t));
+            const int next = buf + operand(RHO, t + 1 < T ? t + 1 : t);
             load_a(b ^ 1);
             if (SECOND && RHO == 1 && t == CENTRE + 1) mul0(small, b, 0, 2);
             else mul(small, b, 0, 2);
@@ -269,29 +311,31 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3
                 mul(acc2, b ^ 1, 0, 0);
                 fold(big);
                 mul0(small, b ^ 1, 0, 2);
-                read_b(RHO, next, 2);
+                read_b(next, 2);
                 mul(small, b ^ 1, 1, 1); mul(small, b ^ 1, 0, 1);
-                read_b(RHO, next, 1);
+                read_b(next, 1);
                 mul(small, b ^ 1, 2, 0); mul(small, b ^ 1, 1, 0);
-                read_b(RHO, next, 0);
+                read_b(next, 0);
                 fold(acc2);
                 continue;
             }
-            if (t + 1 < T) read_b(RHO, next, 2);
+            if (t + 1 < T) read_b(next, 2);
             mul(small, b, 1, 1); mul(small, b, 0, 1);
-            if (t + 1 < T) read_b(RHO, next, 1);
+            if (t + 1 < T) read_b(next, 1);
             mul(small, b, 2, 0); mul(small, b, 1, 0); mul(big, b, 0, 0);
-            if (t + 1 < T) read_b(RHO, next, 0);
+            if (t + 1 < T) read_b(next, 0);
         }
     };
     load_a(0);
     clear();
     asm volatile("s_barrier" ::: "memory");
     for (int c = c_lo; c < c_hi; ++c) {
-        phase(std::integral_constant<int, 0>{});
+        phase(std::integral_constant<int, 0>{}, PH == 1 && ((c - c_lo) & 1) ? BUF : 0);
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        phase(std::integral_constant<int, 1>{});
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if constexpr (PH == 2) {
+            phase(std::integral_constant<int, 1>{}, BUF);
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        }
         if constexpr (NS & 1) {
 #pragma unroll
             for (int p = 0; p < 3; ++p) { const u32x4 t = ua[0][p]; ua[0][p] = ua[1][p]; ua[1][p] = t; }
@@ -368,7 +412,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3
             const int64_t at = static_cast<int64_t>(n * a.O + o) * a.OHW + rem;
             float s = 0.0f;
 #pragma unroll 1
-            for (int c = c_lo * kStep; c < c_hi * kStep; ++c) {
+            for (int c = c_lo * kStep * CS; c < min(c_hi * kStep * CS, a.C); ++c) {
                 const float* const xc = a.x + static_cast<int64_t>(n * a.C + c) * a.HW;
                 if (one_tap) {
                     s = __fadd_rn(s, __fmul_rn(xc[oh * S * a.W + ow * S], w[static_cast<int64_t>(o) * a.C + c]));
@@ -391,32 +435,44 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3
 }
 
 // ------------------------------------------------------------------------------------------
-// The packed filter: [o / 32][c / 16][step][part][lane][16 bytes], lane = o % 32 + 32 * (c / 8 % 2).  A workgroup of 256
-// threads takes 32 output x 16 input channels; thread (step % 4, half, o) makes the fragments of every fourth step.
-// `raw`: 32 * (16 * 9 + 1) floats of LDS.
+// The packed filter: [o / 32][c / 16 (64 for 1x1 filters)][step][part][lane][16 bytes], lane = o % 32 + 32 * (c / 8 % 2).  A
+// workgroup of 256 threads takes 8 output channels of one [c]: their filters pass through LDS (PackFloats(K) floats), so that they
+// are read as they lie in memory.
 // ------------------------------------------------------------------------------------------
-__device__ __forceinline__ void pack_tile(const float* __restrict__ w, const float* __restrict__ w2, char* __restrict__ u, int32_t O, int32_t C,
-                                          int tile, float* raw) {
-    constexpr int K = 3, S = 2, RS = kStep * K * K + 1;
+template <int K, int S>
+__device__ __forceinline__ void pack_block(const float* __restrict__ w, const float* __restrict__ w2, char* __restrict__ u, int32_t O, int32_t C,
+                                           int block, float* raw) {
+    constexpr int KK = K * K, CH = kStep * ChannelSteps(K), RUN = CH * KK, PH = Phases(K, S);
     const bool second = w2 != nullptr;
-    const int ns = Steps(K, second), csteps = (C + kStep - 1) / kStep;
-    const int ob = tile / csteps, c0 = (tile - ob * csteps) * kStep;
-    const int tid = static_cast<int>(threadIdx.x), ol = tid & 31, half = (tid >> 5) & 1;
-    stage_filters<kStep>(w, O, C, ob * 32, c0, min(kStep, C - c0), raw);
+    const int ns = Steps(K, second), csteps = (C + CH - 1) / CH;
+    const int og = block / csteps, cs = block - og * csteps, c0 = cs * CH, run = min(CH, C - c0) * KK;
+    const int tid = static_cast<int>(threadIdx.x);
+    float t[(8 * RUN + 255) / 256];
+#pragma unroll
+    for (int k = 0; k < (8 * RUN + 255) / 256; ++k) {
+        const int i = k * 256 + tid, ol = i / RUN, r = i - ol * RUN;
+        const bool ok = ol < 8 && og * 8 + ol < O && r < run;
+        const float x = w[ok ? (static_cast<int64_t>(og * 8 + ol) * C + c0) * KK + r : 0];
+        t[k] = ok ? x : 0.0f;
+    }
+#pragma unroll
+    for (int k = 0; k < (8 * RUN + 255) / 256; ++k) {
+        const int i = k * 256 + tid, ol = i / RUN;
+        if (ol < 8) raw[ol * (RUN + 1) + i - ol * RUN] = t[k];
+    }
     __syncthreads();
-    const int n0 = PhaseTaps(K, S, 0), centre = n0 + 1;             // (K = 3, S = 2: tap (1, 1))
-    for (int step = tid >> 6; step < ns; step += 4) {
+    const int n0 = PhaseTaps(K, PH, 0), centre = n0 + 1;            // (second: K = 3, S = 2, tap (1, 1))
+    for (int i = tid; i < ns * 16; i += 256) {
+        const int ol = i & 7, half = (i >> 3) & 1, step = i >> 4, o = og * 8 + ol;
         const bool is2 = second && step == centre + 1;
-        const int t = second && step > centre ? step - 1 : step;
-        const int tap = t < n0 ? TapOf(K, S, 0, t) : TapOf(K, S, 1, t - n0);
+        const int tt = second && step > centre ? step - 1 : step;
+        const int tap = K == 1 ? 0 : tt < n0 ? TapOf(K, PH, 0, tt) : TapOf(K, PH, 1, tt - n0), first = (K == 1 ? step * kStep : 0) + half * 8;
         float v[8];
 #pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            const int o = ob * 32 + ol, cc = c0 + half * 8 + c;
-            v[c] = is2 ? (o < O && cc < C ? w2[static_cast<int64_t>(o) * C + cc] : 0.0f) : raw[ol * RS + (half * 8 + c) * K * K + tap];
-        }
+        for (int c = 0; c < 8; ++c)
+            v[c] = is2 ? (o < O && c0 + half * 8 + c < C ? w2[static_cast<int64_t>(o) * C + c0 + half * 8 + c] : 0.0f) : raw[ol * (RUN + 1) + (first + c) * KK + tap];
         const Split8 s = split8(v);
-        char* const dst = u + (static_cast<int64_t>(tile) * ns + step) * 3072 + (half * 32 + ol) * 16;
+        char* const dst = u + ((static_cast<int64_t>(o / 32) * csteps + cs) * ns + step) * 3072 + (half * 32 + o % 32) * 16;
         *reinterpret_cast<u32x4*>(dst) = s.h;
         *reinterpret_cast<u32x4*>(dst + 1024) = s.m;
         *reinterpret_cast<u32x4*>(dst + 2048) = s.l;

@@ -171,10 +171,14 @@ typedef struct kxc_hip_conv2d_desc {
  * values of 1 costs its neighbours their digits; Inf and NaN do not: such outputs are evaluated by the definition).
  * KXC_HIP_CONV_WINOGRAD=0 in the environment keeps the kernels that add only what an output's window holds.
  *
- * Scratch.  A launch that splits its reduction over workgroups, and a large 3x3 stride-1 call that runs as Winograd and
- * transforms its filter first, keep intermediate values in a buffer that the library holds per (device, stream handle):
- * calls on one stream are safe from any thread.  While the stream is being captured, and on hipStreamPerThread, large 3x3
- * stride-1 calls, 5x5 filters, calls of fewer than 32 output channels or pixels and 1x1 filters whose reduction can be split
+ * Large calls of other filters (..._variant says "..._bf16x3") run on the bf16 matrix cores with every operand as three bf16
+ * parts: exact from 2^-109 on, below it an operand is off by at most 2^-134; sums that are not finite are evaluated by the
+ * definition.  KXC_HIP_CONV_BF16X3=0 keeps the fp32 instructions.
+ *
+ * Scratch.  A launch that splits its reduction over workgroups, and a large call that transforms or packs its filter first
+ * (..._variant says "winograd_..." or "..._bf16x3"), keep intermediate values in a buffer that the library holds per (device, stream handle):
+ * calls on one stream are safe from any thread.  While the stream is being captured, and on hipStreamPerThread, those large
+ * calls, 5x5 filters, calls of fewer than 32 output channels or pixels and 1x1 filters whose reduction can be split
  * over the waves of a workgroup instead take a kernel that needs no buffer (the same bits whether or not an earlier call grew
  * one).  Other launches with a split reduction use the buffer there too:
  * their graph must be replayed on the stream it was captured on (or with nothing else running on that stream's buffer),
@@ -190,8 +194,8 @@ const char* kxc_hip_conv2d_variant(const kxc_hip_conv2d_desc* desc);
 const char* kxc_hip_conv2d_node_variant(const kxc_hip_conv2d_desc* desc);
 /* The same operator for callers that cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  Same arguments and
- * results (up to fp32 rounding where kxc_hip_conv2d_variant says "winograd_...", whose filter takes scratch this entry
- * point does not have) as kxc_hip_conv2d_nchw_f32, but it calls no hipMalloc / hipFree or allocating library routine: the partial sums
+ * results (up to fp32 rounding where kxc_hip_conv2d_variant says "winograd_..." or "..._bf16x3", whose filter takes scratch
+ * this entry point does not have) as kxc_hip_conv2d_nchw_f32, but it calls no hipMalloc / hipFree or allocating library routine: the partial sums
  * of a reduction split over workgroups (small launches with long reductions, e.g. batch-1 512-channel layers) go
  * to a device array built into the library, kxc_hip_conv2d_noalloc_scratch_bytes() = 8 MiB per GPU, held until the
  * process ends.  A launch whose partial sums would not fit fails with KXC_HIP_ERR_INVALID and launches nothing
@@ -293,7 +297,7 @@ int32_t kxc_hip_global_avg_pool2d_f32(const float* x, float* y, int64_t n, int64
  * multiplies, unless transB = 1 and k is a multiple of 32).  Products of more than four rows run on the bf16 matrix cores, every operand as three bf16
  * parts: exact from 2^-109 on, below it an operand is off by at most 2^-134; KXC_HIP_GEMM_BF16X3=0 in the environment keeps
  * the fp32 instructions, KXC_HIP_WINOGRAD_BF16X3=0 those of the convolutions (large 3x3 stride-1 ones),
- * KXC_HIP_CONV_BF16X3=0 those of a plan's large 3x3 stride-2 ones. */
+ * KXC_HIP_CONV_BF16X3=0 those of the others. */
 int32_t kxc_hip_gemm_f32(const float* a, const float* b, const float* c, float* y,
                          int64_t m, int64_t n, int64_t k, float alpha, float beta,
                          int32_t transB, int64_t c_len, void* stream);

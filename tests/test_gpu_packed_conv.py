@@ -1,6 +1,7 @@
 """Plan nodes on a packed filter (kxc_hip_plan_add_conv2d_packed): the three-part kernels for 3x3 stride-2 convolutions, with
 and without the second output, and for 7x7 stride-2 convolutions of three channels, with and without the column maxima, at the
-edges of their tiles, against float64; their values that are not finite; their filters."""
+edges of their tiles, against float64; their values that are not finite; their filters.  And single calls on a filter that
+they pack themselves."""
 import numpy as np
 import pytest
 import torch
@@ -195,3 +196,48 @@ def test_packed_filters_follow_their_weights(pkg, monkeypatch):
     node.check(node.run(again))
     again.close()
     assert pkg.conv2d_node_filter_bytes(node.desc, True) == 0
+
+
+@pytest.mark.parametrize("xs, o, k, stride, pad, residual, bias, relu", [
+    ((1, 16, 5, 6), 32, 5, 1, 2, False, True, True),        # one step
+    ((2, 50, 27, 27), 96, 5, 1, 2, True, True, True),       # channels short of a step, images meet inside a tile
+    ((3, 33, 20, 31), 64, 5, 2, 2, True, False, False),     # stride 2, an odd number of rows per phase
+    ((1, 20, 23, 21), 40, 7, 1, 3, False, True, True),
+    ((2, 10, 30, 30), 20, 7, 2, 0, True, True, True),       # no padding
+    ((2, 48, 15, 40), 130, 3, 1, 1, True, True, True),      # the second block of channels holds two
+    ((1, 35, 9, 14), 24, 3, 2, 2, False, True, False),
+    ((3, 96, 4, 5), 200, 1, 1, 0, True, True, True),        # images of 20 pixels: tiles across four of them, whole quads
+    ((2, 70, 5, 5), 33, 1, 1, 0, False, True, True),        # 25: pixel by pixel; six channels of a step of 64
+    ((4, 64, 13, 18), 64, 1, 2, 0, True, True, True),
+    ((1, 130, 8, 8), 32, 1, 1, 1, False, False, False),     # a padded 1x1 filter
+    ((2, 512, 6, 6), 256, 3, 1, 1, True, True, True),       # a reduction in parts
+    ((16, 64, 33, 36), 256, 1, 1, 0, True, True, True),     # a launch that fills the GPU
+])
+def test_single_convolution_on_a_packed_filter(pkg, monkeypatch, xs, o, k, stride, pad, residual, bias, relu):
+    rng = np.random.default_rng(sum(xs) + o + k)
+    n, c, h, w = xs
+    f32 = lambda s, scale=1.0: (rng.standard_normal(s) * scale).astype(np.float32)
+    oh, ow = (h + 2 * pad - k) // stride + 1, (w + 2 * pad - k) // stride + 1
+    x, wt, b = f32(xs), f32((o, c, k, k), (2 / (k * k * c)) ** 0.5), f32((o,)) if bias else None
+    res = f32((n, o, oh, ow)) if residual else None
+    gpu = lambda a: dev(a) if a is not None else None
+    run = lambda: host(pkg.conv2d(gpu(x), gpu(wt), gpu(b), gpu(res), stride, pad, 1, relu))
+    monkeypatch.setenv("KXC_HIP_CONV_BF16X3", "0")
+    assert "bf16x3" not in pkg.conv2d_variant(x.shape, wt.shape, stride, pad)
+    monkeypatch.setenv("KXC_HIP_CONV_WINOGRAD", "0")
+    monkeypatch.setenv("KXC_HIP_CONV_BF16X3", "1")
+    assert pkg.conv2d_variant(x.shape, wt.shape, stride, pad) == "mfma_k%dx%ds%d_bf16x3" % (k, k, stride)
+    first = run()
+    want = _want(x, wt, b, res, relu, stride, pad)
+    assert np.linalg.norm(first - want) <= (k * k * c + 16) ** 0.5 * 2.0 ** -23 * np.linalg.norm(want)
+    assert_bit_exact(run(), first, "second run")
+    wt *= 2                                                 # the filter is read by every call
+    want = _want(x, wt, b, res, relu, stride, pad)
+    assert np.linalg.norm(run() - want) <= (k * k * c + 16) ** 0.5 * 2.0 ** -23 * np.linalg.norm(want)
+    # values that are not finite
+    x[0, c - 1, h // 2, w // 2], x[n - 1, 0, 0, 0], wt[o - 1, c // 2, 0, 0] = np.inf, np.nan, -np.inf
+    want, got = _want(x, wt, b, res, False, stride, pad), run()
+    want = np.where(want > 0, want, 0.0) if relu else want
+    assert (np.isnan(got) == np.isnan(want)).all() and (got[np.isinf(want)] == want[np.isinf(want)]).all()
+    m = np.isfinite(want)
+    assert (np.abs(got[m] - want[m]) <= 1e-5 * np.maximum(np.abs(want[m]), 1.0)).all()
