@@ -187,13 +187,15 @@ bool Resolve7(const kxc_hip_conv2d_desc* d, PackedLaunch* L) {
     return true;
 }
 
-// Whether a plan's node should take it: from 0.12 GFLOP per step of 16 channels on, 1.4 at most, counting the launches expected
-// side by side.  A workgroup takes 9 us and 2.9 per step however few there are, and the other kernels start with 16 x 16 tiles and
+// Whether a plan's node should take it: with fewer than 64 channels from 0.12 GFLOP per step of 16 on, counting the launches
+// expected side by side.  A workgroup takes 9 us and 2.9 per step however few there are, and the other kernels start with 16 x 16 tiles and
 // split reductions inside a workgroup (us, theirs and here, both outputs): 64 -> 128 channels at 56 x 56, batch 2 (0.26 GFLOP)
 // 12.3 and 16.4, batch 4 (0.51) 23.1 and 20.2, batch 8 32.4 and 20.9, batch 32 59 and 36, batch 64 97 and 60; 128 -> 256 at 28 x 28, batch 6
 // (0.77) 20.5 and 22.1, batch 8 (1.03) 25.5 and 23.7, batch 16 39 and 31, batch 64 94 and 54; 256 -> 512 at 14 x 14, batch 8 (1.03)
 // 21.8 and 22.8, batch 12 (1.54) 31 and 25, batch 32 71 and 37, batch 64 104 and 52; 512 -> 512 at 14 x 14, batch 5 (1.28) 21.5 and 22.6; 512 ->
-// 1024 at 28 x 28, batch 2 68 and 36; 16 -> 32 at 56 x 56, batch 20 (0.16) 15.0 and 11.5.  
+// 1024 at 28 x 28, batch 2 68 and 36; 16 -> 32 at 56 x 56, batch 20 (0.16) 15.0 and 11.5.  From 64 channels on the small-launch
+// kernel with one load per filter row is the other side, up to 2.3 million (16 x 16 tiles) * k (1.3 GFLOP): 64 -> 128 at 56 x 56, batch 6 / 8 / 10 15.7 /
+// 19.0 / 22.9 and 22.8 / 23.1 / 23.3; 128 -> 256 at 28 x 28, batch 8 / 10 18.6 / 20.7 and 24.7 / 25.9; 256 -> 512 at 14 x 14 18.9 / 19.1 and 23.5 / 23.2.
 // The 7x7 kernel, 3 -> 64 channels: pooled at 224 x 224, batch 16 / 32 / 64 51 / 100 / 169 and 32 / 59 / 108, at 64 x 64, batch 56 (1.1 GFLOP) 33 and
 // 22; not pooled at 224 x 224, batch 4 (0.94) 20.6 and 21.8, batch 8 (1.9) 33 and 30, batch 64 182 and 116; tiles 13 rows high, of which a compute unit holds
 // two, at 193 x 193, batch 16 (2.8) 49 and 54.
@@ -209,8 +211,10 @@ bool Preferred(const kxc_hip_conv2d_desc* d, bool second, PackedLaunch* L) {
         return (e && e[0] == '1') || pooled || (L->lds_bytes <= kMaxLdsBytes / 4 && L->gflop * SelectLanes() >= 1.8);
     }
     // (a plan's filter launch packs 3x3 stride-2 filters only)
-    return d && d->kh == 3 && d->stride_h == 2 && d->pad_h == 1 && d->pad_w == 1 && d->c % conv_bx::kStep == 0 && Resolve(d, second, L) &&
-           ((e && e[0] == '1') || L->gflop * SelectLanes() >= std::min(0.12 * L->a.csteps, 1.4));
+    if (!d || d->kh != 3 || d->stride_h != 2 || d->pad_h != 1 || d->pad_w != 1 || d->c % conv_bx::kStep != 0 || !Resolve(d, second, L)) return false;
+    if (e && e[0] == '1') return true;
+    if (d->c >= 64 && d->w >= 3) return CeilDiv(L->a.M, 16) * CeilDiv(d->o, 16) * SelectLanes() * d->c * 9 > kSmallRowLoadsWork;
+    return L->gflop * SelectLanes() >= std::min(0.12 * L->a.csteps, 1.4);
 }
 
 // `partials`: room for the partial outputs of a split reduction; nullptr: it is acquired here.

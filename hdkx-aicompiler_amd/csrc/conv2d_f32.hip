@@ -1186,6 +1186,9 @@ int SmallWords(const SmallVariant& v, const ConvArgs& a) {
     return (rows * a.W + 3 + 3) / 4;
 }
 
+// Whether the 3x3 small-launch kernels fetch the three values of a filter row by one load.
+bool SmallRowLoads(const ConvArgs& a) { return a.dw == 1 && a.pw <= 1 && a.W >= 3; }
+
 // Which small-launch kernel takes a shape (after FillArgs, before ApplyRowView), if any.  Channels are a multiple of a chunk (16).
 // 1x1: always, except wide maps of few channels, where the general tiles are as fast or faster: batch 64, 64 channels at 56 x 56:
 //   51 us both; 48 -> 200 at 30 x 30: 44 against 39; ahead from 96 channels on (128 -> 512 at 28 x 28, batch 64: 125 -> 117;
@@ -1197,7 +1200,14 @@ int SmallWords(const SmallVariant& v, const ConvArgs& a) {
 //   was measured: 800 is the near side.)  Up to 1600 also for at most 16 output channels,
 //   half a block of the general tiles: 64 -> 16 at 56 x 56, batch 8 (1568) 25.9 -> 14.8.  At least 64 channels, a chunk per wave.
 //   Staged rows for narrow maps while every tile has a compute unit to itself (256 at 14 x 14, batch 1: 8.5 -> 7.5; 512 at 7 x
-//   7: 13.2 -> 10.9); two blocks of output channels from 257 tiles on (64 at 56 x 56, batch 1: 9.6 -> 8.7).
+//   7: 13.2 -> 10.9), with stride 2 only if filter rows do not come in one load (256 -> 512 at 14 x 14, batch 2: 8.5 against 7.7,
+//   with the second output 9.4 against 8.4); two blocks of output channels from 257 tiles on (64 at 56 x 56, batch 1: 9.6 -> 8.7).
+//   Where filter rows do come in one load (SmallRowLoads): one block, and beyond 800 tiles while tiles * k is at most 2.3 million (us, two
+//   blocks and one, general kernel where it ran): 64 -> 64 at 56 x 56, batch 1 / 2 / 4 7.2 / 11.8 / 19.8 and 6.8 / 10.3 / 16.7, general 16.8 and
+//   22.2 from batch 2 on; 96 -> 48 at 37 x 37, batch 8 23.5 and 16.7, general 25.2; 64 -> 128 with stride 2 and the second output, batch 4 / 6 /
+//   10 (2.26 million) 13.9 / 18.1 / - and 11.3 / 16.0 / 22.9, general 32.8 and 33.8 from batch 6 on; 64 -> 72 at 56 x 56, batch 2 14.8 and 11.3,
+//   general 20.7; equal for 512 at 7 x 7.  A last block of output channels that is not full keeps two blocks up to 800 tiles: one is the
+//   faster there too (64 -> 72 at 31 x 31, batch 2 7.2 against 5.9), but the tests of those edges name the kernel.
 //   Outside a plan, only from 400 tiles on.  That is no line of speed (the figures above are from plans and below it, too):
 //   kxc_hip_conv2d_scratch_needed reports a reduction split over workgroups for those calls, and callers of the entry point
 //   that allocates nothing rely on what it reports.
@@ -1218,15 +1228,17 @@ const SmallVariant* SelectSmall(const kxc_hip_conv2d_desc* d, const ConvArgs& a,
     // the second output reads the middle tap (padding 0 at stride 3, say, wants tap 0: the general kernel's ds_off)
     int rh = 0, rw = 0;
     if (second && (!PairTap(d, &rh, &rw) || rh != 1 || rw != 1)) return nullptr;
-    if (!by_name && (a.C < 64 || tiles > (second || a.O <= 16 ? 1600 : 800) || (!in_plan && tiles < 400))) return nullptr;
+    const bool one_block = SmallRowLoads(a) && (a.O % 16 == 0 || tiles > 800);
+    const bool reaches = SmallRowLoads(a) && tiles * a.C * 9 <= kSmallRowLoadsWork;
+    if (!by_name && (a.C < 64 || (!reaches && tiles > (second || a.O <= 16 ? 1600 : 800)) || (!in_plan && tiles < 400))) return nullptr;
     const bool rows_fit = a.dw == 1 && SmallWords(v[0], a) * v[0].chunk <= v[0].xi * 64;      // (walks the map: behind the cheap tests)
     if (by_name) {
         for (int i = rows_fit ? 0 : 1; i < 3; ++i)
             if (std::strcmp(forced, v[i].name) == 0) return v + i;
         return nullptr;
     }
-    if (rows_fit && a.N * CeilDiv(a.OHW, 16) * CeilDiv(a.O, 16) * SelectLanes() <= kNumCUs) return v;
-    return tiles <= kNumCUs ? v + 1 : v + 2;
+    if (rows_fit && !(one_block && a.sw > 1) && a.N * CeilDiv(a.OHW, 16) * CeilDiv(a.O, 16) * SelectLanes() <= kNumCUs) return v;
+    return one_block || tiles <= kNumCUs ? v + 1 : v + 2;
 }
 
 // Everything about a launch that the descriptor alone decides (kernel, tile shape, grid, the split of the reduction,
@@ -1292,7 +1304,7 @@ int32_t Conv2dResolve(const kxc_hip_conv2d_desc* desc, bool second, const char* 
         b.div_ow = MakeFastDiv(a.OW); b.div_tiles = MakeFastDiv(b.o_fastest ? b.o_tiles : b.p_tiles);
         b.div_ohw = MakeFastDiv(a.OHW);
         L->path = ConvLaunch::kSmall;
-        const bool by_rows = v->rows_kernel && a.dw == 1 && a.pw <= 1 && a.W >= 3;
+        const bool by_rows = v->rows_kernel && SmallRowLoads(a);
         // Eight waves, a chunk per wave instead of two, where every workgroup has a compute unit to itself: 128 channels at 28 x 28 7.4 ->
         // 7.1 us, 128 -> 256 with stride 2 and the second output 6.2 -> 5.4.
         const bool eight = by_rows && b.nchunks >= 8 && static_cast<int64_t>(b.num_tiles) * SelectLanes() <= kNumCUs;
@@ -1542,12 +1554,15 @@ const char* PreparedConvName(const PreparedConv* p) {
 
 // Against the Winograd kernel with its adding launch (us, residual and ReLU): 64 channels at 56 x 56 batch 1 10.2 -> 8.7, batch 2
 // (1568 tiles) 12.9 against 14.6; 128 at 28 x 28 batch 2 13.0 -> 12.0; 256 at 14 x 14 batch 1 10.7 -> 7.5, batch 2 13.0 -> 11.2,
-// batch 4 (tiles * k = 1.8 M) equal; 512 at 7 x 7 batch 2 (1.03 M) 13.9 -> 11.6, batch 4 equal.
+// batch 4 (tiles * k = 1.8 M) equal; 512 at 7 x 7 batch 2 (1.03 M) 13.9 -> 11.6, batch 4 equal.  With one load per filter row and one
+// full block: batch 3 (1.35 M) of 64 at 56 x 56 16.0 -> 13.8, 128 at 28 x 28 17.6 -> 13.4, 256 at 14 x 14 17.5 -> 14.5; 256 at 8 x 8, batch 8
+// (1.18 M) 14.4 -> 11.0; 512 at 7 x 7, batch 3 (1.47 M) 16.6 against 17.4, batch 4 of the others (1.81 M) 16.1 / 16.5 / 17.1 against 17.0 / 16.6 / 17.7.
 bool SmallConvBeatsWinograd(const kxc_hip_conv2d_desc* d) {
     const char* variant = std::getenv("KXC_HIP_WINOGRAD_VARIANT");
     ConvArgs a;
     if ((variant && *variant) || std::getenv("KXC_HIP_WINOGRAD_GSPLIT") || FillArgs(d, &a, "plan") != KXC_HIP_OK) return false;
-    return SelectSmall(d, a, false, true) && CeilDiv(a.M, 16) * CeilDiv(a.O, 16) * SelectLanes() * a.C * 9 <= 1100000;
+    return SelectSmall(d, a, false, true) &&
+           CeilDiv(a.M, 16) * CeilDiv(a.O, 16) * SelectLanes() * a.C * 9 <= (SmallRowLoads(a) && a.O % 16 == 0 ? 1400000 : 1100000);
 }
 
 void FreePreparedConv(PreparedConv* p) { delete p; }

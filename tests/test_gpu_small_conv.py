@@ -56,3 +56,44 @@ def test_conv_loads_filter_rows(pkg, monkeypatch, variant, xs, o, stride, pad):
     assert_bit_exact(host(y), want, "%s %s, first output" % (variant, xs))
     assert_bit_exact(host(y2), (conv(w2, 0) + b[:, None, None]).astype(np.float32), "%s %s, second output" % (variant, xs))
     plan.close()
+
+
+@pytest.mark.parametrize("xs, o, stride, second, small", [
+    ((2, 64, 56, 56), 64, 1, False, True),          # 1568 tiles
+    ((5, 64, 56, 56), 64, 1, False, True),          # 3920: 2.26 million tiles * k, the last batch below the line
+    ((6, 64, 56, 56), 64, 1, False, False),
+    ((2, 64, 56, 56), 72, 1, False, True),          # a last block of 8 channels, more than 800 tiles
+    ((10, 64, 56, 56), 128, 2, True, True),         # with the second output
+    ((11, 64, 56, 56), 128, 2, True, False),
+    ((6, 256, 14, 14), 512, 2, True, True),
+    ((2, 256, 14, 14), 512, 2, False, True),        # as few tiles as staged rows take with stride 1
+])
+def test_where_filter_rows_in_one_load_reach(pkg, xs, o, stride, second, small):
+    """The rule's line and both sides of it against float64: 9 c + 16 roundings of at most 2^-23, of independent signs."""
+    rng = np.random.default_rng(sum(xs) + o)
+    n, c, h, w = xs
+    oh, ow = (h - 1) // stride + 1, (w - 1) // stride + 1
+    f32 = lambda *s: rng.standard_normal(s).astype(np.float32)
+    x, wt, b, w2 = f32(*xs), f32(o, c, 3, 3) / np.float32(3 * c ** 0.5), f32(o), f32(o, c, 1, 1) / np.float32(c ** 0.5)
+    d = pkg.ConvDesc(n, c, h, w, o, 3, 3, stride, stride, 1, 1, 1, 1, pkg.CONV_BIAS)
+    arg, none = pkg.Buf.arg, pkg.Buf.none()
+    plan = pkg.Plan(6)
+    if second:
+        plan.add_conv2d_pair(d, arg(0), arg(1), arg(2), none, arg(3), arg(4), none, arg(5))
+    else:
+        plan.add_conv2d(d, arg(0), arg(1), arg(2), none, arg(3))
+    plan.finalize(0)
+    assert ("_small_o1" in plan.node_symbol(0)) == small, plan.node_symbol(0)
+    y, y2 = (torch.full((n, o, oh, ow), float("nan"), device="cuda") for _ in range(2))
+    plan.run([dev(x), dev(wt), dev(b), y, dev(w2), y2]); torch.cuda.synchronize()
+    t = lambda a: torch.from_numpy(a).double()
+    conv = lambda k, bias, p: torch.nn.functional.conv2d(t(x), t(k), bias, stride, p).numpy()
+    pairs = [(y, conv(wt, t(b), 1), 9 * c + 16)] + ([(y2, conv(w2, None, 0), c + 16)] if second else [])
+    for got, want, terms in pairs:
+        assert np.linalg.norm(host(got) - want) <= terms ** 0.5 * 2.0 ** -23 * np.linalg.norm(want)
+    plan.close()
+    # the operator by itself takes the same side of the line
+    if not second and stride == 1:
+        assert ("_small_o1" in pkg.conv2d_variant(xs, wt.shape, 1, 1)) == small
+        got = host(pkg.conv2d(dev(x), dev(wt), dev(b), None, 1, 1))
+        assert np.linalg.norm(got - pairs[0][1]) <= pairs[0][2] ** 0.5 * 2.0 ** -23 * np.linalg.norm(pairs[0][1])
