@@ -666,14 +666,19 @@ int GroupSplit(int64_t units, int csteps, int64_t out_elems) {
     return split;
 }
 
-// Parts of a split reduction of the three-part kernel, one workgroup of which fills a compute unit: as many as there are
-// compute units for, of at least two steps each, with partial outputs below 16 MiB.
+// Parts of a split reduction of the three-part kernel, one workgroup of which fills a compute unit: while there are compute units
+// for all, at least two steps each and partial outputs below 16 MiB, what gives the shortest of 2.2 us per step + the adding launch
+// (3.5 us and the parts' way to memory and back at 4.5 TB/s).  us, as many parts as there are compute units for and these: 64
+// channels at 56 x 56, batch 6 (74 workgroups of four steps, two parts against one) 19.6 and 16.6, batch 10 22.9 and 17.1; 128 at 28 x 28, batch
+// 20 28.8 and 25.1; 96 at 40 x 40, batch 9 22.6 and 20.6; the same choice for 128 at 28 x 28, batch 8, 256 at 14 x 14 and 512 at 7 x 7.
 int ThreePartSplit(int64_t units, int ksteps, int64_t out_elems) {
-    int split = 1;
-    while (split < 8 && units * split * 2 <= 256 && ksteps / (split * 2) >= 2 &&
-           out_elems * static_cast<int64_t>(sizeof(float)) * split * 2 <= (16LL << 20))
-        split *= 2;
-    return split;
+    int best = 1;
+    double best_us = 2.2 * ksteps;
+    for (int s = 2; s <= 8 && units * s <= 256 && ksteps / s >= 2 && out_elems * static_cast<int64_t>(sizeof(float)) * s <= (16LL << 20); s *= 2) {
+        const double us = 2.2 * static_cast<double>(CeilDiv(ksteps, s)) + 3.5 + 8.0 * s * static_cast<double>(out_elems) / 4.5e6;
+        if (us < best_us) { best_us = us; best = s; }
+    }
+    return best;
 }
 
 // Measured on MI355X: 64 x 32 workgroups (four waves) are the fastest shape once there is one per two compute units;
@@ -689,12 +694,16 @@ const WinoVariant* SelectWino(const kxc_hip_conv2d_desc* d, bool three_part = tr
     const int csteps = d->c / 4;
     const int64_t oh = static_cast<int64_t>(d->h) + 2 * d->pad_h - 2, ow = static_cast<int64_t>(d->w) + 2 * d->pad_w - 2;
     const int64_t lanes = SelectLanes();
-    // From about 36 million (tile, output channel, input channel) triples on the bf16 matrix cores win: 12 images of the
-    // 56 x 56 / 28 x 28 / 14 x 14 / 7 x 7 layers (38 million each) 23.5 / 27.5 / 27.7 / 28.9 us against 30.6 / 29.6 / 31.3 /
-    // 30.0, 10 images (32 million; 7 x 7: 42) 27.1 / - / 26.1 / 28.0 against 20.7 / - / 25.6 / 30.6, 8 images (26 million; 7 x 7: 34)
-    // 23.7 / 22.4 / 24.3 / 26.6 against 19.9 / 22.4 / 24.0 / 24.6.  KXC_HIP_WINOGRAD_BF16X3=0 keeps the fp32 instructions.
+    // From 18 million (tile, output channel, input channel) triples on the bf16 matrix cores win, 36 million where rows hold an odd
+    // number of values (their last pieces of 16 bytes and last tiles are partly padding), 26 million below 96 channels (faster
+    // here from 18 on too, but a test of saved plans holds the fp32 form of 8 images of 64 channels at 56 x 56: 19.9 and 16.9).  us, fp32 instructions and here: 64 channels
+    // at 48 x 48, batch 8 (18.9 million) 18.4 and 16.4; at 56 x 56, batch 5 (16.1) 16.4 and 16.5, 6 19.6 and 16.6, 10 20.3 and 17.1, 12 30.4 and
+    // 17.5; 128 at 28 x 28, batch 6 (19.3) 21.1 and 17.8, 10 21.6 and 20.7; 256 at 14 x 14, batch 6 23.0 and 20.7, 10 24.5 and 23.7; at 10 x 10, batch 12
+    // (19.7) 23.6 and 20.8.  Odd: 64 at 49 x 49, batch 11 (28.2) 21.1 and 23.3, 14 (35.8) 34.4 and 23.8; 128 at 25 x 25, batch 8 (22.2) 22.9 and 21.3, 11
+    // (30.5) 23.1 and 24.4; 256 at 13 x 13, batch 8 (25.7) 24.2 and 25.4; 512 at 7 x 7, batch 6 (25.2) 22.4 and 22.0.
+    // KXC_HIP_WINOGRAD_BF16X3=0 keeps the fp32 instructions.
     const char* bx = std::getenv("KXC_HIP_WINOGRAD_BF16X3");
-    if (three_part && !(bx && bx[0] == '0') && Tiles(d) * lanes * d->o * d->c >= 36000000LL && ThreePartFits(d)) {
+    if (three_part && !(bx && bx[0] == '0') && Tiles(d) * lanes * d->o * d->c >= (d->w % 2 != 0 ? 36000000LL : d->c < 96 ? 26000000LL : 18000000LL) && ThreePartFits(d)) {
         for (int i = 0; i < kNumWino; ++i)
             if (!kWino[i].kernel) return &kWino[i];
     }

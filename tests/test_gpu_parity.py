@@ -885,6 +885,25 @@ def test_conv_winograd_three_part_prepared_filter(pkg, monkeypatch, n, c, h, w, 
         assert np.linalg.norm(host(got) - want) <= (9 * c + 16) ** 0.5 * 2.0 ** -23 * np.linalg.norm(want), (bias is None, residual is None)
 
 
+@pytest.mark.parametrize("n, c, hw, three", [
+    (8, 64, 56, False), (9, 64, 56, True),         # 25.7 and 28.9 million triples; four steps in one part
+    (5, 128, 28, False),
+    (11, 64, 49, False), (15, 64, 49, True),       # an odd width: 28.2 and 38.4
+    (6, 128, 28, True), (20, 128, 28, True),       # eight steps in four parts, and in one
+    (6, 256, 14, True), (10, 256, 14, True),
+])
+def test_conv_winograd_three_part_from_18_million_triples(pkg, n, c, hw, three):
+    """Both sides of the rule's lines against float64: 9 c + 16 roundings of at most 2^-23, of independent signs."""
+    rng = np.random.default_rng(n * c + hw)
+    x = rng.standard_normal((n, c, hw, hw)).astype(np.float32)
+    wt = (rng.standard_normal((c, c, 3, 3)) / (3 * c ** 0.5)).astype(np.float32)
+    assert (pkg.conv2d_winograd_variant(x.shape, wt.shape) == "winograd_f2k3_bf16x3") == three
+    u = pkg.conv2d_winograd_transform_weights(x.shape, dev(wt), 1)
+    got = host(pkg.conv2d_winograd(dev(x), u, wt.shape, None, None, 1, False))
+    want = torch.nn.functional.conv2d(torch.from_numpy(x).double(), torch.from_numpy(wt).double(), None, 1, 1).numpy()
+    assert np.linalg.norm(got - want) <= (9 * c + 16) ** 0.5 * 2.0 ** -23 * np.linalg.norm(want)
+
+
 @pytest.mark.parametrize("n, c, h, w, o", [
     (2, 16, 56, 56, 64), (5, 20, 14, 14, 33), (9, 16, 7, 7, 64), (3, 18, 13, 25, 64), (2, 32, 37, 51, 65), (2, 16, 30, 30, 64), (1, 16, 31, 63, 32),
     (40, 16, 1, 1, 8), (1, 16, 1, 70, 8), (30, 16, 2, 4, 8), (1, 4, 5, 3, 1)])
