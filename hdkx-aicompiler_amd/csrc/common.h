@@ -178,10 +178,11 @@ int32_t LaunchPreparedPacked(const PreparedPacked* p, const float* x, const floa
                              float* y, const float* w2, const float* bias2, float* y2, hipStream_t stream);
 void FreePreparedPacked(PreparedPacked* p);
 // A single nn_conv2d by one of these kernels, its filter packed first: the kernel's name (nullptr: not for this shape), and the
-// call.  *launched = false, nothing enqueued: not for this shape, no scratch for the filter, or the stream does not order it.
+// call.  *launched = false, nothing enqueued: not for this shape (*preferred says), no scratch for the filter, or the stream does
+// not order it.
 const char* PackedOperatorName(const kxc_hip_conv2d_desc* desc);
 int32_t RunPackedOperator(const kxc_hip_conv2d_desc* desc, const float* x, const float* w, const float* bias, const float* residual, float* y,
-                          hipStream_t stream, bool* launched);
+                          hipStream_t stream, bool* launched, bool* preferred);
 
 // A single nn_conv2d by the three-part Winograd kernel, filter transform included (conv2d_wino_f32.hip): which shapes it is
 // for, and the call.  *launched = false, nothing enqueued: there is no scratch for the filter, or the stream does not order it.

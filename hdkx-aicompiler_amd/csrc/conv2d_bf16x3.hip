@@ -306,12 +306,13 @@ const char* PackedOperatorName(const kxc_hip_conv2d_desc* desc) {
 }
 
 int32_t RunPackedOperator(const kxc_hip_conv2d_desc* desc, const float* x, const float* w, const float* bias, const float* residual, float* y,
-                          hipStream_t stream, bool* launched) {
+                          hipStream_t stream, bool* launched, bool* preferred) {
     const char* const who = "kxc_hip_conv2d_nchw_f32";
     *launched = false;
     PackedLaunch L;
+    *preferred = OperatorPreferred(desc, &L);
     // (kernels meet in the scratch: one packs the filter, the convolution reads it, and its parts are added)
-    if (!OperatorPreferred(desc, &L) || !StreamOrdersScratch(stream)) return KXC_HIP_OK;
+    if (!*preferred || !StreamOrdersScratch(stream)) return KXC_HIP_OK;
     KXC_HIP_REQUIRE(x && w && y, "%s: NULL pointer", who);
     KXC_HIP_REQUIRE(!(desc->flags & KXC_HIP_CONV_BIAS) || bias, "%s: bias flag without bias", who);
     KXC_HIP_REQUIRE(!(desc->flags & KXC_HIP_CONV_RESIDUAL) || residual, "%s: residual flag without residual", who);

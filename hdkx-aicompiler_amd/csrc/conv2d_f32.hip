@@ -845,6 +845,7 @@ const Variant kVariants[] = {
     KXC_VARIANT(7, 7, 4, 1, 8, 1, 1, 8),   // 32 x 256, one chunk (3 input channels padded to 4)
     KXC_VARIANT(7, 7, 2, 1, 4, 1, 1, 12),  // 32 x 128
     KXC_VARIANT(7, 7, 4, 1, 4, 1, 1, 12),
+    KXC_VARIANT_KS(7, 7, 2, 1, 4, 1, 1, 12, 4),   // 32 x 128, split 4 ways: only where the reduction must not be split over workgroups
 };
 constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
 
@@ -918,8 +919,8 @@ bool Fits(const Variant& v, const ConvArgs& a, Choice* out, bool ds = false) {
     return true;
 }
 
-// Picks the MFMA variant for a shape, or leaves choice.v == nullptr for the direct kernel.  in_workgroup: 1x1 filters split their
-// reduction as deep over wave groups as 3x3 ones before they split it over workgroups.
+// Picks the MFMA variant for a shape, or leaves choice.v == nullptr for the direct kernel.  in_workgroup: for a launch that should
+// not, or must not, split its reduction over workgroups: it is split deeper over wave groups.
 void Select(const ConvArgs& real, int kh, int kw, Choice* choice, bool ds = false, bool in_workgroup = false) {
     choice->v = nullptr;
     // Fewer than 32 channels or pixels leave part of a 32 x 32 block empty, and the block still wins against one thread per
@@ -996,7 +997,15 @@ void Select(const ConvArgs& real, int kh, int kw, Choice* choice, bool ds = fals
                     // splits on 32 x 64 tiles from batch 1 to 16, at stride 2 (batch 8, 128 -> 256 channels at
                     // 28 x 28: 20.5 against 31.5 us) and at stride 1 (batch 1, 256 channels at 14 x 14: 12.6
                     // against 19.8 us with the adding kernel; batch 4, 512 channels at 7 x 7: 23.8 against 37.9)
-                    if (kh == 3) break;
+                    if (kh == 3 && !in_workgroup) break;
+                }
+            }
+            // (us, 32 x 256 tiles with whole reductions and here: 226 -> 161 channels at 26 x 33, one image 459 and 210; 232 -> 343 at
+            // 8 x 14, batch 19 479 and 216.  3x3 split deeper, as above: 370 -> 363 at 9 x 8, batch 17 74 and 45)
+            if (in_workgroup && kh == 7 && first_fit.v && first_waves < kEnoughWaves) {
+                for (int i = 0; i < kNumVariants; ++i) {
+                    Choice c;
+                    if (std::strcmp(kVariants[i].name, "mfma_k7x7_c2_o1x1_p4x1_ks4") == 0 && Fits(kVariants[i], a, &c, ds)) *choice = c;
                 }
             }
             // Every workgroup of a launch does the same work, so the launch takes as long as the compute unit with
@@ -1261,6 +1270,7 @@ struct ConvLaunch {
     int64_t total = 0;
     bool second = false;
     bool in_plan = false;
+    bool in_workgroup = false;
 };
 
 // small = false: without the small-launch kernels (operands that are not aligned for them).  in_workgroup: see Select.
@@ -1270,6 +1280,7 @@ int32_t Conv2dResolve(const kxc_hip_conv2d_desc* desc, bool second, const char* 
     if (int32_t rc = FillArgs(desc, &a, who)) return rc;
     L->second = second;
     L->in_plan = in_plan;
+    L->in_workgroup = in_workgroup;
     L->desc = *desc;
     L->kh = desc->kh; L->kw = desc->kw;
     L->total = static_cast<int64_t>(a.N) * a.O * a.OHW;
@@ -1409,9 +1420,10 @@ struct SecondOutput {
 };
 
 // no_alloc: the partial sums of a split reduction go to the file-scope scratch array instead of the grow-only
-// per-stream buffer, and a launch that would need more is refused.
+// per-stream buffer, and a launch that would need more is refused.  whole: the reduction stays in one piece where the
+// stream does not order the buffer's users (it stands in for a call that keeps its filter in that buffer).
 int32_t Conv2dLaunch(const ConvLaunch& L, const char* who, const float* x, const float* w, const float* bias,
-                     const float* residual, float* y, void* stream, bool no_alloc, const SecondOutput* second) {
+                     const float* residual, float* y, void* stream, bool no_alloc, const SecondOutput* second, bool whole = false) {
     if (L.path == ConvLaunch::kEmpty) return KXC_HIP_OK;
     KXC_HIP_REQUIRE(x && w && y, "%s: NULL pointer", who);
     KXC_HIP_REQUIRE(!(L.a.flags & KXC_HIP_CONV_BIAS) || bias, "%s: bias flag without bias", who);
@@ -1438,7 +1450,7 @@ int32_t Conv2dLaunch(const ConvLaunch& L, const char* who, const float* x, const
         if (((reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(second ? second->w2 : w)) & 15u) != 0) {
             ConvLaunch other;       // weights are read in 16-byte words
             if (int32_t rc = Conv2dResolve(&L.desc, L.second, who, &other, L.in_plan, false)) return rc;
-            return Conv2dLaunch(other, who, x, w, bias, residual, y, stream, no_alloc, second);
+            return Conv2dLaunch(other, who, x, w, bias, residual, y, stream, no_alloc, second, whole);
         }
         conv_small::Args b = L.sm;
         b.x = x; b.w = w; b.bias = bias; b.res = residual; b.y = y;
@@ -1461,17 +1473,20 @@ int32_t Conv2dLaunch(const ConvLaunch& L, const char* who, const float* x, const
             if (int32_t rc = NoAllocScratch(&a.partial)) return rc;
         } else {
             // Launches that can do without the buffer of the stream's handle do so where the stream does not order its users:
-            // one thread per output, without scratch, is what these filters and shapes are compared with.  For the others
+            // one thread per output, without scratch, is what these filters and shapes are compared with.  So do calls that stand in
+            // for one on a packed or transformed filter: their eager neighbours keep it in that buffer.  For the others
             // a reduction in one piece would take up to five times as long (kxc_hip.h says what their graphs need); a
             // plan's own graph is replayed on its capture stream.  1x1 launches that take two parts for speed
-            // (697 -> 222 channels at 7 x 188, batch 3) have a kernel that splits over wave groups only.
+            // (697 -> 222 channels at 7 x 188, batch 3) have a kernel that splits over wave groups only; most that stand in have one
+            // as well (us, split into the buffer and here: 226 -> 161 at 26 x 33, 7x7 70 and 210, 232 -> 343 at 8 x 14, 7x7, batch 19
+            // 248 and 216, 370 -> 363 at 9 x 8, 3x3, batch 17 41 and 45).
             const bool ordered = L.in_plan || StreamOrdersScratch(s);
-            if (!ordered && L.kh == 1) {
+            if (!ordered && (L.kh == 1 || whole) && !L.in_workgroup) {
                 ConvLaunch other;
                 if (int32_t rc = Conv2dResolve(&L.desc, L.second, who, &other, false, false, true)) return rc;
-                if (other.scratch_bytes == 0) return Conv2dLaunch(other, who, x, w, bias, residual, y, stream, false, second);
+                if (other.scratch_bytes == 0 || whole) return Conv2dLaunch(other, who, x, w, bias, residual, y, stream, false, second, whole);
             }
-            bool split = ordered || !(a.O < 32 || a.M < 32 || L.kh == 5);
+            bool split = ordered || !(whole || a.O < 32 || a.M < 32 || L.kh == 5);
             if (split)
                 if (int32_t rc = AcquireSplitScratch(s, L.scratch_bytes, &lease, &split)) return rc;
             a.partial = lease.ptr;
@@ -1505,6 +1520,7 @@ int32_t Conv2dRun(const kxc_hip_conv2d_desc* desc, const float* x, const float* 
                   const float* residual, float* y, void* stream, bool no_alloc, const SecondOutput* second = nullptr) {
     const char* const who = second ? "kxc_hip_conv2d_pair_nchw_f32" : no_alloc ? "kxc_hip_conv2d_nchw_f32_noalloc" : "kxc_hip_conv2d_nchw_f32";
     ConvLaunch L;
+    bool stands_in = false;
     // (the entry point that allocates nothing has no scratch for a transformed filter)
     if (!second && !no_alloc && desc && WinogradOperatorPreferred(desc)) {
         KXC_HIP_REQUIRE(x && w && y, "%s: NULL pointer", who);
@@ -1513,14 +1529,15 @@ int32_t Conv2dRun(const kxc_hip_conv2d_desc* desc, const float* x, const float* 
         bool launched = false;
         if (int32_t rc = RunWinogradOperator(desc, x, w, bias, residual, y, ResolveStream(stream), &launched)) return rc;
         if (launched) return KXC_HIP_OK;
+        stands_in = true;
     }
-    if (!second && !no_alloc && desc) {
+    if (!second && !no_alloc && desc && !stands_in) {
         bool launched = false;
-        if (int32_t rc = RunPackedOperator(desc, x, w, bias, residual, y, ResolveStream(stream), &launched)) return rc;
+        if (int32_t rc = RunPackedOperator(desc, x, w, bias, residual, y, ResolveStream(stream), &launched, &stands_in)) return rc;
         if (launched) return KXC_HIP_OK;
     }
     if (int32_t rc = Conv2dResolve(desc, second != nullptr, who, &L)) return rc;
-    return Conv2dLaunch(L, who, x, w, bias, residual, y, stream, no_alloc, second);
+    return Conv2dLaunch(L, who, x, w, bias, residual, y, stream, no_alloc, second, stands_in);
 }
 
 }  // namespace

@@ -180,7 +180,7 @@ typedef struct kxc_hip_conv2d_desc {
  * calls on one stream are safe from any thread.  While the stream is being captured, and on hipStreamPerThread, those large
  * calls, 5x5 filters, calls of fewer than 32 output channels or pixels and 1x1 filters whose reduction can be split
  * over the waves of a workgroup instead take a kernel that needs no buffer (the same bits whether or not an earlier call grew
- * one).  Other launches with a split reduction use the buffer there too:
+ * one; small 7x7 calls take up to three times as long there as with the buffer).  Other launches with a split reduction use the buffer there too:
  * their graph must be replayed on the stream it was captured on (or with nothing else running on that stream's buffer),
  * and threads must not run them on hipStreamPerThread at the same time.  A buffer that cannot be had (a first call under
  * capture, no memory, more than KXC_HIP_SCRATCH_MAX bytes where the environment sets it) is done without, never an error. */

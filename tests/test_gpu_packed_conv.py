@@ -2,6 +2,9 @@
 and without the second output, and for 7x7 stride-2 convolutions of three channels, with and without the column maxima, at the
 edges of their tiles, against float64; their values that are not finite; their filters.  And single calls on a filter that
 they pack themselves."""
+import ctypes
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -241,3 +244,97 @@ def test_single_convolution_on_a_packed_filter(pkg, monkeypatch, xs, o, k, strid
     assert (np.isnan(got) == np.isnan(want)).all() and (got[np.isinf(want)] == want[np.isinf(want)]).all()
     m = np.isfinite(want)
     assert (np.abs(got[m] - want[m]) <= 1e-5 * np.maximum(np.abs(want[m]), 1.0)).all()
+
+
+def _filters(pkg, xs, o, k, count, seed):
+    """Input, `count` filters of one shape and what a stride-1 call gives for each in float64; the tolerance of a float32 sum."""
+    rng = np.random.default_rng(seed)
+    n, c, h, w = xs
+    x = rng.standard_normal(xs).astype(np.float32)
+    wt = [(rng.standard_normal((o, c, k, k)) * (2 / (k * k * c)) ** 0.5).astype(np.float32) for _ in range(count)]
+    want = [_want(x, v, None, None, False, 1, k // 2) for v in wt]
+    close = lambda got, i: np.linalg.norm(host(got) - want[i]) <= (k * k * c + 16) ** 0.5 * 2.0 ** -23 * np.linalg.norm(want[i])
+    return dev(x), [dev(v) for v in wt], want[0].shape, close
+
+
+@pytest.mark.parametrize("xs, o, k, variant", [
+    ((1, 226, 26, 33), 161, 7, "mfma_k7x7s1_bf16x3"),       # 113 chunks of the reduction on four wave groups
+    ((19, 232, 8, 14), 343, 7, "mfma_k7x7s1_bf16x3"), ((17, 370, 9, 8), 363, 3, "mfma_k3x3s1_bf16x3"), ((18, 124, 53, 7), 100, 5, "mfma_k5x5s1_bf16x3"),
+    ((2, 52, 24, 22), 184, 1, "mfma_k1x1s1_bf16x3"),        # too few channels for the kernel that splits over wave groups
+    ((13, 731, 37, 22), 94, 3, "winograd_f2k3_bf16x3")])
+def test_calls_with_a_filter_in_the_scratch_keep_it_out_of_graphs(pkg, monkeypatch, xs, o, k, variant):
+    """The kernels that take these shapes' place under capture and on hipStreamPerThread would split their reductions into the very
+    buffer that the eager calls keep their filters in: a graph, captured before any call, replays on another stream beside eager
+    calls with another filter on the capture stream; captured again after those, and on hipStreamPerThread, the bits are the same."""
+    x, w, shape, close = _filters(pkg, xs, o, k, 2, sum(xs) + o)
+    assert pkg.conv2d_variant(xs, tuple(w[0].shape), 1, k // 2) == variant
+    need = ctypes.c_size_t(0)
+    assert pkg.lib().kxc_hip_conv2d_scratch_needed(ctypes.byref(pkg.conv_desc(xs, tuple(w[0].shape), 1, k // 2)), ctypes.byref(need)) == 0
+    assert need.value > 0
+    y = [torch.empty(shape, device="cuda") for _ in range(3)]
+    call = lambda i, out: pkg.conv2d(x, w[i], None, None, 1, k // 2, out=out)
+    capture, other = torch.cuda.Stream(), torch.cuda.Stream()
+    graphs = [torch.cuda.CUDAGraph() for _ in range(2)]
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graphs[0], stream=capture):
+        call(0, y[0])
+    for replay in range(5):
+        y[0].zero_(); y[1].zero_()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(other):
+            graphs[0].replay()
+        with torch.cuda.stream(capture):
+            call(1, y[1])
+        torch.cuda.synchronize()
+        if replay == 0:
+            first, eager = y[0].clone(), y[1].clone()
+            assert close(first, 0) and close(eager, 1)
+        assert torch.equal(y[0], first) and torch.equal(y[1], eager), "replay %d" % replay
+    with torch.cuda.graph(graphs[1], stream=capture):
+        call(0, y[2])
+    graphs[1].replay()
+    torch.cuda.synchronize()
+    assert torch.equal(y[2], first)
+    monkeypatch.setattr(pkg.hipabi, "_stream", lambda: ctypes.c_void_p(2))        # hipStreamPerThread
+    outs = [[torch.zeros(shape, device="cuda") for _ in range(3)] for _ in range(2)]
+    torch.cuda.synchronize()
+    # (a thread waits for its stream itself: nothing does once it has ended)
+    _in_threads(2, lambda i: ([call(0, out) for out in outs[i]], torch.cuda.synchronize()))
+    assert all(torch.equal(out, first) for per_thread in outs for out in per_thread)
+
+
+def _in_threads(count, f):
+    errors = []
+
+    def body(i):
+        try:
+            f(i)
+        except Exception as e:      # (an exception of a thread would pass unseen)
+            errors.append(e)
+    threads = [threading.Thread(target=body, args=(i,)) for i in range(count)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors
+
+
+@pytest.mark.parametrize("xs, o, k", [((8, 64, 27, 27), 96, 5), ((32, 128, 28, 28), 512, 1)])
+def test_packed_calls_from_threads_and_streams(pkg, xs, o, k):
+    """Eager calls with filters of their own, four threads on two streams at once: the buffer for a call's packed filter (and, at
+    5x5 here, its partial sums) is kept per stream, whose order keeps the calls of its two threads apart."""
+    x, w, shape, close = _filters(pkg, xs, o, k, 4, 78)
+    assert pkg.conv2d_variant(xs, tuple(w[0].shape), 1, k // 2) == "mfma_k%dx%ds1_bf16x3" % (k, k)
+    want = [pkg.conv2d(x, v, None, None, 1, k // 2) for v in w]
+    assert all(close(y, i) for i, y in enumerate(want))
+    out = [[torch.empty(shape, device="cuda") for _ in range(6)] for _ in w]
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+
+    def calls(i):
+        with torch.cuda.stream(streams[i % 2]):
+            for y in out[i]:
+                pkg.conv2d(x, w[i], None, None, 1, k // 2, out=y)
+    _in_threads(4, calls)
+    torch.cuda.synchronize()
+    assert all(torch.equal(y, want[i]) for i in range(4) for y in out[i])
