@@ -7,8 +7,9 @@
 // under bf16's smallest step, 2^-133 (the matrix instructions take subnormal parts as they are), and h + m + l is off by
 // at most 2^-134, which is all of an x of that size.  Multiplying operands by 2^16 while they are split, and sums by 2^-32,
 // keeps those bits as well and was not taken: 300 x 1000 x 2048 15.4 -> 16.6 us, 64 x 1000 x 512 4.7 -> 5.0 (with
-// v_dot2_f32_bf16 in the place of each unpacking and subtraction, which is exact, 16.8 and 4.9); KXC_HIP_GEMM_BF16X3=0,
-// KXC_HIP_WINOGRAD_BF16X3=0 and KXC_HIP_CONV_BF16X3=0 keep the fp32 instructions for callers whose operands are that small.
+// v_dot2_f32_bf16 in the place of each unpacking and subtraction, which is exact, 16.8 and 4.9); KXC_HIP_GEMM_BF16X3=0 and
+// KXC_HIP_WINOGRAD_BF16X3=0 keep the fp32 instructions for callers whose operands are that small, in products and in all convolutions
+// (KXC_HIP_CONV_BF16X3=0: in those that are no Winograd launches).
 // A product of two such numbers is nine bf16 products, each exact in fp32; the three that are left out (m*l', l*m', l*l')
 // add up to at most 2^-24 |x x'|, what rounding the product to fp32 may lose as well.  The six others are accumulated in
 // fp32 by v_mfma_f32_32x32x16_bf16, smallest first.  Measured on random dot products of 64, 576 and 4608 terms against a

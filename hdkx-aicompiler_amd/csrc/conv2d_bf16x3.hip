@@ -187,6 +187,15 @@ bool Resolve7(const kxc_hip_conv2d_desc* d, PackedLaunch* L) {
     return true;
 }
 
+// What the environment says: '1' these kernels wherever they cover a launch, '0' none of them, 0 nothing.  KXC_HIP_WINOGRAD_BF16X3=0 keeps
+// every convolution on the fp32 instructions, as it did when no other kernel had three-part operands.
+char Switch() {
+    const char* e = std::getenv("KXC_HIP_CONV_BF16X3");
+    if (e && (e[0] == '0' || e[0] == '1')) return e[0];
+    const char* w = std::getenv("KXC_HIP_WINOGRAD_BF16X3");
+    return w && w[0] == '0' ? '0' : 0;
+}
+
 // Whether a plan's node should take it: with fewer than 64 channels from 0.12 GFLOP per step of 16 on, counting the launches
 // expected side by side.  A workgroup takes 9 us and 2.9 per step however few there are, and the other kernels start with 16 x 16 tiles and
 // split reductions inside a workgroup (us, theirs and here, both outputs): 64 -> 128 channels at 56 x 56, batch 2 (0.26 GFLOP)
@@ -199,20 +208,19 @@ bool Resolve7(const kxc_hip_conv2d_desc* d, PackedLaunch* L) {
 // The 7x7 kernel, 3 -> 64 channels: pooled at 224 x 224, batch 16 / 32 / 64 51 / 100 / 169 and 32 / 59 / 108, at 64 x 64, batch 56 (1.1 GFLOP) 33 and
 // 22; not pooled at 224 x 224, batch 4 (0.94) 20.6 and 21.8, batch 8 (1.9) 33 and 30, batch 64 182 and 116; tiles 13 rows high, of which a compute unit holds
 // two, at 193 x 193, batch 16 (2.8) 49 and 54.
-// KXC_HIP_CONV_BF16X3=0 keeps the kernels on the fp32 instructions (=1 takes these wherever they cover the launch), and so
-// does KXC_HIP_CONV_VARIANT, which names one of theirs.
+// KXC_HIP_CONV_VARIANT, which names one of the other kernels, keeps those as well.
 bool Preferred(const kxc_hip_conv2d_desc* d, bool second, PackedLaunch* L) {
-    const char* e = std::getenv("KXC_HIP_CONV_BF16X3");
+    const char e = Switch();
     const char* variant = std::getenv("KXC_HIP_CONV_VARIANT");
-    if ((e && e[0] == '0') || (variant && *variant)) return false;
+    if (e == '0' || (variant && *variant)) return false;
     if (!second && Resolve7(d, L)) {
         // Pooled rows: always.  Others: four workgroups to a compute unit (tiles that are few rows high) and work for them.
         const bool pooled = (d->flags & KXC_HIP_CONV_HPOOL) != 0;
-        return (e && e[0] == '1') || pooled || (L->lds_bytes <= kMaxLdsBytes / 4 && L->gflop * SelectLanes() >= 1.8);
+        return e == '1' || pooled || (L->lds_bytes <= kMaxLdsBytes / 4 && L->gflop * SelectLanes() >= 1.8);
     }
     // (a plan's filter launch packs 3x3 stride-2 filters only)
     if (!d || d->kh != 3 || d->stride_h != 2 || d->pad_h != 1 || d->pad_w != 1 || d->c % conv_bx::kStep != 0 || !Resolve(d, second, L)) return false;
-    if (e && e[0] == '1') return true;
+    if (e == '1') return true;
     if (d->c >= 64 && d->w >= 3) return CeilDiv(L->a.M, 16) * CeilDiv(d->o, 16) * SelectLanes() * d->c * 9 > kSmallRowLoadsWork;
     return L->gflop * SelectLanes() >= std::min(0.12 * L->a.csteps, 1.4);
 }
@@ -269,8 +277,9 @@ bool OperatorPreferred(const kxc_hip_conv2d_desc* d, PackedLaunch* L) {
     using namespace conv_bx;
     const int K = d->kh, S = d->stride_h;
     if (K != d->kw || S != d->stride_w || d->n <= 0 || d->c <= 0 || d->o <= 0 || (S != 1 && S != 2) || K > 7) return false;
-    const char* e = std::getenv("KXC_HIP_CONV_BF16X3");
-    if (!(e && e[0] == '1')) {
+    const char e = Switch();
+    if (e == '0') return false;
+    if (e != '1') {
         // (3x3, stride 2: single calls agree with the outputs of kxc_hip_conv2d_pair_nchw_f32, which packs nothing.  Stride 1: Winograd
         // takes large ones; half of a block of 128 output channels empty is no gain)
         if (K == 3 && (S == 2 || d->o < 96)) return false;
@@ -289,8 +298,6 @@ bool OperatorPreferred(const kxc_hip_conv2d_desc* d, PackedLaunch* L) {
         const double adding = split > 1 ? 5 + 2.0 * split * out_bytes / 4.5e6 : 0;
         const double compute = 0.29 * steps * static_cast<double>(CeilDiv(csteps, split)) * load;
         if (10 + (K == 1 ? compute + memory : std::max(compute, memory)) + adding >= others) return false;
-        const char* w = K == 3 ? std::getenv("KXC_HIP_WINOGRAD_BF16X3") : nullptr;      // (it says so for all large 3x3 stride-1 convolutions)
-        if ((e && e[0] == '0') || (w && w[0] == '0')) return false;
     }
     const char* variant = std::getenv("KXC_HIP_CONV_VARIANT");
     return !(variant && *variant) && Resolve(d, false, L) && L->filter_bytes <= (32u << 20);      // (bounds the scratch kept per stream)

@@ -173,7 +173,8 @@ typedef struct kxc_hip_conv2d_desc {
  *
  * Large calls of other filters (..._variant says "..._bf16x3") run on the bf16 matrix cores with every operand as three bf16
  * parts: exact from 2^-109 on, below it an operand is off by at most 2^-134; sums that are not finite are evaluated by the
- * definition.  KXC_HIP_CONV_BF16X3=0 keeps the fp32 instructions.
+ * definition.  KXC_HIP_CONV_BF16X3=0 keeps the fp32 instructions, and so does KXC_HIP_WINOGRAD_BF16X3=0, which keeps them in every
+ * convolution, unless KXC_HIP_CONV_BF16X3=1 asks for these kernels.
  *
  * Scratch.  A launch that splits its reduction over workgroups, and a large call that transforms or packs its filter first
  * (..._variant says "winograd_..." or "..._bf16x3"), keep intermediate values in a buffer that the library holds per (device, stream handle):
@@ -296,8 +297,8 @@ int32_t kxc_hip_global_avg_pool2d_f32(const float* x, float* y, int64_t n, int64
  * c may be NULL (nn_dense); c_len is n or 1.  fp32 sums in an order of the kernel's own (the CPU loop's below 2^15
  * multiplies, unless transB = 1 and k is a multiple of 32).  Products of more than four rows run on the bf16 matrix cores, every operand as three bf16
  * parts: exact from 2^-109 on, below it an operand is off by at most 2^-134; KXC_HIP_GEMM_BF16X3=0 in the environment keeps
- * the fp32 instructions, KXC_HIP_WINOGRAD_BF16X3=0 those of the convolutions (large 3x3 stride-1 ones),
- * KXC_HIP_CONV_BF16X3=0 those of the others. */
+ * the fp32 instructions, KXC_HIP_WINOGRAD_BF16X3=0 those of all convolutions (KXC_HIP_CONV_BF16X3=0: of those that are no
+ * Winograd launches). */
 int32_t kxc_hip_gemm_f32(const float* a, const float* b, const float* c, float* y,
                          int64_t m, int64_t n, int64_t k, float alpha, float beta,
                          int32_t transB, int64_t c_len, void* stream);
