@@ -27,19 +27,19 @@ struct PackedLaunch {
     size_t scratch_bytes = 0;
 };
 
-// Rows of a row phase that a workgroup's pixels touch at most.  Where a tile starts within an image repeats after
-// OHW / gcd(OHW, kPix) tiles.
-int64_t MaxRows(const conv_bx::Args& a, int extra) {
-    int64_t rem = a.OHW, gcd = conv_bx::kPix;
-    while (rem != 0) { const int64_t r = gcd % rem; gcd = rem; rem = r; }
-    const int64_t tiles = std::min<int64_t>(CeilDiv(a.M, conv_bx::kPix), a.OHW / gcd);
-    int64_t best = 0;
-    for (int64_t t = 0; t < tiles; ++t) {
-        const int64_t m0 = t * conv_bx::kPix, ml = std::min<int64_t>(m0 + conv_bx::kPix, a.M) - 1;
-        const int64_t q0 = m0 / a.OHW * a.Hq + m0 % a.OHW / a.OW, q1 = ml / a.OHW * a.Hq + ml % a.OHW / a.OW;
-        best = std::max(best, q1 - q0 + extra + 1);
-    }
-    return best;
+// How far `pix` neighbouring pixels (flattened over n, oh, ow) that start at a multiple of pix reach at most: `row` for every step to
+// the next output row and `image` for every step to the next image.  Within an image, where tiles start in a row repeats after
+// at most OW tiles; where the border of two images lies in a tile repeats after at most pix images.
+int32_t TileReach(int32_t N, int32_t OHW, int32_t OW, int32_t pix, int32_t row, int32_t image) {
+    const uint32_t p = static_cast<uint32_t>(pix), ow = static_cast<uint32_t>(OW), ohw = static_cast<uint32_t>(OHW), M = static_cast<uint32_t>(N) * ohw;
+    uint32_t best = 0;
+    auto tile = [&](uint32_t m0) {
+        const uint32_t last = std::min(p, M - m0) - 1;
+        best = std::max(best, (m0 % ow + last) / ow * static_cast<uint32_t>(row) + (m0 % ohw + last) / ohw * static_cast<uint32_t>(image));
+    };
+    for (uint32_t t = 0; t < ow && t * p < M; ++t) tile(t * p);
+    for (uint32_t n = 1; n < static_cast<uint32_t>(N) && n <= p; ++n) tile(n * ohw / p * p);
+    return static_cast<int32_t>(best);
 }
 
 // Parts of a reduction, while all of them together are at most one workgroup per compute unit: what gives the shortest of
@@ -98,8 +98,10 @@ bool Resolve(const kxc_hip_conv2d_desc* d, bool second, PackedLaunch* L) {
     a.Hq = a.OH + (K - 1) / S;
     a.w4 = (a.W + 3) / 4;
     if (K > 1) {
-        const int64_t rows = MaxRows(a, (K - 1) / S);
-        if (a.W > 4 * kPlane || 2 * rows * a.w4 > 64 * kProducers * kUnits) return false;
+        // (every call whose cost asks for the kernel comes here: wide maps go before the tiles are walked)
+        if (a.W > 4 * kPlane || ((K - 1) / S + 1) * (a.OW + K - 1) > kPlane) return false;
+        const int64_t rows = TileReach(a.N, a.OHW, a.OW, kPix, 1, a.Hq - a.OH) + (K - 1) / S + 1;
+        if (2 * rows * a.w4 > 64 * kProducers * kUnits) return false;
         // Stride 2: even columns, odd ones behind them.  Where it fits, a row pitch that continues the banks of a row's last pixel
         // with the next row's first one (a lane reads 16 bytes: 16 positions go through all banks).
         a.hp = std::max(a.OW + (K - 1) / 2, (a.W - 1 + a.pw) / 2 + 1);
@@ -159,15 +161,11 @@ bool Resolve7(const kxc_hip_conv2d_desc* d, PackedLaunch* L) {
     a.N = d->n; a.H = d->h; a.W = d->w; a.O = d->o; a.OH = static_cast<int32_t>(OH); a.OW = static_cast<int32_t>(OW);
     a.OHW = a.OH * a.OW; a.HW = a.H * a.W; a.M = static_cast<int32_t>(M); a.ph = d->pad_h; a.pw = d->pad_w;
     a.Hp = static_cast<int32_t>(Hp); a.PW = a.OW / 2;
-    int64_t rows = 0, rem = a.OHW, gcd = kPix;        // (where a tile starts within an image repeats after OHW / gcd(OHW, kPix) tiles)
-    while (rem != 0) { const int64_t r = gcd % rem; gcd = rem; rem = r; }
-    for (int64_t t = 0; t < std::min<int64_t>(CeilDiv(M, kPix), a.OHW / gcd); ++t) {
-        const int64_t m0 = t * kPix, ml = std::min<int64_t>(m0 + kPix, M) - 1;
-        rows = std::max(rows, (ml / a.OHW - m0 / a.OHW) * Hp + 2 * (ml % a.OHW / OW - m0 % a.OHW / OW) + kK);
-    }
-    a.row_max = static_cast<int32_t>(rows);
     const int pitch = OW + 3 <= 64 ? 64 : 120;      // (the last pixel's window takes four words; three parts within the reach of a ds_read2)
-    if (OW + 3 > pitch || LdsBytes(rows, pitch) > kMaxLdsBytes / 2) return false;
+    if (OW + 3 > pitch) return false;
+    const int64_t rows = TileReach(a.N, a.OHW, a.OW, kPix, 2, a.Hp - 2 * a.OH) + kK;
+    a.row_max = static_cast<int32_t>(rows);
+    if (LdsBytes(rows, pitch) > kMaxLdsBytes / 2) return false;
     a.o_tiles = static_cast<int32_t>(CeilDiv(a.O, kOut));
     const int64_t units = CeilDiv(M, kPix) * a.o_tiles;
     if (units >= (1LL << 30)) return false;
@@ -187,13 +185,15 @@ bool Resolve7(const kxc_hip_conv2d_desc* d, PackedLaunch* L) {
     return true;
 }
 
-// What the environment says: '1' these kernels wherever they cover a launch, '0' none of them, 0 nothing.  KXC_HIP_WINOGRAD_BF16X3=0 keeps
-// every convolution on the fp32 instructions, as it did when no other kernel had three-part operands.
-char Switch() {
+// Whether to take a kernel that the rule for its launch does or does not ask for.  KXC_HIP_CONV_BF16X3=1: wherever it covers the launch,
+// =0: nowhere.  KXC_HIP_WINOGRAD_BF16X3=0 keeps every convolution on the fp32 instructions, as it did when no other kernel had
+// three-part operands.
+bool Switched(bool by_rule) {
     const char* e = std::getenv("KXC_HIP_CONV_BF16X3");
-    if (e && (e[0] == '0' || e[0] == '1')) return e[0];
+    if (e && (e[0] == '0' || e[0] == '1')) return e[0] == '1';
+    if (!by_rule) return false;
     const char* w = std::getenv("KXC_HIP_WINOGRAD_BF16X3");
-    return w && w[0] == '0' ? '0' : 0;
+    return !(w && w[0] == '0');
 }
 
 // Whether a plan's node should take it: with fewer than 64 channels from 0.12 GFLOP per step of 16 on, counting the launches
@@ -210,19 +210,17 @@ char Switch() {
 // two, at 193 x 193, batch 16 (2.8) 49 and 54.
 // KXC_HIP_CONV_VARIANT, which names one of the other kernels, keeps those as well.
 bool Preferred(const kxc_hip_conv2d_desc* d, bool second, PackedLaunch* L) {
-    const char e = Switch();
     const char* variant = std::getenv("KXC_HIP_CONV_VARIANT");
-    if (e == '0' || (variant && *variant)) return false;
+    if (variant && *variant) return false;
     if (!second && Resolve7(d, L)) {
         // Pooled rows: always.  Others: four workgroups to a compute unit (tiles that are few rows high) and work for them.
         const bool pooled = (d->flags & KXC_HIP_CONV_HPOOL) != 0;
-        return e == '1' || pooled || (L->lds_bytes <= kMaxLdsBytes / 4 && L->gflop * SelectLanes() >= 1.8);
+        return Switched(pooled || (L->lds_bytes <= kMaxLdsBytes / 4 && L->gflop * SelectLanes() >= 1.8));
     }
     // (a plan's filter launch packs 3x3 stride-2 filters only)
     if (!d || d->kh != 3 || d->stride_h != 2 || d->pad_h != 1 || d->pad_w != 1 || d->c % conv_bx::kStep != 0 || !Resolve(d, second, L)) return false;
-    if (e == '1') return true;
-    if (d->c >= 64 && d->w >= 3) return CeilDiv(L->a.M, 16) * CeilDiv(d->o, 16) * SelectLanes() * d->c * 9 > kSmallRowLoadsWork;
-    return L->gflop * SelectLanes() >= std::min(0.12 * L->a.csteps, 1.4);
+    return Switched(d->c >= 64 && d->w >= 3 ? CeilDiv(L->a.M, 16) * CeilDiv(d->o, 16) * SelectLanes() * d->c * 9 > kSmallRowLoadsWork
+                                            : L->gflop * SelectLanes() >= std::min(0.12 * L->a.csteps, 1.4));
 }
 
 // `partials`: room for the partial outputs of a split reduction; nullptr: it is acquired here.
@@ -272,33 +270,35 @@ int32_t LaunchConv(const PackedLaunch& L, const float* x, const float* w, const 
 // batch 11 13.8 and 12.6; 1x1, 128 -> 512 at 28 x 28, batch 32 57.9 and 44.2; 63 -> 376 at 18 x 32, batch 13 20.1 and 14.4.  Not taken: 5x5,
 // 32 -> 32 at 19 x 12, batch 37 16.0 and 21.2; 7x7, 64 -> 96 at 15 x 16 17.9 and 25.2; 3x3, 16 -> 144 at 90 x 9, batch 11 12.0 and 16.5; 1x1, 224 -> 160 at 30 x 34,
 // batch 21 28.5 and 31.3; images of no whole 16 bytes, whose pixels come one by one, 160 -> 400 at 37 x 23, batch 7 17.5 and 29.6.
-// (Every single call asks: from the shape alone first, then whether the kernel covers it.)
-bool OperatorPreferred(const kxc_hip_conv2d_desc* d, PackedLaunch* L) {
+bool OperatorRule(const kxc_hip_conv2d_desc* d) {
     using namespace conv_bx;
     const int K = d->kh, S = d->stride_h;
+    // (3x3, stride 2: single calls agree with the outputs of kxc_hip_conv2d_pair_nchw_f32, which packs nothing.  Stride 1: Winograd
+    // takes large ones; half of a block of 128 output channels empty is no gain)
+    if (K == 3 && (S == 2 || d->o < 96)) return false;
+    const int64_t oh = (static_cast<int64_t>(d->h) + 2 * d->pad_h - K) / S + 1, ow = (static_cast<int64_t>(d->w) + 2 * d->pad_w - K) / S + 1;
+    if (oh <= 0 || ow <= 0) return false;
+    if (K == 1 && (S != 1 || d->pad_h != 0 || d->pad_w != 0 || static_cast<int64_t>(d->h) * d->w % 4 != 0)) return false;
+    const double pixels = static_cast<double>(d->n) * oh * ow, out_bytes = 4.0 * pixels * d->o, gflop = 2e-9 * pixels * d->o * d->c * K * K;
+    const double memory = (4.0 * d->n * d->c * d->h * d->w + out_bytes * ((d->flags & KXC_HIP_CONV_RESIDUAL) ? 2 : 1)) / 4.5e6;
+    const double others = (K == 1 && d->c % 16 != 0 ? 14 : 9) + (K >= 5 ? 16 : K == 1 ? 13 : 12) * gflop - (K == 3 ? 0.15 * (9 + 12 * gflop) : 0);
+    if (10 + memory >= others || pixels >= 1e9) return false;
+    const int64_t units = CeilDiv(static_cast<int64_t>(pixels), kPix) * CeilDiv(d->o, kOut);
+    const int csteps = static_cast<int>(CeilDiv(d->c, kStep * ChannelSteps(K))), steps = Steps(K, false);
+    const int64_t lanes = SelectLanes();
+    const int split = Split(units * lanes, csteps, steps, static_cast<int64_t>(out_bytes));
+    const double groups = static_cast<double>(units * split * lanes);
+    const double load = groups <= 256 ? 1.0 : groups <= 512 ? 1.65 : 1.65 * groups / 512;
+    const double adding = split > 1 ? 5 + 2.0 * split * out_bytes / 4.5e6 : 0;
+    const double compute = 0.29 * steps * static_cast<double>(CeilDiv(csteps, split)) * load;
+    return 10 + (K == 1 ? compute + memory : std::max(compute, memory)) + adding < others;
+}
+
+// (Every single call asks: from the shape alone first, then the environment, then whether the kernel covers it.)
+bool OperatorPreferred(const kxc_hip_conv2d_desc* d, PackedLaunch* L) {
+    const int K = d->kh, S = d->stride_h;
     if (K != d->kw || S != d->stride_w || d->n <= 0 || d->c <= 0 || d->o <= 0 || (S != 1 && S != 2) || K > 7) return false;
-    const char e = Switch();
-    if (e == '0') return false;
-    if (e != '1') {
-        // (3x3, stride 2: single calls agree with the outputs of kxc_hip_conv2d_pair_nchw_f32, which packs nothing.  Stride 1: Winograd
-        // takes large ones; half of a block of 128 output channels empty is no gain)
-        if (K == 3 && (S == 2 || d->o < 96)) return false;
-        const int64_t oh = (static_cast<int64_t>(d->h) + 2 * d->pad_h - K) / S + 1, ow = (static_cast<int64_t>(d->w) + 2 * d->pad_w - K) / S + 1;
-        if (oh <= 0 || ow <= 0) return false;
-        if (K == 1 && (S != 1 || d->pad_h != 0 || d->pad_w != 0 || static_cast<int64_t>(d->h) * d->w % 4 != 0)) return false;
-        const double pixels = static_cast<double>(d->n) * oh * ow, out_bytes = 4.0 * pixels * d->o, gflop = 2e-9 * pixels * d->o * d->c * K * K;
-        const double memory = (4.0 * d->n * d->c * d->h * d->w + out_bytes * ((d->flags & KXC_HIP_CONV_RESIDUAL) ? 2 : 1)) / 4.5e6;
-        const double others = (K == 1 && d->c % 16 != 0 ? 14 : 9) + (K >= 5 ? 16 : K == 1 ? 13 : 12) * gflop - (K == 3 ? 0.15 * (9 + 12 * gflop) : 0);
-        if (10 + memory >= others || pixels >= 1e9) return false;
-        const int64_t units = CeilDiv(static_cast<int64_t>(pixels), kPix) * CeilDiv(d->o, kOut);
-        const int csteps = static_cast<int>(CeilDiv(d->c, kStep * ChannelSteps(K))), steps = Steps(K, false);
-        const int split = Split(units * SelectLanes(), csteps, steps, static_cast<int64_t>(out_bytes));
-        const double groups = static_cast<double>(units) * split * SelectLanes();
-        const double load = groups <= 256 ? 1.0 : groups <= 512 ? 1.65 : 1.65 * groups / 512;
-        const double adding = split > 1 ? 5 + 2.0 * split * out_bytes / 4.5e6 : 0;
-        const double compute = 0.29 * steps * static_cast<double>(CeilDiv(csteps, split)) * load;
-        if (10 + (K == 1 ? compute + memory : std::max(compute, memory)) + adding >= others) return false;
-    }
+    if (!Switched(OperatorRule(d))) return false;
     const char* variant = std::getenv("KXC_HIP_CONV_VARIANT");
     return !(variant && *variant) && Resolve(d, false, L) && L->filter_bytes <= (32u << 20);      // (bounds the scratch kept per stream)
 }

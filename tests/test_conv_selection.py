@@ -1,4 +1,8 @@
 """Which kernel a convolution takes, asked from the library on the host: no GPU is needed."""
+import ctypes
+import random
+import time
+
 import pytest
 
 
@@ -29,3 +33,41 @@ def test_switches_of_the_three_part_kernels(pkg, monkeypatch, switches, packed):
         assert _variant(pkg, xs, o, k).endswith("_bf16x3") == packed, (xs, o, k)
     for xs, o, k, second, hpool in NODES:
         assert (_node(pkg, xs, o, k, second, hpool) > 0) == packed, (xs, o, k)
+
+
+def _us(f):
+    best = 1e9
+    for _ in range(20):
+        t = time.perf_counter()
+        for _ in range(50):
+            f()
+        best = min(best, (time.perf_counter() - t) / 50 * 1e6)
+    return best
+
+
+@pytest.mark.parametrize("xs, o, k", [((64, 64, 111, 111), 128, 5), ((16, 64, 87, 87), 128, 5)])
+def test_maps_too_wide_for_the_packed_kernel_are_refused_at_once(pkg, monkeypatch, xs, o, k):
+    """A call asks for the packed kernel first; where the rows of its map do not fit, that must cost little beside the selection of
+    the kernel that takes it (which a plan's node, asked here for comparison, does without the question)."""
+    monkeypatch.delenv("KXC_HIP_CONV_BF16X3", raising=False)
+    d = pkg.conv_desc(xs, (o, xs[1], k, k), 1, k // 2, 1, 0)
+    lib, p = pkg.lib(), ctypes.byref(d)
+    assert "bf16x3" not in _variant(pkg, xs, o, k)
+    assert _us(lambda: lib.kxc_hip_conv2d_variant(p)) <= 1.5 * _us(lambda: lib.kxc_hip_conv2d_node_variant(p)) + 2
+
+
+@pytest.mark.parametrize("seed", range(4))
+def test_packed_kernel_covers_the_maps_whose_rows_fit(pkg, monkeypatch, seed):
+    """Two rows of waves and an LDS plane of 384 positions: the rows that a tile of 64 pixels touches, from a walk over every tile."""
+    monkeypatch.setenv("KXC_HIP_CONV_BF16X3", "1")
+    monkeypatch.setenv("KXC_HIP_CONV_WINOGRAD", "0")
+    rng = random.Random(seed)
+    for _ in range(150):
+        k, s = rng.choice((3, 5, 7)), rng.choice((1, 2))
+        n, h, w, pad = rng.randint(1, 9), rng.randint(k, 60), rng.randint(k, 90), rng.randint(0, 3)
+        oh, ow = (h + 2 * pad - k) // s + 1, (w + 2 * pad - k) // s + 1
+        at = lambda m: m // (oh * ow) * (oh + (k - 1) // s) + m % (oh * ow) // ow
+        rows = max(at(min(m + 64, n * oh * ow) - 1) - at(m) for m in range(0, n * oh * ow, 64)) + 1 + (k - 1) // s
+        pitch = 2 * max(ow + (k - 1) // 2, (w - 1 + pad) // 2 + 1) if s == 2 else max(ow + k - 1, w + pad)
+        covers = rows * pitch <= 384 and 2 * rows * -(-w // 4) <= 256
+        assert _variant(pkg, (n, 16, h, w), 32, k, s, pad).endswith("_bf16x3") == covers, (n, h, w, k, s, pad)
