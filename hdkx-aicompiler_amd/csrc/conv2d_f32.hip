@@ -1227,11 +1227,11 @@ const SmallVariant* SelectSmall(const kxc_hip_conv2d_desc* d, const ConvArgs& a,
     if (x_elems >= (1 << 29) || y_elems >= (1 << 29) || w_elems >= (1 << 29)) return nullptr;       // 31-bit byte offsets
     const char* forced = std::getenv("KXC_HIP_CONV_VARIANT");
     const bool by_name = forced && *forced;
-    const int64_t tiles = CeilDiv(a.M, 16) * CeilDiv(a.O, 16) * SelectLanes();
+    const int64_t lanes = SelectLanes(), tiles = CeilDiv(a.M, 16) * CeilDiv(a.O, 16) * lanes;
     const SmallVariant* const v = kSmall;
     if (d->kh == 1) {
         if (by_name ? std::strcmp(forced, v[3].name) != 0 : a.C < 96 && static_cast<int64_t>(a.M) * a.O > 6000000) return nullptr;
-        return second ? nullptr : CeilDiv(a.M, 16) * CeilDiv(a.O, 64) * SelectLanes() >= 512 ? v + 4 : v + 3;
+        return second ? nullptr : CeilDiv(a.M, 16) * CeilDiv(a.O, 64) * lanes >= 512 ? v + 4 : v + 3;
     }
     if (d->kh != 3 || (second && !in_plan)) return nullptr;
     // the second output reads the middle tap (padding 0 at stride 3, say, wants tap 0: the general kernel's ds_off)
@@ -1240,13 +1240,13 @@ const SmallVariant* SelectSmall(const kxc_hip_conv2d_desc* d, const ConvArgs& a,
     const bool one_block = SmallRowLoads(a) && (a.O % 16 == 0 || tiles > 800);
     const bool reaches = SmallRowLoads(a) && tiles * a.C * 9 <= kSmallRowLoadsWork;
     if (!by_name && (a.C < 64 || (!reaches && tiles > (second || a.O <= 16 ? 1600 : 800)) || (!in_plan && tiles < 400))) return nullptr;
-    const bool rows_fit = a.dw == 1 && SmallWords(v[0], a) * v[0].chunk <= v[0].xi * 64;      // (walks the map: behind the cheap tests)
+    auto rows_fit = [&]() { return a.dw == 1 && SmallWords(v[0], a) * v[0].chunk <= v[0].xi * 64; };      // (walks the map: behind the cheap tests)
     if (by_name) {
-        for (int i = rows_fit ? 0 : 1; i < 3; ++i)
-            if (std::strcmp(forced, v[i].name) == 0) return v + i;
+        for (int i = 0; i < 3; ++i)
+            if (std::strcmp(forced, v[i].name) == 0) return i > 0 || rows_fit() ? v + i : nullptr;
         return nullptr;
     }
-    if (rows_fit && !(one_block && a.sw > 1) && a.N * CeilDiv(a.OHW, 16) * CeilDiv(a.O, 16) * SelectLanes() <= kNumCUs) return v;
+    if (!(one_block && a.sw > 1) && a.N * CeilDiv(a.OHW, 16) * CeilDiv(a.O, 16) * lanes <= kNumCUs && rows_fit()) return v;
     return one_block || tiles <= kNumCUs ? v + 1 : v + 2;
 }
 

@@ -71,3 +71,14 @@ def test_packed_kernel_covers_the_maps_whose_rows_fit(pkg, monkeypatch, seed):
         pitch = 2 * max(ow + (k - 1) // 2, (w - 1 + pad) // 2 + 1) if s == 2 else max(ow + k - 1, w + pad)
         covers = rows * pitch <= 384 and 2 * rows * -(-w // 4) <= 256
         assert _variant(pkg, (n, 16, h, w), 32, k, s, pad).endswith("_bf16x3") == covers, (n, h, w, k, s, pad)
+
+
+def test_small_calls_are_chosen_without_walking_their_map(pkg):
+    """A call of a few microseconds: the kernel that stages whole rows asks how many a tile touches, tile by tile, and is out of the
+    question from 257 tiles on.  Compared with the selection of a 1x1 filter, which walks nothing."""
+    lib = pkg.lib()
+    us = {}
+    for k in (1, 3):
+        d = pkg.conv_desc((1, 64, 56, 56), (64, 64, k, k), 1, k // 2, 1, 0)
+        us[k] = _us(lambda: lib.kxc_hip_conv2d_variant(ctypes.byref(d)))
+    assert us[3] <= 1.6 * us[1] + 0.1, us
