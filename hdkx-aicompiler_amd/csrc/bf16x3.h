@@ -6,10 +6,11 @@
 // |m| <= 2^-8 |x|, |l| <= 2^-17 |x|, and from |x| = 2^-109 on the three parts hold all 24 bits of x.  Below, the last bits lie
 // under bf16's smallest step, 2^-133 (the matrix instructions take subnormal parts as they are), and h + m + l is off by
 // at most 2^-134, which is all of an x of that size.  Multiplying operands by 2^16 while they are split, and sums by 2^-32,
-// keeps those bits as well and was not taken: 300 x 1000 x 2048 15.4 -> 16.6 us, 64 x 1000 x 512 4.7 -> 5.0 (with
-// v_dot2_f32_bf16 in the place of each unpacking and subtraction, which is exact, 16.8 and 4.9); KXC_HIP_GEMM_BF16X3=0 and
-// KXC_HIP_WINOGRAD_BF16X3=0 keep the fp32 instructions for callers whose operands are that small, in products and in all convolutions
-// (KXC_HIP_CONV_BF16X3=0: in those that are no Winograd launches).
+// keeps those bits as well (every float times 2^16 is a whole number of such steps): the convolutions on a packed filter do it
+// (conv_bf16x3.h, conv7_bf16x3.h), whose sums that are not finite, from 2^96 on, are formed again.  Not taken in products: 300 x
+// 1000 x 2048 15.4 -> 16.6 us, 64 x 1000 x 512 4.7 -> 5.0 (with v_dot2_f32_bf16 in the place of each unpacking and subtraction,
+// which is exact, 16.8 and 4.9), nor in a plan's Winograd layers, which have no second way to form a sum; KXC_HIP_GEMM_BF16X3=0
+// and KXC_HIP_WINOGRAD_BF16X3=0 keep the fp32 instructions for callers whose operands are that small.
 // A product of two such numbers is nine bf16 products, each exact in fp32; the three that are left out (m*l', l*m', l*l')
 // add up to at most 2^-24 |x x'|, what rounding the product to fp32 may lose as well.  The six others are accumulated in
 // fp32 by v_mfma_f32_32x32x16_bf16, smallest first.  Measured on random dot products of 64, 576 and 4608 terms against a
@@ -39,6 +40,8 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 #if defined(__HIPCC__)
+
+constexpr float kOperandScale = 65536.0f, kSumScale = 1.0f / (65536.0f * 65536.0f);      // for operands below 2^-109 (see above)
 
 // Two floats -> two packed bf16, round to nearest even (one instruction on gfx950).
 __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {

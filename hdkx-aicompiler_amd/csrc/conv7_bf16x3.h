@@ -117,7 +117,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
             for (int k = 0; k < kBatch; ++k) {
                 const int rc = i0 + k * kPar + (kPar == 2 ? wave : 0), row = rc / kC, c = rc - row * kC;
                 uint32_t h, m, l;
-                split_pair(v[k][0], v[k][1], h, m, l);
+                split_pair(__fmul_rn(v[k][0], kOperandScale), __fmul_rn(v[k][1], kOperandScale), h, m, l);
                 if (rc < total && d < kPitch) {
                     uint32_t* const dst = lds + (c * a.row_max + row) * 3 * kPitch + d;
                     dst[0] = h;
@@ -196,12 +196,14 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
     }
     __syncthreads();          // (the patch is dead)
 
-    // ---- Splitting turns an infinite operand into NaN, and so does it to one above 3.39e38, and products next to the largest float
-    // may overflow in their large part: a sum that is not finite is formed again by the operator's definition.
+    // ---- Splitting turns an infinite operand into NaN, and so does it to one of 2^112 and more, and sums (times 2^32 here) overflow
+    // from 2^96 on: a sum that is not finite is formed again by the operator's definition.
     float* const area = reinterpret_cast<float*>(lds) + wave * 16 * 64;
 #pragma unroll
     for (int j = 0; j < kBlocks; ++j) {
         float odd = 0.0f;
+#pragma unroll
+        for (int g = 0; g < 16; ++g) acc[j][g] = __fmul_rn(acc[j][g], kSumScale);
 #pragma unroll
         for (int g = 0; g < 16; ++g) odd = __builtin_fmaf(acc[j][g], 0.0f, odd);
         if (__builtin_amdgcn_ballot_w64(!(odd == 0.0f)) == 0) continue;
@@ -311,7 +313,7 @@ __device__ __forceinline__ void pack_tile(const float* __restrict__ w, char* __r
         const int s = i >> 6, lane = i & 63, o = tile * 32 + (lane & 31), g = 2 * s + (lane >> 5);
         float v[8];
 #pragma unroll
-        for (int t = 0; t < 8; ++t) v[t] = t < kK && g < kGroups && o < O ? w[(static_cast<int64_t>(o) * kGroups + g) * kK + t] : 0.0f;
+        for (int t = 0; t < 8; ++t) v[t] = t < kK && g < kGroups && o < O ? kOperandScale * w[(static_cast<int64_t>(o) * kGroups + g) * kK + t] : 0.0f;
         const Split8 p = split8(v);
         char* const dst = u + (static_cast<int64_t>(tile) * kSteps + s) * 3072 + lane * 16;
         *reinterpret_cast<u32x4*>(dst) = p.h;

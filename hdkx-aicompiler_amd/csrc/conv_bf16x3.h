@@ -187,8 +187,9 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3
                 if (k > 0 && 2 * per_half <= 64 * kProducers * k) break;
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    const float t[8] = {v[SET][k][0][j], v[SET][k][1][j], v[SET][k][2][j], v[SET][k][3][j],
-                                        v[SET][k][4][j], v[SET][k][5][j], v[SET][k][6][j], v[SET][k][7][j]};
+                    float t[8];
+#pragma unroll
+                    for (int c = 0; c < 8; ++c) t[c] = __fmul_rn(v[SET][k][c][j], kOperandScale);
                     const Split8 s = split8(t);
                     if (j < left[k]) {
                         const int at = K == 1 ? j : ((j + a.pw) % S) * a.hp + (j + a.pw) / S;
@@ -389,7 +390,10 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int g = 0; g < 16; ++g) big[j][g] = __fadd_rn(big[j][g], small[j][g]);
+        for (int g = 0; g < 16; ++g) {
+            big[j][g] = __fmul_rn(__fadd_rn(big[j][g], small[j][g]), kSumScale);
+            if constexpr (SECOND) acc2[j][g] = __fmul_rn(acc2[j][g], kSumScale);
+        }
     const float* const bias = has_bias ? a.bias : nullptr;
     const float* const res = has_res ? a.res : nullptr;
     const float* const bias2 = raw ? nullptr : a.bias2;
@@ -399,8 +403,8 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3
     const uint32_t odd = finish(big, bias, res, do_relu, y);
     uint32_t odd2 = 0;
     if constexpr (SECOND) odd2 = finish(acc2, bias2, nullptr, false, y2);
-    // Splitting turns an infinite operand into NaN, and so does it to one above 3.39e38, and products next to the largest float may
-    // overflow in their large part: a sum that is not finite is formed again by the operator's definition, over the channels of
+    // Splitting turns an infinite operand into NaN, and so does it to one of 2^112 and more, and sums (times 2^32 here) overflow
+    // from 2^96 on: a sum that is not finite is formed again by the operator's definition, over the channels of
     // this part.  Nothing is stored before (the residual may be the output's own buffer).
     if ((odd | odd2) == 0) return;
     auto again = [&](uint32_t mask, const float* w, bool one_tap, const float* bias, const float* res, bool do_relu, float* out) __attribute__((always_inline)) {
@@ -470,7 +474,7 @@ __device__ __forceinline__ void pack_block(const float* __restrict__ w, const fl
         float v[8];
 #pragma unroll
         for (int c = 0; c < 8; ++c)
-            v[c] = is2 ? (o < O && c0 + half * 8 + c < C ? w2[static_cast<int64_t>(o) * C + c0 + half * 8 + c] : 0.0f) : raw[ol * (RUN + 1) + (first + c) * KK + tap];
+            v[c] = kOperandScale * (is2 ? (o < O && c0 + half * 8 + c < C ? w2[static_cast<int64_t>(o) * C + c0 + half * 8 + c] : 0.0f) : raw[ol * (RUN + 1) + (first + c) * KK + tap]);
         const Split8 s = split8(v);
         char* const dst = u + ((static_cast<int64_t>(o / 32) * csteps + cs) * ns + step) * 3072 + (half * 32 + o % 32) * 16;
         *reinterpret_cast<u32x4*>(dst) = s.h;

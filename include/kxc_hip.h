@@ -171,9 +171,9 @@ typedef struct kxc_hip_conv2d_desc {
  * values of 1 costs its neighbours their digits; Inf and NaN do not: such outputs are evaluated by the definition).
  * KXC_HIP_CONV_WINOGRAD=0 in the environment keeps the kernels that add only what an output's window holds.
  *
- * Large calls of other filters (..._variant says "..._bf16x3") run on the bf16 matrix cores with every operand as three bf16
- * parts: exact from 2^-109 on, below it an operand is off by at most 2^-134; sums that are not finite are evaluated by the
- * definition.  KXC_HIP_CONV_BF16X3=0 keeps the fp32 instructions, and so does KXC_HIP_WINOGRAD_BF16X3=0, which keeps them in every
+ * Large calls of other filters (..._variant says "mfma_..._bf16x3") run on the bf16 matrix cores with every operand as three bf16
+ * parts that hold all its bits; sums of 2^96 and more and those that are not finite are evaluated by the definition (the same
+ * results, much slower).  KXC_HIP_CONV_BF16X3=0 keeps the fp32 instructions, and so does KXC_HIP_WINOGRAD_BF16X3=0, which keeps them in every
  * convolution, unless KXC_HIP_CONV_BF16X3=1 asks for these kernels.
  *
  * Scratch.  A launch that splits its reduction over workgroups, and a large call that transforms or packs its filter first

@@ -155,6 +155,22 @@ def test_conv_on_a_packed_filter_keeps_values_that_are_not_finite(pkg, monkeypat
     node.plan.close()
 
 
+@pytest.mark.parametrize("xs, o, second, k, hpool", [((2, 64, 13, 18), 96, True, 3, False), ((2, 512, 8, 8), 128, True, 3, False),
+                                                     ((2, 3, 45, 50), 40, False, 7, False), ((7, 3, 64, 64), 40, False, 7, True)])
+@pytest.mark.parametrize("sx, sw", [(2.0 ** -122, 1.0), (1.0, 2.0 ** -122), (2.0 ** -128, 2.0 ** 20), (2.0 ** 100, 1.0), (1.0, 2.0 ** 100)])
+def test_conv_on_a_packed_filter_at_both_ends_of_the_range(pkg, monkeypatch, xs, o, second, k, hpool, sx, sw):
+    """Operands that bf16 parts hold in fewer bits than float32 does unless they are scaled, and sums that then overflow: the
+    error of a float32 sum, as for operands of ordinary size.  (2^-128: float32 holds a value within 2^-150.)"""
+    monkeypatch.setenv("KXC_HIP_CONV_BF16X3", "1")
+    node = _Node(pkg, xs, o, second, bias=False, relu=hpool, seed=9, k=k, pad=k // 2, hpool=hpool)
+    for i, name, scale in ((0, "x", sx), (1, "w", sw), (5, "w2", sw)):
+        a = getattr(node, name) * np.float32(scale)
+        setattr(node, name, a)
+        node.args[i].copy_(torch.from_numpy(a))
+    node.check(node.run())
+    node.plan.close()
+
+
 def test_packed_filters_follow_their_weights(pkg, monkeypatch):
     """Rewritten in place they are read in the next run; frozen, only another pointer or an invalidation counts, for either
     of the two filters; the plan's text keeps the node; a graph replays it."""
@@ -244,6 +260,21 @@ def test_single_convolution_on_a_packed_filter(pkg, monkeypatch, xs, o, k, strid
     assert (np.isnan(got) == np.isnan(want)).all() and (got[np.isinf(want)] == want[np.isinf(want)]).all()
     m = np.isfinite(want)
     assert (np.abs(got[m] - want[m]) <= 1e-5 * np.maximum(np.abs(want[m]), 1.0)).all()
+
+
+@pytest.mark.parametrize("xs, o, k", [((2, 50, 27, 27), 96, 5), ((2, 512, 6, 6), 256, 3), ((3, 96, 4, 5), 200, 1)])
+@pytest.mark.parametrize("sx, sw", [(2.0 ** -122, 1.0), (1.0, 2.0 ** -122), (2.0 ** 100, 1.0)])
+def test_single_convolution_on_a_packed_filter_at_both_ends_of_the_range(pkg, monkeypatch, xs, o, k, sx, sw):
+    monkeypatch.setenv("KXC_HIP_CONV_WINOGRAD", "0")
+    monkeypatch.setenv("KXC_HIP_CONV_BF16X3", "1")
+    rng = np.random.default_rng(k)
+    x = rng.standard_normal(xs).astype(np.float32) * np.float32(sx)
+    w = (rng.standard_normal((o, xs[1], k, k)) * (2 / (k * k * xs[1])) ** 0.5).astype(np.float32) * np.float32(sw)
+    assert "bf16x3" in pkg.conv2d_variant(x.shape, w.shape, 1, k // 2)
+    want = _want(x, w, None, None, False, 1, k // 2)
+    got = host(pkg.conv2d(dev(x), dev(w), None, None, 1, k // 2))
+    assert np.isfinite(got).all()
+    assert np.linalg.norm(got - want) <= (k * k * xs[1] + 16) ** 0.5 * 2.0 ** -23 * np.linalg.norm(want)
 
 
 def _filters(pkg, xs, o, k, count, seed):
