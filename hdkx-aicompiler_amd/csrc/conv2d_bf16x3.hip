@@ -196,6 +196,18 @@ bool Switched(bool by_rule) {
     return !(w && w[0] == '0');
 }
 
+// us of the launches but `fixed`: workgroups of `start` + `step` per step, `second` times that where two share a compute unit, and
+// the adding launch.
+double PackedUs(double fixed, double start, double step, double second, int64_t groups, int64_t steps, int split, double out_bytes) {
+    const double load = groups <= 256 ? 1.0 : second * std::max(1.0, static_cast<double>(groups) / 512);
+    return fixed + (start + step * static_cast<double>(steps)) * load + (split > 1 ? 5 + 2.0 * split * out_bytes / 4.5e6 : 0);
+}
+
+// GFLOP of the other kernels, whose blocks of outputs are `block` x `block`.
+double BlockGflop(const kxc_hip_conv2d_desc* d, int64_t pixels, int taps, int block) {
+    return 2e-9 * static_cast<double>(CeilDiv(pixels, block) * block) * static_cast<double>(CeilDiv(d->o, block) * block) * d->c * taps;
+}
+
 // Whether a plan's node should take it: with fewer than 64 channels from 0.12 GFLOP per step of 16 on, counting the launches
 // expected side by side.  A workgroup takes 9 us and 2.9 per step however few there are, and the other kernels start with 16 x 16 tiles and
 // split reductions inside a workgroup (us, theirs and here, both outputs): 64 -> 128 channels at 56 x 56, batch 2 (0.26 GFLOP)
@@ -208,6 +220,13 @@ bool Switched(bool by_rule) {
 // The 7x7 kernel, 3 -> 64 channels: pooled at 224 x 224, batch 16 / 32 / 64 51 / 100 / 169 and 32 / 59 / 108, at 64 x 64, batch 56 (1.1 GFLOP) 33 and
 // 22; not pooled at 224 x 224, batch 4 (0.94) 20.6 and 21.8, batch 8 (1.9) 33 and 30, batch 64 182 and 116; tiles 13 rows high, of which a compute unit holds
 // two, at 193 x 193, batch 16 (2.8) 49 and 54.
+// At 3x3 that must also be the shorter time by what either side takes, fitted within a tenth to 1000 shapes of 16 to 512 and 8 to 512 channels: here
+// 2 us and a workgroup's 4 + 0.28 per tap and step, the others 10.5 and 12.7 per GFLOP of 32 x 32 blocks or, by the small-launch kernels, 4.9
+// and 12.4 of 16 x 16 ones.  A workgroup has 128 output channels: no more than 48 of them (256 -> 8 at 60 x 38, batch 38 24.5 and 99.4, 384 ->
+// 16 at 32 x 31, batch 43 34 and 61, 384 -> 48 at 21 x 45, batch 30 41.6 and 50.5) and a reduction of one step (16 -> 32 at 46 x 51, batch 59 15.3
+// and 24.6, 16 -> 72 at 82 x 58, batch 15 12.9 and 14.8) are never worth it.  384 -> 64 at 13 x 56, batch 18 25.8 and 33.7, 512 -> 160 at 8 x
+// 38, batch 14 23.9 and 36.2.  Of 237 of these shapes that are taken four are slower by more than 3 % (at most 16), of 322 by the first
+// line alone 51 (up to four times).
 // KXC_HIP_CONV_VARIANT, which names one of the other kernels, keeps those as well.
 bool Preferred(const kxc_hip_conv2d_desc* d, bool second, PackedLaunch* L) {
     const char* variant = std::getenv("KXC_HIP_CONV_VARIANT");
@@ -219,8 +238,18 @@ bool Preferred(const kxc_hip_conv2d_desc* d, bool second, PackedLaunch* L) {
     }
     // (a plan's filter launch packs 3x3 stride-2 filters only)
     if (!d || d->kh != 3 || d->stride_h != 2 || d->pad_h != 1 || d->pad_w != 1 || d->c % conv_bx::kStep != 0 || !Resolve(d, second, L)) return false;
-    return Switched(d->c >= 64 && d->w >= 3 ? CeilDiv(L->a.M, 16) * CeilDiv(d->o, 16) * SelectLanes() * d->c * 9 > kSmallRowLoadsWork
-                                            : L->gflop * SelectLanes() >= std::min(0.12 * L->a.csteps, 1.4));
+    auto rule = [&]() {
+        const int64_t lanes = SelectLanes();
+        if (d->o <= 48 || d->c <= conv_bx::kStep) return false;
+        if (d->c >= 64 && d->w >= 3 ? CeilDiv(L->a.M, 16) * CeilDiv(d->o, 16) * lanes * d->c * 9 <= kSmallRowLoadsWork
+                                    : L->gflop * lanes < std::min(0.12 * L->a.csteps, 1.4)) return false;
+        const int taps = second ? 10 : 9;
+        const double out_bytes = 4.0 * L->a.M * d->o * (second ? 2 : 1);
+        const bool small = SmallConvTakes(d, second, true);
+        const double others = small ? 4.9 + 12.4 * lanes * BlockGflop(d, L->a.M, taps, 16) : 10.5 + 12.7 * lanes * BlockGflop(d, L->a.M, taps, 32);
+        return PackedUs(2, 4, 0.28, 2, lanes * L->a.num_units * L->a.gsplit, static_cast<int64_t>(taps) * L->a.cps, L->a.gsplit, out_bytes) < others;
+    };
+    return Switched(rule());
 }
 
 // `partials`: room for the partial outputs of a split reduction; nullptr: it is acquired here.

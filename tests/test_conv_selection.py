@@ -82,3 +82,24 @@ def test_small_calls_are_chosen_without_walking_their_map(pkg):
         d = pkg.conv_desc((1, 64, 56, 56), (64, 64, k, k), 1, k // 2, 1, 0)
         us[k] = _us(lambda: lib.kxc_hip_conv2d_variant(ctypes.byref(d)))
     assert us[3] <= 1.6 * us[1] + 0.1, us
+
+
+@pytest.mark.parametrize("xs, o, second, packed", [
+    # us, fp32 instructions and packed
+    ((64, 64, 56, 56), 128, True, True),        # 97, 61
+    ((64, 128, 28, 28), 256, True, True),       # 94, 54
+    ((64, 256, 14, 14), 512, True, True),       # 104, 52
+    ((21, 96, 26, 16), 512, False, True),       # 37, 21
+    ((46, 96, 63, 16), 64, False, True),        # 27, 20: half of a workgroup's output channels
+    ((38, 256, 60, 38), 8, False, False),       # 24, 99
+    ((43, 384, 32, 31), 16, False, False),      # 34, 61
+    ((59, 16, 46, 51), 32, True, False),        # 15, 25
+    ((30, 384, 21, 45), 48, False, False),      # 42, 50
+    ((18, 384, 13, 56), 64, True, False),       # 26, 34: small-launch kernel
+    ((14, 512, 8, 38), 160, False, False),      # 24, 36
+    ((2, 64, 56, 56), 128, True, False),        # 12, 16
+])
+def test_stride_2_nodes_take_the_packed_kernel_where_it_is_the_faster_one(pkg, monkeypatch, xs, o, second, packed):
+    for name in ("KXC_HIP_CONV_BF16X3", "KXC_HIP_WINOGRAD_BF16X3"):
+        monkeypatch.delenv(name, raising=False)
+    assert (_node(pkg, xs, o, 3, second) > 0) == packed
