@@ -196,6 +196,12 @@ bool Switched(bool by_rule) {
     return !(w && w[0] == '0');
 }
 
+// A switch that names one of the other kernels keeps those.
+bool OthersForced() {
+    const char* variant = std::getenv("KXC_HIP_CONV_VARIANT");
+    return variant && *variant;
+}
+
 // us of the launches but `fixed`: workgroups of `start` + `step` per step, `second` times that where two share a compute unit, and
 // the adding launch.
 double PackedUs(double fixed, double start, double step, double second, int64_t groups, int64_t steps, int split, double out_bytes) {
@@ -227,10 +233,8 @@ double BlockGflop(const kxc_hip_conv2d_desc* d, int64_t pixels, int taps, int bl
 // and 24.6, 16 -> 72 at 82 x 58, batch 15 12.9 and 14.8) are never worth it.  384 -> 64 at 13 x 56, batch 18 25.8 and 33.7, 512 -> 160 at 8 x
 // 38, batch 14 23.9 and 36.2.  Of 237 of these shapes that are taken four are slower by more than 3 % (at most 16), of 322 by the first
 // line alone 51 (up to four times).
-// KXC_HIP_CONV_VARIANT, which names one of the other kernels, keeps those as well.
 bool Preferred(const kxc_hip_conv2d_desc* d, bool second, PackedLaunch* L) {
-    const char* variant = std::getenv("KXC_HIP_CONV_VARIANT");
-    if (variant && *variant) return false;
+    if (OthersForced()) return false;
     if (!second && Resolve7(d, L)) {
         // Pooled rows: always.  Others: four workgroups to a compute unit (tiles that are few rows high) and work for them.
         const bool pooled = (d->flags & KXC_HIP_CONV_HPOOL) != 0;
@@ -289,16 +293,16 @@ int32_t LaunchConv(const PackedLaunch& L, const float* x, const float* w, const 
     return LaunchSplitReduce(s, r);
 }
 
-// Whether a single call, which packs its filter first, should take the kernel.  Its time: 10 us for two launches and what surrounds the
-// steps, the longer of the bytes at 4.5 TB/s and 0.29 us per tap and 16 channels (two workgroups on a compute unit take
-// 1.65 times as long as one; a 1x1 filter's few steps do not hide the bytes: the sum), and the adding launch.  The other kernels
-// take 9 us and 12 per GFLOP (13 for 1x1, 16 for 5x5 and 7x7; 14 us where a 1x1 filter's channels are no multiple of 16); at 3x3 a seventh of
-// that in hand (20 -> 439 at 7 x 29, batch 33 21.1 and 23.9).  us, with the
-// residual, theirs and here: 5x5, 64 -> 96 channels at 27 x 27, batch 8 40.0 and 27.3; 16 -> 192 at 76 x 35, stride 2, batch 6 19.5 and 17.4; 7x7,
-// 226 -> 161 at 26 x 33 72 and 44; 13 -> 356 at 64 x 12, batch 4 31.9 and 24.7; 3x3, 220 -> 260 at 9 x 10, batch 27 47.9 and 35.1; 16 -> 221 at 53 x 11,
-// batch 11 13.8 and 12.6; 1x1, 128 -> 512 at 28 x 28, batch 32 57.9 and 44.2; 63 -> 376 at 18 x 32, batch 13 20.1 and 14.4.  Not taken: 5x5,
-// 32 -> 32 at 19 x 12, batch 37 16.0 and 21.2; 7x7, 64 -> 96 at 15 x 16 17.9 and 25.2; 3x3, 16 -> 144 at 90 x 9, batch 11 12.0 and 16.5; 1x1, 224 -> 160 at 30 x 34,
-// batch 21 28.5 and 31.3; images of no whole 16 bytes, whose pixels come one by one, 160 -> 400 at 37 x 23, batch 7 17.5 and 29.6.
+// Whether a single call, which packs its filter first, should take the kernel: a twentieth shorter than the others, by what both
+// sides take, fitted to 500 calls of 0.05 to 4 GFLOP within 5 % here and a tenth there.  Here by filter: two launches, a workgroup's start and its steps
+// (a 1x1 filter's few steps do not hide the bytes, from caches mostly).  The others: GFLOP of whole blocks, at 1x1 the bytes as well; the
+// small-launch kernels take smaller blocks.  Of 1x1 calls 35 of 160 take it and none is slower by more than 3 %, 7x7 20 of 80 and none, 5x5 25 of
+// 153 and one (11 -> 329 at 65 x 37, stride 2, batch 18 28.5 and 34.6), 3x3 11 of 107 and two (up to 9 %).  us, theirs and here: 5x5, 64 -> 96 channels at 27 x 27, batch 8 38.4 and 25.4; 7x7,
+// 226 -> 161 at 26 x 33 72 and 44; 13 -> 356 at 64 x 12, batch 4 31.9 and 24.7; 3x3, 220 -> 260 at 9 x 10, batch 27 47.9 and 35.1; 1x1, 128 -> 512 at
+// 28 x 28, batch 32 73.6 and 50.2.  Not taken: 5x5, 32 -> 32 at 19 x 12, batch 37 16.0 and 21.2; 6 -> 126 at 60 x 48, batch 11 18.4 and 26.6; 7x7, 64 ->
+// 96 at 15 x 16 17.9 and 25.2; 3x3, 16 -> 144 at 90 x 9, batch 11 12.0 and 16.5; 32 -> 208 at 100 x 31, batch 3 18.2 and 22.4; 1x1, 120 -> 35 at 14 x 48,
+// batch 2 6.4 and 10.8; 400 -> 448 at 22 x 78, batch 3 26.6 and 30.8; images of no whole 16 bytes, whose pixels come one by one, 160 ->
+// 400 at 37 x 23, batch 7 17.5 and 29.6.
 bool OperatorRule(const kxc_hip_conv2d_desc* d) {
     using namespace conv_bx;
     const int K = d->kh, S = d->stride_h;
@@ -308,28 +312,30 @@ bool OperatorRule(const kxc_hip_conv2d_desc* d) {
     const int64_t oh = (static_cast<int64_t>(d->h) + 2 * d->pad_h - K) / S + 1, ow = (static_cast<int64_t>(d->w) + 2 * d->pad_w - K) / S + 1;
     if (oh <= 0 || ow <= 0) return false;
     if (K == 1 && (S != 1 || d->pad_h != 0 || d->pad_w != 0 || static_cast<int64_t>(d->h) * d->w % 4 != 0)) return false;
-    const double pixels = static_cast<double>(d->n) * oh * ow, out_bytes = 4.0 * pixels * d->o, gflop = 2e-9 * pixels * d->o * d->c * K * K;
-    const double memory = (4.0 * d->n * d->c * d->h * d->w + out_bytes * ((d->flags & KXC_HIP_CONV_RESIDUAL) ? 2 : 1)) / 4.5e6;
-    const double others = (K == 1 && d->c % 16 != 0 ? 14 : 9) + (K >= 5 ? 16 : K == 1 ? 13 : 12) * gflop - (K == 3 ? 0.15 * (9 + 12 * gflop) : 0);
-    if (10 + memory >= others || pixels >= 1e9) return false;
-    const int64_t units = CeilDiv(static_cast<int64_t>(pixels), kPix) * CeilDiv(d->o, kOut);
+    const double pixels_d = static_cast<double>(d->n) * oh * ow, out_bytes = 4.0 * pixels_d * d->o;
+    if (pixels_d >= 1e9 || out_bytes >= 1e10) return false;
+    const int64_t pixels = static_cast<int64_t>(pixels_d), lanes = SelectLanes();
+    const double memory = lanes * (4.0 * d->n * d->c * d->h * d->w + out_bytes * ((d->flags & KXC_HIP_CONV_RESIDUAL) ? 2 : 1)) / 4.5e6;
+    const double blocks = lanes * BlockGflop(d, pixels, K * K, 32);
+    const int64_t units = CeilDiv(pixels, kPix) * CeilDiv(d->o, kOut);
     const int csteps = static_cast<int>(CeilDiv(d->c, kStep * ChannelSteps(K))), steps = Steps(K, false);
-    const int64_t lanes = SelectLanes();
     const int split = Split(units * lanes, csteps, steps, static_cast<int64_t>(out_bytes));
-    const double groups = static_cast<double>(units * split * lanes);
-    const double load = groups <= 256 ? 1.0 : groups <= 512 ? 1.65 : 1.65 * groups / 512;
-    const double adding = split > 1 ? 5 + 2.0 * split * out_bytes / 4.5e6 : 0;
-    const double compute = 0.29 * steps * static_cast<double>(CeilDiv(csteps, split)) * load;
-    return 10 + (K == 1 ? compute + memory : std::max(compute, memory)) + adding < others;
+    const int64_t groups = units * split * lanes, own = static_cast<int64_t>(steps) * CeilDiv(csteps, split);
+    const double here = K == 1 ? PackedUs(6.7 + 0.35 * memory, 1.7, 0.29, 2.16, groups, own, split, out_bytes)
+                        : K == 3 ? PackedUs(7, 2, 0.25, 2.6, groups, own, split, out_bytes)
+                        : K == 5 ? PackedUs(4.6, 5.7, 0.205, 1.9, groups, own, split, out_bytes) : PackedUs(2.3, 8.8, 0.213, 1.9, groups, own, split, out_bytes);
+    double others = K == 1 ? 9 + 17.5 * blocks + 0.33 * memory : K == 3 ? 7.5 + 10.5 * lanes * BlockGflop(d, pixels, 9, 16)
+                    : K == 5 ? 10.5 + 10.9 * blocks : 12.5 + 11.5 * blocks;
+    if (here >= 0.95 * others || K > 3 || !SmallConvTakes(d, false, false)) return here < 0.95 * others;
+    others = K == 1 ? 3.3 + 7.7 * blocks + 0.96 * memory : 4.4 + 11.2 * lanes * BlockGflop(d, pixels, 9, 16);
+    return here < 0.95 * others;
 }
 
 // (Every single call asks: from the shape alone first, then the environment, then whether the kernel covers it.)
 bool OperatorPreferred(const kxc_hip_conv2d_desc* d, PackedLaunch* L) {
     const int K = d->kh, S = d->stride_h;
     if (K != d->kw || S != d->stride_w || d->n <= 0 || d->c <= 0 || d->o <= 0 || (S != 1 && S != 2) || K > 7) return false;
-    if (!Switched(OperatorRule(d))) return false;
-    const char* variant = std::getenv("KXC_HIP_CONV_VARIANT");
-    return !(variant && *variant) && Resolve(d, false, L) && L->filter_bytes <= (32u << 20);      // (bounds the scratch kept per stream)
+    return Switched(OperatorRule(d)) && !OthersForced() && Resolve(d, false, L) && L->filter_bytes <= (32u << 20);      // (bounds the scratch kept per stream)
 }
 
 }  // namespace

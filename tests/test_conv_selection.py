@@ -103,3 +103,26 @@ def test_stride_2_nodes_take_the_packed_kernel_where_it_is_the_faster_one(pkg, m
     for name in ("KXC_HIP_CONV_BF16X3", "KXC_HIP_WINOGRAD_BF16X3"):
         monkeypatch.delenv(name, raising=False)
     assert (_node(pkg, xs, o, 3, second) > 0) == packed
+
+
+@pytest.mark.parametrize("xs, o, k, stride, packed", [
+    # us, fp32 instructions and packed
+    ((8, 64, 27, 27), 96, 5, 1, True),          # 38, 25
+    ((32, 128, 28, 28), 512, 1, 1, True),       # 74, 50
+    ((1, 226, 26, 33), 161, 7, 1, True),        # 72, 44
+    ((4, 13, 64, 12), 356, 7, 1, True),         # 32, 25
+    ((27, 220, 9, 10), 260, 3, 1, True),        # 48, 35
+    ((37, 32, 19, 12), 32, 5, 1, False),        # 16, 21
+    ((11, 6, 60, 48), 126, 5, 1, False),        # 18, 27
+    ((1, 64, 15, 16), 96, 7, 1, False),         # 18, 25
+    ((11, 16, 90, 9), 144, 3, 1, False),        # 12, 17
+    ((3, 32, 100, 31), 208, 3, 1, False),       # 18, 22
+    ((2, 120, 14, 48), 35, 1, 1, False),        # 6, 11
+    ((3, 400, 22, 78), 448, 1, 1, False),       # 27, 31
+    ((7, 160, 37, 23), 400, 1, 1, False),       # 18, 30
+])
+def test_single_calls_take_the_packed_kernel_where_it_is_the_faster_one(pkg, monkeypatch, xs, o, k, stride, packed):
+    for name in ("KXC_HIP_CONV_BF16X3", "KXC_HIP_WINOGRAD_BF16X3"):
+        monkeypatch.delenv(name, raising=False)
+    for flags in (5, 7):
+        assert _variant(pkg, xs, o, k, stride, flags=flags).endswith("_bf16x3") == packed
