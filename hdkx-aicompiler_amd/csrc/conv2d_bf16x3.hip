@@ -196,10 +196,10 @@ bool Switched(bool by_rule) {
     return !(w && w[0] == '0');
 }
 
-// A switch that names one of the other kernels keeps those.
+// Switches that name one of the other kernels or say in how many parts it splits its reduction keep those.
 bool OthersForced() {
     const char* variant = std::getenv("KXC_HIP_CONV_VARIANT");
-    return variant && *variant;
+    return (variant && *variant) || std::getenv("KXC_HIP_CONV_GSPLIT");
 }
 
 // us of the launches but `fixed`: workgroups of `start` + `step` per step, `second` times that where two share a compute unit, and

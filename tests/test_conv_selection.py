@@ -126,3 +126,12 @@ def test_single_calls_take_the_packed_kernel_where_it_is_the_faster_one(pkg, mon
         monkeypatch.delenv(name, raising=False)
     for flags in (5, 7):
         assert _variant(pkg, xs, o, k, stride, flags=flags).endswith("_bf16x3") == packed
+
+
+@pytest.mark.parametrize("name, value", [("KXC_HIP_CONV_VARIANT", "direct"), ("KXC_HIP_CONV_GSPLIT", "2")])
+def test_switches_that_force_another_kernel_s_shape(pkg, monkeypatch, name, value):
+    """A workgroup shape or a split that the environment names is that of the kernels on the fp32 instructions."""
+    monkeypatch.delenv("KXC_HIP_CONV_BF16X3", raising=False)
+    monkeypatch.setenv(name, value)
+    assert not any(_variant(pkg, xs, o, k).startswith("mfma_") and _variant(pkg, xs, o, k).endswith("_bf16x3") for xs, o, k in CALLS)
+    assert not any(_node(pkg, *n) for n in NODES)
