@@ -681,6 +681,23 @@ int ThreePartSplit(int64_t units, int ksteps, int64_t out_elems) {
     return best;
 }
 
+// us of a launch on the bf16 matrix cores and of one on the fp32 instructions (`v`), both with their adding launch; fitted to 500 shapes
+// of 32 to 512 and 8 to 512 channels within 7 % (nine in ten: 16 and 20 %).  A workgroup of the one fills a compute unit.
+double ThreePartUs(const kxc_hip_conv2d_desc* d, int64_t out_elems, int64_t lanes) {
+    const int64_t units = CeilDiv(Tiles(d), wino_bx::kTiles) * CeilDiv(d->o, wino_bx::kOut) * lanes;
+    const int ksteps = static_cast<int>(CeilDiv(d->c, wino_bx::kStep)), split = ThreePartSplit(units, ksteps, out_elems);
+    return 2.5 + static_cast<double>(CeilDiv(units * split, 256)) * (6.9 + 2.16 * static_cast<double>(CeilDiv(ksteps, split))) +
+           (split > 1 ? 1 + 8.0 * split * static_cast<double>(out_elems) / 4.5e6 : 0);
+}
+double Fp32Us(const kxc_hip_conv2d_desc* d, const WinoVariant* v, int64_t out_elems, int64_t lanes) {
+    const int64_t units = CeilDiv(Tiles(d), 16 * v->wt) * CeilDiv(d->o, 64) * lanes;
+    const int csteps = d->c / 4, split = v->ks == 1 ? GroupSplit(units, csteps, out_elems) : 1;
+    const double fixed = v->ks == 2 ? (v->wt == 2 ? 10 : 6.6) : v->wt == 2 ? 7.4 : 5.5;
+    const double step = v->ks == 2 ? (v->wt == 2 ? 1.18 : 0.87) : v->wt == 2 ? 0.7 : 0.56;
+    return fixed + step * static_cast<double>(CeilDiv(csteps, split * v->ks)) * std::max(1.0, static_cast<double>(units * split) / 215) +
+           (split > 1 ? 8.0 * split * static_cast<double>(out_elems) / 4.5e6 : 0);
+}
+
 // Measured on MI355X: 64 x 32 workgroups (four waves) are the fastest shape once there is one per two compute units;
 // smaller launches run faster as twice as many 64 x 16 workgroups of two waves.
 // (three_part = false: the fp32 instructions)
@@ -694,16 +711,20 @@ const WinoVariant* SelectWino(const kxc_hip_conv2d_desc* d, bool three_part = tr
     const int csteps = d->c / 4;
     const int64_t oh = static_cast<int64_t>(d->h) + 2 * d->pad_h - 2, ow = static_cast<int64_t>(d->w) + 2 * d->pad_w - 2;
     const int64_t lanes = SelectLanes();
-    // From 18 million (tile, output channel, input channel) triples on the bf16 matrix cores win, 36 million where rows hold an odd
-    // number of values (their last pieces of 16 bytes and last tiles are partly padding), 26 million below 96 channels (faster
-    // here from 18 on too, but a test of saved plans holds the fp32 form of 8 images of 64 channels at 56 x 56: 19.9 and 16.9).  us, fp32 instructions and here: 64 channels
+    // From 36 million (tile, output channel, input channel) triples on the bf16 matrix cores win; where rows hold an even number of values
+    // (of odd ones the last pieces of 16 bytes and last tiles are partly padding) from 18 million, 26 million below 96 channels (faster
+    // here from 18 on too, but a test of saved plans holds the fp32 form of 8 images of 64 channels at 56 x 56: 19.9 and 16.9), if what
+    // both sides take says so (54 of 65 shapes between the lines, none slower by more than 3 %): a second round of workgroups that is nearly empty (32 ->
+    // 300 at 16 x 58, batch 16 24.8 and 29.6) or a few in many parts (512 -> 64 at 10 x 60, batch 4 20.4 and 23.4) cost more.  us, fp32 instructions and here: 64 channels
     // at 48 x 48, batch 8 (18.9 million) 18.4 and 16.4; at 56 x 56, batch 5 (16.1) 16.4 and 16.5, 6 19.6 and 16.6, 10 20.3 and 17.1, 12 30.4 and
     // 17.5; 128 at 28 x 28, batch 6 (19.3) 21.1 and 17.8, 10 21.6 and 20.7; 256 at 14 x 14, batch 6 23.0 and 20.7, 10 24.5 and 23.7; at 10 x 10, batch 12
     // (19.7) 23.6 and 20.8.  Odd: 64 at 49 x 49, batch 11 (28.2) 21.1 and 23.3, 14 (35.8) 34.4 and 23.8; 128 at 25 x 25, batch 8 (22.2) 22.9 and 21.3, 11
     // (30.5) 23.1 and 24.4; 256 at 13 x 13, batch 8 (25.7) 24.2 and 25.4; 512 at 7 x 7, batch 6 (25.2) 22.4 and 22.0.
     // KXC_HIP_WINOGRAD_BF16X3=0 keeps the fp32 instructions.
     const char* bx = std::getenv("KXC_HIP_WINOGRAD_BF16X3");
-    if (three_part && !(bx && bx[0] == '0') && Tiles(d) * lanes * d->o * d->c >= (d->w % 2 != 0 ? 36000000LL : d->c < 96 ? 26000000LL : 18000000LL) && ThreePartFits(d)) {
+    const int64_t triples = Tiles(d) * lanes * d->o * d->c, out_elems = static_cast<int64_t>(d->n) * d->o * oh * ow;
+    if (three_part && !(bx && bx[0] == '0') && triples >= (d->w % 2 != 0 ? 36000000LL : d->c < 96 ? 26000000LL : 18000000LL) && ThreePartFits(d) &&
+        (triples >= 36000000LL || ThreePartUs(d, out_elems, lanes) < 0.97 * Fp32Us(d, SelectWino(d, false), out_elems, lanes))) {
         for (int i = 0; i < kNumWino; ++i)
             if (!kWino[i].kernel) return &kWino[i];
     }
@@ -713,7 +734,7 @@ const WinoVariant* SelectWino(const kxc_hip_conv2d_desc* d, bool three_part = tr
     // 256 channels at 13 x 13, batch 6 26.0 -> 22.9 us, 512 at 7 x 7 26.4 -> 22.8, 128 at 28 x 28, batch 4 18.2 -> 16.3;
     // below it 13.0 against 13.5 (128 at 28 x 28, batch 2), 14.2 against 16.3 (512 at 7 x 7).
     const int64_t units_t1 = CeilDiv(Tiles(d), 16) * CeilDiv(d->o, 64) * lanes;
-    if (GroupSplit(units_t1, csteps, static_cast<int64_t>(d->n) * d->o * oh * ow) > 1) {
+    if (GroupSplit(units_t1, csteps, out_elems) > 1) {
         const int wt = Tiles(d) * lanes * d->o * d->c >= 12000000LL ? 2 : 1;
         for (int i = 0; i < kNumWino; ++i)
             if (kWino[i].wk == 2 && kWino[i].wt == wt && kWino[i].ks == 1) return &kWino[i];

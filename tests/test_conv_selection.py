@@ -135,3 +135,22 @@ def test_switches_that_force_another_kernel_s_shape(pkg, monkeypatch, name, valu
     monkeypatch.setenv(name, value)
     assert not any(_variant(pkg, xs, o, k).startswith("mfma_") and _variant(pkg, xs, o, k).endswith("_bf16x3") for xs, o, k in CALLS)
     assert not any(_node(pkg, *n) for n in NODES)
+
+
+@pytest.mark.parametrize("xs, o, three_part", [
+    # us, fp32 instructions and bf16 matrix cores
+    ((6, 128, 28, 28), 128, True),              # 21.1, 17.8
+    ((6, 256, 14, 14), 256, True),              # 23.0, 20.7
+    ((12, 256, 10, 10), 256, True),             # 23.6, 20.8
+    ((13, 384, 65, 16), 16, True),              # 45, 23: fp32 workgroups a quarter full
+    ((9, 512, 20, 24), 64, True),               # 35, 20
+    ((16, 32, 16, 58), 300, False),             # 24.8, 29.6: a nearly empty second round of workgroups
+    ((4, 512, 10, 60), 64, False),              # 20.4, 23.4
+    ((12, 128, 43, 14), 128, False),            # 20.3, 24.6
+    ((3, 200, 9, 70), 192, False),              # 19.3, 20.8
+])
+def test_winograd_nodes_take_the_bf16_matrix_cores_where_they_are_faster(pkg, monkeypatch, xs, o, three_part):
+    """18 to 36 million (tile, output channel, input channel) triples."""
+    for name in ("KXC_HIP_WINOGRAD_BF16X3", "KXC_HIP_WINOGRAD_VARIANT"):
+        monkeypatch.delenv(name, raising=False)
+    assert pkg.conv2d_winograd_variant(xs, (o, xs[1], 3, 3)).endswith("_bf16x3") == three_part
