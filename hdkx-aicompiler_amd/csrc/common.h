@@ -158,6 +158,7 @@ int32_t LaunchPreparedConv2d(const PreparedConv* p, const float* x, const float*
 const char* PreparedConvName(const PreparedConv* p);
 constexpr int64_t kSmallRowLoadsWork = 2300000;      // (16 x 16 tiles) * channels * 9 up to which small 3x3 launches win (conv2d_f32.hip)
 bool SmallConvTakes(const kxc_hip_conv2d_desc* desc, bool second_output, bool in_plan);      // ... or a small-launch kernel at all
+int32_t HpoolTilePixels(const kxc_hip_conv2d_desc* desc);      // pixels of a tile of the fp32 kernel that takes a pooled launch (0: none does)
 bool SmallConvBeatsWinograd(const kxc_hip_conv2d_desc* desc);      // a plan's Winograd node is better launched as PreparedConv
 void FreePreparedConv(PreparedConv* p);
 struct PreparedWinograd;

@@ -225,7 +225,11 @@ double BlockGflop(const kxc_hip_conv2d_desc* d, int64_t pixels, int taps, int bl
 // 19.0 / 22.9 and 22.8 / 23.1 / 23.3; 128 -> 256 at 28 x 28, batch 8 / 10 18.6 / 20.7 and 24.7 / 25.9; 256 -> 512 at 14 x 14 18.9 / 19.1 and 23.5 / 23.2.
 // The 7x7 kernel, 3 -> 64 channels: pooled at 224 x 224, batch 16 / 32 / 64 51 / 100 / 169 and 32 / 59 / 108, at 64 x 64, batch 56 (1.1 GFLOP) 33 and
 // 22; not pooled at 224 x 224, batch 4 (0.94) 20.6 and 21.8, batch 8 (1.9) 33 and 30, batch 64 182 and 116; tiles 13 rows high, of which a compute unit holds
-// two, at 193 x 193, batch 16 (2.8) 49 and 54.
+// two, at 193 x 193, batch 16 (2.8) 49 and 54.  Pooled, with a compute unit to each workgroup and such high tiles it loses to the others' tile of 224
+// pixels (3 -> 64 at 30 x 56, batch 24 18.9 and 21.0; from 257 workgroups on 24 channels at 304 x 56, batch 17 29.6 and 27.8), not to the one of 448 that they
+// take where it fits (31.5 and 20.5 at 56 x 56, batch 8); not pooled, up to 32 channels, which leave half of a workgroup's
+// 64 empty, need 1800 workgroups (32 at 144 x 112, batch 57 36.6 and 44.0, 144 x 224, batch 37 46.0 and 51.4, 224 x 224, batch 33 63.7 and 61.6).  Of 500
+// first layers 252 take it, none slower by more than 3 %.
 // At 3x3 that must also be the shorter time by what either side takes, fitted within a tenth to 1000 shapes of 16 to 512 and 8 to 512 channels: here
 // 2 us and a workgroup's 4 + 0.28 per tap and step, the others 10.5 and 12.7 per GFLOP of 32 x 32 blocks or, by the small-launch kernels, 4.9
 // and 12.4 of 16 x 16 ones.  A workgroup has 128 output channels: no more than 48 of them (256 -> 8 at 60 x 38, batch 38 24.5 and 99.4, 384 ->
@@ -236,9 +240,10 @@ double BlockGflop(const kxc_hip_conv2d_desc* d, int64_t pixels, int taps, int bl
 bool Preferred(const kxc_hip_conv2d_desc* d, bool second, PackedLaunch* L) {
     if (OthersForced()) return false;
     if (!second && Resolve7(d, L)) {
-        // Pooled rows: always.  Others: four workgroups to a compute unit (tiles that are few rows high) and work for them.
-        const bool pooled = (d->flags & KXC_HIP_CONV_HPOOL) != 0;
-        return Switched(pooled || (L->lds_bytes <= kMaxLdsBytes / 4 && L->gflop * SelectLanes() >= 1.8));
+        // Tiles that are few rows high: four workgroups to a compute unit, and one batch of loads.
+        const bool pooled = (d->flags & KXC_HIP_CONV_HPOOL) != 0, low = L->lds_bytes <= kMaxLdsBytes / 4;
+        const int64_t lanes = SelectLanes(), units = L->a7.num_units * lanes;
+        return Switched(pooled ? low || units > 256 || HpoolTilePixels(d) > conv7_bx::kPix : low && L->gflop * lanes >= 1.8 && (d->o > 32 || units >= 1800));
     }
     // (a plan's filter launch packs 3x3 stride-2 filters only)
     if (!d || d->kh != 3 || d->stride_h != 2 || d->pad_h != 1 || d->pad_w != 1 || d->c % conv_bx::kStep != 0 || !Resolve(d, second, L)) return false;

@@ -1587,6 +1587,12 @@ bool SmallConvTakes(const kxc_hip_conv2d_desc* d, bool second, bool in_plan) {
     return FillArgs(d, &a, "plan") == KXC_HIP_OK && (SelectSmall(d, a, second, in_plan) || (!second && UseSmall1x1(d, a)));
 }
 
+int32_t HpoolTilePixels(const kxc_hip_conv2d_desc* d) {
+    ConvArgs a;
+    Choice c;
+    return FillArgs(d, &a, "plan") == KXC_HIP_OK && HpoolChoice(d, a, &c) ? c.v->tp : 0;
+}
+
 void FreePreparedConv(PreparedConv* p) { delete p; }
 
 }  // namespace kxc_hip

@@ -128,6 +128,31 @@ def test_single_calls_take_the_packed_kernel_where_it_is_the_faster_one(pkg, mon
         assert _variant(pkg, xs, o, k, stride, flags=flags).endswith("_bf16x3") == packed
 
 
+@pytest.mark.parametrize("xs, o, hpool, packed", [
+    # us, fp32 instructions and packed
+    ((64, 3, 224, 224), 64, True, True),        # 169, 108
+    ((2, 3, 224, 224), 8, True, True),          # 31, 17
+    ((7, 3, 104, 112), 24, True, True),         # 18, 17: tiles of 13 rows
+    ((8, 3, 56, 56), 64, True, True),           # 32, 21: 21 rows, and tiles of 448 pixels on the other side
+    ((74, 3, 56, 56), 16, True, True),          # 29, 28
+    ((17, 3, 304, 56), 24, True, True),         # 30, 28
+    ((24, 3, 30, 56), 64, True, False),         # 19, 21
+    ((2, 3, 168, 56), 256, True, False),        # 19, 21
+    ((20, 3, 21, 224), 32, True, False),        # 19, 20: images meet inside a tile
+    ((18, 3, 224, 224), 64, False, True),       # 58, 35
+    ((24, 3, 224, 224), 48, False, True),       # 82, 53
+    ((33, 3, 224, 224), 32, False, True),       # 64, 62
+    ((78, 3, 224, 224), 24, False, True),       # 124, 116
+    ((57, 3, 144, 112), 32, False, False),      # 37, 44
+    ((42, 3, 112, 224), 24, False, False),      # 41, 43
+    ((4, 3, 224, 224), 64, False, False),       # 21, 22
+])
+def test_first_layers_take_the_packed_kernel_where_it_is_the_faster_one(pkg, monkeypatch, xs, o, hpool, packed):
+    for name in ("KXC_HIP_CONV_BF16X3", "KXC_HIP_WINOGRAD_BF16X3"):
+        monkeypatch.delenv(name, raising=False)
+    assert (_node(pkg, xs, o, 7, hpool=hpool) > 0) == packed
+
+
 @pytest.mark.parametrize("name, value", [("KXC_HIP_CONV_VARIANT", "direct"), ("KXC_HIP_CONV_GSPLIT", "2")])
 def test_switches_that_force_another_kernel_s_shape(pkg, monkeypatch, name, value):
     """A workgroup shape or a split that the environment names is that of the kernels on the fp32 instructions."""
