@@ -198,8 +198,11 @@ bool Switched(bool by_rule) {
 
 // Switches that name one of the other kernels or say in how many parts it splits its reduction keep those.
 bool OthersForced() {
-    const char* variant = std::getenv("KXC_HIP_CONV_VARIANT");
-    return (variant && *variant) || std::getenv("KXC_HIP_CONV_GSPLIT");
+    for (const char* name : {"KXC_HIP_CONV_VARIANT", "KXC_HIP_CONV_HPOOL_VARIANT"}) {
+        const char* variant = std::getenv(name);
+        if (variant && *variant) return true;
+    }
+    return std::getenv("KXC_HIP_CONV_GSPLIT") != nullptr;
 }
 
 // us of the launches but `fixed`: workgroups of `start` + `step` per step, `second` times that where two share a compute unit, and

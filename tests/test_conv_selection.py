@@ -153,7 +153,7 @@ def test_first_layers_take_the_packed_kernel_where_it_is_the_faster_one(pkg, mon
     assert (_node(pkg, xs, o, 7, hpool=hpool) > 0) == packed
 
 
-@pytest.mark.parametrize("name, value", [("KXC_HIP_CONV_VARIANT", "direct"), ("KXC_HIP_CONV_GSPLIT", "2")])
+@pytest.mark.parametrize("name, value", [("KXC_HIP_CONV_VARIANT", "direct"), ("KXC_HIP_CONV_GSPLIT", "2"), ("KXC_HIP_CONV_HPOOL_VARIANT", "mfma_k7x7_t1_o1x2_p7x1")])
 def test_switches_that_force_another_kernel_s_shape(pkg, monkeypatch, name, value):
     """A workgroup shape or a split that the environment names is that of the kernels on the fp32 instructions."""
     monkeypatch.delenv("KXC_HIP_CONV_BF16X3", raising=False)
