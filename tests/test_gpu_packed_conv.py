@@ -99,6 +99,24 @@ def test_conv_on_a_packed_filter(pkg, monkeypatch, xs, o, second, residual, bias
     node.plan.close()
 
 
+@pytest.mark.parametrize("xs, o, second, k, hpool, packed", [
+    ((16, 64, 56, 56), 128, True, 3, False, True), ((2, 64, 56, 56), 128, True, 3, False, False),
+    ((21, 96, 26, 16), 512, False, 3, False, True), ((14, 512, 8, 38), 160, False, 3, False, False),
+    ((8, 48, 74, 74), 64, False, 3, False, True), ((2, 48, 74, 74), 64, False, 3, False, False),      # fewer than 64 channels
+    ((38, 64, 60, 38), 8, False, 3, False, False),                                                    # few output channels
+    ((18, 3, 224, 224), 64, False, 7, False, True), ((4, 3, 224, 224), 64, False, 7, False, False),
+    ((7, 3, 104, 112), 24, False, 7, True, True), ((24, 3, 30, 56), 64, False, 7, True, False),
+])
+def test_nodes_on_both_sides_of_the_lines(pkg, monkeypatch, xs, o, second, k, hpool, packed):
+    """What a plan's stride-2 nodes launch when no switch is set."""
+    for name in ("KXC_HIP_CONV_BF16X3", "KXC_HIP_WINOGRAD_BF16X3"):
+        monkeypatch.delenv(name, raising=False)
+    node = _Node(pkg, xs, o, second, seed=o, k=k, pad=k // 2, hpool=hpool)
+    assert (node.bytes > 0) == packed == ("bf16x3" in node.plan.node_symbol(0))
+    node.check(node.run())
+    node.plan.close()
+
+
 @pytest.mark.parametrize("xs, o, pad, residual, bias, relu, hpool", [
     ((1, 3, 224, 224), 64, 3, False, True, True, True),     # two rows of 112 columns a tile
     ((7, 3, 64, 64), 40, 3, False, True, True, True),       # seven rows of 32; the second block of channels ends after 8
