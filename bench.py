@@ -444,7 +444,8 @@ def bench_conv_layers(torch, pkg, synth, dev, batch):
                                "matrix_core_frac": round(executed / (wms * 1e-3) / 1e12 / matrix_peak, 4), "matrix_core_peak": matrix_peak}
         if name == "conv1":
             row["note"] = ("launched back to back: the 205 MB of output of one launch compete with the write-back of the "
-                           "launch before; inside the network the same launch takes about 0.18 ms (launches_in_network)")
+                           "launch before; a batch-64 plan runs this layer by another kernel, on packed filters and with the columns "
+                           "of the max pool, in about 0.1 ms (launches_in_network)")
         rows.append(row)
     return rows
 
