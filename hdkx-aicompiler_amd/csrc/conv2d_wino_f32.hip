@@ -977,7 +977,8 @@ const char* const kWinogradOperatorName = kThreePart;
 
 // A call pays for the filter transform (a launch, about 5 us) and for whole workgroups of 64 channels x 64 tiles, one per
 // compute unit at a time.  Both sides' times follow a line within about 10 % (us): here 12 + rounds * (10 + 2.5 * steps of 16
-// channels), the other kernels 14 + 10.5 per GFLOP.  Measured, other kernels and here: 90 -> 150 channels at 37 x 51, batch 7
+// channels; measured with 4-byte patch loads, 16-byte ones take 2.2, which keeps so much more in hand), the other kernels 14 + 10.5
+// per GFLOP.  Measured, other kernels and here: 90 -> 150 channels at 37 x 51, batch 7
 // 54 and 40; 64 -> 64 at 56 x 56, batch 8 29.6 both, 16 52 and 33, 64 148 and 94; 128 -> 128 at 28 x 28, batch 8 34 and 41, 16
 // 50 and 42, 64 153 and 76; 256 -> 256 at 14 x 14, batch 16 52 and 59, 64 161 and 64; 512 -> 512 at 7 x 7, batch 64 169 and
 // 98; 16 -> 64 at 60 x 60, batch 40 41 and 46.  A tenth in hand also keeps out the launches whose reduction the other
