@@ -7,6 +7,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <string>
 
@@ -160,13 +161,15 @@ constexpr int64_t kSmallRowLoadsWork = 2300000;      // (16 x 16 tiles) * channe
 bool SmallConvTakes(const kxc_hip_conv2d_desc* desc, bool second_output, bool in_plan);      // ... or a small-launch kernel at all
 int32_t HpoolTilePixels(const kxc_hip_conv2d_desc* desc);      // pixels of a tile of the fp32 kernel that takes a pooled launch (0: none does)
 bool SmallConvBeatsWinograd(const kxc_hip_conv2d_desc* desc);      // a plan's Winograd node is better launched as PreparedConv
+bool SmallConvStagesRows(const kxc_hip_conv2d_desc* desc);         // ... by the kernel that stages whole rows
 void FreePreparedConv(PreparedConv* p);
 struct PreparedWinograd;
 // A node whose filter buffer has u_bytes, holding the one form that the launch reads.  *out = nullptr: no form fits.
-int32_t PrepareWinograd(const kxc_hip_conv2d_desc* desc, size_t u_bytes, PreparedWinograd** out);
+int32_t PrepareWinograd(const kxc_hip_conv2d_desc* desc, size_t u_bytes, PreparedWinograd** out, bool may_slice = true);
 const char* PreparedWinogradName(const PreparedWinograd* p);
 size_t WinogradF32FilterBytes(const kxc_hip_conv2d_desc* desc);
-int32_t LaunchPreparedWinograd(const PreparedWinograd* p, const float* x, const float* u, const float* bias,
+double WinogradNodeUs(const kxc_hip_conv2d_desc* desc);      // us of a plan's Winograd node without the kernel of conv_slice.h (0: never take that)
+int32_t LaunchPreparedWinograd(const PreparedWinograd* p, const float* x, const float* w, const float* u, const float* bias,
                                const float* residual, float* y, hipStream_t stream);
 void FreePreparedWinograd(PreparedWinograd* p);
 
@@ -179,6 +182,18 @@ const char* PreparedPackedName(const PreparedPacked* p);
 int32_t LaunchPreparedPacked(const PreparedPacked* p, const float* x, const float* w, const void* u, const float* bias, const float* residual,
                              float* y, const float* w2, const float* bias2, float* y2, hipStream_t stream);
 void FreePreparedPacked(PreparedPacked* p);
+// The same for small launches (conv2d_slice.hip), 3x3 with stride 1 or, with the second output, 2.
+struct PreparedSlice;
+size_t SliceFilterBytes(const kxc_hip_conv2d_desc* desc, bool second_output);
+PreparedSlice* PrepareSlice(const kxc_hip_conv2d_desc* desc, bool second_output, size_t u_bytes);
+const char* PreparedSliceName(const PreparedSlice* p);
+int32_t LaunchPreparedSlice(const PreparedSlice* p, const float* x, const float* w, const void* u, const float* bias, const float* residual, float* y,
+                            const float* w2, const float* bias2, float* y2, hipStream_t stream);
+void FreePreparedSlice(PreparedSlice* p);
+struct PreparedSliceDelete {
+    void operator()(PreparedSlice* p) const { FreePreparedSlice(p); }
+};
+using PreparedSlicePtr = std::unique_ptr<PreparedSlice, PreparedSliceDelete>;
 // A single nn_conv2d by one of these kernels, its filter packed first: the kernel's name (nullptr: not for this shape), and the
 // call.  *launched = false, nothing enqueued: not for this shape (*preferred says), no scratch for the filter, or the stream does
 // not order it.
@@ -195,12 +210,12 @@ extern const char* const kWinogradOperatorName;
 
 // The filter transforms of several Winograd layers, and the packed filters of other convolutions, in one launch
 // (conv2d_wino_f32.hip).
-constexpr uint32_t kWinoFormF32 = 1, kWinoFormThreePart = 2, kFormPacked = 4;
+constexpr uint32_t kWinoFormF32 = 1, kWinoFormThreePart = 2, kFormPacked = 4, kFormSlice = 8;
 struct WinoWeightJob {
     const kxc_hip_conv2d_desc* desc;
     const float* w;      // OIHW weights
     float* u;            // where they go, the fp32 form first
-    uint32_t forms;      // kWinoForm*: the forms of the filter to write (PreparedWinogradForms: what a node's launch reads), or kFormPacked
+    uint32_t forms;      // kWinoForm*: the forms of the filter to write (PreparedWinogradForms: what a node's launch reads), kFormPacked or kFormSlice
     const float* w2;     // kFormPacked: the second output's weights, or nullptr
 };
 uint32_t PreparedWinogradForms(const PreparedWinograd* p);

@@ -27,21 +27,6 @@ struct PackedLaunch {
     size_t scratch_bytes = 0;
 };
 
-// How far `pix` neighbouring pixels (flattened over n, oh, ow) that start at a multiple of pix reach at most: `row` for every step to
-// the next output row and `image` for every step to the next image.  Within an image, where tiles start in a row repeats after
-// at most OW tiles; where the border of two images lies in a tile repeats after at most pix images.
-int32_t TileReach(int32_t N, int32_t OHW, int32_t OW, int32_t pix, int32_t row, int32_t image) {
-    const uint32_t p = static_cast<uint32_t>(pix), ow = static_cast<uint32_t>(OW), ohw = static_cast<uint32_t>(OHW), M = static_cast<uint32_t>(N) * ohw;
-    uint32_t best = 0;
-    auto tile = [&](uint32_t m0) {
-        const uint32_t last = std::min(p, M - m0) - 1;
-        best = std::max(best, (m0 % ow + last) / ow * static_cast<uint32_t>(row) + (m0 % ohw + last) / ohw * static_cast<uint32_t>(image));
-    };
-    for (uint32_t t = 0; t < ow && t * p < M; ++t) tile(t * p);
-    for (uint32_t n = 1; n < static_cast<uint32_t>(N) && n <= p; ++n) tile(n * ohw / p * p);
-    return static_cast<int32_t>(best);
-}
-
 // Parts of a reduction, while all of them together are at most one workgroup per compute unit: what gives the shortest of
 // 0.29 us per tap and 16 channels + the adding launch (5 us and the parts' way to memory and back at 4.5 TB/s).  us, 1 / 2 / 4 / 8
 // parts without the adding launch: 64 -> 128 channels at 49 x 49, batch 6 (59 workgroups) 19.9 / 14.8 / 12.9; 128 -> 256 at 25 x
@@ -163,7 +148,7 @@ bool Resolve7(const kxc_hip_conv2d_desc* d, PackedLaunch* L) {
     a.Hp = static_cast<int32_t>(Hp); a.PW = a.OW / 2;
     const int pitch = OW + 3 <= 64 ? 64 : 120;      // (the last pixel's window takes four words; three parts within the reach of a ds_read2)
     if (OW + 3 > pitch) return false;
-    const int64_t rows = TileReach(a.N, a.OHW, a.OW, kPix, 2, a.Hp - 2 * a.OH) + kK;
+    const int64_t rows = conv_bx::TileReach(a.N, a.OHW, a.OW, kPix, 2, a.Hp - 2 * a.OH) + kK;
     a.row_max = static_cast<int32_t>(rows);
     if (LdsBytes(rows, pitch) > kMaxLdsBytes / 2) return false;
     a.o_tiles = static_cast<int32_t>(CeilDiv(a.O, kOut));
@@ -380,23 +365,31 @@ int32_t RunPackedOperator(const kxc_hip_conv2d_desc* desc, const float* x, const
 
 struct PreparedPacked {
     PackedLaunch launch;
+    PreparedSlicePtr slice;      // the launch, where it is set
 };
 
 size_t PackedFilterBytes(const kxc_hip_conv2d_desc* desc, bool second) {
     PackedLaunch L;
+    if (const size_t bytes = desc && desc->stride_h == 2 ? SliceFilterBytes(desc, second) : 0) return bytes;
     return Preferred(desc, second, &L) ? L.filter_bytes : 0;
 }
 
 void PreparePacked(const kxc_hip_conv2d_desc* desc, bool second, size_t u_bytes, PreparedPacked** out) {
     std::unique_ptr<PreparedPacked> p(new PreparedPacked);
+    if (desc->stride_h == 2) p->slice.reset(PrepareSlice(desc, second, u_bytes));
+    if (p->slice) {
+        *out = p.release();
+        return;
+    }
     *out = Preferred(desc, second, &p->launch) && u_bytes >= p->launch.filter_bytes ? p.release() : nullptr;
 }
 
-const char* PreparedPackedName(const PreparedPacked* p) { return p->launch.name; }
+const char* PreparedPackedName(const PreparedPacked* p) { return p->slice ? PreparedSliceName(p->slice.get()) : p->launch.name; }
 void FreePreparedPacked(PreparedPacked* p) { delete p; }
 
 int32_t LaunchPreparedPacked(const PreparedPacked* p, const float* x, const float* w, const void* u, const float* bias, const float* residual,
                              float* y, const float* w2, const float* bias2, float* y2, hipStream_t s) {
+    if (p->slice) return LaunchPreparedSlice(p->slice.get(), x, w, u, bias, residual, y, w2, bias2, y2, s);
     const PackedLaunch& L = p->launch;
     const uint32_t flags = L.kernel7 ? L.a7.flags : L.a.flags;
     KXC_HIP_REQUIRE(x && w && u && y && (!L.second || (w2 && y2)), "%s: NULL pointer", L.name);

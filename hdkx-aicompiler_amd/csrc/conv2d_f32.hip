@@ -1582,6 +1582,11 @@ bool SmallConvBeatsWinograd(const kxc_hip_conv2d_desc* d) {
            CeilDiv(a.M, 16) * CeilDiv(a.O, 16) * SelectLanes() * a.C * 9 <= (SmallRowLoads(a) && a.O % 16 == 0 ? 1400000 : 1100000);
 }
 
+bool SmallConvStagesRows(const kxc_hip_conv2d_desc* d) {
+    ConvArgs a;
+    return FillArgs(d, &a, "plan") == KXC_HIP_OK && SelectSmall(d, a, false, true) == kSmall;
+}
+
 bool SmallConvTakes(const kxc_hip_conv2d_desc* d, bool second, bool in_plan) {
     ConvArgs a;
     return FillArgs(d, &a, "plan") == KXC_HIP_OK && (SelectSmall(d, a, second, in_plan) || (!second && UseSmall1x1(d, a)));

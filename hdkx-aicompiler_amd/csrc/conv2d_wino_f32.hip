@@ -156,7 +156,7 @@ struct WinoWeightBatch {
     int32_t O[kMaxWeightJobs], C[kMaxWeightJobs], first_block[kMaxWeightJobs + 1];
     const float* w2[kMaxWeightJobs];
     uint32_t three_part;       // bit j: job j writes the three-part form
-    uint32_t packed, packed7;  // ... the filter of conv_bf16x3.h, of conv7_bf16x3.h
+    uint32_t packed, packed7, slice;  // ... the filter of conv_bf16x3.h with stride 2, of conv7_bf16x3.h, of conv_slice.h with stride 1
     int32_t count;
 };
 __global__ void __launch_bounds__(256) wino_weight_batch_kernel(const WinoWeightBatch b) {
@@ -167,6 +167,7 @@ __global__ void __launch_bounds__(256) wino_weight_batch_kernel(const WinoWeight
     static_assert(conv_bx::PackFloats(3) <= sizeof(raw) / sizeof(float), "one block of LDS for all forms");
     if ((b.packed7 >> j) & 1u) conv7_bx::pack_tile(b.w[j], b.u[j], b.O[j], tile);
     else if ((b.packed >> j) & 1u) conv_bx::pack_block<3, 2>(b.w[j], b.w2[j], b.u[j], b.O[j], b.C[j], tile, raw);
+    else if ((b.slice >> j) & 1u) conv_bx::pack_block<3, 1>(b.w[j], nullptr, b.u[j], b.O[j], b.C[j], tile, raw);
     else if ((b.three_part >> j) & 1u) wino_bx::weight_tile(b.w[j], b.u[j], b.O[j], b.C[j], tile, raw);
     else wino_weight_tile(b.w[j], reinterpret_cast<float*>(b.u[j]), b.O[j], b.C[j], tile, raw);
 }
@@ -948,11 +949,17 @@ namespace kxc_hip {
 
 struct PreparedWinograd {
     WinoLaunch launch;
+    PreparedSlicePtr slice;      // the launch, where it is set
 };
 
-int32_t PrepareWinograd(const kxc_hip_conv2d_desc* desc, size_t u_bytes, PreparedWinograd** out) {
+int32_t PrepareWinograd(const kxc_hip_conv2d_desc* desc, size_t u_bytes, PreparedWinograd** out, bool may_slice) {
     *out = nullptr;
     std::unique_ptr<PreparedWinograd> p(new PreparedWinograd);
+    if (may_slice) p->slice.reset(PrepareSlice(desc, false, u_bytes));
+    if (p->slice) {
+        *out = p.release();
+        return KXC_HIP_OK;
+    }
     if (int32_t rc = WinoResolve(desc, &p->launch, u_bytes >= wino_bx::WeightBytes(desc->o, desc->c))) return rc;
     if (!p->launch.three_part && u_bytes < F32FilterBytes(desc)) return KXC_HIP_OK;
     p->launch.u_offset = 0;
@@ -960,18 +967,35 @@ int32_t PrepareWinograd(const kxc_hip_conv2d_desc* desc, size_t u_bytes, Prepare
     return KXC_HIP_OK;
 }
 
-const char* PreparedWinogradName(const PreparedWinograd* p) { return p->launch.v->name; }
+const char* PreparedWinogradName(const PreparedWinograd* p) { return p->slice ? PreparedSliceName(p->slice.get()) : p->launch.v->name; }
+
+// Fitted to 1700 shapes within 8 to 10 % (rms).  Where the three-part kernel would be the faster one but is held back by the lines of
+// SelectWino, its estimate counts as well.
+double WinogradNodeUs(const kxc_hip_conv2d_desc* d) {
+    if (!Supported(d)) return 0;
+    const int64_t lanes = SelectLanes(), oh = static_cast<int64_t>(d->h) + 2 * d->pad_h - 2, ow = static_cast<int64_t>(d->w) + 2 * d->pad_w - 2;
+    if (SmallConvBeatsWinograd(d)) {
+        if (SmallConvStagesRows(d)) return 0;      // (the faster one on all of 289 shapes)
+        const double gflop = 18e-9 * static_cast<double>(CeilDiv(d->n * oh * ow, 16) * 16) * static_cast<double>(CeilDiv(d->o, 16) * 16) * d->c;
+        return 4.2 + 13.8 * static_cast<double>(lanes) * gflop;
+    }
+    const WinoVariant* v = SelectWino(d);
+    const int64_t out_elems = static_cast<int64_t>(d->n) * d->o * oh * ow;
+    const double three = ThreePartFits(d) ? 1.11 * ThreePartUs(d, out_elems, lanes) - 0.9 : 1e9;
+    return v->kernel ? std::min(three, 1.11 * Fp32Us(d, v, out_elems, lanes) - 0.7) : three;
+}
 
 size_t WinogradF32FilterBytes(const kxc_hip_conv2d_desc* desc) { return F32FilterBytes(desc); }
 
-int32_t LaunchPreparedWinograd(const PreparedWinograd* p, const float* x, const float* u, const float* bias,
+int32_t LaunchPreparedWinograd(const PreparedWinograd* p, const float* x, const float* w, const float* u, const float* bias,
                                const float* residual, float* y, hipStream_t stream) {
+    if (p->slice) return LaunchPreparedSlice(p->slice.get(), x, w, u, bias, residual, y, nullptr, nullptr, nullptr, stream);
     return WinoRun(p->launch, x, u, bias, residual, y, stream);
 }
 
 void FreePreparedWinograd(PreparedWinograd* p) { delete p; }
 
-uint32_t PreparedWinogradForms(const PreparedWinograd* p) { return p->launch.three_part ? kWinoFormThreePart : kWinoFormF32; }
+uint32_t PreparedWinogradForms(const PreparedWinograd* p) { return p->slice ? kFormSlice : p->launch.three_part ? kWinoFormThreePart : kWinoFormF32; }
 
 const char* const kWinogradOperatorName = kThreePart;
 
@@ -1043,7 +1067,7 @@ int32_t LaunchWinogradWeightTransforms(const WinoWeightJob* jobs, int32_t count,
     for (int32_t j = 0; j < count; ++j) {
         const WinoWeightJob& job = jobs[j];
         KXC_HIP_REQUIRE(job.desc && (job.forms == kFormPacked || Supported(job.desc)) && job.w && job.u, "winograd weight transform: bad job %d", j);
-        for (uint32_t form : {kWinoFormF32, kWinoFormThreePart, kFormPacked}) {
+        for (uint32_t form : {kWinoFormF32, kWinoFormThreePart, kFormPacked, kFormSlice}) {
             if (!(job.forms & form)) continue;
             if (b.count == kMaxWeightJobs)
                 if (int32_t rc = flush()) return rc;
@@ -1055,10 +1079,11 @@ int32_t LaunchWinogradWeightTransforms(const WinoWeightJob* jobs, int32_t count,
             b.first_block[b.count] = static_cast<int32_t>(blocks);
             if (three) b.three_part |= 1u << b.count;
             const bool seven = form == kFormPacked && job.desc->kh == conv7_bx::kK;
+            if (form == kFormSlice) b.slice |= 1u << b.count;
             if (form == kFormPacked) (seven ? b.packed7 : b.packed) |= 1u << b.count;
             b.w2[b.count] = job.w2;
             ++b.count;
-            blocks += seven ? CeilDiv(O, 32) : form == kFormPacked ? conv_bx::PackBlocks(O, C, 3) : form != kWinoFormF32 ? wino_bx::WeightTiles(O, C) : WeightTiles(CeilDiv(O, 32) * 32, C);
+            blocks += seven ? CeilDiv(O, 32) : form == kFormPacked || form == kFormSlice ? conv_bx::PackBlocks(O, C, 3) : form != kWinoFormF32 ? wino_bx::WeightTiles(O, C) : WeightTiles(CeilDiv(O, 32) * 32, C);
             KXC_HIP_REQUIRE(blocks < kMaxGridX, "winograd weight transform: too many blocks");
         }
     }
@@ -1095,7 +1120,10 @@ int32_t kxc_hip_conv2d_winograd_weight_bytes(const kxc_hip_conv2d_desc* desc, si
 int32_t kxc_hip_conv2d_winograd_node_bytes(const kxc_hip_conv2d_desc* desc, size_t* out_bytes) {
     KXC_HIP_REQUIRE(desc && out_bytes, "kxc_hip_conv2d_winograd_node_bytes: NULL argument");
     KXC_HIP_REQUIRE(Supported(desc), "kxc_hip_conv2d_winograd_node_bytes: shape is not a 3x3 stride-1 convolution with C %% 4 == 0");
-    *out_bytes = SmallConvBeatsWinograd(desc) ? 0 : SelectWino(desc)->kernel ? F32FilterBytes(desc) : wino_bx::WeightBytes(desc->o, desc->c);
+    // (room for the fp32 form beside the slice kernel's: what nodes of different shapes that share a buffer fall back to)
+    const size_t slice = SliceFilterBytes(desc, false);
+    *out_bytes = slice > 0 ? std::max(slice, F32FilterBytes(desc))
+                 : SmallConvBeatsWinograd(desc) ? 0 : SelectWino(desc)->kernel ? F32FilterBytes(desc) : wino_bx::WeightBytes(desc->o, desc->c);
     return KXC_HIP_OK;
 }
 

@@ -26,6 +26,8 @@
 // access; the input 5 to 13, the stores 6 to 14, of 5 to 7 per workgroup before the first matrix instruction and behind the last.
 #pragma once
 
+#include <algorithm>
+
 #include "bf16x3.h"
 #include "common.h"
 
@@ -59,6 +61,21 @@ inline size_t FilterBytes(int64_t O, int64_t C, int K, bool second) {
 }
 inline int64_t PackBlocks(int64_t O, int64_t C, int K) { return CeilDiv(O, 32) * 4 * CeilDiv(C, kStep * ChannelSteps(K)); }
 constexpr int PackFloats(int K) { return 8 * (kStep * ChannelSteps(K) * K * K + 1); }
+
+// How far `pix` neighbouring pixels (flattened over n, oh, ow) that start at a multiple of pix reach at most: `row` for every step to
+// the next output row and `image` for every step to the next image.  Within an image, where tiles start in a row repeats after
+// at most OW tiles; where the border of two images lies in a tile repeats after at most pix images.
+inline int32_t TileReach(int32_t N, int32_t OHW, int32_t OW, int32_t pix, int32_t row, int32_t image) {
+    const uint32_t p = static_cast<uint32_t>(pix), ow = static_cast<uint32_t>(OW), ohw = static_cast<uint32_t>(OHW), M = static_cast<uint32_t>(N) * ohw;
+    uint32_t best = 0;
+    auto tile = [&](uint32_t m0) {
+        const uint32_t last = std::min(p, M - m0) - 1;
+        best = std::max(best, (m0 % ow + last) / ow * static_cast<uint32_t>(row) + (m0 % ohw + last) / ohw * static_cast<uint32_t>(image));
+    };
+    for (uint32_t t = 0; t < ow && t * p < M; ++t) tile(t * p);
+    for (uint32_t n = 1; n < static_cast<uint32_t>(N) && n <= p; ++n) tile(n * ohw / p * p);
+    return static_cast<int32_t>(best);
+}
 
 struct Args {
     const float* x;

@@ -843,7 +843,7 @@ int32_t kxc_hip_plan_finalize(kxc_hip_plan* plan, size_t workspace_bytes) {
             if (p) { n.prepared_packed.reset(p, kxc_hip::FreePreparedPacked); continue; }
         }
         // (a small Winograd node, and one whose filter buffer holds no form, runs on its weights as they are, in one launch)
-        if (n.i32[0] == 1 && !kxc_hip::SmallConvBeatsWinograd(&n.conv)) {
+        if (n.i32[0] == 1 && (kxc_hip::SliceFilterBytes(&n.conv, false) > 0 || !kxc_hip::SmallConvBeatsWinograd(&n.conv))) {
             kxc_hip::PreparedWinograd* p = nullptr;
             if (int32_t rc = kxc_hip::PrepareWinograd(&n.conv, FilterRoom(n), &p)) return rc;
             if (p) n.prepared_wino.reset(p, kxc_hip::FreePreparedWinograd);
@@ -862,11 +862,12 @@ int32_t kxc_hip_plan_finalize(kxc_hip_plan* plan, size_t workspace_bytes) {
     for (Node& n : plan->nodes) {
         if (!n.prepared_wino || kxc_hip::PreparedWinogradForms(n.prepared_wino.get()) == kxc_hip::kWinoFormF32) continue;
         for (const Node& other : plan->nodes) {
-            if (!other.prepared_wino || !shares_filter(n, other) || kxc_hip::PreparedWinogradForms(other.prepared_wino.get()) != kxc_hip::kWinoFormF32) continue;
+            if (!other.prepared_wino || !shares_filter(n, other) ||
+                kxc_hip::PreparedWinogradForms(other.prepared_wino.get()) == kxc_hip::PreparedWinogradForms(n.prepared_wino.get())) continue;
             KXC_HIP_REQUIRE(FilterRoom(n) >= kxc_hip::WinogradF32FilterBytes(&n.conv),
                             "kxc_hip_plan_finalize: nodes that share a transformed filter need room for its fp32 form");
             kxc_hip::PreparedWinograd* p = nullptr;
-            if (int32_t rc = kxc_hip::PrepareWinograd(&n.conv, kxc_hip::WinogradF32FilterBytes(&n.conv), &p)) return rc;
+            if (int32_t rc = kxc_hip::PrepareWinograd(&n.conv, kxc_hip::WinogradF32FilterBytes(&n.conv), &p, false)) return rc;
             n.prepared_wino.reset(p, kxc_hip::FreePreparedWinograd);
             break;
         }
@@ -1007,7 +1008,7 @@ int32_t RunNode(kxc_hip_plan* plan, Node& n, void** args, void* s) {
                 // (launches resolved at finalize; s is never NULL here)
                 if (n.prepared_wino) {
                     // (the transformed weights in B(5) were written by TransformConstants at the start of the run)
-                    rc = kxc_hip::LaunchPreparedWinograd(n.prepared_wino.get(), static_cast<const float*>(B(0)),
+                    rc = kxc_hip::LaunchPreparedWinograd(n.prepared_wino.get(), static_cast<const float*>(B(0)), static_cast<const float*>(B(1)),
                                                          static_cast<const float*>(B(5)), static_cast<const float*>(B(2)),
                                                          static_cast<const float*>(B(3)), static_cast<float*>(B(4)),
                                                          kxc_hip::ResolveStream(s));
