@@ -182,6 +182,7 @@ __global__ void __launch_bounds__(256) wino_weight_batch_kernel(const WinoWeight
 template <int WK, int WT, int KS, bool FUSE = false>
 __global__ void __launch_bounds__(64 * WK * WT * KS) __attribute__((amdgpu_waves_per_eu(2)))
 wino_kernel(const WinoArgs a) {
+    request_args(a);
     static_assert(!FUSE || KS == 1, "the split over workgroups is never combined with the split over wave groups");
     constexpr int NW = WK * WT;                     // waves of one reduction group
     constexpr int NTH = 64 * NW;                    // threads of one reduction group

@@ -68,6 +68,7 @@ __device__ __forceinline__ void to_lds16(__amdgpu_buffer_rsrc_t rs, char* lds, u
 // values that a filter row touches by one 12-byte load, moved to the row's end where it would reach across it.
 template <int KH, int KW, int CPG, int XI, int RO, int KS, bool DS = false, bool ROWS = false>
 __global__ void __launch_bounds__(64 * KS) __attribute__((amdgpu_waves_per_eu(2))) conv_small_kernel(const Args a) {
+    request_args(a);
     constexpr bool STAGED = XI > 0;
     constexpr int KHW = KH * KW, E = CPG * KHW, WI = RO * E / 4, NB = DS ? 2 * RO : RO;
     static_assert(E % 4 == 0 && E <= 36 && (!DS || CPG == 4), "chunk layout");      // (36 loads of X in flight: vmcnt holds 63)

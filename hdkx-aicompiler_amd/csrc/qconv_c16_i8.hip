@@ -217,6 +217,7 @@ __device__ __forceinline__ void epilogue_c16(const intx16 (&acc)[RP][RO], const 
 // the window's tap at ds_off against the second packed weights, into a second set of accumulators.
 template <int KH, int KW, int CBC, int WP, int RO, int PPT, int RP = 1, int WD = 0, bool DS = false>
 __global__ void __launch_bounds__(64 * WP) __attribute__((amdgpu_waves_per_eu(2))) qconv_mfma_kernel(const QArgs a) {
+    request_args(a);
     constexpr int KHW = KH * KW;
     constexpr int NS = (KHW * CBC + 1) / 2;          // matrix k-steps per chunk
     constexpr int NS2 = DS ? (CBC + 1) / 2 : 0;      // ... of the second output
@@ -436,6 +437,7 @@ __global__ void __launch_bounds__(64 * WP) __attribute__((amdgpu_waves_per_eu(2)
 // Same tiles, accumulators, epilogue and second output as qconv_mfma_kernel; PPT = load slots per wave.
 template <int KH, int KW, int CBC, int WP, int RO, int PPT, int RP, int P, bool DS = false>
 __global__ void __launch_bounds__(64 * WP) __attribute__((amdgpu_waves_per_eu(2))) qconv_rows_kernel(const QArgs a) {
+    request_args(a);
     constexpr int KHW = KH * KW;
     constexpr int NS = (KHW * CBC + 1) / 2;          // matrix k-steps per chunk
     constexpr int NS2 = DS ? (CBC + 1) / 2 : 0;      // ... of the second output
@@ -764,6 +766,7 @@ __global__ void __launch_bounds__(64 * WP) __attribute__((amdgpu_waves_per_eu(2)
 // ------------------------------------------------------------------------------------------
 template <int RO, bool RELU>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) qconv_k7s2_c4_pool_kernel(const QArgs a) {
+    request_args(a);
     constexpr int KH = 7;
     constexpr int WP = 4;
     constexpr int WSEG = RO * KH;
@@ -1258,6 +1261,7 @@ __global__ void __launch_bounds__(kBlock) gap_c16_kernel(const int8_t* __restric
 // shortest: 512 -> 512 channels at 7 x 7, batch 5: 23.1 -> 4.8 us.  SelectDirect has the line between the two.
 template <int KH, int RO, int RP, int KS, bool DS = false>
 __global__ void __launch_bounds__(64 * KS) __attribute__((amdgpu_waves_per_eu(2))) qconv_direct_kernel(const QArgs a) {
+    request_args(a);
     constexpr int KHW = KH * KH, CBC = KH == 1 ? 4 : 2, NS = KHW * CBC / 2;
     constexpr int G = KH == 1 ? 3 : 1;               // chunks per loop trip
     constexpr int NB = RO * RP, NBA = DS ? 2 * NB : NB;
