@@ -7,6 +7,7 @@ missing, loading fails loudly.
 """
 import ctypes as C
 import os
+import struct
 
 PKG = os.path.dirname(os.path.abspath(__file__))
 # KXC_HIP_LIB points at an alternative build of the same library (kernel experiments).
@@ -102,17 +103,56 @@ def _p(t):
     return C.c_void_p(t.data_ptr()) if t is not None else C.c_void_p(0)
 
 
-def _stream():
-    import torch
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
-
-
 def _need(t, dtype, name):
-    import torch
     if t is None:
         return
     if not (t.is_cuda and t.is_contiguous() and t.dtype == dtype):
         raise KxcHipError("%s must be a contiguous %s tensor on the GPU" % (name, dtype))
+
+
+# The operators below cost their caller more time in Python than most of their kernels take, so their entry points have
+# prototypes of their own (numbers, addresses and bytes go in as they are, without an object for each) and their
+# descriptors are packed without a ctypes structure.  us per call in a row, before and now: nn_conv2d 64 channels at 56 x 56, batch
+# 1 10.7 and 7.1.
+_PTR, _I32, _I64, _F32 = C.c_void_p, C.c_int32, C.c_int64, C.c_float
+_SIGNATURES = {
+    "kxc_hip_conv2d_nchw_f32": [_PTR] * 7, "kxc_hip_conv2d_nchw_f32_noalloc": [_PTR] * 7, "kxc_hip_qconv2d_c16_i8": [_PTR] * 8,
+    "kxc_hip_gemm_f32": [_PTR] * 4 + [_I64] * 3 + [_F32] * 2 + [_I32, _I64, _PTR], "kxc_hip_pool2d_f32": [_PTR] * 4,
+    "kxc_hip_broadcast_binary_f32": [_I32, _PTR, _PTR, _I32, _PTR, _PTR, _I32, _PTR, _I32, _PTR],
+    "kxc_hip_global_avg_pool2d_f32": [_PTR] * 2 + [_I64] * 4 + [_PTR],
+}
+_entries = {}
+_CONV, _QCONV = struct.Struct("=13iI"), struct.Struct("=11iIf")
+
+
+def _entry(name):
+    f = _entries.get(name)
+    if f is None:
+        f = lib()[name]          # (a function object of its own: other users of the library's are not affected)
+        f.argtypes = _SIGNATURES[name]
+        _entries[name] = f
+    return f
+
+
+def _bytes(packer, structure, *fields):
+    """The descriptor as bytes; what does not fit goes through the ctypes structure, which wraps or refuses it."""
+    try:
+        return packer.pack(*fields)
+    except struct.error:
+        return bytes(structure(*fields))
+
+
+def _a(t):
+    return t.data_ptr() if t is not None else None
+
+
+def _stream():
+    """The current stream of the current device."""
+    import torch
+    try:
+        return C.c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
+    except AttributeError:
+        return C.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
 def device_attributes(device_id=0):
@@ -155,12 +195,16 @@ def conv2d(x, w, bias=None, residual=None, stride=1, pad=0, dil=1, relu=False, f
         raise KxcHipError("nn_conv2d input channel mismatch")
     flags = (CONV_BIAS if bias is not None else 0) | (CONV_RESIDUAL if residual is not None else 0) | \
             (CONV_RELU if relu else 0) | (CONV_FORCE_DIRECT if force_direct else 0) | (CONV_HPOOL if hpool else 0)
-    d = conv_desc(tuple(x.shape), tuple(w.shape), stride, pad, dil, flags)
+    n, c, h, wd = x.shape
+    o, _, kh, kw = w.shape
+    d = _bytes(_CONV, ConvDesc, n, c, h, wd, o, kh, kw, stride, stride, pad, pad, dil, dil, flags)
+    ow = (wd + 2 * pad - ((kw - 1) * dil + 1)) // stride + 1
+    shape = (n, o, (h + 2 * pad - ((kh - 1) * dil + 1)) // stride + 1, ow // 2 if hpool else ow)
     if out is not None:
-        _check_out(out, conv_out_shape(d))
-    y = out if out is not None else torch.empty(conv_out_shape(d), dtype=torch.float32, device=x.device)
-    entry = lib().kxc_hip_conv2d_nchw_f32_noalloc if no_alloc else lib().kxc_hip_conv2d_nchw_f32
-    _check(entry(C.byref(d), _p(x), _p(w), _p(bias), _p(residual), _p(y), _stream()))
+        _check_out(out, shape)
+    y = out if out is not None else torch.empty(shape, dtype=torch.float32, device=x.device)
+    entry = _entry("kxc_hip_conv2d_nchw_f32_noalloc" if no_alloc else "kxc_hip_conv2d_nchw_f32")
+    _check(entry(d, x.data_ptr(), w.data_ptr(), _a(bias), _a(residual), y.data_ptr(), _stream()))
     return y
 
 
@@ -276,14 +320,13 @@ def relu(x):
 def binary(op, a, b, relu=False, out=None):
     import torch
     _need(a, torch.float32, "a"); _need(b, torch.float32, "b")
-    shape = torch.broadcast_shapes(a.shape, b.shape)
+    shape = a.shape if a.shape == b.shape else torch.broadcast_shapes(a.shape, b.shape)
     y = out if out is not None else torch.empty(shape, dtype=torch.float32, device=a.device)
     _need(y, torch.float32, "out")
-    if tuple(y.shape) != tuple(shape):
+    if y is out and tuple(y.shape) != tuple(shape):
         raise ValueError("binary: out has shape %s, expected %s" % (tuple(y.shape), tuple(shape)))
-    sa = (C.c_int64 * max(1, a.dim()))(*a.shape); sb = (C.c_int64 * max(1, b.dim()))(*b.shape)
-    _check(lib().kxc_hip_broadcast_binary_f32(C.c_int32(op), _p(a), sa, C.c_int32(a.dim()), _p(b), sb,
-                                              C.c_int32(b.dim()), _p(y), C.c_int32(int(relu)), _stream()))
+    sa, sb = struct.pack("=%dq" % a.dim(), *a.shape), struct.pack("=%dq" % b.dim(), *b.shape)
+    _check(_entry("kxc_hip_broadcast_binary_f32")(op, a.data_ptr(), sa, a.dim(), b.data_ptr(), sb, b.dim(), y.data_ptr(), int(relu), _stream()))
     return y
 
 
@@ -322,7 +365,7 @@ def pool2d(x, k, s, pad, ceil_mode=False, avg=False, out=None):
     if out is not None:
         _check_out(out, pool_out_shape(d))
     y = out if out is not None else torch.empty(pool_out_shape(d), dtype=torch.float32, device=x.device)
-    _check(lib().kxc_hip_pool2d_f32(C.byref(d), _p(x), _p(y), _stream()))
+    _check(_entry("kxc_hip_pool2d_f32")(C.byref(d), x.data_ptr(), y.data_ptr(), _stream()))
     return y
 
 
@@ -334,8 +377,7 @@ def global_avg_pool2d(x, out=None):
     _need(y, torch.float32, "out")
     if y.numel() != n * c:
         raise ValueError("global_avg_pool2d: out has %d elements, expected %d" % (y.numel(), n * c))
-    _check(lib().kxc_hip_global_avg_pool2d_f32(_p(x), _p(y), C.c_int64(n), C.c_int64(c), C.c_int64(h), C.c_int64(w),
-                                               _stream()))
+    _check(_entry("kxc_hip_global_avg_pool2d_f32")(x.data_ptr(), y.data_ptr(), n, c, h, w, _stream()))
     return y
 
 
@@ -348,9 +390,8 @@ def gemm(a, b, c=None, alpha=1.0, beta=1.0, transB=1, out=None):
     _need(y, torch.float32, "out")
     if y.numel() != m * n:
         raise ValueError("gemm: out has %d elements, expected %d" % (y.numel(), m * n))
-    _check(lib().kxc_hip_gemm_f32(_p(a), _p(b), _p(c), _p(y), C.c_int64(m), C.c_int64(n), C.c_int64(k),
-                                  C.c_float(alpha), C.c_float(beta), C.c_int32(transB),
-                                  C.c_int64(c.numel() if c is not None else 0), _stream()))
+    _check(_entry("kxc_hip_gemm_f32")(a.data_ptr(), b.data_ptr(), _a(c), y.data_ptr(), m, n, k, alpha, beta, transB,
+                                      c.numel() if c is not None else 0, _stream()))
     return y
 
 
@@ -488,11 +529,10 @@ def qconv2d_c16(x, c, w_packed, w_shape, bias, mult, residual=None, res_mult=0.0
     o, _, kh, kw = w_shape
     flags = (CONV_BIAS if bias is not None else 0) | (CONV_RESIDUAL if residual is not None else 0) | \
             (CONV_RELU if relu else 0)
-    d = qconv_desc(n, c, h, wd, o, kh, kw, stride, pad, flags, res_mult)
+    d = _bytes(_QCONV, QConvDesc, n, c, h, wd, o, kh, kw, stride, stride, pad, pad, flags, res_mult)
     oh = (h + 2 * pad - kh) // stride + 1; ow = (wd + 2 * pad - kw) // stride + 1
     y = torch.empty(c16_shape(n, o, oh, ow), dtype=torch.int8, device=x.device)
-    _check(lib().kxc_hip_qconv2d_c16_i8(C.byref(d), _p(x), _p(w_packed), _p(bias), _p(mult), _p(residual), _p(y),
-                                        _stream()))
+    _check(_entry("kxc_hip_qconv2d_c16_i8")(d, x.data_ptr(), _a(w_packed), _a(bias), _a(mult), _a(residual), y.data_ptr(), _stream()))
     return y
 
 
