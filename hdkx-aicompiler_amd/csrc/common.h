@@ -178,13 +178,14 @@ constexpr int64_t kSmallRowLoadsWork = 2300000;      // (16 x 16 tiles) * channe
 bool SmallConvTakes(const kxc_hip_conv2d_desc* desc, bool second_output, bool in_plan);      // ... or a small-launch kernel at all
 int32_t HpoolTilePixels(const kxc_hip_conv2d_desc* desc);      // pixels of a tile of the fp32 kernel that takes a pooled launch (0: none does)
 bool SmallConvBeatsWinograd(const kxc_hip_conv2d_desc* desc);      // a plan's Winograd node is better launched as PreparedConv
-bool SmallConvStagesRows(const kxc_hip_conv2d_desc* desc);         // ... by the kernel that stages whole rows
+bool SmallConvStagesRows(const kxc_hip_conv2d_desc* desc, bool second_output);      // ... by the kernel that stages whole rows
 void FreePreparedConv(PreparedConv* p);
 struct PreparedWinograd;
 // A node whose filter buffer has u_bytes, holding the one form that the launch reads.  *out = nullptr: no form fits.
 int32_t PrepareWinograd(const kxc_hip_conv2d_desc* desc, size_t u_bytes, PreparedWinograd** out, bool may_slice = true);
 const char* PreparedWinogradName(const PreparedWinograd* p);
 size_t WinogradF32FilterBytes(const kxc_hip_conv2d_desc* desc);
+double PairNodeUs(const kxc_hip_conv2d_desc* desc);          // us of a plan's two-output node without the kernel of conv_slice.h (0: never take that)
 double WinogradNodeUs(const kxc_hip_conv2d_desc* desc);      // us of a plan's Winograd node without the kernel of conv_slice.h (0: never take that)
 int32_t LaunchPreparedWinograd(const PreparedWinograd* p, const float* x, const float* w, const float* u, const float* bias,
                                const float* residual, float* y, hipStream_t stream);

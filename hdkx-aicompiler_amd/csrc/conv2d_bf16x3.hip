@@ -363,6 +363,21 @@ int32_t RunPackedOperator(const kxc_hip_conv2d_desc* desc, const float* x, const
     return LaunchConv(L, x, w, u, bias, residual, y, nullptr, nullptr, nullptr, stream, reinterpret_cast<float*>(u + filter));
 }
 
+// Fitted to 1320 shapes, within a tenth (packed kernel), 13 % (small-launch kernels) and 17 % (rms).
+double PairNodeUs(const kxc_hip_conv2d_desc* d) {
+    PackedLaunch L;
+    const int64_t lanes = SelectLanes();
+    if (d->c < 64 || d->kh != 3 || d->kw != 3 || d->stride_h != 2 || d->stride_w != 2) return 0;
+    if (Preferred(d, true, &L)) {
+        const double out_bytes = 8.0 * L.a.M * d->o;
+        return 9.7 + 0.74 * PackedUs(2, 4, 0.28, 2, lanes * L.a.num_units * L.a.gsplit, 10LL * L.a.cps, L.a.gsplit, out_bytes);
+    }
+    const int64_t pixels = d->n * ((static_cast<int64_t>(d->h) + 2 * d->pad_h - 3) / 2 + 1) * ((static_cast<int64_t>(d->w) + 2 * d->pad_w - 3) / 2 + 1);
+    if (pixels <= 0 || pixels >= (1LL << 31)) return 0;
+    if (!SmallConvTakes(d, true, true)) return 10.5 + 12.7 * static_cast<double>(lanes) * BlockGflop(d, pixels, 10, 32);
+    return SmallConvStagesRows(d, true) ? 0 : 4.9 + 13.4 * static_cast<double>(lanes) * BlockGflop(d, pixels, 10, 16);
+}
+
 struct PreparedPacked {
     PackedLaunch launch;
     PreparedSlicePtr slice;      // the launch, where it is set

@@ -1582,9 +1582,9 @@ bool SmallConvBeatsWinograd(const kxc_hip_conv2d_desc* d) {
            CeilDiv(a.M, 16) * CeilDiv(a.O, 16) * SelectLanes() * a.C * 9 <= (SmallRowLoads(a) && a.O % 16 == 0 ? 1400000 : 1100000);
 }
 
-bool SmallConvStagesRows(const kxc_hip_conv2d_desc* d) {
+bool SmallConvStagesRows(const kxc_hip_conv2d_desc* d, bool second) {
     ConvArgs a;
-    return FillArgs(d, &a, "plan") == KXC_HIP_OK && SelectSmall(d, a, false, true) == kSmall;
+    return FillArgs(d, &a, "plan") == KXC_HIP_OK && SelectSmall(d, a, second, true) == kSmall;
 }
 
 bool SmallConvTakes(const kxc_hip_conv2d_desc* d, bool second, bool in_plan) {

@@ -1,4 +1,4 @@
-// conv2d_slice.hip -- which of a launch plan's 3x3 convolutions take the kernel of conv_slice.h, and their launch.
+// conv2d_slice.hip -- which of a launch plan's 3x3 convolutions (stride 1, or 2 with the second output) take the kernel of conv_slice.h, and their launch.
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
@@ -27,7 +27,8 @@ struct SliceVariant {
 };
 #define KXC_SLICE(RO, KS) {"mfma_k3x3_slice_o" #RO "_k" #KS, 1, RO, KS, false, conv_sl::conv_slice_kernel<1, RO, KS, false>}
 // name = slice_o<blocks of 32 output channels>_k<waves along the input channels>
-const SliceVariant kSlices[] = {KXC_SLICE(1, 4), KXC_SLICE(1, 8), KXC_SLICE(2, 4), KXC_SLICE(2, 8)};
+#define KXC_SLICE_DS(KS) {"mfma_k3x3s2_slice_o1_k" #KS "_ds", 2, 1, KS, true, conv_sl::conv_slice_kernel<2, 1, KS, true>}
+const SliceVariant kSlices[] = {KXC_SLICE(1, 4), KXC_SLICE(1, 8), KXC_SLICE(2, 4), KXC_SLICE(2, 8), KXC_SLICE_DS(4), KXC_SLICE_DS(8)};
 
 bool Resolve(const kxc_hip_conv2d_desc* d, bool second, const SliceVariant& v, PreparedSlice* L) {
     using namespace conv_sl;
@@ -95,9 +96,14 @@ bool Resolve(const kxc_hip_conv2d_desc* d, bool second, const SliceVariant& v, P
 
 // us of a launch in a plan, fitted to 1700 shapes of 16 to 512 channels and 0.01 to 4 GFLOP (rms 7 % with four waves, 12 with eight; the
 // variant it picks is on average 1.4 % slower than the fastest): a workgroup's start and its steps of 16 channels, per round of
-// workgroups.  A compute unit holds two of four waves, which alone take 0.6 of what they take together, or one of eight.
+// workgroups.  A compute unit holds two of four waves, which alone take 0.6 of what they take together, or one of eight.  Two outputs (1300 shapes, 5
+// and 9 %): one workgroup either way.
 double SliceUs(const SliceVariant& v, int64_t tiles, int64_t csteps) {
     const double steps = static_cast<double>(CeilDiv(csteps, v.ks));
+    if (v.second) {
+        const double w = static_cast<double>(tiles) / 256, whole = static_cast<double>(CeilDiv(tiles, 256));
+        return v.ks == 4 ? 5.0 + (0.76 + 2.95 * steps) * (tiles <= 256 ? 1.0 : w + 0.36 * (whole - w)) : 2.1 + (2.15 + 4.56 * steps) * whole;
+    }
     if (v.ks == 8) return (v.ro == 1 ? 2.1 : 2.4) + (v.ro == 1 ? 1.15 + 2.93 * steps : 0.55 + 4.65 * steps) * static_cast<double>(CeilDiv(tiles, 256));
     const double w = static_cast<double>(tiles) / 512, whole = static_cast<double>(CeilDiv(tiles, 512));
     const double rounds = tiles <= 256 ? 0.6 : tiles <= 512 ? 1.0 : w + 0.65 * (whole - w);
@@ -106,24 +112,28 @@ double SliceUs(const SliceVariant& v, int64_t tiles, int64_t csteps) {
 
 // Whether a plan's node should take it: where its estimate is a twentieth below that of the kernel that the node takes otherwise
 // (WinogradNodeUs).  Of 1700 shapes 1090 take it, 1.45 times as fast on average; twelve of them are slower by more than 3 %.
+// Nodes with a second output (PairNodeUs) leave 0.08 in hand: 256 of 1320 shapes, 1.19 times as fast, three slower by more than 3 %.
 // KXC_HIP_CONV_SLICE=0: nowhere, =<name>: that variant wherever it covers the node.  Switches that keep convolutions on the fp32
 // instructions or name other kernels keep those.
 bool Preferred(const kxc_hip_conv2d_desc* d, bool second, PreparedSlice* L) {
-    if (!d || second) return false;
+    if (!d) return false;
     if (const char* e = std::getenv("KXC_HIP_CONV_SLICE"); e && *e) {
         for (const SliceVariant& v : kSlices)
             if (std::strcmp(e, v.name) == 0) return Resolve(d, second, v, L);
         return false;
     }
     for (const char* name : {"KXC_HIP_WINOGRAD_BF16X3", "KXC_HIP_CONV_BF16X3"})
-        if (const char* e = std::getenv(name); e && e[0] == '0') return false;
+        if (const char* e = std::getenv(name); e && (e[0] == '0' || (second && e[0] == '1'))) return false;
     for (const char* name : {"KXC_HIP_WINOGRAD_VARIANT", "KXC_HIP_WINOGRAD_GSPLIT", "KXC_HIP_CONV_VARIANT", "KXC_HIP_CONV_GSPLIT"})
         if (const char* e = std::getenv(name); e && *e) return false;
-    double best_us = 0.95 * WinogradNodeUs(d);
-    const int64_t pixels = static_cast<int64_t>(d->n) * (d->h + 2 * d->pad_h - 2) * (d->w + 2 * d->pad_w - 2), csteps = CeilDiv(d->c, conv_sl::kStep);
+    double best_us = second ? 0.92 * PairNodeUs(d) : 0.95 * WinogradNodeUs(d);
+    if (best_us <= 0) return false;
+    const int stride = second ? 2 : 1;
+    const int64_t oh = (static_cast<int64_t>(d->h) + 2 * d->pad_h - 3) / stride + 1, ow = (static_cast<int64_t>(d->w) + 2 * d->pad_w - 3) / stride + 1;
+    const int64_t pixels = d->n * oh * ow, csteps = CeilDiv(d->c, conv_sl::kStep);
     const SliceVariant* best = nullptr;
     for (const SliceVariant& v : kSlices) {
-        if (csteps < v.ks) continue;      // (a wave without a step)
+        if (csteps < v.ks || v.second != second) continue;      // (a wave without a step)
         const double us = SliceUs(v, CeilDiv(pixels, conv_sl::kPix) * CeilDiv(d->o, 32 * v.ro) * SelectLanes(), csteps);
         if (us < best_us) { best_us = us; best = &v; }
     }

@@ -976,7 +976,7 @@ double WinogradNodeUs(const kxc_hip_conv2d_desc* d) {
     if (!Supported(d)) return 0;
     const int64_t lanes = SelectLanes(), oh = static_cast<int64_t>(d->h) + 2 * d->pad_h - 2, ow = static_cast<int64_t>(d->w) + 2 * d->pad_w - 2;
     if (SmallConvBeatsWinograd(d)) {
-        if (SmallConvStagesRows(d)) return 0;      // (the faster one on all of 289 shapes)
+        if (SmallConvStagesRows(d, false)) return 0;      // (the faster one on all of 289 shapes)
         const double gflop = 18e-9 * static_cast<double>(CeilDiv(d->n * oh * ow, 16) * 16) * static_cast<double>(CeilDiv(d->o, 16) * 16) * d->c;
         return 4.2 + 13.8 * static_cast<double>(lanes) * gflop;
     }

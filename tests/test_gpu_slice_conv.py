@@ -92,7 +92,7 @@ def test_slice_kernel_forms_sums_that_are_not_finite_again(pkg, monkeypatch, var
     got = node.run()
     assert (np.isnan(got) == np.isnan(want)).all() and (np.isinf(got) == np.isinf(want)).all()
     ok = np.isfinite(want)
-    assert (np.abs(got - want)[ok] <= (9 * 128 + 16) * 2.0 ** -24 * np.maximum(np.abs(want[ok]), 8)).all()
+    assert (np.abs(got[ok] - want[ok]) <= (9 * 128 + 16) * 2.0 ** -24 * np.maximum(np.abs(want[ok]), 8)).all()
     plan = pkg.Plan(3)
     A, none = pkg.Buf.arg, pkg.Buf.none()
     plan.add_conv2d_winograd(pkg.ConvDesc(2, 128, 9, 11, 48, 3, 3, 1, 1, 1, 1, 1, 1, pkg.CONV_RESIDUAL), A(0), A(1), none, A(2), A(2), pkg.Buf.ws(0), node.room)
@@ -156,3 +156,59 @@ def test_node_without_room_for_the_filter_runs_on_its_weights(pkg, monkeypatch):
     assert "_small" in node.plan.node_symbol(0)
     node.check(node.run())
     node.plan.close()
+
+
+PAIRS = ["mfma_k3x3s2_slice_o1_k%d_ds" % k for k in (4, 8)]
+
+
+def _pair(pkg, xs, o, seed):
+    """A two-output node (3x3 with stride 2, 1x1 with stride 2), its operands and what it should give."""
+    rng = np.random.default_rng(seed)
+    n, c, h, w = xs
+    f32 = lambda s, k=1.0: (rng.standard_normal(s) * k).astype(np.float32)
+    x, w1, w2, b1, b2 = f32(xs), f32((o, c, 3, 3), (2 / (9 * c)) ** 0.5), f32((o, c, 1, 1), (2 / c) ** 0.5), f32((o,)), f32((o,))
+    t = lambda a: torch.from_numpy(a).double()
+    want = [np.maximum(torch.nn.functional.conv2d(t(x), t(w1), t(b1), 2, 1).numpy(), 0), torch.nn.functional.conv2d(t(x), t(w2), t(b2), 2, 0).numpy()]
+    desc = pkg.ConvDesc(n, c, h, w, o, 3, 3, 2, 2, 1, 1, 1, 1, pkg.CONV_BIAS | pkg.CONV_RELU)
+    size = pkg.conv2d_node_filter_bytes(desc, True)
+    args = [dev(a) for a in (x, w1, b1, w2, b2)] + [torch.empty(y.shape, device="cuda") for y in want]
+    A, none = pkg.Buf.arg, pkg.Buf.none()
+    plan = pkg.Plan(7)
+    plan.add_conv2d_packed(desc, A(0), A(1), A(2), none, A(5), A(3), A(4), A(6), pkg.Buf.ws(0), size or 256)
+    plan.finalize(size or 256)
+
+    def run(p=plan):
+        for y in args[5:]:
+            y.fill_(float("nan"))
+        p.run(args); torch.cuda.synchronize()
+        got = [host(y) for y in args[5:]]
+        for y, ref, terms in zip(got, want, (9 * c + 16, c + 16)):
+            assert np.isfinite(y).all() and np.linalg.norm(y - ref) <= terms ** 0.5 * 2.0 ** -23 * np.linalg.norm(ref)
+        return got
+    return plan, size, run
+
+
+@pytest.mark.parametrize("variant", PAIRS)
+@pytest.mark.parametrize("xs, o", [
+    ((1, 128, 3, 40), 32), ((3, 128, 13, 13), 40), ((5, 132, 7, 6), 33), ((2, 128, 49, 49), 64), ((1, 144, 9, 203), 64), ((4, 256, 5, 5), 96), ((2, 256, 14, 14), 512)])
+def test_slice_kernel_with_a_second_output(pkg, monkeypatch, variant, xs, o):
+    monkeypatch.setenv("KXC_HIP_CONV_SLICE", variant)
+    plan, size, run = _pair(pkg, xs, o, sum(xs) + o)
+    assert size > 0 and variant in plan.node_symbol(0)
+    first = run()
+    again = pkg.Plan.deserialize(plan.serialize(), 0)
+    for p in (plan, again):
+        for a, b in zip(run(p), first):
+            assert_bit_exact(a, b, "again")
+    again.close()
+    plan.close()
+
+
+@pytest.mark.parametrize("xs, o, takes", [((6, 128, 25, 25), 256, True), ((1, 128, 28, 28), 256, False), ((64, 64, 56, 56), 128, False)])
+def test_which_two_output_nodes_take_the_slice_kernel(pkg, monkeypatch, xs, o, takes):
+    for name in ("KXC_HIP_CONV_SLICE", "KXC_HIP_CONV_BF16X3", "KXC_HIP_WINOGRAD_BF16X3"):
+        monkeypatch.delenv(name, raising=False)
+    plan, size, run = _pair(pkg, xs, o, o)
+    assert ("slice" in plan.node_symbol(0)) == takes, plan.node_symbol(0)
+    run()
+    plan.close()
