@@ -662,7 +662,16 @@ __global__ void __launch_bounds__(64 * WP) __attribute__((amdgpu_waves_per_eu(2)
 // kw = 4h-1 .. 4h+2 (the window is widened by one tap on the left, with zero weight, so that it starts on
 // an 8-byte boundary).  7 k-steps per 32x32 block instead of the 25 that padding 3 channels to a 16-channel
 // block costs, and a quarter of the input bytes.  LDS rows hold [4 zero pixels][W pixels][4 zero pixels]
-// as 16-byte positions; a tile's rows are loaded once (single chunk).  Output is c16.
+// as 16-byte positions; a tile's rows are loaded once (single chunk).  Output is c16.  Rows that are no multiple of four pixels are
+// loaded in the same pieces, on 4-byte boundaries; the last piece of a row ends in the next row's first pixels, which clear_row_ends
+// replaces by zeros.  (Such widths used to take the general NCHW kernel, one thread per output: 3 -> 64 channels at 193 x 193, batch 16
+// 805 us and a pool of 19; 10.1 here with the pool.)
+__device__ __forceinline__ void clear_row_ends(char* lds, int rows, int row_bytes, int width, int tid, int threads) {
+    if ((width & 3) == 0) return;
+    for (int q = tid; q < rows; q += threads)
+        for (int e = width & 3; e < 4; ++e) *reinterpret_cast<int*>(lds + q * row_bytes + 16 + ((width >> 2) * 4 + e) * 4) = 0;
+    __syncthreads();
+}
 template <int WP, int RO, int PPT>
 __global__ void __launch_bounds__(64 * WP) __attribute__((amdgpu_waves_per_eu(2))) qconv_k7s2_c4_kernel(const QArgs a) {
     constexpr int KH = 7;
@@ -675,7 +684,7 @@ __global__ void __launch_bounds__(64 * WP) __attribute__((amdgpu_waves_per_eu(2)
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int half = lane >> 5;
     const int r = lane & 31;
-    const int W4 = (a.W >> 2) + 2;                  // 16-byte positions per LDS row
+    const int W4 = ((a.W + 3) >> 2) + 2;            // 16-byte positions per LDS row
     const int xs_bytes = a.chs * 16;
 
     const int tile = (blockIdx.x & 7) * a.tiles_per_xcd + (blockIdx.x >> 3);
@@ -703,7 +712,7 @@ __global__ void __launch_bounds__(64 * WP) __attribute__((amdgpu_waves_per_eu(2)
             const int q = fast_div(pos, a.div_wp), c4 = pos - q * W4;
             const int Q = qmin + q;
             const int n = fast_div(Q, a.div_hp), ih = Q - n * a.Hp - 3;
-            const bool ok = pos < P && n < a.N && ih >= 0 && ih < a.H && c4 >= 1 && c4 <= (a.W >> 2);
+            const bool ok = pos < P && n < a.N && ih >= 0 && ih < a.H && c4 >= 1 && c4 <= ((a.W + 3) >> 2);
             const uint32_t off = ok ? static_cast<uint32_t>((n * a.H + ih) * a.W + (c4 - 1) * 4) * 4u : kOob;
             load16_to_lds(xr, (lds_ptr_t)(lds + seg * 1024), off, 0);
         }
@@ -731,6 +740,7 @@ __global__ void __launch_bounds__(64 * WP) __attribute__((amdgpu_waves_per_eu(2)
     init_acc_with_bias<RO>(acc[0], a.bias, (a.flags & KXC_HIP_CONV_BIAS) != 0, a.O, ob0, half);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
+    clear_row_ends(lds, qlast - qmin + 1, W4 * 16, a.W, tid, 64 * WP);
     const char* ws = lds + xs_bytes + lane * 16;
 #pragma unroll
     for (int kh = 0; kh < KH; ++kh) {
@@ -776,7 +786,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) q
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int half = lane >> 5;
     const int r = lane & 31;
-    const int W4 = (a.W >> 2) + 2;                  // 16-byte positions per LDS row
+    const int W4 = ((a.W + 3) >> 2) + 2;            // 16-byte positions per LDS row
     const int row_bytes = W4 * 16;
     const int xs_bytes = a.chs * 16;
 
@@ -796,7 +806,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) q
         const int pos = seg * 64 + lane;
         const int q = fast_div(pos, a.div_wp), c4 = pos - q * W4;
         const int ih = 2 * c_lo + q - 3;
-        const bool ok = pos < P && ih >= 0 && ih < a.H && c4 >= 1 && c4 <= (a.W >> 2);
+        const bool ok = pos < P && ih >= 0 && ih < a.H && c4 >= 1 && c4 <= ((a.W + 3) >> 2);
         const uint32_t off = ok ? static_cast<uint32_t>((n * a.H + ih) * a.W + (c4 - 1) * 4) * 4u : kOob;
         load16_to_lds(xr, (lds_ptr_t)(lds + seg * 1024), off, 0);
     }
@@ -828,6 +838,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) q
         }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
+    clear_row_ends(lds, nrows, row_bytes, a.W, tid, 64 * WP);
     const char* ws = lds + xs_bytes + lane * 16;
 
     // One convolution row: for every accumulator register the requantised value before rounding, already the maximum
@@ -933,16 +944,20 @@ __global__ void __launch_bounds__(kBlock) pack_weights_k7_c4_kernel(const int8_t
 
 // fp32 NCHW -> int8 c4 ([N][H][W][4]); one thread per pixel.
 __global__ void __launch_bounds__(kBlock) quantize_to_c4_kernel(const float* __restrict__ x, int8_t* __restrict__ y,
-                                                                int32_t C, int64_t HW, int64_t total, float scale) {
+                                                                int32_t C, int64_t HW, FastDiv div_hw, int64_t total, float scale) {
     const int64_t s = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
     if (s >= total) return;
-    const int64_t p = s % HW, n = s / HW;
+    // (64-bit division only where 32 bits do not number the pixels: 150 instructions ahead of the first load)
+    const int64_t n = total < (1LL << 31) ? fast_div(static_cast<int32_t>(s), div_hw) : s / HW, p = s - n * HW;
+    float e[4];      // every channel's load ahead of the first division
+#pragma unroll
+    for (int c = 0; c < 4; ++c) e[c] = x[(n * C + min(c, C - 1)) * HW + p];
     uint32_t word = 0;
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
         int32_t q = 0;
         if (c < C) {
-            const float v = __fdiv_rn(x[(n * C + c) * HW + p], scale);
+            const float v = __fdiv_rn(e[c], scale);
             float rr = rintf(v);
             rr = (v == v) ? rr : 0.0f;
             rr = fminf(fmaxf(rr, -127.0f), 127.0f);
@@ -956,17 +971,19 @@ __global__ void __launch_bounds__(kBlock) quantize_to_c4_kernel(const float* __r
 // The same for four consecutive pixels per thread (plane size a multiple of 4, 16-byte aligned tensors): one 16-byte
 // load per channel, one 16-byte store, a quarter of the index arithmetic.  Same arithmetic per element.
 __global__ void __launch_bounds__(kBlock) quantize_to_c4_x4_kernel(const float* __restrict__ x, int8_t* __restrict__ y,
-                                                                   int32_t C, int32_t HW4, int64_t total4, float scale) {
-    const int64_t s = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+                                                                   int32_t C, int32_t HW4, FastDiv div_hw4, int32_t total4, float scale) {
+    const int32_t s = static_cast<int32_t>(blockIdx.x) * kBlock + static_cast<int32_t>(threadIdx.x);
     if (s >= total4) return;
-    const int64_t n = s / HW4;
-    const int32_t p4 = static_cast<int32_t>(s - n * HW4);
+    const int32_t image = fast_div(s, div_hw4), p4 = s - image * HW4;      // (64-bit division: 150 instructions ahead of the first load)
+    const int64_t n = image;
+    float4 all[4];      // every channel's load ahead of the first division
+#pragma unroll
+    for (int c = 0; c < 4; ++c) all[c] = reinterpret_cast<const float4*>(x)[(n * C + min(c, C - 1)) * HW4 + p4];
     uint32_t word[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
         if (c < C) {
-            const float4 v4 = reinterpret_cast<const float4*>(x)[(n * C + c) * HW4 + p4];
-            const float e[4] = {v4.x, v4.y, v4.z, v4.w};
+            const float e[4] = {all[c].x, all[c].y, all[c].z, all[c].w};
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const float v = __fdiv_rn(e[i], scale);
@@ -1951,7 +1968,7 @@ int32_t PrepareK7(const kxc_hip_qconv2d_desc* d, QLaunch* L, const K7Variant** o
     KXC_HIP_REQUIRE(d->kh == 7 && d->kw == 7 && d->stride_h == 2 && d->stride_w == 2 && d->pad_h == 3 && d->pad_w == 3,
                     "%s: only a 7x7 filter with stride 2 and padding 3 runs on the c4 layout", who);
     KXC_HIP_REQUIRE(d->c >= 1 && d->c <= 4, "%s: at most 4 input channels (got %d)", who, d->c);
-    KXC_HIP_REQUIRE(d->n >= 0 && d->h >= 1 && d->w >= 4 && d->w % 4 == 0, "%s: width must be a positive multiple of 4", who);
+    KXC_HIP_REQUIRE(d->n >= 0 && d->h >= 1 && d->w >= 4, "%s: rows of at least four pixels", who);
     KXC_HIP_REQUIRE(d->o > 0 && d->o % 32 == 0, "%s: output channels must be a multiple of 32 (got %d)", who, d->o);
     KXC_HIP_REQUIRE(!(d->flags & KXC_HIP_CONV_RESIDUAL), "%s: no residual operand on the first layer", who);
     QArgs& a = L->args;
@@ -1965,7 +1982,7 @@ int32_t PrepareK7(const kxc_hip_qconv2d_desc* d, QLaunch* L, const K7Variant** o
     const int64_t M = static_cast<int64_t>(a.N) * a.OHW;
     const int64_t xb = static_cast<int64_t>(a.N) * a.H * a.W * 4;
     KXC_HIP_REQUIRE(M < (1LL << 30) && xb < (1LL << 31) && M * a.O < (1LL << 31) &&
-                    static_cast<int64_t>(a.N + 1) * a.Hp * (a.W / 4 + 2) < (1LL << 26),
+                    static_cast<int64_t>(a.N + 1) * a.Hp * ((static_cast<int64_t>(a.W) + 3) / 4 + 2) < (1LL << 26),
                     "%s: tensor too large for 32-bit addressing", who);
     a.M = static_cast<int32_t>(M);
     a.x_bytes = static_cast<uint32_t>(xb);
@@ -1974,7 +1991,7 @@ int32_t PrepareK7(const kxc_hip_qconv2d_desc* d, QLaunch* L, const K7Variant** o
     a.w_bytes = static_cast<uint32_t>((a.O / 32) * 7 * 1024);
     *out = nullptr;
     if (M == 0) return KXC_HIP_OK;
-    const int W4 = a.W / 4 + 2;
+    const int W4 = (a.W + 3) / 4 + 2;
     a.div_wp = MakeFastDiv(W4); a.div_hp = MakeFastDiv(a.Hp); a.div_ohw = MakeFastDiv(a.OHW);
     a.div_ow = MakeFastDiv(a.OW);
     if (!select_variant) return KXC_HIP_OK;
@@ -2025,7 +2042,7 @@ int32_t PrepareK7Pool(const kxc_hip_qconv2d_desc* d, K7PoolLaunch* L, const char
     if (a.M == 0) return KXC_HIP_OK;
     const int ro = (a.O / 32) % 2 == 0 ? 2 : 1;
     a.o_tiles = (a.O / 32) / ro;
-    const int W4 = a.W / 4 + 2;
+    const int W4 = (a.W + 3) / 4 + 2;
     // measured on the 224 x 224 first layer (us, rows 2 / 3 / 4 / 5 / 7 / 8): batch 16 10.8 / 13.7 / 11.5 / 13.2 / 17.2 /
     // 19.1, batch 32 19.0 / 19.8 / 17.0 / 20.0 / 17.6 / 19.4, batch 64 30.9 / 30.1 / 30.4 / 29.4 / 27.1 / 29.9, batch 128
     // 59.1 / 55.9 / 51.2 / 53.8 / 49.8 / 55.3: as many rows as leave about two workgroups per compute unit, at most 7
@@ -2133,13 +2150,13 @@ int32_t kxc_hip_quantize_f32_nchw_to_c4_i8(const float* x, int8_t* y, int64_t n,
     if (total == 0) return KXC_HIP_OK;
     KXC_HIP_REQUIRE(x && y, "kxc_hip_quantize_f32_nchw_to_c4_i8: NULL pointer");
     KXC_HIP_REQUIRE(CeilDiv(total, kBlock) <= kMaxGridX, "kxc_hip_quantize_f32_nchw_to_c4_i8: tensor too large");
-    if (hw % 4 == 0 && hw / 4 < (1LL << 31) && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) & 15u) == 0) {
+    if (hw % 4 == 0 && total / 4 < (1LL << 31) - kBlock && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) & 15u) == 0) {
         quantize_to_c4_x4_kernel<<<NoteGrid(static_cast<int>(CeilDiv(total / 4, kBlock))), NoteBlock(kBlock), NoteLds(0),
-                                   ResolveStream(stream)>>>(x, y, static_cast<int32_t>(c), static_cast<int32_t>(hw / 4), total / 4, scale);
+                                   ResolveStream(stream)>>>(x, y, static_cast<int32_t>(c), static_cast<int32_t>(hw / 4), MakeFastDiv(static_cast<int32_t>(hw / 4)), static_cast<int32_t>(total / 4), scale);
         return CheckLaunch("quantize_f32_nchw_to_c4_i8");
     }
     quantize_to_c4_kernel<<<NoteGrid(static_cast<int>(CeilDiv(total, kBlock))), NoteBlock(kBlock), NoteLds(0),
-                            ResolveStream(stream)>>>(x, y, static_cast<int32_t>(c), hw, total, scale);
+                            ResolveStream(stream)>>>(x, y, static_cast<int32_t>(c), hw, MakeFastDiv(total < (1LL << 31) ? static_cast<int32_t>(hw) : 1), total, scale);
     return CheckLaunch("quantize_f32_nchw_to_c4_i8");
 }
 

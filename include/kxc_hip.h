@@ -367,7 +367,7 @@ int32_t kxc_hip_i8_nchw_to_c16(const int8_t* x, int8_t* y, int64_t n, int64_t c,
 int32_t kxc_hip_i8_c16_to_nchw(const int8_t* x, int8_t* y, int64_t n, int64_t c, int64_t hw, void* stream);
 int32_t kxc_hip_quantize_f32_nchw_to_c16_i8(const float* x, int8_t* y, int64_t n, int64_t c, int64_t hw,
                                             float scale, void* stream);
-/* First layer (7x7, stride 2, padding 3, at most 4 input channels, width a multiple of 4) on the "c4" input
+/* First layer (7x7, stride 2, padding 3, at most 4 input channels, rows of at least four pixels) on the "c4" input
  * layout [N][H][W][4] (4 bytes per pixel, channels >= C zero): a k-step of the matrix instruction is one
  * filter row of 8 taps x 4 channels.  Output is c16.  Weights are packed by the _c4_pack_weights call. */
 int32_t kxc_hip_qconv2d_c4_supported(const kxc_hip_qconv2d_desc* desc);

@@ -672,3 +672,28 @@ def test_plan_packs_many_weight_tensors_in_one_launch(pkg):
         torch.cuda.synchronize()
         assert_bit_exact(got, want, "batched pack of tensor %d %s" % (i, cases[i][1:]))
     plan.close()
+
+
+@pytest.mark.parametrize("shape", [(2, 3, 193, 193, 64), (3, 3, 70, 93, 32), (1, 4, 33, 66, 96), (2, 1, 9, 7, 32), (1, 2, 5, 5, 32), (2, 3, 40, 239, 64)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_qconv_first_layer_on_rows_of_any_width(pkg, orc, shape):
+    """Rows that are no multiple of four pixels: the last 16-byte piece of a row ends in the next row's pixels (or behind the tensor),
+    which must count as padding.  Byte for byte, with the max pool in the kernel and without."""
+    n, c, h, w, o = shape
+    rng = np.random.default_rng(sum(shape))
+    x = rng.integers(-128, 128, (n, c, h, w), dtype=np.int8)
+    wq = rng.integers(-127, 128, (o, c, 7, 7), dtype=np.int8)
+    bias = rng.integers(-20000, 20000, (o,), dtype=np.int32)
+    mult = rng.uniform(0.5, 2.0, (o,)).astype(np.float32) * np.float32(1.0 / (8.0 * np.sqrt(c * 49) * 64))
+    want = orc.qconv(x, wq, bias, mult, 2, 3, None, 0.0, True)
+    room = torch.full((n * h * w * 4 + 64,), 77, dtype=torch.int8, device="cuda")      # (what lies behind the tensor is not zero)
+    x4 = room[:n * h * w * 4].view(n, h, w, 4)
+    x4.zero_()
+    x4[..., :c] = dev(np.ascontiguousarray(x.transpose(0, 2, 3, 1)))
+    wp = pkg.qconv2d_c4_pack_weights(dev(wq))
+    got = pkg.qconv2d_c4(x4, c, wp, wq.shape, dev(bias), dev(mult), True)
+    assert_bit_exact(from_c16(pkg, got, o), want, "first layer")
+    if pkg.qconv2d_c4_maxpool_supported(x4.shape, o, c, True):
+        got = pkg.qconv2d_c4_maxpool(x4, c, wp, wq.shape, dev(bias), dev(mult), True)
+        assert_bit_exact(from_c16(pkg, got, o), orc.qmaxpool(want, 3, 2, 1), "first layer + max pool")
+    assert len(np.unique(want)) > 5
