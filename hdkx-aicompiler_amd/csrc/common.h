@@ -89,6 +89,16 @@ __device__ __forceinline__ void request_args(const Args& a) {
                  "s"(at(24)), "s"(at(25)), "s"(at(26)), "s"(at(27)), "s"(at(28)), "s"(at(29)));
 #endif
 }
+// The same for kernels that have no scalar registers to hold them all: one word of every 64 bytes, which brings the rest near.
+template <typename Args>
+__device__ __forceinline__ void request_lines(const Args& a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    constexpr int n = static_cast<int>(sizeof(Args) / 4);
+    const uint32_t* const q = reinterpret_cast<const uint32_t*>(&a);
+    auto at = [&](int i) __attribute__((always_inline)) { return q[i < n ? i : n - 1]; };
+    asm volatile("" ::"s"(at(0)), "s"(at(16)), "s"(at(32)), "s"(at(48)), "s"(at(64)), "s"(at(80)), "s"(at(96)));
+#endif
+}
 #endif
 
 // Reductions split over workgroups (both convolution kernels): every part writes raw partial outputs to

@@ -139,6 +139,7 @@ template <int KH, int KW, int CC, int WO, int WP, int RO, int RP, int PPT, int K
           bool HP = false>
 __global__ void __launch_bounds__(64 * WO * WP * KS) __attribute__((amdgpu_waves_per_eu(2)))
 conv_mfma_kernel(const ConvArgs a) {
+    request_lines(a);
     static_assert(!(DS && TPAIR), "the second output pairs channels");
     static_assert(!HP || (KS == 1 && !DS), "the pooling epilogue handles one reduction group and one output");
     constexpr int NW = WO * WP;                               // waves per reduction group

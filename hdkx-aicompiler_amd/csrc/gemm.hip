@@ -465,10 +465,10 @@ typedef int intx16_t __attribute__((ext_vector_type(16)));
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) qdense_mfma_kernel(const int8_t* __restrict__ a, const int8_t* __restrict__ b,
                                                          const int32_t* __restrict__ bias, const float* __restrict__ mult,
                                                          float* __restrict__ y, int32_t M, int32_t N, int32_t K,
-                                                         int32_t col_blocks) {
+                                                         int32_t col_blocks, FastDiv div_cols) {
     const int lane = threadIdx.x;
     const int r = lane & 31, half = lane >> 5;
-    const int ib = blockIdx.x / col_blocks, jb = blockIdx.x - ib * col_blocks;
+    const int ib = fast_div(static_cast<int>(blockIdx.x), div_cols), jb = static_cast<int>(blockIdx.x) - ib * col_blocks;
     const int i0 = ib * 32, j0 = jb * 32;
     const int8_t* ap = a + static_cast<int64_t>(min(i0 + r, M - 1)) * K + 16 * half;
     const int8_t* bp = b + static_cast<int64_t>(min(j0 + r, N - 1)) * K + 16 * half;
@@ -587,7 +587,7 @@ int32_t kxc_hip_qdense_i8(const int8_t* a, const int8_t* b, const int32_t* bias,
         const int32_t col_blocks = static_cast<int32_t>(CeilDiv(n, 32));
         qdense_mfma_kernel<<<NoteGrid(static_cast<int>(CeilDiv(m, 32) * col_blocks)), NoteBlock(64), NoteLds(0),
                              ResolveStream(stream)>>>(a, b, bias, mult, y, static_cast<int32_t>(m),
-                                                      static_cast<int32_t>(n), static_cast<int32_t>(k), col_blocks);
+                                                      static_cast<int32_t>(n), static_cast<int32_t>(k), col_blocks, MakeFastDiv(col_blocks));
         return CheckLaunch("qdense_mfma");
     }
     if (k % 16 == 0 && m < (1LL << 31) && n < (1LL << 31) && CeilDiv(n, 4) <= kMaxGridX &&

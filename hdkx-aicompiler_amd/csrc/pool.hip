@@ -5,6 +5,8 @@
 // contribute -1e30f), so results are bit-identical to the CPU loop nest, NaN and -0 included.
 // Global average pooling sums each plane sequentially in row-major order from 0.0f and then
 // performs a true IEEE division by (float)(H*W), which is the CPU loop nest's exact order too.
+#include <algorithm>
+
 #include "common.h"
 
 using namespace kxc_hip;
@@ -55,7 +57,8 @@ __global__ void __launch_bounds__(kBlock) pool_generic_kernel(const float* __res
 // issues two 16-byte loads (columns 2*ow0 .. 2*ow0+7); the ninth value, column 2*ow0-1,
 // is the left neighbour lane's last element, taken with a lane shuffle (a scalar reload only for
 // the first lane of a wave).  Consecutive lanes read consecutive 32-byte pieces of a row, every
-// input element is requested once per strip (plus the one shared row between vertical strips).
+// input element is requested once per strip (plus the one shared row between vertical strips).  Threads are numbered in 32 bits and their
+// numbers divided by multiplication (by 64-bit division, 300 instructions ahead of the first load).
 // ALIGNED (checked on the host): W % 8 == 0, OW == W/2, OH == H/2 (H even), 16-byte aligned planes.
 // Otherwise any extent: the same loads on 4-byte boundaries, columns past the row replaced by the padding value, single
 // elements where a load would pass the end of the tensor (64 channels at 97 x 97, batch 6: 9.8 us one thread per output with
@@ -64,15 +67,14 @@ struct __attribute__((packed, aligned(4))) Float4U { float x, y, z, w; };
 template <int ROWS, bool ALIGNED>
 __global__ void __launch_bounds__(kBlock) maxpool3x3s2_kernel(const float* __restrict__ x, float* __restrict__ y,
                                                               int32_t h, int32_t w, int32_t oh_total, int32_t ow_total,
-                                                              int32_t col_groups, int32_t row_groups, int64_t planes,
-                                                              int64_t total) {
-    const int64_t tid = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+                                                              int32_t col_groups, int32_t row_groups, FastDiv div_cols,
+                                                              FastDiv div_rows, int64_t planes, int32_t total) {
+    const int32_t tid = static_cast<int32_t>(blockIdx.x) * kBlock + static_cast<int32_t>(threadIdx.x);
     const bool active = tid < total;
-    const int64_t t = active ? tid : total - 1;
-    const int32_t cg = static_cast<int32_t>(t % col_groups);
-    const int64_t t2 = t / col_groups;
-    const int32_t rg = static_cast<int32_t>(t2 % row_groups);
-    const int64_t plane = t2 / row_groups;
+    const int32_t t = active ? tid : total - 1;
+    const int32_t t2 = fast_div(t, div_cols), cg = t - t2 * col_groups;
+    const int32_t first_plane = fast_div(t2, div_rows), rg = t2 - first_plane * row_groups;
+    const int64_t plane = first_plane;
     const float* xp = x + plane * h * w;
     const int64_t left_in_tensor = (planes - plane) * h * w;
     float* yp = y + plane * oh_total * ow_total;
@@ -162,13 +164,13 @@ __global__ void __launch_bounds__(kBlock) maxpool3x3s2_kernel(const float* __res
 template <int ROWS>
 __global__ void __launch_bounds__(kBlock) maxpool3x1s2_kernel(const float* __restrict__ x, float* __restrict__ y,
                                                               int32_t h, int32_t w, int32_t oh_total,
-                                                              int32_t col_groups, int32_t row_groups, int64_t total) {
-    const int64_t tid = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+                                                              int32_t col_groups, int32_t row_groups, FastDiv div_cols,
+                                                              FastDiv div_rows, int32_t total) {
+    const int32_t tid = static_cast<int32_t>(blockIdx.x) * kBlock + static_cast<int32_t>(threadIdx.x);
     if (tid >= total) return;
-    const int32_t cg = static_cast<int32_t>(tid % col_groups);
-    const int64_t t2 = tid / col_groups;
-    const int32_t rg = static_cast<int32_t>(t2 % row_groups);
-    const int64_t plane = t2 / row_groups;
+    const int32_t t2 = fast_div(tid, div_cols), cg = tid - t2 * col_groups;
+    const int32_t first_plane = fast_div(t2, div_rows), rg = t2 - first_plane * row_groups;
+    const int64_t plane = first_plane;
     const float* xp = x + plane * h * w + cg * 4;
     float* yp = y + plane * oh_total * w + cg * 4;
     const int32_t oh0 = rg * ROWS;
@@ -348,7 +350,9 @@ int32_t kxc_hip_pool2d_f32(const kxc_hip_pool2d_desc* desc, const float* x, floa
     if (total == 0) return KXC_HIP_OK;
     KXC_HIP_REQUIRE(x && y, "kxc_hip_pool2d_f32: NULL pointer");
     hipStream_t s = ResolveStream(stream);
-    if (!desc->is_avg && d.kh == 3 && d.kw == 3 && d.sh == 2 && d.sw == 2 && d.pt == 1 && d.pl == 1) {
+    // (more threads than 32 bits number: one thread per output below)
+    const bool countable = planes * (d.oh + 3) * ((std::max(d.ow, d.w) + 3) / 4) < (1LL << 31) - kBlock;
+    if (!desc->is_avg && d.kh == 3 && d.kw == 3 && d.sh == 2 && d.sw == 2 && d.pt == 1 && d.pl == 1 && countable) {
         const bool aligned = desc->pad_bottom == 1 && desc->pad_right == 1 && !desc->ceil_mode && (d.w % 8) == 0 &&
                              (d.h % 2) == 0 && d.ow == d.w / 2 && d.oh == d.h / 2 &&
                              (reinterpret_cast<uintptr_t>(x) & 15u) == 0 && (reinterpret_cast<uintptr_t>(y) & 15u) == 0;
@@ -364,10 +368,10 @@ int32_t kxc_hip_pool2d_f32(const kxc_hip_pool2d_desc* desc, const float* x, floa
         auto* const kernel = small ? (aligned ? maxpool3x3s2_kernel<1, true> : maxpool3x3s2_kernel<1, false>)
                                    : (aligned ? maxpool3x3s2_kernel<4, true> : maxpool3x3s2_kernel<4, false>);
         kernel<<<NoteGrid(static_cast<int>(blocks)), NoteBlock(kBlock), NoteLds(0), s>>>(x, y, d.h, d.w, d.oh, d.ow, col_groups, row_groups,
-                                                                                         planes, threads);
+                                                                                         MakeFastDiv(col_groups), MakeFastDiv(row_groups), planes, static_cast<int32_t>(threads));
         return CheckLaunch("maxpool3x3s2");
     }
-    const bool columns = !desc->is_avg && d.kh == 3 && d.kw == 1 && d.sh == 2 && d.sw == 1 && d.pt == 1 && d.pl == 0 &&
+    const bool columns = countable && !desc->is_avg && d.kh == 3 && d.kw == 1 && d.sh == 2 && d.sw == 1 && d.pt == 1 && d.pl == 0 &&
                          desc->pad_right == 0 && desc->pad_bottom <= 1 && !desc->ceil_mode && (d.w % 4) == 0 &&
                          (reinterpret_cast<uintptr_t>(x) & 15u) == 0 && (reinterpret_cast<uintptr_t>(y) & 15u) == 0;
     if (columns) {
@@ -378,12 +382,9 @@ int32_t kxc_hip_pool2d_f32(const kxc_hip_pool2d_desc* desc, const float* x, floa
         const int64_t threads = planes * row_groups * col_groups;
         const int64_t blocks = CeilDiv(threads, kBlock);
         KXC_HIP_REQUIRE(blocks <= kMaxGridX, "kxc_hip_pool2d_f32: tensor too large");
-        if (small)
-            maxpool3x1s2_kernel<1><<<NoteGrid(static_cast<int>(blocks)), NoteBlock(kBlock), NoteLds(0), s>>>(
-                x, y, d.h, d.w, d.oh, col_groups, row_groups, threads);
-        else
-            maxpool3x1s2_kernel<4><<<NoteGrid(static_cast<int>(blocks)), NoteBlock(kBlock), NoteLds(0), s>>>(
-                x, y, d.h, d.w, d.oh, col_groups, row_groups, threads);
+        auto* const kernel = small ? maxpool3x1s2_kernel<1> : maxpool3x1s2_kernel<4>;
+        kernel<<<NoteGrid(static_cast<int>(blocks)), NoteBlock(kBlock), NoteLds(0), s>>>(x, y, d.h, d.w, d.oh, col_groups, row_groups, MakeFastDiv(col_groups),
+                                                                                         MakeFastDiv(row_groups), static_cast<int32_t>(threads));
         return CheckLaunch("maxpool3x1s2");
     }
     if (desc->is_avg) pool_generic_kernel<true><<<NoteGrid(GridFor(total)), NoteBlock(kBlock), NoteLds(0), s>>>(x, y, d, total);
