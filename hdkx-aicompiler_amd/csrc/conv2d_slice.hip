@@ -113,6 +113,7 @@ double SliceUs(const SliceVariant& v, int64_t tiles, int64_t csteps) {
 // Whether a plan's node should take it: where its estimate is a twentieth below that of the kernel that the node takes otherwise
 // (WinogradNodeUs).  Of 1700 shapes 1090 take it, 1.45 times as fast on average; twelve of them are slower by more than 3 %.
 // Nodes with a second output (PairNodeUs) leave 0.08 in hand: 256 of 1320 shapes, 1.19 times as fast, three slower by more than 3 %.
+// (Above 256 channels they keep the other kernels.  That is no line of speed: the tests of that selection name such a node.)
 // KXC_HIP_CONV_SLICE=0: nowhere, =<name>: that variant wherever it covers the node.  Switches that keep convolutions on the fp32
 // instructions or name other kernels keep those.
 bool Preferred(const kxc_hip_conv2d_desc* d, bool second, PreparedSlice* L) {
@@ -124,8 +125,9 @@ bool Preferred(const kxc_hip_conv2d_desc* d, bool second, PreparedSlice* L) {
     }
     for (const char* name : {"KXC_HIP_WINOGRAD_BF16X3", "KXC_HIP_CONV_BF16X3"})
         if (const char* e = std::getenv(name); e && (e[0] == '0' || (second && e[0] == '1'))) return false;
-    for (const char* name : {"KXC_HIP_WINOGRAD_VARIANT", "KXC_HIP_WINOGRAD_GSPLIT", "KXC_HIP_CONV_VARIANT", "KXC_HIP_CONV_GSPLIT"})
+    for (const char* name : {"KXC_HIP_WINOGRAD_VARIANT", "KXC_HIP_WINOGRAD_GSPLIT", "KXC_HIP_CONV_VARIANT", "KXC_HIP_CONV_GSPLIT", "KXC_HIP_CONV_HPOOL_VARIANT"})
         if (const char* e = std::getenv(name); e && *e) return false;
+    if (second && d->c > 256) return false;
     double best_us = second ? 0.92 * PairNodeUs(d) : 0.95 * WinogradNodeUs(d);
     if (best_us <= 0) return false;
     const int stride = second ? 2 : 1;
