@@ -9,6 +9,7 @@
 
 #include "conv7_bf16x3.h"
 #include "conv_bf16x3.h"
+#include "conv_point.h"
 
 using namespace kxc_hip;
 
@@ -20,6 +21,8 @@ struct PackedLaunch {
     void (*pack)(const float*, char*, int32_t, int32_t) = nullptr;
     conv7_bx::Args a7;                                    // kernel7
     void (*kernel7)(const conv7_bx::Args) = nullptr;
+    conv_pt::Args ap;                                     // kernel1
+    void (*kernel1)(const conv_pt::Args) = nullptr;
     size_t lds_bytes = 0, filter_bytes = 0;
     double gflop = 0;
     const char* name = "";
@@ -170,6 +173,35 @@ bool Resolve7(const kxc_hip_conv2d_desc* d, PackedLaunch* L) {
     return true;
 }
 
+// conv_point.h: workgroups that share a tile of pixels.  As many as give 384 workgroups, each with a block for every wave (us, 1 / 2 / 4 groups:
+// 128 -> 512 channels at 28 x 28, batch 32, 392 tiles, 34.1 / 37.3 / 39.8, batch 8, 98 tiles, 22.5 / 16.2 / 14.7; 128 -> 1024 at 14 x 14,
+// batch 64, 196 tiles, 43.1 / 34.6 / 38.5), and at most 64 blocks to one: their biases lie in LDS, which two workgroups share.
+int64_t PointGroups(int64_t tiles, int64_t all) {
+    return std::max(CeilDiv(all, conv_pt::kMaxBlocks), std::min(CeilDiv(384, tiles), all / conv_pt::kWaves));
+}
+
+// The same for the 1x1 kernel that keeps a workgroup's pixels (after Resolve).
+void ResolvePoint(const kxc_hip_conv2d_desc* d, PackedLaunch* L) {
+    using namespace conv_pt;
+    if (d->kh != 1 || d->stride_h != 1 || d->pad_h != 0 || d->pad_w != 0 || d->c > 16 * kMaxSteps || L->a.HW % 4 != 0) return;
+    Args& a = L->ap;
+    std::memset(&a, 0, sizeof(a));
+    a.C = d->c; a.O = d->o; a.HW = L->a.HW; a.M = L->a.M;
+    a.csteps = L->a.csteps;
+    const int64_t all = CeilDiv(a.O, 32), tiles = CeilDiv(a.M, kPix);
+    a.blocks = static_cast<int32_t>(CeilDiv(all, PointGroups(tiles, all)));
+    a.groups = static_cast<int32_t>(CeilDiv(all, a.blocks));
+    a.num_units = static_cast<int32_t>(tiles * a.groups);
+    a.units_per_xcd = static_cast<int32_t>(CeilDiv(a.num_units, 8));
+    a.x_bytes = L->a.x_bytes; a.u_bytes = L->a.u_bytes; a.flags = d->flags;
+    a.y_bytes = static_cast<uint32_t>(a.M) * static_cast<uint32_t>(a.O) * 4u;
+    a.div_hw = MakeFastDiv(a.HW); a.div_groups = MakeFastDiv(a.groups);
+    const int steps = d->c <= 64 ? 4 : 8;
+    L->kernel1 = steps == 4 ? conv_point_kernel<4> : conv_point_kernel<8>;
+    L->lds_bytes = LdsBytes(steps, a.blocks);
+    L->scratch_bytes = 0;
+}
+
 // Whether to take a kernel that the rule for its launch does or does not ask for.  KXC_HIP_CONV_BF16X3=1: wherever it covers the launch,
 // =0: nowhere.  KXC_HIP_WINOGRAD_BF16X3=0 keeps every convolution on the fp32 instructions, as it did when no other kernel had
 // three-part operands.
@@ -252,6 +284,14 @@ bool Preferred(const kxc_hip_conv2d_desc* d, bool second, PackedLaunch* L) {
 // `partials`: room for the partial outputs of a split reduction; nullptr: it is acquired here.
 int32_t LaunchConv(const PackedLaunch& L, const float* x, const float* w, const void* u, const float* bias, const float* residual, float* y,
                    const float* w2, const float* bias2, float* y2, hipStream_t s, float* partials) {
+    if (L.kernel1) {
+        conv_pt::Args b = L.ap;
+        b.x = x; b.w = w; b.u = static_cast<const char*>(u); b.bias = bias; b.res = residual; b.y = y;
+        if (L.lds_bytes > 64 * 1024)
+            if (int32_t rc = GrantLds(reinterpret_cast<const void*>(L.kernel1))) return rc;
+        hipLaunchKernelGGL(L.kernel1, NoteGrid(dim3(static_cast<unsigned>(b.units_per_xcd * 8))), NoteBlock(dim3(conv_pt::kThreads)), NoteLds(L.lds_bytes), s, b);
+        return CheckLaunch(L.name);
+    }
     conv_bx::Args a = L.a;
     a.x = x; a.w = w; a.u = static_cast<const char*>(u); a.bias = bias; a.res = residual; a.y = y;
     a.w2 = w2; a.bias2 = bias2; a.y2 = y2;
@@ -286,6 +326,20 @@ int32_t LaunchConv(const PackedLaunch& L, const float* x, const float* w, const 
     return LaunchSplitReduce(s, r);
 }
 
+// Whether a 1x1 call of at most 128 channels should take conv_point.h: a twentieth shorter by the estimates, which are fitted to 420 calls of 0.01
+// to 4 GFLOP within 8 % here, 9 % (small-launch kernel) and a quarter (the others: whole tiles of 128 channels; below 32 the direct kernel).
+// 126 of them take it and run 1.37 times as fast, eight slower (23.3 us against 19.4 for 112 -> 48 at 53 x 96, batch 14, the furthest); 27
+// others would have gained a tenth.
+bool PointRule(const kxc_hip_conv2d_desc* d, int64_t pixels, int64_t lanes, double blocks, double memory) {
+    const int64_t all = CeilDiv(d->o, 32), tiles = CeilDiv(pixels, conv_pt::kPix);
+    const int64_t own = CeilDiv(all, PointGroups(tiles, all)), units = tiles * CeilDiv(all, own) * lanes;
+    const double walk = 0.44 + (d->c <= 64 ? 1.86 : 2.77) * static_cast<double>(CeilDiv(own, conv_pt::kWaves));
+    const double here = 6.5 + 0.71 * memory + walk * std::max(1.0, static_cast<double>(units) / 512), m = 2e-9 * static_cast<double>(lanes * pixels);
+    const double others = SmallConvTakes(d, false, false) ? 3.3 + 8.5 * blocks + 1.06 * memory
+                          : d->o < 32 ? 480 * m * d->o * d->c : 8.7 + 18.7 * m * (CeilDiv(d->o, 128) * 128) * (CeilDiv(d->c, 16) * 16) + 0.46 * memory;
+    return here < 0.95 * others;
+}
+
 // Whether a single call, which packs its filter first, should take the kernel: a twentieth shorter than the others, by what both
 // sides take, fitted to 500 calls of 0.05 to 4 GFLOP within 5 % here and a tenth there.  Here by filter: two launches, a workgroup's start and its steps
 // (a 1x1 filter's few steps do not hide the bytes, from caches mostly).  The others: GFLOP of whole blocks, at 1x1 the bytes as well; the
@@ -310,6 +364,7 @@ bool OperatorRule(const kxc_hip_conv2d_desc* d) {
     const int64_t pixels = static_cast<int64_t>(pixels_d), lanes = SelectLanes();
     const double memory = lanes * (4.0 * d->n * d->c * d->h * d->w + out_bytes * ((d->flags & KXC_HIP_CONV_RESIDUAL) ? 2 : 1)) / 4.5e6;
     const double blocks = lanes * BlockGflop(d, pixels, K * K, 32);
+    if (K == 1 && d->c <= 16 * conv_pt::kMaxSteps) return PointRule(d, pixels, lanes, blocks, memory);
     const int64_t units = CeilDiv(pixels, kPix) * CeilDiv(d->o, kOut);
     const int csteps = static_cast<int>(CeilDiv(d->c, kStep * ChannelSteps(K))), steps = Steps(K, false);
     const int split = Split(units * lanes, csteps, steps, static_cast<int64_t>(out_bytes));
@@ -328,7 +383,9 @@ bool OperatorRule(const kxc_hip_conv2d_desc* d) {
 bool OperatorPreferred(const kxc_hip_conv2d_desc* d, PackedLaunch* L) {
     const int K = d->kh, S = d->stride_h;
     if (K != d->kw || S != d->stride_w || d->n <= 0 || d->c <= 0 || d->o <= 0 || (S != 1 && S != 2) || K > 7) return false;
-    return Switched(OperatorRule(d)) && !OthersForced() && Resolve(d, false, L) && L->filter_bytes <= (32u << 20);      // (bounds the scratch kept per stream)
+    if (!(Switched(OperatorRule(d)) && !OthersForced() && Resolve(d, false, L) && L->filter_bytes <= (32u << 20))) return false;      // (bounds the scratch kept per stream)
+    ResolvePoint(d, L);
+    return true;
 }
 
 }  // namespace

@@ -387,3 +387,50 @@ def test_packed_calls_from_threads_and_streams(pkg, xs, o, k):
     _in_threads(4, calls)
     torch.cuda.synchronize()
     assert all(torch.equal(y, want[i]) for i in range(4) for y in out[i])
+
+
+@pytest.mark.parametrize("xs, o, residual, bias, relu", [
+    ((1, 1, 2, 2), 1, True, True, True),                    # one channel, four pixels of a tile of 64
+    ((3, 17, 4, 5), 33, True, True, False),                 # images meet inside a tile; one channel in the second step and the second block
+    ((2, 64, 10, 18), 96, False, False, True),              # the last channels of the kernel of four steps; three blocks, a wave without one
+    ((2, 65, 6, 14), 130, True, False, True),               # ... the first of the kernel of eight; waves with two blocks and one
+    ((5, 128, 7, 12), 1000, True, True, True),              # workgroups that share their pixels, the last with fewer blocks
+    ((1, 20, 8, 8), 2100, False, True, False),
+    ((400, 33, 8, 8), 160, True, True, True),               # more tiles than workgroups that share them: one to a tile
+])
+def test_pointwise_convolution_of_few_channels(pkg, monkeypatch, xs, o, residual, bias, relu):
+    """conv_point.h at the edges of its tiles, on operands that are aligned and that are not, with the residual in the output's place, and
+    no further from float64 than the fp32 instructions beyond what the last roundings differ by."""
+    rng = np.random.default_rng(sum(xs) + o)
+    n, c, h, w = xs
+    f32 = lambda s, scale=1.0: (rng.standard_normal(s) * scale).astype(np.float32)
+    x, wt, b, ys = f32(xs), f32((o, c, 1, 1), (2 / c) ** 0.5), f32((o,)) if bias else None, (n, o, h, w)
+    res = f32(ys) if residual else None
+
+    def gpu(a, shift):
+        if a is None:
+            return None
+        t = torch.empty(a.size + 4, device="cuda")[shift:shift + a.size].view(a.shape)
+        return t.copy_(dev(a))
+
+    want = _want(x, wt, b, res, relu, 1, 0)
+    error = lambda y: np.linalg.norm(y - want) / np.linalg.norm(want)
+    monkeypatch.setenv("KXC_HIP_CONV_BF16X3", "0")
+    plain = error(host(pkg.conv2d(gpu(x, 0), gpu(wt, 0), gpu(b, 0), gpu(res, 0), 1, 0, 1, relu)))
+    monkeypatch.setenv("KXC_HIP_CONV_BF16X3", "1")
+    assert pkg.conv2d_variant(x.shape, wt.shape, 1, 0) == "mfma_k1x1s1_bf16x3"
+    first = None
+    for shift in (0, 1):
+        r, out = gpu(res, shift), gpu(np.zeros(ys, np.float32), shift)
+        for y in (out, r) if residual else (out,):
+            y = pkg.conv2d(gpu(x, shift), gpu(wt, shift), gpu(b, shift), r, 1, 0, 1, relu, out=y)
+            first = host(y) if first is None else first
+            assert_bit_exact(host(y), first, "shift %d" % shift)
+    assert error(first) <= (c + 16) ** 0.5 * 2.0 ** -23
+    assert error(first) <= max(1.05 * plain, 2.0 ** -24)     # (of few terms both are the last rounding's)
+    x[n - 1, c - 1, h - 1, w - 1], x[0, 0, 0, 1], wt[o - 1, c // 2, 0, 0] = np.inf, np.nan, -np.inf
+    want = _want(x, wt, b, res, False, 1, 0)
+    got, want = host(pkg.conv2d(dev(x), dev(wt), gpu(b, 0), gpu(res, 0), 1, 0, 1, relu)), np.where(want > 0, want, 0.0) if relu else want
+    assert (np.isnan(got) == np.isnan(want)).all() and (got[np.isinf(want)] == want[np.isinf(want)]).all()
+    m = np.isfinite(want)
+    assert (np.abs(got[m] - want[m]) <= 1e-5 * np.maximum(np.abs(want[m]), 1.0)).all()
