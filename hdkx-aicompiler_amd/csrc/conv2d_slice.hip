@@ -113,6 +113,10 @@ double SliceUs(const SliceVariant& v, int64_t tiles, int64_t csteps) {
 // Whether a plan's node should take it: where its estimate is a twentieth below that of the kernel that the node takes otherwise
 // (WinogradNodeUs).  Of 1700 shapes 1090 take it, 1.45 times as fast on average; twelve of them are slower by more than 3 %.
 // Nodes with a second output (PairNodeUs) leave 0.08 in hand: 256 of 1320 shapes, 1.19 times as fast, three slower by more than 3 %.
+// Those fits are to nodes that run alone, again and again.  Between the other layers of a network, where the matrix cores' clock is lower, they take
+// longer by their arithmetic, which is 2.25 times the others' (162 nodes of ResNet-18 at batch 4 to 63, within 7 %): 64 channels at 56 x 56, batch 24 41 us
+// for 34 alone, the others 33; 128 at 28 x 28, batch 20 33 for 23, the others 25; 256 at 14 x 14, batch 24 41 for 32, the others 34, batch 8 14.5 and 21; 512 at 7 x 7, batch
+// 20 26.5 and 33.6.
 // (Above 256 channels they keep the other kernels.  That is no line of speed: the tests of that selection name such a node.)
 // KXC_HIP_CONV_SLICE=0: nowhere, =<name>: that variant wherever it covers the node.  Switches that keep convolutions on the fp32
 // instructions or name other kernels keep those.
@@ -133,10 +137,12 @@ bool Preferred(const kxc_hip_conv2d_desc* d, bool second, PreparedSlice* L) {
     const int stride = second ? 2 : 1;
     const int64_t oh = (static_cast<int64_t>(d->h) + 2 * d->pad_h - 3) / stride + 1, ow = (static_cast<int64_t>(d->w) + 2 * d->pad_w - 3) / stride + 1;
     const int64_t pixels = d->n * oh * ow, csteps = CeilDiv(d->c, conv_sl::kStep);
+    const double gflop = 2e-9 * static_cast<double>(SelectLanes() * pixels) * d->o * d->c * (second ? 10 : 9);
     const SliceVariant* best = nullptr;
     for (const SliceVariant& v : kSlices) {
         if (csteps < v.ks || v.second != second) continue;      // (a wave without a step)
-        const double us = SliceUs(v, CeilDiv(pixels, conv_sl::kPix) * CeilDiv(d->o, 32 * v.ro) * SelectLanes(), csteps);
+        const double alone = SliceUs(v, CeilDiv(pixels, conv_sl::kPix) * CeilDiv(d->o, 32 * v.ro) * SelectLanes(), csteps);
+        const double us = std::max(alone, second ? 3.0 + 0.73 * alone + 3.37 * gflop : 1.06 + 0.745 * alone + 2.44 * gflop);
         if (us < best_us) { best_us = us; best = &v; }
     }
     return best && Resolve(d, second, *best, L);
