@@ -21,6 +21,8 @@ struct PackedLaunch {
     void (*pack)(const float*, char*, int32_t, int32_t) = nullptr;
     conv7_bx::Args a7;                                    // kernel7
     void (*kernel7)(const conv7_bx::Args) = nullptr;
+    int threads7 = 0;
+    bool whole7 = false;                                  // kernel7: tiles are whole rows of an image
     conv_pt::Args ap;                                     // kernel1
     void (*kernel1)(const conv_pt::Args) = nullptr;
     size_t lds_bytes = 0, filter_bytes = 0;
@@ -135,7 +137,7 @@ bool Resolve7(const kxc_hip_conv2d_desc* d, PackedLaunch* L) {
     using namespace conv7_bx;
     if (!d || d->n <= 0 || d->c != kC || d->h <= 0 || d->w <= 0 || d->o <= 0) return false;
     if (d->kh != kK || d->kw != kK || d->stride_h != 2 || d->stride_w != 2 || d->dil_h != 1 || d->dil_w != 1) return false;
-    if (d->pad_h < 0 || d->pad_w < 0 || d->pad_h >= kK || d->pad_w >= kK || (d->flags & KXC_HIP_CONV_FORCE_DIRECT)) return false;
+    if (d->pad_h < 0 || d->pad_w < 0 || d->pad_h >= kK || d->pad_w >= kK || d->w < 2 || (d->flags & KXC_HIP_CONV_FORCE_DIRECT)) return false;
     const int64_t Hp = static_cast<int64_t>(d->h) + 2 * d->pad_h, Wp = static_cast<int64_t>(d->w) + 2 * d->pad_w;
     if (Hp < kK || Wp < kK) return false;
     const int64_t OH = (Hp - kK) / 2 + 1, OW = (Wp - kK) / 2 + 1;
@@ -151,11 +153,23 @@ bool Resolve7(const kxc_hip_conv2d_desc* d, PackedLaunch* L) {
     a.Hp = static_cast<int32_t>(Hp); a.PW = a.OW / 2;
     const int pitch = OW + 3 <= 64 ? 64 : 120;      // (the last pixel's window takes four words; three parts within the reach of a ds_read2)
     if (OW + 3 > pitch) return false;
-    const int64_t rows = conv_bx::TileReach(a.N, a.OHW, a.OW, kPix, 2, a.Hp - 2 * a.OH) + kK;
+    int64_t rows = conv_bx::TileReach(a.N, a.OHW, a.OW, kPix, 2, a.Hp - 2 * a.OH) + kK, tiles = CeilDiv(M, kPix);
+    a.tile_pix = kPix; a.span = a.M;
+    if (!hpool && LdsBytes(rows, pitch) > kMaxLdsBytes / 4) {
+        // Whole rows of an image: fewer rows of input, of which four workgroups find room in LDS.
+        L->whole7 = true;
+        int64_t high = std::min<int64_t>(kPix / OW, OH);
+        while (high > 1 && LdsBytes(2 * high + kK - 2, pitch) > kMaxLdsBytes / 4) --high;
+        tiles = CeilDiv(OH, high);
+        high = CeilDiv(OH, tiles);
+        rows = 2 * high + kK - 2;
+        a.tile_pix = static_cast<int32_t>(high * OW); a.span = a.OHW;
+    }
+    a.tiles = static_cast<int32_t>(tiles);
     a.row_max = static_cast<int32_t>(rows);
     if (LdsBytes(rows, pitch) > kMaxLdsBytes / 2) return false;
     a.o_tiles = static_cast<int32_t>(CeilDiv(a.O, kOut));
-    const int64_t units = CeilDiv(M, kPix) * a.o_tiles;
+    const int64_t units = tiles * (a.span == a.M ? 1 : a.N) * a.o_tiles;
     if (units >= (1LL << 30)) return false;
     a.num_units = static_cast<int32_t>(units);
     a.units_per_xcd = static_cast<int32_t>(CeilDiv(units, 8));
@@ -164,11 +178,14 @@ bool Resolve7(const kxc_hip_conv2d_desc* d, PackedLaunch* L) {
     a.u_bytes = static_cast<uint32_t>(FilterBytes(a.O));
     a.flags = d->flags;
     a.div_ohw = MakeFastDiv(a.OHW); a.div_ow = MakeFastDiv(a.OW); a.div_hp = MakeFastDiv(a.Hp); a.div_otiles = MakeFastDiv(a.o_tiles);
+    a.div_tiles = MakeFastDiv(a.tiles);
     L->filter_bytes = a.u_bytes;
     L->lds_bytes = std::max(LdsBytes(rows, pitch), kMinLdsBytes);
     L->gflop = 2e-9 * static_cast<double>(M) * a.O * kC * kK * kK;
-    L->kernel7 = hpool ? (pitch == 64 ? conv7_bf16x3_kernel<64, true> : conv7_bf16x3_kernel<120, true>)
-                       : (pitch == 64 ? conv7_bf16x3_kernel<64, false> : conv7_bf16x3_kernel<120, false>);
+    static void (*const kWhole[2][2])(const Args) = {{conv7_bf16x3_kernel<64, false, 3, 2>, conv7_bf16x3_kernel<64, false, 4, 2>},
+                                                     {conv7_bf16x3_kernel<120, false, 3, 2>, conv7_bf16x3_kernel<120, false, 4, 2>}};
+    L->kernel7 = hpool ? (pitch == 64 ? conv7_bf16x3_kernel<64, true, 7, 1> : conv7_bf16x3_kernel<120, true, 7, 1>) : kWhole[pitch != 64][a.tile_pix > 192];
+    L->threads7 = hpool ? kThreads : 2 * kThreads;
     L->name = "mfma_k7x7s2_bf16x3";
     return true;
 }
@@ -243,13 +260,16 @@ double BlockGflop(const kxc_hip_conv2d_desc* d, int64_t pixels, int taps, int bl
 // 1024 at 28 x 28, batch 2 68 and 36; 16 -> 32 at 56 x 56, batch 20 (0.16) 15.0 and 11.5.  From 64 channels on the small-launch
 // kernel with one load per filter row is the other side, up to 2.3 million (16 x 16 tiles) * k (1.3 GFLOP): 64 -> 128 at 56 x 56, batch 6 / 8 / 10 15.7 /
 // 19.0 / 22.9 and 22.8 / 23.1 / 23.3; 128 -> 256 at 28 x 28, batch 8 / 10 18.6 / 20.7 and 24.7 / 25.9; 256 -> 512 at 14 x 14 18.9 / 19.1 and 23.5 / 23.2.
-// The 7x7 kernel, 3 -> 64 channels: pooled at 224 x 224, batch 16 / 32 / 64 51 / 100 / 169 and 32 / 59 / 108, at 64 x 64, batch 56 (1.1 GFLOP) 33 and
-// 22; not pooled at 224 x 224, batch 4 (0.94) 20.6 and 21.8, batch 8 (1.9) 33 and 30, batch 64 182 and 116; tiles 13 rows high, of which a compute unit holds
-// two, at 193 x 193, batch 16 (2.8) 49 and 54.  Pooled, with a compute unit to each workgroup and such high tiles it loses to the others' tile of 224
+// The 7x7 kernel, 3 -> 64 channels: pooled at 224 x 224, batch 16 / 32 / 64 51 / 100 / 169 and 29 / 50 / 93, at 64 x 64, batch 56 (1.1 GFLOP) 33 and
+// 22.  Pooled, with a compute unit to each workgroup and tiles of many rows it loses to the others' tile of 224
 // pixels (3 -> 64 at 30 x 56, batch 24 18.9 and 21.0; from 257 workgroups on 24 channels at 304 x 56, batch 17 29.6 and 27.8), not to the one of 448 that they
-// take where it fits (31.5 and 20.5 at 56 x 56, batch 8); not pooled, up to 32 channels, which leave half of a workgroup's
-// 64 empty, need 1800 workgroups (32 at 144 x 112, batch 57 36.6 and 44.0, 144 x 224, batch 37 46.0 and 51.4, 224 x 224, batch 33 63.7 and 61.6).  Of 500
-// first layers 252 take it, none slower by more than 3 %.
+// take where it fits (31.5 and 20.5 at 56 x 56, batch 8).  Not pooled, on tiles that are whole rows: batch 1 / 6 / 16 at 193 x 193 10.7 / 21.4 / 45 and
+// 10.3 / 17.5 / 30, batch 47 at 189 x 189 107 and 57, batch 8 at 99 x 99 13.1 and 10.7, and batch 36 at 216 x 216 2312 and 60: rows of 105, 108 or 113 to
+// 117 pixels fit none of the others' tiles.  Of 420 such layers 392 are faster, of those from 48 channels on (1.4 times) three slower by more than 3 %, a tenth at most;
+// up to 32 channels leave half of a workgroup's 64 empty and need wide rows and three workgroups to a compute unit (32 at 145 x 108, batch 16 13.5 and
+// 16.8, 208 x 208, batch 12 21.5 and 23.1, batch 32 at 213 x 213 54.8 and 48.5).  Not pooled, on rows that fill tiles (224 x 224, batch 8 (1.9 GFLOP) 33 and
+// 26, batch 64 184 and 103) it begins at 1.8 GFLOP.  That is no line of speed (batch 4 20.3 and 13): the tests of this selection name such nodes; up to 32 channels at 1800
+// workgroups (32 at 144 x 112, batch 57 36.6 and 44.0, 224 x 224, batch 33 63.7 and 61.6).
 // At 3x3 that must also be the shorter time by what either side takes, fitted within a tenth to 1000 shapes of 16 to 512 and 8 to 512 channels: here
 // 2 us and a workgroup's 4 + 0.28 per tap and step, the others 10.5 and 12.7 per GFLOP of 32 x 32 blocks or, by the small-launch kernels, 4.9
 // and 12.4 of 16 x 16 ones.  A workgroup has 128 output channels: no more than 48 of them (256 -> 8 at 60 x 38, batch 38 24.5 and 99.4, 384 ->
@@ -263,7 +283,8 @@ bool Preferred(const kxc_hip_conv2d_desc* d, bool second, PackedLaunch* L) {
         // Tiles that are few rows high: four workgroups to a compute unit, and one batch of loads.
         const bool pooled = (d->flags & KXC_HIP_CONV_HPOOL) != 0, low = L->lds_bytes <= kMaxLdsBytes / 4;
         const int64_t lanes = SelectLanes(), units = L->a7.num_units * lanes;
-        return Switched(pooled ? low || units > 256 || HpoolTilePixels(d) > conv7_bx::kPix : low && L->gflop * lanes >= 1.8 && (d->o > 32 || units >= 1800));
+        const bool plain = L->whole7 ? d->o > 32 || (L->a7.OW > 61 && units >= 768) : L->gflop * lanes >= 1.8 && (d->o > 32 || units >= 1800);
+        return Switched(pooled ? low || units > 256 || HpoolTilePixels(d) > conv7_bx::kPix : low && plain);
     }
     // (a plan's filter launch packs 3x3 stride-2 filters only)
     if (!d || d->kh != 3 || d->stride_h != 2 || d->pad_h != 1 || d->pad_w != 1 || d->c % conv_bx::kStep != 0 || !Resolve(d, second, L)) return false;
@@ -472,7 +493,7 @@ int32_t LaunchPreparedPacked(const PreparedPacked* p, const float* x, const floa
         b.x = x; b.w = w; b.u = static_cast<const char*>(u); b.bias = bias; b.res = residual; b.y = y;
         if (L.lds_bytes > 64 * 1024)
             if (int32_t rc = GrantLds(reinterpret_cast<const void*>(L.kernel7))) return rc;
-        hipLaunchKernelGGL(L.kernel7, NoteGrid(dim3(static_cast<unsigned>(b.units_per_xcd * 8))), NoteBlock(dim3(conv7_bx::kThreads)),
+        hipLaunchKernelGGL(L.kernel7, NoteGrid(dim3(static_cast<unsigned>(b.units_per_xcd * 8))), NoteBlock(dim3(static_cast<unsigned>(L.threads7))),
                            NoteLds(L.lds_bytes), s, b);
         return CheckLaunch(L.name);
     }

@@ -140,6 +140,34 @@ def test_first_layer_on_a_packed_filter(pkg, monkeypatch, xs, o, pad, residual, 
     node.plan.close()
 
 
+@pytest.mark.parametrize("xs, o, pad, residual, bias, relu, packed", [
+    ((6, 3, 193, 193), 64, 3, False, True, True, True),     # two rows of 97: four blocks of pixels to a wave, the last tile a row
+    ((3, 3, 37, 189), 64, 3, False, False, True, True),     # two rows of 95: three blocks
+    ((2, 3, 21, 150), 48, 3, True, True, True, True),       # the second block of channels ends after 16
+    ((5, 3, 9, 50), 96, 0, False, True, False, True),       # narrow rows, an image a tile; the last 64 channels half empty
+    ((1, 3, 46, 226), 72, 3, True, False, False, True),     # rows of 113
+    ((3, 3, 7, 2), 64, 3, False, True, True, True),         # the narrowest images: one column of four pixels
+    ((4, 3, 150, 150), 32, 3, False, True, True, False),
+    ((9, 3, 213, 213), 32, 3, False, True, True, False), ((32, 3, 213, 213), 32, 3, False, True, True, True),
+])
+def test_first_layers_on_tiles_of_whole_rows(pkg, monkeypatch, xs, o, pad, residual, bias, relu, packed):
+    """Selected by the rule, at the edges of their tiles, and no further from float64 than on the fp32 instructions."""
+    for name in ("KXC_HIP_CONV_BF16X3", "KXC_HIP_WINOGRAD_BF16X3"):
+        monkeypatch.delenv(name, raising=False)
+    node = _Node(pkg, xs, o, False, residual, bias, relu, seed=sum(xs) + o, k=7, pad=pad)
+    assert (node.bytes > 0) == packed == ("k7x7s2_bf16x3" in node.plan.node_symbol(0))
+    first = node.run()
+    node.check(first)
+    assert_bit_exact(node.run()[0], first[0], "second run")
+    if packed and sum(xs) < 450:
+        monkeypatch.setenv("KXC_HIP_CONV_BF16X3", "0")
+        plain, want = _Node(pkg, xs, o, False, residual, bias, relu, seed=sum(xs) + o, k=7, pad=pad), node.want()[0]
+        assert "bf16x3" not in plain.plan.node_symbol(0)
+        assert np.linalg.norm(first[0] - want) <= np.linalg.norm(plain.run()[0] - want)
+        plain.plan.close()
+    node.plan.close()
+
+
 @pytest.mark.parametrize("xs, o, second, k, hpool", [((2, 128, 13, 18), 96, True, 3, False), ((2, 3, 45, 50), 96, False, 7, False),
                                                      ((7, 3, 64, 64), 96, False, 7, True)])
 def test_conv_on_a_packed_filter_keeps_values_that_are_not_finite(pkg, monkeypatch, xs, o, second, k, hpool):
