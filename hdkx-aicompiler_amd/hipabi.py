@@ -113,7 +113,7 @@ def _need(t, dtype, name):
 # The operators below cost their caller more time in Python than most of their kernels take, so their entry points have
 # prototypes of their own (numbers, addresses and bytes go in as they are, without an object for each) and their
 # descriptors are packed without a ctypes structure.  us per call in a row, before and now: nn_conv2d 64 channels at 56 x 56, batch
-# 1 10.7 and 7.1.
+# 1 10.7 and 7.3.
 _PTR, _I32, _I64, _F32 = C.c_void_p, C.c_int32, C.c_int64, C.c_float
 _SIGNATURES = {
     "kxc_hip_conv2d_nchw_f32": [_PTR] * 7, "kxc_hip_conv2d_nchw_f32_noalloc": [_PTR] * 7, "kxc_hip_qconv2d_c16_i8": [_PTR] * 8,

@@ -454,7 +454,9 @@ int32_t kxc_hip_plan_add_conv2d_winograd(kxc_hip_plan* plan, const kxc_hip_conv2
                                          kxc_hip_buf w, kxc_hip_buf bias, kxc_hip_buf residual, kxc_hip_buf y,
                                          kxc_hip_buf u);
 /* The same with the size of `u` given: a node reads one form of the filter at most, chosen when the plan is finalized
- * among those that fit u_bytes (none: the node runs on `w` itself).  kxc_hip_conv2d_winograd_node_bytes says what the
+ * among those that fit u_bytes (none: the node runs on `w` itself): transformed, for small nodes packed as three bf16 parts
+ * (..._node_symbol says "slice"; nodes that share `u` and would take different forms take the transformed one in fp32).
+ * kxc_hip_conv2d_winograd_node_bytes says what the
  * form costs that a node of this shape would take under the calling thread's kxc_hip_set_select_lanes; it may be 0
  * (`u` is then any workspace offset).  Nodes of a plan may share `u` when they share `w` (the shares of a batch). */
 int32_t kxc_hip_plan_add_conv2d_winograd_sized(kxc_hip_plan* plan, const kxc_hip_conv2d_desc* desc, kxc_hip_buf x,
