@@ -128,9 +128,10 @@ typedef __attribute__((address_space(3))) void* lds_void_t;
 // ------------------------------------------------------------------------------------------
 // Filter transform into the packed three-part form.  A workgroup takes 32 output channels x 16 input channels; thread
 // (i, half, o) makes row i of U = G g G^T for eight channels and stores its four positions' fragments: the 32 lanes of a
-// half-wave write 512 contiguous bytes.
+// half-wave write 512 contiguous bytes.  PARTS: workgroups that share a tile's four columns of U.
 // ------------------------------------------------------------------------------------------
-__device__ __forceinline__ void weight_tile(const float* __restrict__ w, char* __restrict__ u, int32_t O, int32_t C, int tile,
+template <int PARTS>
+__device__ __forceinline__ void weight_tile(const float* __restrict__ w, char* __restrict__ u, int32_t O, int32_t C, int tile, int part,
                                             float* raw) {
     constexpr int RS = kStep * 9 + 1;
     const int ksteps = (C + kStep - 1) / kStep;
@@ -159,6 +160,7 @@ __device__ __forceinline__ void weight_tile(const float* __restrict__ w, char* _
     char* const dst = u + (static_cast<int64_t>(tile) * 16 + i * 4) * 3072 + (half * 32 + ol) * 16;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
+        if (j / (4 / PARTS) != part) continue;
         const Split8 s = split8(v[j]);
         *reinterpret_cast<u32x4*>(dst + j * 3072) = s.h;
         *reinterpret_cast<u32x4*>(dst + j * 3072 + 1024) = s.m;

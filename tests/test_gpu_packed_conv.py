@@ -462,3 +462,16 @@ def test_pointwise_convolution_of_few_channels(pkg, monkeypatch, xs, o, residual
     assert (np.isnan(got) == np.isnan(want)).all() and (got[np.isinf(want)] == want[np.isinf(want)]).all()
     m = np.isfinite(want)
     assert (np.abs(got[m] - want[m]) <= 1e-5 * np.maximum(np.abs(want[m]), 1.0)).all()
+
+
+@pytest.mark.parametrize("xs, o", [
+    ((16, 250, 14, 14), 500),       # 256 tiles of the filter, the last: four workgroups to a tile; channels short of a tile on both sides
+    ((12, 257, 14, 14), 512),       # 272: one; one channel in the last tile
+])
+def test_single_winograd_convolution_transforms_its_filter(pkg, monkeypatch, xs, o):
+    for name in ("KXC_HIP_CONV_BF16X3", "KXC_HIP_WINOGRAD_BF16X3"):
+        monkeypatch.delenv(name, raising=False)
+    x, wt, _, close = _filters(pkg, xs, o, 3, 2, o)
+    assert pkg.conv2d_variant(xs, tuple(wt[0].shape), 1, 1) == "winograd_f2k3_bf16x3"
+    for i in (0, 1, 0):             # the filter is read by every call
+        assert close(pkg.conv2d(x, wt[i], None, None, 1, 1), i)
