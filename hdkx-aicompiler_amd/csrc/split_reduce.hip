@@ -15,7 +15,6 @@ namespace {
 __device__ __forceinline__ float relu_sel(float v) { return (v > 0.0f) ? v : 0.0f; }
 
 __global__ void __launch_bounds__(256) conv_split_reduce_kernel(const SplitReduceArgs a) {
-    request_args(a);
     // XCD x (blockIdx % 8) takes the x-th eighth of the elements, like the kernels that wrote the parts
     const int32_t per_xcd = static_cast<int32_t>(gridDim.x >> 3);
     const int32_t block = static_cast<int32_t>(blockIdx.x & 7) * per_xcd + static_cast<int32_t>(blockIdx.x >> 3);
